@@ -53,6 +53,10 @@ int launch_generic_forward(hipStream_t stream, const GenericForwardArgs& args,
 // (attn_f32_mfma.hip).
 bool f32_forward_supported(const GenericForwardArgs& args);
 int launch_f32_forward(hipStream_t stream, const GenericForwardArgs& args, int sequences);
+// The FP32-storage backward on the FP32 matrix cores, head widths 32/64/128
+// (attn_f32_backward.hip); fills args.deltas itself.
+bool f32_backward_supported(const GenericBackwardArgs& args);
+int launch_f32_backward(hipStream_t stream, const GenericBackwardArgs& args);
 int launch_generic_probabilities(hipStream_t stream,
                                  const GenericForwardArgs& args, int sequences,
                                  float* probabilities);

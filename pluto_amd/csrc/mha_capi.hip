@@ -201,6 +201,10 @@ int pluto_hip_mha_backward(void* stream, int dtype, const void* qkv,
     return launch_flash_backward(s, a, reinterpret_cast<float*>(scratch + stats),
                                  reinterpret_cast<uint16_t*>(scratch + 2 * stats));
   }
+  if (!force_generic() && f32_backward_supported(a)) {
+    note_path(PLUTO_HIP_PATH_MATRIX_F32);
+    return launch_f32_backward(s, a);
+  }
   note_path(PLUTO_HIP_PATH_GENERIC);
   return launch_generic_backward(s, a);
 }

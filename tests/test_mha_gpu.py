@@ -92,6 +92,14 @@ def test_matches_oracle_across_configurations(capi, oracle, T, H, E, B, bf16):
     check(capi, oracle, T, H, E, B, bf16, seed=T * 7 + E)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 129, 200])
+def test_fp32_matrix_core_backward_at_tile_edges(capi, oracle, T, D):
+    # one streamed tile a wave and fewer, several, and ragged last tiles on both sides
+    check(capi, oracle, T, 2, 2 * D, 2, False, seed=T + D)
+    assert capi.last_path() == capi.PATH_MATRIX_F32
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_peaked_scores(capi, oracle, bf16):
     check(capi, oracle, 65, 1, 64, 2, bf16, seed=5, qk_scale=20.0 if not bf16 else 4.0)
