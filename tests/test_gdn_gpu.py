@@ -352,3 +352,25 @@ def test_layer_forward_matches_scalar_specification(capi, oracle, kh, vh, kd, vd
             # sequence_delta_net_test.cc:253-255
             assert np.all(np.abs(got[i] - want["out"]) <= 1.5e-4 + 1.5e-2 * np.abs(want["out"]))
             assert_close(state[i].cpu().numpy(), want["state"], 2e-3, "delta-net layer state")
+
+
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 15, 17, 70])
+def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T):
+    """The convolution walks sixteen rows a thread where there are enough of them and
+    four otherwise: the batch takes the one, its sequences alone the other.
+    Bit for bit the same, at row counts around either walk."""
+    kh, vh, kd, vd = 16, 48, 128, 128
+    channels = 2 * kh * kd + vh * vd
+    B = (1 << 23) // (T * channels) + 1
+    p = capi.delta_params(kh, vh, kd, vd)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    qkv, z, a, b = values(B, T, channels), values(B, T, vh * vd), values(B, T, vh), values(B, T, vh)
+    weights = tuple(dev(w) for w in layer_weights(kh, vh, kd, vd, 4))
+    state = torch.zeros((B, vh, kd, vd), device="cuda")
+    got = capi.gdn_layer_forward(p, qkv, z, a, b, *weights, state)
+    for i in sorted({0, 1, B - 1} & set(range(B))):
+        one = torch.zeros((1, vh, kd, vd), device="cuda")
+        want = capi.gdn_layer_forward(p, qkv[i:i + 1], z[i:i + 1], a[i:i + 1], b[i:i + 1], *weights, one)
+        assert torch.equal(got[i], want[0]) and torch.equal(state[i], one[0]), i
