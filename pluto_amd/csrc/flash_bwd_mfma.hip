@@ -71,11 +71,11 @@ __device__ inline BackwardUnit backward_unit(int tiles, int heads) {
 }
 
 // dQ^T[d, query] = sum_keys K^T[d, key] dS^T[key, query]
-template <int D, bool PAIRED>
+// PREPARED: dO arrives as bf16 with its row statistics, else the prologue makes them.
+template <int D, bool PAIRED, bool PREPARED>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
-flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
-                uint16_t* __restrict__ d_out_bf16) {
+flash_dq_kernel(FlashBackwardArgs a) {
   constexpr int BM = 128, BN = 64;
   constexpr int KCH = D / 8, KS = D / 16, DB = D / 32, KB = BN / 32;
   constexpr int LOADS = BN * KCH / kThreads;
@@ -90,26 +90,24 @@ flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
 
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
-  const int T = a.context_length, H = a.num_heads, E = a.embedding_dim;
+  const int T = a.context_length, H = a.num_heads, E = H * D;
   const int q_tiles = (T + BM - 1) / BM;
   const BackwardUnit unit = backward_unit<PAIRED>(q_tiles, H);
   const int pair = unit.pair, head = unit.head, seq = unit.seq;
   const long long seq_row0 = static_cast<long long>(seq) * T;
   const long long stats_base = (static_cast<long long>(seq) * H + head) * T;
-  const uint16_t* qkv = static_cast<const uint16_t*>(a.qkv);
-  const uint16_t* q_base = qkv + seq_row0 * 3 * E + head * D;
-  const uint16_t* k_base = q_base + E;
-  const uint16_t* v_base = q_base + 2 * E;
-  const uint16_t* o_base = static_cast<const uint16_t*>(a.out) + seq_row0 * E + head * D;
-  const float* g_base = a.d_out + seq_row0 * E + head * D;
-  uint16_t* gb_base = d_out_bf16 + seq_row0 * E + head * D;
+  const long long q_stride = a.q_row, kv_stride = a.kv_row;
+  const uint16_t* q_base = a.q + seq_row0 * q_stride + head * D;
+  const uint16_t* k_base = a.k + seq_row0 * kv_stride + head / a.group * D;
+  const uint16_t* v_base = a.v + seq_row0 * kv_stride + head / a.group * D;
+  uint16_t* gb_base = a.d_out_bf16 + seq_row0 * E + head * D;
   const float scale2 = a.scale * kLog2e;
 
-  // K and V rows share the packed row stride, hence one set of fill offsets.
+  // K and V rows share their row stride, hence one set of fill offsets.
   uint32_t fill[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i)
-    fill[i] = tile_fill_offset<D>((wave * LOADS + i) * 64 + lane, 3LL * E);
+    fill[i] = tile_fill_offset<D>((wave * LOADS + i) * 64 + lane, kv_stride);
   int row_read[KS], tr_read[DB];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) row_read[ks] = tile_row_read<D>(n, 2 * ks + h);
@@ -124,8 +122,8 @@ flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
     const int q0 = q_tile * BM;
     const int last_row = min(q0 + BM, T) - 1;
     const int tiles = last_row / BN + 1;
-    tile_fill<D, LOADS>(lds, wave, k_base, 3LL * E, 0, T, fill);
-    tile_fill<D, LOADS>(lds + kTileBytes, wave, v_base, 3LL * E, 0, T, fill);
+    tile_fill<D, LOADS>(lds, wave, k_base, kv_stride, 0, T, fill);
+    tile_fill<D, LOADS>(lds + kTileBytes, wave, v_base, kv_stride, 0, T, fill);
 
     const int wave_first_row = q0 + 32 * wave;
     const int q_row = wave_first_row + n;
@@ -134,49 +132,64 @@ flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
     // Rows beyond the sequence are clamped to its last row and never stored.
     const int q_load = min(q_row, T - 1);
     bf16x8 qf[KS], gf[KS];
-    float partial = 0.0f;
+    float row_delta, row_lse2;
+    if constexpr (PREPARED) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int c = 16 * ks + 8 * h;
-      qf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-          q_base + static_cast<long long>(q_load) * 3 * E + c));
-      const float4 g0 = *reinterpret_cast<const float4*>(g_base + static_cast<long long>(q_load) * E + c);
-      const float4 g1 = *reinterpret_cast<const float4*>(g_base + static_cast<long long>(q_load) * E + c + 4);
-      const uint4 o = *reinterpret_cast<const uint4*>(o_base + static_cast<long long>(q_load) * E + c);
-      const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-      const uint32_t ow[4] = {o.x, o.y, o.z, o.w};
-      uint32_t packed[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        partial += g[2 * i] * __uint_as_float(ow[i] << 16);
-        partial += g[2 * i + 1] * __uint_as_float(ow[i] & 0xffff0000u);
-        packed[i] = pack_bf16(g[2 * i], g[2 * i + 1]);
+      for (int ks = 0; ks < KS; ++ks) {
+        const int c = 16 * ks + 8 * h;
+        qf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(q_base + q_load * q_stride + c));
+        gf[ks] = as_bf16x8(
+            *reinterpret_cast<const uint4*>(gb_base + static_cast<long long>(q_load) * E + c));
       }
-      const uint4 bits = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-      gf[ks] = as_bf16x8(bits);
-      copy_area[n * KCH + ((2 * ks + h) ^ (n & 7))] = bits;
-    }
-    // The bf16 copy of dO leaves through LDS (the wave's slice of the stage
-    // that no fill has been issued into yet): a lane holds 16-byte pieces of its
-    // own row, and stored from there a store instruction touches 32 lines;
-    // from LDS it writes whole rows (25 MB in 17 us against 5 us).
+      row_delta = -a.deltas[stats_base + q_load];
+      row_lse2 = -a.lse2[stats_base + q_load] * scale2;
+    } else {
+      const uint16_t* o_base = a.out + seq_row0 * E + head * D;
+      const float* g_base = a.d_out + seq_row0 * E + head * D;
+      float partial = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32 * KCH / 64; ++i) {
-      const int at = i * 64 + lane, row = at / KCH, chunk = at % KCH;
-      const uint4 bits = copy_area[row * KCH + (chunk ^ (row & 7))];
-      if (wave_first_row + row < T)
-        *reinterpret_cast<uint4*>(gb_base + static_cast<long long>(wave_first_row + row) * E +
-                                  8 * chunk) = bits;
-    }
-    // delta of attention.cc:283-291 (uses the stored, rounded output)
-    const float row_delta = half_swap_sum(partial);
-    const float normalizer = a.normalizers[stats_base + q_load];
-    const float row_lse2 = a.maxima[stats_base + q_load] * kLog2e +
-                           __log2f(normalizer > 0.0f ? normalizer : 1.0f);
-    if (h == 0 && q_row < T) {
-      // the key-owned kernel starts its accumulators from these
-      a.deltas[stats_base + q_row] = -row_delta;
-      lse2[stats_base + q_row] = -row_lse2 / scale2;
+      for (int ks = 0; ks < KS; ++ks) {
+        const int c = 16 * ks + 8 * h;
+        qf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
+            q_base + q_load * q_stride + c));
+        const float4 g0 = *reinterpret_cast<const float4*>(g_base + static_cast<long long>(q_load) * E + c);
+        const float4 g1 = *reinterpret_cast<const float4*>(g_base + static_cast<long long>(q_load) * E + c + 4);
+        const uint4 o = *reinterpret_cast<const uint4*>(o_base + static_cast<long long>(q_load) * E + c);
+        const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+        const uint32_t ow[4] = {o.x, o.y, o.z, o.w};
+        uint32_t packed[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          partial += g[2 * i] * __uint_as_float(ow[i] << 16);
+          partial += g[2 * i + 1] * __uint_as_float(ow[i] & 0xffff0000u);
+          packed[i] = pack_bf16(g[2 * i], g[2 * i + 1]);
+        }
+        const uint4 bits = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+        gf[ks] = as_bf16x8(bits);
+        copy_area[n * KCH + ((2 * ks + h) ^ (n & 7))] = bits;
+      }
+      // The bf16 copy of dO leaves through LDS (the wave's slice of the stage
+      // that no fill has been issued into yet): a lane holds 16-byte pieces of its
+      // own row, and stored from there a store instruction touches 32 lines;
+      // from LDS it writes whole rows (25 MB in 17 us against 5 us).
+#pragma unroll
+      for (int i = 0; i < 32 * KCH / 64; ++i) {
+        const int at = i * 64 + lane, row = at / KCH, chunk = at % KCH;
+        const uint4 bits = copy_area[row * KCH + (chunk ^ (row & 7))];
+        if (wave_first_row + row < T)
+          *reinterpret_cast<uint4*>(gb_base + static_cast<long long>(wave_first_row + row) * E +
+                                    8 * chunk) = bits;
+      }
+      // delta of attention.cc:283-291 (uses the stored, rounded output)
+      row_delta = half_swap_sum(partial);
+      const float normalizer = a.normalizers[stats_base + q_load];
+      row_lse2 = a.maxima[stats_base + q_load] * kLog2e +
+                             __log2f(normalizer > 0.0f ? normalizer : 1.0f);
+      if (h == 0 && q_row < T) {
+        // the key-owned kernel starts its accumulators from these
+        a.deltas[stats_base + q_row] = -row_delta;
+        a.lse2[stats_base + q_row] = -row_lse2 / scale2;
+      }
     }
     floatx16 dq_acc[DB];
 #pragma unroll
@@ -193,11 +206,9 @@ flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
       __syncthreads();
       if (tile + 1 < tiles) {
         unsigned char* stage = lds + ((tile + 1) & 1) * kStageBytes;
-        tile_fill<D, LOADS>(stage, wave, k_base + static_cast<long long>(k0 + BN) * 3 * E,
-                            3LL * E, k0 + BN, T, fill);
-        tile_fill<D, LOADS>(stage + kTileBytes, wave,
-                            v_base + static_cast<long long>(k0 + BN) * 3 * E, 3LL * E, k0 + BN, T,
-                            fill);
+        tile_fill<D, LOADS>(stage, wave, k_base + (k0 + BN) * kv_stride, kv_stride, k0 + BN, T, fill);
+        tile_fill<D, LOADS>(stage + kTileBytes, wave, v_base + (k0 + BN) * kv_stride, kv_stride,
+                            k0 + BN, T, fill);
       }
       const unsigned char* k_tile = lds + (tile & 1) * kStageBytes;
       const unsigned char* v_tile = k_tile + kTileBytes;
@@ -251,7 +262,7 @@ flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
       // instruction then writes eight whole 128-byte half rows instead of
       // 32-byte pieces of 32 rows
       float4* area = reinterpret_cast<float4*>(own_area) + wave * 256;
-      float* dst = a.d_qkv + (seq_row0 + wave_first_row) * 3 * E + head * D;
+      float* dst = a.dq + (seq_row0 + wave_first_row) * a.dq_row + head * D;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
 #pragma unroll
@@ -268,12 +279,11 @@ flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
           const int row = 8 * i + lane / 8, piece = lane % 8;
           const float4 value = area[row * 8 + (piece ^ (row & 7))];
           if (wave_first_row + row < T)
-            *reinterpret_cast<float4*>(dst + static_cast<long long>(row) * 3 * E + 32 * db +
-                                       4 * piece) = value;
+            *reinterpret_cast<float4*>(dst + row * a.dq_row + 32 * db + 4 * piece) = value;
         }
       }
     } else if (q_row < T) {
-      float* dst = a.d_qkv + (seq_row0 + q_row) * 3 * E + head * D;
+      float* dst = a.dq + (seq_row0 + q_row) * a.dq_row + head * D;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -296,12 +306,11 @@ flash_dq_kernel(GenericBackwardArgs a, float* __restrict__ lse2,
 template <int D, int BQ, int LOADS>
 __device__ inline void dkv_fill_stage(unsigned char* stage, int wave, int lane,
                                       const uint16_t* q_base, const uint16_t* g_base,
-                                      const float* lse2_base, const float* delta_base, int E,
-                                      int q0, int T, const uint32_t* q_fill,
+                                      const float* lse2_base, const float* delta_base,
+                                      long long q_stride, int E, int q0, int T, const uint32_t* q_fill,
                                       const uint32_t* g_fill) {
   constexpr int kTileBytes = BQ * D * 2;
-  tile_fill<D, LOADS>(stage, wave, q_base + static_cast<long long>(q0) * 3 * E, 3LL * E, q0, T,
-                      q_fill);
+  tile_fill<D, LOADS>(stage, wave, q_base + q0 * q_stride, q_stride, q0, T, q_fill);
   tile_fill<D, LOADS>(stage + kTileBytes, wave, g_base + static_cast<long long>(q0) * E, 1LL * E,
                       q0, T, g_fill);
   if (wave < 2) {
@@ -317,8 +326,7 @@ __device__ inline void dkv_fill_stage(unsigned char* stage, int wave, int lane,
 template <int D, bool PAIRED>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(2, 2)))
-flash_dkv_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
-                 const uint16_t* __restrict__ d_out_bf16) {
+flash_dkv_kernel(FlashBackwardArgs a) {
   constexpr int BNK = 128;
   constexpr int BQ = D == 64 ? 64 : 32;  // query rows per LDS tile
   constexpr int KCH = D / 8, KS = D / 16, DB = D / 32, QB = BQ / 32;
@@ -331,18 +339,18 @@ flash_dkv_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
 
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
-  const int T = a.context_length, H = a.num_heads, E = a.embedding_dim;
+  const int T = a.context_length, H = a.num_heads, E = H * D;
   const int key_tiles = (T + BNK - 1) / BNK;
   const BackwardUnit unit = backward_unit<PAIRED>(key_tiles, H);
   const int pair = unit.pair, head = unit.head, seq = unit.seq;
   const long long seq_row0 = static_cast<long long>(seq) * T;
   const long long stats_base = (static_cast<long long>(seq) * H + head) * T;
-  const uint16_t* qkv = static_cast<const uint16_t*>(a.qkv);
-  const uint16_t* q_base = qkv + seq_row0 * 3 * E + head * D;
-  const uint16_t* k_base = q_base + E;
-  const uint16_t* v_base = q_base + 2 * E;
-  const uint16_t* g_base = d_out_bf16 + seq_row0 * E + head * D;
-  const float* lse2_base = lse2 + stats_base;
+  const long long q_stride = a.q_row, kv_stride = a.kv_row;
+  const uint16_t* q_base = a.q + seq_row0 * q_stride + head * D;
+  const uint16_t* k_base = a.k + seq_row0 * kv_stride + head / a.group * D;
+  const uint16_t* v_base = a.v + seq_row0 * kv_stride + head / a.group * D;
+  const uint16_t* g_base = a.d_out_bf16 + seq_row0 * E + head * D;
+  const float* lse2_base = a.lse2 + stats_base;
   const float* delta_base = a.deltas + stats_base;  // holds -delta
   const float scale2 = a.scale * kLog2e;
   const int tiles = (T + BQ - 1) / BQ;
@@ -350,7 +358,7 @@ flash_dkv_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
   uint32_t q_fill[LOADS], g_fill[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
-    q_fill[i] = tile_fill_offset<D>((wave * LOADS + i) * 64 + lane, 3LL * E);
+    q_fill[i] = tile_fill_offset<D>((wave * LOADS + i) * 64 + lane, q_stride);
     g_fill[i] = tile_fill_offset<D>((wave * LOADS + i) * 64 + lane, 1LL * E);
   }
   int row_read[KS], tr_read[DB];
@@ -369,16 +377,16 @@ flash_dkv_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
     const int first_tile = k0 / BQ;
     if (first_tile < tiles)
       dkv_fill_stage<D, BQ, LOADS>(lds + ((first_tile) & 1) * kStageBytes, wave, lane, q_base, g_base,
-                                   lse2_base, delta_base, E, (first_tile) * BQ, T, q_fill, g_fill);
+                                   lse2_base, delta_base, q_stride, E, (first_tile) * BQ, T, q_fill, g_fill);
     const int key_row = k0 + 32 * wave + n;
     const int key_load = min(key_row, T - 1);
     bf16x8 kf[KS], vf[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       kf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-          k_base + static_cast<long long>(key_load) * 3 * E + 16 * ks + 8 * h));
+          k_base + key_load * kv_stride + 16 * ks + 8 * h));
       vf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-          v_base + static_cast<long long>(key_load) * 3 * E + 16 * ks + 8 * h));
+          v_base + key_load * kv_stride + 16 * ks + 8 * h));
     }
     floatx16 dk_acc[DB], dv_acc[DB];
 #pragma unroll
@@ -396,7 +404,7 @@ flash_dkv_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
       __syncthreads();
       if (tile + 1 < tiles)
         dkv_fill_stage<D, BQ, LOADS>(lds + ((tile + 1) & 1) * kStageBytes, wave, lane, q_base, g_base,
-                                     lse2_base, delta_base, E, (tile + 1) * BQ, T, q_fill, g_fill);
+                                     lse2_base, delta_base, q_stride, E, (tile + 1) * BQ, T, q_fill, g_fill);
       const unsigned char* q_tile = lds + (tile & 1) * kStageBytes;
       const unsigned char* g_tile = q_tile + kTileBytes;
       const float* stat_lse2 = reinterpret_cast<const float*>(q_tile + 2 * kTileBytes);
@@ -504,14 +512,14 @@ flash_dkv_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
             area[n * kPieces + (piece ^ (n % kPieces))] = value;
           }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads what its own lanes wrote
-        float* dst = a.d_qkv + (seq_row0 + k0 + 32 * wave) * 3 * E + (1 + tensor) * E + head * D +
-                     64 * half;
+        float* dst = (tensor == 0 ? a.dk : a.dv) + (seq_row0 + k0 + 32 * wave) * a.dkv_row +
+                     head * D + 64 * half;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int row = 4 * i + out_row;
           const float4 value = area[row * kPieces + (out_piece ^ (row % kPieces))];
           if (k0 + 32 * wave + row < T)
-            *reinterpret_cast<float4*>(dst + static_cast<long long>(row) * 3 * E + 4 * out_piece) = value;
+            *reinterpret_cast<float4*>(dst + row * a.dkv_row + 4 * out_piece) = value;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the area is overwritten
       }
@@ -522,51 +530,84 @@ flash_dkv_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
 
 }  // namespace
 
-bool flash_backward_supported(const GenericBackwardArgs& a) {
-  const int dim = a.embedding_dim / a.num_heads;
-  if (a.dtype != PLUTO_HIP_BF16 || (dim != 64 && dim != 128)) return false;
-  auto aligned = [](const void* p) {
-    return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
-  };
-  // tiles of one sequence are addressed through 32-bit buffer offsets and a
-  // 32-bit descriptor size: a sequence's rows of the packed operand (the
-  // widest, 3E bf16 per row) must stay below 2 GiB
-  if (static_cast<long long>(a.context_length) * 3 * a.embedding_dim * 2 >= (1LL << 31))
-    return false;
-  return aligned(a.qkv) && aligned(a.out) && aligned(a.d_out) && aligned(a.d_qkv);
+FlashBackwardArgs packed_flash_backward(const GenericBackwardArgs& g, float* lse2,
+                                        uint16_t* d_out_bf16) {
+  FlashBackwardArgs a;
+  const long long E = g.embedding_dim;
+  a.q = static_cast<const uint16_t*>(g.qkv);
+  a.k = a.q + E;
+  a.v = a.q + 2 * E;
+  a.q_row = a.kv_row = 3 * E;
+  a.d_out = g.d_out;
+  a.out = static_cast<const uint16_t*>(g.out);
+  a.maxima = g.maxima;
+  a.normalizers = g.normalizers;
+  a.d_out_bf16 = d_out_bf16;
+  a.deltas = g.deltas;
+  a.lse2 = lse2;
+  a.dq = g.d_qkv;
+  a.dk = g.d_qkv + E;
+  a.dv = g.d_qkv + 2 * E;
+  a.dq_row = a.dkv_row = 3 * E;
+  a.sequences = g.rows / g.context_length;
+  a.context_length = g.context_length;
+  a.num_heads = g.num_heads;
+  a.head_dim = g.embedding_dim / g.num_heads;
+  a.scale = g.scale;
+  return a;
 }
 
-int launch_flash_backward(hipStream_t stream, const GenericBackwardArgs& a,
-                          float* lse2, uint16_t* d_out_bf16) {
-  const int dim = a.embedding_dim / a.num_heads;
-  const int sequences = a.rows / a.context_length;
-  int status = 0;
-  const long long tiles128 = (a.context_length + 127) / 128;
-  const long long units = 1LL * a.num_heads * sequences;
-  if (tiles128 * units > 0x7fffffffLL) return PLUTO_HIP_EINVAL;
-  const dim3 paired(static_cast<unsigned>(((tiles128 + 1) / 2) * units));
-  const dim3 unpaired(static_cast<unsigned>(tiles128 * units));
-  if (!kernel_enabled(kQueryKernel)) {
-  } else if (dim == 64)
-    flash_dq_kernel<64, kDqPaired64><<<kDqPaired64 ? paired : unpaired, kThreads, 0, stream>>>(
-        a, lse2, d_out_bf16);
+bool flash_backward_supported(const FlashBackwardArgs& a) {
+  if (a.head_dim != 64 && a.head_dim != 128) return false;
+  // tiles of one sequence are addressed through 32-bit buffer offsets and a
+  // 32-bit descriptor size: a sequence's rows of each operand must stay below 2 GiB
+  auto in_range = [&](long long row) { return a.context_length * row * 2 < (1LL << 31); };
+  if (!in_range(a.q_row) || !in_range(a.kv_row) || !in_range(1LL * a.num_heads * a.head_dim))
+    return false;
+  for (const void* p : {static_cast<const void*>(a.q), static_cast<const void*>(a.k),
+                        static_cast<const void*>(a.v), static_cast<const void*>(a.out),
+                        static_cast<const void*>(a.d_out), static_cast<const void*>(a.dq),
+                        static_cast<const void*>(a.dk), static_cast<const void*>(a.dv)})
+    if ((reinterpret_cast<uintptr_t>(p) & 15u) != 0) return false;
+  return true;
+}
+
+namespace {
+template <int D, bool DQ_PAIRED>
+void launch_dq(hipStream_t stream, const FlashBackwardArgs& a, unsigned grid) {
+  if (a.d_out)
+    flash_dq_kernel<D, DQ_PAIRED, false><<<grid, kThreads, 0, stream>>>(a);
   else
-    flash_dq_kernel<128, kOtherPaired><<<kOtherPaired ? paired : unpaired, kThreads, 0, stream>>>(
-        a, lse2, d_out_bf16);
-  status = launch_status();
+    flash_dq_kernel<D, DQ_PAIRED, true><<<grid, kThreads, 0, stream>>>(a);
+}
+}  // namespace
+
+int launch_flash_backward(hipStream_t stream, const FlashBackwardArgs& a) {
+  const int dim = a.head_dim;
+  const long long tiles128 = (a.context_length + 127) / 128;
+  const long long units = 1LL * a.num_heads * a.sequences;
+  if (tiles128 * units > 0x7fffffffLL) return PLUTO_HIP_EINVAL;
+  const unsigned paired = static_cast<unsigned>(((tiles128 + 1) / 2) * units);
+  const unsigned unpaired = static_cast<unsigned>(tiles128 * units);
+  if (!kernel_enabled(kQueryKernel)) {
+  } else if (dim == 64) {
+    launch_dq<64, kDqPaired64>(stream, a, kDqPaired64 ? paired : unpaired);
+  } else {
+    launch_dq<128, kOtherPaired>(stream, a, kOtherPaired ? paired : unpaired);
+  }
+  const int status = launch_status();
   if (status != 0) return status;
   if (!kernel_enabled(kMainKernel)) return 0;
   // The hand-scheduled kernel (one wave a SIMD, 64 keys a wave) gives the same
   // bits; it is level with the kernel below at 2048 rows and 6 % ahead at 4096.
   if (dim == 64 && kernel_enabled(kEightWave) &&
       (a.context_length >= kWideFromRows || !kernel_enabled(kFromLength)))
-    return launch_flash_dkv_wide(stream, a, lse2, d_out_bf16);
+    return launch_flash_dkv_wide(stream, a);
+  const unsigned grid = kOtherPaired ? paired : unpaired;
   if (dim == 64)
-    flash_dkv_kernel<64, kOtherPaired><<<kOtherPaired ? paired : unpaired, kThreads, 0, stream>>>(
-        a, lse2, d_out_bf16);
+    flash_dkv_kernel<64, kOtherPaired><<<grid, kThreads, 0, stream>>>(a);
   else
-    flash_dkv_kernel<128, kOtherPaired><<<kOtherPaired ? paired : unpaired, kThreads, 0, stream>>>(
-        a, lse2, d_out_bf16);
+    flash_dkv_kernel<128, kOtherPaired><<<grid, kThreads, 0, stream>>>(a);
   return launch_status();
 }
 

@@ -27,15 +27,14 @@ constexpr int kStageBytes = FLASH_DKV_D64_STAGE_BYTES;
 constexpr int kTileBytes = FLASH_DKV_D64_TILE_BYTES;
 
 __global__ void __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-flash_dkv_wide_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
-                      const uint16_t* __restrict__ d_out_bf16) {
+flash_dkv_wide_kernel(FlashBackwardArgs a) {
   constexpr int D = 64, BNK = 128, KS = D / 16, DB = D / 32;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
   static_assert(kTileBytes == 32 * D * 2);
 
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
-  const int T = a.context_length, H = a.num_heads, E = a.embedding_dim;
+  const int T = a.context_length, H = a.num_heads, E = H * D;
   const int key_tiles = (T + BNK - 1) / BNK;
   // one tile per workgroup, the tiles that see the most queries first; a
   // (sequence, head) unit keeps its XCD across tiles whenever the number of
@@ -45,11 +44,11 @@ flash_dkv_wide_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
   const int head = (blockIdx.x % units) % H, seq = (blockIdx.x % units) / H;
   const long long seq_row0 = static_cast<long long>(seq) * T;
   const long long stats_base = (static_cast<long long>(seq) * H + head) * T;
-  const uint16_t* qkv = static_cast<const uint16_t*>(a.qkv);
-  const uint16_t* q_base = qkv + seq_row0 * 3 * E + head * D;
-  const uint16_t* k_base = q_base + E;
-  const uint16_t* v_base = q_base + 2 * E;
-  const uint16_t* g_base = d_out_bf16 + seq_row0 * E + head * D;
+  const long long q_stride = a.q_row, kv_stride = a.kv_row;
+  const uint16_t* q_base = a.q + seq_row0 * q_stride + head * D;
+  const uint16_t* k_base = a.k + seq_row0 * kv_stride + head / a.group * D;
+  const uint16_t* v_base = a.v + seq_row0 * kv_stride + head / a.group * D;
+  const uint16_t* g_base = a.d_out_bf16 + seq_row0 * E + head * D;
   const int k0 = key_tile * BNK;
   const int first_block = k0 / 32;                       // query blocks first_block .. last_block
   const int steps = (T - 1) / 32 - first_block + 1;      // see some key of this tile
@@ -63,9 +62,9 @@ flash_dkv_wide_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       kf[c][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-          k_base + static_cast<long long>(key_load) * 3 * E + 16 * ks + 8 * h));
+          k_base + key_load * kv_stride + 16 * ks + 8 * h));
       vf[c][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-          v_base + static_cast<long long>(key_load) * 3 * E + 16 * ks + 8 * h));
+          v_base + key_load * kv_stride + 16 * ks + 8 * h));
     }
   }
 
@@ -79,23 +78,23 @@ flash_dkv_wide_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
                             tile_row_read<D>(n, 4 + h), tile_row_read<D>(n, 6 + h)};
   const int tr_read[DB] = {tile_transpose_read<D>(lane, 0), tile_transpose_read<D>(lane, 1)};
   const int stat_read = 2 * kTileBytes + 16 * h;
-  const uint32_t q_fill0 = tile_fill_offset<D>((wave * 2 + 0) * 64 + lane, 3LL * E);
-  const uint32_t q_fill1 = tile_fill_offset<D>((wave * 2 + 1) * 64 + lane, 3LL * E) - 1024u;
+  const uint32_t q_fill0 = tile_fill_offset<D>((wave * 2 + 0) * 64 + lane, q_stride);
+  const uint32_t q_fill1 = tile_fill_offset<D>((wave * 2 + 1) * 64 + lane, q_stride) - 1024u;
   const uint32_t g_fill0 = tile_fill_offset<D>((wave * 2 + 0) * 64 + lane, 1LL * E);
   const uint32_t g_fill1 = tile_fill_offset<D>((wave * 2 + 1) * 64 + lane, 1LL * E) - 1024u;
   const uint32_t s_fill = lane < 32 ? lane * 4u : 0x40000000u;
   const int rows_left = T - 1 - 32 * first_block;  // >= 0
-  const int32x4 q_rsrc = make_rsrc(q_base + static_cast<long long>(32 * first_block) * 3 * E,
-                                   static_cast<uint32_t>((static_cast<long long>(rows_left) * 3 * E + D) * 2));
+  const int32x4 q_rsrc = make_rsrc(q_base + 32 * first_block * q_stride,
+                                   static_cast<uint32_t>((rows_left * q_stride + D) * 2));
   const int32x4 g_rsrc = make_rsrc(g_base + static_cast<long long>(32 * first_block) * E,
                                    static_cast<uint32_t>((static_cast<long long>(rows_left) * E + D) * 2));
-  const float* stat_source = (wave == 0 ? lse2 : a.deltas) + stats_base + 32 * first_block;
+  const float* stat_source = (wave == 0 ? a.lse2 : a.deltas) + stats_base + 32 * first_block;
   const int32x4 s_rsrc = make_rsrc(stat_source, static_cast<uint32_t>(rows_left + 1) * 4u);
   const uint32_t lds_address = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds));
   const uint32_t lds_base = __builtin_amdgcn_readfirstlane(lds_address);
   const uint32_t lds_q = __builtin_amdgcn_readfirstlane(lds_address + wave * 2048);
   const uint32_t lds_s = __builtin_amdgcn_readfirstlane(lds_address + 2 * kTileBytes + wave * 256);
-  const uint32_t q_step = static_cast<uint32_t>(32LL * 3 * E * 2), g_step = static_cast<uint32_t>(32LL * E * 2);
+  const uint32_t q_step = static_cast<uint32_t>(32 * q_stride * 2), g_step = static_cast<uint32_t>(32LL * E * 2);
   const float scale2 = a.scale * kLog2e;
   const uint32_t scale2_bits = __builtin_amdgcn_readfirstlane(__float_as_uint(scale2));
   // a wave's blocks start two steps after the workgroup's per 64 keys of offset
@@ -172,13 +171,13 @@ flash_dkv_wide_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
         }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads what its own lanes wrote
       const int key0 = wave_first_key + 32 * c;
-      float* dst = a.d_qkv + (seq_row0 + key0) * 3 * E + (1 + tensor) * E + head * D;
+      float* dst = (tensor == 0 ? a.dk : a.dv) + (seq_row0 + key0) * a.dkv_row + head * D;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int row = 4 * i + out_row;
         const float4 value = area[row * kPieces + (out_piece ^ (row % kPieces))];
         if (key0 + row < T)
-          *reinterpret_cast<float4*>(dst + static_cast<long long>(row) * 3 * E + 4 * out_piece) = value;
+          *reinterpret_cast<float4*>(dst + row * a.dkv_row + 4 * out_piece) = value;
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the area is overwritten
     }
@@ -187,13 +186,11 @@ flash_dkv_wide_kernel(GenericBackwardArgs a, const float* __restrict__ lse2,
 
 }  // namespace
 
-int launch_flash_dkv_wide(hipStream_t stream, const GenericBackwardArgs& a, const float* lse2,
-                          const uint16_t* d_out_bf16) {
+int launch_flash_dkv_wide(hipStream_t stream, const FlashBackwardArgs& a) {
   const long long tiles = (a.context_length + 127) / 128;
-  const long long units = 1LL * a.num_heads * (a.rows / a.context_length);
+  const long long units = 1LL * a.num_heads * a.sequences;
   if (tiles * units > 0x7fffffffLL) return PLUTO_HIP_EINVAL;
-  flash_dkv_wide_kernel<<<dim3(static_cast<unsigned>(tiles * units)), kWideThreads, 0, stream>>>(
-      a, lse2, d_out_bf16);
+  flash_dkv_wide_kernel<<<dim3(static_cast<unsigned>(tiles * units)), kWideThreads, 0, stream>>>(a);
   return launch_status();
 }
 

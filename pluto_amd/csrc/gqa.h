@@ -131,12 +131,27 @@ int launch_pack_heads(hipStream_t stream, const void* q, const void* k, const vo
 int launch_gate_backward(hipStream_t stream, const void* qg, const void* core, int core_dtype,
                          const float* dy, int length, int query_heads, int head_dim, bool round,
                          float* dc, float* dqg);
-int launch_norm_rope_backward(hipStream_t stream, const void* input, const float* weight,
-                              const float* packed_grad, const float* cosines, const float* sines,
-                              int length, int heads, int query_heads, int head_dim, int rotary_dim,
-                              int input_stride, float epsilon, bool key_mode, float* dx,
-                              float* dv, float* parts);
-int launch_reduce_norm(hipStream_t stream, const float* parts, long long rows, int head_dim,
-                       float* partial, int chunks, float* dw);
+// The same for the matrix-core backward (head widths 64 and 128).
+int launch_gate_rows(hipStream_t stream, const void* qg, const void* core, const float* dy,
+                     const float* maxima, const float* normalizers, int length, int query_heads,
+                     int head_dim, float scale2, uint16_t* dc, float* dqg, float* deltas,
+                     float* lse2);
+// The attention gradients the norm backward starts from: one dQ, dK and dV per
+// query head, heads d elements apart, rows as given.
+struct NormBackwardGrads {
+  const float* dq = nullptr;
+  const float* dk = nullptr;
+  const float* dv = nullptr;
+  long long dq_row = 0, dkv_row = 0;
+};
+// Workgroups of the norm backward at most: `partial` holds a row of head_dim
+// floats for each.  (1536 workgroups of four waves are six waves a SIMD.)
+constexpr int kNormQueryBlocks = 1024, kNormKeyBlocks = 512;
+int launch_norm_rope_backward(hipStream_t stream, const void* qg, const void* k,
+                              const float* q_norm, const float* k_norm,
+                              const NormBackwardGrads& grads, const float* cosines,
+                              const float* sines, int length, int query_heads, int key_value_heads,
+                              int head_dim, int rotary_dim, float epsilon, float* dqg, float* dk,
+                              float* dv, float* dq_norm, float* dk_norm, float* partial);
 
 }  // namespace pluto_hip

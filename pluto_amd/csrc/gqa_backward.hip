@@ -4,16 +4,18 @@
 // buffers (saved probabilities and score gradients).
 //
 // The attention core of the backward is the multi-head kernel pair of this
-// library run on a packed [T, 3 * qh * d] view in which every query head
-// carries a copy of its kv head's K and V rows; the dK and dV of the copies
-// are then summed per kv head in ascending head order.  Around it:
-//   gate_backward_kernel        GateBackwardKernel        (:124-141)
-//   pack_heads_kernel           layout only
-//   norm_rope_backward_kernel   NormBackwardKernel        (:201-228), fused with
-//                               the per-kv-head sums
-//   reduce_norm_*_kernel        ReduceNormKernel          (:230-239), two
-//                               levels, fixed order
+// library.  The matrix-core pair reads each kv head's K and V where they lie; the
+// FP32 kernels run on a packed [T, 3 * qh * d] view in which every query head
+// carries a copy of them.  Both leave one dK and dV per query head, which are
+// summed per kv head in ascending head order.  Around it:
+//   gate_backward_kernel, gate_rows_kernel   GateBackwardKernel  (:124-141)
+//   pack_heads_kernel                        layout only
+//   norm_rope_*_kernel                       NormBackwardKernel  (:201-228), fused
+//                                            with the per-kv-head sums and the first
+//                                            level of ReduceNormKernel (:230-239)
+//   norm_weight_kernel                       its second level, fixed order
 #include "gqa.h"
+#include "mfma_tile.h"
 
 namespace pluto_hip {
 namespace {
@@ -61,115 +63,316 @@ gate_backward_kernel(const uint16_t* qg, const void* core, int core_dtype, const
   }
 }
 
-struct NormBackwardArgs {
+// Eight consecutive elements as floats, in one or two accesses when WIDE.
+template <bool WIDE>
+__device__ inline void load8(const uint16_t* p, float (&x)[8]) {
+  if constexpr (WIDE) {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      x[e] = __uint_as_float(e % 2 ? words[e / 2] & 0xffff0000u : words[e / 2] << 16);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = bf16_bits_to_float(p[e]);
+  }
+}
+template <bool WIDE>
+__device__ inline void load8(const float* p, float (&x)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 4) {
+    if constexpr (WIDE) {
+      const float4 v = *reinterpret_cast<const float4*>(p + e);
+      x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
+    } else {
+      x[e] = p[e]; x[e + 1] = p[e + 1]; x[e + 2] = p[e + 2]; x[e + 3] = p[e + 3];
+    }
+  }
+}
+template <bool WIDE>
+__device__ inline void store8(float* p, const float (&x)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 4) {
+    if constexpr (WIDE) {
+      *reinterpret_cast<float4*>(p + e) = make_float4(x[e], x[e + 1], x[e + 2], x[e + 3]);
+    } else {
+      p[e] = x[e]; p[e + 1] = x[e + 1]; p[e + 2] = x[e + 2]; p[e + 3] = x[e + 3];
+    }
+  }
+}
+
+// The same for the matrix-core kernels, which take dC as bf16 together with two
+// values of each row: -sum(dC * core) and the row's log2-sum-exp in the form
+// FlashBackwardArgs states.  Sixteen bytes of bf16 a lane, D / 8 lanes a row; a
+// workgroup walks 64 rows of one head, whose statistics are then contiguous.
+// 350 MB in and out at T = 8192, 24 heads of 128; written as an FP32 dC that
+// the query-owned kernel read again in pieces of its own rows, the same work moved
+// 550 MB (83 us for this pass alone).  WIDE: every tensor is 16-byte aligned.
+template <int D, bool WIDE>
+__global__ void __launch_bounds__(256)
+gate_rows_kernel(const uint16_t* __restrict__ qg, const uint16_t* __restrict__ core,
+                 const float* __restrict__ dy, const float* __restrict__ maxima,
+                 const float* __restrict__ normalizers, int length, int heads, float scale2,
+                 uint16_t* __restrict__ dc, float* __restrict__ dqg, float* __restrict__ deltas,
+                 float* __restrict__ lse2) {
+  constexpr int LANES = D / 8, ROWS = 256 / LANES;
+  const int piece = threadIdx.x % LANES, head = blockIdx.y;
+  for (int i = 0; i < 64; i += ROWS) {
+    const int row = blockIdx.x * 64 + i + threadIdx.x / LANES;
+    const bool exists = row < length;
+    const long long unit = 1LL * min(row, length - 1) * heads + head;
+    float grad[8], gates[8], values[8];
+    load8<WIDE>(dy + unit * D + 8 * piece, grad);
+    load8<WIDE>(qg + (unit * 2 + 1) * D + 8 * piece, gates);
+    load8<WIDE>(core + unit * D + 8 * piece, values);
+    float scaled[8], gate_grad[8];
+    float dot = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float sigmoid = 1.0f / (1.0f + expf(-gates[e]));
+      scaled[e] = grad[e] * round_to_bf16(sigmoid);
+      gate_grad[e] = grad[e] * values[e] * sigmoid * (1.0f - sigmoid);
+      dot += scaled[e] * values[e];
+    }
+#pragma unroll
+    for (int offset = LANES / 2; offset > 0; offset >>= 1) dot += __shfl_xor(dot, offset, 64);
+    if (!exists) continue;
+    *reinterpret_cast<uint4*>(dc + unit * D + 8 * piece) =
+        make_uint4(pack_bf16(scaled[0], scaled[1]), pack_bf16(scaled[2], scaled[3]),
+                   pack_bf16(scaled[4], scaled[5]), pack_bf16(scaled[6], scaled[7]));
+    store8<WIDE>(dqg + (unit * 2 + 1) * D + 8 * piece, gate_grad);
+    if (piece == 0) {
+      const long long at = 1LL * head * length + row;
+      const float normalizer = normalizers[at];
+      deltas[at] = -dot;
+      lse2[at] = -(maxima[at] * kLog2e + __log2f(normalizer > 0.0f ? normalizer : 1.0f)) / scale2;
+    }
+  }
+}
+
+// What one of the two halves (queries, keys) of the norm backward works on.
+struct NormSide {
   const uint16_t* input = nullptr;  // raw bf16 rows, `input_stride` apart
   const float* weight = nullptr;    // zero-centred norm weight [d]
-  const float* packed_grad = nullptr;  // fp32 [T, 3E]
-  const float* cosines = nullptr;      // [T, rotary/2]
+  float* dx = nullptr;              // rows `input_stride` apart
+  float* partial = nullptr;         // optional [blocks, d]: sums of the weight's gradient
+  float* weight_grad = nullptr;
+  int heads = 0, input_stride = 0, blocks = 0;
+};
+struct NormBackwardArgs {
+  NormSide queries, keys;
+  NormBackwardGrads grads;
+  const float* cosines = nullptr;  // [T, rotary/2]
   const float* sines = nullptr;
-  float* dx = nullptr;        // rows `input_stride` apart
-  float* dv = nullptr;        // key mode: [T, kh, d]
-  float* parts = nullptr;     // optional [T * heads, d]
-  int length = 0, heads = 0, d = 0, rotary = 0, input_stride = 0;
-  int query_heads = 0, group = 0;
-  bool key_mode = false;
+  float* dv = nullptr;  // [T, kh, d]
+  int length = 0, d = 0, rotary = 0, group = 0;
   float epsilon = 1e-6f;
 };
 
-// One wave per (row, head).  Query mode: the gradient of head h is its slice
-// of the packed dQ.  Key mode: the gradients of the kv head's `group` copies
-// are summed in ascending head order, for dK (which continues through RoPE and
-// the norm) and for dV (which is final).
+// Both kernels below: the first `queries.blocks` workgroups take the (row, head)
+// units of the queries, whose gradient is the head's dQ, the others those of
+// the keys, where the gradients of the kv head's `group` copies are summed in
+// ascending head order, for dK (which continues through RoPE and the norm) and
+// for dV (which is final).  A workgroup walks units blocks apart and keeps its
+// share of the weight's gradient in registers, so nothing per row is stored for
+// it (a stored row each cost 100 MB out and, summed by 128 workgroups, 620 us
+// back in at T = 8192, 24 heads of 128).
+
+// D / 8 lanes a unit, eight channels a lane; RoPE partners are whole pieces.
+template <int D>
+__global__ void __launch_bounds__(256)
+norm_rope_rows_kernel(NormBackwardArgs a) {
+  constexpr int LANES = D / 8, UNITS = 256 / LANES;
+  __shared__ float sums[UNITS][D];
+  const bool key_mode = static_cast<int>(blockIdx.x) >= a.queries.blocks;
+  const NormSide side = key_mode ? a.keys : a.queries;
+  const int block = blockIdx.x - (key_mode ? a.queries.blocks : 0);
+  const int piece = threadIdx.x % LANES, slot = threadIdx.x / LANES, c = 8 * piece;
+  const int half = a.rotary / 2;
+  const bool rotated = c < a.rotary, lower = c < half;
+  const int frequency = lower ? c : c - half;
+  // the lane of the same unit that holds the RoPE partner's piece
+  const int partner = threadIdx.x % 64 - piece + (rotated ? (lower ? c + half : c - half) / 8 : piece);
+  float factor[8], weight_sum[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    factor[e] = 1.0f + side.weight[c + e];
+    weight_sum[e] = 0.0f;
+  }
+  const long long units = 1LL * a.length * side.heads;
+  for (long long first = 1LL * block * UNITS; first < units; first += 1LL * side.blocks * UNITS) {
+    const bool exists = first + slot < units;
+    const long long unit = exists ? first + slot : units - 1;
+    const long long row = unit / side.heads;
+    const int head = static_cast<int>(unit % side.heads);
+    float x[8], g[8];
+    load8<true>(side.input + unit * side.input_stride + c, x);
+    if (!key_mode) {
+      load8<true>(a.grads.dq + row * a.grads.dq_row + head * D + c, g);
+    } else {
+      const long long at = row * a.grads.dkv_row + 1LL * head * a.group * D + c;
+      float value_sum[8], key[8], value[8];
+      load8<true>(a.grads.dk + at, g);
+      load8<true>(a.grads.dv + at, value_sum);
+      for (int copy = 1; copy < a.group; ++copy) {
+        load8<true>(a.grads.dk + at + copy * D, key);
+        load8<true>(a.grads.dv + at + copy * D, value);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          g[e] += key[e];
+          value_sum[e] += value[e];
+        }
+      }
+      if (exists) store8<true>(a.dv + unit * D + c, value_sum);
+    }
+    float squares = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) squares += x[e] * x[e];
+    float normalized[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) normalized[e] = g[e];
+    float other[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) other[e] = __shfl(g[e], partner, 64);
+    if (rotated) {
+      float co[8], si[8];
+      load8<true>(a.cosines + row * half + frequency, co);
+      load8<true>(a.sines + row * half + frequency, si);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        normalized[e] = g[e] * co[e] + (lower ? other[e] * si[e] : -other[e] * si[e]);
+    }
+    float dot = 0.0f, weighted[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      weighted[e] = normalized[e] * factor[e];
+      dot += weighted[e] * x[e];
+    }
+#pragma unroll
+    for (int offset = LANES / 2; offset > 0; offset >>= 1) {
+      squares += __shfl_xor(squares, offset, 64);
+      dot += __shfl_xor(dot, offset, 64);
+    }
+    const float inv = rsqrtf(squares / static_cast<float>(D) + a.epsilon);
+    const float cubic = inv * inv * inv / static_cast<float>(D) * dot;
+    if (!exists) continue;
+    float dx[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      dx[e] = inv * weighted[e] - x[e] * cubic;
+      weight_sum[e] += normalized[e] * x[e] * inv;
+    }
+    store8<true>(side.dx + unit * side.input_stride + c, dx);
+  }
+  if (!side.partial) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sums[slot][c + e] = weight_sum[e];
+  __syncthreads();
+  if (threadIdx.x < D) {
+    float total = 0.0f;
+    for (int u = 0; u < UNITS; ++u) total += sums[u][threadIdx.x];
+    side.partial[1LL * block * D + threadIdx.x] = total;
+  }
+}
+
+// Any head width up to 256: one wave a workgroup, one channel of four a lane.
 __global__ void __launch_bounds__(64)
 norm_rope_backward_kernel(NormBackwardArgs a) {
   __shared__ float grads[256];
-  const int lane = threadIdx.x;
-  const int unit = blockIdx.x, row = unit / a.heads, head = unit % a.heads;
-  const int d = a.d;
-  const long long E = 1LL * a.query_heads * d;
-  const float* packed_row = a.packed_grad + 3 * E * row;
-  float x[4], g[4];
-  float sum_squares = 0.0f;
+  const bool key_mode = static_cast<int>(blockIdx.x) >= a.queries.blocks;
+  const NormSide side = key_mode ? a.keys : a.queries;
+  const int block = blockIdx.x - (key_mode ? a.queries.blocks : 0);
+  const int lane = threadIdx.x, d = a.d, half = a.rotary / 2;
+  float weight_sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  const long long units = 1LL * a.length * side.heads;
+  for (long long unit = block; unit < units; unit += side.blocks) {
+    const long long row = unit / side.heads;
+    const int head = static_cast<int>(unit % side.heads);
+    float x[4], g[4];
+    float sum_squares = 0.0f;
+    __syncthreads();  // the unit before has read its partners
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = lane + 64 * j;
-    x[j] = 0.0f;
-    g[j] = 0.0f;
-    if (c < d) {
-      x[j] = bf16_bits_to_float(a.input[1LL * unit * a.input_stride + c]);
-      if (!a.key_mode) {
-        g[j] = packed_row[head * d + c];
-      } else {
-        float key_sum = 0.0f, value_sum = 0.0f;
-        for (int copy = 0; copy < a.group; ++copy) {
-          const int h = head * a.group + copy;
-          key_sum += packed_row[E + h * d + c];
-          value_sum += packed_row[2 * E + h * d + c];
+    for (int j = 0; j < 4; ++j) {
+      const int c = lane + 64 * j;
+      x[j] = 0.0f;
+      g[j] = 0.0f;
+      if (c < d) {
+        x[j] = bf16_bits_to_float(side.input[unit * side.input_stride + c]);
+        if (!key_mode) {
+          g[j] = a.grads.dq[row * a.grads.dq_row + head * d + c];
+        } else {
+          float key_sum = 0.0f, value_sum = 0.0f;
+          for (int copy = 0; copy < a.group; ++copy) {
+            const long long at = row * a.grads.dkv_row + 1LL * (head * a.group + copy) * d + c;
+            key_sum += a.grads.dk[at];
+            value_sum += a.grads.dv[at];
+          }
+          g[j] = key_sum;
+          a.dv[unit * d + c] = value_sum;
         }
-        g[j] = key_sum;
-        a.dv[1LL * unit * d + c] = value_sum;
+        grads[c] = g[j];
       }
-      grads[c] = g[j];
+      sum_squares += x[j] * x[j];
     }
-    sum_squares += x[j] * x[j];
+    __syncthreads();
+    sum_squares = wave_sum(sum_squares);
+    const float inv = rsqrtf(sum_squares / static_cast<float>(d) + a.epsilon);
+    float normalized[4], weighted[4];
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = lane + 64 * j;
+      normalized[j] = 0.0f;
+      weighted[j] = 0.0f;
+      if (c < d) {
+        float ng = g[j];
+        if (c < a.rotary) {
+          const int frequency = c < half ? c : c - half;
+          const float co = a.cosines[row * half + frequency];
+          const float si = a.sines[row * half + frequency];
+          const float partner = grads[c < half ? c + half : c - half];
+          ng = g[j] * co + (c < half ? partner * si : -partner * si);
+        }
+        normalized[j] = ng;
+        weighted[j] = ng * (1.0f + side.weight[c]);
+        dot += weighted[j] * x[j];
+      }
+    }
+    dot = wave_sum(dot);
+    const float cubic = inv * inv * inv / static_cast<float>(d);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = lane + 64 * j;
+      if (c < d) {
+        side.dx[unit * side.input_stride + c] = inv * weighted[j] - x[j] * cubic * dot;
+        weight_sum[j] += normalized[j] * x[j] * inv;
+      }
+    }
   }
+  if (!side.partial) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (lane + 64 * j < d) side.partial[1LL * block * d + lane + 64 * j] = weight_sum[j];
+}
+
+// dw[c] += sum over the workgroups of partial[block, c], in a fixed order:
+// workgroup 0 the queries' weight, workgroup 1 the keys'.
+__global__ void __launch_bounds__(1024)
+norm_weight_kernel(NormBackwardArgs a) {
+  __shared__ float sums[1024];
+  const NormSide side = blockIdx.x == 0 ? a.queries : a.keys;
+  if (!side.partial) return;
+  const int d = a.d, groups = 1024 / d;
+  const int c = threadIdx.x % d, g = threadIdx.x / d;
+  float sum = 0.0f;
+  if (g < groups)
+    for (int block = g; block < side.blocks; block += groups) sum += side.partial[1LL * block * d + c];
+  sums[threadIdx.x] = sum;
   __syncthreads();
-  sum_squares = wave_sum(sum_squares);
-  const float inv = rsqrtf(sum_squares / static_cast<float>(d) + a.epsilon);
-  const int half = a.rotary / 2;
-  float normalized[4], weighted[4];
-  float dot = 0.0f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = lane + 64 * j;
-    normalized[j] = 0.0f;
-    weighted[j] = 0.0f;
-    if (c < d) {
-      float ng = g[j];
-      if (c < a.rotary) {
-        const int frequency = c < half ? c : c - half;
-        const float co = a.cosines[1LL * row * half + frequency];
-        const float si = a.sines[1LL * row * half + frequency];
-        const float partner = grads[c < half ? c + half : c - half];
-        ng = g[j] * co + (c < half ? partner * si : -partner * si);
-      }
-      normalized[j] = ng;
-      weighted[j] = ng * (1.0f + a.weight[c]);
-      dot += weighted[j] * x[j];
-    }
-  }
-  dot = wave_sum(dot);
-  const float cubic = inv * inv * inv / static_cast<float>(d);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = lane + 64 * j;
-    if (c < d) {
-      a.dx[1LL * unit * a.input_stride + c] = inv * weighted[j] - x[j] * cubic * dot;
-      if (a.parts) a.parts[1LL * unit * d + c] = normalized[j] * x[j] * inv;
-    }
-  }
-}
-
-// dw[c] += sum over rows of parts[row, c], in two levels with a fixed order.
-__global__ void __launch_bounds__(256)
-reduce_norm_partial_kernel(const float* parts, long long rows, int d, int chunks, float* partial) {
-  const int c = threadIdx.x;
-  if (c >= d) return;
-  const long long per = (rows + chunks - 1) / chunks;
-  const long long first = blockIdx.x * per;
-  const long long last = first + per < rows ? first + per : rows;
-  float sum = 0.0f;
-  for (long long row = first; row < last; ++row) sum += parts[row * d + c];
-  partial[1LL * blockIdx.x * d + c] = sum;
-}
-
-__global__ void __launch_bounds__(256)
-reduce_norm_final_kernel(const float* partial, int chunks, int d, float* dw) {
-  const int c = threadIdx.x;
-  if (c >= d) return;
-  float sum = 0.0f;
-  for (int chunk = 0; chunk < chunks; ++chunk) sum += partial[1LL * chunk * d + c];
-  dw[c] += sum;
+  if (threadIdx.x >= d) return;
+  float total = 0.0f;
+  for (int k = 0; k < groups; ++k) total += sums[k * d + c];
+  side.weight_grad[c] += total;
 }
 
 int grid_for(long long elements) {
@@ -217,39 +420,73 @@ int launch_gate_backward(hipStream_t stream, const void* qg, const void* core, i
   return launch_status();
 }
 
-int launch_norm_rope_backward(hipStream_t stream, const void* input, const float* weight,
-                              const float* packed_grad, const float* cosines, const float* sines,
-                              int length, int heads, int query_heads, int d, int rotary,
-                              int input_stride, float epsilon, bool key_mode, float* dx,
-                              float* dv, float* parts) {
-  NormBackwardArgs a;
-  a.input = static_cast<const uint16_t*>(input);
-  a.weight = weight;
-  a.packed_grad = packed_grad;
-  a.cosines = cosines;
-  a.sines = sines;
-  a.dx = dx;
-  a.dv = dv;
-  a.parts = parts;
-  a.length = length;
-  a.heads = heads;
-  a.d = d;
-  a.rotary = rotary;
-  a.input_stride = input_stride;
-  a.query_heads = query_heads;
-  a.group = query_heads / (key_mode ? heads : query_heads);
-  a.key_mode = key_mode;
-  a.epsilon = epsilon;
-  norm_rope_backward_kernel<<<static_cast<unsigned>(length) * heads, 64, 0, stream>>>(a);
+int launch_gate_rows(hipStream_t stream, const void* qg, const void* core, const float* dy,
+                     const float* maxima, const float* normalizers, int length, int qh, int d,
+                     float scale2, uint16_t* dc, float* dqg, float* deltas, float* lse2) {
+  const dim3 grid((length + 63) / 64, qh);
+  const auto* gates = static_cast<const uint16_t*>(qg);
+  const auto* values = static_cast<const uint16_t*>(core);
+  bool wide = true;
+  for (const void* p : {qg, core, static_cast<const void*>(dy), static_cast<const void*>(dqg)})
+    wide = wide && (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, 256, 0, stream>>>(gates, values, dy, maxima, normalizers, length, qh, scale2, dc,
+                                     dqg, deltas, lse2);
+  };
+  if (d == 64)
+    launch(wide ? gate_rows_kernel<64, true> : gate_rows_kernel<64, false>);
+  else if (d == 128)
+    launch(wide ? gate_rows_kernel<128, true> : gate_rows_kernel<128, false>);
+  else
+    return PLUTO_HIP_EUNSUPPORTED;
   return launch_status();
 }
 
-int launch_reduce_norm(hipStream_t stream, const float* parts, long long rows, int d,
-                       float* partial, int chunks, float* dw) {
-  reduce_norm_partial_kernel<<<chunks, 256, 0, stream>>>(parts, rows, d, chunks, partial);
-  int status = launch_status();
-  if (status != 0) return status;
-  reduce_norm_final_kernel<<<1, 256, 0, stream>>>(partial, chunks, d, dw);
+int launch_norm_rope_backward(hipStream_t stream, const void* qg, const void* k,
+                              const float* q_norm, const float* k_norm,
+                              const NormBackwardGrads& grads, const float* cosines,
+                              const float* sines, int length, int qh, int kh, int d, int rotary,
+                              float epsilon, float* dqg, float* dk, float* dv, float* dq_norm,
+                              float* dk_norm, float* partial) {
+  NormBackwardArgs a;
+  a.queries = {static_cast<const uint16_t*>(qg), q_norm, dqg, nullptr, dq_norm, qh, 2 * d, 0};
+  a.keys = {static_cast<const uint16_t*>(k), k_norm, dk, nullptr, dk_norm, kh, d, 0};
+  a.grads = grads;
+  a.cosines = cosines;
+  a.sines = sines;
+  a.dv = dv;
+  a.length = length;
+  a.d = d;
+  a.rotary = rotary;
+  a.group = qh / kh;
+  a.epsilon = epsilon;
+  bool rows = (d == 64 || d == 128 || d == 256) && rotary % 16 == 0 && grads.dq_row % 4 == 0 &&
+              grads.dkv_row % 4 == 0;
+  for (const void* p : {qg, k, static_cast<const void*>(dqg), static_cast<const void*>(dk),
+                        static_cast<const void*>(dv), static_cast<const void*>(grads.dq),
+                        static_cast<const void*>(grads.dk), static_cast<const void*>(grads.dv)})
+    rows = rows && (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
+  const long long per = rows ? 2048 / d : 1;  // units a workgroup works on at once
+  auto blocks = [&](int heads, int most) {
+    const long long wanted = (1LL * length * heads + per - 1) / per;
+    return static_cast<int>(wanted < most ? wanted : most);
+  };
+  a.queries.blocks = blocks(qh, kNormQueryBlocks);
+  a.keys.blocks = blocks(kh, kNormKeyBlocks);
+  if (dq_norm) a.queries.partial = partial;
+  if (dk_norm) a.keys.partial = partial + 1LL * kNormQueryBlocks * d;
+  const int grid = a.queries.blocks + a.keys.blocks;
+  if (!rows)
+    norm_rope_backward_kernel<<<grid, 64, 0, stream>>>(a);
+  else if (d == 64)
+    norm_rope_rows_kernel<64><<<grid, 256, 0, stream>>>(a);
+  else if (d == 128)
+    norm_rope_rows_kernel<128><<<grid, 256, 0, stream>>>(a);
+  else
+    norm_rope_rows_kernel<256><<<grid, 256, 0, stream>>>(a);
+  const int status = launch_status();
+  if (status != 0 || (!dq_norm && !dk_norm)) return status;
+  norm_weight_kernel<<<2, 1024, 0, stream>>>(a);
   return launch_status();
 }
 

@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "attn_generic.h"
+#include "flash_bwd_mfma.h"
 #include "flash_fwd_mfma.h"
 #include "gqa.h"
 
@@ -96,25 +97,29 @@ PrefillLayout prefill_layout(const pluto_hip_attention_params* p, int length) {
   return l;
 }
 
-// Scratch of the whole-sequence backward.
+// Scratch of the whole-sequence backward.  d_heads: dQ, dK and dV of every query
+// head, three tensors [T, qh * d] for the matrix-core kernels and one packed
+// [T, 3 * qh * d] for the others, as `packed` is there.
 struct PrefillBackwardLayout {
-  size_t cosines, sines, queries, keys, values, packed, core, maxima, normalizers, dc, d_packed,
-      q_parts, k_parts, partial, attention, total;
+  size_t cosines, sines, queries, keys, values, packed, core, maxima, normalizers, dc, deltas, lse2,
+      d_heads, partial, attention, total;
   size_t attention_bytes;
-  int dtype;  // storage of the packed view and of the recomputed core
+  bool flash;
+  int dtype;  // storage of the prepared heads and of the recomputed core
 };
-constexpr int kNormReduceChunks = 128;
 
 PrefillBackwardLayout prefill_backward_layout(const pluto_hip_attention_params* p, int length,
-                                              bool q_weight_grad, bool k_weight_grad) {
+                                              bool weight_grad) {
   PrefillBackwardLayout l{};
   const size_t T = static_cast<size_t>(length);
   const size_t qh = p->query_heads, kh = p->key_value_heads, d = p->head_dim;
   // bf16 storage (matrix-core kernels, bf16 tolerance) where those kernels
-  // exist; everything else runs the FP32 kernels on FP32 storage.
-  const bool flash = p->round_to_bfloat16 && (d == 64 || d == 128) && !force_generic();
-  l.dtype = flash ? PLUTO_HIP_BF16 : PLUTO_HIP_F32;
-  const size_t element = flash ? 2 : 4;
+  // exist and a tensor's rows can be addressed through their 32-bit offsets;
+  // everything else runs the FP32 kernels on FP32 storage.
+  l.flash = p->round_to_bfloat16 && (d == 64 || d == 128) && !force_generic() &&
+            T * qh * d * 2 < (1ull << 31);
+  l.dtype = l.flash ? PLUTO_HIP_BF16 : PLUTO_HIP_F32;
+  const size_t element = l.flash ? 2 : 4;
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t offset = at;
@@ -126,19 +131,19 @@ PrefillBackwardLayout prefill_backward_layout(const pluto_hip_attention_params* 
   l.queries = take(T * qh * d * element);
   l.keys = take(T * kh * d * element);
   l.values = take(T * kh * d * element);
-  l.packed = take(3 * T * qh * d * element);
+  l.packed = take(l.flash ? 0 : 3 * T * qh * d * element);
   l.core = take(T * qh * d * element);
   l.maxima = take(T * qh * 4);
   l.normalizers = take(T * qh * 4);
-  l.dc = take(T * qh * d * 4);
-  l.d_packed = take(3 * T * qh * d * 4);
-  l.q_parts = take(q_weight_grad ? T * qh * d * 4 : 0);
-  l.k_parts = take(k_weight_grad ? T * kh * d * 4 : 0);
-  l.partial = take((q_weight_grad || k_weight_grad) ? kNormReduceChunks * d * 4 : 0);
+  l.dc = take(T * qh * d * element);
+  l.deltas = take(l.flash ? T * qh * 4 : 0);
+  l.lse2 = take(l.flash ? T * qh * 4 : 0);
+  l.d_heads = take(3 * T * qh * d * 4);
+  l.partial = take(weight_grad ? (kNormQueryBlocks + kNormKeyBlocks) * d * 4 : 0);
   l.attention_bytes = pluto_hip_mha_backward_workspace_bytes(
       l.dtype, length, length, p->query_heads, p->query_heads * p->head_dim);
-  l.attention = take(l.attention_bytes);
-  l.total = at;
+  l.attention = take(l.flash ? 0 : l.attention_bytes);
+  l.total = at + 256;  // the scratch starts at the next multiple of 256
   return l;
 }
 
@@ -308,7 +313,7 @@ size_t pluto_hip_gqa_prefill_backward_workspace_bytes(const pluto_hip_attention_
                                                       int length, int q_weight_grad,
                                                       int k_weight_grad) {
   if (validate_params(p) != 0 || length <= 0) return 0;
-  return prefill_backward_layout(p, length, q_weight_grad != 0, k_weight_grad != 0).total;
+  return prefill_backward_layout(p, length, q_weight_grad != 0 || k_weight_grad != 0).total;
 }
 
 int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_params* p, int length,
@@ -321,13 +326,13 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   if (status != 0) return status;
   if (length <= 0) return PLUTO_HIP_EINVAL;
   if (!qg || !k || !v || !q_norm || !k_norm || !dy || !dqg || !dk || !dv) return PLUTO_HIP_EINVAL;
-  const PrefillBackwardLayout l = prefill_backward_layout(p, length, dq_norm != nullptr,
-                                                          dk_norm != nullptr);
+  const PrefillBackwardLayout l =
+      prefill_backward_layout(p, length, dq_norm != nullptr || dk_norm != nullptr);
   if (l.attention_bytes == 0) return PLUTO_HIP_EINVAL;
   if (!workspace || workspace_bytes < l.total) return PLUTO_HIP_EWORKSPACE;
-  if (saved && l.dtype != PLUTO_HIP_BF16) return PLUTO_HIP_EUNSUPPORTED;
+  if (saved && !saved_supported(p, PLUTO_HIP_BF16)) return PLUTO_HIP_EUNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  char* scratch = static_cast<char*>(workspace);
+  char* scratch = reinterpret_cast<char*>(align_up(reinterpret_cast<size_t>(workspace), 256));
   float* cosines = reinterpret_cast<float*>(scratch + l.cosines);
   float* sines = reinterpret_cast<float*>(scratch + l.sines);
   const bool round = p->round_to_bfloat16 != 0;
@@ -360,56 +365,84 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   prep.round = round;
   status = launch_prefill_prepare(s, prep);
   if (status != 0) return status;
-  status = launch_pack_heads(s, scratch + l.queries, scratch + l.keys, scratch + l.values, l.dtype,
-                             length, qh, kh, d, scratch + l.packed);
-  if (status != 0) return status;
   const void* core = scratch + l.core;
-  const float* maxima = reinterpret_cast<const float*>(scratch + l.maxima);
-  const float* normalizers = reinterpret_cast<const float*>(scratch + l.normalizers);
-  if (saved) {
-    const SavedLayout sl = saved_layout(p, length);
-    const char* base = static_cast<const char*>(saved);
-    core = base + sl.core;
-    maxima = reinterpret_cast<const float*>(base + sl.maxima);
-    normalizers = reinterpret_cast<const float*>(base + sl.normalizers);
+  float* maxima = reinterpret_cast<float*>(scratch + l.maxima);
+  float* normalizers = reinterpret_cast<float*>(scratch + l.normalizers);
+  float* d_heads = reinterpret_cast<float*>(scratch + l.d_heads);
+  NormBackwardGrads grads;
+  if (l.flash) {
+    const long long head_rows = 1LL * length * E;
+    grads = {d_heads, d_heads + head_rows, d_heads + 2 * head_rows, E, E};
+    FlashBackwardArgs f;
+    f.q = reinterpret_cast<const uint16_t*>(scratch + l.queries);
+    f.k = reinterpret_cast<const uint16_t*>(scratch + l.keys);
+    f.v = reinterpret_cast<const uint16_t*>(scratch + l.values);
+    f.q_row = E;
+    f.kv_row = 1LL * kh * d;
+    f.group = qh / kh;
+    f.d_out_bf16 = reinterpret_cast<uint16_t*>(scratch + l.dc);
+    f.deltas = reinterpret_cast<float*>(scratch + l.deltas);
+    f.lse2 = reinterpret_cast<float*>(scratch + l.lse2);
+    f.dq = d_heads;
+    f.dk = d_heads + head_rows;
+    f.dv = d_heads + 2 * head_rows;
+    f.dq_row = f.dkv_row = E;
+    f.sequences = 1;
+    f.context_length = length;
+    f.num_heads = qh;
+    f.head_dim = d;
+    f.scale = 1.0f / std::sqrt(static_cast<float>(d));
+    if (saved) {
+      const SavedLayout sl = saved_layout(p, length);
+      const char* base = static_cast<const char*>(saved);
+      core = base + sl.core;
+      maxima = reinterpret_cast<float*>(const_cast<char*>(base) + sl.maxima);
+      normalizers = reinterpret_cast<float*>(const_cast<char*>(base) + sl.normalizers);
+    } else {
+      FlashForwardArgs forward;
+      forward.q = f.q;
+      forward.k = f.k;
+      forward.v = f.v;
+      forward.q_row_stride = forward.o_row_stride = E;
+      forward.k_row_stride = forward.v_row_stride = f.kv_row;
+      forward.q_head_stride = forward.k_head_stride = forward.v_head_stride = d;
+      forward.o_head_stride = d;
+      forward.out = reinterpret_cast<uint16_t*>(scratch + l.core);
+      forward.maxima = maxima;
+      forward.normalizers = normalizers;
+      forward.q_rows = forward.kv_rows = length;
+      forward.query_heads = qh;
+      forward.group = f.group;
+      forward.scale = f.scale;
+      if (!flash_forward_supported(forward, d)) return PLUTO_HIP_EUNSUPPORTED;
+      status = launch_flash_forward(s, forward, d, 1);
+      if (status != 0) return status;
+    }
+    if (!flash_backward_supported(f)) return PLUTO_HIP_EUNSUPPORTED;
+    note_path(PLUTO_HIP_PATH_FLASH);
+    status = launch_gate_rows(s, qg, core, dy, maxima, normalizers, length, qh, d, f.scale * kLog2e,
+                              f.d_out_bf16, dqg, f.deltas, f.lse2);
+    if (status != 0) return status;
+    status = launch_flash_backward(s, f);
   } else {
+    grads = {d_heads, d_heads + E, d_heads + 2LL * E, 3LL * E, 3LL * E};
+    status = launch_pack_heads(s, scratch + l.queries, scratch + l.keys, scratch + l.values,
+                               l.dtype, length, qh, kh, d, scratch + l.packed);
+    if (status != 0) return status;
     status = pluto_hip_mha_forward(stream, l.dtype, scratch + l.packed, length, length, qh, E,
-                                   scratch + l.core,
-                                   reinterpret_cast<float*>(scratch + l.maxima),
-                                   reinterpret_cast<float*>(scratch + l.normalizers));
+                                   scratch + l.core, maxima, normalizers);
     if (status != 0) return status;
-  }
-
-  float* dc = reinterpret_cast<float*>(scratch + l.dc);
-  status = launch_gate_backward(s, qg, core, l.dtype, dy, length, qh, d, round, dc, dqg);
-  if (status != 0) return status;
-  float* d_packed = reinterpret_cast<float*>(scratch + l.d_packed);
-  status = pluto_hip_mha_backward(stream, l.dtype, scratch + l.packed, core, dc, maxima,
-                                  normalizers, length, length, qh, E, d_packed,
-                                  scratch + l.attention, l.attention_bytes);
-  if (status != 0) return status;
-
-  float* q_parts = dq_norm ? reinterpret_cast<float*>(scratch + l.q_parts) : nullptr;
-  float* k_parts = dk_norm ? reinterpret_cast<float*>(scratch + l.k_parts) : nullptr;
-  status = launch_norm_rope_backward(s, qg, q_norm, d_packed, cosines, sines, length, qh, qh, d,
-                                     p->rotary_dim, 2 * d, p->rms_norm_epsilon, false, dqg, nullptr,
-                                     q_parts);
-  if (status != 0) return status;
-  status = launch_norm_rope_backward(s, k, k_norm, d_packed, cosines, sines, length, kh, qh, d,
-                                     p->rotary_dim, d, p->rms_norm_epsilon, true, dk, dv, k_parts);
-  if (status != 0) return status;
-  float* partial = reinterpret_cast<float*>(scratch + l.partial);
-  if (dq_norm) {
-    status = launch_reduce_norm(s, q_parts, 1LL * length * qh, d, partial, kNormReduceChunks,
-                                dq_norm);
+    float* dc = reinterpret_cast<float*>(scratch + l.dc);
+    status = launch_gate_backward(s, qg, core, l.dtype, dy, length, qh, d, round, dc, dqg);
     if (status != 0) return status;
+    status = pluto_hip_mha_backward(stream, l.dtype, scratch + l.packed, core, dc, maxima,
+                                    normalizers, length, length, qh, E, d_heads,
+                                    scratch + l.attention, l.attention_bytes);
   }
-  if (dk_norm) {
-    status = launch_reduce_norm(s, k_parts, 1LL * length * kh, d, partial, kNormReduceChunks,
-                                dk_norm);
-    if (status != 0) return status;
-  }
-  return 0;
+  if (status != 0) return status;
+  return launch_norm_rope_backward(s, qg, k, q_norm, k_norm, grads, cosines, sines, length, qh, kh,
+                                   d, p->rotary_dim, p->rms_norm_epsilon, dqg, dk, dv, dq_norm,
+                                   dk_norm, reinterpret_cast<float*>(scratch + l.partial));
 }
 
 int pluto_hip_gqa_prefill_probabilities(void* stream, const pluto_hip_attention_params* p,

@@ -192,14 +192,17 @@ int pluto_hip_mha_backward(void* stream, int dtype, const void* qkv,
   a.embedding_dim = embedding_dim;
   const int D = embedding_dim / num_heads;
   a.scale = 1.0f / std::sqrt(static_cast<float>(D));
-  if (dtype == PLUTO_HIP_BF16 && !force_generic() &&
-      flash_backward_supported(a)) {
+  if (dtype == PLUTO_HIP_BF16 && !force_generic()) {
     const size_t stats =
         align_up(static_cast<size_t>(rows) * num_heads * sizeof(float), 256);
     char* scratch = static_cast<char*>(workspace);
-    note_path(PLUTO_HIP_PATH_FLASH);
-    return launch_flash_backward(s, a, reinterpret_cast<float*>(scratch + stats),
-                                 reinterpret_cast<uint16_t*>(scratch + 2 * stats));
+    const FlashBackwardArgs f =
+        packed_flash_backward(a, reinterpret_cast<float*>(scratch + stats),
+                              reinterpret_cast<uint16_t*>(scratch + 2 * stats));
+    if (flash_backward_supported(f)) {
+      note_path(PLUTO_HIP_PATH_FLASH);
+      return launch_flash_backward(s, f);
+    }
   }
   if (!force_generic() && f32_backward_supported(a)) {
     note_path(PLUTO_HIP_PATH_MATRIX_F32);
