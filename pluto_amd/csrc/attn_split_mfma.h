@@ -1,0 +1,39 @@
+// Attention forward and backward to FP32 accuracy for bf16 queries, keys and
+// values of head width 256 (attn_split_mfma.hip).
+#pragma once
+
+#include "common.h"
+
+namespace pluto_hip {
+
+constexpr int kSplitHeadDim = 256;
+
+// All heads are 256 elements apart within a row.
+struct SplitArgs {
+  const uint16_t* q = nullptr;  // [T, heads, 256]
+  const uint16_t* k = nullptr;  // [T, heads / group, 256]
+  const uint16_t* v = nullptr;
+  int length = 0, heads = 0, group = 1;
+  float scale = 1.0f;
+  float* core = nullptr;      // [T, heads, 256] attention output
+  float* maxima = nullptr;    // [heads, T] of the scaled scores
+  float* inverses = nullptr;  // [heads, T] 1 / normalizer
+  // backward: the gradient of core as three bf16 tensors [T, heads, 256] whose sum
+  // it is, `piece` elements apart, and its row products with core
+  uint16_t* d_core = nullptr;
+  long long piece = 0;
+  float* deltas = nullptr;  // [heads, T]
+  float* dq = nullptr;      // [T, heads, 256], one gradient per query head
+  float* dk = nullptr;
+  float* dv = nullptr;
+};
+
+bool split_attention_supported(int length, int heads, int head_dim);
+int launch_split_forward(hipStream_t stream, const SplitArgs& args);
+// dC = dy * Round(sigmoid(gate)) into args.d_core and args.deltas;
+// d gate = dy * Round(core) * s (1 - s) into the gate half of dqg.
+int launch_split_gate(hipStream_t stream, const SplitArgs& args, const void* qg, const float* dy,
+                      float* dqg);
+int launch_split_backward(hipStream_t stream, const SplitArgs& args);
+
+}  // namespace pluto_hip

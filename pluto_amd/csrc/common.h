@@ -72,6 +72,44 @@ __device__ inline void store_element(void* base, long long index, int dtype,
     static_cast<float*>(base)[index] = value;
 }
 
+// Eight consecutive elements as floats, in one or two accesses when WIDE.
+template <bool WIDE>
+__device__ inline void load8(const uint16_t* p, float (&x)[8]) {
+  if constexpr (WIDE) {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      x[e] = __uint_as_float(e % 2 ? words[e / 2] & 0xffff0000u : words[e / 2] << 16);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = bf16_bits_to_float(p[e]);
+  }
+}
+template <bool WIDE>
+__device__ inline void load8(const float* p, float (&x)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 4) {
+    if constexpr (WIDE) {
+      const float4 v = *reinterpret_cast<const float4*>(p + e);
+      x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
+    } else {
+      x[e] = p[e]; x[e + 1] = p[e + 1]; x[e + 2] = p[e + 2]; x[e + 3] = p[e + 3];
+    }
+  }
+}
+template <bool WIDE>
+__device__ inline void store8(float* p, const float (&x)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 4) {
+    if constexpr (WIDE) {
+      *reinterpret_cast<float4*>(p + e) = make_float4(x[e], x[e + 1], x[e + 2], x[e + 3]);
+    } else {
+      p[e] = x[e]; p[e + 1] = x[e + 1]; p[e + 2] = x[e + 2]; p[e + 3] = x[e + 3];
+    }
+  }
+}
+
 __device__ inline float wave_half_max(float v) {
   // reduction over 32 consecutive lanes (one half of a wave64)
   for (int offset = 16; offset > 0; offset >>= 1)

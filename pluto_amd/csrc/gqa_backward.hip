@@ -63,44 +63,6 @@ gate_backward_kernel(const uint16_t* qg, const void* core, int core_dtype, const
   }
 }
 
-// Eight consecutive elements as floats, in one or two accesses when WIDE.
-template <bool WIDE>
-__device__ inline void load8(const uint16_t* p, float (&x)[8]) {
-  if constexpr (WIDE) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    const uint32_t words[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      x[e] = __uint_as_float(e % 2 ? words[e / 2] & 0xffff0000u : words[e / 2] << 16);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = bf16_bits_to_float(p[e]);
-  }
-}
-template <bool WIDE>
-__device__ inline void load8(const float* p, float (&x)[8]) {
-#pragma unroll
-  for (int e = 0; e < 8; e += 4) {
-    if constexpr (WIDE) {
-      const float4 v = *reinterpret_cast<const float4*>(p + e);
-      x[e] = v.x; x[e + 1] = v.y; x[e + 2] = v.z; x[e + 3] = v.w;
-    } else {
-      x[e] = p[e]; x[e + 1] = p[e + 1]; x[e + 2] = p[e + 2]; x[e + 3] = p[e + 3];
-    }
-  }
-}
-template <bool WIDE>
-__device__ inline void store8(float* p, const float (&x)[8]) {
-#pragma unroll
-  for (int e = 0; e < 8; e += 4) {
-    if constexpr (WIDE) {
-      *reinterpret_cast<float4*>(p + e) = make_float4(x[e], x[e + 1], x[e + 2], x[e + 3]);
-    } else {
-      p[e] = x[e]; p[e + 1] = x[e + 1]; p[e + 2] = x[e + 2]; p[e + 3] = x[e + 3];
-    }
-  }
-}
-
 // The same for the matrix-core kernels, which take dC as bf16 together with two
 // values of each row: -sum(dC * core) and the row's log2-sum-exp in the form
 // FlashBackwardArgs states.  Sixteen bytes of bf16 a lane, D / 8 lanes a row; a
@@ -355,23 +317,32 @@ norm_rope_backward_kernel(NormBackwardArgs a) {
     if (lane + 64 * j < d) side.partial[1LL * block * d + lane + 64 * j] = weight_sum[j];
 }
 
-// dw[c] += sum over the workgroups of partial[block, c], in a fixed order:
-// workgroup 0 the queries' weight, workgroup 1 the keys'.
+// dw[c] += sum over the workgroups of partial[block, c], in a fixed order: row 0 of
+// the grid the queries' weight, row 1 the keys'.  A workgroup takes eight
+// channels, 128 threads each (one workgroup for all channels took 34 us over the
+// same half megabyte).
 __global__ void __launch_bounds__(1024)
 norm_weight_kernel(NormBackwardArgs a) {
-  __shared__ float sums[1024];
-  const NormSide side = blockIdx.x == 0 ? a.queries : a.keys;
+  __shared__ float sums[128][8], quarter[16][8];
+  const NormSide side = blockIdx.y == 0 ? a.queries : a.keys;
   if (!side.partial) return;
-  const int d = a.d, groups = 1024 / d;
-  const int c = threadIdx.x % d, g = threadIdx.x / d;
+  const int k = threadIdx.x % 8, g = threadIdx.x / 8, c = blockIdx.x * 8 + k;
   float sum = 0.0f;
-  if (g < groups)
-    for (int block = g; block < side.blocks; block += groups) sum += side.partial[1LL * block * d + c];
-  sums[threadIdx.x] = sum;
+  if (c < a.d)
+    for (int block = g; block < side.blocks; block += 128) sum += side.partial[1LL * block * a.d + c];
+  sums[g][k] = sum;
   __syncthreads();
-  if (threadIdx.x >= d) return;
+  if (g < 16) {
+    float total = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) total += sums[8 * g + i][k];
+    quarter[g][k] = total;
+  }
+  __syncthreads();
+  if (g != 0 || c >= a.d) return;
   float total = 0.0f;
-  for (int k = 0; k < groups; ++k) total += sums[k * d + c];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) total += quarter[i][k];
   side.weight_grad[c] += total;
 }
 
@@ -486,7 +457,7 @@ int launch_norm_rope_backward(hipStream_t stream, const void* qg, const void* k,
     norm_rope_rows_kernel<256><<<grid, 256, 0, stream>>>(a);
   const int status = launch_status();
   if (status != 0 || (!dq_norm && !dk_norm)) return status;
-  norm_weight_kernel<<<2, 1024, 0, stream>>>(a);
+  norm_weight_kernel<<<dim3((d + 7) / 8, 2), 1024, 0, stream>>>(a);
   return launch_status();
 }
 

@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "attn_generic.h"
+#include "attn_split_mfma.h"
 #include "flash_bwd_mfma.h"
 #include "flash_fwd_mfma.h"
 #include "gqa.h"
@@ -104,8 +105,8 @@ struct PrefillBackwardLayout {
   size_t cosines, sines, queries, keys, values, packed, core, maxima, normalizers, dc, deltas, lse2,
       d_heads, partial, attention, total;
   size_t attention_bytes;
-  bool flash;
-  int dtype;  // storage of the prepared heads and of the recomputed core
+  bool flash, split;  // bf16 kernels; FP32-accurate kernels on bf16 heads; neither: FP32 kernels
+  int dtype;          // storage of the prepared heads
 };
 
 PrefillBackwardLayout prefill_backward_layout(const pluto_hip_attention_params* p, int length,
@@ -118,8 +119,11 @@ PrefillBackwardLayout prefill_backward_layout(const pluto_hip_attention_params* 
   // everything else runs the FP32 kernels on FP32 storage.
   l.flash = p->round_to_bfloat16 && (d == 64 || d == 128) && !force_generic() &&
             T * qh * d * 2 < (1ull << 31);
-  l.dtype = l.flash ? PLUTO_HIP_BF16 : PLUTO_HIP_F32;
-  const size_t element = l.flash ? 2 : 4;
+  l.split = p->round_to_bfloat16 && split_attention_supported(length, p->query_heads, p->head_dim) &&
+            !force_generic();
+  const bool matrix = l.flash || l.split;
+  l.dtype = matrix ? PLUTO_HIP_BF16 : PLUTO_HIP_F32;
+  const size_t element = matrix ? 2 : 4;
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t offset = at;
@@ -131,18 +135,18 @@ PrefillBackwardLayout prefill_backward_layout(const pluto_hip_attention_params* 
   l.queries = take(T * qh * d * element);
   l.keys = take(T * kh * d * element);
   l.values = take(T * kh * d * element);
-  l.packed = take(l.flash ? 0 : 3 * T * qh * d * element);
-  l.core = take(T * qh * d * element);
+  l.packed = take(matrix ? 0 : 3 * T * qh * d * element);
+  l.core = take(T * qh * d * (l.flash ? 2 : 4));
   l.maxima = take(T * qh * 4);
   l.normalizers = take(T * qh * 4);
-  l.dc = take(T * qh * d * element);
-  l.deltas = take(l.flash ? T * qh * 4 : 0);
+  l.dc = take(T * qh * d * (l.flash ? 2 : l.split ? 6 : 4));
+  l.deltas = take(matrix ? T * qh * 4 : 0);
   l.lse2 = take(l.flash ? T * qh * 4 : 0);
   l.d_heads = take(3 * T * qh * d * 4);
   l.partial = take(weight_grad ? (kNormQueryBlocks + kNormKeyBlocks) * d * 4 : 0);
   l.attention_bytes = pluto_hip_mha_backward_workspace_bytes(
       l.dtype, length, length, p->query_heads, p->query_heads * p->head_dim);
-  l.attention = take(l.flash ? 0 : l.attention_bytes);
+  l.attention = take(matrix ? 0 : l.attention_bytes);
   l.total = at + 256;  // the scratch starts at the next multiple of 256
   return l;
 }
@@ -424,6 +428,32 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
                               f.d_out_bf16, dqg, f.deltas, f.lse2);
     if (status != 0) return status;
     status = launch_flash_backward(s, f);
+  } else if (l.split) {
+    const long long head_rows = 1LL * length * E;
+    grads = {d_heads, d_heads + head_rows, d_heads + 2 * head_rows, E, E};
+    SplitArgs a;
+    a.q = reinterpret_cast<const uint16_t*>(scratch + l.queries);
+    a.k = reinterpret_cast<const uint16_t*>(scratch + l.keys);
+    a.v = reinterpret_cast<const uint16_t*>(scratch + l.values);
+    a.length = length;
+    a.heads = qh;
+    a.group = qh / kh;
+    a.scale = 1.0f / std::sqrt(static_cast<float>(d));
+    a.core = reinterpret_cast<float*>(scratch + l.core);
+    a.maxima = maxima;
+    a.inverses = normalizers;
+    a.d_core = reinterpret_cast<uint16_t*>(scratch + l.dc);
+    a.piece = head_rows;
+    a.deltas = reinterpret_cast<float*>(scratch + l.deltas);
+    a.dq = d_heads;
+    a.dk = d_heads + head_rows;
+    a.dv = d_heads + 2 * head_rows;
+    note_path(PLUTO_HIP_PATH_MATRIX_F32);
+    status = launch_split_forward(s, a);
+    if (status != 0) return status;
+    status = launch_split_gate(s, a, qg, dy, dqg);
+    if (status != 0) return status;
+    status = launch_split_backward(s, a);
   } else {
     grads = {d_heads, d_heads + E, d_heads + 2LL * E, 3LL * E, 3LL * E};
     status = launch_pack_heads(s, scratch + l.queries, scratch + l.keys, scratch + l.values,
