@@ -10,7 +10,7 @@
 // are 2^-24 of the product, what one FP32 rounding costs.  Per 32 x 32 block of
 // scores in products of depth 256: S 1, P V 3 (forward); S 1, dP 3, dQ 3; and
 // S 1, dP 3, dK 3, dV 6.  At sixteen times the rate of the FP32 matrix
-// instruction that is a third of its time.  T = 1024, 24/4 heads: 0.03, 0.06
+// instruction that is a third of its time.  T = 1024, 24/4 heads: 0.05, 0.07
 // and 0.12 ms for the three kernels, where the kernels that multiply one element
 // at a time took 3.9, 5.0 and 7.4 ms.
 //
@@ -26,7 +26,7 @@ namespace pluto_hip {
 namespace {
 
 constexpr int D = kSplitHeadDim;
-constexpr int kThreads = 256, kRows = 32, kOwned = 128;
+constexpr int kThreads = 256, kRows = 32;
 constexpr int KCH = D / 8, KS = D / 16, DB = D / 32;
 constexpr int kLoads = kRows * KCH / kThreads;
 constexpr int kTileBytes = kRows * D * 2;
@@ -69,64 +69,134 @@ __device__ inline void load_row_operand(const uint16_t* row, int h, bf16x8 (&out
     out[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(row + 16 * ks + 8 * h));
 }
 
-// Where a wave's lanes read a tile, and what they fetch of one.
+// Where a wave's lanes read a tile, and what they fetch of one.  The swizzle
+// permutes pieces within groups of eight, so operand addresses repeat every 128
+// bytes of a row and four (two) registers serve all of them.
 struct TileAccess {
   uint32_t fill[kLoads];
-  int row_read[KS], tr_read[DB];
+  int row_read[4], tr_read[2];
   __device__ TileAccess(int wave, int lane, long long row_stride) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i)
       fill[i] = tile_fill_offset<D>((wave * kLoads + i) * 64 + lane, row_stride);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) row_read[ks] = tile_row_read<D>(lane % 32, 2 * ks + lane / 32);
+    for (int i = 0; i < 4; ++i) row_read[i] = tile_row_read<D>(lane % 32, 2 * i + lane / 32);
 #pragma unroll
-    for (int db = 0; db < DB; ++db) tr_read[db] = tile_transpose_read<D>(lane, db);
+    for (int i = 0; i < 2; ++i) tr_read[i] = tile_transpose_read<D>(lane, i);
+  }
+  // A operand: row n of the tile, contraction step ks
+  __device__ bf16x8 row(const unsigned char* tile, int ks) const {
+    return as_bf16x8(*reinterpret_cast<const uint4*>(tile + row_read[ks % 4] + ks / 4 * 128));
+  }
+  // A operand: channels 32 db + n of rows 16 s2 ..
+  __device__ bf16x8 transposed(const unsigned char* tile, int db, int s2) const {
+    return tile_transposed_operand<D>(tile + db / 2 * 128, tr_read[db % 2], s2);
   }
 };
-__device__ inline bf16x8 row_operand(const unsigned char* tile, int offset) {
-  return as_bf16x8(*reinterpret_cast<const uint4*>(tile + offset));
-}
+
+// Nothing moves across: the operands of a step are requested before the matrix
+// instructions of the step before it, one step ahead of their use.  (Left to
+// itself the compiler requests an operand and waits for it before every one to
+// three matrix instructions: 282 us for dK/dV at T = 1024, 24 heads.)
+__device__ inline void fence_schedule() { __builtin_amdgcn_sched_barrier(0); }
 
 __device__ inline void stage_ready() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 }
 
+// The two query-owned kernels: a workgroup owns 64 queries, waves 0 and 1 the two
+// halves at even key tiles, waves 2 and 3 the same at odd ones, and the upper
+// waves' results are added in at the end.  One wave a SIMD has nothing to cover
+// the chain scores -> softmax -> products of a tile; at T = 1024 the longest chain
+// is what the kernel takes, and this halves it (forward 79 -> 52 us, dQ 103 -> 70).
+constexpr int kQueries = 64;
+constexpr int kQueryStageBytes = 4 * kTileBytes;  // K and V of two tiles
+struct QueryWave {
+  int head, half, parity, steps, first_query, query, query_load;
+  __device__ QueryWave(const SplitArgs& a, int wave, int n) {
+    head = blockIdx.x % a.heads;
+    const int q0 = ((a.length + kQueries - 1) / kQueries - 1 - static_cast<int>(blockIdx.x) / a.heads) * kQueries;
+    half = wave % 2;
+    parity = wave / 2;
+    steps = ((min(q0 + kQueries, a.length) - 1) / kRows) / 2 + 1;  // two tiles each
+    first_query = q0 + 32 * half;
+    query = first_query + n;
+    query_load = min(query, a.length - 1);
+  }
+};
+// Queues the fill of step's two tiles: K, V of the even one, K, V of the odd one.
+__device__ inline void fill_query_stage(const SplitArgs& a, unsigned char* lds, int step, int wave,
+                                        int head, const uint32_t* offsets) {
+  const long long kv_row = 1LL * (a.heads / a.group) * D;
+  const long long column = head / a.group * D;
+  unsigned char* stage = lds + (step & 1) * kQueryStageBytes;
+#pragma unroll
+  for (int tile = 0; tile < 2; ++tile) {
+    const int k0 = (2 * step + tile) * kRows;
+    tile_fill<D, kLoads>(stage + 2 * tile * kTileBytes, wave, a.k + column + k0 * kv_row, kv_row, k0,
+                         a.length, offsets);
+    tile_fill<D, kLoads>(stage + (2 * tile + 1) * kTileBytes, wave, a.v + column + k0 * kv_row,
+                         kv_row, k0, a.length, offsets);
+  }
+}
+// The accumulators of the upper waves into LDS, 32 KiB each.
+__device__ inline void store_upper(unsigned char* lds, int half, int lane, const floatx16 (&acc)[DB]) {
+  float4* area = reinterpret_cast<float4*>(lds + half * 2 * kTileBytes);
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      area[(4 * db + j) * 64 + lane] =
+          make_float4(acc[db][4 * j], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]);
+}
+__device__ inline float4 load_upper(const unsigned char* lds, int half, int lane, int piece) {
+  return reinterpret_cast<const float4*>(lds + half * 2 * kTileBytes)[piece * 64 + lane];
+}
+
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 split_forward_kernel(SplitArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2][2 * kTileBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQueryStageBytes];
+  __shared__ float upper_stats[2][2][64];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
-  const int T = a.length, head = blockIdx.x % a.heads;
-  const int q0 = ((T + kOwned - 1) / kOwned - 1 - static_cast<int>(blockIdx.x) / a.heads) * kOwned;
-  const long long q_row = 1LL * a.heads * D, kv_row = 1LL * (a.heads / a.group) * D;
-  const uint16_t* k_base = a.k + head / a.group * D;
-  const uint16_t* v_base = a.v + head / a.group * D;
-  const int first_query = q0 + 32 * wave, query = first_query + n, query_load = min(query, T - 1);
-  const TileAccess at(wave, lane, kv_row);
-  const int tiles = (min(q0 + kOwned, T) - 1) / kRows + 1;
-  auto fill = [&](int tile) {
-    unsigned char* stage = lds[tile & 1];
-    const int k0 = tile * kRows;
-    tile_fill<D, kLoads>(stage, wave, k_base + k0 * kv_row, kv_row, k0, T, at.fill);
-    tile_fill<D, kLoads>(stage + kTileBytes, wave, v_base + k0 * kv_row, kv_row, k0, T, at.fill);
-  };
-  fill(0);
+  const QueryWave w(a, wave, n);
+  const int T = a.length, query = w.query, query_load = w.query_load, head = w.head;
+  const long long q_row = 1LL * a.heads * D;
+  const TileAccess at(wave, lane, 1LL * (a.heads / a.group) * D);
+  fill_query_stage(a, lds, 0, wave, head, at.fill);
   bf16x8 qf[KS];
   load_row_operand(a.q + query_load * q_row + head * D, h, qf);
   floatx16 o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) o[db] = zero16();
   float running_max = kMasked, running_sum = 0.0f;  // of the scaled scores
-  for (int tile = 0; tile < tiles; ++tile) {
-    const int k0 = tile * kRows;
+  for (int step = 0; step < w.steps; ++step) {
+    const int k0 = (2 * step + w.parity) * kRows;
     stage_ready();
-    if (tile + 1 < tiles) fill(tile + 1);
-    if (k0 > first_query + 31) continue;  // every key follows my queries
-    const unsigned char* k_tile = lds[tile & 1];
+    if (step + 1 < w.steps) fill_query_stage(a, lds, step + 1, wave, head, at.fill);
+    if (k0 > w.first_query + 31) continue;  // every key follows my queries
+    const unsigned char* k_tile = lds + (step & 1) * kQueryStageBytes + w.parity * 2 * kTileBytes;
     const unsigned char* v_tile = k_tile + kTileBytes;
     floatx16 s = zero16();
+    {
+      bf16x8 kf[2][4];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) s = mfma32(row_operand(k_tile, at.row_read[ks]), qf[ks], s);
+      for (int i = 0; i < 4; ++i) kf[0][i] = at.row(k_tile, i);
+#pragma unroll
+      for (int g = 0; g < KS / 4; ++g) {
+        if (g + 1 < KS / 4)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) kf[(g + 1) % 2][i] = at.row(k_tile, 4 * (g + 1) + i);
+        fence_schedule();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s = mfma32(kf[g % 2][i], qf[4 * g + i], s);
+        fence_schedule();
+      }
+    }
+    bf16x8 vt[3];
+    vt[0] = at.transposed(v_tile, 0, 0);
+    vt[1] = at.transposed(v_tile, 1, 0);
+    fence_schedule();
     // register i = (key k0 + 8(i/4) + 4h + i%4, query n)
     const int limit = query_load - k0 - 4 * h;
     float tile_max = kMasked;
@@ -156,24 +226,45 @@ split_forward_kernel(SplitArgs a) {
       const Pieces p = split_accumulator(s, s2);
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        const bf16x8 vt = tile_transposed_operand<D>(v_tile, at.tr_read[db], s2);
+        const int at_step = s2 * DB + db;
+        if (at_step + 2 < 2 * DB)
+          vt[(at_step + 2) % 3] = at.transposed(v_tile, (at_step + 2) % DB, (at_step + 2) / DB);
+        fence_schedule();
 #pragma unroll
-        for (int part = 2; part >= 0; --part) o[db] = mfma32(vt, p.part[part], o[db]);
+        for (int part = 2; part >= 0; --part) o[db] = mfma32(vt[at_step % 3], p.part[part], o[db]);
+        fence_schedule();
       }
     }
   }
-  if (query >= T) return;
-  const float inverse = 1.0f / (running_sum > 0.0f ? running_sum : 1.0f);
+  __syncthreads();  // nobody reads the stages any more
+  if (w.parity == 1) {
+    store_upper(lds, w.half, lane, o);
+    upper_stats[w.half][0][lane] = running_max;
+    upper_stats[w.half][1][lane] = running_sum;
+  }
+  __syncthreads();
+  if (w.parity == 1 || query >= T) return;
+  // a wave without tiles contributes weight 2^(kMasked - maximum) = 0
+  const float upper_max = upper_stats[w.half][0][lane];
+  const float maximum = fmaxf(running_max, upper_max);
+  const float own = __builtin_amdgcn_exp2f((running_max - maximum) * kLog2e);
+  const float other = __builtin_amdgcn_exp2f((upper_max - maximum) * kLog2e);
+  const float sum = running_sum * own + upper_stats[w.half][1][lane] * other;
+  const float inverse = 1.0f / (sum > 0.0f ? sum : 1.0f);
   float* out = a.core + query * q_row + head * D + 4 * h;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      const float4 u = load_upper(lds, w.half, lane, 4 * db + j);
       *reinterpret_cast<float4*>(out + 32 * db + 8 * j) =
-          make_float4(o[db][4 * j] * inverse, o[db][4 * j + 1] * inverse,
-                      o[db][4 * j + 2] * inverse, o[db][4 * j + 3] * inverse);
+          make_float4((o[db][4 * j] * own + u.x * other) * inverse,
+                      (o[db][4 * j + 1] * own + u.y * other) * inverse,
+                      (o[db][4 * j + 2] * own + u.z * other) * inverse,
+                      (o[db][4 * j + 3] * own + u.w * other) * inverse);
+    }
   if (h == 0) {
-    a.maxima[1LL * head * T + query] = running_max;
+    a.maxima[1LL * head * T + query] = maximum;
     a.inverses[1LL * head * T + query] = inverse;
   }
 }
@@ -222,23 +313,13 @@ split_gate_kernel(SplitArgs a, const uint16_t* __restrict__ qg, const float* __r
 
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 split_dq_kernel(SplitArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2][2 * kTileBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQueryStageBytes];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
-  const int T = a.length, head = blockIdx.x % a.heads;
-  const int q0 = ((T + kOwned - 1) / kOwned - 1 - static_cast<int>(blockIdx.x) / a.heads) * kOwned;
-  const long long q_row = 1LL * a.heads * D, kv_row = 1LL * (a.heads / a.group) * D;
-  const uint16_t* k_base = a.k + head / a.group * D;
-  const uint16_t* v_base = a.v + head / a.group * D;
-  const int first_query = q0 + 32 * wave, query = first_query + n, query_load = min(query, T - 1);
-  const TileAccess at(wave, lane, kv_row);
-  const int tiles = (min(q0 + kOwned, T) - 1) / kRows + 1;
-  auto fill = [&](int tile) {
-    unsigned char* stage = lds[tile & 1];
-    const int k0 = tile * kRows;
-    tile_fill<D, kLoads>(stage, wave, k_base + k0 * kv_row, kv_row, k0, T, at.fill);
-    tile_fill<D, kLoads>(stage + kTileBytes, wave, v_base + k0 * kv_row, kv_row, k0, T, at.fill);
-  };
-  fill(0);
+  const QueryWave w(a, wave, n);
+  const int T = a.length, query = w.query, query_load = w.query_load, head = w.head;
+  const long long q_row = 1LL * a.heads * D;
+  const TileAccess at(wave, lane, 1LL * (a.heads / a.group) * D);
+  fill_query_stage(a, lds, 0, wave, head, at.fill);
   bf16x8 qf[KS], gf[3][KS];
   load_row_operand(a.q + query_load * q_row + head * D, h, qf);
 #pragma unroll
@@ -249,21 +330,36 @@ split_dq_kernel(SplitArgs a) {
   floatx16 dq[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) dq[db] = zero16();
-  for (int tile = 0; tile < tiles; ++tile) {
-    const int k0 = tile * kRows;
+  for (int step = 0; step < w.steps; ++step) {
+    const int k0 = (2 * step + w.parity) * kRows;
     stage_ready();
-    if (tile + 1 < tiles) fill(tile + 1);
-    if (k0 > first_query + 31) continue;
-    const unsigned char* k_tile = lds[tile & 1];
+    if (step + 1 < w.steps) fill_query_stage(a, lds, step + 1, wave, head, at.fill);
+    if (k0 > w.first_query + 31) continue;  // every key follows my queries
+    const unsigned char* k_tile = lds + (step & 1) * kQueryStageBytes + w.parity * 2 * kTileBytes;
     const unsigned char* v_tile = k_tile + kTileBytes;
     floatx16 s = zero16(), dp = zero16();
+    bf16x8 kf[3], vf[3];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      kf[i] = at.row(k_tile, i);
+      vf[i] = at.row(v_tile, i);
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      s = mfma32(row_operand(k_tile, at.row_read[ks]), qf[ks], s);
-      const bf16x8 vf = row_operand(v_tile, at.row_read[ks]);
+      if (ks + 2 < KS) {
+        kf[(ks + 2) % 3] = at.row(k_tile, ks + 2);
+        vf[(ks + 2) % 3] = at.row(v_tile, ks + 2);
+      }
+      fence_schedule();
+      s = mfma32(kf[ks % 3], qf[ks], s);
 #pragma unroll
-      for (int part = 2; part >= 0; --part) dp = mfma32(vf, gf[part][ks], dp);
+      for (int part = 2; part >= 0; --part) dp = mfma32(vf[ks % 3], gf[part][ks], dp);
+      fence_schedule();
     }
+    bf16x8 kt[3];
+    kt[0] = at.transposed(k_tile, 0, 0);
+    kt[1] = at.transposed(k_tile, 1, 0);
+    fence_schedule();
     const int limit = query_load - k0 - 4 * h;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -276,33 +372,46 @@ split_dq_kernel(SplitArgs a) {
       const Pieces ds = split_accumulator(s, s2);
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        const bf16x8 kt = tile_transposed_operand<D>(k_tile, at.tr_read[db], s2);
+        const int at_step = s2 * DB + db;
+        if (at_step + 2 < 2 * DB)
+          kt[(at_step + 2) % 3] = at.transposed(k_tile, (at_step + 2) % DB, (at_step + 2) / DB);
+        fence_schedule();
 #pragma unroll
-        for (int part = 2; part >= 0; --part) dq[db] = mfma32(kt, ds.part[part], dq[db]);
+        for (int part = 2; part >= 0; --part) dq[db] = mfma32(kt[at_step % 3], ds.part[part], dq[db]);
+        fence_schedule();
       }
     }
   }
-  if (query >= T) return;
+  __syncthreads();  // nobody reads the stages any more
+  if (w.parity == 1) store_upper(lds, w.half, lane, dq);
+  __syncthreads();
+  if (w.parity == 1 || query >= T) return;
   float* out = a.dq + query * q_row + head * D + 4 * h;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      const float4 u = load_upper(lds, w.half, lane, 4 * db + j);
       *reinterpret_cast<float4*>(out + 32 * db + 8 * j) =
-          make_float4(dq[db][4 * j] * a.scale, dq[db][4 * j + 1] * a.scale,
-                      dq[db][4 * j + 2] * a.scale, dq[db][4 * j + 3] * a.scale);
+          make_float4((dq[db][4 * j] + u.x) * a.scale, (dq[db][4 * j + 1] + u.y) * a.scale,
+                      (dq[db][4 * j + 2] + u.z) * a.scale, (dq[db][4 * j + 3] + u.w) * a.scale);
+    }
 }
 
+constexpr int kKeys = 128;  // of a workgroup of the key-owned kernel
 // Stage: Q tile, the three tiles of dC, and 64 floats each of the rows' maxima,
 // inverse normalizers and deltas.
 constexpr int kDkvStageBytes = 4 * kTileBytes + 1024;
 
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-split_dkv_kernel(SplitArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kDkvStageBytes];
+// dK or dV of 128 keys: both in one workgroup need 256 accumulator registers a
+// lane and leave none for requests ahead of their use.  Apart they repeat the
+// 16 of 112 products that make the scores, and there are twice as many
+// workgroups, of equal length, which short sequences need.
+template <bool VALUES>
+__device__ __forceinline__ void split_key_owned(const SplitArgs& a, unsigned char* lds, int head,
+                                                int k0) {
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
-  const int T = a.length, head = blockIdx.x % a.heads;
-  const int k0 = static_cast<int>(blockIdx.x) / a.heads * kOwned;
+  const int T = a.length;
   const long long q_row = 1LL * a.heads * D, kv_row = 1LL * (a.heads / a.group) * D;
   const int first_key = k0 + 32 * wave, key = first_key + n, key_load = min(key, T - 1);
   const TileAccess at(wave, lane, q_row);
@@ -322,12 +431,12 @@ split_dkv_kernel(SplitArgs a) {
     }
   };
   fill(first_tile);
-  bf16x8 kf[KS], vf[KS];
+  bf16x8 kf[KS], vf[VALUES ? 1 : KS];
   load_row_operand(a.k + key_load * kv_row + head / a.group * D, h, kf);
-  load_row_operand(a.v + key_load * kv_row + head / a.group * D, h, vf);
-  floatx16 dk[DB], dv[DB];
+  if constexpr (!VALUES) load_row_operand(a.v + key_load * kv_row + head / a.group * D, h, vf);
+  floatx16 acc[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = zero16();
+  for (int db = 0; db < DB; ++db) acc[db] = zero16();
   for (int tile = first_tile; tile < tiles; ++tile) {
     const int q0 = tile * kRows;
     stage_ready();
@@ -337,13 +446,52 @@ split_dkv_kernel(SplitArgs a) {
     const unsigned char* g_tile = q_tile + kTileBytes;
     const float* stats = reinterpret_cast<const float*>(q_tile + 4 * kTileBytes);
     floatx16 s = zero16(), dp = zero16();
+    if constexpr (VALUES) {
+      bf16x8 qa[2][4];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      s = mfma32(row_operand(q_tile, at.row_read[ks]), kf[ks], s);
+      for (int i = 0; i < 4; ++i) qa[0][i] = at.row(q_tile, i);
 #pragma unroll
-      for (int part = 2; part >= 0; --part)
-        dp = mfma32(row_operand(g_tile + part * kTileBytes, at.row_read[ks]), vf[ks], dp);
+      for (int g = 0; g < KS / 4; ++g) {
+        if (g + 1 < KS / 4)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) qa[(g + 1) % 2][i] = at.row(q_tile, 4 * (g + 1) + i);
+        fence_schedule();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s = mfma32(qa[g % 2][i], kf[4 * g + i], s);
+        fence_schedule();
+      }
+    } else {
+      bf16x8 qa[3], ga[3][3];
+      auto request = [&](int ks) {
+        qa[ks % 3] = at.row(q_tile, ks);
+#pragma unroll
+        for (int part = 0; part < 3; ++part)
+          ga[ks % 3][part] = at.row(g_tile + part * kTileBytes, ks);
+      };
+      request(0);
+      request(1);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (ks + 2 < KS) request(ks + 2);
+        fence_schedule();
+        s = mfma32(qa[ks % 3], kf[ks], s);
+#pragma unroll
+        for (int part = 2; part >= 0; --part) dp = mfma32(ga[ks % 3][part], vf[ks], dp);
+        fence_schedule();
+      }
     }
+    // transposed operands of step (s2, db): dC's pieces for dV, Q for dK
+    constexpr int kAhead = VALUES ? 1 : 2, kParts = VALUES ? 3 : 1;
+    bf16x8 t[kAhead + 1][kParts];
+    auto request_transposed = [&](int step) {
+#pragma unroll
+      for (int part = 0; part < kParts; ++part)
+        t[step % (kAhead + 1)][part] = at.transposed(VALUES ? g_tile + part * kTileBytes : q_tile,
+                                                     step % DB, step / DB);
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) request_transposed(i);
+    fence_schedule();
     // register i = (query q0 + 8(i/4) + 4h + i%4, key n)
     const int first = key - q0 - 4 * h, last = T - 1 - q0 - 4 * h;
 #pragma unroll
@@ -357,45 +505,52 @@ split_dkv_kernel(SplitArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 4 * j + e, local = 8 * j + e;
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale, -m[e]) * kLog2e) * r[e];
-        const bool hidden = (local < first) | (local > last);
-        s[i] = hidden ? 0.0f : p;
-        dp[i] = hidden ? 0.0f : p * (dp[i] - dl[e]);
+        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale, -m[e]) * kLog2e) * r[e];
+        if constexpr (!VALUES) p *= dp[i] - dl[e];
+        s[i] = ((local < first) | (local > last)) ? 0.0f : p;
       }
     }
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-      const Pieces p = split_accumulator(s, s2), ds = split_accumulator(dp, s2);
+      const Pieces p = split_accumulator(s, s2);
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        const bf16x8 qt = tile_transposed_operand<D>(q_tile, at.tr_read[db], s2);
+        const int step = s2 * DB + db;
+        if (step + kAhead < 2 * DB) request_transposed(step + kAhead);
+        fence_schedule();
 #pragma unroll
-        for (int part = 2; part >= 0; --part) dk[db] = mfma32(qt, ds.part[part], dk[db]);
+        for (int gp = kParts - 1; gp >= 0; --gp)
 #pragma unroll
-        for (int gp = 2; gp >= 0; --gp) {
-          const bf16x8 gt = tile_transposed_operand<D>(g_tile + gp * kTileBytes, at.tr_read[db], s2);
-#pragma unroll
-          for (int part = 2 - gp; part >= 0; --part) dv[db] = mfma32(gt, p.part[part], dv[db]);
-        }
+          for (int part = 2 - gp; part >= 0; --part)
+            acc[db] = mfma32(t[step % (kAhead + 1)][gp], p.part[part], acc[db]);
+        fence_schedule();
       }
     }
   }
   if (key >= T) return;
-  const long long out = key * q_row + head * D + 4 * h;
+  const float factor = VALUES ? 1.0f : a.scale;
+  float* out = (VALUES ? a.dv : a.dk) + key * q_row + head * D + 4 * h;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      *reinterpret_cast<float4*>(a.dk + out + 32 * db + 8 * j) =
-          make_float4(dk[db][4 * j] * a.scale, dk[db][4 * j + 1] * a.scale,
-                      dk[db][4 * j + 2] * a.scale, dk[db][4 * j + 3] * a.scale);
-      *reinterpret_cast<float4*>(a.dv + out + 32 * db + 8 * j) =
-          make_float4(dv[db][4 * j], dv[db][4 * j + 1], dv[db][4 * j + 2], dv[db][4 * j + 3]);
-    }
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<float4*>(out + 32 * db + 8 * j) =
+          make_float4(acc[db][4 * j] * factor, acc[db][4 * j + 1] * factor,
+                      acc[db][4 * j + 2] * factor, acc[db][4 * j + 3] * factor);
 }
 
-unsigned tile_grid(const SplitArgs& a) {
-  return static_cast<unsigned>((a.length + kOwned - 1) / kOwned) * a.heads;
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+split_dkv_kernel(SplitArgs a) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kDkvStageBytes];
+  const int unit = blockIdx.x % (2 * a.heads), k0 = static_cast<int>(blockIdx.x) / (2 * a.heads) * kKeys;
+  if (unit < a.heads)
+    split_key_owned<true>(a, lds, unit, k0);
+  else
+    split_key_owned<false>(a, lds, unit - a.heads, k0);
+}
+
+unsigned tile_grid(const SplitArgs& a, int owned) {
+  return static_cast<unsigned>((a.length + owned - 1) / owned) * a.heads;
 }
 
 }  // namespace
@@ -406,7 +561,7 @@ bool split_attention_supported(int length, int heads, int head_dim) {
 }
 
 int launch_split_forward(hipStream_t stream, const SplitArgs& a) {
-  split_forward_kernel<<<tile_grid(a), kThreads, 0, stream>>>(a);
+  split_forward_kernel<<<tile_grid(a, kQueries), kThreads, 0, stream>>>(a);
   return launch_status();
 }
 
@@ -423,10 +578,10 @@ int launch_split_gate(hipStream_t stream, const SplitArgs& a, const void* qg, co
 }
 
 int launch_split_backward(hipStream_t stream, const SplitArgs& a) {
-  if (kernel_enabled(kQueryKernel)) split_dq_kernel<<<tile_grid(a), kThreads, 0, stream>>>(a);
+  if (kernel_enabled(kQueryKernel)) split_dq_kernel<<<tile_grid(a, kQueries), kThreads, 0, stream>>>(a);
   const int status = launch_status();
   if (status != 0) return status;
-  if (kernel_enabled(kMainKernel)) split_dkv_kernel<<<tile_grid(a), kThreads, 0, stream>>>(a);
+  if (kernel_enabled(kMainKernel)) split_dkv_kernel<<<2 * tile_grid(a, kKeys), kThreads, 0, stream>>>(a);
   return launch_status();
 }
 
