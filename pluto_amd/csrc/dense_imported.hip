@@ -8,8 +8,9 @@
 // FP8 E4M3 with FP32 scales [ceil(out/128), ceil(in/128)] times one bf16
 // token.  Byte-bound: every weight is read once.  A wave owns four output
 // rows and reads them in 16-byte pieces (whenever rows start 16-byte aligned),
-// the token comes from the FP32 copy the first kernel leaves in the workspace;
-// all arithmetic is FP32, the 64 lane sums are added by a butterfly.
+// a single token is prepared by the workgroups themselves, several come from the
+// FP32 copy a kernel of their own leaves in the workspace; all arithmetic is
+// FP32, the 64 lane sums are added by a butterfly.
 #include <algorithm>
 
 #include "dense.h"
@@ -33,17 +34,33 @@ __device__ inline float fp8_value(uint32_t bits) {
   return (bits & 0x80u) ? -magnitude : magnitude;
 }
 
-// The FP8 E4M3 value nearest to v (ties to even, saturating at +-448), as a
-// float: what element_cast to FP8 and back gives (fully_connected.cc:86-87).
-__device__ inline float fp8_round(float v) {
-  const float a = fabsf(v);
-  if (a >= 448.0f) return copysignf(448.0f, v);
-  int exponent = static_cast<int>((__float_as_uint(a) >> 23) & 255u) - 127;  // floor(log2 a)
-  if (exponent < -6) exponent = -6;                                          // subnormal grid
-  const float step = __uint_as_float(static_cast<uint32_t>(exponent - 3 + 127) << 23);
-  const float rounded = __builtin_rintf(a / step) * step;  // a / step is exact
-  return copysignf(fminf(rounded, 448.0f), v);
-}
+// FP8 quantization of a group of 128 token values (fully_connected.cc:70-88):
+// scale = largest / 448, code = fp8(v / max(scale, 1e-12)), value = code * scale
+// (only the divisor is floored).  The division is a multiplication by the
+// group's reciprocal with one correction step, which rounds as the division
+// does, and the rounding is the hardware conversion: six instructions a value
+// where a divide and a rounding by parts took sixty, 9 us of a one-token
+// projection whose workgroups each prepare the token.
+struct GroupQuantizer {
+  float scale, divisor, inverse;
+  __device__ explicit GroupQuantizer(float largest) {
+    scale = largest / 448.0f;
+    divisor = fmaxf(scale, 1e-12f);
+    inverse = 1.0f / divisor;
+  }
+  __device__ float quotient(float v) const {
+    const float q = v * inverse;
+    const float corrected = __builtin_fmaf(__builtin_fmaf(-q, divisor, v), inverse, q);
+    return fminf(fmaxf(corrected, -448.0f), 448.0f);
+  }
+  // The FP8 values (unscaled) nearest to the two quotients, as floats.
+  __device__ void round(float first, float second, float& a, float& b) const {
+    const int codes = __builtin_amdgcn_cvt_pk_fp8_f32(quotient(first), quotient(second), 0, false);
+    const auto values = __builtin_amdgcn_cvt_pk_f32_fp8(codes, false);
+    a = values[0];
+    b = values[1];
+  }
+};
 
 // token[i] = float(x[i]), for FP8 storage quantized per group of 128.
 template <bool FP8>
@@ -60,18 +77,26 @@ imported_token_kernel(const uint16_t* x, int n, float* token) {
     const float mine = wave_max(fabsf(v));
     if (threadIdx.x % 64 == 0) largest[threadIdx.x / 64] = mine;
     __syncthreads();
-    const float scale = fmaxf(largest[0], largest[1]) / 448.0f;
-    // only the divisor is floored: the result keeps the group's own scale
-    if (i < n) token[i] = fp8_round(v / fmaxf(scale, 1e-12f)) * scale;
+    const GroupQuantizer quantizer(fmaxf(largest[0], largest[1]));
+    float value, unused;
+    quantizer.round(v, 0.0f, value, unused);
+    if (i < n) token[i] = value * quantizer.scale;
   }
 }
 
+// Several matrices applied to the same tokens in one launch: workgroup b works on
+// matrix i with first_block[i] <= b < first_block[i + 1].
+constexpr int kManyMax = 8;
 struct MatVecArgs {
-  const void* weights = nullptr;
-  const float* scales = nullptr;  // FP8 only
-  const float* token = nullptr;  // [tokens, cols]
-  uint16_t* out = nullptr;       // [tokens, rows]
-  int cols = 0, rows = 0;
+  const void* weights[kManyMax];
+  const float* scales[kManyMax];  // FP8 only
+  uint16_t* out[kManyMax];        // [tokens, rows]
+  int rows[kManyMax];
+  int first_block[kManyMax + 1];
+  int matrices = 0;
+  const uint16_t* input = nullptr;  // one bf16 token, when the kernel prepares it itself
+  const float* token = nullptr;     // else [tokens, cols], prepared
+  int cols = 0;
 };
 
 typedef float floatx2 __attribute__((ext_vector_type(2)));
@@ -85,102 +110,218 @@ __device__ inline void fp8_word(uint32_t word, float* out) {
 
 constexpr int kRowsPerWave = 4;
 
+// The matrix a workgroup works on.
+struct MatVecTarget {
+  const unsigned char* weights;
+  const float* scales;
+  uint16_t* out;
+  int rows, block;
+};
+__device__ inline MatVecTarget matvec_target(const MatVecArgs& a) {
+  int which = 0;
+  while (which + 1 < a.matrices && static_cast<int>(blockIdx.x) >= a.first_block[which + 1]) ++which;
+  return {static_cast<const unsigned char*>(a.weights[which]), a.scales[which], a.out[which],
+          a.rows[which], static_cast<int>(blockIdx.x) - a.first_block[which]};
+}
+
 // STORAGE: 0 bf16, 1 fp32, 2 FP8 E4M3.  A wave owns four consecutive output
-// rows: a lane takes 16-byte pieces of them at the same columns, so the token
-// values of a piece are loaded once for four rows and four weight loads are
-// in flight per lane.  TOKENS tokens share one pass over the weights; each
-// token's sum is formed exactly as in the one-token kernel.
-template <int STORAGE, int TOKENS>
-__global__ void __launch_bounds__(256) imported_matvec_kernel(MatVecArgs a) {
+// rows, a lane takes 16-byte pieces of them at the same columns: pieces lane,
+// lane + 64, ...  BATCH pieces of all four rows are requested before the first is
+// used: a workgroup's whole share of the weights is a few tens of KiB and the
+// grid of a projection fits the chip at once, so what matters is how much of it
+// travels together.  TOKENS tokens share one pass over the weights; each token's
+// sum is formed in the order of the one-token kernel.  PREPARE (one token): the
+// workgroup converts (FP8: quantizes) the token itself while its first weights
+// travel, instead of reading what a launch of its own left in memory; in LDS the
+// quarters of a piece lie apart, so that the lanes read consecutive 16 bytes.
+// 5120 -> 12288 + 1024 + 1024 in FP8, one token: 41 us as a token and a mat-vec
+// launch a matrix, 17 us as one launch.
+template <int STORAGE, int TOKENS, int STEPS, bool PREPARE>
+__global__ void __launch_bounds__(256, TOKENS > 1 ? 1 : PREPARE && STORAGE == 2 && STEPS < 8 ? 4 : 3)
+imported_matvec_kernel(MatVecArgs a) {
   constexpr int kElementBytes = STORAGE == 0 ? 2 : (STORAGE == 1 ? 4 : 1);
   constexpr int kPiece = 16 / kElementBytes;  // elements per 16-byte load
-  constexpr int R = kRowsPerWave;
+  constexpr int kQuads = kPiece / 4;
+  constexpr int R = kRowsPerWave, BATCH = STEPS < 4 ? STEPS : 4;
+  extern __shared__ float4 token_lds[];  // PREPARE: [kQuads][pieces]
   const int lane = threadIdx.x % 64;
-  const int row0 = (blockIdx.x * 4 + threadIdx.x / 64) * R;
-  if (row0 >= a.rows) return;
-  const int scale_cols = (a.cols + kGroup - 1) / kGroup;
-  size_t row_start[R];
-  const float* scale_row[R];
+  const MatVecTarget m = matvec_target(a);
+  const int row0 = (m.block * 4 + threadIdx.x / 64) * R;
+  const int pieces = a.cols / kPiece;
+  const unsigned char* row_start[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int row = min(row0 + r, a.rows - 1);  // rows past the end repeat the last one
-    row_start[r] = static_cast<size_t>(row) * a.cols;
-    scale_row[r] =
-        STORAGE == 2 ? a.scales + static_cast<size_t>(row / kGroup) * scale_cols : nullptr;
+  for (int r = 0; r < R; ++r)  // rows past the end repeat the last one
+    row_start[r] = m.weights + static_cast<size_t>(min(row0 + r, m.rows - 1)) * a.cols * kElementBytes;
+  // the four rows lie in one 128-row block of scales
+  const float* scale_row =
+      STORAGE == 2 ? m.scales + static_cast<size_t>(min(row0, m.rows - 1) / kGroup) *
+                                    ((a.cols + kGroup - 1) / kGroup)
+                   : nullptr;
+  uint4 raw[BATCH][R];
+  float scale[BATCH];
+  auto request = [&](int b, int first) {
+    const int p = min(first + lane, pieces - 1);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      raw[b][r] = *reinterpret_cast<const uint4*>(row_start[r] + static_cast<size_t>(p) * 16);
+    scale[b] = STORAGE == 2 ? scale_row[p * kPiece / kGroup] : 1.0f;
+  };
+#pragma unroll
+  for (int b = 0; b < BATCH; ++b) request(b, 64 * b);
+  if constexpr (PREPARE) {
+    static_assert(TOKENS == 1);
+    for (int c = threadIdx.x * 8; c < (a.cols + 127) / 128 * 128; c += 2048) {
+      // sixteen lanes hold a group of 128
+      uint4 bits = make_uint4(0, 0, 0, 0);
+      if (c < a.cols) bits = *reinterpret_cast<const uint4*>(a.input + c);
+      const uint32_t words[4] = {bits.x, bits.y, bits.z, bits.w};
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        v[e] = __uint_as_float(e % 2 ? words[e / 2] & 0xffff0000u : words[e / 2] << 16);
+      if constexpr (STORAGE == 2) {
+        float largest = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) largest = fmaxf(largest, fabsf(v[e]));
+#pragma unroll
+        for (int offset = 8; offset > 0; offset >>= 1)
+          largest = fmaxf(largest, __shfl_xor(largest, offset, 64));
+        const GroupQuantizer quantizer(largest);
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          quantizer.round(v[e], v[e + 1], v[e], v[e + 1]);
+          v[e] *= quantizer.scale;
+          v[e + 1] *= quantizer.scale;
+        }
+      }
+      if (c < a.cols) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int quad = c / 4 + q;  // of the whole token
+          token_lds[quad % kQuads * pieces + quad / kQuads] =
+              make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        }
+      }
+    }
+    __syncthreads();
   }
+  if (row0 >= m.rows) return;
   float sum[TOKENS][R];
 #pragma unroll
   for (int t = 0; t < TOKENS; ++t)
 #pragma unroll
     for (int r = 0; r < R; ++r) sum[t][r] = 0.0f;
-  auto element = [&](int r, int c) {
-    const size_t i = row_start[r] + c;
-    if constexpr (STORAGE == 0)
-      return bf16_bits_to_float(static_cast<const uint16_t*>(a.weights)[i]);
-    else if constexpr (STORAGE == 1)
-      return static_cast<const float*>(a.weights)[i];
-    else
-      return fp8_value(static_cast<const uint8_t*>(a.weights)[i]) * scale_row[r][c / kGroup];
-  };
-  int done = 0;
-  if ((static_cast<size_t>(a.cols) * kElementBytes) % 16 == 0) {
-    // every row starts on a 16-byte boundary (the buffer itself is at least
-    // 256-byte aligned): whole pieces, a piece never straddles a scale block
-    const unsigned char* base = static_cast<const unsigned char*>(a.weights);
-    const int pieces = a.cols / kPiece;
-    for (int p = lane; p < pieces; p += 64) {
-      const int c0 = p * kPiece;
-      uint4 raw[R];
+  for (int first = 0; first < pieces; first += 64 * STEPS) {
+    if (first > 0) {
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        raw[r] = *reinterpret_cast<const uint4*>(base + row_start[r] * kElementBytes +
-                                                 static_cast<size_t>(p) * 16);
-      // the rows' values of this piece, decoded once for all tokens
-      float w[R][kPiece];
+      for (int b = 0; b < BATCH; ++b) request(b, first + 64 * b);
+    }
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const uint32_t words[4] = {raw[r].x, raw[r].y, raw[r].z, raw[r].w};
+    for (int step = 0; step < STEPS; ++step) {
+      const int b = step % BATCH;
+      // lanes past the end repeat the last piece and count it as nothing
+      const bool exists = first + 64 * step + lane < pieces;
+      const int p = exists ? first + 64 * step + lane : pieces - 1;
+      auto decode = [&](int r, float (&w)[kPiece]) {
+        const uint32_t words[4] = {raw[b][r].x, raw[b][r].y, raw[b][r].z, raw[b][r].w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           if constexpr (STORAGE == 0) {
-            w[r][2 * k] = __uint_as_float(words[k] << 16);
-            w[r][2 * k + 1] = __uint_as_float(words[k] & 0xffff0000u);
+            w[2 * k] = __uint_as_float(words[k] << 16);
+            w[2 * k + 1] = __uint_as_float(words[k] & 0xffff0000u);
           } else if constexpr (STORAGE == 1) {
-            w[r][k] = __uint_as_float(words[k]);
+            w[k] = __uint_as_float(words[k]);
           } else {
-            fp8_word(words[k], &w[r][4 * k]);
+            fp8_word(words[k], &w[4 * k]);
           }
         }
-      }
+      };
+      auto token_piece = [&](int t, float (&x)[kPiece]) {
 #pragma unroll
-      for (int t = 0; t < TOKENS; ++t) {
-        float x[kPiece];
-#pragma unroll
-        for (int q = 0; q < kPiece / 4; ++q) {
-          const float4 v = *reinterpret_cast<const float4*>(
-              a.token + static_cast<size_t>(t) * a.cols + c0 + 4 * q);
+        for (int q = 0; q < kQuads; ++q) {
+          const float4 v = PREPARE ? token_lds[q * pieces + p]
+                                   : *reinterpret_cast<const float4*>(
+                                         a.token + static_cast<size_t>(t) * a.cols + p * kPiece + 4 * q);
           x[4 * q] = v.x, x[4 * q + 1] = v.y, x[4 * q + 2] = v.z, x[4 * q + 3] = v.w;
         }
+      };
+      auto add = [&](int t, int r, const float (&w)[kPiece], const float (&x)[kPiece]) {
+        if constexpr (STORAGE == 2) {
+          float part = 0.0f;
+#pragma unroll
+          for (int e = 0; e < kPiece; ++e) part += w[e] * x[e];
+          const float total = sum[t][r] + part * scale[b];
+          sum[t][r] = exists ? total : sum[t][r];
+        } else {
+          float total = sum[t][r];
+#pragma unroll
+          for (int e = 0; e < kPiece; ++e) total += w[e] * x[e];
+          sum[t][r] = exists ? total : sum[t][r];
+        }
+      };
+      if constexpr (TOKENS == 1) {
+        float x[kPiece];
+        token_piece(0, x);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-          if constexpr (STORAGE == 2) {
-            float part = 0.0f;
+          float w[kPiece];
+          decode(r, w);
+          add(0, r, w, x);
+        }
+      } else {
+        // decoded once for all tokens
+        float w[R][kPiece];
 #pragma unroll
-            for (int e = 0; e < kPiece; ++e) part += w[r][e] * x[e];
-            sum[t][r] += part * scale_row[r][c0 / kGroup];
-          } else {
+        for (int r = 0; r < R; ++r) decode(r, w[r]);
 #pragma unroll
-            for (int e = 0; e < kPiece; ++e) sum[t][r] += w[r][e] * x[e];
-          }
+        for (int t = 0; t < TOKENS; ++t) {
+          float x[kPiece];
+          token_piece(t, x);
+#pragma unroll
+          for (int r = 0; r < R; ++r) add(t, r, w[r], x);
         }
       }
+      if (step + BATCH < STEPS) request(b, first + 64 * (step + BATCH));
     }
-    done = pieces * kPiece;
   }
-  for (int c = done + lane; c < a.cols; c += 64) {
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float total = wave_sum(sum[t][r]);
+      if (lane == 0 && row0 + r < m.rows)
+        m.out[static_cast<size_t>(t) * m.rows + row0 + r] = float_to_bf16_bits(total);
+    }
+}
+
+// Rows that do not start 16-byte aligned: one element a lane.
+template <int STORAGE, int TOKENS>
+__global__ void __launch_bounds__(256) imported_matvec_ragged_kernel(MatVecArgs a) {
+  constexpr int R = kRowsPerWave;
+  const int lane = threadIdx.x % 64;
+  const MatVecTarget m = matvec_target(a);
+  const int row0 = (m.block * 4 + threadIdx.x / 64) * R;
+  if (row0 >= m.rows) return;
+  const int scale_cols = (a.cols + kGroup - 1) / kGroup;
+  float sum[TOKENS][R];
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t)
+#pragma unroll
+    for (int r = 0; r < R; ++r) sum[t][r] = 0.0f;
+  for (int c = lane; c < a.cols; c += 64) {
     float value[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) value[r] = element(r, c);
+    for (int r = 0; r < R; ++r) {
+      const int row = min(row0 + r, m.rows - 1);  // rows past the end repeat the last one
+      const size_t i = static_cast<size_t>(row) * a.cols + c;
+      if constexpr (STORAGE == 0)
+        value[r] = bf16_bits_to_float(reinterpret_cast<const uint16_t*>(m.weights)[i]);
+      else if constexpr (STORAGE == 1)
+        value[r] = reinterpret_cast<const float*>(m.weights)[i];
+      else
+        value[r] = fp8_value(m.weights[i]) *
+                   m.scales[static_cast<size_t>(row / kGroup) * scale_cols + c / kGroup];
+    }
 #pragma unroll
     for (int t = 0; t < TOKENS; ++t) {
       const float x = a.token[static_cast<size_t>(t) * a.cols + c];
@@ -193,8 +334,8 @@ __global__ void __launch_bounds__(256) imported_matvec_kernel(MatVecArgs a) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const float total = wave_sum(sum[t][r]);
-      if (lane == 0 && row0 + r < a.rows)
-        a.out[static_cast<size_t>(t) * a.rows + row0 + r] = float_to_bf16_bits(total);
+      if (lane == 0 && row0 + r < m.rows)
+        m.out[static_cast<size_t>(t) * m.rows + row0 + r] = float_to_bf16_bits(total);
     }
 }
 
@@ -228,13 +369,15 @@ imported_token_fp8_kernel(const uint16_t* x, int n, uint16_t* values, float* sca
   const float mine = wave_max(fabsf(v));
   if (threadIdx.x % 64 == 0) largest[threadIdx.x / 64] = mine;
   __syncthreads();
-  const float scale = fmaxf(largest[0], largest[1]) / 448.0f;
+  const GroupQuantizer quantizer(fmaxf(largest[0], largest[1]));
+  float value, unused;
+  quantizer.round(v, 0.0f, value, unused);
   const size_t pass = token / 32;
   const int lane = token % 32 + 32 * (c / 64), step = (c % 64) / 8;
   if (i < n)
     values[(((pass * gridDim.x + block) * 8 + step) * 64 + lane) * 8 + c % 8] =
-        float_to_bf16_bits(fp8_round(v / fmaxf(scale, 1e-12f)));
-  if (threadIdx.x == 0) scales[static_cast<size_t>(token) * gridDim.x + block] = scale;
+        float_to_bf16_bits(value);
+  if (threadIdx.x == 0) scales[static_cast<size_t>(token) * gridDim.x + block] = quantizer.scale;
 }
 
 struct TileArgs {
@@ -254,9 +397,7 @@ __device__ inline uint32_t fp8_pair_to_bf16(uint32_t word) {
 
 constexpr int kTileWaves = 8;  // waves that split a tile's contraction
 
-// Several matrices applied to the same tokens in one launch: workgroup b works
-// on matrix i with first_block[i] <= b < first_block[i + 1], tile b - first_block[i].
-constexpr int kManyMax = 8;
+// Several matrices in one launch, numbered as in MatVecArgs.
 struct TileManyArgs {
   const void* weights[kManyMax];
   const float* weight_scales[kManyMax];
@@ -380,13 +521,7 @@ __device__ __forceinline__ void imported_tile(const TileArgs& a, int tile,
 }
 
 template <bool FP8, int AHEAD = 1>
-__global__ void __launch_bounds__(64 * kTileWaves) imported_tile_kernel(TileArgs a) {
-  __shared__ float partial[kTileWaves - 1][16][64];
-  imported_tile<FP8, AHEAD>(a, blockIdx.x, partial);
-}
-
-template <bool FP8, int AHEAD = 1>
-__global__ void __launch_bounds__(64 * kTileWaves) imported_tile_many_kernel(TileManyArgs m) {
+__global__ void __launch_bounds__(64 * kTileWaves) imported_tile_kernel(TileManyArgs m) {
   __shared__ float partial[kTileWaves - 1][16][64];
   int which = 0;
   while (which + 1 < m.matrices && static_cast<int>(blockIdx.x) >= m.first_block[which + 1])
@@ -403,42 +538,19 @@ __global__ void __launch_bounds__(64 * kTileWaves) imported_tile_many_kernel(Til
   imported_tile<FP8, AHEAD>(a, blockIdx.x - m.first_block[which], partial);
 }
 
-template <int AHEAD>
-void launch_fp8_tiles_ahead(hipStream_t s, const TileArgs& t, int blocks) {
-  imported_tile_kernel<true, AHEAD><<<blocks, 64 * kTileWaves, 0, s>>>(t);
-}
-
 // Picks AHEAD = blocks a wave owns, up to eight.
-void launch_fp8_tiles(hipStream_t s, const TileArgs& t, int blocks) {
+void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t, int blocks) {
   const int groups = t.cols / kGroup;
+  auto launch = [&](auto kernel) { kernel<<<blocks, 64 * kTileWaves, 0, s>>>(t); };
   switch (std::min(8, (groups + kTileWaves - 1) / kTileWaves)) {
-    case 1: return launch_fp8_tiles_ahead<1>(s, t, blocks);
-    case 2: return launch_fp8_tiles_ahead<2>(s, t, blocks);
-    case 3: return launch_fp8_tiles_ahead<3>(s, t, blocks);
-    case 4: return launch_fp8_tiles_ahead<4>(s, t, blocks);
-    case 5: return launch_fp8_tiles_ahead<5>(s, t, blocks);
-    case 6: return launch_fp8_tiles_ahead<6>(s, t, blocks);
-    case 7: return launch_fp8_tiles_ahead<7>(s, t, blocks);
-    default: return launch_fp8_tiles_ahead<8>(s, t, blocks);
-  }
-}
-
-template <int AHEAD>
-void launch_fp8_tiles_many_ahead(hipStream_t s, const TileManyArgs& t, int blocks) {
-  imported_tile_many_kernel<true, AHEAD><<<blocks, 64 * kTileWaves, 0, s>>>(t);
-}
-
-void launch_fp8_tiles_many(hipStream_t s, const TileManyArgs& t, int blocks) {
-  const int groups = t.cols / kGroup;
-  switch (std::min(8, (groups + kTileWaves - 1) / kTileWaves)) {
-    case 1: return launch_fp8_tiles_many_ahead<1>(s, t, blocks);
-    case 2: return launch_fp8_tiles_many_ahead<2>(s, t, blocks);
-    case 3: return launch_fp8_tiles_many_ahead<3>(s, t, blocks);
-    case 4: return launch_fp8_tiles_many_ahead<4>(s, t, blocks);
-    case 5: return launch_fp8_tiles_many_ahead<5>(s, t, blocks);
-    case 6: return launch_fp8_tiles_many_ahead<6>(s, t, blocks);
-    case 7: return launch_fp8_tiles_many_ahead<7>(s, t, blocks);
-    default: return launch_fp8_tiles_many_ahead<8>(s, t, blocks);
+    case 1: return launch(imported_tile_kernel<true, 1>);
+    case 2: return launch(imported_tile_kernel<true, 2>);
+    case 3: return launch(imported_tile_kernel<true, 3>);
+    case 4: return launch(imported_tile_kernel<true, 4>);
+    case 5: return launch(imported_tile_kernel<true, 5>);
+    case 6: return launch(imported_tile_kernel<true, 6>);
+    case 7: return launch(imported_tile_kernel<true, 7>);
+    default: return launch(imported_tile_kernel<true, 8>);
   }
 }
 
@@ -448,25 +560,67 @@ bool tile_path(int storage, int tokens, int input_dim) {
   return storage != PLUTO_HIP_MATRIX_F32 && tokens > 8 && input_dim % kGroup == 0;
 }
 
+template <int STORAGE, int TOKENS, bool PREPARE>
+void launch_matvec_batches(hipStream_t s, const MatVecArgs& a, unsigned blocks) {
+  constexpr int kPiece = STORAGE == 0 ? 8 : STORAGE == 1 ? 4 : 16;
+  const size_t lds = PREPARE ? static_cast<size_t>(a.cols) * 4 : 0;
+  auto launch = [&](auto kernel) { kernel<<<blocks, 256, lds, s>>>(a); };
+  const int steps = (a.cols / kPiece + 63) / 64;  // pieces a lane takes
+  switch ((steps + (steps + 7) / 8 - 1) / ((steps + 7) / 8)) {
+    case 1: return launch(imported_matvec_kernel<STORAGE, TOKENS, 1, PREPARE>);
+    case 2: return launch(imported_matvec_kernel<STORAGE, TOKENS, 2, PREPARE>);
+    case 3: return launch(imported_matvec_kernel<STORAGE, TOKENS, 3, PREPARE>);
+    case 4: return launch(imported_matvec_kernel<STORAGE, TOKENS, 4, PREPARE>);
+    case 5: return launch(imported_matvec_kernel<STORAGE, TOKENS, 5, PREPARE>);
+    case 6: return launch(imported_matvec_kernel<STORAGE, TOKENS, 6, PREPARE>);
+    case 7: return launch(imported_matvec_kernel<STORAGE, TOKENS, 7, PREPARE>);
+    default: return launch(imported_matvec_kernel<STORAGE, TOKENS, 8, PREPARE>);
+  }
+}
+
+// The vector path: up to eight tokens share a pass over the weights.  `token`
+// holds the prepared tokens unless a.input is set.
 template <int STORAGE>
 void launch_matvec(hipStream_t s, MatVecArgs a, int tokens) {
-  const unsigned blocks =
-      static_cast<unsigned>((a.rows + 4 * kRowsPerWave - 1) / (4 * kRowsPerWave));
-  // up to eight tokens share a pass over the weights
+  constexpr int kElementBytes = STORAGE == 0 ? 2 : STORAGE == 1 ? 4 : 1;
+  const unsigned blocks = static_cast<unsigned>(a.first_block[a.matrices]);
+  const bool whole = static_cast<size_t>(a.cols) * kElementBytes % 16 == 0;
   while (tokens > 0) {
     const int now = tokens >= 8 ? 8 : (tokens >= 4 ? 4 : (tokens >= 2 ? 2 : 1));
-    if (now == 8)
-      imported_matvec_kernel<STORAGE, 8><<<blocks, 256, 0, s>>>(a);
-    else if (now == 4)
-      imported_matvec_kernel<STORAGE, 4><<<blocks, 256, 0, s>>>(a);
-    else if (now == 2)
-      imported_matvec_kernel<STORAGE, 2><<<blocks, 256, 0, s>>>(a);
-    else
-      imported_matvec_kernel<STORAGE, 1><<<blocks, 256, 0, s>>>(a);
+    if (!whole) {
+      if (now == 8)
+        imported_matvec_ragged_kernel<STORAGE, 8><<<blocks, 256, 0, s>>>(a);
+      else if (now == 4)
+        imported_matvec_ragged_kernel<STORAGE, 4><<<blocks, 256, 0, s>>>(a);
+      else if (now == 2)
+        imported_matvec_ragged_kernel<STORAGE, 2><<<blocks, 256, 0, s>>>(a);
+      else
+        imported_matvec_ragged_kernel<STORAGE, 1><<<blocks, 256, 0, s>>>(a);
+    } else if (a.input != nullptr) {
+      launch_matvec_batches<STORAGE, 1, true>(s, a, blocks);
+    } else if (now == 8) {
+      launch_matvec_batches<STORAGE, 8, false>(s, a, blocks);
+    } else if (now == 4) {
+      launch_matvec_batches<STORAGE, 4, false>(s, a, blocks);
+    } else if (now == 2) {
+      launch_matvec_batches<STORAGE, 2, false>(s, a, blocks);
+    } else {
+      launch_matvec_batches<STORAGE, 1, false>(s, a, blocks);
+    }
     a.token += static_cast<size_t>(now) * a.cols;
-    a.out += static_cast<size_t>(now) * a.rows;
+    for (int i = 0; i < a.matrices; ++i) a.out[i] += static_cast<size_t>(now) * a.rows[i];
     tokens -= now;
   }
+}
+
+// One token of up to 16384 columns (64 KiB as FP32 in LDS) is prepared by the
+// workgroups that use it.
+bool matvec_prepares(int storage, const void* input, int tokens, int input_dim) {
+  const int element_bytes =
+      storage == PLUTO_HIP_MATRIX_BF16 ? 2 : storage == PLUTO_HIP_MATRIX_F32 ? 4 : 1;
+  return tokens == 1 && input_dim <= 16384 && input_dim % 8 == 0 &&
+         static_cast<size_t>(input_dim) * element_bytes % 16 == 0 &&
+         (reinterpret_cast<uintptr_t>(input) & 15u) == 0;
 }
 
 }  // namespace
@@ -487,90 +641,57 @@ size_t dense_imported_workspace_bytes(int tokens, int input_dim) {
   return std::max(vector_path, tile_path) + 256;
 }
 
-int launch_dense_imported_forward(hipStream_t s, int storage, const void* weights,
-                                  const float* scales, const void* input, int tokens,
-                                  int input_dim, int output_dim, void* output, void* workspace) {
+// Matrices of one storage kind and input width applied to the same tokens: the
+// tokens are prepared once, and every pass (up to 8 tokens on the vector path,
+// 32 on the matrix cores) is one launch over all matrices.
+int launch_dense_imported_forward(hipStream_t s, int storage, int matrices,
+                                  const void* const* weights, const float* const* scales,
+                                  const int* output_dims, const void* input, int tokens,
+                                  int input_dim, void* const* outputs, void* workspace) {
+  const bool fp8 = storage == PLUTO_HIP_MATRIX_FP8_E4M3;
   const dim3 groups(static_cast<unsigned>((input_dim + kGroup - 1) / kGroup),
                     static_cast<unsigned>(tokens));
-  if (tile_path(storage, tokens, input_dim)) {
-    const bool fp8 = storage == PLUTO_HIP_MATRIX_FP8_E4M3;
-    TileArgs t;
-    t.weights = weights;
-    t.weight_scales = scales;
-    t.tokens = static_cast<const uint16_t*>(input);
-    t.cols = input_dim;
-    t.rows = output_dim;
-    if (fp8) {
-      uint16_t* values = static_cast<uint16_t*>(workspace);
-      float* token_scales = reinterpret_cast<float*>(static_cast<char*>(workspace) +
-                                                     tile_values_bytes(tokens, input_dim));
-      imported_token_fp8_kernel<<<groups, kGroup, 0, s>>>(static_cast<const uint16_t*>(input),
-                                                          input_dim, values, token_scales);
-      t.tokens = values;
-      t.token_scales = token_scales;
+  auto fill = [&](auto& args, auto& scale_list, int rows_per_block) {
+    args.matrices = matrices;
+    args.cols = input_dim;
+    args.first_block[0] = 0;
+    for (int i = 0; i < kManyMax; ++i) {
+      const bool used = i < matrices;
+      args.weights[i] = used ? weights[i] : nullptr;
+      scale_list[i] = used && fp8 ? scales[i] : nullptr;
+      args.out[i] = used ? static_cast<uint16_t*>(outputs[i]) : nullptr;
+      args.rows[i] = used ? output_dims[i] : 0;
+      args.first_block[i + 1] =
+          args.first_block[i] + (used ? (output_dims[i] + rows_per_block - 1) / rows_per_block : 0);
     }
-    t.out = static_cast<uint16_t*>(output);
-    const unsigned blocks = static_cast<unsigned>((output_dim + 31) / 32);
-    for (int done = 0; done < tokens; done += 32) {
-      t.count = tokens - done < 32 ? tokens - done : 32;
+  };
+  if (!tile_path(storage, tokens, input_dim)) {
+    MatVecArgs a;
+    fill(a, a.scales, 4 * kRowsPerWave);
+    if (matvec_prepares(storage, input, tokens, input_dim)) {
+      a.input = static_cast<const uint16_t*>(input);
+    } else {
+      float* token = static_cast<float*>(workspace);
       if (fp8)
-        launch_fp8_tiles(s, t, blocks);
+        imported_token_kernel<true><<<groups, kGroup, 0, s>>>(static_cast<const uint16_t*>(input),
+                                                              input_dim, token);
       else
-        imported_tile_kernel<false><<<blocks, 64 * kTileWaves, 0, s>>>(t);
-      t.tokens += static_cast<size_t>(32) * input_dim;
-      if (fp8) t.token_scales += static_cast<size_t>(32) * (input_dim / kGroup);
-      t.out += static_cast<size_t>(32) * output_dim;
+        imported_token_kernel<false><<<groups, kGroup, 0, s>>>(static_cast<const uint16_t*>(input),
+                                                               input_dim, token);
+      a.token = token;
     }
+    if (storage == PLUTO_HIP_MATRIX_BF16)
+      launch_matvec<0>(s, a, tokens);
+    else if (storage == PLUTO_HIP_MATRIX_F32)
+      launch_matvec<1>(s, a, tokens);
+    else
+      launch_matvec<2>(s, a, tokens);
     return launch_status();
   }
-  float* token = static_cast<float*>(workspace);
-  if (storage == PLUTO_HIP_MATRIX_FP8_E4M3)
-    imported_token_kernel<true><<<groups, kGroup, 0, s>>>(static_cast<const uint16_t*>(input),
-                                                          input_dim, token);
-  else
-    imported_token_kernel<false><<<groups, kGroup, 0, s>>>(static_cast<const uint16_t*>(input),
-                                                           input_dim, token);
-  MatVecArgs a;
-  a.weights = weights;
-  a.scales = scales;
-  a.token = token;
-  a.out = static_cast<uint16_t*>(output);
-  a.cols = input_dim;
-  a.rows = output_dim;
-  if (storage == PLUTO_HIP_MATRIX_BF16)
-    launch_matvec<0>(s, a, tokens);
-  else if (storage == PLUTO_HIP_MATRIX_F32)
-    launch_matvec<1>(s, a, tokens);
-  else
-    launch_matvec<2>(s, a, tokens);
-  return launch_status();
-}
-
-// Several matrices of one storage kind and input width applied to the same
-// tokens: the tokens are prepared once and every pass of 32 tokens is one
-// launch over the tiles of all matrices.  Takes the matrix-core path only
-// (tile_path()); the caller falls back to one call a matrix otherwise.
-int launch_dense_imported_forward_many(hipStream_t s, int storage, int matrices,
-                                       const void* const* weights, const float* const* scales,
-                                       const int* output_dims, const void* input, int tokens,
-                                       int input_dim, void* const* outputs, void* workspace) {
-  const bool fp8 = storage == PLUTO_HIP_MATRIX_FP8_E4M3;
   TileManyArgs t;
-  t.matrices = matrices;
-  t.cols = input_dim;
+  fill(t, t.weight_scales, 32);
   t.tokens = static_cast<const uint16_t*>(input);
-  t.first_block[0] = 0;
-  for (int i = 0; i < kManyMax; ++i) {
-    const bool used = i < matrices;
-    t.weights[i] = used ? weights[i] : nullptr;
-    t.weight_scales[i] = used && fp8 ? scales[i] : nullptr;
-    t.out[i] = used ? static_cast<uint16_t*>(outputs[i]) : nullptr;
-    t.rows[i] = used ? output_dims[i] : 0;
-    t.first_block[i + 1] = t.first_block[i] + (used ? (output_dims[i] + 31) / 32 : 0);
-  }
   if (fp8) {
-    const dim3 groups(static_cast<unsigned>((input_dim + kGroup - 1) / kGroup),
-                      static_cast<unsigned>(tokens));
     uint16_t* values = static_cast<uint16_t*>(workspace);
     float* token_scales = reinterpret_cast<float*>(static_cast<char*>(workspace) +
                                                    tile_values_bytes(tokens, input_dim));
@@ -583,9 +704,9 @@ int launch_dense_imported_forward_many(hipStream_t s, int storage, int matrices,
   for (int done = 0; done < tokens; done += 32) {
     t.count = tokens - done < 32 ? tokens - done : 32;
     if (fp8)
-      launch_fp8_tiles_many(s, t, blocks);
+      launch_fp8_tiles(s, t, blocks);
     else
-      imported_tile_many_kernel<false><<<blocks, 64 * kTileWaves, 0, s>>>(t);
+      imported_tile_kernel<false><<<blocks, 64 * kTileWaves, 0, s>>>(t);
     t.tokens += static_cast<size_t>(32) * input_dim;
     if (fp8) t.token_scales += static_cast<size_t>(32) * (input_dim / kGroup);
     for (int i = 0; i < matrices; ++i) t.out[i] += static_cast<size_t>(32) * output_dims[i];
@@ -643,8 +764,9 @@ int pluto_hip_dense_imported_forward_batch(void* stream, int storage, const void
   if (!weights || !input || !output) return PLUTO_HIP_EINVAL;
   if (!workspace || workspace_bytes < dense_imported_workspace_bytes(tokens, input_dim))
     return PLUTO_HIP_EWORKSPACE;
-  return launch_dense_imported_forward(static_cast<hipStream_t>(stream), storage, weights, scales,
-                                       input, tokens, input_dim, output_dim, output, workspace);
+  return launch_dense_imported_forward(static_cast<hipStream_t>(stream), storage, 1, &weights,
+                                       &scales, &output_dim, input, tokens, input_dim, &output,
+                                       workspace);
 }
 
 int pluto_hip_dense_imported_forward_many(void* stream, int storage, int matrices,
@@ -670,19 +792,9 @@ int pluto_hip_dense_imported_forward_many(void* stream, int storage, int matrice
   if (tiles > 0x7fffffffLL) return PLUTO_HIP_EINVAL;
   if (!workspace || workspace_bytes < dense_imported_workspace_bytes(tokens, input_dim))
     return PLUTO_HIP_EWORKSPACE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (tile_path(storage, tokens, input_dim))
-    return launch_dense_imported_forward_many(s, storage, matrices, weights, scales, output_dims,
-                                              input, tokens, input_dim, outputs, workspace);
-  // few tokens, FP32 matrices or a ragged width: one call a matrix, same results
-  for (int i = 0; i < matrices; ++i) {
-    const int status = launch_dense_imported_forward(s, storage, weights[i],
-                                                     fp8 ? scales[i] : nullptr, input, tokens,
-                                                     input_dim, output_dims[i], outputs[i],
-                                                     workspace);
-    if (status != 0) return status;
-  }
-  return 0;
+  return launch_dense_imported_forward(static_cast<hipStream_t>(stream), storage, matrices, weights,
+                                       scales, output_dims, input, tokens, input_dim, outputs,
+                                       workspace);
 }
 
 }  // extern "C"

@@ -264,3 +264,26 @@ def test_rejects_bad_arguments(capi):
     assert lib.pluto_hip_dense_imported_workspace_bytes(0) == 0
     assert lib.pluto_hip_dense_imported_workspace_bytes(3) >= 12
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("storage", ["bf16", "f32", "fp8"])
+@pytest.mark.parametrize("cols,rows", [(16, 5), (128, 33), (144, 17), (1000, 16), (3328, 40), (5120, 130),
+                                       (9216, 20), (20480, 9)])
+def test_one_token_is_prepared_as_for_several(capi, storage, cols, rows):
+    """One token is prepared by the workgroups that use it, two by a launch of their
+    own: the same row, bit for bit, at widths of one to more than eight pieces a lane,
+    with and without a ragged last group, and too wide for the first way."""
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn((2, cols), generator=gen, device="cuda").to(torch.bfloat16)
+    x[:, :7] *= 300.0
+    w = torch.randn((rows, cols), generator=gen, device="cuda")
+    scales = None
+    code = {"bf16": capi.MATRIX_BF16, "f32": capi.MATRIX_F32, "fp8": capi.MATRIX_FP8_E4M3}[storage]
+    if storage == "bf16":
+        w = w.to(torch.bfloat16)
+    elif storage == "fp8":
+        w = torch.randint(0, 0x7f, (rows, cols), generator=gen, device="cuda", dtype=torch.uint8)
+        scales = torch.rand(((rows + 127) // 128, (cols + 127) // 128), generator=gen, device="cuda")
+    both = capi.dense_imported_forward_batch(code, w, scales, x)
+    for t in range(2):
+        assert torch.equal(capi.dense_imported_forward(code, w, scales, x[t].contiguous()), both[t]), t
