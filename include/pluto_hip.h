@@ -280,9 +280,11 @@ int pluto_hip_gqa_prefill_probabilities(void* stream,
  *             be NULL), each fp32 [qh, positions[b] + 1]
  *             (AttentionProbabilitiesKernel, cached_attention_ops.cc:131-178)
  *   split_tokens: cache rows per split-K block: a multiple of 64 up to 512, or
- *             1024 at head width 256; 0 selects the default (512, and 1024
- *             at head width 256).  Anything else is PLUTO_HIP_EINVAL, and the
- *             workspace size is then reported as 0.
+ *             1024 at head width 256; 0 lets the library choose by the batch
+ *             and its positions: 512 (1024 at head width 256), or less where
+ *             such blocks would leave compute units idle.  Anything else is
+ *             PLUTO_HIP_EINVAL, and the workspace size is then reported as 0.
+ *             A workspace for given positions also serves smaller ones.
  * Returns PLUTO_HIP_ERANGE if any positions[b] >= capacity; nothing is
  * queued in that case. */
 size_t pluto_hip_gqa_decode_workspace_bytes(const pluto_hip_attention_params* p,

@@ -151,14 +151,55 @@ PrefillBackwardLayout prefill_backward_layout(const pluto_hip_attention_params* 
   return l;
 }
 
-int split_or_default(int split_tokens, int head_dim) {
-  return split_tokens == 0 ? decode_split_default(head_dim) : split_tokens;
-}
 
 long long decode_blocks(int batch, const int* positions, int split) {
   long long blocks = 0;
   for (int b = 0; b < batch; ++b) blocks += (static_cast<long long>(positions[b]) + split) / split;
   return blocks;
+}
+
+// The block size of a call that leaves it to the library: of the default and its
+// halves the one whose estimated time is least.  What the estimate is made of was
+// fitted to calls of 1 to 32 sequences of 100 to 32000 rows: a workgroup takes a
+// fixed time whatever it does and some more for every 64 rows of its block; the
+// chip holds two (head width 256) or three a compute unit at once, and a call
+// takes as many rounds of them as it needs; the workgroup that ends a sequence
+// adds up its blocks.  (One sequence of 777 rows at width 256: 34 us with one block
+// of 1024 rows, 18 with blocks of 128.)  Sizes below the default are taken only
+// up to two rounds, which bounds the scratch such a call needs.
+long long decode_resident(int head_dim) { return head_dim == 256 ? 512 : 768; }
+int decode_split(const pluto_hip_attention_params* p, int batch, const int* positions,
+                 int split_tokens) {
+  if (split_tokens != 0) return split_tokens;
+  const bool wide = p->head_dim == 256;
+  const double fixed = wide ? 12.0 : 11.0, rows64 = wide ? 1.2 : 0.45, combine = wide ? 0.25 : 0.19;
+  const long long resident = decode_resident(p->head_dim);
+  const int standard = decode_split_default(p->head_dim);
+  int longest = 0;
+  for (int b = 0; b < batch; ++b) longest = positions[b] > longest ? positions[b] : longest;
+  int best = standard;
+  double least = 0.0;
+  for (int split = standard; split >= 64; split /= 2) {
+    const long long workgroups = decode_blocks(batch, positions, split) * p->key_value_heads;
+    if (split < standard && workgroups > 2 * resident) break;
+    const double rounds = static_cast<double>((workgroups + resident - 1) / resident);
+    const double estimate = rounds * (fixed + rows64 * (split / 64)) +
+                            combine * static_cast<double>(longest / split + 1);
+    if (split == standard || estimate < least) {
+      best = split;
+      least = estimate;
+    }
+  }
+  return best;
+}
+// An upper bound of the blocks of such a call that also holds for every call at
+// smaller positions.
+long long decode_blocks_bound(const pluto_hip_attention_params* p, int batch, const int* positions,
+                              int split_tokens) {
+  if (split_tokens != 0) return decode_blocks(batch, positions, split_tokens);
+  const long long standard = decode_blocks(batch, positions, decode_split_default(p->head_dim));
+  const long long smaller = 2 * decode_resident(p->head_dim) / p->key_value_heads;
+  return standard > smaller ? standard : smaller;
 }
 
 // What the forward pass can leave for the backward pass: the attention output
@@ -529,11 +570,10 @@ static DecodeLayout decode_layout(const pluto_hip_attention_params* p, int batch
 size_t pluto_hip_gqa_decode_workspace_bytes(const pluto_hip_attention_params* p, int batch,
                                             const int* positions, int split_tokens) {
   if (validate_params(p) != 0 || batch <= 0 || !positions) return 0;
-  const int split = split_or_default(split_tokens, p ? p->head_dim : 0);
-  if (!decode_split_valid(p->head_dim, split)) return 0;
+  if (split_tokens != 0 && !decode_split_valid(p->head_dim, split_tokens)) return 0;
   for (int b = 0; b < batch; ++b)
     if (positions[b] < 0) return 0;
-  const long long blocks = decode_blocks(batch, positions, split);
+  const long long blocks = decode_blocks_bound(p, batch, positions, split_tokens);
   return decode_layout(p, batch, blocks,
                        static_cast<size_t>(batch) * p->key_value_heads * sizeof(unsigned))
       .total;
@@ -544,7 +584,8 @@ size_t pluto_hip_gqa_decode_workspace_bytes(const pluto_hip_attention_params* p,
 static int decode_check(const pluto_hip_attention_params* p, int batch, int io_dtype,
                         const void* q_gate, const void* k, const void* v, const float* q_norm,
                         const float* k_norm, const int* positions,
-                        const pluto_hip_kv_cache_view* caches, const void* out, int split) {
+                        const pluto_hip_kv_cache_view* caches, const void* out,
+                        int split_tokens) {
   int status = validate_params(p);
   if (status != 0) return status;
   if (batch <= 0 || (io_dtype != PLUTO_HIP_F32 && io_dtype != PLUTO_HIP_BF16))
@@ -552,7 +593,7 @@ static int decode_check(const pluto_hip_attention_params* p, int batch, int io_d
   // cached_attention_ops.cc:314-317: null pointers are rejected before any work.
   if (!q_gate || !k || !v || !q_norm || !k_norm || !out || !positions || !caches)
     return PLUTO_HIP_EINVAL;
-  if (!decode_split_valid(p->head_dim, split)) return PLUTO_HIP_EINVAL;
+  if (split_tokens != 0 && !decode_split_valid(p->head_dim, split_tokens)) return PLUTO_HIP_EINVAL;
   for (int b = 0; b < batch; ++b) {
     status = validate_cache(&caches[b], p);
     if (status != 0) return status;
@@ -584,10 +625,10 @@ int pluto_hip_gqa_decode(void* stream, const pluto_hip_attention_params* p, int 
                          const pluto_hip_kv_cache_view* caches, void* out,
                          float* const* probabilities, int split_tokens, void* workspace,
                          size_t workspace_bytes) {
-  const int split = split_or_default(split_tokens, p ? p->head_dim : 0);
-  const int status =
-      decode_check(p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions, caches, out, split);
+  const int status = decode_check(p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions,
+                                  caches, out, split_tokens);
   if (status != 0) return status;
+  const int split = decode_split(p, batch, positions, split_tokens);
   const DecodeLayout layout =
       decode_layout(p, batch, decode_blocks(batch, positions, split),
                     static_cast<size_t>(batch) * p->key_value_heads * sizeof(unsigned));
@@ -609,10 +650,10 @@ int pluto_hip_gqa_decode_static(void* stream, const pluto_hip_attention_params* 
                                 const float* q_norm, const float* k_norm, const int* positions,
                                 const pluto_hip_kv_cache_view* caches, void* out,
                                 float* const* probabilities, int split_tokens) {
-  const int split = split_or_default(split_tokens, p ? p->head_dim : 0);
-  int status =
-      decode_check(p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions, caches, out, split);
+  int status = decode_check(p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions, caches,
+                            out, split_tokens);
   if (status != 0) return status;
+  const int split = decode_split(p, batch, positions, split_tokens);
   if (static_cast<size_t>(batch) * p->key_value_heads * sizeof(unsigned) > kStaticArrivalBytes)
     return PLUTO_HIP_ELIMIT;
   const DecodeLayout layout =

@@ -42,7 +42,7 @@ namespace {
 
 constexpr int kMaxSplit = 512;
 constexpr int kThreads = 256;
-constexpr int kCombineChunk = 128;  // blocks combined per pass over the LDS weights
+constexpr int kCombineChunk = 64;  // blocks combined per pass over the LDS weights: one a lane
 
 __device__ inline bf16x8 load_bf16x8(const uint16_t* p) {
   return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
@@ -68,6 +68,20 @@ __device__ inline void store_shared(float* p, float v) {
 __device__ inline float load_shared(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Two neighbouring values (8-byte aligned) in one access.
+__device__ inline void store_shared(float* p, float2 v) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p),
+                     __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline float2 load_shared2(const float* p) {
+  return __builtin_bit_cast(
+      float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// (the kernel has an array named like the helper)
+__device__ inline float max_over_wave(float v) { return wave_max(v); }
 
 // Workgroup barrier that orders LDS traffic only: unlike __syncthreads() it
 // does not wait for the wave's outstanding global loads.
@@ -555,16 +569,22 @@ __device__ inline void decode_block(const DecodeArgs& a, const BlockContext& ctx
   // the four waves' results, each relative to its own maximum, become the
   // block's: o = sum_w o_w 2^(m_w - m), l likewise, m = max_w m_w
   const long long slot = ctx.slot;
-  for (int i = tid; i < GROUP * D; i += kThreads) {
+  for (int i = 2 * tid; i < GROUP * D; i += 2 * kThreads) {
     const int hh = i / D, c = i % D;
     const float m = fmaxf(fmaxf(wave_max[0][hh], wave_max[1][hh]),
                           fmaxf(wave_max[2][hh], wave_max[3][hh]));
-    float w[4];
+    float2 total[2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) w[q] = __builtin_amdgcn_exp2f(wave_max[q][hh] - m);
+    for (int q = 0; q < 4; ++q) {
+      const float w = __builtin_amdgcn_exp2f(wave_max[q][hh] - m);
+      const float2 o = *reinterpret_cast<const float2*>(&o_lds[q][hh][c]);
+      if (q % 2 == 0)
+        total[q / 2] = make_float2(o.x * w, o.y * w);
+      else
+        total[q / 2] = make_float2(total[q / 2].x + o.x * w, total[q / 2].y + o.y * w);
+    }
     store_shared(&a.part_o[(slot * GROUP + hh) * D + c],
-                 (o_lds[0][hh][c] * w[0] + o_lds[1][hh][c] * w[1]) +
-                     (o_lds[2][hh][c] * w[2] + o_lds[3][hh][c] * w[3]));
+                 make_float2(total[0].x + total[1].x, total[0].y + total[1].y));
   }
   if (tid < GROUP) {
     const float m = fmaxf(fmaxf(wave_max[0][tid], wave_max[1][tid]),
@@ -651,90 +671,99 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
   }
 
   // ---- combine: blocks in ascending order, kCombineChunk at a time --------
-  // LDS: m, l and then the weights of the chunk's blocks per head; running
-  // maximum, normalizer and rescale factor per head.
-  float* chunk_m = shared_area;                           // [kCombineChunk][GROUP]
-  float* chunk_l = shared_area + kCombineChunk * GROUP;   // [kCombineChunk][GROUP]
-  float* head_state = shared_area + 2 * kCombineChunk * GROUP;  // [3][GROUP]
-  static_assert((2 * kCombineChunk * GROUP + 3 * GROUP) * 4 <= value_area_bytes<D>());
+  // A wave computes the weights of its heads with one block a lane; the partial
+  // outputs are requested kAhead blocks at a time, the first of them before the
+  // weights are known, two channels an access.  (With one channel an access, eight
+  // blocks at a time, and the weights summed by one thread a head, a block cost
+  // 0.36 us here: 11 us of a 36 us step at 32 blocks.)
+  float* chunk_w = shared_area;                            // [kCombineChunk][GROUP] weights
+  float* head_state = shared_area + kCombineChunk * GROUP;  // [3][GROUP]: max, normalizer, rescale
+  static_assert((kCombineChunk * GROUP + 3 * GROUP) * 4 <= value_area_bytes<D>());
   static_assert(4 * GROUP * D * 4 <= value_area_bytes<D>());
-  constexpr int kOutputs = (GROUP * D + kThreads - 1) / kThreads;  // per thread
+  constexpr int kPairs = (GROUP * D / 2 + kThreads - 1) / kThreads;  // per thread
+  constexpr int kAhead = kPairs <= 2 ? 16 : 8;
   const long long first_slot = (a.block_base + batch.block_start[b]) * kh + g;
   const long long slot_step = kh;  // consecutive blocks of one kv head
-  float o[kOutputs];
+  float2 o[kPairs];
 #pragma unroll
-  for (int u = 0; u < kOutputs; ++u) o[u] = 0.0f;
+  for (int u = 0; u < kPairs; ++u) o[u] = make_float2(0.0f, 0.0f);
   if (tid < GROUP) {
     head_state[0 * GROUP + tid] = kMasked;  // running maximum
     head_state[1 * GROUP + tid] = 0.0f;     // running normalizer
   }
   for (int j0 = 0; j0 < blocks_here; j0 += kCombineChunk) {
     const int count = min(kCombineChunk, blocks_here - j0);
-    __syncthreads();  // the previous chunk's weights are no longer read
-    for (int i = tid; i < count * GROUP; i += kThreads) {
-      const long long at = (first_slot + (j0 + i / GROUP) * slot_step) * GROUP + i % GROUP;
-      chunk_m[i] = load_shared(&a.part_m[at]);
-      chunk_l[i] = load_shared(&a.part_l[at]);
-    }
-    __syncthreads();
-    if (tid < GROUP) {
-      const float old_max = head_state[0 * GROUP + tid];
-      float maximum = old_max;
-      for (int jj = 0; jj < count; ++jj) maximum = fmaxf(maximum, chunk_m[jj * GROUP + tid]);
-      const float rescale = __builtin_amdgcn_exp2f(old_max - maximum);
-      float normalizer = head_state[1 * GROUP + tid] * rescale;
-      for (int jj = 0; jj < count; ++jj) {
-        const float w = __builtin_amdgcn_exp2f(chunk_m[jj * GROUP + tid] - maximum);
-        normalizer += chunk_l[jj * GROUP + tid] * w;
-        chunk_m[jj * GROUP + tid] = w;  // from here on: the block's weight
-      }
-      head_state[0 * GROUP + tid] = maximum;
-      head_state[1 * GROUP + tid] = normalizer;
-      head_state[2 * GROUP + tid] = rescale;
-    }
-    __syncthreads();
+    float2 part[kAhead][kPairs];
+    auto request = [&](int jj) {
 #pragma unroll
-    for (int u = 0; u < kOutputs; ++u) {
-      const int i = tid + u * kThreads;
-      if (i < GROUP * D) o[u] *= head_state[2 * GROUP + i / D];
-    }
-    // eight blocks per step: their loads are issued before their use
-    for (int jj = 0; jj < count; jj += 8) {
-      float part[8][kOutputs];
-#pragma unroll
-      for (int step = 0; step < 8; ++step) {
+      for (int step = 0; step < kAhead; ++step) {
         const int block_j = min(jj + step, count - 1);
         const float* base = a.part_o + (first_slot + (j0 + block_j) * slot_step) * GROUP * D;
 #pragma unroll
-        for (int u = 0; u < kOutputs; ++u) {
-          const int i = tid + u * kThreads;
-          part[step][u] = i < GROUP * D ? load_shared(&base[i]) : 0.0f;
+        for (int u = 0; u < kPairs; ++u) {
+          const int i = 2 * (tid + u * kThreads);
+          part[step][u] = i < GROUP * D ? load_shared2(&base[i]) : make_float2(0.0f, 0.0f);
         }
       }
+    };
+    request(0);
+    __syncthreads();  // the chunk before has been added up, and the states written
+    for (int hh = ctx.wave; hh < GROUP; hh += 4) {
+      const long long at = (first_slot + (j0 + min(ctx.lane, count - 1)) * slot_step) * GROUP + hh;
+      const float block_max = load_shared(&a.part_m[at]), block_sum = load_shared(&a.part_l[at]);
+      const float old_max = head_state[0 * GROUP + hh], old_sum = head_state[1 * GROUP + hh];
+      const float maximum = fmaxf(old_max, max_over_wave(block_max));
+      const float weight =
+          ctx.lane < count ? __builtin_amdgcn_exp2f(block_max - maximum) : 0.0f;
+      const float sum = wave_sum(block_sum * weight);
+      const float rescale = __builtin_amdgcn_exp2f(old_max - maximum);
+      chunk_w[ctx.lane * GROUP + hh] = weight;
+      if (ctx.lane == 0) {
+        head_state[0 * GROUP + hh] = maximum;
+        head_state[1 * GROUP + hh] = old_sum * rescale + sum;
+        head_state[2 * GROUP + hh] = rescale;
+      }
+    }
+    __syncthreads();
 #pragma unroll
-      for (int step = 0; step < 8; ++step) {
-        if (jj + step < count) {
+    for (int u = 0; u < kPairs; ++u) {
+      const int i = 2 * (tid + u * kThreads);
+      if (i >= GROUP * D) continue;
+      const float rescale = head_state[2 * GROUP + i / D];
+      o[u].x *= rescale;
+      o[u].y *= rescale;
+    }
+    for (int jj = 0; jj < count; jj += kAhead) {
+      if (jj > 0) request(jj);
 #pragma unroll
-          for (int u = 0; u < kOutputs; ++u) {
-            const int i = tid + u * kThreads;
-            if (i < GROUP * D) o[u] += part[step][u] * chunk_m[(jj + step) * GROUP + i / D];
-          }
+      for (int step = 0; step < kAhead; ++step) {
+        if (jj + step >= count) continue;
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) {
+          const int i = 2 * (tid + u * kThreads);
+          if (i >= GROUP * D) continue;
+          const float weight = chunk_w[(jj + step) * GROUP + i / D];
+          o[u].x += part[step][u].x * weight;
+          o[u].y += part[step][u].y * weight;
         }
       }
     }
   }
   // gate: cached_attention_ops.cc:119-125
 #pragma unroll
-  for (int u = 0; u < kOutputs; ++u) {
-    const int i = tid + u * kThreads;
+  for (int u = 0; u < kPairs; ++u) {
+    const int i = 2 * (tid + u * kThreads);
     if (i >= GROUP * D) continue;
     const int hh = i / D, c = i % D;
-    const float core = o[u] / head_state[1 * GROUP + hh];
     const long long at = static_cast<long long>(seq) * a.query_heads + g * GROUP + hh;
-    const float logit = load_element(a.q_gate, (at * 2 + 1) * D + c, a.io_dtype);
-    const float sigmoid = gate_sigmoid(logit);
-    store_element(a.out, at * D + c, a.io_dtype,
-                  round_to_bf16(round_to_bf16(core) * round_to_bf16(sigmoid)));
+    const float core[2] = {o[u].x / head_state[1 * GROUP + hh], o[u].y / head_state[1 * GROUP + hh]};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float logit = load_element(a.q_gate, (at * 2 + 1) * D + c + e, a.io_dtype);
+      const float sigmoid = gate_sigmoid(logit);
+      store_element(a.out, at * D + c + e, a.io_dtype,
+                    round_to_bf16(round_to_bf16(core[e]) * round_to_bf16(sigmoid)));
+    }
   }
 }
 

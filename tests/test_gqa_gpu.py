@@ -453,6 +453,35 @@ def test_batched_decode_block_sizes_and_head_widths(capi, oracle, d, qh, kh, rot
     assert torch.equal(out, capi.gqa_decode(*args, split_tokens=split, advance=False))
 
 
+@pytest.mark.parametrize("d,batch", [(256, 1), (256, 5), (128, 1), (128, 3), (64, 2)])
+def test_decode_block_size_chosen_by_the_library(capi, d, batch):
+    """Lengths on both sides of every block size the library may choose, on one
+    workspace sized for the longest: within two bf16 ulps of the core of what blocks
+    of 512 rows give (the two add up in different orders)."""
+    qh, kh, longest = 12, 2, 5000
+    p = capi.attention_params(qh, kh, d, 32, capacity=longest)
+    gen = torch.Generator(device="cuda").manual_seed(d + batch)
+    bf = torch.bfloat16
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(bf)
+    workspace = capi.gqa_decode_workspace(p, [longest - 1] * batch)
+    q_gate, k, v = values(batch, qh, 2, d), values(batch, kh, d), values(batch, kh, d)
+    w = torch.zeros(d, device="cuda")
+    caches = []
+    for _ in range(batch):
+        c = capi.KvCache(longest, kh, d)
+        c.keys.copy_(values(kh, longest, d))
+        c.values.copy_(values(kh, longest, d))
+        caches.append(c)
+    for length in (1, 63, 64, 65, 129, 513, 777, 1025, 2100, longest):
+        positions = [max(0, length - 1 - 37 * i) for i in range(batch)]
+        got = capi.gqa_decode(p, q_gate, k, v, w, w, caches, positions=positions, workspace=workspace,
+                              advance=False).float()
+        want = capi.gqa_decode(p, q_gate, k, v, w, w, caches, positions=positions, split_tokens=512,
+                               advance=False).float()
+        assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-4), length
+
+
 def test_decode_more_than_one_launch_slice(capi, oracle):
     # 70 sequences > 64 per launch, ragged short lengths, split 64
     batch, qh, kh, d = 70, 4, 2, 64
