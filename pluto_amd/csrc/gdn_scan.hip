@@ -322,13 +322,13 @@ gdn_chunk_prepare(GdnArgs a) {
 
 // LDS stage of the sequential kernel for one chunk: the chunk's scratch as it
 // sits in memory (T | A2 | factors, 14 KiB), the raw K and Q rows gathered
-// into matrix-core operand order (16 KiB each), and the 16 value columns of the
-// workgroup's slice (2 KiB).
+// into matrix-core operand order (16 KiB each), and the 16 value columns of each
+// of the workgroup's slices (2 KiB).
 constexpr int kStageScratch = 0;
 constexpr int kStageK = static_cast<int>(kGdnChunkBytes);
 constexpr int kStageQ = kStageK + 16384;
 constexpr int kStageV = kStageQ + 16384;
-constexpr int kScanStageBytes = kStageV + 2048;
+constexpr int scan_stage_bytes(int slices) { return kStageV + 2048 * slices; }
 constexpr int kScanStages = 2;
 
 typedef __attribute__((address_space(3))) unsigned char lds_byte;
@@ -382,10 +382,10 @@ struct ScanSources {
 };
 
 // The direct-to-LDS loads of one chunk, 1 KiB each: 14 of scratch, 16 of K,
-// 16 of Q, 2 of V.  Loader wave LOADER of LOADERS issues every LOADERS-th.
+// 16 of Q, 2 of V a slice.  Loader wave LOADER of LOADERS issues every LOADERS-th.
 constexpr int kFillScratch = static_cast<int>(kGdnChunkBytes) / 1024;
-constexpr int kScanFillLoads = kFillScratch + 16 + 16 + 2;
-template <int LOADER, int LOADERS>
+constexpr int scan_fill_loads(int slices) { return kFillScratch + 16 + 16 + 2 * slices; }
+template <int LOADER, int LOADERS, int WG_SLICES>
 __device__ __forceinline__ void scan_fill(uint32_t stage_address, const ScanSources& src, int chunk,
                                           int lane) {
   const uint32_t lane_bytes = static_cast<uint32_t>(lane) * 16u;
@@ -393,7 +393,7 @@ __device__ __forceinline__ void scan_fill(uint32_t stage_address, const ScanSour
   // fully unrolled: a lone wave issues a loop's scalar bookkeeping far slower
   // than the memory pipeline takes loads
 #pragma unroll
-  for (int f = LOADER; f < kScanFillLoads; f += LOADERS) {
+  for (int f = LOADER; f < scan_fill_loads(WG_SLICES); f += LOADERS) {
     if (f < kFillScratch) {
       lds_dma_16(src.scratch, stage_address + f * 1024, lane_bytes,
                  static_cast<uint32_t>(chunk) * static_cast<uint32_t>(kGdnChunkBytes) + f * 1024);
@@ -408,9 +408,9 @@ __device__ __forceinline__ void scan_fill(uint32_t stage_address, const ScanSour
         lds_dma_16(src.q, stage_address + kStageQ + g * 1024,
                    src.q_lane + (row0 + 16 * tile) * src.q_row_bytes + 64 * kb, 0);
     } else {
-      const int half = f - kFillScratch - 32;
-      lds_dma_16(src.v, stage_address + kStageV + half * 1024,
-                 src.v_lane + (row0 + 32 * half) * src.v_row_bytes, 0);
+      const int slice = (f - kFillScratch - 32) / 2, half = (f - kFillScratch - 32) % 2;
+      lds_dma_16(src.v, stage_address + kStageV + slice * 2048 + half * 1024,
+                 src.v_lane + (row0 + 32 * half) * src.v_row_bytes + 32 * slice, 0);
     }
   }
 }
@@ -419,28 +419,28 @@ __device__ __forceinline__ void scan_fill(uint32_t stage_address, const ScanSour
 // index, and a wait that lets exactly its share of one (the younger) fill stay
 // in flight.
 constexpr int kScanLoaders = 2;
-static_assert(kScanLoaders == 2 || kScanLoaders == 3, "scan_fill_as and scan_wait_older_fill list the loaders");
-constexpr int scan_fill_share(int loader) {
-  return (kScanFillLoads - loader + kScanLoaders - 1) / kScanLoaders;
+constexpr int scan_fill_share(int loader, int slices) {
+  return (scan_fill_loads(slices) - loader + kScanLoaders - 1) / kScanLoaders;
 }
 // (a wave whose two fills exceed the 63 operations its vector-memory counter
 // holds merely stalls at the issue of the last few loads)
-static_assert(scan_fill_share(0) <= 63, "the wait for the older fill must be encodable");
+static_assert(scan_fill_share(0, 2) <= 63, "the wait for the older fill must be encodable");
+template <int WG_SLICES>
 __device__ __forceinline__ void scan_fill_as(int loader, uint32_t stage_address,
                                              const ScanSources& src, int chunk, int lane) {
-  if (loader == 0) scan_fill<0, kScanLoaders>(stage_address, src, chunk, lane);
-  else if (loader == 1 || kScanLoaders == 2) scan_fill<1, kScanLoaders>(stage_address, src, chunk, lane);
-  else scan_fill<kScanLoaders - 1, kScanLoaders>(stage_address, src, chunk, lane);
+  if (loader == 0) scan_fill<0, kScanLoaders, WG_SLICES>(stage_address, src, chunk, lane);
+  else scan_fill<1, kScanLoaders, WG_SLICES>(stage_address, src, chunk, lane);
 }
+template <int WG_SLICES>
 __device__ __forceinline__ void scan_wait_older_fill(int loader) {
-  if (loader == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(scan_fill_share(0)) : "memory");
-  else if (loader == 1 || kScanLoaders == 2)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(scan_fill_share(1)) : "memory");
-  else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(scan_fill_share(kScanLoaders - 1)) : "memory");
+  if (loader == 0)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(scan_fill_share(0, WG_SLICES)) : "memory");
+  else
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(scan_fill_share(1, WG_SLICES)) : "memory");
 }
 
-// Pulls this workgroup's eighth of a future chunk (its scratch, its K rows and
-// its Q rows; the eight workgroups of a (sequence, head) share all three) and
+// Pulls a slice's eighth of a future chunk (its scratch, its K rows and
+// its Q rows; the eight slices of a (sequence, head) share all three) and
 // its own V columns through L2 so that it is there by the time the workgroups fetch it for real:
 // the loader waves cannot keep enough real loads in flight to cover the latency
 // of HBM.  These are full-width loads (1 KiB per instruction): what bounds a
@@ -450,7 +450,7 @@ __device__ __forceinline__ void scan_wait_older_fill(int loader) {
 // for them.
 constexpr int kScanAhead = 4;
 __device__ inline void scan_touch(const ScanSources& src, uint32_t dump_address, int chunk,
-                                  int slice, int lane) {
+                                  int slice, uint32_t v_column_bytes, int lane) {
   const uint32_t lane_bytes = static_cast<uint32_t>(lane) * 16u;
   // scratch: 14 KiB / 8 = 1792 bytes, two loads (the second runs into the
   // next slice's share, or past the end of the scratch, where it reads zeros)
@@ -470,11 +470,12 @@ __device__ inline void scan_touch(const ScanSources& src, uint32_t dump_address,
 #pragma unroll
   for (int half = 0; half < 2; ++half)
     lds_dma_16(src.v, dump_address,
-               src.v_lane + (static_cast<uint32_t>(chunk) * C + 32 * half) * src.v_row_bytes, 0);
+               src.v_lane + (static_cast<uint32_t>(chunk) * C + 32 * half) * src.v_row_bytes +
+                   v_column_bytes,
+               0);
 }
 
-// One workgroup per (sequence, head, slice of 16 state columns), one wave per
-// SIMD so that each may use the whole register file: the chain wave (the
+// One workgroup per (sequence, head, slice of 16 state columns): the chain wave (the
 // sequential dependence from state to state: P = K S0, D, the state update),
 // the output wave (Q S0, the causal product with D, the stores, and the loads
 // that warm L2), and kScanLoaders loader waves.  A stage holds one chunk.  The
@@ -487,8 +488,12 @@ __device__ inline void scan_touch(const ScanSources& src, uint32_t dump_address,
 // computing waves are done with the stage, and the chain wave has published D).
 // A wave that issues long runs of loads stalls at issue while the memory
 // pipeline digests them, which is why the chain wave issues none.
-constexpr int kScanThreads = 64 * (2 + kScanLoaders);
-static_assert(kScanThreads <= 256, "one wave per SIMD");
+//
+// WG_SLICES = 2: a workgroup of six waves walks two slices of a head from one
+// copy of the stage, a chain and an output wave each.  A compute unit holds one
+// workgroup, and 48 heads are 384 single slices, one and a half rounds of the
+// chip that take two; as 192 pairs they take one (8191 tokens: 290 -> 192 us).
+constexpr int scan_threads(int slices) { return 64 * (2 * slices + kScanLoaders); }
 
 // The workgroup barriers that hand an LDS stage over.  A loader arrives at the
 // "landed" barrier once the stage's direct-to-LDS loads are complete (the
@@ -503,7 +508,7 @@ __device__ __forceinline__ void scan_handover_compute() {
 struct ScanContext {
   uint16_t* out;
   int length, value_heads;
-  int slice, lane, hq, m, seq, head;
+  int slice, local, lane, hq, m, seq, head;  // local: the slice within the workgroup
 };
 
 __device__ inline float bf16_half(uint32_t word, int upper) {
@@ -563,7 +568,7 @@ __device__ __forceinline__ void chain_step(const ScanContext ctx, const lds_byte
     if (i == 0) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        v_reg[j] = lds_transposed(stage + kStageV + (16 * j + 4 * hq + kk) * 32 + 8 * piece);
+        v_reg[j] = lds_transposed(stage + kStageV + 2048 * ctx.local + (16 * j + 4 * hq + kk) * 32 + 8 * piece);
         f1[j] = factor_in[4 * j];
       }
     } else if (i == 1) {
@@ -751,11 +756,13 @@ __device__ inline uint32x4 raw_descriptor(const void* base, uint32_t bytes) {
                   bytes, 0x00020000u};
 }
 
-__global__ void __launch_bounds__(kScanThreads)
+template <int WG_SLICES>
+__global__ void __launch_bounds__(scan_threads(WG_SLICES))
 gdn_chunk_scan(GdnArgs a) {
+  constexpr int kScanStageBytes = scan_stage_bytes(WG_SLICES);
   __shared__ __attribute__((aligned(1024))) unsigned char stages[kScanStages * kScanStageBytes];
   __shared__ __attribute__((aligned(256))) unsigned char dump[1024];
-  __shared__ __attribute__((aligned(16))) ScanExchange exchange;
+  __shared__ __attribute__((aligned(16))) ScanExchange exchanges[WG_SLICES];
   const int lane = threadIdx.x % 64, hq = lane / 16, m = lane % 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int chunks = (a.length + C - 1) / C;
@@ -763,8 +770,9 @@ gdn_chunk_scan(GdnArgs a) {
   // on one XCD so that its L2 serves all but the first read.
   int logical = blockIdx.x;
   if (gridDim.x % 8 == 0) logical = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-  const int slice = logical % SLICES;
-  const int bh = logical / SLICES;
+  constexpr int kGroups = SLICES / WG_SLICES;
+  const int first_slice = logical % kGroups * WG_SLICES;
+  const int bh = logical / kGroups;
   const int head = bh % a.value_heads, seq = bh / a.value_heads;
   const int key_head = head / (a.value_heads / a.key_heads);
   float* state = a.state + static_cast<size_t>(bh) * DK * DV;
@@ -780,8 +788,8 @@ gdn_chunk_scan(GdnArgs a) {
                          static_cast<uint32_t>(a.length - 1) * src.k_row_bytes + DK * 2);
   src.q = raw_descriptor(a.q + first_token * a.q_token_stride + key_head * DK,
                          static_cast<uint32_t>(a.length - 1) * src.q_row_bytes + DK * 2);
-  src.v = raw_descriptor(a.v + first_token * a.v_token_stride + head * DV + 16 * slice,
-                         static_cast<uint32_t>(a.length - 1) * src.v_row_bytes + 16 * 2);
+  src.v = raw_descriptor(a.v + first_token * a.v_token_stride + head * DV + 16 * first_slice,
+                         static_cast<uint32_t>(a.length - 1) * src.v_row_bytes + 16 * WG_SLICES * 2);
   {
     // LDS slot `lane` of a K or Q fragment belongs to the logical lane whose
     // operand_slot it is: token lane / 4 of the tile, piece (lane % 4 - token / 4) mod 4
@@ -800,43 +808,48 @@ gdn_chunk_scan(GdnArgs a) {
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte*)dump));
 
   // Every wave passes two barriers per chunk: "landed" and "free".
-  if (wave >= 2) {
-    const int loader = wave - 2;
-    scan_fill_as(loader, stage0_address, src, 0, lane);
-    if (chunks > 1) scan_fill_as(loader, stage1_address, src, 1, lane);
+  if (wave >= 2 * WG_SLICES) {
+    const int loader = wave - 2 * WG_SLICES;
+    scan_fill_as<WG_SLICES>(loader, stage0_address, src, 0, lane);
+    if (chunks > 1) scan_fill_as<WG_SLICES>(loader, stage1_address, src, 1, lane);
     for (int chunk = 0; chunk < chunks; ++chunk) {
       // loads complete in issue order: all but the younger fill have landed
-      if (chunk + 1 < chunks) scan_wait_older_fill(loader);
+      if (chunk + 1 < chunks) scan_wait_older_fill<WG_SLICES>(loader);
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       scan_barrier();  // landed
       scan_barrier();  // free
       if (chunk + 2 < chunks)
-        scan_fill_as(loader, (chunk & 1) ? stage1_address : stage0_address, src, chunk + 2, lane);
+        scan_fill_as<WG_SLICES>(loader, (chunk & 1) ? stage1_address : stage0_address, src, chunk + 2,
+                                lane);
     }
     return;
   }
 
+  const int local = wave % WG_SLICES, slice = first_slice + local;
+  const lds_byte* stage_base = (const lds_byte*)stages;
+  lds_exchange* exchange = (lds_exchange*)&exchanges[local];
   ScanContext ctx;
   ctx.out = a.out;
   ctx.length = a.length;
   ctx.value_heads = a.value_heads;
   ctx.slice = slice;
+  ctx.local = local;
   ctx.lane = lane;
   ctx.hq = hq;
   ctx.m = m;
   ctx.seq = seq;
   ctx.head = head;
-  if (wave == 1) {
+  // (the loaders share the output waves' SIMDs)
+  if (wave < WG_SLICES) {
     for (int chunk = 2; chunk < min(kScanAhead + 2, chunks); ++chunk)
-      scan_touch(src, dump_address, chunk, slice, lane);
+      scan_touch(src, dump_address, chunk, slice, 32 * local, lane);
     for (int chunk = 0; chunk < chunks; ++chunk) {
       if (chunk + 2 + kScanAhead < chunks)
-        scan_touch(src, dump_address, chunk + 2 + kScanAhead, slice, lane);
+        scan_touch(src, dump_address, chunk + 2 + kScanAhead, slice, 32 * local, lane);
       scan_barrier();  // landed
       // passes the "free" barrier once it has read all it needs of the stage,
       // and has read D by the time it returns
-      output_step(ctx, chunk, (lds_byte*)stages + (chunk & 1) * kScanStageBytes,
-                  (const lds_exchange*)&exchange);
+      output_step(ctx, chunk, stage_base + (chunk & 1) * kScanStageBytes, exchange);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     return;
@@ -853,14 +866,13 @@ gdn_chunk_scan(GdnArgs a) {
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
     sb[kb] = tiles_to_operand(s[2 * kb], s[2 * kb + 1]);
-    exchange.state[kb][lane] = bf16x8_to_words(sb[kb]);
+    exchange->state[kb][lane] = bf16x8_to_words(sb[kb]);
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   for (int chunk = 0; chunk < chunks; ++chunk) {
     scan_barrier();  // landed
     // passes the "free" barrier once it has read all it needs of the stage
-    chain_step(ctx, (lds_byte*)stages + (chunk & 1) * kScanStageBytes, (lds_exchange*)&exchange, s,
-               sb);
+    chain_step(ctx, stage_base + (chunk & 1) * kScanStageBytes, exchange, s, sb);
   }
 #pragma unroll
   for (int t = 0; t < 8; ++t)
@@ -966,7 +978,18 @@ int launch_gdn_chunked(hipStream_t stream, const GdnArgs& a) {
   int status = launch_status();
   if (status != 0) return status;
   if (!kernel_enabled(kMainKernel)) return 0;
-  gdn_chunk_scan<<<static_cast<unsigned>(heads * SLICES), kScanThreads, 0, stream>>>(a);
+  // one workgroup a compute unit: two slices a workgroup where that saves a round
+  int device = 0, units = 0;
+  status = static_cast<int>(hipGetDevice(&device));
+  if (status == 0)
+    status = static_cast<int>(
+        hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device));
+  if (status != 0) return status;
+  auto rounds = [&](long long workgroups) { return (workgroups + units - 1) / units; };
+  if (rounds(heads * SLICES / 2) < rounds(heads * SLICES))
+    gdn_chunk_scan<2><<<static_cast<unsigned>(heads * SLICES / 2), scan_threads(2), 0, stream>>>(a);
+  else
+    gdn_chunk_scan<1><<<static_cast<unsigned>(heads * SLICES), scan_threads(1), 0, stream>>>(a);
   return launch_status();
 }
 

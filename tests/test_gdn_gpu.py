@@ -374,3 +374,24 @@ def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T):
         one = torch.zeros((1, vh, kd, vd), device="cuda")
         want = capi.gdn_layer_forward(p, qkv[i:i + 1], z[i:i + 1], a[i:i + 1], b[i:i + 1], *weights, one)
         assert torch.equal(got[i], want[0]) and torch.equal(state[i], one[0]), i
+
+
+@pytest.mark.parametrize("T", [1, 64, 65, 200, 449])
+def test_scan_with_two_slices_a_workgroup(capi, T):
+    """48 heads are more single slices than compute units, so a workgroup walks two of
+    them; the 16 heads of one sequence alone take one each.  Bit for bit the same."""
+    B, H, d = 3, 16, 128
+    p = capi.delta_params(H, H, d, d)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda")
+    q, k, v = (values(B, T, H, d).to(torch.bfloat16) for _ in range(3))
+    g, beta = -torch.nn.functional.softplus(values(B, T, H)), torch.sigmoid(values(B, T, H))
+    start = values(B, H, d, d)
+    state = start.clone()
+    got = capi.gdn_scan(p, q, k, v, g, beta, state, normalize_qk=True, q_scale=d ** -0.5)
+    for i in range(B):
+        one = start[i:i + 1].clone()
+        want = capi.gdn_scan(p, *(x[i:i + 1] for x in (q, k, v, g, beta)), one, normalize_qk=True,
+                             q_scale=d ** -0.5)
+        assert torch.equal(got[i], want[0]) and torch.equal(state[i], one[0]), i
