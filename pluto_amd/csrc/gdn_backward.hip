@@ -22,6 +22,7 @@
 // row, added up by one thread per row).  What a token reads from global memory
 // is requested one token ahead.
 #include "gdn.h"
+#include "mfma_tile.h"
 
 namespace pluto_hip {
 namespace {
@@ -99,6 +100,190 @@ conv_train_kernel(const uint16_t* input, const float* __restrict__ weight, int l
   }
   store_floats<VEC>(pre + 1LL * t * channels + c, sum);
   store_floats<VEC>(post + 1LL * t * channels + c, activated);
+}
+
+// ---- four taps ---------------------------------------------------------------
+// The convolution and its backward with the taps' rows in registers: a thread owns
+// VEC channels and walks a run of tokens.  ALIGNED: rows and weights may be
+// accessed VEC elements at once.
+template <int VEC, bool ALIGNED>
+__device__ inline void read_bf16(const uint16_t* p, float (&x)[VEC]) {
+  static_assert(VEC == 2 || VEC == 4);
+  if constexpr (ALIGNED) {
+    uint32_t words[VEC / 2];
+    if constexpr (VEC == 4) {
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
+      words[0] = v.x, words[1] = v.y;
+    } else {
+      words[0] = *reinterpret_cast<const uint32_t*>(p);
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+      x[e] = __uint_as_float(e % 2 ? words[e / 2] & 0xffff0000u : words[e / 2] << 16);
+  } else {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) x[e] = bf16_bits_to_float(p[e]);
+  }
+}
+template <int VEC, bool ALIGNED>
+__device__ inline void read_taps(const float* weight, int c, float (&w)[VEC][4]) {
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    const float* p = weight + 4LL * (c + e);
+    if constexpr (ALIGNED) {
+      const float4 v = *reinterpret_cast<const float4*>(p);
+      w[e][0] = v.x, w[e][1] = v.y, w[e][2] = v.z, w[e][3] = v.w;
+    } else {
+#pragma unroll
+      for (int tap = 0; tap < 4; ++tap) w[e][tap] = p[tap];
+    }
+  }
+}
+
+// post = SiLU(conv(input)) as FP32, both rounded to bf16 on request.  (One channel
+// and one token a thread, four loads each, took 108 us at 2048 tokens of 10240
+// channels; in and out are 126 MB.)
+constexpr int kConvRun = 8;
+template <bool ALIGNED>
+__global__ void __launch_bounds__(256)
+conv_train4_kernel(const uint16_t* __restrict__ input, const float* __restrict__ weight, int length,
+                   int channels, bool round, float* __restrict__ post) {
+  constexpr int VEC = 4;
+  const int c = (blockIdx.x * 256 + threadIdx.x) * VEC, t0 = blockIdx.y * kConvRun;
+  if (c >= channels) return;
+  float w[VEC][4], x[4][VEC];
+  read_taps<VEC, ALIGNED>(weight, c, w);
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    read_bf16<VEC, ALIGNED>(input + 1LL * max(t0 - 3 + j, 0) * channels + c, x[j]);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) x[j][e] = t0 - 3 + j >= 0 ? x[j][e] : 0.0f;
+  }
+  float rows[kConvRun][VEC];
+#pragma unroll
+  for (int r = 0; r < kConvRun; ++r)
+    read_bf16<VEC, ALIGNED>(input + 1LL * min(t0 + r, length - 1) * channels + c, rows[r]);
+#pragma unroll
+  for (int r = 0; r < kConvRun; ++r) {
+    float out[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      x[3][e] = rows[r][e];
+      float sum = 0.0f;
+#pragma unroll
+      for (int tap = 0; tap < 4; ++tap) sum += x[tap][e] * w[e][tap];
+      sum = round_if(sum, round);
+      out[e] = round_if(sum / (1.0f + expf(-sum)), round);
+      x[0][e] = x[1][e], x[1][e] = x[2][e], x[2][e] = x[3][e];
+    }
+    if (t0 + r < length)
+      *reinterpret_cast<float4*>(post + 1LL * (t0 + r) * channels + c) =
+          make_float4(out[0], out[1], out[2], out[3]);
+  }
+}
+
+// Everything behind the gradient of `post` in one pass: back through SiLU (with
+// the convolution repeated instead of stored), the input's gradient, and this run's
+// share of the weights' gradient.  The q and k channels' gradient is the sum of
+// their value heads' partials, in ascending order.  (As five kernels that stored
+// the convolution, the gathered and the inner gradient: 258 us at 2048 tokens of
+// 10240 channels; what it cannot do without is 290 MB.)
+struct ConvBackwardArgs {
+  const uint16_t* input = nullptr;
+  const float* weight = nullptr;
+  const float* qk_partials = nullptr;  // [T, vh, tiles, 2, kd]
+  const float* dpost = nullptr;        // [T, channels]: the value channels
+  float* dx = nullptr;
+  float* partial = nullptr;  // optional [runs, channels, 4]
+  int length = 0, channels = 0, kh = 0, vh = 0, kd = 0, tiles = 0, run = 0;
+  bool round = true;
+};
+template <bool ALIGNED>
+__global__ void __launch_bounds__(256)
+conv_backward4_kernel(ConvBackwardArgs a) {
+  constexpr int VEC = 2;
+  const int c = (blockIdx.x * 256 + threadIdx.x) * VEC;
+  if (c >= a.channels) return;
+  const int t0 = blockIdx.y * a.run, t1 = min(t0 + a.run, a.length);
+  const int keys = a.kh * a.kd, group = a.vh / a.kh;
+  const bool gathered = c < 2 * keys;
+  // where a token's partials of these channels start, and how they continue
+  const int key_head = c % keys / a.kd, channel = c % a.kd;
+  const float* gather = a.qk_partials + (1LL * key_head * group * a.tiles * 2 + (c >= keys ? 1 : 0)) * a.kd + channel;
+  const long long gather_token = 2LL * a.vh * a.tiles * a.kd;
+  float w[VEC][4];
+  read_taps<VEC, ALIGNED>(a.weight, c, w);
+  float x[4][VEC], d[4][VEC], dw[VEC][4];  // rows t - 3 .. t of the input, of the inner gradient
+#pragma unroll
+  for (int e = 0; e < VEC; ++e)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) d[j][e] = dw[e][j] = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    read_bf16<VEC, ALIGNED>(a.input + 1LL * max(t0 - 3 + j, 0) * a.channels + c, x[j]);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) x[j][e] = t0 - 3 + j >= 0 ? x[j][e] : 0.0f;
+  }
+  // a token's gradient and input, requested two tokens ahead
+  auto fetch = [&](int t, float (&input)[VEC], float (&upstream)[VEC]) {
+    const int row = min(t, a.length - 1);
+    read_bf16<VEC, ALIGNED>(a.input + 1LL * row * a.channels + c, input);
+    float2 g = *reinterpret_cast<const float2*>(
+        gathered ? gather + row * gather_token : a.dpost + 1LL * row * a.channels + c);
+    if (gathered) {
+      for (int part = 1; part < group * a.tiles; ++part) {
+        const float2 v = *reinterpret_cast<const float2*>(gather + row * gather_token + 2LL * part * a.kd);
+        g.x += v.x, g.y += v.y;
+      }
+    }
+    upstream[0] = g.x, upstream[1] = g.y;
+  };
+  float next_x[2][VEC], next_g[2][VEC];
+  fetch(t0, next_x[0], next_g[0]);
+  fetch(t0 + 1, next_x[1], next_g[1]);
+  // rows t1 .. t1 + 2 only complete the gradients of the rows before them
+#pragma unroll 2
+  for (int t = t0; t < t1 + 3; ++t) {
+    float upstream[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) x[3][e] = next_x[0][e], upstream[e] = next_g[0][e];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) next_x[0][e] = next_x[1][e], next_g[0][e] = next_g[1][e];
+    fetch(t + 2, next_x[1], next_g[1]);
+    float out[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      float pre = 0.0f;
+#pragma unroll
+      for (int tap = 0; tap < 4; ++tap) pre += x[tap][e] * w[e][tap];
+      pre = round_if(pre, a.round);
+      const float sigmoid = 1.0f / (1.0f + expf(-pre));
+      d[3][e] = t < a.length ? upstream[e] * sigmoid * (1.0f + pre * (1.0f - sigmoid)) : 0.0f;
+      out[e] = 0.0f;
+#pragma unroll
+      for (int tap = 0; tap < 4; ++tap) {
+        out[e] += d[3 - tap][e] * w[e][tap];
+        if (t < t1) dw[e][tap] += d[3][e] * x[tap][e];
+      }
+    }
+    if (t - 3 >= t0) {
+      float* p = a.dx + 1LL * (t - 3) * a.channels + c;
+      if constexpr (ALIGNED) {
+        *reinterpret_cast<float2*>(p) = make_float2(out[0], out[1]);
+      } else {
+        p[0] = out[0], p[1] = out[1];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) x[j][e] = x[j + 1][e], d[j][e] = d[j + 1][e];
+  }
+  if (!a.partial) return;
+#pragma unroll
+  for (int e = 0; e < VEC; ++e)
+    *reinterpret_cast<float4*>(a.partial + (1LL * blockIdx.y * a.channels + c + e) * 4) =
+        make_float4(dw[e][0], dw[e][1], dw[e][2], dw[e][3]);
 }
 
 struct RecurrenceArgs {
@@ -422,6 +607,94 @@ output_backward_kernel(const float* core, const uint16_t* z, const float* __rest
   }
 }
 
+// The same for rows of 128: sixteen lanes a row, eight channels a lane; a workgroup
+// walks rows `blocks` runs of sixteen apart and keeps its share of the norm weight's
+// gradient in registers.  WIDE: the caller's tensors are 16-byte aligned.
+constexpr int kOutputBlocks = 1024;
+template <bool WIDE>
+__global__ void __launch_bounds__(256)
+output_backward128_kernel(const float* __restrict__ core, const uint16_t* __restrict__ z,
+                          const float* __restrict__ norm, const float* __restrict__ dy,
+                          long long rows, float epsilon, bool round, float* __restrict__ dcore,
+                          float* __restrict__ dz, float* __restrict__ norm_partial) {
+  __shared__ float sums[16][128];
+  const int c = 8 * (threadIdx.x % 16), slot = threadIdx.x / 16;
+  float weight[8], total[8];
+  load8<WIDE>(norm + c, weight);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) total[e] = 0.0f;
+  for (long long first = 16LL * blockIdx.x; first < rows; first += 16LL * gridDim.x) {
+    const bool exists = first + slot < rows;
+    const long long at = (exists ? first + slot : rows - 1) * 128 + c;
+    float x[8], gate[8], grad[8], sigmoid[8], dn[8];
+    load8<true>(core + at, x);
+    load8<WIDE>(z + at, gate);
+    load8<WIDE>(dy + at, grad);
+    float squares = 0.0f, dot = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      sigmoid[e] = 1.0f / (1.0f + expf(-gate[e]));
+      dn[e] = grad[e] * gate[e] * sigmoid[e] * weight[e];
+      squares += x[e] * x[e];
+      dot += dn[e] * x[e];
+    }
+#pragma unroll
+    for (int offset = 8; offset > 0; offset >>= 1) {
+      squares += __shfl_xor(squares, offset, 64);
+      dot += __shfl_xor(dot, offset, 64);
+    }
+    if (!exists) continue;
+    const float inverse = rsqrtf(squares / 128.0f + epsilon);
+    const float cubic = inverse * inverse * inverse / 128.0f * dot;
+    float dx[8], dgate[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float normalized = round_if(x[e] * inverse, round);
+      const float affine = round_if(normalized * weight[e], round);
+      dx[e] = inverse * dn[e] - x[e] * cubic;
+      dgate[e] = grad[e] * affine * sigmoid[e] * (1.0f + gate[e] * (1.0f - sigmoid[e]));
+      total[e] += grad[e] * gate[e] * sigmoid[e] * normalized;
+    }
+    store8<true>(dcore + at, dx);
+    store8<WIDE>(dz + at, dgate);
+  }
+  if (!norm_partial) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sums[slot][c + e] = total[e];
+  __syncthreads();
+  if (threadIdx.x < 128) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum += sums[i][threadIdx.x];
+    norm_partial[128LL * blockIdx.x + threadIdx.x] = sum;
+  }
+}
+
+// gradient[c] += sum over rows of parts[row, c], eight columns a workgroup, 128
+// threads a column, in a fixed order.
+__global__ void __launch_bounds__(1024)
+sum_columns_kernel(const float* parts, int rows, int width, float* gradient) {
+  __shared__ float sums[128][8], groups[16][8];
+  const int k = threadIdx.x % 8, g = threadIdx.x / 8, c = blockIdx.x * 8 + k;
+  float sum = 0.0f;
+  if (c < width)
+    for (int row = g; row < rows; row += 128) sum += parts[1LL * row * width + c];
+  sums[g][k] = sum;
+  __syncthreads();
+  if (g < 16) {
+    float total = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) total += sums[8 * g + i][k];
+    groups[g][k] = total;
+  }
+  __syncthreads();
+  if (g != 0 || c >= width) return;
+  float total = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) total += groups[i][k];
+  gradient[c] += total;
+}
+
 // Heads of a key head and their column tiles add up, in ascending order.
 __global__ void __launch_bounds__(128)
 gather_qk_kernel(const float* partials, int kh, int vh, int kd, int tiles, int channels,
@@ -534,6 +807,7 @@ conv_weight_final_kernel(const float* partial, long long elements, int slices, f
   const long long i = blockIdx.x * 256LL + threadIdx.x;
   if (i >= elements) return;
   float sum = 0.0f;
+#pragma unroll 16
   for (int slice = 0; slice < slices; ++slice) sum += partial[slice * elements + i];
   dw[i] += sum;
 }
@@ -586,6 +860,11 @@ namespace {
 bool use_chunks(const pluto_hip_delta_params* p) {
   return !force_generic() && gdn_backward_chunked_supported(p);
 }
+// Whether the kernels for four taps serve these widths.
+bool four_taps(const pluto_hip_delta_params* p) {
+  const int channels = 2 * p->key_heads * p->key_head_dim + p->value_heads * p->value_head_dim;
+  return p->conv_kernel_dim == 4 && channels % 4 == 0 && p->key_head_dim % 2 == 0;
+}
 }  // namespace
 
 size_t gdn_backward_workspace_bytes(const pluto_hip_delta_params* p, int length, bool norm_grad) {
@@ -595,13 +874,17 @@ size_t gdn_backward_workspace_bytes(const pluto_hip_delta_params* p, int length,
   const bool chunked = use_chunks(p);
   const size_t tiles = chunked ? 1 : (vd + kColumns - 1) / kColumns;
   size_t bytes = 0;
-  bytes += 4 * align_up(T * channels * 4, 256);          // pre, post, dpost, dpre
+  // post, dpost, and what only the general convolution stores: pre, dpre
+  bytes += (four_taps(p) ? 2 : 4) * align_up(T * channels * 4, 256);
   bytes += 2 * align_up(T * vh * vd * 4, 256);           // core, dcore
   bytes += chunked ? gdn_backward_chunked_bytes(p, length)
                    : align_up((T + 1) * vh * kd * vd * 4, 256);  // states
   bytes += align_up(T * vh * tiles * 2 * kd * 4, 256);   // q/k partials
   bytes += align_up(T * vh * tiles * 3 * 4, 256);        // scalar partials
-  if (norm_grad) bytes += align_up(T * vh * vd * 4, 256) + align_up(kGdnSumChunks * vd * 4, 256);
+  if (norm_grad && vd == 128)
+    bytes += align_up(kOutputBlocks * vd * 4, 256);
+  else if (norm_grad)
+    bytes += align_up(T * vh * vd * 4, 256) + align_up(kGdnSumChunks * vd * 4, 256);
   bytes += align_up(kConvSlices * channels * p->conv_kernel_dim * 4, 256);  // conv weight partials
   return bytes;
 }
@@ -625,24 +908,38 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     at += align_up(bytes, 256);
     return reinterpret_cast<float*>(result);
   };
-  float* pre = take(T * channels * 4);
+  const bool taps4 = four_taps(p);
+  float* pre = taps4 ? nullptr : take(T * channels * 4);
   float* post = take(T * channels * 4);
   float* dpost = take(T * channels * 4);
-  float* dpre = take(T * channels * 4);
+  float* dpre = taps4 ? nullptr : take(T * channels * 4);
   float* core = take(T * vh * vd * 4);
   float* dcore = take(T * vh * vd * 4);
   float* states = take(chunked ? gdn_backward_chunked_bytes(p, length) : (T + 1) * vh * kd * vd * 4);
   float* qk_partials = take(T * vh * tiles * 2 * kd * 4);
   float* scalar_partials = take(T * vh * tiles * 3 * 4);
-  float* norm_partials = d_norm ? take(T * vh * vd * 4) : nullptr;
-  float* norm_chunks = d_norm ? take(static_cast<size_t>(kGdnSumChunks) * vd * 4) : nullptr;
+  float* norm_partials =
+      d_norm ? take((vd == 128 ? static_cast<size_t>(kOutputBlocks) : T * vh) * vd * 4) : nullptr;
+  float* norm_chunks =
+      d_norm && vd != 128 ? take(static_cast<size_t>(kGdnSumChunks) * vd * 4) : nullptr;
   float* conv_partials = take(static_cast<size_t>(kConvSlices) * channels * kernel * 4);
 
   const long long elements = 1LL * length * channels;
   // one channel a thread: four a thread (one wide access instead of four) was
   // measured slower for the two kernels that also read the weights
-  conv_train_kernel<1><<<blocks_for(elements), 256, 0, stream>>>(
-      static_cast<const uint16_t*>(qkv), conv_weight, length, channels, kernel, round, pre, post);
+  auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+  const bool rows_aligned = aligned(qkv) && aligned(conv_weight) && aligned(dqkv);
+  if (taps4) {
+    const dim3 grid((channels / 4 + 255) / 256, (length + kConvRun - 1) / kConvRun);
+    const auto* input = static_cast<const uint16_t*>(qkv);
+    if (rows_aligned)
+      conv_train4_kernel<true><<<grid, 256, 0, stream>>>(input, conv_weight, length, channels, round, post);
+    else
+      conv_train4_kernel<false><<<grid, 256, 0, stream>>>(input, conv_weight, length, channels, round, post);
+  } else {
+    conv_train_kernel<1><<<blocks_for(elements), 256, 0, stream>>>(
+        static_cast<const uint16_t*>(qkv), conv_weight, length, channels, kernel, round, pre, post);
+  }
   int status = launch_status();
   if (status != 0) return status;
   RecurrenceArgs r;
@@ -686,12 +983,25 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     status = launch_status();
   }
   if (status != 0) return status;
-  output_backward_kernel<<<static_cast<unsigned>(length) * vh, 64, 0, stream>>>(
-      core, static_cast<const uint16_t*>(z), norm, dy, vd, p->rms_norm_epsilon, round, dcore, dz,
-      norm_partials);
+  if (vd == 128) {
+    const long long rows = 1LL * length * vh, runs = (rows + 15) / 16;
+    const int blocks = static_cast<int>(runs < kOutputBlocks ? runs : kOutputBlocks);
+    const auto* gates = static_cast<const uint16_t*>(z);
+    if (aligned(z) && aligned(norm) && aligned(dy) && aligned(dz))
+      output_backward128_kernel<true><<<blocks, 256, 0, stream>>>(
+          core, gates, norm, dy, rows, p->rms_norm_epsilon, round, dcore, dz, norm_partials);
+    else
+      output_backward128_kernel<false><<<blocks, 256, 0, stream>>>(
+          core, gates, norm, dy, rows, p->rms_norm_epsilon, round, dcore, dz, norm_partials);
+    if (d_norm) sum_columns_kernel<<<16, 1024, 0, stream>>>(norm_partials, blocks, vd, d_norm);
+  } else {
+    output_backward_kernel<<<static_cast<unsigned>(length) * vh, 64, 0, stream>>>(
+        core, static_cast<const uint16_t*>(z), norm, dy, vd, p->rms_norm_epsilon, round, dcore, dz,
+        norm_partials);
+  }
   status = launch_status();
   if (status != 0) return status;
-  if (d_norm) {
+  if (d_norm && vd != 128) {
     sum_rows_partial_kernel<<<kGdnSumChunks, 256, 0, stream>>>(norm_partials, 1LL * length * vh, vd,
                                                                kGdnSumChunks, norm_chunks);
     sum_rows_final_kernel<<<1, 256, 0, stream>>>(norm_chunks, kGdnSumChunks, vd, d_norm);
@@ -705,10 +1015,41 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     status = launch_status();
   }
   if (status != 0) return status;
-  gather_qk_kernel<<<dim3(kh, length), 128, 0, stream>>>(qk_partials, kh, vh, kd, tiles, channels,
-                                                         dpost);
   gather_scalar_kernel<<<vh, 256, 0, stream>>>(scalar_partials, length, vh, tiles, da, db, d_a_log,
                                                d_dt_bias);
+  const long long weights = 1LL * channels * kernel;
+  if (taps4) {
+    ConvBackwardArgs b;
+    b.input = static_cast<const uint16_t*>(qkv);
+    b.weight = conv_weight;
+    b.qk_partials = qk_partials;
+    b.dpost = dpost;
+    b.dx = dqkv;
+    b.partial = d_conv_weight ? conv_partials : nullptr;
+    b.length = length;
+    b.channels = channels;
+    b.kh = kh;
+    b.vh = vh;
+    b.kd = kd;
+    b.tiles = tiles;
+    // a run repeats three rows of the next one: sixteen tokens at least, and no
+    // more runs than there are slices of partial sums
+    b.run = (length + kConvSlices - 1) / kConvSlices;
+    if (b.run < 16) b.run = 16;
+    b.round = round;
+    const int runs = (length + b.run - 1) / b.run;
+    const dim3 grid((channels / 2 + 255) / 256, runs);
+    if (rows_aligned)
+      conv_backward4_kernel<true><<<grid, 256, 0, stream>>>(b);
+    else
+      conv_backward4_kernel<false><<<grid, 256, 0, stream>>>(b);
+    if (d_conv_weight)
+      conv_weight_final_kernel<<<blocks_for(weights), 256, 0, stream>>>(conv_partials, weights, runs,
+                                                                        d_conv_weight);
+    return launch_status();
+  }
+  gather_qk_kernel<<<dim3(kh, length), 128, 0, stream>>>(qk_partials, kh, vh, kd, tiles, channels,
+                                                         dpost);
   if (elements % 4 == 0)
     conv_silu_backward_kernel<4><<<blocks_for(elements / 4), 256, 0, stream>>>(pre, dpost, elements,
                                                                                dpre);
@@ -721,7 +1062,6 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     conv_weight_partial_kernel<<<dim3((channels + 255) / 256, kernel, kConvSlices), 256, 0, stream>>>(
         static_cast<const uint16_t*>(qkv), dpre, length, channels, kernel, kConvSlices,
         conv_partials);
-    const long long weights = 1LL * channels * kernel;
     conv_weight_final_kernel<<<blocks_for(weights), 256, 0, stream>>>(conv_partials, weights,
                                                                       kConvSlices, d_conv_weight);
   }
