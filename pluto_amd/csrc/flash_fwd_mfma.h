@@ -29,7 +29,13 @@ struct FlashForwardArgs {
   int query_heads = 0;
   int group = 1;
   float scale = 1.0f;
+  // Optional room for split keys (flash_forward_split_bytes), one sequence only.
+  void* partial = nullptr;
 };
+
+// Scratch for the partial results of any call with these rows and at most kv_rows
+// keys; 0: never split.
+size_t flash_forward_split_bytes(int head_dim, int q_rows, int kv_rows);
 
 bool flash_forward_supported(const FlashForwardArgs& args, int head_dim);
 int launch_flash_forward(hipStream_t stream, const FlashForwardArgs& args,
@@ -38,5 +44,9 @@ int launch_flash_forward(hipStream_t stream, const FlashForwardArgs& args,
 // main loop; what launch_flash_forward picks for long sequences.
 int launch_flash_forward_pipelined(hipStream_t stream, const FlashForwardArgs& args,
                                    int head_dim, int sequences);
+// The same kernels where splitting the keys of query tiles brings the call's end
+// closer (a.partial is set): false when it does not, and nothing was launched.
+bool launch_flash_forward_split(hipStream_t stream, const FlashForwardArgs& args, int head_dim,
+                                int* status);
 
 }  // namespace pluto_hip

@@ -436,6 +436,11 @@ int launch_flash_forward(hipStream_t stream, const FlashForwardArgs& a,
   const dim3 grid(static_cast<unsigned>(blocks));
   const int unit_count = static_cast<int>(units);
   if (!kernel_enabled(kMainKernel)) return 0;
+  if (a.partial && sequences == 1 && kernel_enabled(kEightWave) && !a.core && !a.maxima &&
+      !a.normalizers) {
+    int status = 0;
+    if (launch_flash_forward_split(stream, a, head_dim, &status)) return status;
+  }
   // Long sequences take the kernel with the hand-scheduled loop
   // (flash_fwd_pipelined.hip): tiles of 256 rows (128 at head widths 64 and
   // 256), which short sequences do not fill.  Its epilogue addresses a head's rows through

@@ -21,6 +21,9 @@
 #include "mfma_tile.h"
 
 #include <algorithm>
+#include <functional>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 namespace pluto_hip {
@@ -55,10 +58,42 @@ template <int D>
 constexpr int kWaves = D == 256 ? FLASH_LOOP_D256_WAVES
                                 : (D == 128 ? FLASH_LOOP_D128_WAVES : FLASH_LOOP_D64_WAVES);
 
-template <int D>
+// Lists whose entries may be a part of a query tile's keys, for a single sequence
+// with too few tiles, or too even ones, to share out whole (34 rows of 24 heads
+// behind 7336 keys are 24 tiles: 332 us whole, 36 with the combining kernel in
+// parts).  An entry is keys 64 begin up to 64 end of a tile; its
+// slot says where its partial result goes (unnormalised output rows, the reference
+// point of their exponents and their sums), kNoItem that it is the whole tile.  The
+// entries of a tile except the last end before the causal mask of its first row does,
+// so every entry sees a key of every row.  All partitions of the kv heads over the
+// XCDs have the same lists.
+constexpr int kSplitEntries = 384, kSplitLists = 256;
+struct SplitEntry {
+  uint16_t tile, begin, end, slot;  // tile: head within the partition * q_tiles + q_tile
+};
+struct SplitScratch {
+  float* rows = nullptr;      // [partitions, slots, slot_rows, D]
+  float2* stats = nullptr;    // [partitions, slots, slot_rows]
+  int slots = 0, slot_rows = 0;
+  int partitions = 1;
+};
+struct Split : SplitScratch {
+  uint16_t first[kSplitLists + 1];  // list j is entries first[j] to first[j + 1] - 1
+  SplitEntry entry[kSplitEntries];
+};
+// The tiles in parts, for the kernel that puts them together.
+struct SplitTiles {
+  int count = 0;
+  struct {
+    uint16_t tile, slot, parts;  // slots slot to slot + parts - 1
+  } tile[kSplitEntries / 2];
+};
+
+template <int D, bool SPLIT>
 __global__ void __launch_bounds__(64 * kWaves<D>)
 __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, D == 256 ? 1 : 2)))
-flash_forward_pipelined_kernel(FlashForwardArgs a_in, int unit_count, Schedule schedule) {
+flash_forward_pipelined_kernel(FlashForwardArgs a_in, int unit_count,
+                               std::conditional_t<SPLIT, Split, Schedule> schedule) {
   struct Args : FlashForwardArgs {
     int unit_count;
   } a;
@@ -80,16 +115,35 @@ flash_forward_pipelined_kernel(FlashForwardArgs a_in, int unit_count, Schedule s
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
   const int q_tiles = (a.q_rows + BM - 1) / BM;
-  const int list_length = schedule.slots > 0 ? schedule.slots : 1;
-  for (int entry = 0; entry < list_length; ++entry) {
-  int q_tile, head, seq;
-  if (schedule.slots > 0) {
-    const int item = schedule.item[blockIdx.x * schedule.slots + entry];
-    if (item == kNoItem) break;
-    q_tile = item % q_tiles;
-    const int column = item / q_tiles;
-    head = column % a.query_heads;
-    seq = column / a.query_heads;
+  int entry = 0, list_end, partition = 0;
+  if constexpr (SPLIT) {
+    const int xcd = blockIdx.x % 8;
+    partition = xcd % schedule.partitions;
+    const int list = blockIdx.x / 8 * (8 / schedule.partitions) + xcd / schedule.partitions;
+    entry = schedule.first[list], list_end = schedule.first[list + 1];
+  } else {
+    list_end = schedule.slots > 0 ? schedule.slots : 1;
+  }
+  for (; entry < list_end; ++entry) {
+  int q_tile, head, seq, key_begin = 0, key_end = 0, slot = kNoItem;
+  bool listed = SPLIT;
+  if constexpr (!SPLIT) listed = schedule.slots > 0;
+  if (listed) {
+    if constexpr (SPLIT) {
+      const SplitEntry part = schedule.entry[entry];
+      q_tile = part.tile % q_tiles;
+      const int local = part.tile / q_tiles;
+      head = (partition + schedule.partitions * (local / a.group)) * a.group + local % a.group;
+      seq = 0;
+      key_begin = part.begin * BN, key_end = part.end * BN, slot = part.slot;
+    } else {
+      const int item = schedule.item[blockIdx.x * schedule.slots + entry];
+      if (item == kNoItem) break;
+      q_tile = item % q_tiles;
+      const int column = item / q_tiles;
+      head = column % a.query_heads;
+      seq = column / a.query_heads;
+    }
   } else {
     // The query heads of a kv head at one query tile run on one XCD (workgroup
     // i lands on XCD i mod 8, each with a private L2), heaviest tiles first.
@@ -107,6 +161,12 @@ flash_forward_pipelined_kernel(FlashForwardArgs a_in, int unit_count, Schedule s
   const uint16_t* q_base = a.q + seq * a.q_seq_stride + head * a.q_head_stride;
   const uint16_t* k_base = a.k + seq * a.k_seq_stride + kv_head * a.k_head_stride;
   const uint16_t* v_base = a.v + seq * a.v_seq_stride + kv_head * a.v_head_stride;
+  if constexpr (SPLIT) {
+    k_base += key_begin * a.k_row_stride;
+    v_base += key_begin * a.v_row_stride;
+    a.kv_rows = min(key_end, a_in.kv_rows) - key_begin;
+    a.start_position = a_in.start_position - key_begin;
+  }
   const float scale2 = a.scale * kLog2e;
   // the loop statement takes the factor as a scalar operand
   const uint32_t scale2_bits = __builtin_amdgcn_readfirstlane(__float_as_uint(scale2));
@@ -303,6 +363,31 @@ flash_forward_pipelined_kernel(FlashForwardArgs a_in, int unit_count, Schedule s
     }
   }
   // ---- epilogue ------------------------------------------------------------------
+  bool partial = false;
+  if constexpr (SPLIT) partial = slot != kNoItem;
+  if (partial) {
+    if constexpr (SPLIT) {
+    constexpr uint32_t kDropped = 0x7fffffffu;
+    const long long at = (static_cast<long long>(partition) * schedule.slots + slot) * schedule.slot_rows;
+    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+        schedule.rows + at * D, 0, schedule.slot_rows * D * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t stats = __builtin_amdgcn_make_buffer_rsrc(
+        schedule.stats + at, 0, schedule.slot_rows * 8, 0x00020000);
+    const int row = 32 * wave + n;
+    const uint32_t row_at = q_row < a.q_rows ? static_cast<uint32_t>(row * D * 4 + 16 * h) : kDropped;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32x4 words = {__float_as_uint(o_acc[db][4 * j]), __float_as_uint(o_acc[db][4 * j + 1]),
+                                __float_as_uint(o_acc[db][4 * j + 2]), __float_as_uint(o_acc[db][4 * j + 3])};
+        __builtin_amdgcn_raw_buffer_store_b128(words, rows, row_at, 128 * db + 32 * j, 0);
+      }
+    const uint32x2 pair = {__float_as_uint(m_used), __float_as_uint(l_acc[0])};
+    __builtin_amdgcn_raw_buffer_store_b64(
+        pair, stats, q_row < a.q_rows && h == 0 ? static_cast<uint32_t>(row * 8) : kDropped, 0, 0);
+    }
+  } else
   // The arithmetic of flash_forward_kernel's epilogue.  Every access goes
   // through a bounds-checked buffer descriptor instead of a branch: rows past
   // the end (and, for the row statistics, the upper lane halves) get an
@@ -430,6 +515,64 @@ flash_forward_pipelined_kernel(FlashForwardArgs a_in, int unit_count, Schedule s
   // the next tile's fills must not overtake this tile's last LDS reads
   __syncthreads();
   }
+}
+
+// The parts of a row put together: D / 8 lanes a row, eight channels a lane.
+template <int D>
+__global__ void __launch_bounds__(256)
+flash_forward_combine_kernel(FlashForwardArgs a, SplitScratch split, SplitTiles tiles) {
+  constexpr int LANES = D / 8, BM = 32 * kWaves<D>;
+  const int q_tiles = (a.q_rows + BM - 1) / BM;
+  const int partition = blockIdx.y % split.partitions;
+  const auto tile = tiles.tile[blockIdx.y / split.partitions];
+  const int local = tile.tile / q_tiles;
+  const int head = (partition + split.partitions * (local / a.group)) * a.group + local % a.group;
+  const int c = 8 * (threadIdx.x % LANES);
+  const int tile_row = blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+  const int row = tile.tile % q_tiles * BM + tile_row;
+  if (tile_row >= split.slot_rows || row >= a.q_rows) return;
+  const long long at =
+      (static_cast<long long>(partition) * split.slots + tile.slot) * split.slot_rows + tile_row;
+  const int step = split.slot_rows;
+  float reference = kMasked;
+  for (int p = 0; p < tile.parts; ++p) reference = fmaxf(reference, split.stats[at + p * step].x);
+  float sum = 0.0f, o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = 0.0f;
+#pragma unroll 4
+  for (int p = 0; p < tile.parts; ++p) {
+    const float2 stat = split.stats[at + p * step];
+    float part[8];
+    load8<true>(split.rows + (at + p * step) * D + c, part);
+    const float weight = __builtin_amdgcn_exp2f(stat.x - reference);
+    sum += stat.y * weight;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] += part[e] * weight;
+  }
+  if (!(sum > 0.0f)) sum = 1.0f;
+  const float inverse = 1.0f / sum;
+  uint32_t words[4], gate_words[4] = {0, 0, 0, 0};
+  if (a.gate) {
+    const uint4 g = *reinterpret_cast<const uint4*>(a.gate + head * a.gate_head_stride +
+                                                    row * a.gate_row_stride + c);
+    gate_words[0] = g.x, gate_words[1] = g.y, gate_words[2] = g.z, gate_words[3] = g.w;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    words[i] = pack_bf16(o[2 * i] * inverse, o[2 * i + 1] * inverse);
+    // out = bf16(bf16(core) * bf16(sigmoid(gate))): qwen_attention.cc:103-108
+    if (a.gate)
+      words[i] = pack_bf16(
+          __uint_as_float(words[i] << 16) *
+              round_to_bf16(gate_sigmoid(__uint_as_float(gate_words[i] << 16))),
+          __uint_as_float(words[i] & 0xffff0000u) *
+              round_to_bf16(gate_sigmoid(__uint_as_float(gate_words[i] & 0xffff0000u))));
+  }
+  *reinterpret_cast<uint4*>(a.out + head * a.o_head_stride + row * a.o_row_stride + c) =
+      make_uint4(words[0], words[1], words[2], words[3]);
+  if (a.lse && c == 0)
+    a.lse[static_cast<long long>(row) * a.query_heads + head] =
+        reference * (1.0f / kLog2e) + __logf(sum);
 }
 
 }  // namespace
@@ -604,18 +747,184 @@ int launch_flash_forward_pipelined(hipStream_t stream, const FlashForwardArgs& a
   }
   if (scheduled_blocks > 0) blocks = scheduled_blocks;
   if (head_dim == 256)
-    flash_forward_pipelined_kernel<256>
+    flash_forward_pipelined_kernel<256, false>
         <<<dim3(static_cast<unsigned>(blocks)), 64 * kWaves<256>, 0, stream>>>(
             a, static_cast<int>(units), schedule);
   else if (head_dim == 128)
-    flash_forward_pipelined_kernel<128>
+    flash_forward_pipelined_kernel<128, false>
         <<<dim3(static_cast<unsigned>(blocks)), 64 * kWaves<128>, 0, stream>>>(
             a, static_cast<int>(units), schedule);
   else
-    flash_forward_pipelined_kernel<64>
+    flash_forward_pipelined_kernel<64, false>
         <<<dim3(static_cast<unsigned>(blocks)), 64 * kWaves<64>, 0, stream>>>(
             a, static_cast<int>(units), schedule);
   return launch_status();
+}
+
+// ---- host side: lists with tiles in parts -----------------------------------------------
+namespace {
+
+// A part shorter than this many key tiles is not worth its fixed part.
+constexpr int kShortestPart = 8;
+// Storing a partial result, in key tiles of time, and the launch and the reading of
+// the kernel that puts the parts together.
+constexpr int kPartCost = 3, kCombineCost = 6;
+
+static_assert(sizeof(FlashForwardArgs) + 8 + sizeof(Split) <= 4096, "kernel arguments");
+
+struct SplitPlan {
+  Split split;
+  SplitTiles tiles;
+  bool useful = false;
+};
+
+// Shares the tiles out so that no list exceeds `limit`: longest first, each to the
+// least loaded list as a whole while it fits there, in parts that fill up the least
+// loaded lists otherwise.
+bool share_out(const std::vector<int>& cost, const std::vector<int>& order, int lists, int limit,
+               SplitPlan* plan) {
+  std::vector<std::pair<int, int>> load(lists);  // a heap, the least loaded list on top
+  for (int j = 0; j < lists; ++j) load[j] = {0, j};
+  const auto above = std::greater<std::pair<int, int>>();
+  std::vector<std::pair<int, SplitEntry>> entries;
+  std::vector<int> cut;
+  for (int tile : order) {
+    if (load.front().first + cost[tile] > limit) {
+      cut.push_back(tile);
+      continue;
+    }
+    std::pop_heap(load.begin(), load.end(), above);
+    entries.push_back({load.back().second, {static_cast<uint16_t>(tile), 0,
+                                            static_cast<uint16_t>(cost[tile] - kFixedCost), kNoItem}});
+    load.back().first += cost[tile];
+    std::push_heap(load.begin(), load.end(), above);
+  }
+  const int slots_limit = kSplitEntries * lists / kSplitLists;  // kSplitEntries in all partitions
+  int slots = 0;
+  plan->tiles.count = 0;
+  for (int tile : cut) {
+    const int end = cost[tile] - kFixedCost;
+    const int first_slot = slots;
+    for (int begin = 0; begin < end;) {
+      std::pop_heap(load.begin(), load.end(), above);
+      const int room = limit - load.back().first - kFixedCost - kPartCost;
+      int length = std::min(room, end - begin);
+      if (length < end - begin && end - begin - length < kShortestPart)
+        length = end - begin - kShortestPart;
+      if (length < kShortestPart || slots == slots_limit) return false;
+      entries.push_back({load.back().second,
+                         {static_cast<uint16_t>(tile), static_cast<uint16_t>(begin),
+                          static_cast<uint16_t>(begin + length), static_cast<uint16_t>(slots++)}});
+      load.back().first += length + kFixedCost + kPartCost;
+      std::push_heap(load.begin(), load.end(), above);
+      begin += length;
+    }
+    plan->tiles.tile[plan->tiles.count++] = {static_cast<uint16_t>(tile),
+                                             static_cast<uint16_t>(first_slot),
+                                             static_cast<uint16_t>(slots - first_slot)};
+  }
+  if (entries.size() > static_cast<size_t>(kSplitEntries)) return false;
+  std::stable_sort(entries.begin(), entries.end(),
+                   [](const auto& x, const auto& y) { return x.first < y.first; });
+  size_t e = 0;
+  for (int j = 0; j < lists; ++j) {
+    plan->split.first[j] = static_cast<uint16_t>(e);
+    for (; e < entries.size() && entries[e].first == j; ++e) plan->split.entry[e] = entries[e].second;
+  }
+  plan->split.first[lists] = static_cast<uint16_t>(e);
+  plan->split.slots = slots;
+  return true;
+}
+
+void build_split(const ScheduleKey& k, SplitPlan* plan) {
+  plan->useful = false;
+  const int q_tiles = (k.q_rows + k.tile_rows - 1) / k.tile_rows;
+  const int kv_heads = k.query_heads / k.group;
+  // Rows that are more than half of the keys have light tiles that fill the gaps the
+  // heavy ones leave, and their results stay those of the other kernels to the bit.
+  if (k.workgroups != kSplitLists || k.kv_rows > BN * 0xffff || k.q_rows > k.kv_rows / 2) return;
+  const int partitions = kv_heads % 8 == 0 ? 8 : 8 % kv_heads == 0 ? kv_heads : 1;
+  const int lists = kSplitLists / partitions;
+  const long long items = 1LL * q_tiles * k.query_heads / partitions;
+  if (items > kSplitEntries) return;
+  std::vector<int> cost(items), order(items);
+  long long total = 0;
+  for (int i = 0; i < items; ++i) order[i] = i, total += cost[i] = tile_cost(k, i % q_tiles);
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+  // the time without parts: longest first
+  std::vector<int> load(lists, 0);
+  for (int tile : order) {
+    std::pop_heap(load.begin(), load.end(), std::greater<int>());
+    load.back() += cost[tile];
+    std::push_heap(load.begin(), load.end(), std::greater<int>());
+  }
+  int low = static_cast<int>(total / lists);
+  int high = *std::max_element(load.begin(), load.end()) - kCombineCost;
+  high -= high / 16;  // lists of whole tiles are packed better than this, and known to fit
+  low = std::max(low, kShortestPart + kFixedCost + kPartCost);
+  while (low <= high) {
+    const int limit = (low + high) / 2;
+    if (share_out(cost, order, lists, limit, plan))
+      plan->useful = true, high = limit - 1;
+    else
+      low = limit + 1;
+  }
+  if (!plan->useful) return;
+  share_out(cost, order, lists, high + 1, plan);
+  plan->useful = plan->split.slots > 0;
+  plan->split.partitions = partitions;
+  plan->split.slot_rows = std::min(k.tile_rows, k.q_rows);
+}
+
+}  // namespace
+
+size_t flash_forward_split_bytes(int head_dim, int q_rows, int kv_rows) {
+  if ((head_dim != 128 && head_dim != 256) || kv_rows < 2 * kShortestPart * BN) return 0;
+  const int tile_rows = 32 * (head_dim == 256 ? kWaves<256> : kWaves<128>);
+  return 1ull * kSplitEntries * std::min(tile_rows, q_rows) * (head_dim + 2) * 4;
+}
+
+bool launch_flash_forward_split(hipStream_t stream, const FlashForwardArgs& a, int head_dim,
+                                int* status) {
+  if (head_dim != 128 && head_dim != 256) return false;
+  const int tile_rows = 32 * (head_dim == 256 ? kWaves<256> : kWaves<128>);
+  // The lists depend on the shape only; a thread keeps the last ones it made.
+  thread_local ScheduleKey known;
+  thread_local SplitPlan plan;
+  ScheduleKey key;
+  key.q_rows = a.q_rows, key.kv_rows = a.kv_rows, key.start_position = a.start_position;
+  key.query_heads = a.query_heads, key.group = a.group, key.sequences = 1;
+  key.tile_rows = tile_rows;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess ||
+      hipDeviceGetAttribute(&key.workgroups, hipDeviceAttributeMultiprocessorCount, device) !=
+          hipSuccess)
+    return false;
+  if (!(key == known)) {
+    build_split(key, &plan);
+    known = key;
+  }
+  if (!plan.useful) return false;
+  Split& split = plan.split;
+  split.rows = static_cast<float*>(a.partial);
+  split.stats = reinterpret_cast<float2*>(
+      split.rows + 1ll * split.partitions * split.slots * split.slot_rows * head_dim);
+  const dim3 rows((split.slot_rows + 2048 / head_dim - 1) / (2048 / head_dim),
+                  plan.tiles.count * split.partitions);
+  if (head_dim == 256)
+    flash_forward_pipelined_kernel<256, true>
+        <<<kSplitLists, 64 * kWaves<256>, 0, stream>>>(a, 0, split);
+  else
+    flash_forward_pipelined_kernel<128, true>
+        <<<kSplitLists, 64 * kWaves<128>, 0, stream>>>(a, 0, split);
+  *status = launch_status();
+  if (*status != 0) return true;
+  if (head_dim == 256)
+    flash_forward_combine_kernel<256><<<rows, 256, 0, stream>>>(a, split, plan.tiles);
+  else
+    flash_forward_combine_kernel<128><<<rows, 256, 0, stream>>>(a, split, plan.tiles);
+  *status = launch_status();
+  return true;
 }
 
 }  // namespace pluto_hip

@@ -83,7 +83,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 size_t element_bytes(int dtype) { return dtype == PLUTO_HIP_BF16 ? 2 : 4; }
 
 struct PrefillLayout {
-  size_t cosines, sines, queries, total;
+  size_t cosines, sines, queries, partial, partial_bytes, total;
 };
 
 PrefillLayout prefill_layout(const pluto_hip_attention_params* p, int length) {
@@ -92,9 +92,13 @@ PrefillLayout prefill_layout(const pluto_hip_attention_params* p, int length) {
   l.cosines = 0;
   l.sines = table;
   l.queries = 2 * table;
-  l.total = l.queries + align_up(static_cast<size_t>(length) * p->query_heads * p->head_dim *
-                                     (p->round_to_bfloat16 ? 2 : 4),
-                                 256);
+  l.partial = l.queries + align_up(static_cast<size_t>(length) * p->query_heads * p->head_dim *
+                                       (p->round_to_bfloat16 ? 2 : 4),
+                                   256);
+  // whatever the start position: a sequence has at most `capacity` keys
+  l.partial_bytes =
+      p->round_to_bfloat16 ? flash_forward_split_bytes(p->head_dim, length, p->capacity) : 0;
+  l.total = l.partial + align_up(l.partial_bytes, 256);
   return l;
 }
 
@@ -326,6 +330,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
     f.query_heads = qh;
     f.group = qh / kh;
     f.scale = scale;
+    if (layout.partial_bytes > 0) f.partial = scratch + layout.partial;
     if (flash_forward_supported(f, d)) {
       note_path(PLUTO_HIP_PATH_FLASH);
       return launch_flash_forward(s, f, d, 1);

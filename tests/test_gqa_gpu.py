@@ -291,6 +291,40 @@ def test_config3_prefill_8192(capi, oracle):
     assert_close_bf16(got, out2.float().cpu().numpy(), "config 3 vs fp32-arithmetic kernel")
 
 
+@pytest.mark.parametrize("start,length,d", [(3999, 1, 256), (4032, 64, 256), (2000, 129, 256),
+                                            (1023, 33, 128), (5037, 257, 128), (3000, 700, 128)])
+def test_prefill_behind_a_long_cache_splits_its_keys(capi, oracle, start, length, d):
+    # A few query tiles behind many keys: every tile's keys are split into pieces
+    # (ends that are and are not multiples of the 64-key blocks, one and several
+    # query tiles, a ragged last one) and the partial results combined.  Against the
+    # unsplit kernels (which the mask selects) and the oracle.
+    qh, kh = 6, 2
+    total = start + length
+    p, po = both_params(capi, oracle, query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=32,
+                        capacity=total)
+    rng = np.random.default_rng(12)
+    qg, k, v = make_sequence(oracle, rng, total, qh, kh, d)
+    qw, kw_ = dev(values(d, 0.2, 0.3)), dev(values(d, 0.8, 0.4))
+    bf = torch.bfloat16
+    results = []
+    for mask in (0xffffffff, 0xffffffff & ~capi.EIGHT_WAVE):
+        cache = capi.KvCache(total, kh, d)
+        with capi.only_kernels(mask):
+            for piece in (slice(0, start), slice(start, total)):
+                out, lse = capi.gqa_prefill(p, dev(qg[piece], bf), dev(k[piece], bf),
+                                            dev(v[piece], bf), qw, kw_, cache,
+                                            start_position=piece.start, want_lse=True)
+                assert capi.last_path() == capi.PATH_FLASH
+        results.append((out.float().cpu().numpy(), lse.cpu().numpy()))
+    (split, split_lse), (whole, whole_lse) = results
+    assert_close_bf16(split, whole, "split keys against whole")
+    np.testing.assert_allclose(split_lse, whole_lse, rtol=1e-4)  # sums of bf16 weights
+    first = max(start, total - 3)
+    want = oracle.gqa_sequence(po, qg, k, v, values(d, 0.2, 0.3), values(d, 0.8, 0.4),
+                               rows=(first, total))
+    assert_close_bf16(split[first - start:], want["out"][first:total], "last rows")
+
+
 @pytest.mark.parametrize("lengths,d", [((2048,), 128), ((2301,), 128), ((2100, 2237), 128),
                                        ((1024,), 256), ((1301,), 256), ((1100, 1237), 256),
                                        ((33,), 256), ((130, 70), 256)])
