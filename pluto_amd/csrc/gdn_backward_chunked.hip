@@ -16,28 +16,29 @@
 //   O   = diag(E) Q^ S + P Dl
 //   S'  = E_63 S + (diag(L) K^)^T Dl
 // which is the recurrence S <- decay S; delta = beta (v - S^T k^); S += k^ x
-// delta; o = S^T q^ unrolled over the chunk.  Eliminating Dl, the state obeys
-// an affine recurrence whose matrices depend on one chunk only,
-//   S' = M S + B,     M = E_63 I - (diag(L) K^)^T W,    B = (diag(L) K^)^T U,
-// and so does its gradient:
-//   dS = M^T dS' + C,  C = Y^T dO,   Y = diag(E) Q^ - P W.
+// delta; o = S^T q^ unrolled over the chunk.  In reverse, from the gradient dS'
+// of the state leaving the chunk,
+//   dDl = P^T dO + diag(L) K^ dS'
+//   dS  = E_63 dS' + (diag(E) Q^)^T dO - W^T dDl.
 // The kernels, in launch order:
 //   chunk_prepare_kernel           T, W, U, P of every chunk          (parallel)
-//   chunk_transfer_kernel          M, M^T, B, Y                       (parallel)
-//   chunk_states_forward_kernel    S entering every chunk             (sequential)
-//   chunk_outputs_kernel           Dl and O from S                    (parallel)
+//   chunk_states_forward_kernel    S entering every chunk, Dl         (sequential)
+//   chunk_outputs_kernel           O                                  (parallel)
 //     -- the caller turns O into dO here --
-//   chunk_local_kernel             C                                  (parallel)
-//   chunk_states_backward_kernel   dS' leaving every chunk            (sequential)
-//   chunk_delta_gradient_kernel    dDl from dO and dS'                (parallel)
-//   chunk_state_products_kernel    dW and the state terms of dq^, dk^ (parallel)
-//   chunk_triangle_kernel          dP, dT, dA: the [64, 64] matrices  (parallel)
-//   chunk_finish_kernel            dq, dk, dv                         (parallel)
-//   chunk_gates_kernel             d beta, d log-decay -> da, db      (parallel)
-// The sequential kernels run one workgroup per (head, 16 value columns) and
-// do one 128 x 128 x 16 product a chunk, with the next chunk's matrix already
-// in registers.  Matrix products run on v_mfma_f32_32x32x2_f32; operands are
-// read straight from global memory or from LDS.
+//   chunk_states_backward_kernel   dS' leaving every chunk, dDl       (sequential)
+//   chunk_gradients_kernel         everything else                    (parallel)
+// The sequential kernels run one workgroup per (head, 16 value columns).
+// Eliminating Dl instead makes both recurrences one 128 x 128 matrix a chunk
+// (S' = M S + B) whose product is one link of the chain instead of two, but M, its
+// transpose, B and the offsets of the reverse recurrence are four 64 KiB records a
+// chunk that have to be computed, written and read: at 2048 tokens of 48 heads the
+// kernels that did so took 624 us where the two below take 380.
+// Everything between two states is consumed in the kernel that makes it (LDS and
+// accumulators), so that a chunk's records are 0.27 MB instead of 0.74 MB: all kernels
+// of this file 1766 -> 930 us at that size.
+// Matrix products run on v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32, whose
+// rate (about 25 GFLOP of them, 165 us of the card's FP32 matrix rate) bounds the
+// gradients kernel; the triangular factors are multiplied by halves.
 #include "gdn.h"
 
 namespace pluto_hip {
@@ -49,24 +50,23 @@ constexpr int kSlice = 16;   // value columns per workgroup of the sequential ke
 constexpr int kWide = kC * kD;     // elements of a [64, 128] record
 constexpr int kSquare = kC * kC;   // elements of a [64, 64] record
 constexpr int kState = kD * kD;    // elements of a state
+constexpr int kWidePad = kD + 4;   // LDS rows: 16-byte aligned, neighbours four banks apart
+constexpr int kSquarePad = kC + 4;
 
 // Per (head, chunk) records in the workspace, in floats.
 struct Records {
-  float *qn, *kn;             // q^, k^                                  [64][128]
-  float *w, *u, *y, *dl;      // W, U, Y, Dl                             [64][128]
-  float *ddl, *dwm;           // dDl, dW                                 [64][128]
-  float *dqp, *dkp;           // the parts of dq^ and dk^ that come from the states
+  float *w, *dl, *ddl;        // W; U, which Dl replaces; dDl            [64][128]
   float *p, *tm, *kkd;        // P, T, strict_lower((k^_i . k^_j) D_ij)  [64][64]
-  float *pd, *rr;             // dP D, diag(beta) dA D                   [64][64]
-  float *gates;               // [6][64]: G, beta, 1/|q|, 1/|k|, E, L
-  float *sums;                // [9][64]: row and column sums for d beta and d log-decay
-  float *m, *mt, *bc, *cc;    // M, M^T, B, C                            [128][128]
+  float *gates;               // [8][64], see Gate
   float *s0, *ds1;            // state entering the chunk, gradient of the state leaving it
 };
 
-constexpr int kGateRows = 6, kSumRows = 9;
-constexpr size_t kRecordFloats = 10 * static_cast<size_t>(kWide) + 5 * kSquare +
-                                 (kGateRows + kSumRows) * kC + 6 * static_cast<size_t>(kState);
+// Rows of a gates record.  q^ and k^ are not stored: their rows are those of the
+// convolved activations times kQScale and kKScale (zero beyond the sequence).
+enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kLK, kEQ, kGateRows };  // kLK = L kKScale, ...
+
+constexpr size_t kRecordFloats = 3 * static_cast<size_t>(kWide) + 3 * kSquare + kGateRows * kC +
+                                 2 * static_cast<size_t>(kState);
 
 struct ChunkedArgs {
   const float* post = nullptr;     // [T, channels]
@@ -97,83 +97,35 @@ __device__ inline floatx16 zero_tile() {
 // column is lane % 32.
 __device__ inline int tile_row(int i, int h) { return 8 * (i / 4) + 4 * h + i % 4; }
 
-// acc[m][n] += sum over k < K of A[m][k] B[k][n] for the lane's operand row m
-// and column n: a(k) returns A[m][k], b(k) returns B[k][n].  Every operand of
-// the product is requested before the first multiplication (one memory
-// latency a product instead of one every few steps) unless STREAM is set:
-// kernels whose registers allow many resident waves do better with the loads
-// spread between the multiplications.
-template <int K, bool STREAM = false, class AF, class BF>
-__device__ inline floatx16 product(floatx16 acc, AF a, BF b) {
-  const int h = (threadIdx.x % 64) / 32;
-  if constexpr (STREAM) {
-#pragma unroll 8
-    for (int k = 0; k < K; k += 2)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a(k + h), b(k + h), acc, 0, 0, 0);
-    return acc;
-  }
-  float av[K / 2], bv[K / 2];
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int s = 0; s < K / 2; ++s) {
-    av[s] = a(2 * s + h);
-    bv[s] = b(2 * s + h);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int s = 0; s < K / 2; ++s)
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s], bv[s], acc, 0, 0, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  return acc;
-}
-
-// The same sum for operands that are contiguous along k: a4(k) returns
-// A[m][k..k+3], b4(k) returns B[k..k+3][n], k a multiple of 4.  The two lane
-// halves take alternate groups of four (the order of a contraction is free).
-template <int K, bool STREAM = false, class AF, class BF>
-__device__ inline floatx16 product4(floatx16 acc, AF a4, BF b4) {
-  const int h = (threadIdx.x % 64) / 32;
-  if constexpr (STREAM) {
-#pragma unroll 4
-    for (int k = 0; k < K; k += 8) {
-      const float4 x = a4(k + 4 * h), y = b4(k + 4 * h);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, acc, 0, 0, 0);
-    }
-    return acc;
-  }
-  float4 av[K / 8], bv[K / 8];
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int s = 0; s < K / 8; ++s) {
-    av[s] = a4(8 * s + 4 * h);
-    bv[s] = b4(8 * s + 4 * h);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int s = 0; s < K / 8; ++s) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s].x, bv[s].x, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s].y, bv[s].y, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s].z, bv[s].z, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[s].w, bv[s].w, acc, 0, 0, 0);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  return acc;
-}
-
 __device__ inline float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-
+__device__ inline void store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ inline float4 scaled(float4 v, float s) {
   return make_float4(v.x * s, v.y * s, v.z * s, v.w * s);
 }
 
-// Rows of tokens beyond the sequence read as zero: the load itself is always
-// made (from the last row), so that it needs no branch.
-__device__ inline float keep(bool ok, float v) { return ok ? v : 0.0f; }
-__device__ inline float4 keep(bool ok, float4 v) {
-  return make_float4(ok ? v.x : 0.0f, ok ? v.y : 0.0f, ok ? v.z : 0.0f, ok ? v.w : 0.0f);
+// acc += a b over four contraction elements a lane half: the halves of a wave take
+// alternate groups of four (element e of half h is 8 s + 4 h + e, the row that
+// accumulator register 4 s + e of that half holds), so that both operands can come
+// in 16-byte pieces and an accumulator can be an operand as it is.
+__device__ inline floatx16 mma(floatx16 acc, float4 a, float4 b) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+  return acc;
+}
+
+// The same for 16 x 16 tiles: quarter q of the wave takes elements 16 s + 4 q + e, the
+// row that register e of that quarter holds.
+__device__ inline floatx4 mma16(floatx4 acc, float4 a, float4 b) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc, 0, 0, 0);
+  return acc;
+}
+__device__ inline floatx4 mma16(floatx4 acc, float4 a, floatx4 b) {
+  return mma16(acc, a, make_float4(b[0], b[1], b[2], b[3]));
 }
 
 __device__ inline float4 gather4(const float* p, int stride) {
@@ -186,797 +138,934 @@ __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// Sums over the 32 lanes of a half wave of sixteen values at once: lanes 2 j and 2 j + 1
+// of a half return the sum of value j.  Each exchange halves the values a lane holds.
+__device__ inline float half_sums(const float (&values)[16]) {
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = values[i];
+  const int n = threadIdx.x % 32;
+#pragma unroll
+  for (int width = 8; width > 0; width /= 2) {
+    const bool upper = n & (2 * width);
+#pragma unroll
+    for (int i = 0; i < width; ++i) {
+      const float kept = upper ? v[i + width] : v[i], sent = upper ? v[i] : v[i + width];
+      v[i] = kept + __shfl_xor(sent, 2 * width, 64);
+    }
+  }
+  return v[0] + __shfl_xor(v[0], 1, 64);
+}
+
+// Memory behind a buffer descriptor: a lane's byte offset, computed once, and a uniform
+// byte offset, so that a kernel keeps no addresses in vector registers.  Rows of
+// TOKENS may lie beyond the end: there the sum is the offset the descriptor checks,
+// reads give zero and writes are dropped, without a branch.
+template <bool TOKENS>
+struct Memory {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ Memory(const float* base, size_t elements)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0,
+                                               static_cast<int>(elements * 4), 0x00020000)) {}
+  __device__ float get(unsigned lane, unsigned uniform) const {
+    const auto bits = TOKENS ? __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane + uniform, 0, 0)
+                             : __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane, uniform, 0);
+    return __uint_as_float(bits);
+  }
+  __device__ float2 get2(unsigned lane, unsigned uniform) const {
+    const auto bits = TOKENS ? __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane + uniform, 0, 0)
+                             : __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane, uniform, 0);
+    return __builtin_bit_cast(float2, bits);
+  }
+  __device__ float4 get4(unsigned lane, unsigned uniform) const {
+    const auto bits = TOKENS ? __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane + uniform, 0, 0)
+                             : __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane, uniform, 0);
+    return __builtin_bit_cast(float4, bits);
+  }
+  // elements `stride` bytes apart
+  __device__ float4 gather4(unsigned lane, unsigned uniform, unsigned stride) const {
+    return make_float4(get(lane, uniform), get(lane, uniform + stride), get(lane, uniform + 2 * stride),
+                       get(lane, uniform + 3 * stride));
+  }
+  __device__ void put(float v, unsigned lane, unsigned uniform) const {
+    if (TOKENS)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, lane + uniform, 0, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, lane, uniform, 0);
+  }
+};
+using Record = Memory<false>;
+using Tokens = Memory<true>;
+
+// One chunk of one head.  Tokens beyond the sequence have zero rows, scales, beta and
+// gradients.
+struct ChunkView {
+  const ChunkedArgs& a;
+  size_t rec;
+  int t0, head, tokens, channels;
+  unsigned row_bytes, out_bytes;   // a token's row in the activations, in dO and O
+  const float* gates;
+  __device__ ChunkView(const ChunkedArgs& args, int chunk, int head_)
+      : a(args), rec(static_cast<size_t>(head_) * args.chunks + chunk), t0(chunk * kC), head(head_),
+        tokens(min(args.length - t0, kC)), channels(2 * args.kh * kD + args.vh * kD),
+        row_bytes(channels * 4), out_bytes(args.vh * kD * 4), gates(args.r.gates + rec * kGateRows * kC) {}
+  __device__ Tokens activations(const float* base, int column) const {
+    return Tokens(base + static_cast<size_t>(t0) * channels + column,
+                  static_cast<size_t>(tokens) * channels - column);
+  }
+  __device__ int key_head() const { return head / (a.vh / a.kh); }
+  __device__ int value_column() const { return (2 * a.kh + head) * kD; }
+  __device__ Tokens q() const { return activations(a.post, key_head() * kD); }
+  __device__ Tokens k() const { return activations(a.post, (a.kh + key_head()) * kD); }
+  __device__ Tokens v() const { return activations(a.post, value_column()); }
+  __device__ Tokens dv() const { return activations(a.dpost, value_column()); }
+  __device__ Tokens heads(const float* base) const {  // O, dO
+    return Tokens(base + (static_cast<size_t>(t0) * a.vh + head) * kD,
+                  (static_cast<size_t>(tokens) * a.vh - head) * kD);
+  }
+  __device__ Tokens qk_partials() const {
+    return Tokens(a.qk_partials + (static_cast<size_t>(t0) * a.vh + head) * 2 * kD,
+                  (static_cast<size_t>(tokens) * a.vh - head) * 2 * kD);
+  }
+  __device__ Record wide(const float* records) const { return Record(records + rec * kWide, kWide); }
+  __device__ Record square(const float* records) const { return Record(records + rec * kSquare, kSquare); }
+  __device__ Record state(const float* records) const { return Record(records + rec * kState, kState); }
+};
+constexpr unsigned kWideRow = kD * 4, kSquareRow = kC * 4;  // bytes
+
 // ---------------------------------------------------------------------------
-// T, W, U, P and the gates of one chunk.
+// T, W, U, P and the gates of one chunk.  68 KiB of LDS, two workgroups a compute
+// unit.  The inverse is made by blocks: the four 16 x 16 diagonal blocks by forward
+// substitution, one wave each, then -T22 A21 T11 twice on the matrix cores (a
+// substitution over all 64 rows by one wave held the other three up for a third of
+// the kernel).
 __global__ void __launch_bounds__(256)
 chunk_prepare_kernel(ChunkedArgs a) {
-  __shared__ float qs[kC][kD + 1], ks[kC][kD + 1];
-  __shared__ float am[kC][kC + 4];                  // A, rows 16-byte aligned
-  __shared__ float tk[kC][kC + 1], tv[kC][kC + 1];  // T diag(beta E), T diag(beta)
-  __shared__ float log_decay[kC], g_cum[kC], beta_s[kC];
-  const int chunk = blockIdx.x, head = blockIdx.y;
-  const int key_head = head / (a.vh / a.kh);
+  __shared__ __attribute__((aligned(16))) struct {
+    float k[kC][kWidePad];
+    union {
+      float q[kC][kWidePad];
+      struct {
+        float a[kC][kSquarePad], t[kC][kSquarePad];
+      };
+    };
+    float g[kC], beta[kC], fk[kC];
+  } sm;
+  const ChunkView v(a, blockIdx.x, blockIdx.y);
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int h = lane / 32, n = lane % 32;
-  const int channels = 2 * a.kh * kD + a.vh * kD;
-  const size_t rec = static_cast<size_t>(head) * a.chunks + chunk;
-  const int t0 = chunk * kC;
-  const float norm_scale = sqrtf(static_cast<float>(kD));
-  float* gates = a.r.gates + rec * kGateRows * kC;
+  const int h = lane / 32, n = lane % 32, quarter = lane / 16, n16 = lane % 16;
+  float* gates = a.r.gates + v.rec * kGateRows * kC;
 
-  // normalised rows (1e-6 added to the sums of squares, sequence_delta_net.cc:84-85)
-  for (int r = 0; r < kC / 4; ++r) {
-    const int i = wave * (kC / 4) + r, t = t0 + i;
-    const bool ok = t < a.length;
-    const float* row = a.post + static_cast<size_t>(ok ? t : 0) * channels;
-    float q[2], k[2];
+  // normalised rows (1e-6 added to the sums of squares, sequence_delta_net.cc:84-85):
+  // half a wave a row, row 16 wave + 2 r + h
+  {
+    const float norm_scale = sqrtf(static_cast<float>(kD));
+    const Tokens q = v.q(), k = v.k();
+    const unsigned at = (16 * wave + h) * v.row_bytes + 16 * n;
+    float4 rows[16];
+    float squares[16];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      q[j] = ok ? row[key_head * kD + lane + 64 * j] : 0.0f;
-      k[j] = ok ? row[(a.kh + key_head) * kD + lane + 64 * j] : 0.0f;
+    for (int r = 0; r < 8; ++r) {
+      rows[2 * r] = q.get4(at, 2 * r * v.row_bytes);
+      rows[2 * r + 1] = k.get4(at, 2 * r * v.row_bytes);
     }
-    const float iq = rsqrtf(wave_sum(q[0] * q[0] + q[1] * q[1]) + 1e-6f);
-    const float ik = rsqrtf(wave_sum(k[0] * k[0] + k[1] * k[1]) + 1e-6f);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float qv = q[j] * iq / norm_scale, kv = k[j] * ik;
-      qs[i][lane + 64 * j] = qv;
-      ks[i][lane + 64 * j] = kv;
-      a.r.qn[rec * kWide + i * kD + lane + 64 * j] = qv;
-      a.r.kn[rec * kWide + i * kD + lane + 64 * j] = kv;
-    }
-    if (lane == 0) {
-      gates[2 * kC + i] = iq;
-      gates[3 * kC + i] = ik;
+    for (int r = 0; r < 16; ++r)
+      squares[r] = (rows[r].x * rows[r].x + rows[r].y * rows[r].y) +
+                   (rows[r].z * rows[r].z + rows[r].w * rows[r].w);
+    const float sum = half_sums(squares);  // lane 2 j holds that of rows[j]
+    const float inverse = rsqrtf(sum + 1e-6f);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int i = 16 * wave + 2 * r + h;
+      const bool ok = i < v.tokens;
+      const float iq = ok ? __shfl(inverse, 32 * h + 4 * r, 64) / norm_scale : 0.0f;
+      const float ik = ok ? __shfl(inverse, 32 * h + 4 * r + 2, 64) : 0.0f;
+      store4(&sm.q[i][4 * n], scaled(rows[2 * r], iq));
+      store4(&sm.k[i][4 * n], scaled(rows[2 * r + 1], ik));
+      if (n == 0) {
+        gates[kQScale * kC + i] = iq;
+        gates[kKScale * kC + i] = ik;
+        sm.fk[i] = ik;  // until the gates below
+        sm.beta[i] = iq;
+      }
     }
   }
+  __syncthreads();
   // gates (sequence_delta_net.cc:88-96); tokens beyond the sequence neither
   // decay nor write
-  if (tid < kC) {
-    const int t = t0 + tid;
-    const bool ok = t < a.length;
+  if (wave == 0) {
+    const int t = v.t0 + lane;
     float g = 0.0f, beta = 0.0f;
-    if (ok) {
-      const float alpha = bf16_bits_to_float(a.a[static_cast<size_t>(t) * a.vh + head]) + a.dt_bias[head];
+    if (lane < v.tokens) {
+      const float alpha =
+          bf16_bits_to_float(a.a[static_cast<size_t>(t) * a.vh + v.head]) + a.dt_bias[v.head];
       const float softplus = fmaxf(alpha, 0.0f) + logf(1.0f + expf(-fabsf(alpha)));
-      g = -expf(a.a_log[head]) * softplus;
-      const float bv = bf16_bits_to_float(a.b[static_cast<size_t>(t) * a.vh + head]);
+      g = -expf(a.a_log[v.head]) * softplus;
+      const float bv = bf16_bits_to_float(a.b[static_cast<size_t>(t) * a.vh + v.head]);
       beta = round_if(1.0f / (1.0f + expf(-bv)), a.round);
     }
-    log_decay[tid] = g;
-    beta_s[tid] = beta;
-    gates[kC + tid] = beta;
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+      const float before = __shfl_up(g, offset, 64);
+      if (lane >= offset) g += before;
+    }
+    const float e = expf(g), l = expf(__shfl(g, 63, 64) - g);
+    gates[kG * kC + lane] = g;
+    gates[kBeta * kC + lane] = beta;
+    gates[kE * kC + lane] = e;
+    gates[kL * kC + lane] = l;
+    gates[kLK * kC + lane] = l * sm.fk[lane];
+    gates[kEQ * kC + lane] = e * sm.beta[lane];
+    sm.g[lane] = g;
+    sm.beta[lane] = beta;
+    sm.fk[lane] = beta * e;
   }
   __syncthreads();
-  if (tid == 0) {
-    float c = 0.0f;
-    for (int i = 0; i < kC; ++i) {
-      c += log_decay[i];
-      g_cum[i] = c;
+  // k^ k^T and q^ k^T by 16 x 16 tiles on and below the diagonal: wave w takes row w of
+  // the first and row 3 - w of the second, five tiles
+  floatx4 kk[4], qk[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) kk[b] = qk[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < kD / 16; ++s) {
+    const float4 kr = load4(&sm.k[16 * wave + n16][16 * s + 4 * quarter]);
+    const float4 qr = load4(&sm.q[16 * (3 - wave) + n16][16 * s + 4 * quarter]);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      if (b > wave && b > 3 - wave) continue;
+      const float4 kc = load4(&sm.k[16 * b + n16][16 * s + 4 * quarter]);
+      if (b <= wave) kk[b] = mma16(kk[b], kr, kc);
+      if (b <= 3 - wave) qk[b] = mma16(qk[b], qr, kc);
     }
   }
-  __syncthreads();
-  if (tid < kC) {
-    gates[tid] = g_cum[tid];
-    gates[4 * kC + tid] = expf(g_cum[tid]);
-    gates[5 * kC + tid] = expf(g_cum[kC - 1] - g_cum[tid]);
-  }
-
-  // k^ k^T and q^ k^T, one 32 x 32 tile a wave (tile (0, 1) is above the diagonal)
+  __syncthreads();  // the rows of q^ make room for A and T
+  const auto kkd = v.square(a.r.kkd), p = v.square(a.r.p);
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 4 * quarter + e, col = 16 * b + n16;
+      const int k_at = 16 * wave + row, q_at = 16 * (3 - wave) + row;
+      const float kv = k_at > col ? kk[b][e] * expf(sm.g[k_at] - sm.g[col]) : 0.0f;
+      kkd.put(kv, 4 * (k_at * kC + n16), 64 * b);
+      p.put(q_at >= col ? qk[b][e] * expf(sm.g[q_at] - sm.g[col]) : 0.0f, 4 * (q_at * kC + n16), 64 * b);
+      sm.a[k_at][col] = sm.beta[k_at] * kv;
+      sm.t[k_at][col] = 0.0f;
+    }
+  lds_barrier();
   {
-    const int ti = wave / 2, tj = wave % 2;
-    floatx16 kk = zero_tile(), qk = zero_tile();
-    if (ti >= tj) {
-      kk = product<kD>(kk, [&](int k) { return ks[32 * ti + n][k]; },
-                       [&](int k) { return ks[32 * tj + n][k]; });
-      qk = product<kD>(qk, [&](int k) { return qs[32 * ti + n][k]; },
-                       [&](int k) { return ks[32 * tj + n][k]; });
+    // diagonal block `wave`, column n16
+    const int first = 16 * wave;
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float row[16];
+#pragma unroll
+      for (int j = 0; j < i; j += 4) {
+        const float4 four = load4(&sm.a[first + i][first + j]);
+        row[j] = four.x, row[j + 1] = four.y, row[j + 2] = four.z, row[j + 3] = four.w;
+      }
+      float s = i == n16 ? 1.0f : 0.0f;
+#pragma unroll
+      for (int j = 0; j < i; ++j) s -= row[j] * x[j];
+      x[i] = s;
     }
-    const int col = 32 * tj + n;
+    if (quarter == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sm.t[first + i][first + n16] = x[i];
+    }
+  }
+  lds_barrier();
+  const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (wave % 2 == 1) {
+    // the block left of diagonal block `wave`: -T_ww A_w,w-1 T_w-1,w-1
+    const int r0 = 16 * wave, c0 = r0 - 16;
+    const floatx4 y = mma16(none, load4(&sm.a[r0 + n16][c0 + 4 * quarter]),
+                            gather4(&sm.t[c0 + 4 * quarter][c0 + n16], kSquarePad));
+    const floatx4 z = mma16(none, load4(&sm.t[r0 + n16][r0 + 4 * quarter]), y);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sm.t[r0 + 4 * quarter + e][c0 + n16] = -z[e];
+  }
+  lds_barrier();
+  {
+    // rows 32.., columns ..31 by 16 x 16 tiles, tile (wave / 2, wave % 2)
+    const int r0 = 32 + 16 * (wave / 2), c0 = 16 * (wave % 2);
+    floatx4 z = none;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      if (m > wave / 2) continue;
+      floatx4 y = none;
+#pragma unroll
+      for (int l = 0; l < 2; ++l)
+        if (l >= wave % 2)
+          y = mma16(y, load4(&sm.a[32 + 16 * m + n16][16 * l + 4 * quarter]),
+                    gather4(&sm.t[16 * l + 4 * quarter][c0 + n16], kSquarePad));
+      z = mma16(z, load4(&sm.t[r0 + n16][32 + 16 * m + 4 * quarter]), y);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sm.t[r0 + 4 * quarter + e][c0 + n16] = -z[e];
+  }
+  // W = T diag(beta E) K^, U = T diag(beta) V: the wave owns 32 columns
+  const int col = 32 * wave + n;
+  const auto value_memory = v.v();
+  float4 values[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    values[s] = value_memory.gather4(4 * h * v.row_bytes + 4 * col, 8 * s * v.row_bytes, v.row_bytes);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < kC * kC / 4 / 256; ++i) {
+    const int at = tid + 256 * i;
+    store4(a.r.tm + v.rec * kSquare + 4 * at, load4(&sm.t[at / 16][at % 16 * 4]));
+  }
+  const auto w_out = v.wide(a.r.w), u_out = v.wide(a.r.dl);
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti) {
+    floatx16 w = zero_tile(), u = zero_tile();
+#pragma unroll
+    for (int s = 0; s < 4 * (ti + 1); ++s) {
+      const int k = 8 * s + 4 * h;
+      const float4 t = load4(&sm.t[32 * ti + n][k]), f = load4(&sm.fk[k]), b = load4(&sm.beta[k]);
+      w = mma(w, make_float4(t.x * f.x, t.y * f.y, t.z * f.z, t.w * f.w), gather4(&sm.k[k][col], kWidePad));
+      u = mma(u, make_float4(t.x * b.x, t.y * b.y, t.z * b.z, t.w * b.w), values[s]);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const unsigned at = 4 * h * kWideRow + 4 * col, row = (32 * ti + tile_row(i, 0)) * kWideRow;
+      w_out.put(w[i], at, row);
+      u_out.put(u[i], at, row);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The workgroups of the sequential kernels.  The eight column slices of a head read
+// the same matrices: they are given block numbers with the same remainder mod 8,
+// which the hardware places on one XCD, so that seven of the eight reads are served
+// by that XCD's L2.
+struct Slice {
+  int head, col0;
+};
+__device__ inline Slice slice_of_block(const ChunkedArgs& a) {
+  constexpr int kSlices = kD / kSlice;
+  static_assert(kSlices == 8, "one slice of a head per block of an XCD's share");
+  if (a.vh % 8 == 0)
+    return {static_cast<int>((blockIdx.x % 8) * (a.vh / 8) + blockIdx.x / 64),
+            static_cast<int>(blockIdx.x / 8 % kSlices * kSlice)};
+  return {static_cast<int>(blockIdx.x / kSlices), static_cast<int>(blockIdx.x % kSlices * kSlice)};
+}
+
+// The state of a slice lives in accumulators: wave w holds rows 32 w .. 32 w + 31, as two
+// 16 x 16 tiles whose rows are interleaved (row 32 w + 2 i + t is row i of tile t), so
+// that an operand row that is contiguous along them is read two elements a lane and a
+// lane's eight elements are rows 32 w + 8 quarter .. + 7.  `rows` is the LDS copy
+// [column][row] that the other waves multiply.
+__device__ inline void publish_state(const floatx4 (&acc)[2], float* rows) {
+  store4(rows, make_float4(acc[0][0], acc[1][0], acc[0][1], acc[1][1]));
+  store4(rows + 4, make_float4(acc[0][2], acc[1][2], acc[0][3], acc[1][3]));
+}
+
+__device__ inline void save_state(const floatx4 (&acc)[2], const Record& state, unsigned lane) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) state.put(acc[t][e], lane, (2 * e + t) * kWideRow);
+}
+
+// S entering every chunk and Dl of every chunk.  Wave w computes rows 16 w .. 16 w + 15
+// of Dl from the whole state and then its rows of the new state from all of Dl: two
+// dependent products of 32 matrix instructions a chunk.  The operands of the chunk
+// after next are requested as soon as this chunk's have been multiplied.
+__global__ void __launch_bounds__(256)
+chunk_states_forward_kernel(ChunkedArgs a) {
+  __shared__ __attribute__((aligned(16))) float state[kSlice][kWidePad], delta[kSlice][kSquarePad];
+  const Slice slice = slice_of_block(a);
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int quarter = lane / 16, n = lane % 16;
+  const int col = slice.col0 + n;
+  struct Operands {
+    float4 w[8];
+    float2 k[16];
+    float u[4];
+    float4 scale;
+    float decay;
+  };
+  auto view = [&](int chunk) { return ChunkView(a, min(chunk, a.chunks - 1), slice.head); };
+  // a lane's places in a record of rows of all channels: its row as the left operand,
+  // its rows as a result, its rows and channels as the transposed left operand
+  const unsigned row_at = (16 * wave + n) * kWideRow + 16 * quarter;
+  const unsigned result_at = (16 * wave + 4 * quarter) * kWideRow + 4 * col;
+  const unsigned state_at = (32 * wave + 8 * quarter) * kWideRow + 4 * col;
+  auto request_delta = [&](const ChunkView& v, Operands& o) {
+    const auto w = v.wide(a.r.w), u = v.wide(a.r.dl);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) o.w[s] = w.get4(row_at, 64 * s);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o.u[e] = u.get(result_at, e * kWideRow);
+    o.scale = load4(v.gates + kLK * kC + 16 * wave + 4 * quarter);
+  };
+  auto request_state = [&](const ChunkView& v, Operands& o) {
+    const auto k = v.k();
+    const unsigned at = 4 * quarter * v.row_bytes + 4 * (32 * wave + 2 * n);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o.k[j] = k.get2(at, (16 * (j / 4) + j % 4) * v.row_bytes);
+    o.decay = v.gates[kE * kC + kC - 1];
+  };
+  floatx4 acc[2];
+  acc[0] = acc[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto advance = [&](int chunk, Operands& o) {
+    const ChunkView v(a, chunk, slice.head), later = view(chunk + 2);
+    const auto dl_out = v.wide(a.r.dl);
+    publish_state(acc, &state[n][32 * wave + 8 * quarter]);
+    save_state(acc, v.state(a.r.s0), state_at);
+    lds_barrier();
+    floatx4 even = {0.0f, 0.0f, 0.0f, 0.0f}, odd = even;
+    float4 b[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) b[s] = load4(&state[n][16 * s + 4 * quarter]);
+#pragma unroll
+    for (int s = 0; s < 8; s += 2) {
+      even = mma16(even, o.w[s], b[s]);
+      odd = mma16(odd, o.w[s + 1], b[s + 1]);
+    }
+    float dl[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      dl[e] = o.u[e] - (even[e] + odd[e]);
+      dl_out.put(dl[e], result_at, e * kWideRow);
+    }
+    store4(&delta[n][16 * wave + 4 * quarter],
+           make_float4(dl[0] * o.scale.x, dl[1] * o.scale.y, dl[2] * o.scale.z, dl[3] * o.scale.w));
+    __builtin_amdgcn_sched_barrier(0);
+    request_delta(later, o);
+    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) b[s] = load4(&delta[n][16 * s + 4 * quarter]);
+    acc[0] *= o.decay;
+    acc[1] *= o.decay;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      acc[0] = mma16(acc[0], make_float4(o.k[4 * s].x, o.k[4 * s + 1].x, o.k[4 * s + 2].x, o.k[4 * s + 3].x), b[s]);
+      acc[1] = mma16(acc[1], make_float4(o.k[4 * s].y, o.k[4 * s + 1].y, o.k[4 * s + 2].y, o.k[4 * s + 3].y), b[s]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    request_state(later, o);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  Operands even, odd;
+  request_delta(view(0), even);
+  request_state(view(0), even);
+  request_delta(view(1), odd);
+  request_state(view(1), odd);
+  for (int chunk = 0; chunk < a.chunks; chunk += 2) {
+    advance(chunk, even);
+    if (chunk + 1 < a.chunks) advance(chunk + 1, odd);
+  }
+}
+
+// The gradient of the state leaving every chunk and dDl of every chunk, chunks in
+// reverse.  112 matrix instructions a wave and chunk; the products with dO do not
+// depend on the chain and run while it waits.
+__global__ void __launch_bounds__(256)
+chunk_states_backward_kernel(ChunkedArgs a) {
+  __shared__ __attribute__((aligned(16))) float state[kSlice][kWidePad], delta[kSlice][kSquarePad],
+      grad[kSlice][kSquarePad], query_grad[kSlice][kSquarePad];
+  const Slice slice = slice_of_block(a);
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int quarter = lane / 16, n = lane % 16;
+  const int col = slice.col0 + n;
+  auto view = [&](int chunk) { return ChunkView(a, max(chunk, 0), slice.head); };
+  float4 k[8];
+  float p[16], out[4];
+  float2 q[16], w[16];
+  float4 k_scale, q_scale;
+  float decay;
+  const int rows = 16 * wave + 4 * quarter;
+  const unsigned result_at = rows * kWideRow + 4 * col;
+  const unsigned state_at = (32 * wave + 8 * quarter) * kWideRow + 4 * col;
+  auto request_out = [&](const ChunkView& v) {
+    const auto d_out = v.heads(a.dcore);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = d_out.get(rows * v.out_bytes + 4 * col, e * v.out_bytes);
+    q_scale = load4(v.gates + kEQ * kC + rows);
+  };
+  auto request_delta = [&](const ChunkView& v) {
+    const Record p_memory = v.square(a.r.p);
+    const Tokens k_memory = v.k();
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      p[j] = p_memory.get(4 * quarter * kSquareRow + 4 * (16 * wave + n), (16 * (j / 4) + j % 4) * kSquareRow);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) k[s] = k_memory.get4((16 * wave + n) * v.row_bytes + 16 * quarter, 64 * s);
+    k_scale = load4(v.gates + kLK * kC + rows);
+  };
+  auto request_query = [&](const ChunkView& v) {
+    const auto q_memory = v.q();
+    const unsigned at = 4 * quarter * v.row_bytes + 4 * (32 * wave + 2 * n);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) q[j] = q_memory.get2(at, (16 * (j / 4) + j % 4) * v.row_bytes);
+    decay = v.gates[kE * kC + kC - 1];
+  };
+  auto request_weights = [&](const ChunkView& v) {
+    const auto w_memory = v.wide(a.r.w);
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      w[j] = w_memory.get2(4 * quarter * kWideRow + 4 * (32 * wave + 2 * n), (16 * (j / 4) + j % 4) * kWideRow);
+  };
+  floatx4 acc[2];
+  acc[0] = acc[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  {
+    const ChunkView v = view(a.chunks - 1);
+    request_out(v);
+    request_delta(v);
+    request_query(v);
+    request_weights(v);
+  }
+  for (int chunk = a.chunks - 1; chunk >= 0; --chunk) {
+    const ChunkView v(a, chunk, slice.head), later = view(chunk - 1);
+    const auto ddl_out = v.wide(a.r.ddl);
+    publish_state(acc, &state[n][32 * wave + 8 * quarter]);
+    store4(&grad[n][rows], make_float4(out[0], out[1], out[2], out[3]));
+    store4(&query_grad[n][rows],
+           make_float4(out[0] * q_scale.x, out[1] * q_scale.y, out[2] * q_scale.z, out[3] * q_scale.w));
+    save_state(acc, v.state(a.r.ds1), state_at);
+    __builtin_amdgcn_sched_barrier(0);
+    request_out(later);
+    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier();
+    floatx4 from_out = {0.0f, 0.0f, 0.0f, 0.0f}, even = from_out, odd = from_out;
+    float4 b[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) b[s] = load4(&state[n][16 * s + 4 * quarter]);
+    float4 g[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) g[s] = load4(&grad[n][16 * s + 4 * quarter]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      even = mma16(even, k[2 * s], b[2 * s]);
+      odd = mma16(odd, k[2 * s + 1], b[2 * s + 1]);
+      from_out = mma16(from_out, make_float4(p[4 * s], p[4 * s + 1], p[4 * s + 2], p[4 * s + 3]), g[s]);
+    }
+    float dd[4];
+    const float scale[4] = {k_scale.x, k_scale.y, k_scale.z, k_scale.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      dd[e] = from_out[e] + scale[e] * (even[e] + odd[e]);
+      ddl_out.put(dd[e], result_at, e * kWideRow);
+    }
+    store4(&delta[n][rows], make_float4(-dd[0], -dd[1], -dd[2], -dd[3]));
+    __builtin_amdgcn_sched_barrier(0);
+    request_delta(later);
+    __builtin_amdgcn_sched_barrier(0);
+    acc[0] *= decay;
+    acc[1] *= decay;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) g[s] = load4(&query_grad[n][16 * s + 4 * quarter]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      acc[0] = mma16(acc[0], make_float4(q[4 * s].x, q[4 * s + 1].x, q[4 * s + 2].x, q[4 * s + 3].x), g[s]);
+      acc[1] = mma16(acc[1], make_float4(q[4 * s].y, q[4 * s + 1].y, q[4 * s + 2].y, q[4 * s + 3].y), g[s]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    request_query(later);
+    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) g[s] = load4(&delta[n][16 * s + 4 * quarter]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      acc[0] = mma16(acc[0], make_float4(w[4 * s].x, w[4 * s + 1].x, w[4 * s + 2].x, w[4 * s + 3].x), g[s]);
+      acc[1] = mma16(acc[1], make_float4(w[4 * s].y, w[4 * s + 1].y, w[4 * s + 2].y, w[4 * s + 3].y), g[s]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    request_weights(later);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// O = diag(E) Q^ S + P Dl of one chunk.  Wave w owns value columns 32w..32w+31 and has
+// its part of S and Dl in registers, requested before the rows of Q^ and P are staged
+// for all waves.
+__global__ void __launch_bounds__(256)
+chunk_outputs_kernel(ChunkedArgs a) {
+  __shared__ __attribute__((aligned(16))) float q_s[kC][kWidePad], p_s[kC][kSquarePad];
+  const ChunkView v(a, blockIdx.x, blockIdx.y);
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int h = lane / 32, n = lane % 32;
+  const int col = 32 * wave + n;
+  const Tokens q = v.q(), core = v.heads(a.core);
+  const Record p = v.square(a.r.p), state = v.state(a.r.s0), delta = v.wide(a.r.dl);
+  float4 rows[8], p_rows[4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    rows[i] = scaled(q.get4(tid / 32 * v.row_bytes + tid % 32 * 16, 8 * i * v.row_bytes),
+                     v.gates[kEQ * kC + tid / 32 + 8 * i]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p_rows[i] = p.get4(16 * tid, 4096 * i);
+  const unsigned column_at = 4 * h * kWideRow + 4 * col;
+  float4 s_col[16], d_col[8];
+#pragma unroll
+  for (int s = 0; s < 16; ++s) s_col[s] = state.gather4(column_at, 8 * s * kWideRow, kWideRow);
+#pragma unroll
+  for (int s = 0; s < 8; ++s) d_col[s] = delta.gather4(column_at, 8 * s * kWideRow, kWideRow);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int at = tid + 256 * i;
+    store4(&q_s[at / 32][at % 32 * 4], rows[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int at = tid + 256 * i;
+    store4(&p_s[at / 16][at % 16 * 4], p_rows[i]);
+  }
+  lds_barrier();
+  floatx16 out[2];
+  out[0] = out[1] = zero_tile();
+#pragma unroll
+  for (int s = 0; s < 16; ++s)
+#pragma unroll
+    for (int ti = 0; ti < 2; ++ti)
+      out[ti] = mma(out[ti], load4(&q_s[32 * ti + n][8 * s + 4 * h]), s_col[s]);
+#pragma unroll
+  for (int s = 0; s < 8; ++s)
+#pragma unroll
+    for (int ti = 0; ti < 2; ++ti)
+      if (s < 4 * (ti + 1)) out[ti] = mma(out[ti], load4(&p_s[32 * ti + n][8 * s + 4 * h]), d_col[s]);
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      core.put(round_if(out[ti][i], a.round), 4 * h * v.out_bytes + 4 * col,
+               (32 * ti + tile_row(i, 0)) * v.out_bytes);
+}
+
+// ---------------------------------------------------------------------------
+// The gradients of one chunk.  Wave w owns columns 32w..32w+31 of the [64, 128]
+// matrices (two 32-row tiles) and one 32 x 32 tile of the [64, 64] matrices, of which
+// only those on and below the diagonal are needed.
+//   1. contractions over value channels, 32 of them at a time, dDl, dO, Dl and V in LDS
+//      and the states straight from memory (each element is used by one wave):
+//        dW = -dDl S^T        dq^ = diag(E) dO S^T        dk^ = diag(L) Dl dS'^T
+//        dP = lower(dO Dl^T)  dT = dDl (diag(beta) V)^T   and <dS', S>
+//   2. dT += dW (diag(beta E) K^)^T;  dA = -strict_lower(T^T dT T^T);  R = diag(beta) dA D
+//   3. dq^ += Pd K^ with Pd = dP D;  dk^ += (R + R^T) K^ + Pd^T Q^ + diag(beta E) T^T dW;
+//      dv = diag(beta) T^T dDl;  dq and dk back through the normalisations
+//   4. d log-decay and d beta from row and column sums of the above, through the gates
+//      to da, db and the contribution to d A_log
+// 75 KiB of LDS and 256 registers: two workgroups a compute unit.
+constexpr int kSlab = 32;
+struct GradientSmem {
+  union {
+    float slab[4][kC][kSlab + 4];  // dDl, dO, Dl, V
+    struct {
+      float dw[kC][kWidePad], pd[kC][kSquarePad], x[kC][kSquarePad];
+    };
+  };
+  float parts[6][kC][4];     // row sums of the waves' columns, see RowSum
+  float row_n[kC][2], col_n[kC][2], row_p[kC][2], col_p[kC][2];  // by tile
+  float gate[kGateRows][kC];
+  float dot[4];
+};
+enum RowSum { kSumQ, kSumK, kSumW, kSumV, kDotQ, kDotK };
+
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+chunk_gradients_kernel(ChunkedArgs a) {
+  __shared__ __attribute__((aligned(16))) GradientSmem sm;
+  const ChunkView v(a, blockIdx.x, blockIdx.y);
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int h = lane / 32, n = lane % 32, col = 32 * wave + n;
+  const int ti_own = wave / 2, tj_own = wave % 2;   // the [64, 64] tile
+  const bool lower = ti_own >= tj_own;
+  for (int i = tid; i < kGateRows * kC; i += 256) sm.gate[i / kC][i % kC] = v.gates[i];
+  if (tid < kC) {
+    sm.row_n[tid][0] = sm.row_n[tid][1] = sm.col_n[tid][0] = sm.col_n[tid][1] = 0.0f;
+    sm.row_p[tid][0] = sm.row_p[tid][1] = sm.col_p[tid][0] = sm.col_p[tid][1] = 0.0f;
+  }
+  floatx16 dw[2], dq[2], dk[2], dp = zero_tile(), dt = zero_tile();
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti) dw[ti] = dq[ti] = dk[ti] = zero_tile();
+  float dot = 0.0f;
+  {
+    const Record s0_memory = v.state(a.r.s0), s1_memory = v.state(a.r.ds1), ddl = v.wide(a.r.ddl),
+                 dl = v.wide(a.r.dl);
+    const Tokens d_out = v.heads(a.dcore), values = v.v();
+    const unsigned state_at = col * kWideRow + 16 * h;
+    // thread (row, piece) of the slabs: rows r and r + 32, 16 bytes
+    const int row = tid / 8, piece = tid % 8 * 4;
+    float4 staged[8];
+    auto request = [&](int slab) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const unsigned c = 4 * kSlab * slab;
+        staged[4 * j] = ddl.get4(row * kWideRow + 4 * piece, 32 * j * kWideRow + c);
+        staged[4 * j + 1] = d_out.get4(row * v.out_bytes + 4 * piece, 32 * j * v.out_bytes + c);
+        staged[4 * j + 2] = dl.get4(row * kWideRow + 4 * piece, 32 * j * kWideRow + c);
+        staged[4 * j + 3] = values.get4(row * v.row_bytes + 4 * piece, 32 * j * v.row_bytes + c);
+      }
+    };
+    request(0);
+    float4 s0[4], s1[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) s0[g] = s0_memory.get4(state_at, 32 * g), s1[g] = s1_memory.get4(state_at, 32 * g);
+    float fv = 0.0f;
+#pragma unroll
+    for (int slab = 0; slab < kD / kSlab; ++slab) {
+      if (slab > 0) lds_barrier();
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+          store4(&sm.slab[m][row + 32 * j][piece], staged[4 * j + m]);
+      if (slab == 0)
+        __syncthreads();
+      else
+        lds_barrier();
+      if (slab == 0) fv = sm.gate[kBeta][32 * tj_own + n];
+      if (slab + 1 < kD / kSlab) request(slab + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int c = 8 * g + 4 * h;
+        dot += (s0[g].x * s1[g].x + s0[g].y * s1[g].y) + (s0[g].z * s1[g].z + s0[g].w * s1[g].w);
+#pragma unroll
+        for (int ti = 0; ti < 2; ++ti) {
+          dw[ti] = mma(dw[ti], load4(&sm.slab[0][32 * ti + n][c]), s0[g]);
+          dq[ti] = mma(dq[ti], load4(&sm.slab[1][32 * ti + n][c]), s0[g]);
+          dk[ti] = mma(dk[ti], load4(&sm.slab[2][32 * ti + n][c]), s1[g]);
+        }
+        if (slab + 1 < kD / kSlab) {
+          s0[g] = s0_memory.get4(state_at, 4 * kSlab * (slab + 1) + 32 * g);
+          s1[g] = s1_memory.get4(state_at, 4 * kSlab * (slab + 1) + 32 * g);
+        }
+        if (lower) {
+          dp = mma(dp, load4(&sm.slab[1][32 * ti_own + n][c]), load4(&sm.slab[2][32 * tj_own + n][c]));
+          dt = mma(dt, load4(&sm.slab[0][32 * ti_own + n][c]), scaled(load4(&sm.slab[3][32 * tj_own + n][c]), fv));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    dot = wave_sum(dot);
+    if (lane == 0) sm.dot[wave] = dot;
+  }
+  lds_barrier();  // the slabs make room for dW, Pd and X
+  const int tile_col = 32 * tj_own + n;
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sm.dw[32 * ti + tile_row(i, h)][col] = -dw[ti][i];
+  // row and column sums of a tile held in an accumulator, for its rows and columns
+  auto tile_sums = [&](const float (&values)[16], float (&row_sums)[kC][2], float (&col_sums)[kC][2],
+                       const float* weights) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      sum += weights ? weights[32 * ti_own + tile_row(i, h)] * values[i] : values[i];
+    sum += __shfl_xor(sum, 32, 64);
+    if (h == 0) col_sums[tile_col][ti_own] = sum;
+    const float row_sum = half_sums(values);
+    if (n % 2 == 0) row_sums[32 * ti_own + tile_row(n / 2, h)][tj_own] = row_sum;
+  };
+  const Record p_memory = v.square(a.r.p), kkd = v.square(a.r.kkd), tm = v.square(a.r.tm),
+               ddl = v.wide(a.r.ddl);
+  const Tokens q_memory = v.q(), k_memory = v.k(), v_memory = v.v(), dv = v.dv();
+  // the accumulator's places in a [64, 64] tile and in a column of the [64, 128] matrices
+  const unsigned tile_at = (32 * ti_own + 4 * h) * kSquareRow + 4 * tile_col;
+  const unsigned column_at = 4 * h * kWideRow + 4 * col, token_at = 4 * h * v.row_bytes + 4 * col;
+  float decay[16];  // D of the tile
+  if (lower) {
+    float products[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 32 * ti_own + tile_row(i, h);
+      const bool in = row >= tile_col;
+      decay[i] = in ? expf(sm.gate[kG][row] - sm.gate[kG][tile_col]) : 0.0f;
+      sm.pd[row][tile_col] = in ? dp[i] * decay[i] : 0.0f;
+      products[i] = in ? dp[i] * p_memory.get(tile_at, tile_row(i, 0) * kSquareRow) : 0.0f;
+    }
+    tile_sums(products, sm.row_p, sm.col_p, nullptr);
+  }
+  lds_barrier();
+  if (lower) {
+    const float fk = sm.gate[kBeta][tile_col] * sm.gate[kE][tile_col] * sm.gate[kKScale][tile_col];
+    const unsigned k_at = tile_col * v.row_bytes + 16 * h;
+#pragma unroll
+    for (int s = 0; s < kD / 8; ++s)
+      dt = mma(dt, load4(&sm.dw[32 * ti_own + n][8 * s + 4 * h]), scaled(k_memory.get4(k_at, 32 * s), fk));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sm.x[32 * ti_own + tile_row(i, h)][tile_col] = dt[i];
+  }
+  lds_barrier();
+  floatx16 z = zero_tile();
+  if (lower) {
+    // T^T dT: rows k < i of T's column i are zero, tile (0, 1) of dT is not needed
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s >= 4 * ti_own)
+        z = mma(z, tm.gather4(4 * h * kSquareRow + 4 * (32 * ti_own + n), 8 * s * kSquareRow, kSquareRow),
+                gather4(&sm.x[8 * s + 4 * h][tile_col], kSquarePad));
+  }
+  lds_barrier();
+  if (lower) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sm.x[32 * ti_own + tile_row(i, h)][tile_col] = z[i];
+  }
+  lds_barrier();
+  floatx16 da = zero_tile();
+  if (lower) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s < 4 * (tj_own + 1))
+        da = mma(da, load4(&sm.x[32 * ti_own + n][8 * s + 4 * h]),
+                 tm.get4(tile_col * kSquareRow + 16 * h, 32 * s));
+  }
+  lds_barrier();
+  if (lower) {
+    // R + R^T, and the sums of N = dA (k^ . k^) D
+    float products[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 32 * ti_own + tile_row(i, h);
+      const bool in = row > tile_col;
+      const float value = in ? -da[i] : 0.0f;
+      products[i] = value * kkd.get(tile_at, tile_row(i, 0) * kSquareRow);
+      const float r = value * sm.gate[kBeta][row] * decay[i];
+      if (row >= tile_col) sm.x[row][tile_col] = sm.x[tile_col][row] = r;
+    }
+    tile_sums(products, sm.row_n, sm.col_n, sm.gate[kBeta]);
+  }
+  // columns of K^ and Q^, both as operands and in the accumulators' rows
+  float4 kc[8], qc[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const int i = 8 * s + 4 * h;
+    const float4 ks = load4(&sm.gate[kKScale][i]), qs = load4(&sm.gate[kQScale][i]);
+    const float4 k = k_memory.gather4(token_at, 8 * s * v.row_bytes, v.row_bytes);
+    const float4 q = q_memory.gather4(token_at, 8 * s * v.row_bytes, v.row_bytes);
+    kc[s] = make_float4(k.x * ks.x, k.y * ks.y, k.z * ks.z, k.w * ks.w);
+    qc[s] = make_float4(q.x * qs.x, q.y * qs.y, q.z * qs.z, q.w * qs.w);
+  }
+  auto element = [](const float4 (&c)[8], int ti, int i) {
+    const float4 four = c[4 * ti + i / 4];
+    return i % 4 == 0 ? four.x : i % 4 == 1 ? four.y : i % 4 == 2 ? four.z : four.w;
+  };
+  auto row_sums = [&](RowSum which, int ti, const float (&values)[16]) {
+    const float sum = half_sums(values);
+    if (n % 2 == 0) sm.parts[which][32 * ti + tile_row(n / 2, h)][wave] = sum;
+  };
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti) {
+    float first[16], second[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = 32 * ti + tile_row(i, h);
-      const float d = row >= col ? expf(g_cum[row] - g_cum[col]) : 0.0f;
-      const float kv = row > col ? kk[i] * d : 0.0f;
-      a.r.p[rec * kSquare + row * kC + col] = row >= col ? qk[i] * d : 0.0f;
-      a.r.kkd[rec * kSquare + row * kC + col] = kv;
-      am[row][col] = beta_s[row] * kv;
+      dq[ti][i] *= sm.gate[kE][row];
+      dk[ti][i] *= sm.gate[kL][row];
+      first[i] = dq[ti][i] * element(qc, ti, i);
+      second[i] = dk[ti][i] * element(kc, ti, i);
     }
+    row_sums(kSumQ, ti, first);
+    row_sums(kSumK, ti, second);
   }
-  __syncthreads();
-  // T = (I + A)^-1 by forward substitution, one column a lane
-  if (wave == 0) {
-    float x[kC];
+  lds_barrier();
 #pragma unroll
-    for (int i = 0; i < kC; ++i) {
-      float s = i == lane ? 1.0f : 0.0f;
+  for (int ti = 0; ti < 2; ++ti) {
+    const int m = 32 * ti + n;
+    float4 t_col[8];
 #pragma unroll
-      for (int j = 0; j < i; ++j) s -= am[i][j] * x[j];
-      x[i] = s;
+    for (int s = 4 * ti; s < 8; ++s) t_col[s] = tm.gather4(4 * h * kSquareRow + 4 * m, 8 * s * kSquareRow, kSquareRow);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int k = 8 * s + 4 * h;
+      if (s < 4 * (ti + 1)) dq[ti] = mma(dq[ti], load4(&sm.pd[m][k]), kc[s]);
+      dk[ti] = mma(dk[ti], load4(&sm.x[m][k]), kc[s]);
+      if (s >= 4 * ti) dk[ti] = mma(dk[ti], gather4(&sm.pd[k][m], kSquarePad), qc[s]);
     }
-    const float fv = beta_s[lane], fk = fv * expf(g_cum[lane]);
+    __builtin_amdgcn_sched_barrier(0);
+    float products[16];
+    {
+      floatx16 tw = zero_tile();
 #pragma unroll
-    for (int i = 0; i < kC; ++i) {
-      tk[i][lane] = x[i] * fk;
-      tv[i][lane] = x[i] * fv;
-      a.r.tm[rec * kSquare + i * kC + lane] = x[i];
-    }
-  }
-  __syncthreads();
-  // W = T diag(beta E) K^, U = T diag(beta) V: the wave owns 32 columns
-  {
-    const int col = 32 * wave + n;
-    const size_t value_offset = 2 * static_cast<size_t>(a.kh) * kD + static_cast<size_t>(head) * kD;
-#pragma unroll
-    for (int ti = 0; ti < 2; ++ti) {
-      const floatx16 wacc = product<kC>(zero_tile(), [&](int k) { return tk[32 * ti + n][k]; },
-                                        [&](int k) { return ks[k][col]; });
-      const floatx16 uacc = product<kC>(
-          zero_tile(), [&](int k) { return tv[32 * ti + n][k]; },
-          [&](int k) {
-            const int t = t0 + k, row = min(t, a.length - 1);
-            return keep(t < a.length, a.post[static_cast<size_t>(row) * channels + value_offset + col]);
-          });
+      for (int s = 4 * ti; s < 8; ++s)
+        tw = mma(tw, t_col[s], gather4(&sm.dw[8 * s + 4 * h][col], kWidePad));
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int row = 32 * ti + tile_row(i, h);
-        a.r.w[rec * kWide + row * kD + col] = wacc[i];
-        a.r.u[rec * kWide + row * kD + col] = uacc[i];
+        products[i] = tw[i] * element(kc, ti, i) * sm.gate[kE][row];
+        dk[ti][i] += sm.gate[kBeta][row] * sm.gate[kE][row] * tw[i];
       }
+      row_sums(kSumW, ti, products);
     }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The matrices of the two affine recurrences that depend on the chunk alone:
-// M, M^T, B and Y.  Wave w owns columns 32w..32w+31 of each.
-__global__ void __launch_bounds__(256)
-chunk_transfer_kernel(ChunkedArgs a) {
-  __shared__ float e_s[kC], l_s[kC];
-  const int chunk = blockIdx.x, head = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int h = lane / 32, n = lane % 32;
-  const size_t rec = static_cast<size_t>(head) * a.chunks + chunk;
-  const float* gates = a.r.gates + rec * kGateRows * kC;
-  const float* Q = a.r.qn + rec * kWide;
-  const float* K = a.r.kn + rec * kWide;
-  const float* W = a.r.w + rec * kWide;
-  const float* U = a.r.u + rec * kWide;
-  const float* P = a.r.p + rec * kSquare;
-  if (tid < kC) {
-    e_s[tid] = gates[4 * kC + tid];
-    l_s[tid] = gates[5 * kC + tid];
-  }
-  __syncthreads();
-  const int col = 32 * wave + n;
-  // Y = diag(E) Q^ - P W
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti) {
-    floatx16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      acc[i] = e_s[row] * Q[row * kD + col];
-    }
-    const int m = 32 * ti + n;
-    acc = product4<kC>(acc, [&](int k) { return scaled(load4(P + m * kC + k), -1.0f); },
-                       [&](int k) { return gather4(W + k * kD + col, kD); });
-#pragma unroll
-    for (int i = 0; i < 16; ++i) a.r.y[rec * kWide + (32 * ti + tile_row(i, h)) * kD + col] = acc[i];
-  }
-  // M = E_63 I - (diag(L) K^)^T W and B = (diag(L) K^)^T U
-  const float e_last = e_s[kC - 1];
-#pragma unroll
-  for (int td = 0; td < 4; ++td) {
-    const int m = 32 * td + n;
-    floatx16 macc;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) macc[i] = 32 * td + tile_row(i, h) == col ? e_last : 0.0f;
-    macc = product<kC>(macc, [&](int k) { return -l_s[k] * K[k * kD + m]; },
-                       [&](int k) { return W[k * kD + col]; });
-    const floatx16 bacc = product<kC>(zero_tile(), [&](int k) { return l_s[k] * K[k * kD + m]; },
-                                      [&](int k) { return U[k * kD + col]; });
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int row = 32 * td + tile_row(4 * i4, h);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        a.r.m[rec * kState + (row + e) * kD + col] = macc[4 * i4 + e];
-        a.r.bc[rec * kState + (row + e) * kD + col] = bacc[4 * i4 + e];
-      }
-      *reinterpret_cast<float4*>(a.r.mt + rec * kState + col * kD + row) =
-          make_float4(macc[4 * i4], macc[4 * i4 + 1], macc[4 * i4 + 2], macc[4 * i4 + 3]);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// next = matrix . state + offset over the chunks of one (head, 16 value
-// columns): forward (REVERSE false) it stores the state entering every chunk,
-// with matrix M (read through its transpose) and offset B; in reverse it
-// stores the state gradient leaving every chunk, with matrix M^T (read through
-// M) and offset C.  Wave w keeps rows 32w..32w+31 of the slice; the matrix
-// column and the offset tile of the next chunk are requested while the
-// current product runs.
-template <bool REVERSE>
-__global__ void __launch_bounds__(256)
-chunk_states_kernel(ChunkedArgs a) {
-  __shared__ float state[2][kD][kSlice];
-  // The eight column slices of a head read the same matrices: they are given
-  // block numbers with the same remainder mod 8, which the hardware places on
-  // one XCD, so that seven of the eight reads are served by that XCD's L2.
-  constexpr int kSlices = kD / kSlice;
-  static_assert(kSlices == 8, "one slice of a head per block of an XCD's share");
-  int head = blockIdx.x / kSlices, slice = blockIdx.x % kSlices;
-  if (a.vh % 8 == 0) {
-    head = (blockIdx.x % 8) * (a.vh / 8) + blockIdx.x / 64;
-    slice = (blockIdx.x / 8) % kSlices;
-  }
-  const int col0 = slice * kSlice;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int quarter = lane / 16, n = lane % 16;
-  const float* matrices = REVERSE ? a.r.m : a.r.mt;
-  const float* offsets = REVERSE ? a.r.cc : a.r.bc;
-  float* saved = REVERSE ? a.r.ds1 : a.r.s0;
-  auto record = [&](int step) {
-    return static_cast<size_t>(head) * a.chunks + (REVERSE ? a.chunks - 1 - step : step);
-  };
-  // v_mfma_f32_16x16x4_f32: lane (quarter, n) supplies A[n][quarter] and
-  // B[quarter][n] and receives C[4 quarter + e][n], e = 0..3.  The wave's 32
-  // rows are two such tiles, interleaved (tile t holds rows 2i + t) so that a
-  // lane's two matrix elements of a step are neighbours in memory.
-  constexpr int kSteps = kD / 4;
-  struct Operands {
-    float2 matrix[kSteps];
-    floatx4 offset[2];
-  };
-  auto row_of = [&](int tile, int e) { return 32 * wave + 8 * quarter + 2 * e + tile; };
-  auto matrix_of = [&](int step) {
-    return matrices + record(min(step, a.chunks - 1)) * kState + 32 * wave + 2 * n + quarter * kD;
-  };
-  auto request_matrix = [&](const float* source, Operands& o, int s) {
-    o.matrix[s] = *reinterpret_cast<const float2*>(source + 4 * s * kD);
-  };
-  auto request_offset = [&](int step, Operands& o) {
-    const size_t rec = record(min(step, a.chunks - 1));
-#pragma unroll
-    for (int tile = 0; tile < 2; ++tile)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        o.offset[tile][e] = offsets[rec * kState + row_of(tile, e) * kD + col0 + n];
-  };
-  auto request = [&](int step, Operands& o) {
-    const float* source = matrix_of(step);
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) request_matrix(source, o, s);
-    request_offset(step, o);
-  };
-  floatx4 acc[2];
-#pragma unroll
-  for (int tile = 0; tile < 2; ++tile)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[tile][e] = 0.0f;
-  // One chunk: publish the state, multiply with the operands requested two
-  // chunks ago, request those of the chunk after next.  Three register sets
-  // take turns.  The requests are spread between the multiplications (their
-  // address arithmetic runs while the matrix pipe is busy) and come after the
-  // first of them in program order: the wait for this chunk's operands then
-  // has fewer than 64 younger memory operations behind it, which is as far as
-  // the counter reaches.  Requests are unconditional (past the end they repeat
-  // the last chunk's) so that the number in flight is the same on every path.
-  auto advance = [&](int step, const Operands& now, Operands& later) {
-    float (*current)[kSlice] = state[step & 1];
-#pragma unroll
-    for (int tile = 0; tile < 2; ++tile)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) current[row_of(tile, e)][n] = acc[tile][e];
-    if (step < a.chunks) {
-      const size_t rec = record(step);
-#pragma unroll
-      for (int tile = 0; tile < 2; ++tile)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          saved[rec * kState + row_of(tile, e) * kD + col0 + n] = acc[tile][e];
-    }
-    lds_barrier();
-    acc[0] = now.offset[0];
-    acc[1] = now.offset[1];
-    const float* source = matrix_of(step + 2);
-    float b[kSteps];
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) b[s] = current[4 * s + quarter][n];
     __builtin_amdgcn_sched_barrier(0);
+    {
+      floatx16 tu = zero_tile();
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.matrix[s].x, b[s], acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.matrix[s].y, b[s], acc[1], 0, 0, 0);
-      request_matrix(source, later, s);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    request_offset(step + 2, later);
-  };
-  Operands set0, set1, set2;
-  request(0, set0);
-  request(1, set1);
-  for (int step = 0; step < a.chunks; step += 3) {
-    advance(step, set0, set2);
-    advance(step + 1, set1, set0);
-    advance(step + 2, set2, set1);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Dl = U - W S and O = diag(E) Q^ S + P Dl of one chunk.  Wave w owns value
-// columns 32w..32w+31.
-__global__ void __launch_bounds__(256)
-chunk_outputs_kernel(ChunkedArgs a) {
-  __shared__ float delta[kC][kD];
-  __shared__ float e_s[kC];
-  const int chunk = blockIdx.x, head = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int h = lane / 32, n = lane % 32;
-  const size_t rec = static_cast<size_t>(head) * a.chunks + chunk;
-  const float* gates = a.r.gates + rec * kGateRows * kC;
-  const float* S0 = a.r.s0 + rec * kState;
-  const float* Q = a.r.qn + rec * kWide;
-  const float* W = a.r.w + rec * kWide;
-  const float* U = a.r.u + rec * kWide;
-  const float* P = a.r.p + rec * kSquare;
-  if (tid < kC) e_s[tid] = gates[4 * kC + tid];
-  const int col = 32 * wave + n;
-  floatx16 out[2];
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti) {
-    const int m = 32 * ti + n;
-    floatx16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = U[(32 * ti + tile_row(i, h)) * kD + col];
-    acc = product4<kD, true>(acc, [&](int k) { return scaled(load4(W + m * kD + k), -1.0f); },
-                       [&](int k) { return gather4(S0 + k * kD + col, kD); });
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      delta[row][col] = acc[i];
-      a.r.dl[rec * kWide + row * kD + col] = acc[i];
-    }
-    out[ti] = product4<kD, true>(zero_tile(), [&](int k) { return load4(Q + m * kD + k); },
-                           [&](int k) { return gather4(S0 + k * kD + col, kD); });
-  }
-  __syncthreads();
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti) {
-    const int m = 32 * ti + n;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) out[ti][i] *= e_s[32 * ti + tile_row(i, h)];
-    // only columns j <= i of P are set: the second row tile needs all 64
-    out[ti] = product4<kC, true>(out[ti], [&](int k) { return load4(P + m * kC + k); },
-                           [&](int k) {
-                             return make_float4(delta[k][col], delta[k + 1][col], delta[k + 2][col],
-                                                delta[k + 3][col]);
-                           });
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int t = chunk * kC + 32 * ti + tile_row(i, h);
-      if (t < a.length)
-        a.core[(static_cast<size_t>(t) * a.vh + head) * kD + col] = round_if(out[ti][i], a.round);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// C = Y^T dO of one chunk.
-__global__ void __launch_bounds__(256)
-chunk_local_kernel(ChunkedArgs a) {
-  const int chunk = blockIdx.x, head = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int h = lane / 32, n = lane % 32;
-  const size_t rec = static_cast<size_t>(head) * a.chunks + chunk;
-  const float* Y = a.r.y + rec * kWide;
-  const int col = 32 * wave + n, t0 = chunk * kC;
-#pragma unroll
-  for (int td = 0; td < 4; ++td) {
-    const int m = 32 * td + n;
-    const floatx16 acc = product<kC>(
-        zero_tile(), [&](int k) { return Y[k * kD + m]; },
-        [&](int k) {
-          const int t = t0 + k, row = min(t, a.length - 1);
-          return keep(t < a.length, a.dcore[(static_cast<size_t>(row) * a.vh + head) * kD + col]);
-        });
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      a.r.cc[rec * kState + (32 * td + tile_row(i, h)) * kD + col] = acc[i];
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The gradients of one chunk, in four kernels that exchange [64, 128] and
-// [64, 64] matrices through the records.  In each, wave w owns columns
-// 32w..32w+31 of the [64, 128] matrices (two 32-row tiles) or one 32 x 32 tile
-// of a [64, 64] matrix.
-
-// Sums over the 32 lanes of a half wave of sixteen values at once: the five
-// exchange stages are the outer loop, so that the sixteen exchanges of a stage
-// are in flight together (one value at a time, each stage waits for the one
-// before and the sums cost ten times as much).
-__device__ inline void half_sums(float (&v)[16]) {
-#pragma unroll
-  for (int offset = 16; offset > 0; offset >>= 1) {
-    float other[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) other[i] = __shfl_xor(v[i], offset, 64);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] += other[i];
-  }
-}
-
-// Sums over the four waves of per-row partial sums left in parts[row][wave].
-__device__ inline float across_waves(const float (*parts)[4], int row) {
-  return (parts[row][0] + parts[row][1]) + (parts[row][2] + parts[row][3]);
-}
-
-struct ChunkView {
-  size_t rec;
-  int t0, head, channels;
-  size_t value_offset;
-  const float *gates, *S0, *dS1, *Dl, *Q, *K, *Tm, *P, *KKD;
-};
-
-__device__ inline ChunkView chunk_view(const ChunkedArgs& a, int chunk, int head) {
-  ChunkView v;
-  v.rec = static_cast<size_t>(head) * a.chunks + chunk;
-  v.t0 = chunk * kC;
-  v.head = head;
-  v.channels = 2 * a.kh * kD + a.vh * kD;
-  v.value_offset = 2 * static_cast<size_t>(a.kh) * kD + static_cast<size_t>(head) * kD;
-  v.gates = a.r.gates + v.rec * kGateRows * kC;
-  v.S0 = a.r.s0 + v.rec * kState;
-  v.dS1 = a.r.ds1 + v.rec * kState;
-  v.Dl = a.r.dl + v.rec * kWide;
-  v.Q = a.r.qn + v.rec * kWide;
-  v.K = a.r.kn + v.rec * kWide;
-  v.Tm = a.r.tm + v.rec * kSquare;
-  v.P = a.r.p + v.rec * kSquare;
-  v.KKD = a.r.kkd + v.rec * kSquare;
-  return v;
-}
-
-// A 1-D grid of `parts` workgroups per (head, chunk) unit that read the same
-// records: the parts of a unit get block numbers with the same remainder mod 8
-// (one XCD, hence one L2) and next to each other in launch order.
-struct UnitPart {
-  int chunk, head, part;
-};
-__device__ inline UnitPart unit_part(const ChunkedArgs& a, int parts) {
-  const int units = a.chunks * a.vh, b = blockIdx.x;
-  int unit = b / parts, part = b % parts;
-  if (units % 8 == 0) {
-    part = (b / 8) % parts;
-    unit = (b / (8 * parts)) * 8 + b % 8;
-  }
-  return {unit % a.chunks, unit / a.chunks, part};
-}
-
-// Rows of dO and V; tokens beyond the sequence read as zero.
-__device__ inline float4 d_out4(const ChunkedArgs& a, const ChunkView& v, int i, int c) {
-  const int t = v.t0 + i, row = min(t, a.length - 1);
-  return keep(t < a.length, load4(a.dcore + (static_cast<size_t>(row) * a.vh + v.head) * kD + c));
-}
-__device__ inline float d_out1(const ChunkedArgs& a, const ChunkView& v, int i, int c) {
-  const int t = v.t0 + i, row = min(t, a.length - 1);
-  return keep(t < a.length, a.dcore[(static_cast<size_t>(row) * a.vh + v.head) * kD + c]);
-}
-__device__ inline float4 value4(const ChunkedArgs& a, const ChunkView& v, int j, int c) {
-  const int t = v.t0 + j, row = min(t, a.length - 1);
-  return keep(t < a.length, load4(a.post + static_cast<size_t>(row) * v.channels + v.value_offset + c));
-}
-__device__ inline float value1(const ChunkedArgs& a, const ChunkView& v, int j, int c) {
-  const int t = v.t0 + j, row = min(t, a.length - 1);
-  return keep(t < a.length, a.post[static_cast<size_t>(row) * v.channels + v.value_offset + c]);
-}
-
-// dDl = P^T dO + diag(L) K^ dS'
-__global__ void __launch_bounds__(256)
-chunk_delta_gradient_kernel(ChunkedArgs a) {
-  const ChunkView v = chunk_view(a, blockIdx.x, blockIdx.y);
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int h = lane / 32, n = lane % 32, col = 32 * wave + n;
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti) {
-    const int m = 32 * ti + n;
-    floatx16 acc = product<kC, true>(zero_tile(), [&](int k) { return v.P[k * kC + m]; },
-                               [&](int k) { return d_out1(a, v, k, col); });
-    const float l = v.gates[5 * kC + m];
-    acc = product4<kD, true>(acc, [&](int k) { return scaled(load4(v.K + m * kD + k), l); },
-                       [&](int k) { return gather4(v.dS1 + k * kD + col, kD); });
-#pragma unroll
-    for (int i = 0; i < 16; ++i) a.r.ddl[v.rec * kWide + (32 * ti + tile_row(i, h)) * kD + col] = acc[i];
-  }
-}
-
-// Products against the two states, one per part of a unit:
-//   0: dW = -dDl S^T
-//   1: diag(E) dO S^T (the first part of dq^) and its row sums against q^
-//   2: diag(L) Dl dS'^T (the first part of dk^), its row sums against k^, <dS', S>
-// Both operands are contiguous along the contraction and are read in 16-byte
-// pieces, one row a lane.  (Staging them in LDS with coalesced loads first
-// measured the same 88 us: the kernel moves 270 MB.)
-__global__ void __launch_bounds__(256)
-chunk_state_products_kernel(ChunkedArgs a) {
-  __shared__ float parts[kC][4];
-  __shared__ float reduce[256];
-  const UnitPart u = unit_part(a, 3);
-  const ChunkView v = chunk_view(a, u.chunk, u.head);
-  const int which = u.part;
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int h = lane / 32, n = lane % 32, col = 32 * wave + n;
-  const float* dDl = a.r.ddl + v.rec * kWide;
-  float* sums = a.r.sums + v.rec * kSumRows * kC;
-  const float* state = which == 2 ? v.dS1 : v.S0;
-  float* target = (which == 0 ? a.r.dwm : which == 1 ? a.r.dqp : a.r.dkp) + v.rec * kWide;
-  const float* against = which == 1 ? v.Q : v.K;
-  float dot = 0.0f;
-  if (which == 2) {
-    const int c4 = 4 * (tid % 32);
-#pragma unroll
-    for (int j = 0; j < kD / 8; ++j) {
-      const int row = tid / 32 + 8 * j;
-      const float4 x = load4(v.S0 + row * kD + c4), y = load4(v.dS1 + row * kD + c4);
-      dot += (x.x * y.x + x.y * y.y) + (x.z * y.z + x.w * y.w);
-    }
-  }
-  reduce[tid] = dot;
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti) {
-    const int m = 32 * ti + n;
-    const float factor = which == 0 ? -1.0f : v.gates[(which == 1 ? 4 : 5) * kC + m];
-    const floatx16 acc = product4<kD, true>(
-        zero_tile(),
-        [&](int k) {
-          const float4 row = which == 0   ? load4(dDl + m * kD + k)
-                             : which == 1 ? d_out4(a, v, m, k)
-                                          : load4(v.Dl + m * kD + k);
-          return scaled(row, factor);
-        },
-        [&](int k) { return load4(state + col * kD + k); });
-    float weighted[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      target[row * kD + col] = acc[i];
-      weighted[i] = which != 0 ? acc[i] * against[row * kD + col] : 0.0f;
-    }
-    if (which != 0) {
-      half_sums(weighted);
-      if (n == 0) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) parts[32 * ti + tile_row(i, h)][wave] = weighted[i];
-      }
-    }
-  }
-  if (which == 0) return;
-  __syncthreads();
-  if (tid < kC) sums[(which - 1) * kC + tid] = across_waves(parts, tid);
-  if (which == 2 && tid == 0) {
-    float total = 0.0f;
-    for (int j = 0; j < 256; ++j) total += reduce[j];
-    sums[6 * kC] = total;
-  }
-}
-
-// The [64, 64] part: dP = lower(dO Dl^T), dT = dW (diag(beta E) K^)^T +
-// dDl (diag(beta) V)^T, dA = -strict_lower(T^T dT T^T); leaves Pd = dP D and
-// R = diag(beta) dA D in the records, and the row and column sums that feed
-// d beta and d log-decay.
-__global__ void __launch_bounds__(256)
-chunk_triangle_kernel(ChunkedArgs a) {
-  __shared__ float mx[kC][kC + 1], mz[kC][kC + 1], mu[kC][kC + 1];
-  __shared__ float g_s[kC], beta_s[kC];
-  const ChunkView v = chunk_view(a, blockIdx.x, blockIdx.y);
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int h = lane / 32, n = lane % 32;
-  const int ti = wave / 2, tj = wave % 2;
-  const float* dDl = a.r.ddl + v.rec * kWide;
-  const float* dW = a.r.dwm + v.rec * kWide;
-  float* sums = a.r.sums + v.rec * kSumRows * kC;
-  if (tid < kC) {
-    g_s[tid] = v.gates[tid];
-    beta_s[tid] = v.gates[kC + tid];
-  }
-  __syncthreads();
-  const int col = 32 * tj + n;
-  {
-    floatx16 dp = zero_tile();
-    if (ti >= tj)
-      dp = product4<kD>(dp, [&](int k) { return d_out4(a, v, 32 * ti + n, k); },
-                        [&](int k) { return load4(v.Dl + col * kD + k); });
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      const bool lower = row >= col;
-      const float value = lower ? dp[i] : 0.0f;
-      a.r.pd[v.rec * kSquare + row * kC + col] = lower ? value * expf(g_s[row] - g_s[col]) : 0.0f;
-      mu[row][col] = value * v.P[row * kC + col];
-    }
-  }
-  {
-    const float fv = beta_s[col], fk = fv * v.gates[4 * kC + col];
-    floatx16 acc = product4<kD>(zero_tile(), [&](int k) { return load4(dW + (32 * ti + n) * kD + k); },
-                                [&](int k) { return scaled(load4(v.K + col * kD + k), fk); });
-    acc = product4<kD>(acc, [&](int k) { return load4(dDl + (32 * ti + n) * kD + k); },
-                       [&](int k) { return scaled(value4(a, v, col, k), fv); });
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mx[32 * ti + tile_row(i, h)][col] = acc[i];
-  }
-  __syncthreads();
-  {
-    const floatx16 acc = product<kC>(zero_tile(), [&](int k) { return v.Tm[k * kC + 32 * ti + n]; },
-                                     [&](int k) { return mx[k][col]; });
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mz[32 * ti + tile_row(i, h)][col] = acc[i];
-  }
-  __syncthreads();
-  {
-    floatx16 acc = zero_tile();
-    if (ti >= tj)
-      acc = product<kC>(acc, [&](int k) { return -mz[32 * ti + n][k]; },
-                        [&](int k) { return v.Tm[col * kC + k]; });
-    __syncthreads();  // X has been read by every wave
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      const bool lower = row > col;
-      const float da = lower ? acc[i] : 0.0f;
-      mz[row][col] = da * v.KKD[row * kC + col];  // N
-      a.r.rr[v.rec * kSquare + row * kC + col] =
-          lower ? da * beta_s[row] * expf(g_s[row] - g_s[col]) : 0.0f;
-    }
-  }
-  __syncthreads();
-  if (tid < kC) {
-    // row sums of N and of dP P; column sums of diag(beta) N and of dP P
-    float row_n = 0.0f, col_m = 0.0f, row_p = 0.0f, col_p = 0.0f;
-    for (int j = 0; j < kC; ++j) {
-      row_n += mz[tid][j];
-      col_m += beta_s[j] * mz[j][tid];
-      row_p += mu[tid][j];
-      col_p += mu[j][tid];
-    }
-    sums[2 * kC + tid] = row_n;
-    sums[3 * kC + tid] = col_m;
-    sums[4 * kC + tid] = row_p;
-    sums[5 * kC + tid] = col_p;
-  }
-}
-
-// dq and dk (back through the normalisations) and dv of 32 rows of a chunk
-// (the unit's part picks the row tile), and the row sums of those rows that the
-// gate gradients need.
-__global__ void __launch_bounds__(256)
-chunk_finish_kernel(ChunkedArgs a) {
-  __shared__ float parts[4][kC / 2][4];
-  __shared__ float e_s[kC], beta_s[kC];
-  const UnitPart u = unit_part(a, 2);
-  const ChunkView v = chunk_view(a, u.chunk, u.head);
-  const int ti = u.part;
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int h = lane / 32, n = lane % 32, col = 32 * wave + n;
-  const float* dDl = a.r.ddl + v.rec * kWide;
-  const float* dW = a.r.dwm + v.rec * kWide;
-  const float* Pd = a.r.pd + v.rec * kSquare;
-  const float* R = a.r.rr + v.rec * kSquare;
-  float* sums = a.r.sums + v.rec * kSumRows * kC;
-  if (tid < kC) {
-    e_s[tid] = v.gates[4 * kC + tid];
-    beta_s[tid] = v.gates[kC + tid];
-  }
-  __syncthreads();
-  const int m = 32 * ti + n;
-  floatx16 dq, dk;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = 32 * ti + tile_row(i, h);
-    dq[i] = a.r.dqp[v.rec * kWide + row * kD + col];
-    dk[i] = a.r.dkp[v.rec * kWide + row * kD + col];
-  }
-  // dq^ += Pd K^
-  dq = product4<kC>(dq, [&](int k) { return load4(Pd + m * kC + k); },
-                    [&](int k) { return gather4(v.K + k * kD + col, kD); });
-  // T^T dW = d(diag(beta E) K^)
-  const floatx16 tw = product<kC>(zero_tile(), [&](int k) { return v.Tm[k * kC + m]; },
-                                  [&](int k) { return dW[k * kD + col]; });
-  {
-    float weighted[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      weighted[i] = tw[i] * v.K[row * kD + col] * e_s[row];
-      dk[i] += beta_s[row] * e_s[row] * tw[i];
-    }
-    half_sums(weighted);
-    if (n == 0) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) parts[0][tile_row(i, h)][wave] = weighted[i];
-    }
-  }
-  // dk^ += (R + R^T) K^ + Pd^T Q^
-  dk = product4<kC>(dk, [&](int k) { return load4(R + m * kC + k); },
-                    [&](int k) { return gather4(v.K + k * kD + col, kD); });
-  dk = product<kC>(dk, [&](int k) { return R[k * kC + m]; },
-                   [&](int k) { return v.K[k * kD + col]; });
-  dk = product<kC>(dk, [&](int k) { return Pd[k * kC + m]; },
-                   [&](int k) { return v.Q[k * kD + col]; });
-  // dv = diag(beta) T^T dDl
-  const floatx16 tu = product<kC>(zero_tile(), [&](int k) { return v.Tm[k * kC + m]; },
-                                  [&](int k) { return dDl[k * kD + col]; });
-  {
-    float rv[16], q_dot[16], k_dot[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h), t = v.t0 + row;
-      rv[i] = tu[i] * value1(a, v, row, col);
-      q_dot[i] = dq[i] * v.Q[row * kD + col];
-      k_dot[i] = dk[i] * v.K[row * kD + col];
-      if (t < a.length)
-        a.dpost[static_cast<size_t>(t) * v.channels + v.value_offset + col] = beta_s[row] * tu[i];
-    }
-    half_sums(rv);
-    half_sums(q_dot);
-    half_sums(k_dot);
-    if (n == 0) {
+      for (int s = 4 * ti; s < 8; ++s)
+        tu = mma(tu, t_col[s], ddl.gather4(column_at, 8 * s * kWideRow, kWideRow));
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int local = tile_row(i, h);
-        parts[1][local][wave] = rv[i];
-        parts[2][local][wave] = q_dot[i];
-        parts[3][local][wave] = k_dot[i];
+        const unsigned row = (32 * ti + tile_row(i, 0)) * v.row_bytes;
+        products[i] = tu[i] * v_memory.get(token_at, row);
+        dv.put(sm.gate[kBeta][32 * ti + tile_row(i, h)] * tu[i], token_at, row);
       }
+      row_sums(kSumV, ti, products);
     }
-  }
-  __syncthreads();
-  // back through the L2 normalisations (and the 1/sqrt(d) of q)
-  const float norm_scale = sqrtf(static_cast<float>(kD));
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int local = tile_row(i, h), row = 32 * ti + local, t = v.t0 + row;
-    if (t >= a.length) continue;
-    const float iq = v.gates[2 * kC + row], ik = v.gates[3 * kC + row];
-    const float qv = v.Q[row * kD + col], kv = v.K[row * kD + col];
-    float* out = a.qk_partials + (static_cast<size_t>(t) * a.vh + v.head) * 2 * kD;
-    out[col] = iq / norm_scale *
-               (dq[i] - static_cast<float>(kD) * qv * across_waves(parts[2], local));
-    out[kD + col] = ik * (dk[i] - kv * across_waves(parts[3], local));
+    for (int i = 0; i < 16; ++i) products[i] = dq[ti][i] * element(qc, ti, i);
+    row_sums(kDotQ, ti, products);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) products[i] = dk[ti][i] * element(kc, ti, i);
+    row_sums(kDotK, ti, products);
   }
-  if (tid < kC / 2) {
-    sums[7 * kC + 32 * ti + tid] = across_waves(parts[0], tid);
-    sums[8 * kC + 32 * ti + tid] = across_waves(parts[1], tid);
+  lds_barrier();
+  auto across_waves = [&](RowSum which, int row) {
+    const float4 four = load4(sm.parts[which][row]);
+    return (four.x + four.y) + (four.z + four.w);
+  };
+  const auto partials = v.qk_partials();
+  // back through the L2 normalisations (and the 1/sqrt(d) of q, which kQScale has)
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = 32 * ti + tile_row(i, h);
+      const unsigned uniform = 2 * (32 * ti + tile_row(i, 0)) * v.out_bytes;
+      partials.put(sm.gate[kQScale][row] *
+                       (dq[ti][i] - static_cast<float>(kD) * element(qc, ti, i) * across_waves(kDotQ, row)),
+                   8 * h * v.out_bytes + 4 * col, uniform);
+      partials.put(sm.gate[kKScale][row] * (dk[ti][i] - element(kc, ti, i) * across_waves(kDotK, row)),
+                   8 * h * v.out_bytes + 4 * (kD + col), uniform);
+    }
+  if (wave != 0) return;
+  // the gates: lane i is token i
+  const float beta = sm.gate[kBeta][lane];
+  const float r = across_waves(kSumW, lane), state_k = across_waves(kSumK, lane);
+  const float row_n = sm.row_n[lane][0] + sm.row_n[lane][1];
+  float dg = across_waves(kSumQ, lane) + beta * r +
+             (beta * row_n - (sm.col_n[lane][0] + sm.col_n[lane][1])) +
+             ((sm.row_p[lane][0] + sm.row_p[lane][1]) - (sm.col_p[lane][0] + sm.col_p[lane][1])) -
+             state_k;
+  const float total = wave_sum(state_k);
+  if (lane == kC - 1)
+    dg += total + ((sm.dot[0] + sm.dot[1]) + (sm.dot[2] + sm.dot[3])) * sm.gate[kE][kC - 1];
+#pragma unroll
+  for (int offset = 1; offset < 64; offset <<= 1) {
+    const float after = __shfl_down(dg, offset, 64);
+    if (lane + offset < 64) dg += after;
   }
-}
-
-// d log-decay and d beta of the 64 tokens of a chunk from the row and column
-// sums the other kernels left, then through the gates to da, db and the
-// contribution to d A_log.
-__global__ void __launch_bounds__(64)
-chunk_gates_kernel(ChunkedArgs a) {
-  __shared__ float dg_s[kC];
-  const ChunkView v = chunk_view(a, blockIdx.x, blockIdx.y);
-  const float* sums = a.r.sums + v.rec * kSumRows * kC;
-  const int tid = threadIdx.x;
-  const float beta = v.gates[kC + tid];
-  const float r = sums[7 * kC + tid];
-  float dG = sums[tid] + beta * r + (beta * sums[2 * kC + tid] - sums[3 * kC + tid]) +
-             (sums[4 * kC + tid] - sums[5 * kC + tid]) - sums[kC + tid];
-  if (tid == kC - 1) {
-    float total = 0.0f;
-    for (int j = 0; j < kC; ++j) total += sums[kC + j];
-    dG += total + sums[6 * kC] * v.gates[4 * kC + kC - 1];
-  }
-  dg_s[tid] = dG;
-  __syncthreads();
-  const int t = v.t0 + tid;
-  if (t >= a.length) return;
-  float dg = 0.0f;
-  for (int i = kC - 1; i >= tid; --i) dg += dg_s[i];
-  const float dbeta = sums[2 * kC + tid] + r + sums[8 * kC + tid];
+  const int t = v.t0 + lane;
+  if (lane >= v.tokens) return;
+  const float dbeta = row_n + r + across_waves(kSumV, lane);
   const float alpha = bf16_bits_to_float(a.a[static_cast<size_t>(t) * a.vh + v.head]) + a.dt_bias[v.head];
   const float softplus = fmaxf(alpha, 0.0f) + logf(1.0f + expf(-fabsf(alpha)));
   const float rate = expf(a.a_log[v.head]);
@@ -1012,27 +1101,13 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
     at += n * floats;
     return result;
   };
-  a.r.qn = take(kWide);
-  a.r.kn = take(kWide);
   a.r.w = take(kWide);
-  a.r.u = take(kWide);
-  a.r.y = take(kWide);
   a.r.dl = take(kWide);
   a.r.ddl = take(kWide);
-  a.r.dwm = take(kWide);
-  a.r.dqp = take(kWide);
-  a.r.dkp = take(kWide);
   a.r.p = take(kSquare);
   a.r.tm = take(kSquare);
   a.r.kkd = take(kSquare);
-  a.r.pd = take(kSquare);
-  a.r.rr = take(kSquare);
-  a.r.sums = take(kSumRows * kC);
   a.r.gates = take(kGateRows * kC);
-  a.r.m = take(kState);
-  a.r.mt = take(kState);
-  a.r.bc = take(kState);
-  a.r.cc = take(kState);
   a.r.s0 = take(kState);
   a.r.ds1 = take(kState);
   return a;
@@ -1056,10 +1131,7 @@ int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBack
   chunk_prepare_kernel<<<per_chunk, 256, 0, stream>>>(a);
   int status = launch_status();
   if (status != 0) return status;
-  chunk_transfer_kernel<<<per_chunk, 256, 0, stream>>>(a);
-  status = launch_status();
-  if (status != 0) return status;
-  chunk_states_kernel<false><<<a.vh * (kD / kSlice), 256, 0, stream>>>(a);
+  chunk_states_forward_kernel<<<a.vh * (kD / kSlice), 256, 0, stream>>>(a);
   status = launch_status();
   if (status != 0) return status;
   chunk_outputs_kernel<<<per_chunk, 256, 0, stream>>>(a);
@@ -1068,26 +1140,10 @@ int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBack
 
 int launch_gdn_backward_chunked_reverse(hipStream_t stream, const GdnChunkedBackward& c) {
   const ChunkedArgs a = make_args(c);
-  const dim3 per_chunk(a.chunks, a.vh);
-  chunk_local_kernel<<<per_chunk, 256, 0, stream>>>(a);
-  int status = launch_status();
+  chunk_states_backward_kernel<<<a.vh * (kD / kSlice), 256, 0, stream>>>(a);
+  const int status = launch_status();
   if (status != 0) return status;
-  chunk_states_kernel<true><<<a.vh * (kD / kSlice), 256, 0, stream>>>(a);
-  status = launch_status();
-  if (status != 0) return status;
-  chunk_delta_gradient_kernel<<<per_chunk, 256, 0, stream>>>(a);
-  status = launch_status();
-  if (status != 0) return status;
-  chunk_state_products_kernel<<<a.chunks * a.vh * 3, 256, 0, stream>>>(a);
-  status = launch_status();
-  if (status != 0) return status;
-  chunk_triangle_kernel<<<per_chunk, 256, 0, stream>>>(a);
-  status = launch_status();
-  if (status != 0) return status;
-  chunk_finish_kernel<<<a.chunks * a.vh * 2, 256, 0, stream>>>(a);
-  status = launch_status();
-  if (status != 0) return status;
-  chunk_gates_kernel<<<per_chunk, kC, 0, stream>>>(a);
+  chunk_gradients_kernel<<<dim3(a.chunks, a.vh), 256, 0, stream>>>(a);
   return launch_status();
 }
 
