@@ -22,23 +22,31 @@
 //   dS  = E_63 dS' + (diag(E) Q^)^T dO - W^T dDl.
 // The kernels, in launch order:
 //   chunk_prepare_kernel           T, W, U, P of every chunk          (parallel)
-//   chunk_states_forward_kernel    S entering every chunk, Dl         (sequential)
-//   chunk_outputs_kernel           O                                  (parallel)
+//   chunk_states_forward_kernel    S entering every chunk, Dl, O      (sequential)
 //     -- the caller turns O into dO here --
 //   chunk_states_backward_kernel   dS' leaving every chunk, dDl       (sequential)
 //   chunk_gradients_kernel         everything else                    (parallel)
-// The sequential kernels run one workgroup per (head, 16 value columns).
+// The sequential kernels run one workgroup per (head, 16 or 32 value columns).
 // Eliminating Dl instead makes both recurrences one 128 x 128 matrix a chunk
 // (S' = M S + B) whose product is one link of the chain instead of two, but M, its
 // transpose, B and the offsets of the reverse recurrence are four 64 KiB records a
-// chunk that have to be computed, written and read: at 2048 tokens of 48 heads the
-// kernels that did so took 624 us where the two below take 380.
-// Everything between two states is consumed in the kernel that makes it (LDS and
-// accumulators), so that a chunk's records are 0.27 MB instead of 0.74 MB: all kernels
-// of this file 1766 -> 930 us at that size.
+// chunk that have to be computed, written and read.
+//
+// Layout of the records.  A memory instruction whose lanes take 16 bytes each of 16
+// rows costs a compute unit about 40 clocks, one that takes a contiguous KiB 16, and
+// the sequential kernels issue more of them than their matrix instructions hide.
+// Every matrix is therefore kept in operand order: rows(M) is M in blocks of 16 rows
+// by 4 columns, blocks of a row block after each other, so that the lanes of an
+// operand of rows and of four contraction elements a lane read 1 KiB (16 x 16
+// tiles) or 256-byte pieces (32 x 32 tiles).  columns(M) is rows(M^T): an
+// accumulator, whose lanes are columns and whose registers are four neighbouring rows,
+// is stored in that order as it is.
+//
 // Matrix products run on v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32, whose
-// rate (about 25 GFLOP of them, 165 us of the card's FP32 matrix rate) bounds the
-// gradients kernel; the triangular factors are multiplied by halves.
+// rate bounds all of this (about 55 GFLOP at 2048 tokens of 48 heads, 360 us of the
+// card's FP32 matrix rate); the triangular factors are multiplied by halves.  At that
+// size the kernels of this file take @TOTAL@ us, where one kernel a term of the
+// formulas above, with M and B, took 1766 us.
 #include "gdn.h"
 
 namespace pluto_hip {
@@ -46,7 +54,7 @@ namespace {
 
 constexpr int kC = 64;       // tokens per chunk
 constexpr int kD = 128;      // key and value channels per head
-constexpr int kSlice = 16;   // value columns per workgroup of the sequential kernels
+constexpr int kTile = 16;    // value columns of a tile of the sequential kernels
 constexpr int kWide = kC * kD;     // elements of a [64, 128] record
 constexpr int kSquare = kC * kC;   // elements of a [64, 64] record
 constexpr int kState = kD * kD;    // elements of a state
@@ -55,17 +63,23 @@ constexpr int kSquarePad = kC + 4;
 
 // Per (head, chunk) records in the workspace, in floats.
 struct Records {
-  float *w, *dl, *ddl;        // W; U, which Dl replaces; dDl            [64][128]
-  float *p, *tm, *kkd;        // P, T, strict_lower((k^_i . k^_j) D_ij)  [64][64]
-  float *gates;               // [8][64], see Gate
-  float *s0, *ds1;            // state entering the chunk, gradient of the state leaving it
+  // of a key head                                                        [64][128]
+  float *q_rows, *q_columns, *k_rows, *k_columns;
+  float *w_rows, *w_columns;                          // W              [64][128]
+  float *dl, *ddl;            // columns(U), which columns(Dl) replaces; columns(dDl)
+  float *p_rows, *p_columns;                          // P               [64][64]
+  float *t_rows, *t_columns;                          // T               [64][64]
+  float *kkd;                 // columns(strict_lower((k^_i . k^_j) D_ij)) [64][64]
+  float *gates;               // [6][64], see Gate
+  float *s0, *ds1;            // rows(state entering the chunk), rows(gradient of the one leaving)
 };
 
-// Rows of a gates record.  q^ and k^ are not stored: their rows are those of the
-// convolved activations times kQScale and kKScale (zero beyond the sequence).
-enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kLK, kEQ, kGateRows };  // kLK = L kKScale, ...
+// Rows of a gates record; q^ and k^ are the convolved activations' rows times kQScale
+// and kKScale (zero beyond the sequence).
+enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kGateRows };
 
-constexpr size_t kRecordFloats = 3 * static_cast<size_t>(kWide) + 3 * kSquare + kGateRows * kC +
+constexpr size_t kKeyRecordFloats = 4 * static_cast<size_t>(kWide);
+constexpr size_t kRecordFloats = 4 * static_cast<size_t>(kWide) + 5 * kSquare + kGateRows * kC +
                                  2 * static_cast<size_t>(kState);
 
 struct ChunkedArgs {
@@ -126,6 +140,43 @@ __device__ inline floatx4 mma16(floatx4 acc, float4 a, float4 b) {
 }
 __device__ inline floatx4 mma16(floatx4 acc, float4 a, floatx4 b) {
   return mma16(acc, a, make_float4(b[0], b[1], b[2], b[3]));
+}
+
+// Lanes 4 i .. 4 i + 3 hold the rows of a 4 x 4 matrix; afterwards its columns.
+__device__ inline float4 quad_transpose(float4 v) {
+  auto swap = [](float& low, float& high, bool upper, auto exchange) {
+    const float other = exchange(upper ? low : high);
+    low = upper ? other : low;
+    high = upper ? high : other;
+  };
+  auto with_1 = [](float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));
+  };
+  auto with_2 = [](float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xf, 0xf, true));
+  };
+  const bool odd = threadIdx.x & 1, second = threadIdx.x & 2;
+  swap(v.x, v.y, odd, with_1);
+  swap(v.z, v.w, odd, with_1);
+  swap(v.x, v.z, second, with_2);
+  swap(v.y, v.w, second, with_2);
+  return v;
+}
+
+// One product of several tiles with the same left operand: their chains take turns.
+template <int TILES, class F>
+__device__ inline void mma16_tiles(floatx4 (&acc)[TILES], float4 a, F right) {
+  float4 b[TILES];
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) b[c] = right(c);
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[c].x, acc[c], 0, 0, 0);
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[c].y, acc[c], 0, 0, 0);
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[c].z, acc[c], 0, 0, 0);
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[c].w, acc[c], 0, 0, 0);
 }
 
 __device__ inline float4 gather4(const float* p, int stride) {
@@ -193,6 +244,12 @@ struct Memory {
     else
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, lane, uniform, 0);
   }
+  __device__ void put4(float4 v, unsigned lane, unsigned uniform) const {
+    if (TOKENS)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint32x4, v), rsrc, lane + uniform, 0, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint32x4, v), rsrc, lane, uniform, 0);
+  }
 };
 using Record = Memory<false>;
 using Tokens = Memory<true>;
@@ -215,8 +272,9 @@ struct ChunkView {
   }
   __device__ int key_head() const { return head / (a.vh / a.kh); }
   __device__ int value_column() const { return (2 * a.kh + head) * kD; }
-  __device__ Tokens q() const { return activations(a.post, key_head() * kD); }
-  __device__ Tokens k() const { return activations(a.post, (a.kh + key_head()) * kD); }
+  __device__ Record key(const float* records) const {
+    return Record(records + (static_cast<size_t>(key_head()) * a.chunks + t0 / kC) * kWide, kWide);
+  }
   __device__ Tokens v() const { return activations(a.post, value_column()); }
   __device__ Tokens dv() const { return activations(a.dpost, value_column()); }
   __device__ Tokens heads(const float* base) const {  // O, dO
@@ -231,7 +289,19 @@ struct ChunkView {
   __device__ Record square(const float* records) const { return Record(records + rec * kSquare, kSquare); }
   __device__ Record state(const float* records) const { return Record(records + rec * kState, kState); }
 };
-constexpr unsigned kWideRow = kD * 4, kSquareRow = kC * 4;  // bytes
+
+// Byte offsets in rows(M) of a matrix with COLUMNS columns: four columns of sixteen rows,
+// and a whole 16 x 16 operand.
+constexpr unsigned kPiece = 16 * 4 * 4, kOperand = 4 * kPiece;
+template <int COLUMNS>
+__device__ constexpr unsigned piece_at(int row_block, int quad) {
+  return (row_block * (COLUMNS / 4) + quad) * kPiece;
+}
+// The lane of half h and row n of a 32 x 32 operand: its quads are 2 s + h.
+template <int COLUMNS>
+__device__ inline unsigned lane_piece(int h, int n) {
+  return piece_at<COLUMNS>(n / 16, h) + n % 16 * 16;
+}
 
 // ---------------------------------------------------------------------------
 // T, W, U, P and the gates of one chunk.  68 KiB of LDS, two workgroups a compute
@@ -260,7 +330,8 @@ chunk_prepare_kernel(ChunkedArgs a) {
   // half a wave a row, row 16 wave + 2 r + h
   {
     const float norm_scale = sqrtf(static_cast<float>(kD));
-    const Tokens q = v.q(), k = v.k();
+    const Tokens q = v.activations(a.post, v.key_head() * kD),
+                 k = v.activations(a.post, (a.kh + v.key_head()) * kD);
     const unsigned at = (16 * wave + h) * v.row_bytes + 16 * n;
     float4 rows[16];
     float squares[16];
@@ -281,17 +352,16 @@ chunk_prepare_kernel(ChunkedArgs a) {
       const bool ok = i < v.tokens;
       const float iq = ok ? __shfl(inverse, 32 * h + 4 * r, 64) / norm_scale : 0.0f;
       const float ik = ok ? __shfl(inverse, 32 * h + 4 * r + 2, 64) : 0.0f;
-      store4(&sm.q[i][4 * n], scaled(rows[2 * r], iq));
-      store4(&sm.k[i][4 * n], scaled(rows[2 * r + 1], ik));
+      rows[2 * r] = scaled(rows[2 * r], iq);
+      rows[2 * r + 1] = scaled(rows[2 * r + 1], ik);
+      store4(&sm.q[i][4 * n], rows[2 * r]);
+      store4(&sm.k[i][4 * n], rows[2 * r + 1]);
       if (n == 0) {
         gates[kQScale * kC + i] = iq;
         gates[kKScale * kC + i] = ik;
-        sm.fk[i] = ik;  // until the gates below
-        sm.beta[i] = iq;
       }
     }
   }
-  __syncthreads();
   // gates (sequence_delta_net.cc:88-96); tokens beyond the sequence neither
   // decay nor write
   if (wave == 0) {
@@ -315,8 +385,6 @@ chunk_prepare_kernel(ChunkedArgs a) {
     gates[kBeta * kC + lane] = beta;
     gates[kE * kC + lane] = e;
     gates[kL * kC + lane] = l;
-    gates[kLK * kC + lane] = l * sm.fk[lane];
-    gates[kEQ * kC + lane] = e * sm.beta[lane];
     sm.g[lane] = g;
     sm.beta[lane] = beta;
     sm.fk[lane] = beta * e;
@@ -324,6 +392,8 @@ chunk_prepare_kernel(ChunkedArgs a) {
   __syncthreads();
   // k^ k^T and q^ k^T by 16 x 16 tiles on and below the diagonal: wave w takes row w of
   // the first and row 3 - w of the second, five tiles
+  const bool first_of_group = v.head % (a.vh / a.kh) == 0;
+  const Record k_rows = v.key(a.r.k_rows), q_rows = v.key(a.r.q_rows);
   floatx4 kk[4], qk[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b) kk[b] = qk[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -338,21 +408,53 @@ chunk_prepare_kernel(ChunkedArgs a) {
       if (b <= wave) kk[b] = mma16(kk[b], kr, kc);
       if (b <= 3 - wave) qk[b] = mma16(qk[b], qr, kc);
     }
-  }
-  __syncthreads();  // the rows of q^ make room for A and T
-  const auto kkd = v.square(a.r.kkd), p = v.square(a.r.p);
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int row = 4 * quarter + e, col = 16 * b + n16;
-      const int k_at = 16 * wave + row, q_at = 16 * (3 - wave) + row;
-      const float kv = k_at > col ? kk[b][e] * expf(sm.g[k_at] - sm.g[col]) : 0.0f;
-      kkd.put(kv, 4 * (k_at * kC + n16), 64 * b);
-      p.put(q_at >= col ? qk[b][e] * expf(sm.g[q_at] - sm.g[col]) : 0.0f, 4 * (q_at * kC + n16), 64 * b);
-      sm.a[k_at][col] = sm.beta[k_at] * kv;
-      sm.t[k_at][col] = 0.0f;
+    if (first_of_group) {
+      k_rows.put4(kr, 16 * lane, piece_at<kD>(wave, 4 * s));
+      q_rows.put4(qr, 16 * lane, piece_at<kD>(3 - wave, 4 * s));
     }
+  }
+  if (first_of_group) {
+    const Record k_columns = v.key(a.r.k_columns), q_columns = v.key(a.r.q_columns);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int b = 2 * wave + t;
+        k_columns.put4(gather4(&sm.k[16 * s + 4 * quarter][16 * b + n16], kWidePad), 16 * lane,
+                       piece_at<kC>(b, 4 * s));
+        q_columns.put4(gather4(&sm.q[16 * s + 4 * quarter][16 * b + n16], kWidePad), 16 * lane,
+                       piece_at<kC>(b, 4 * s));
+      }
+  }
+  lds_barrier();  // the rows of q^ make room for P, then A, and for T
+  {
+    const Record kkd = v.square(a.r.kkd), p_columns = v.square(a.r.p_columns), p_rows = v.square(a.r.p_rows);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      float p[4], masked[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = 4 * quarter + e, col = 16 * b + n16;
+        const int k_at = 16 * wave + row, q_at = 16 * (3 - wave) + row;
+        masked[e] = k_at > col ? kk[b][e] * expf(sm.g[k_at] - sm.g[col]) : 0.0f;
+        p[e] = q_at >= col ? qk[b][e] * expf(sm.g[q_at] - sm.g[col]) : 0.0f;
+        kk[b][e] = sm.beta[k_at] * masked[e];
+        sm.a[q_at][col] = p[e];
+        sm.t[k_at][col] = 0.0f;
+      }
+      kkd.put4(make_float4(masked[0], masked[1], masked[2], masked[3]), 16 * lane, piece_at<kC>(b, 4 * wave));
+      p_columns.put4(make_float4(p[0], p[1], p[2], p[3]), 16 * lane, piece_at<kC>(b, 4 * (3 - wave)));
+    }
+    lds_barrier();
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      p_rows.put4(load4(&sm.a[16 * wave + n16][16 * s + 4 * quarter]), 16 * lane, piece_at<kC>(wave, 4 * s));
+    lds_barrier();
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sm.a[16 * wave + 4 * quarter + e][16 * b + n16] = kk[b][e];
+  }
   lds_barrier();
   {
     // diagonal block `wave`, column n16
@@ -416,333 +518,389 @@ chunk_prepare_kernel(ChunkedArgs a) {
   }
   __builtin_amdgcn_sched_barrier(0);
   lds_barrier();
+  {
+    const Record t_rows = v.square(a.r.t_rows), t_columns = v.square(a.r.t_columns);
 #pragma unroll
-  for (int i = 0; i < kC * kC / 4 / 256; ++i) {
-    const int at = tid + 256 * i;
-    store4(a.r.tm + v.rec * kSquare + 4 * at, load4(&sm.t[at / 16][at % 16 * 4]));
+    for (int s = 0; s < 4; ++s) {
+      t_rows.put4(load4(&sm.t[16 * wave + n16][16 * s + 4 * quarter]), 16 * lane, piece_at<kC>(wave, 4 * s));
+      t_columns.put4(gather4(&sm.t[16 * s + 4 * quarter][16 * wave + n16], kSquarePad), 16 * lane,
+                     piece_at<kC>(wave, 4 * s));
+    }
   }
-  const auto w_out = v.wide(a.r.w), u_out = v.wide(a.r.dl);
+  const Record w_columns = v.wide(a.r.w_columns), w_rows = v.wide(a.r.w_rows), u_columns = v.wide(a.r.dl);
+  const unsigned column_at = piece_at<kC>(2 * wave, 0) + lane_piece<kC>(h, n);
+  floatx16 w[2];
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti) {
-    floatx16 w = zero_tile(), u = zero_tile();
+    floatx16 u = zero_tile();
+    w[ti] = zero_tile();
 #pragma unroll
     for (int s = 0; s < 4 * (ti + 1); ++s) {
       const int k = 8 * s + 4 * h;
       const float4 t = load4(&sm.t[32 * ti + n][k]), f = load4(&sm.fk[k]), b = load4(&sm.beta[k]);
-      w = mma(w, make_float4(t.x * f.x, t.y * f.y, t.z * f.z, t.w * f.w), gather4(&sm.k[k][col], kWidePad));
+      w[ti] = mma(w[ti], make_float4(t.x * f.x, t.y * f.y, t.z * f.z, t.w * f.w),
+                  gather4(&sm.k[k][col], kWidePad));
       u = mma(u, make_float4(t.x * b.x, t.y * b.y, t.z * b.z, t.w * b.w), values[s]);
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const unsigned at = 4 * h * kWideRow + 4 * col, row = (32 * ti + tile_row(i, 0)) * kWideRow;
-      w_out.put(w[i], at, row);
-      u_out.put(u[i], at, row);
+    for (int j = 0; j < 4; ++j) {
+      const unsigned at = piece_at<kC>(0, 8 * ti + 2 * j);
+      w_columns.put4(make_float4(w[ti][4 * j], w[ti][4 * j + 1], w[ti][4 * j + 2], w[ti][4 * j + 3]), column_at, at);
+      u_columns.put4(make_float4(u[4 * j], u[4 * j + 1], u[4 * j + 2], u[4 * j + 3]), column_at, at);
     }
   }
+  lds_barrier();  // the rows of k^ make room for W
+#pragma unroll
+  for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sm.k[32 * ti + tile_row(i, h)][col] = w[ti][i];
+  lds_barrier();
+#pragma unroll
+  for (int s = 0; s < 8; ++s)
+    w_rows.put4(load4(&sm.k[16 * wave + n16][16 * s + 4 * quarter]), 16 * lane, piece_at<kD>(wave, 4 * s));
 }
 
 // ---------------------------------------------------------------------------
-// The workgroups of the sequential kernels.  The eight column slices of a head read
-// the same matrices: they are given block numbers with the same remainder mod 8,
-// which the hardware places on one XCD, so that seven of the eight reads are served
-// by that XCD's L2.
+// The workgroups of the sequential kernels: TILES times sixteen value columns of a head.
+// The slices of a head read the same matrices: they are given block numbers with the
+// same remainder mod 8, which the hardware places on one XCD, so that all reads but the
+// first are served by that XCD's L2.
 struct Slice {
   int head, col0;
 };
+template <int TILES>
 __device__ inline Slice slice_of_block(const ChunkedArgs& a) {
-  constexpr int kSlices = kD / kSlice;
-  static_assert(kSlices == 8, "one slice of a head per block of an XCD's share");
+  constexpr int kSlices = kD / (kTile * TILES);
   if (a.vh % 8 == 0)
-    return {static_cast<int>((blockIdx.x % 8) * (a.vh / 8) + blockIdx.x / 64),
-            static_cast<int>(blockIdx.x / 8 % kSlices * kSlice)};
-  return {static_cast<int>(blockIdx.x / kSlices), static_cast<int>(blockIdx.x % kSlices * kSlice)};
+    return {static_cast<int>((blockIdx.x % 8) * (a.vh / 8) + blockIdx.x / (8 * kSlices)),
+            static_cast<int>(blockIdx.x / 8 % kSlices * kTile * TILES)};
+  return {static_cast<int>(blockIdx.x / kSlices), static_cast<int>(blockIdx.x % kSlices * kTile * TILES)};
 }
 
-// The state of a slice lives in accumulators: wave w holds rows 32 w .. 32 w + 31, as two
-// 16 x 16 tiles whose rows are interleaved (row 32 w + 2 i + t is row i of tile t), so
-// that an operand row that is contiguous along them is read two elements a lane and a
-// lane's eight elements are rows 32 w + 8 quarter .. + 7.  `rows` is the LDS copy
-// [column][row] that the other waves multiply.
-__device__ inline void publish_state(const floatx4 (&acc)[2], float* rows) {
-  store4(rows, make_float4(acc[0][0], acc[1][0], acc[0][1], acc[1][1]));
-  store4(rows + 4, make_float4(acc[0][2], acc[1][2], acc[0][3], acc[1][3]));
+// The state of a slice lives in accumulators: tile t of wave w holds rows 32 w + 16 t ..
+// + 15 of sixteen columns.  The LDS copy [column][row] is what the other waves multiply
+// and where the rows of the saved state come from.
+__device__ inline void publish_state(const floatx4& first, const floatx4& second, float* rows) {
+  store4(rows, make_float4(first[0], first[1], first[2], first[3]));
+  store4(rows + 16, make_float4(second[0], second[1], second[2], second[3]));
 }
 
-__device__ inline void save_state(const floatx4 (&acc)[2], const Record& state, unsigned lane) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-#pragma unroll
-    for (int t = 0; t < 2; ++t) state.put(acc[t][e], lane, (2 * e + t) * kWideRow);
+// The records of a head as the sequential kernels walk them: one descriptor for all
+// chunks, a lane offset that moves with the chunk and a uniform place in the record.
+// Chunks have the same size in all records of one kind, so that the kinds share their
+// lane offsets.
+__device__ inline Record head_records(const ChunkedArgs& a, const float* records, int head, size_t elements) {
+  return Record(records + static_cast<size_t>(head) * a.chunks * elements, a.chunks * elements);
 }
 
-// S entering every chunk and Dl of every chunk.  Wave w computes rows 16 w .. 16 w + 15
-// of Dl from the whole state and then its rows of the new state from all of Dl: two
-// dependent products of 32 matrix instructions a chunk.  The operands of the chunk
-// after next are requested as soon as this chunk's have been multiplied.
+// Both sequential kernels are chains of products with a barrier between them; requests
+// and stores stand between the multiplications, each request for a register right
+// after the multiplication that read it, and none between a product and the barrier
+// that publishes it.  The fences keep that order.
+__device__ inline void keep_order() { __builtin_amdgcn_sched_barrier(0); }
+
+// S entering every chunk, Dl and O of every chunk.  Wave w computes rows 16 w .. 16 w +
+// 15 of Dl and O from the whole state and then its rows of the new state from all of
+// Dl: 112 matrix instructions a wave, chunk and tile, the 48 of O off the chain.
+// Operands are requested a chunk ahead.
+template <int TILES>
 __global__ void __launch_bounds__(256)
 chunk_states_forward_kernel(ChunkedArgs a) {
-  __shared__ __attribute__((aligned(16))) float state[kSlice][kWidePad], delta[kSlice][kSquarePad];
-  const Slice slice = slice_of_block(a);
+  __shared__ __attribute__((aligned(16))) float state[TILES][kTile][kWidePad], delta[TILES][kTile][kSquarePad],
+      left_delta[TILES][kTile][kSquarePad];
+  const Slice slice = slice_of_block<TILES>(a);
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int quarter = lane / 16, n = lane % 16;
-  const int col = slice.col0 + n;
-  struct Operands {
-    float4 w[8];
-    float2 k[16];
-    float u[4];
-    float4 scale;
-    float decay;
-  };
-  auto view = [&](int chunk) { return ChunkView(a, min(chunk, a.chunks - 1), slice.head); };
-  // a lane's places in a record of rows of all channels: its row as the left operand,
-  // its rows as a result, its rows and channels as the transposed left operand
-  const unsigned row_at = (16 * wave + n) * kWideRow + 16 * quarter;
-  const unsigned result_at = (16 * wave + 4 * quarter) * kWideRow + 4 * col;
-  const unsigned state_at = (32 * wave + 8 * quarter) * kWideRow + 4 * col;
-  auto request_delta = [&](const ChunkView& v, Operands& o) {
-    const auto w = v.wide(a.r.w), u = v.wide(a.r.dl);
+  const int rows = 16 * wave + 4 * quarter;  // of the lane's part of Dl and O
+  float4 w[8], q[8], k[2][4], p[4], u[TILES], e_rows, l_rows;
+  float decay;
+  const int head = slice.head, key_head = head / (a.vh / a.kh);
+  const Record w_memory = head_records(a, a.r.w_rows, head, kWide), q_memory = head_records(a, a.r.q_rows, key_head, kWide),
+               k_memory = head_records(a, a.r.k_columns, key_head, kWide),
+               p_memory = head_records(a, a.r.p_rows, head, kSquare), dl_memory = head_records(a, a.r.dl, head, kWide),
+               s0_memory = head_records(a, a.r.s0, head, kState),
+               gates = head_records(a, a.r.gates, head, kGateRows * kC);
+  // the lane's places in the records of the chunk whose operands are requested next
+  const unsigned core_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
+  unsigned wide_at = 16 * lane, square_at = 16 * lane, gates_at = 4 * rows;
+  const unsigned delta_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
+  auto request_w = [&](int s) { w[s] = w_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
+  auto request_q = [&](int s) { q[s] = q_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
+  auto request_k = [&](int t, int s) { k[t][s] = k_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+  auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
+  auto request_rest = [&]() {
 #pragma unroll
-    for (int s = 0; s < 8; ++s) o.w[s] = w.get4(row_at, 64 * s);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o.u[e] = u.get(result_at, e * kWideRow);
-    o.scale = load4(v.gates + kLK * kC + 16 * wave + 4 * quarter);
+    for (int c = 0; c < TILES; ++c) u[c] = dl_memory.get4(wide_at, delta_at + piece_at<kC>(c, 0));
+    e_rows = gates.get4(gates_at, 4 * kE * kC);
+    l_rows = gates.get4(gates_at, 4 * kL * kC);
+    decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
   };
-  auto request_state = [&](const ChunkView& v, Operands& o) {
-    const auto k = v.k();
-    const unsigned at = 4 * quarter * v.row_bytes + 4 * (32 * wave + 2 * n);
+  const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+  floatx4 acc[2][TILES];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) o.k[j] = k.get2(at, (16 * (j / 4) + j % 4) * v.row_bytes);
-    o.decay = v.gates[kE * kC + kC - 1];
-  };
-  floatx4 acc[2];
-  acc[0] = acc[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  auto advance = [&](int chunk, Operands& o) {
-    const ChunkView v(a, chunk, slice.head), later = view(chunk + 2);
-    const auto dl_out = v.wide(a.r.dl);
-    publish_state(acc, &state[n][32 * wave + 8 * quarter]);
-    save_state(acc, v.state(a.r.s0), state_at);
+  for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
+  {
+    // in the loop's order, so that the waits in it need not cover another one
+#pragma unroll
+    for (int s = 0; s < 8; ++s) request_w(s), keep_order();
+    request_rest();
+    keep_order();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) request_q(s), keep_order();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) request_k(s % 2, s / 2), keep_order();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) request_p(s), keep_order();
+  }
+  for (int chunk = 0; chunk < a.chunks; ++chunk) {
+    const Tokens core = ChunkView(a, chunk, head).heads(a.core);
+    // past the end the last chunk's operands are requested again
+    const unsigned wide_now = wide_at, state_now = 16 * lane + chunk * (kState * 4);
+    if (chunk + 1 < a.chunks)
+      wide_at += kWide * 4, square_at += kSquare * 4, gates_at += kGateRows * kC * 4;
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) publish_state(acc[0][c], acc[1][c], &state[c][n][32 * wave + 4 * quarter]);
+    keep_order();
     lds_barrier();
-    floatx4 even = {0.0f, 0.0f, 0.0f, 0.0f}, odd = even;
-    float4 b[8];
+    floatx4 part[2][TILES], out[TILES];
+    float4 b[TILES][8];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) b[s] = load4(&state[n][16 * s + 4 * quarter]);
+    for (int s = 0; s < 8; ++s)
 #pragma unroll
-    for (int s = 0; s < 8; s += 2) {
-      even = mma16(even, o.w[s], b[s]);
-      odd = mma16(odd, o.w[s + 1], b[s + 1]);
+      for (int c = 0; c < TILES; ++c) b[c][s] = load4(&state[c][n][16 * s + 4 * quarter]);
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) part[0][c] = part[1][c] = out[c] = none;
+    keep_order();  // all of them before the first is waited for
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      mma16_tiles<TILES>(part[s % 2], w[s], [&](int c) { return b[c][s]; });
+      keep_order();
+      request_w(s);
+      keep_order();
     }
-    float dl[4];
+    float4 dl[TILES];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      dl[e] = o.u[e] - (even[e] + odd[e]);
-      dl_out.put(dl[e], result_at, e * kWideRow);
+    for (int c = 0; c < TILES; ++c) {
+      const floatx4 ws = part[0][c] + part[1][c];
+      dl[c] = make_float4(u[c].x - ws[0], u[c].y - ws[1], u[c].z - ws[2], u[c].w - ws[3]);
+      store4(&delta[c][n][rows], dl[c]);
+      store4(&left_delta[c][n][rows],
+             make_float4(dl[c].x * l_rows.x, dl[c].y * l_rows.y, dl[c].z * l_rows.z, dl[c].w * l_rows.w));
+      acc[0][c] *= decay;
+      acc[1][c] *= decay;
     }
-    store4(&delta[n][16 * wave + 4 * quarter],
-           make_float4(dl[0] * o.scale.x, dl[1] * o.scale.y, dl[2] * o.scale.z, dl[3] * o.scale.w));
-    __builtin_amdgcn_sched_barrier(0);
-    request_delta(later, o);
-    __builtin_amdgcn_sched_barrier(0);
+    const float4 e_now = e_rows;
+    keep_order();
+    request_rest();
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) dl_memory.put4(dl[c], wide_now, delta_at + piece_at<kC>(c, 0));
+    keep_order();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      mma16_tiles<TILES>(out, q[s], [&](int c) { return b[c][s]; });
+      keep_order();
+      request_q(s);
+      if (s % 4 == 3) {
+        const int t = s / 4;  // rows(S): 16 rows a store, four columns a lane
+#pragma unroll
+        for (int c = 0; c < TILES; ++c)
+          s0_memory.put4(gather4(&state[c][4 * quarter][32 * wave + 16 * t + n], kWidePad), state_now,
+                      piece_at<kD>(2 * wave + t, (slice.col0 + kTile * c) / 4));
+      }
+      keep_order();
+    }
     lds_barrier();
 #pragma unroll
-    for (int s = 0; s < 4; ++s) b[s] = load4(&delta[n][16 * s + 4 * quarter]);
-    acc[0] *= o.decay;
-    acc[1] *= o.decay;
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) {
+        b[c][s] = load4(&left_delta[c][n][16 * s + 4 * quarter]);
+        b[c][4 + s] = load4(&delta[c][n][16 * s + 4 * quarter]);
+      }
+    keep_order();
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      acc[0] = mma16(acc[0], make_float4(o.k[4 * s].x, o.k[4 * s + 1].x, o.k[4 * s + 2].x, o.k[4 * s + 3].x), b[s]);
-      acc[1] = mma16(acc[1], make_float4(o.k[4 * s].y, o.k[4 * s + 1].y, o.k[4 * s + 2].y, o.k[4 * s + 3].y), b[s]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        mma16_tiles<TILES>(acc[t], k[t][s], [&](int c) { return b[c][s]; });
+        keep_order();
+        request_k(t, s);
+        keep_order();
+      }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    request_state(later, o);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  Operands even, odd;
-  request_delta(view(0), even);
-  request_state(view(0), even);
-  request_delta(view(1), odd);
-  request_state(view(1), odd);
-  for (int chunk = 0; chunk < a.chunks; chunk += 2) {
-    advance(chunk, even);
-    if (chunk + 1 < a.chunks) advance(chunk + 1, odd);
+#pragma unroll
+    for (int c = 0; c < TILES; ++c)
+      out[c][0] *= e_now.x, out[c][1] *= e_now.y, out[c][2] *= e_now.z, out[c][3] *= e_now.w;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      mma16_tiles<TILES>(out, p[s], [&](int c) { return b[c][4 + s]; });
+      keep_order();
+      request_p(s);
+      keep_order();
+    }
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) {
+      // four tokens of a column -> four columns of a token
+      const float4 o =
+          quad_transpose(make_float4(round_if(out[c][0], a.round), round_if(out[c][1], a.round),
+                                     round_if(out[c][2], a.round), round_if(out[c][3], a.round)));
+      core.put4(o, core_at, 4 * kTile * c);
+    }
   }
 }
 
 // The gradient of the state leaving every chunk and dDl of every chunk, chunks in
-// reverse.  112 matrix instructions a wave and chunk; the products with dO do not
-// depend on the chain and run while it waits.
+// reverse.  112 matrix instructions a wave, chunk and tile, those with dO off the chain
+// (Q^ dO fills the wait for the other waves' dDl).
+template <int TILES>
 __global__ void __launch_bounds__(256)
 chunk_states_backward_kernel(ChunkedArgs a) {
-  __shared__ __attribute__((aligned(16))) float state[kSlice][kWidePad], delta[kSlice][kSquarePad],
-      grad[kSlice][kSquarePad], query_grad[kSlice][kSquarePad];
-  const Slice slice = slice_of_block(a);
+  __shared__ __attribute__((aligned(16))) float state[TILES][kTile][kWidePad], delta[TILES][kTile][kSquarePad],
+      grad[TILES][kTile][kSquarePad], query_grad[TILES][kTile][kSquarePad];
+  const Slice slice = slice_of_block<TILES>(a);
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int quarter = lane / 16, n = lane % 16;
-  const int col = slice.col0 + n;
-  auto view = [&](int chunk) { return ChunkView(a, max(chunk, 0), slice.head); };
-  float4 k[8];
-  float p[16], out[4];
-  float2 q[16], w[16];
-  float4 k_scale, q_scale;
-  float decay;
   const int rows = 16 * wave + 4 * quarter;
-  const unsigned result_at = rows * kWideRow + 4 * col;
-  const unsigned state_at = (32 * wave + 8 * quarter) * kWideRow + 4 * col;
-  auto request_out = [&](const ChunkView& v) {
-    const auto d_out = v.heads(a.dcore);
+  float4 k[8], p[4], q[2][4], w[2][4], out[TILES], k_scale, q_scale;
+  float decay;
+  const int head = slice.head, key_head = head / (a.vh / a.kh);
+  const Record k_memory = head_records(a, a.r.k_rows, key_head, kWide),
+               p_memory = head_records(a, a.r.p_columns, head, kSquare),
+               q_memory = head_records(a, a.r.q_columns, key_head, kWide),
+               w_memory = head_records(a, a.r.w_columns, head, kWide),
+               ddl_memory = head_records(a, a.r.ddl, head, kWide), ds1_memory = head_records(a, a.r.ds1, head, kState),
+               gates = head_records(a, a.r.gates, head, kGateRows * kC);
+  const unsigned last = a.chunks - 1;
+  unsigned wide_at = 16 * lane + last * (kWide * 4), square_at = 16 * lane + last * (kSquare * 4),
+           gates_at = 4 * rows + last * (kGateRows * kC * 4);
+  const unsigned delta_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
+  const unsigned out_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
+  auto request_out = [&](int chunk) {
+    const Tokens d_out = ChunkView(a, max(chunk, 0), head).heads(a.dcore);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = d_out.get(rows * v.out_bytes + 4 * col, e * v.out_bytes);
-    q_scale = load4(v.gates + kEQ * kC + rows);
+    for (int c = 0; c < TILES; ++c) out[c] = d_out.get4(out_at, 4 * kTile * c);
+    q_scale = gates.get4(gates_at, 4 * kE * kC);
+    k_scale = gates.get4(gates_at, 4 * kL * kC);
+    decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
   };
-  auto request_delta = [&](const ChunkView& v) {
-    const Record p_memory = v.square(a.r.p);
-    const Tokens k_memory = v.k();
+  auto request_k = [&](int s) { k[s] = k_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
+  auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
+  auto request_q = [&](int t, int s) { q[t][s] = q_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+  auto request_w = [&](int t, int s) { w[t][s] = w_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+  const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+  floatx4 acc[2][TILES];
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-      p[j] = p_memory.get(4 * quarter * kSquareRow + 4 * (16 * wave + n), (16 * (j / 4) + j % 4) * kSquareRow);
-#pragma unroll
-    for (int s = 0; s < 8; ++s) k[s] = k_memory.get4((16 * wave + n) * v.row_bytes + 16 * quarter, 64 * s);
-    k_scale = load4(v.gates + kLK * kC + rows);
-  };
-  auto request_query = [&](const ChunkView& v) {
-    const auto q_memory = v.q();
-    const unsigned at = 4 * quarter * v.row_bytes + 4 * (32 * wave + 2 * n);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) q[j] = q_memory.get2(at, (16 * (j / 4) + j % 4) * v.row_bytes);
-    decay = v.gates[kE * kC + kC - 1];
-  };
-  auto request_weights = [&](const ChunkView& v) {
-    const auto w_memory = v.wide(a.r.w);
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-      w[j] = w_memory.get2(4 * quarter * kWideRow + 4 * (32 * wave + 2 * n), (16 * (j / 4) + j % 4) * kWideRow);
-  };
-  floatx4 acc[2];
-  acc[0] = acc[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
   {
-    const ChunkView v = view(a.chunks - 1);
-    request_out(v);
-    request_delta(v);
-    request_query(v);
-    request_weights(v);
+    // in the loop's order, so that the waits in it need not cover another one
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      request_k(2 * s), keep_order();
+      request_k(2 * s + 1), keep_order();
+      request_p(s), keep_order();
+    }
+    request_out(last);
+    keep_order();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) request_q(s % 2, s / 2), keep_order();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) request_w(s % 2, s / 2), keep_order();
   }
   for (int chunk = a.chunks - 1; chunk >= 0; --chunk) {
-    const ChunkView v(a, chunk, slice.head), later = view(chunk - 1);
-    const auto ddl_out = v.wide(a.r.ddl);
-    publish_state(acc, &state[n][32 * wave + 8 * quarter]);
-    store4(&grad[n][rows], make_float4(out[0], out[1], out[2], out[3]));
-    store4(&query_grad[n][rows],
-           make_float4(out[0] * q_scale.x, out[1] * q_scale.y, out[2] * q_scale.z, out[3] * q_scale.w));
-    save_state(acc, v.state(a.r.ds1), state_at);
-    __builtin_amdgcn_sched_barrier(0);
-    request_out(later);
-    __builtin_amdgcn_sched_barrier(0);
+    // before the first the first chunk's operands are requested again
+    const unsigned wide_now = wide_at, state_now = 16 * lane + chunk * (kState * 4);
+    if (chunk > 0) wide_at -= kWide * 4, square_at -= kSquare * 4, gates_at -= kGateRows * kC * 4;
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) {
+      publish_state(acc[0][c], acc[1][c], &state[c][n][32 * wave + 4 * quarter]);
+      const float4 o = quad_transpose(out[c]);  // four columns of a token -> four tokens of a column
+      store4(&grad[c][n][rows], o);
+      store4(&query_grad[c][n][rows],
+             make_float4(o.x * q_scale.x, o.y * q_scale.y, o.z * q_scale.z, o.w * q_scale.w));
+    }
+    const float4 scale = k_scale;
+    const float decay_now = decay;
+    keep_order();
     lds_barrier();
-    floatx4 from_out = {0.0f, 0.0f, 0.0f, 0.0f}, even = from_out, odd = from_out;
-    float4 b[8];
+    floatx4 from_out[TILES], part[2][TILES];
+    float4 b[TILES][8], g[TILES][4];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) b[s] = load4(&state[n][16 * s + 4 * quarter]);
-    float4 g[4];
+    for (int s = 0; s < 8; ++s)
 #pragma unroll
-    for (int s = 0; s < 4; ++s) g[s] = load4(&grad[n][16 * s + 4 * quarter]);
+      for (int c = 0; c < TILES; ++c) b[c][s] = load4(&state[c][n][16 * s + 4 * quarter]);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      even = mma16(even, k[2 * s], b[2 * s]);
-      odd = mma16(odd, k[2 * s + 1], b[2 * s + 1]);
-      from_out = mma16(from_out, make_float4(p[4 * s], p[4 * s + 1], p[4 * s + 2], p[4 * s + 3]), g[s]);
-    }
-    float dd[4];
-    const float scale[4] = {k_scale.x, k_scale.y, k_scale.z, k_scale.w};
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      dd[e] = from_out[e] + scale[e] * (even[e] + odd[e]);
-      ddl_out.put(dd[e], result_at, e * kWideRow);
-    }
-    store4(&delta[n][rows], make_float4(-dd[0], -dd[1], -dd[2], -dd[3]));
-    __builtin_amdgcn_sched_barrier(0);
-    request_delta(later);
-    __builtin_amdgcn_sched_barrier(0);
-    acc[0] *= decay;
-    acc[1] *= decay;
+      for (int c = 0; c < TILES; ++c) g[c][s] = load4(&grad[c][n][16 * s + 4 * quarter]);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) g[s] = load4(&query_grad[n][16 * s + 4 * quarter]);
+    for (int c = 0; c < TILES; ++c) part[0][c] = part[1][c] = from_out[c] = none;
+    keep_order();
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      acc[0] = mma16(acc[0], make_float4(q[4 * s].x, q[4 * s + 1].x, q[4 * s + 2].x, q[4 * s + 3].x), g[s]);
-      acc[1] = mma16(acc[1], make_float4(q[4 * s].y, q[4 * s + 1].y, q[4 * s + 2].y, q[4 * s + 3].y), g[s]);
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        mma16_tiles<TILES>(part[half], k[2 * s + half], [&](int c) { return b[c][2 * s + half]; });
+        keep_order();
+        request_k(2 * s + half);
+        keep_order();
+      }
+      mma16_tiles<TILES>(from_out, p[s], [&](int c) { return g[c][s]; });
+      keep_order();
+      request_p(s);
+      keep_order();
     }
-    __builtin_amdgcn_sched_barrier(0);
-    request_query(later);
-    __builtin_amdgcn_sched_barrier(0);
+    float4 dd[TILES];
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) {
+      const floatx4 ks = part[0][c] + part[1][c];
+      dd[c] = make_float4(from_out[c][0] + scale.x * ks[0], from_out[c][1] + scale.y * ks[1],
+                          from_out[c][2] + scale.z * ks[2], from_out[c][3] + scale.w * ks[3]);
+      store4(&delta[c][n][rows], scaled(dd[c], -1.0f));
+      acc[0][c] *= decay_now;
+      acc[1][c] *= decay_now;
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) g[c][s] = load4(&query_grad[c][n][16 * s + 4 * quarter]);
+    keep_order();
+    request_out(chunk - 1);
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) ddl_memory.put4(dd[c], wide_now, delta_at + piece_at<kC>(c, 0));
+    keep_order();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        mma16_tiles<TILES>(acc[t], q[t][s], [&](int c) { return g[c][s]; });
+        keep_order();
+        request_q(t, s);
+        if (s % 2 == 1 && t == 1) {
+#pragma unroll
+          for (int c = 0; c < TILES; ++c)
+            ds1_memory.put4(gather4(&state[c][4 * quarter][32 * wave + 16 * (s / 2) + n], kWidePad), state_now,
+                         piece_at<kD>(2 * wave + s / 2, (slice.col0 + kTile * c) / 4));
+        }
+        keep_order();
+      }
+    }
     lds_barrier();
 #pragma unroll
-    for (int s = 0; s < 4; ++s) g[s] = load4(&delta[n][16 * s + 4 * quarter]);
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) g[c][s] = load4(&delta[c][n][16 * s + 4 * quarter]);
+    keep_order();
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      acc[0] = mma16(acc[0], make_float4(w[4 * s].x, w[4 * s + 1].x, w[4 * s + 2].x, w[4 * s + 3].x), g[s]);
-      acc[1] = mma16(acc[1], make_float4(w[4 * s].y, w[4 * s + 1].y, w[4 * s + 2].y, w[4 * s + 3].y), g[s]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        mma16_tiles<TILES>(acc[t], w[t][s], [&](int c) { return g[c][s]; });
+        keep_order();
+        request_w(t, s);
+        keep_order();
+      }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    request_weights(later);
-    __builtin_amdgcn_sched_barrier(0);
   }
-}
-
-// ---------------------------------------------------------------------------
-// O = diag(E) Q^ S + P Dl of one chunk.  Wave w owns value columns 32w..32w+31 and has
-// its part of S and Dl in registers, requested before the rows of Q^ and P are staged
-// for all waves.
-__global__ void __launch_bounds__(256)
-chunk_outputs_kernel(ChunkedArgs a) {
-  __shared__ __attribute__((aligned(16))) float q_s[kC][kWidePad], p_s[kC][kSquarePad];
-  const ChunkView v(a, blockIdx.x, blockIdx.y);
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int h = lane / 32, n = lane % 32;
-  const int col = 32 * wave + n;
-  const Tokens q = v.q(), core = v.heads(a.core);
-  const Record p = v.square(a.r.p), state = v.state(a.r.s0), delta = v.wide(a.r.dl);
-  float4 rows[8], p_rows[4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    rows[i] = scaled(q.get4(tid / 32 * v.row_bytes + tid % 32 * 16, 8 * i * v.row_bytes),
-                     v.gates[kEQ * kC + tid / 32 + 8 * i]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) p_rows[i] = p.get4(16 * tid, 4096 * i);
-  const unsigned column_at = 4 * h * kWideRow + 4 * col;
-  float4 s_col[16], d_col[8];
-#pragma unroll
-  for (int s = 0; s < 16; ++s) s_col[s] = state.gather4(column_at, 8 * s * kWideRow, kWideRow);
-#pragma unroll
-  for (int s = 0; s < 8; ++s) d_col[s] = delta.gather4(column_at, 8 * s * kWideRow, kWideRow);
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int at = tid + 256 * i;
-    store4(&q_s[at / 32][at % 32 * 4], rows[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int at = tid + 256 * i;
-    store4(&p_s[at / 16][at % 16 * 4], p_rows[i]);
-  }
-  lds_barrier();
-  floatx16 out[2];
-  out[0] = out[1] = zero_tile();
-#pragma unroll
-  for (int s = 0; s < 16; ++s)
-#pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
-      out[ti] = mma(out[ti], load4(&q_s[32 * ti + n][8 * s + 4 * h]), s_col[s]);
-#pragma unroll
-  for (int s = 0; s < 8; ++s)
-#pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
-      if (s < 4 * (ti + 1)) out[ti] = mma(out[ti], load4(&p_s[32 * ti + n][8 * s + 4 * h]), d_col[s]);
-#pragma unroll
-  for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      core.put(round_if(out[ti][i], a.round), 4 * h * v.out_bytes + 4 * col,
-               (32 * ti + tile_row(i, 0)) * v.out_bytes);
 }
 
 // ---------------------------------------------------------------------------
@@ -797,24 +955,26 @@ chunk_gradients_kernel(ChunkedArgs a) {
     const Record s0_memory = v.state(a.r.s0), s1_memory = v.state(a.r.ds1), ddl = v.wide(a.r.ddl),
                  dl = v.wide(a.r.dl);
     const Tokens d_out = v.heads(a.dcore), values = v.v();
-    const unsigned state_at = col * kWideRow + 16 * h;
-    // thread (row, piece) of the slabs: rows r and r + 32, 16 bytes
+    const unsigned state_at = piece_at<kD>(2 * wave, 0) + lane_piece<kD>(h, n);
+    // thread (row, piece) of the slabs of dO and V: rows r and r + 32, 16 bytes; of dDl and
+    // Dl, which lie as columns: four tokens of one column in each half of the slab
     const int row = tid / 8, piece = tid % 8 * 4;
+    const int row4 = tid / 16 * 4, column = tid % 16;
     float4 staged[8];
     auto request = [&](int slab) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const unsigned c = 4 * kSlab * slab;
-        staged[4 * j] = ddl.get4(row * kWideRow + 4 * piece, 32 * j * kWideRow + c);
+        staged[4 * j] = ddl.get4(16 * tid, piece_at<kC>(2 * slab + j, 0));
         staged[4 * j + 1] = d_out.get4(row * v.out_bytes + 4 * piece, 32 * j * v.out_bytes + c);
-        staged[4 * j + 2] = dl.get4(row * kWideRow + 4 * piece, 32 * j * kWideRow + c);
+        staged[4 * j + 2] = dl.get4(16 * tid, piece_at<kC>(2 * slab + j, 0));
         staged[4 * j + 3] = values.get4(row * v.row_bytes + 4 * piece, 32 * j * v.row_bytes + c);
       }
     };
     request(0);
     float4 s0[4], s1[4];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) s0[g] = s0_memory.get4(state_at, 32 * g), s1[g] = s1_memory.get4(state_at, 32 * g);
+    for (int g = 0; g < 4; ++g) s0[g] = s0_memory.get4(state_at, piece_at<kD>(0, 2 * g)), s1[g] = s1_memory.get4(state_at, piece_at<kD>(0, 2 * g));
     float fv = 0.0f;
 #pragma unroll
     for (int slab = 0; slab < kD / kSlab; ++slab) {
@@ -822,8 +982,17 @@ chunk_gradients_kernel(ChunkedArgs a) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
-          store4(&sm.slab[m][row + 32 * j][piece], staged[4 * j + m]);
+        for (int m = 0; m < 4; ++m) {
+          const float4 four = staged[4 * j + m];
+          if (m % 2 == 1) {
+            store4(&sm.slab[m][row + 32 * j][piece], four);
+          } else {
+            sm.slab[m][row4][16 * j + column] = four.x;
+            sm.slab[m][row4 + 1][16 * j + column] = four.y;
+            sm.slab[m][row4 + 2][16 * j + column] = four.z;
+            sm.slab[m][row4 + 3][16 * j + column] = four.w;
+          }
+        }
       if (slab == 0)
         __syncthreads();
       else
@@ -842,8 +1011,8 @@ chunk_gradients_kernel(ChunkedArgs a) {
           dk[ti] = mma(dk[ti], load4(&sm.slab[2][32 * ti + n][c]), s1[g]);
         }
         if (slab + 1 < kD / kSlab) {
-          s0[g] = s0_memory.get4(state_at, 4 * kSlab * (slab + 1) + 32 * g);
-          s1[g] = s1_memory.get4(state_at, 4 * kSlab * (slab + 1) + 32 * g);
+          s0[g] = s0_memory.get4(state_at, piece_at<kD>(0, kSlab / 4 * (slab + 1) + 2 * g));
+          s1[g] = s1_memory.get4(state_at, piece_at<kD>(0, kSlab / 4 * (slab + 1) + 2 * g));
         }
         if (lower) {
           dp = mma(dp, load4(&sm.slab[1][32 * ti_own + n][c]), load4(&sm.slab[2][32 * tj_own + n][c]));
@@ -873,32 +1042,42 @@ chunk_gradients_kernel(ChunkedArgs a) {
     const float row_sum = half_sums(values);
     if (n % 2 == 0) row_sums[32 * ti_own + tile_row(n / 2, h)][tj_own] = row_sum;
   };
-  const Record p_memory = v.square(a.r.p), kkd = v.square(a.r.kkd), tm = v.square(a.r.tm),
-               ddl = v.wide(a.r.ddl);
-  const Tokens q_memory = v.q(), k_memory = v.k(), v_memory = v.v(), dv = v.dv();
-  // the accumulator's places in a [64, 64] tile and in a column of the [64, 128] matrices
-  const unsigned tile_at = (32 * ti_own + 4 * h) * kSquareRow + 4 * tile_col;
-  const unsigned column_at = 4 * h * kWideRow + 4 * col, token_at = 4 * h * v.row_bytes + 4 * col;
+  const Record p_memory = v.square(a.r.p_columns), kkd = v.square(a.r.kkd), t_rows = v.square(a.r.t_rows),
+               t_columns = v.square(a.r.t_columns), ddl = v.wide(a.r.ddl), q_memory = v.key(a.r.q_columns),
+               k_memory = v.key(a.r.k_columns), k_rows = v.key(a.r.k_rows);
+  const Tokens v_memory = v.v(), dv = v.dv();
+  // the lane's places in columns(M) of [64, 64] and [64, 128] matrices (four rows of one
+  // column, as in an accumulator), and a token's in the activations
+  const unsigned square_at = lane_piece<kC>(h, n), tile_at = square_at + piece_at<kC>(2 * tj_own, 8 * ti_own);
+  const unsigned column_at = square_at + piece_at<kC>(2 * wave, 0), token_at = 4 * h * v.row_bytes + 4 * col;
+  auto tile_of = [&](const Record& m, float (&values)[16]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 four = m.get4(tile_at, piece_at<kC>(0, 2 * j));
+      values[4 * j] = four.x, values[4 * j + 1] = four.y, values[4 * j + 2] = four.z, values[4 * j + 3] = four.w;
+    }
+  };
   float decay[16];  // D of the tile
   if (lower) {
     float products[16];
+    tile_of(p_memory, products);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = 32 * ti_own + tile_row(i, h);
       const bool in = row >= tile_col;
       decay[i] = in ? expf(sm.gate[kG][row] - sm.gate[kG][tile_col]) : 0.0f;
       sm.pd[row][tile_col] = in ? dp[i] * decay[i] : 0.0f;
-      products[i] = in ? dp[i] * p_memory.get(tile_at, tile_row(i, 0) * kSquareRow) : 0.0f;
+      products[i] = in ? dp[i] * products[i] : 0.0f;
     }
     tile_sums(products, sm.row_p, sm.col_p, nullptr);
   }
   lds_barrier();
   if (lower) {
-    const float fk = sm.gate[kBeta][tile_col] * sm.gate[kE][tile_col] * sm.gate[kKScale][tile_col];
-    const unsigned k_at = tile_col * v.row_bytes + 16 * h;
+    const float fk = sm.gate[kBeta][tile_col] * sm.gate[kE][tile_col];
+    const unsigned k_at = piece_at<kD>(2 * tj_own, 0) + lane_piece<kD>(h, n);
 #pragma unroll
     for (int s = 0; s < kD / 8; ++s)
-      dt = mma(dt, load4(&sm.dw[32 * ti_own + n][8 * s + 4 * h]), scaled(k_memory.get4(k_at, 32 * s), fk));
+      dt = mma(dt, load4(&sm.dw[32 * ti_own + n][8 * s + 4 * h]), scaled(k_rows.get4(k_at, piece_at<kD>(0, 2 * s)), fk));
 #pragma unroll
     for (int i = 0; i < 16; ++i) sm.x[32 * ti_own + tile_row(i, h)][tile_col] = dt[i];
   }
@@ -909,7 +1088,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
 #pragma unroll
     for (int s = 0; s < 8; ++s)
       if (s >= 4 * ti_own)
-        z = mma(z, tm.gather4(4 * h * kSquareRow + 4 * (32 * ti_own + n), 8 * s * kSquareRow, kSquareRow),
+        z = mma(z, t_columns.get4(square_at, piece_at<kC>(2 * ti_own, 2 * s)),
                 gather4(&sm.x[8 * s + 4 * h][tile_col], kSquarePad));
   }
   lds_barrier();
@@ -924,18 +1103,19 @@ chunk_gradients_kernel(ChunkedArgs a) {
     for (int s = 0; s < 8; ++s)
       if (s < 4 * (tj_own + 1))
         da = mma(da, load4(&sm.x[32 * ti_own + n][8 * s + 4 * h]),
-                 tm.get4(tile_col * kSquareRow + 16 * h, 32 * s));
+                 t_rows.get4(square_at, piece_at<kC>(2 * tj_own, 2 * s)));
   }
   lds_barrier();
   if (lower) {
     // R + R^T, and the sums of N = dA (k^ . k^) D
     float products[16];
+    tile_of(kkd, products);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = 32 * ti_own + tile_row(i, h);
       const bool in = row > tile_col;
       const float value = in ? -da[i] : 0.0f;
-      products[i] = value * kkd.get(tile_at, tile_row(i, 0) * kSquareRow);
+      products[i] = value * products[i];
       const float r = value * sm.gate[kBeta][row] * decay[i];
       if (row >= tile_col) sm.x[row][tile_col] = sm.x[tile_col][row] = r;
     }
@@ -945,12 +1125,8 @@ chunk_gradients_kernel(ChunkedArgs a) {
   float4 kc[8], qc[8];
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
-    const int i = 8 * s + 4 * h;
-    const float4 ks = load4(&sm.gate[kKScale][i]), qs = load4(&sm.gate[kQScale][i]);
-    const float4 k = k_memory.gather4(token_at, 8 * s * v.row_bytes, v.row_bytes);
-    const float4 q = q_memory.gather4(token_at, 8 * s * v.row_bytes, v.row_bytes);
-    kc[s] = make_float4(k.x * ks.x, k.y * ks.y, k.z * ks.z, k.w * ks.w);
-    qc[s] = make_float4(q.x * qs.x, q.y * qs.y, q.z * qs.z, q.w * qs.w);
+    kc[s] = k_memory.get4(column_at, piece_at<kC>(0, 2 * s));
+    qc[s] = q_memory.get4(column_at, piece_at<kC>(0, 2 * s));
   }
   auto element = [](const float4 (&c)[8], int ti, int i) {
     const float4 four = c[4 * ti + i / 4];
@@ -981,7 +1157,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
     const int m = 32 * ti + n;
     float4 t_col[8];
 #pragma unroll
-    for (int s = 4 * ti; s < 8; ++s) t_col[s] = tm.gather4(4 * h * kSquareRow + 4 * m, 8 * s * kSquareRow, kSquareRow);
+    for (int s = 4 * ti; s < 8; ++s) t_col[s] = t_columns.get4(square_at, piece_at<kC>(2 * ti, 2 * s));
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -1010,7 +1186,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
       floatx16 tu = zero_tile();
 #pragma unroll
       for (int s = 4 * ti; s < 8; ++s)
-        tu = mma(tu, t_col[s], ddl.gather4(column_at, 8 * s * kWideRow, kWideRow));
+        tu = mma(tu, t_col[s], ddl.get4(column_at, piece_at<kC>(0, 2 * s)));
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const unsigned row = (32 * ti + tile_row(i, 0)) * v.row_bytes;
@@ -1101,17 +1277,30 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
     at += n * floats;
     return result;
   };
-  a.r.w = take(kWide);
+  a.r.w_rows = take(kWide);
+  a.r.w_columns = take(kWide);
   a.r.dl = take(kWide);
   a.r.ddl = take(kWide);
-  a.r.p = take(kSquare);
-  a.r.tm = take(kSquare);
+  a.r.p_rows = take(kSquare);
+  a.r.p_columns = take(kSquare);
+  a.r.t_rows = take(kSquare);
+  a.r.t_columns = take(kSquare);
   a.r.kkd = take(kSquare);
   a.r.gates = take(kGateRows * kC);
   a.r.s0 = take(kState);
   a.r.ds1 = take(kState);
+  const size_t keys = static_cast<size_t>(a.chunks) * a.kh * kWide;
+  a.r.q_rows = at;
+  a.r.q_columns = at + keys;
+  a.r.k_rows = at + 2 * keys;
+  a.r.k_columns = at + 3 * keys;
   return a;
 }
+
+// Tiles of sixteen columns a workgroup of the sequential kernels takes.  While every
+// tile gets a compute unit of its own one is faster; beyond that compute units hold
+// two tiles anyway, and one workgroup with both loads the operands once.
+int column_tiles(int value_heads) { return value_heads * (kD / kTile) > 256 ? 2 : 1; }
 
 }  // namespace
 
@@ -1122,25 +1311,29 @@ bool gdn_backward_chunked_supported(const pluto_hip_delta_params* p) {
 
 size_t gdn_backward_chunked_bytes(const pluto_hip_delta_params* p, int length) {
   const size_t chunks = (static_cast<size_t>(length) + kC - 1) / kC;
-  return align_up(chunks * p->value_heads * kRecordFloats * sizeof(float), 256);
+  return align_up(chunks * (p->value_heads * kRecordFloats + p->key_heads * kKeyRecordFloats) * sizeof(float),
+                  256);
 }
 
 int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBackward& c) {
   const ChunkedArgs a = make_args(c);
   const dim3 per_chunk(a.chunks, a.vh);
   chunk_prepare_kernel<<<per_chunk, 256, 0, stream>>>(a);
-  int status = launch_status();
+  const int status = launch_status();
   if (status != 0) return status;
-  chunk_states_forward_kernel<<<a.vh * (kD / kSlice), 256, 0, stream>>>(a);
-  status = launch_status();
-  if (status != 0) return status;
-  chunk_outputs_kernel<<<per_chunk, 256, 0, stream>>>(a);
+  if (column_tiles(a.vh) == 2)
+    chunk_states_forward_kernel<2><<<a.vh * (kD / (2 * kTile)), 256, 0, stream>>>(a);
+  else
+    chunk_states_forward_kernel<1><<<a.vh * (kD / kTile), 256, 0, stream>>>(a);
   return launch_status();
 }
 
 int launch_gdn_backward_chunked_reverse(hipStream_t stream, const GdnChunkedBackward& c) {
   const ChunkedArgs a = make_args(c);
-  chunk_states_backward_kernel<<<a.vh * (kD / kSlice), 256, 0, stream>>>(a);
+  if (column_tiles(a.vh) == 2)
+    chunk_states_backward_kernel<2><<<a.vh * (kD / (2 * kTile)), 256, 0, stream>>>(a);
+  else
+    chunk_states_backward_kernel<1><<<a.vh * (kD / kTile), 256, 0, stream>>>(a);
   const int status = launch_status();
   if (status != 0) return status;
   chunk_gradients_kernel<<<dim3(a.chunks, a.vh), 256, 0, stream>>>(a);
