@@ -49,6 +49,10 @@
 // formulas above, with M and B, took 1766 us.
 #include "gdn.h"
 
+#include "mfma_tile.h"
+
+#include <type_traits>
+
 namespace pluto_hip {
 namespace {
 
@@ -66,7 +70,7 @@ struct Records {
   // of a key head                                                        [64][128]
   float *q_rows, *q_columns, *k_rows, *k_columns;
   float *w_rows, *w_columns;                          // W              [64][128]
-  float *dl, *ddl;            // columns(U), which columns(Dl) replaces; columns(dDl)
+  float *u_columns, *dl_rows, *ddl_rows, *ddl_columns;  // U, Dl, dDl    [64][128]
   float *p_rows, *p_columns;                          // P               [64][64]
   float *t_rows, *t_columns;                          // T               [64][64]
   float *kkd;                 // columns(strict_lower((k^_i . k^_j) D_ij)) [64][64]
@@ -79,7 +83,7 @@ struct Records {
 enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kGateRows };
 
 constexpr size_t kKeyRecordFloats = 4 * static_cast<size_t>(kWide);
-constexpr size_t kRecordFloats = 4 * static_cast<size_t>(kWide) + 5 * kSquare + kGateRows * kC +
+constexpr size_t kRecordFloats = 6 * static_cast<size_t>(kWide) + 5 * kSquare + kGateRows * kC +
                                  2 * static_cast<size_t>(kState);
 
 struct ChunkedArgs {
@@ -189,23 +193,29 @@ __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// Sums over the 32 lanes of a half wave of sixteen values at once: lanes 2 j and 2 j + 1
-// of a half return the sum of value j.  Each exchange halves the values a lane holds.
+// Sums over the 32 lanes of a half wave of sixteen values at once: lanes i and 16 + i of a
+// half return the sum of value i.  Every step halves the values a lane holds; its
+// partners mirror rows of 16, 8, 4 and 2 lanes, which is part of a vector addition.
 __device__ inline float half_sums(const float (&values)[16]) {
   float v[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) v[i] = values[i];
-  const int n = threadIdx.x % 32;
+  const int n = threadIdx.x;
+  auto step = [&](auto control, int width) {
+    const bool upper = n & width;
 #pragma unroll
-  for (int width = 8; width > 0; width /= 2) {
-    const bool upper = n & (2 * width);
-#pragma unroll
-    for (int i = 0; i < width; ++i) {
+    for (int i = 0; i < 8; ++i) {
+      if (i >= width) break;
       const float kept = upper ? v[i + width] : v[i], sent = upper ? v[i] : v[i + width];
-      v[i] = kept + __shfl_xor(sent, 2 * width, 64);
+      v[i] = kept + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sent), decltype(control)::value,
+                                                               0xf, 0xf, true));
     }
-  }
-  return v[0] + __shfl_xor(v[0], 1, 64);
+  };
+  step(std::integral_constant<int, 0x140>(), 8);  // row_mirror
+  step(std::integral_constant<int, 0x141>(), 4);  // row_half_mirror
+  step(std::integral_constant<int, 0x4E>(), 2);   // quad_perm 2, 3, 0, 1
+  step(std::integral_constant<int, 0xB1>(), 1);   // quad_perm 1, 0, 3, 2
+  return v[0] + __shfl_xor(v[0], 16, 64);
 }
 
 // Memory behind a buffer descriptor: a lane's byte offset, computed once, and a uniform
@@ -214,10 +224,14 @@ __device__ inline float half_sums(const float (&values)[16]) {
 // reads give zero and writes are dropped, without a branch.
 template <bool TOKENS>
 struct Memory {
+  const float* base;
+  uint32_t bytes;
   __amdgpu_buffer_rsrc_t rsrc;
-  __device__ Memory(const float* base, size_t elements)
-      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0,
-                                               static_cast<int>(elements * 4), 0x00020000)) {}
+  __device__ Memory(const float* base_, size_t elements)
+      : base(base_), bytes(static_cast<uint32_t>(elements * 4)),
+        rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, static_cast<int>(bytes),
+                                               0x00020000)) {}
+  __device__ int32x4 words() const { return make_rsrc(base, bytes); }
   __device__ float get(unsigned lane, unsigned uniform) const {
     const auto bits = TOKENS ? __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane + uniform, 0, 0)
                              : __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane, uniform, 0);
@@ -344,14 +358,14 @@ chunk_prepare_kernel(ChunkedArgs a) {
     for (int r = 0; r < 16; ++r)
       squares[r] = (rows[r].x * rows[r].x + rows[r].y * rows[r].y) +
                    (rows[r].z * rows[r].z + rows[r].w * rows[r].w);
-    const float sum = half_sums(squares);  // lane 2 j holds that of rows[j]
+    const float sum = half_sums(squares);  // lane j holds that of rows[j]
     const float inverse = rsqrtf(sum + 1e-6f);
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const int i = 16 * wave + 2 * r + h;
       const bool ok = i < v.tokens;
-      const float iq = ok ? __shfl(inverse, 32 * h + 4 * r, 64) / norm_scale : 0.0f;
-      const float ik = ok ? __shfl(inverse, 32 * h + 4 * r + 2, 64) : 0.0f;
+      const float iq = ok ? __shfl(inverse, 32 * h + 2 * r, 64) / norm_scale : 0.0f;
+      const float ik = ok ? __shfl(inverse, 32 * h + 2 * r + 1, 64) : 0.0f;
       rows[2 * r] = scaled(rows[2 * r], iq);
       rows[2 * r + 1] = scaled(rows[2 * r + 1], ik);
       store4(&sm.q[i][4 * n], rows[2 * r]);
@@ -527,7 +541,7 @@ chunk_prepare_kernel(ChunkedArgs a) {
                      piece_at<kC>(wave, 4 * s));
     }
   }
-  const Record w_columns = v.wide(a.r.w_columns), w_rows = v.wide(a.r.w_rows), u_columns = v.wide(a.r.dl);
+  const Record w_columns = v.wide(a.r.w_columns), w_rows = v.wide(a.r.w_rows), u_columns = v.wide(a.r.u_columns);
   const unsigned column_at = piece_at<kC>(2 * wave, 0) + lane_piece<kC>(h, n);
   floatx16 w[2];
 #pragma unroll
@@ -617,20 +631,23 @@ chunk_states_forward_kernel(ChunkedArgs a) {
   const int head = slice.head, key_head = head / (a.vh / a.kh);
   const Record w_memory = head_records(a, a.r.w_rows, head, kWide), q_memory = head_records(a, a.r.q_rows, key_head, kWide),
                k_memory = head_records(a, a.r.k_columns, key_head, kWide),
-               p_memory = head_records(a, a.r.p_rows, head, kSquare), dl_memory = head_records(a, a.r.dl, head, kWide),
+               p_memory = head_records(a, a.r.p_rows, head, kSquare), u_memory = head_records(a, a.r.u_columns, head, kWide),
+               dl_memory = head_records(a, a.r.dl_rows, head, kWide),
                s0_memory = head_records(a, a.r.s0, head, kState),
                gates = head_records(a, a.r.gates, head, kGateRows * kC);
   // the lane's places in the records of the chunk whose operands are requested next
+  // four tokens of a column -> four columns of a token: the lane's place in rows(Dl)
+  const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;
   const unsigned core_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
   unsigned wide_at = 16 * lane, square_at = 16 * lane, gates_at = 4 * rows;
-  const unsigned delta_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
+  const unsigned u_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
   auto request_w = [&](int s) { w[s] = w_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
   auto request_q = [&](int s) { q[s] = q_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
   auto request_k = [&](int t, int s) { k[t][s] = k_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
   auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
   auto request_rest = [&]() {
 #pragma unroll
-    for (int c = 0; c < TILES; ++c) u[c] = dl_memory.get4(wide_at, delta_at + piece_at<kC>(c, 0));
+    for (int c = 0; c < TILES; ++c) u[c] = u_memory.get4(wide_at, u_at + piece_at<kC>(c, 0));
     e_rows = gates.get4(gates_at, 4 * kE * kC);
     l_rows = gates.get4(gates_at, 4 * kL * kC);
     decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
@@ -655,7 +672,7 @@ chunk_states_forward_kernel(ChunkedArgs a) {
   for (int chunk = 0; chunk < a.chunks; ++chunk) {
     const Tokens core = ChunkView(a, chunk, head).heads(a.core);
     // past the end the last chunk's operands are requested again
-    const unsigned wide_now = wide_at, state_now = 16 * lane + chunk * (kState * 4);
+    const unsigned delta_now = wide_at + transposed_at, state_now = 16 * lane + chunk * (kState * 4);
     if (chunk + 1 < a.chunks)
       wide_at += kWide * 4, square_at += kSquare * 4, gates_at += kGateRows * kC * 4;
 #pragma unroll
@@ -693,7 +710,8 @@ chunk_states_forward_kernel(ChunkedArgs a) {
     keep_order();
     request_rest();
 #pragma unroll
-    for (int c = 0; c < TILES; ++c) dl_memory.put4(dl[c], wide_now, delta_at + piece_at<kC>(c, 0));
+    for (int c = 0; c < TILES; ++c)
+      dl_memory.put4(quad_transpose(dl[c]), delta_now, piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
     keep_order();
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -768,12 +786,14 @@ chunk_states_backward_kernel(ChunkedArgs a) {
                p_memory = head_records(a, a.r.p_columns, head, kSquare),
                q_memory = head_records(a, a.r.q_columns, key_head, kWide),
                w_memory = head_records(a, a.r.w_columns, head, kWide),
-               ddl_memory = head_records(a, a.r.ddl, head, kWide), ds1_memory = head_records(a, a.r.ds1, head, kState),
+               ddl_memory = head_records(a, a.r.ddl_columns, head, kWide),
+               ddl_rows = head_records(a, a.r.ddl_rows, head, kWide), ds1_memory = head_records(a, a.r.ds1, head, kState),
                gates = head_records(a, a.r.gates, head, kGateRows * kC);
   const unsigned last = a.chunks - 1;
   unsigned wide_at = 16 * lane + last * (kWide * 4), square_at = 16 * lane + last * (kSquare * 4),
            gates_at = 4 * rows + last * (kGateRows * kC * 4);
   const unsigned delta_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
+  const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;  // as above
   const unsigned out_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
   auto request_out = [&](int chunk) {
     const Tokens d_out = ChunkView(a, max(chunk, 0), head).heads(a.dcore);
@@ -866,7 +886,11 @@ chunk_states_backward_kernel(ChunkedArgs a) {
     keep_order();
     request_out(chunk - 1);
 #pragma unroll
-    for (int c = 0; c < TILES; ++c) ddl_memory.put4(dd[c], wide_now, delta_at + piece_at<kC>(c, 0));
+    for (int c = 0; c < TILES; ++c) {
+      ddl_memory.put4(dd[c], wide_now, delta_at + piece_at<kC>(c, 0));
+      ddl_rows.put4(quad_transpose(dd[c]), wide_now + transposed_at,
+                    piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
+    }
     keep_order();
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -918,16 +942,17 @@ chunk_states_backward_kernel(ChunkedArgs a) {
 //      to da, db and the contribution to d A_log
 // 75 KiB of LDS and 256 registers: two workgroups a compute unit.
 constexpr int kSlab = 32;
+constexpr unsigned kSlabBytes = kC * kSlab * 4;
 struct GradientSmem {
   union {
-    float slab[4][kC][kSlab + 4];  // dDl, dO, Dl, V
+    unsigned char slab[2][4][kSlabBytes];  // two stages of rows(M) of dDl, dO, Dl, V, 32 columns each
     struct {
       float dw[kC][kWidePad], pd[kC][kSquarePad], x[kC][kSquarePad];
     };
   };
   float parts[6][kC][4];     // row sums of the waves' columns, see RowSum
   float row_n[kC][2], col_n[kC][2], row_p[kC][2], col_p[kC][2];  // by tile
-  float gate[kGateRows][kC];
+  float gate[kGateRows][kC], dots[2][kC];
   float dot[4];
 };
 enum RowSum { kSumQ, kSumK, kSumW, kSumV, kDotQ, kDotK };
@@ -951,146 +976,180 @@ chunk_gradients_kernel(ChunkedArgs a) {
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti) dw[ti] = dq[ti] = dk[ti] = zero_tile();
   float dot = 0.0f;
+  const int tile_col = 32 * tj_own + n;
+  const unsigned square_at = lane_piece<kC>(h, n);
+  const Record p_memory = v.square(a.r.p_columns), kkd = v.square(a.r.kkd), t_rows = v.square(a.r.t_rows),
+               t_columns = v.square(a.r.t_columns), ddl = v.wide(a.r.ddl_columns), q_memory = v.key(a.r.q_columns),
+               k_memory = v.key(a.r.k_columns), k_rows = v.key(a.r.k_rows);
+  const Tokens v_memory = v.v(), dv = v.dv();
+  // the lane's places in columns(M) of [64, 64] and [64, 128] matrices (four rows of one
+  // column, as in an accumulator), and a token's in the activations
+  const unsigned tile_at = square_at + piece_at<kC>(2 * tj_own, 8 * ti_own);
+  const unsigned column_at = square_at + piece_at<kC>(2 * wave, 0);
+  // rows of tokens are read and written four columns of one token a lane: token n % 4 of
+  // the four of a register quad, columns 4 (n / 4) .. + 3 of the wave's
+  const unsigned token_row = 4 * h + n % 4, token_column = 4 * (32 * wave + n / 4 * 4);
+  const unsigned token_at = token_row * v.row_bytes + token_column;
+  // row tile t of a per-row quantity in LDS, rows of register quad j
+  auto rows4 = [&](const float* rows, int t, int j) { return load4(rows + 32 * t + 8 * j + 4 * h); };
+  auto element = [](const float4& four, int i) {
+    return i % 4 == 0 ? four.x : i % 4 == 1 ? four.y : i % 4 == 2 ? four.z : four.w;
+  };
   {
-    const Record s0_memory = v.state(a.r.s0), s1_memory = v.state(a.r.ds1), ddl = v.wide(a.r.ddl),
-                 dl = v.wide(a.r.dl);
-    const Tokens d_out = v.heads(a.dcore), values = v.v();
+    const Record s0_memory = v.state(a.r.s0), s1_memory = v.state(a.r.ds1);
     const unsigned state_at = piece_at<kD>(2 * wave, 0) + lane_piece<kD>(h, n);
-    // thread (row, piece) of the slabs of dO and V: rows r and r + 32, 16 bytes; of dDl and
-    // Dl, which lie as columns: four tokens of one column in each half of the slab
-    const int row = tid / 8, piece = tid % 8 * 4;
-    const int row4 = tid / 16 * 4, column = tid % 16;
-    float4 staged[8];
-    auto request = [&](int slab) {
+    // fills of a stage: wave w brings row block w of the four matrices, in two parts
+    const int32x4 sources[4] = {
+        make_rsrc(a.r.ddl_rows + v.rec * kWide, kWide * 4), v.heads(a.dcore).words(),
+        make_rsrc(a.r.dl_rows + v.rec * kWide, kWide * 4), v.v().words()};
+    const unsigned record_at = piece_at<kD>(wave, 0) + 16 * lane;
+    const unsigned fill_at[4] = {record_at, (16 * wave + lane % 16) * v.out_bytes + lane / 16 * 16, record_at,
+                                 (16 * wave + lane % 16) * v.row_bytes + lane / 16 * 16};
+    auto fill = [&](int slab) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const unsigned c = 4 * kSlab * slab;
-        staged[4 * j] = ddl.get4(16 * tid, piece_at<kC>(2 * slab + j, 0));
-        staged[4 * j + 1] = d_out.get4(row * v.out_bytes + 4 * piece, 32 * j * v.out_bytes + c);
-        staged[4 * j + 2] = dl.get4(16 * tid, piece_at<kC>(2 * slab + j, 0));
-        staged[4 * j + 3] = values.get4(row * v.row_bytes + 4 * piece, 32 * j * v.row_bytes + c);
-      }
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+          const int quad = kSlab / 4 * slab + 4 * part;
+          lds_fill<16>(sources[m], sm.slab[slab % 2][m] + piece_at<kSlab>(wave, 4 * part),
+                       fill_at[m] + quad * (m % 2 == 0 ? kPiece : 16));
+        }
     };
-    request(0);
+    // a lane's place in a matrix of a stage: row n of row tile 0, quads 2 g + h
+    const unsigned tile_row_at = piece_at<kSlab>(n / 16, h) + n % 16 * 16;
     float4 s0[4], s1[4];
+    auto request = [&](int slab, int g) {
+      s0[g] = s0_memory.get4(state_at, piece_at<kD>(0, kSlab / 4 * slab + 2 * g));
+      s1[g] = s1_memory.get4(state_at, piece_at<kD>(0, kSlab / 4 * slab + 2 * g));
+    };
 #pragma unroll
-    for (int g = 0; g < 4; ++g) s0[g] = s0_memory.get4(state_at, piece_at<kD>(0, 2 * g)), s1[g] = s1_memory.get4(state_at, piece_at<kD>(0, 2 * g));
+    for (int g = 0; g < 4; ++g) request(0, g);
+    keep_order();
+    fill(0);
     float fv = 0.0f;
 #pragma unroll
     for (int slab = 0; slab < kD / kSlab; ++slab) {
-      if (slab > 0) lds_barrier();
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          const float4 four = staged[4 * j + m];
-          if (m % 2 == 1) {
-            store4(&sm.slab[m][row + 32 * j][piece], four);
-          } else {
-            sm.slab[m][row4][16 * j + column] = four.x;
-            sm.slab[m][row4 + 1][16 * j + column] = four.y;
-            sm.slab[m][row4 + 2][16 * j + column] = four.z;
-            sm.slab[m][row4 + 3][16 * j + column] = four.w;
-          }
-        }
-      if (slab == 0)
-        __syncthreads();
-      else
-        lds_barrier();
+      // The stage and the states' registers have arrived; naming the registers keeps the
+      // compiler from waiting for them below, behind requests it does not count.
+      asm volatile("s_waitcnt vmcnt(0)"
+                   : "+v"(s0[0].x), "+v"(s0[1].x), "+v"(s0[2].x), "+v"(s0[3].x), "+v"(s1[0].x), "+v"(s1[1].x),
+                     "+v"(s1[2].x), "+v"(s1[3].x)
+                   :
+                   : "memory");
+      __syncthreads();
       if (slab == 0) fv = sm.gate[kBeta][32 * tj_own + n];
-      if (slab + 1 < kD / kSlab) request(slab + 1);
-      __builtin_amdgcn_sched_barrier(0);
+      if (slab + 1 < kD / kSlab) fill(slab + 1);
+      keep_order();
+      const unsigned char(&stage)[4][kSlabBytes] = sm.slab[slab % 2];
+      auto operand = [&](int m, int ti, int g) {
+        return *reinterpret_cast<const float4*>(stage[m] + tile_row_at + piece_at<kSlab>(2 * ti, 2 * g));
+      };
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int c = 8 * g + 4 * h;
         dot += (s0[g].x * s1[g].x + s0[g].y * s1[g].y) + (s0[g].z * s1[g].z + s0[g].w * s1[g].w);
 #pragma unroll
         for (int ti = 0; ti < 2; ++ti) {
-          dw[ti] = mma(dw[ti], load4(&sm.slab[0][32 * ti + n][c]), s0[g]);
-          dq[ti] = mma(dq[ti], load4(&sm.slab[1][32 * ti + n][c]), s0[g]);
-          dk[ti] = mma(dk[ti], load4(&sm.slab[2][32 * ti + n][c]), s1[g]);
+          dw[ti] = mma(dw[ti], operand(0, ti, g), s0[g]);
+          dq[ti] = mma(dq[ti], operand(1, ti, g), s0[g]);
+          dk[ti] = mma(dk[ti], operand(2, ti, g), s1[g]);
         }
-        if (slab + 1 < kD / kSlab) {
-          s0[g] = s0_memory.get4(state_at, piece_at<kD>(0, kSlab / 4 * (slab + 1) + 2 * g));
-          s1[g] = s1_memory.get4(state_at, piece_at<kD>(0, kSlab / 4 * (slab + 1) + 2 * g));
-        }
+        keep_order();
+        if (slab + 1 < kD / kSlab) request(slab + 1, g);
+        keep_order();
         if (lower) {
-          dp = mma(dp, load4(&sm.slab[1][32 * ti_own + n][c]), load4(&sm.slab[2][32 * tj_own + n][c]));
-          dt = mma(dt, load4(&sm.slab[0][32 * ti_own + n][c]), scaled(load4(&sm.slab[3][32 * tj_own + n][c]), fv));
+          dp = mma(dp, operand(1, ti_own, g), operand(2, tj_own, g));
+          dt = mma(dt, operand(0, ti_own, g), scaled(operand(3, tj_own, g), fv));
         }
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
       }
     }
     dot = wave_sum(dot);
     if (lane == 0) sm.dot[wave] = dot;
   }
   lds_barrier();  // the slabs make room for dW, Pd and X
-  const int tile_col = 32 * tj_own + n;
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
     for (int i = 0; i < 16; ++i) sm.dw[32 * ti + tile_row(i, h)][col] = -dw[ti][i];
+  keep_order();
+  // Everything the [64, 64] part reads is requested a step before it is used.
+  float4 p_tile[4], k_own[kD / 8];
+  if (lower) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p_tile[j] = p_memory.get4(tile_at, piece_at<kC>(0, 2 * j));
+    keep_order();
+    const unsigned k_at = piece_at<kD>(2 * tj_own, 0) + lane_piece<kD>(h, n);
+#pragma unroll
+    for (int s = 0; s < kD / 8; ++s) k_own[s] = k_rows.get4(k_at, piece_at<kD>(0, 2 * s));
+  }
+  keep_order();
   // row and column sums of a tile held in an accumulator, for its rows and columns
   auto tile_sums = [&](const float (&values)[16], float (&row_sums)[kC][2], float (&col_sums)[kC][2],
-                       const float* weights) {
+                       bool weighted) {
     float sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      sum += weights ? weights[32 * ti_own + tile_row(i, h)] * values[i] : values[i];
+      sum += weighted ? element(rows4(sm.gate[kBeta], ti_own, i / 4), i) * values[i] : values[i];
     sum += __shfl_xor(sum, 32, 64);
     if (h == 0) col_sums[tile_col][ti_own] = sum;
     const float row_sum = half_sums(values);
-    if (n % 2 == 0) row_sums[32 * ti_own + tile_row(n / 2, h)][tj_own] = row_sum;
-  };
-  const Record p_memory = v.square(a.r.p_columns), kkd = v.square(a.r.kkd), t_rows = v.square(a.r.t_rows),
-               t_columns = v.square(a.r.t_columns), ddl = v.wide(a.r.ddl), q_memory = v.key(a.r.q_columns),
-               k_memory = v.key(a.r.k_columns), k_rows = v.key(a.r.k_rows);
-  const Tokens v_memory = v.v(), dv = v.dv();
-  // the lane's places in columns(M) of [64, 64] and [64, 128] matrices (four rows of one
-  // column, as in an accumulator), and a token's in the activations
-  const unsigned square_at = lane_piece<kC>(h, n), tile_at = square_at + piece_at<kC>(2 * tj_own, 8 * ti_own);
-  const unsigned column_at = square_at + piece_at<kC>(2 * wave, 0), token_at = 4 * h * v.row_bytes + 4 * col;
-  auto tile_of = [&](const Record& m, float (&values)[16]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float4 four = m.get4(tile_at, piece_at<kC>(0, 2 * j));
-      values[4 * j] = four.x, values[4 * j + 1] = four.y, values[4 * j + 2] = four.z, values[4 * j + 3] = four.w;
-    }
+    if (n < 16) row_sums[32 * ti_own + tile_row(n, h)][tj_own] = row_sum;
   };
   float decay[16];  // D of the tile
   if (lower) {
     float products[16];
-    tile_of(p_memory, products);
+    const float g_col = sm.gate[kG][tile_col];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = 32 * ti_own + tile_row(i, h);
       const bool in = row >= tile_col;
-      decay[i] = in ? expf(sm.gate[kG][row] - sm.gate[kG][tile_col]) : 0.0f;
+      decay[i] = in ? expf(element(rows4(sm.gate[kG], ti_own, i / 4), i) - g_col) : 0.0f;
       sm.pd[row][tile_col] = in ? dp[i] * decay[i] : 0.0f;
-      products[i] = in ? dp[i] * products[i] : 0.0f;
+      products[i] = in ? dp[i] * element(p_tile[i / 4], i) : 0.0f;
     }
-    tile_sums(products, sm.row_p, sm.col_p, nullptr);
+    tile_sums(products, sm.row_p, sm.col_p, false);
   }
+  float4 t_own[8];  // T^T for rows of the tile, then T for its columns
+  keep_order();
+  if (lower) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s >= 4 * ti_own) t_own[s] = t_columns.get4(square_at, piece_at<kC>(2 * ti_own, 2 * s));
+  }
+  keep_order();
   lds_barrier();
   if (lower) {
     const float fk = sm.gate[kBeta][tile_col] * sm.gate[kE][tile_col];
-    const unsigned k_at = piece_at<kD>(2 * tj_own, 0) + lane_piece<kD>(h, n);
 #pragma unroll
     for (int s = 0; s < kD / 8; ++s)
-      dt = mma(dt, load4(&sm.dw[32 * ti_own + n][8 * s + 4 * h]), scaled(k_rows.get4(k_at, piece_at<kD>(0, 2 * s)), fk));
+      dt = mma(dt, load4(&sm.dw[32 * ti_own + n][8 * s + 4 * h]), scaled(k_own[s], fk));
 #pragma unroll
     for (int i = 0; i < 16; ++i) sm.x[32 * ti_own + tile_row(i, h)][tile_col] = dt[i];
   }
+  keep_order();
+  // columns of K^ and Q^, both as operands and in the accumulators' rows
+  float4 kc[8], qc[8], kkd_tile[4];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) kc[s] = k_memory.get4(column_at, piece_at<kC>(0, 2 * s));
+  keep_order();
   lds_barrier();
   floatx16 z = zero_tile();
   if (lower) {
     // T^T dT: rows k < i of T's column i are zero, tile (0, 1) of dT is not needed
 #pragma unroll
     for (int s = 0; s < 8; ++s)
-      if (s >= 4 * ti_own)
-        z = mma(z, t_columns.get4(square_at, piece_at<kC>(2 * ti_own, 2 * s)),
-                gather4(&sm.x[8 * s + 4 * h][tile_col], kSquarePad));
+      if (s >= 4 * ti_own) z = mma(z, t_own[s], gather4(&sm.x[8 * s + 4 * h][tile_col], kSquarePad));
+    keep_order();
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s < 4 * (tj_own + 1)) t_own[s] = t_rows.get4(square_at, piece_at<kC>(2 * tj_own, 2 * s));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kkd_tile[j] = kkd.get4(tile_at, piece_at<kC>(0, 2 * j));
   }
+  keep_order();
+#pragma unroll
+  for (int s = 0; s < 8; ++s) qc[s] = q_memory.get4(column_at, piece_at<kC>(0, 2 * s));
+  keep_order();
   lds_barrier();
   if (lower) {
 #pragma unroll
@@ -1101,64 +1160,91 @@ chunk_gradients_kernel(ChunkedArgs a) {
   if (lower) {
 #pragma unroll
     for (int s = 0; s < 8; ++s)
-      if (s < 4 * (tj_own + 1))
-        da = mma(da, load4(&sm.x[32 * ti_own + n][8 * s + 4 * h]),
-                 t_rows.get4(square_at, piece_at<kC>(2 * tj_own, 2 * s)));
+      if (s < 4 * (tj_own + 1)) da = mma(da, load4(&sm.x[32 * ti_own + n][8 * s + 4 * h]), t_own[s]);
   }
   lds_barrier();
   if (lower) {
     // R + R^T, and the sums of N = dA (k^ . k^) D
     float products[16];
-    tile_of(kkd, products);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = 32 * ti_own + tile_row(i, h);
-      const bool in = row > tile_col;
-      const float value = in ? -da[i] : 0.0f;
-      products[i] = value * products[i];
-      const float r = value * sm.gate[kBeta][row] * decay[i];
+      const float value = row > tile_col ? -da[i] : 0.0f;
+      products[i] = value * element(kkd_tile[i / 4], i);
+      const float r = value * element(rows4(sm.gate[kBeta], ti_own, i / 4), i) * decay[i];
       if (row >= tile_col) sm.x[row][tile_col] = sm.x[tile_col][row] = r;
     }
-    tile_sums(products, sm.row_n, sm.col_n, sm.gate[kBeta]);
+    tile_sums(products, sm.row_n, sm.col_n, true);
   }
-  // columns of K^ and Q^, both as operands and in the accumulators' rows
-  float4 kc[8], qc[8];
+  keep_order();
+  // T^T for both row tiles (the columns of T of the second start at row 32), dDl's columns
+  float4 t_first[8], t_second[4], dd[8];
 #pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    kc[s] = k_memory.get4(column_at, piece_at<kC>(0, 2 * s));
-    qc[s] = q_memory.get4(column_at, piece_at<kC>(0, 2 * s));
-  }
-  auto element = [](const float4 (&c)[8], int ti, int i) {
-    const float4 four = c[4 * ti + i / 4];
-    return i % 4 == 0 ? four.x : i % 4 == 1 ? four.y : i % 4 == 2 ? four.z : four.w;
-  };
+  for (int s = 0; s < 8; ++s) t_first[s] = t_columns.get4(square_at, piece_at<kC>(0, 2 * s));
+#pragma unroll
+  for (int s = 0; s < 8; ++s) dd[s] = ddl.get4(column_at, piece_at<kC>(0, 2 * s));
+  keep_order();
   auto row_sums = [&](RowSum which, int ti, const float (&values)[16]) {
     const float sum = half_sums(values);
-    if (n % 2 == 0) sm.parts[which][32 * ti + tile_row(n / 2, h)][wave] = sum;
+    if (n < 16) sm.parts[which][32 * ti + tile_row(n, h)][wave] = sum;
   };
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti) {
-    float first[16], second[16];
+    float products[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      dq[ti][i] *= sm.gate[kE][row];
-      dk[ti][i] *= sm.gate[kL][row];
-      first[i] = dq[ti][i] * element(qc, ti, i);
-      second[i] = dk[ti][i] * element(kc, ti, i);
+      dq[ti][i] *= element(rows4(sm.gate[kE], ti, i / 4), i);
+      products[i] = dq[ti][i] * element(qc[4 * ti + i / 4], i);
     }
-    row_sums(kSumQ, ti, first);
-    row_sums(kSumK, ti, second);
+    row_sums(kSumQ, ti, products);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      dk[ti][i] *= element(rows4(sm.gate[kL], ti, i / 4), i);
+      products[i] = dk[ti][i] * element(kc[4 * ti + i / 4], i);
+    }
+    row_sums(kSumK, ti, products);
   }
+  keep_order();
   lds_barrier();
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti) {
     const int m = 32 * ti + n;
-    float4 t_col[8];
+    auto t_col = [&](int s) { return ti == 0 ? t_first[s] : t_second[s - 4]; };
+    float products[16];
+    floatx16 tu = zero_tile();
 #pragma unroll
-    for (int s = 4 * ti; s < 8; ++s) t_col[s] = t_columns.get4(square_at, piece_at<kC>(2 * ti, 2 * s));
-    __builtin_amdgcn_sched_barrier(0);
+    for (int s = 4 * ti; s < 8; ++s) tu = mma(tu, t_col(s), dd[s]);
+    floatx16 tw = zero_tile();
+#pragma unroll
+    for (int s = 4 * ti; s < 8; ++s) tw = mma(tw, t_col(s), gather4(&sm.dw[8 * s + 4 * h][col], kWidePad));
+    keep_order();
+    float4 values[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) values[j] = v_memory.get4(token_at, (32 * ti + 8 * j) * v.row_bytes);
+    if (ti == 0) {
+#pragma unroll
+      for (int s = 4; s < 8; ++s) t_second[s - 4] = t_columns.get4(square_at, piece_at<kC>(2, 2 * s));
+    }
+    keep_order();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float e = element(rows4(sm.gate[kE], ti, i / 4), i);
+      products[i] = tw[i] * element(kc[4 * ti + i / 4], i) * e;
+      dk[ti][i] += element(rows4(sm.gate[kBeta], ti, i / 4), i) * e * tw[i];
+    }
+    row_sums(kSumW, ti, products);
+    keep_order();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 value = quad_transpose(values[j]), beta = rows4(sm.gate[kBeta], ti, j);
+      products[4 * j] = tu[4 * j] * value.x, products[4 * j + 1] = tu[4 * j + 1] * value.y;
+      products[4 * j + 2] = tu[4 * j + 2] * value.z, products[4 * j + 3] = tu[4 * j + 3] * value.w;
+      dv.put4(quad_transpose(make_float4(beta.x * tu[4 * j], beta.y * tu[4 * j + 1], beta.z * tu[4 * j + 2],
+                                         beta.w * tu[4 * j + 3])),
+              token_at, (32 * ti + 8 * j) * v.row_bytes);
+    }
+    row_sums(kSumV, ti, products);
+    keep_order();
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const int k = 8 * s + 4 * h;
@@ -1166,61 +1252,44 @@ chunk_gradients_kernel(ChunkedArgs a) {
       dk[ti] = mma(dk[ti], load4(&sm.x[m][k]), kc[s]);
       if (s >= 4 * ti) dk[ti] = mma(dk[ti], gather4(&sm.pd[k][m], kSquarePad), qc[s]);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    float products[16];
-    {
-      floatx16 tw = zero_tile();
+    keep_order();
 #pragma unroll
-      for (int s = 4 * ti; s < 8; ++s)
-        tw = mma(tw, t_col[s], gather4(&sm.dw[8 * s + 4 * h][col], kWidePad));
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = 32 * ti + tile_row(i, h);
-        products[i] = tw[i] * element(kc, ti, i) * sm.gate[kE][row];
-        dk[ti][i] += sm.gate[kBeta][row] * sm.gate[kE][row] * tw[i];
-      }
-      row_sums(kSumW, ti, products);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      floatx16 tu = zero_tile();
-#pragma unroll
-      for (int s = 4 * ti; s < 8; ++s)
-        tu = mma(tu, t_col[s], ddl.get4(column_at, piece_at<kC>(0, 2 * s)));
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const unsigned row = (32 * ti + tile_row(i, 0)) * v.row_bytes;
-        products[i] = tu[i] * v_memory.get(token_at, row);
-        dv.put(sm.gate[kBeta][32 * ti + tile_row(i, h)] * tu[i], token_at, row);
-      }
-      row_sums(kSumV, ti, products);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) products[i] = dq[ti][i] * element(qc, ti, i);
+    for (int i = 0; i < 16; ++i) products[i] = dq[ti][i] * element(qc[4 * ti + i / 4], i);
     row_sums(kDotQ, ti, products);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) products[i] = dk[ti][i] * element(kc, ti, i);
+    for (int i = 0; i < 16; ++i) products[i] = dk[ti][i] * element(kc[4 * ti + i / 4], i);
     row_sums(kDotK, ti, products);
+    keep_order();
   }
   lds_barrier();
+  // over the waves; the two that every lane needs below once for all of them
   auto across_waves = [&](RowSum which, int row) {
     const float4 four = load4(sm.parts[which][row]);
     return (four.x + four.y) + (four.z + four.w);
   };
-  const auto partials = v.qk_partials();
+  if (tid < 2 * kC) sm.dots[tid / kC][tid % kC] = across_waves(tid < kC ? kDotQ : kDotK, tid % kC);
+  lds_barrier();
+  const Tokens partials = v.qk_partials();
   // back through the L2 normalisations (and the 1/sqrt(d) of q, which kQScale has)
+  const unsigned partial_at = 2 * token_row * v.out_bytes + token_column;
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 32 * ti + tile_row(i, h);
-      const unsigned uniform = 2 * (32 * ti + tile_row(i, 0)) * v.out_bytes;
-      partials.put(sm.gate[kQScale][row] *
-                       (dq[ti][i] - static_cast<float>(kD) * element(qc, ti, i) * across_waves(kDotQ, row)),
-                   8 * h * v.out_bytes + 4 * col, uniform);
-      partials.put(sm.gate[kKScale][row] * (dk[ti][i] - element(kc, ti, i) * across_waves(kDotK, row)),
-                   8 * h * v.out_bytes + 4 * (kD + col), uniform);
+    for (int j = 0; j < 4; ++j) {
+      const float4 q = qc[4 * ti + j], k = kc[4 * ti + j], q_dot = rows4(sm.dots[0], ti, j),
+                   k_dot = rows4(sm.dots[1], ti, j), q_scale = rows4(sm.gate[kQScale], ti, j),
+                   k_scale = rows4(sm.gate[kKScale], ti, j);
+      float from_q[4], from_k[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        from_q[e] = element(q_scale, e) *
+                    (dq[ti][4 * j + e] - static_cast<float>(kD) * element(q, e) * element(q_dot, e));
+        from_k[e] = element(k_scale, e) * (dk[ti][4 * j + e] - element(k, e) * element(k_dot, e));
+      }
+      const unsigned uniform = 2 * (32 * ti + 8 * j) * v.out_bytes;
+      partials.put4(quad_transpose(make_float4(from_q[0], from_q[1], from_q[2], from_q[3])), partial_at, uniform);
+      partials.put4(quad_transpose(make_float4(from_k[0], from_k[1], from_k[2], from_k[3])), partial_at,
+                    uniform + 4 * kD);
     }
   if (wave != 0) return;
   // the gates: lane i is token i
@@ -1279,8 +1348,10 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
   };
   a.r.w_rows = take(kWide);
   a.r.w_columns = take(kWide);
-  a.r.dl = take(kWide);
-  a.r.ddl = take(kWide);
+  a.r.u_columns = take(kWide);
+  a.r.dl_rows = take(kWide);
+  a.r.ddl_rows = take(kWide);
+  a.r.ddl_columns = take(kWide);
   a.r.p_rows = take(kSquare);
   a.r.p_columns = take(kSquare);
   a.r.t_rows = take(kSquare);
