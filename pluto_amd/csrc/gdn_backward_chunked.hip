@@ -45,7 +45,7 @@
 // Matrix products run on v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32, whose
 // rate bounds all of this (about 55 GFLOP at 2048 tokens of 48 heads, 360 us of the
 // card's FP32 matrix rate); the triangular factors are multiplied by halves.  At that
-// size the kernels of this file take @TOTAL@ us, where one kernel a term of the
+// size the kernels of this file take 770 us, where one kernel a term of the
 // formulas above, with M and B, took 1766 us.
 #include "gdn.h"
 
@@ -340,38 +340,69 @@ chunk_prepare_kernel(ChunkedArgs a) {
   const int h = lane / 32, n = lane % 32, quarter = lane / 16, n16 = lane % 16;
   float* gates = a.r.gates + v.rec * kGateRows * kC;
 
-  // normalised rows (1e-6 added to the sums of squares, sequence_delta_net.cc:84-85):
-  // half a wave a row, row 16 wave + 2 r + h
+  // normalised rows (1e-6 added to the sums of squares, sequence_delta_net.cc:84-85) of
+  // sixteen tokens a wave, a row a quarter of it: channels 4 n16 .. + 3 and 64 further a
+  // lane.  A row's squares are added by the tree of wave_sum over channels c and c +
+  // 64, so that the scales are those of the other kernels to the bit (an error of a
+  // scale moves a whole row of outputs over the ties of their rounding); the trees of
+  // eight rows share their steps.
   {
-    const float norm_scale = sqrtf(static_cast<float>(kD));
+    const float norm_scale = sqrtf(static_cast<float>(kD)), inverse_norm_scale = 1.0f / norm_scale;
     const Tokens q = v.activations(a.post, v.key_head() * kD),
                  k = v.activations(a.post, (a.kh + v.key_head()) * kD);
-    const unsigned at = (16 * wave + h) * v.row_bytes + 16 * n;
-    float4 rows[16];
-    float squares[16];
+    const unsigned at = (16 * wave + quarter) * v.row_bytes + 16 * n16;
+    float rows[8][2][4], squares[8][4];  // q^ and k^ of rows quarter, 4 + quarter, ...
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      rows[2 * r] = q.get4(at, 2 * r * v.row_bytes);
-      rows[2 * r + 1] = k.get4(at, 2 * r * v.row_bytes);
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float4 qv = q.get4(at, 4 * g * v.row_bytes + 256 * j), kv = k.get4(at, 4 * g * v.row_bytes + 256 * j);
+        rows[2 * g][j][0] = qv.x, rows[2 * g][j][1] = qv.y, rows[2 * g][j][2] = qv.z, rows[2 * g][j][3] = qv.w;
+        rows[2 * g + 1][j][0] = kv.x, rows[2 * g + 1][j][1] = kv.y, rows[2 * g + 1][j][2] = kv.z,
+        rows[2 * g + 1][j][3] = kv.w;
+      }
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        squares[r][c] = rows[r][0][c] * rows[r][0][c] + rows[r][1][c] * rows[r][1][c];
+    // lane n16 is left with row n16 / 2
+#pragma unroll
+    for (int width = 4; width > 0; width /= 2) {
+      const bool upper = n16 & (2 * width);
+#pragma unroll
+      for (int r = 0; r < width; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float kept = upper ? squares[r + width][c] : squares[r][c];
+          const float sent = upper ? squares[r][c] : squares[r + width][c];
+          squares[r][c] = kept + __shfl_xor(sent, 2 * width, 64);
+        }
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      squares[r] = (rows[r].x * rows[r].x + rows[r].y * rows[r].y) +
-                   (rows[r].z * rows[r].z + rows[r].w * rows[r].w);
-    const float sum = half_sums(squares);  // lane j holds that of rows[j]
-    const float inverse = rsqrtf(sum + 1e-6f);
+    for (int c = 0; c < 4; ++c) squares[0][c] += __shfl_xor(squares[0][c], 1, 64);
+    const float inverse =
+        rsqrtf((squares[0][0] + squares[0][2]) + (squares[0][1] + squares[0][3]) + 1e-6f);
+    // x / norm_scale, rounded once: quotient, remainder and its part of the quotient
+    auto normed = [&](float x) {
+      const float y = x * inverse_norm_scale;
+      return fmaf(fmaf(-y, norm_scale, x), inverse_norm_scale, y);
+    };
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int i = 16 * wave + 2 * r + h;
+    for (int g = 0; g < 4; ++g) {
+      const int i = 16 * wave + 4 * g + quarter;
       const bool ok = i < v.tokens;
-      const float iq = ok ? __shfl(inverse, 32 * h + 2 * r, 64) / norm_scale : 0.0f;
-      const float ik = ok ? __shfl(inverse, 32 * h + 2 * r + 1, 64) : 0.0f;
-      rows[2 * r] = scaled(rows[2 * r], iq);
-      rows[2 * r + 1] = scaled(rows[2 * r + 1], ik);
-      store4(&sm.q[i][4 * n], rows[2 * r]);
-      store4(&sm.k[i][4 * n], rows[2 * r + 1]);
-      if (n == 0) {
-        gates[kQScale * kC + i] = iq;
+      const float iq = ok ? __shfl(inverse, 16 * quarter + 4 * g, 64) : 0.0f;
+      const float ik = ok ? __shfl(inverse, 16 * quarter + 4 * g + 2, 64) : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float(&qv)[4] = rows[2 * g][j], (&kv)[4] = rows[2 * g + 1][j];
+        store4(&sm.q[i][4 * n16 + 64 * j], make_float4(normed(qv[0] * iq), normed(qv[1] * iq), normed(qv[2] * iq),
+                                                       normed(qv[3] * iq)));
+        store4(&sm.k[i][4 * n16 + 64 * j], make_float4(kv[0] * ik, kv[1] * ik, kv[2] * ik, kv[3] * ik));
+      }
+      if (n16 == 0) {
+        gates[kQScale * kC + i] = iq / norm_scale;
         gates[kKScale * kC + i] = ik;
       }
     }
@@ -389,11 +420,14 @@ chunk_prepare_kernel(ChunkedArgs a) {
       const float bv = bf16_bits_to_float(a.b[static_cast<size_t>(t) * a.vh + v.head]);
       beta = round_if(1.0f / (1.0f + expf(-bv)), a.round);
     }
+    // one after the other: an error of the running sum scales whole rows
+    float sum = 0.0f;
 #pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-      const float before = __shfl_up(g, offset, 64);
-      if (lane >= offset) g += before;
+    for (int i = 0; i < kC; ++i) {
+      const float next = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g), i));
+      sum = lane >= i ? sum + next : sum;
     }
+    g = sum;
     const float e = expf(g), l = expf(__shfl(g, 63, 64) - g);
     gates[kG * kC + lane] = g;
     gates[kBeta * kC + lane] = beta;
