@@ -20,6 +20,8 @@
 
 #include "mfma_tile.h"
 
+#include <algorithm>
+
 namespace pluto_hip {
 namespace {
 
@@ -57,30 +59,49 @@ __device__ inline float operand_value(float value) {
     return round_to_bf16(value);
 }
 
-// out[r, c] = operand(in[r, c]) or, transposed, out[c, r] = operand(in[r, c]).
-template <bool HALF, bool TRANSPOSE>
+// out[i] = operand(in[i]): eight elements a thread where both are aligned, thread `index`
+// of `threads`.
+template <bool HALF>
+__device__ inline void convert_elements(const float* in, long long total, uint16_t* out,
+                                        long long index, long long threads) {
+  const bool wide = reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  const long long eights = wide ? total / 8 : 0;
+  for (long long i = index; i < eights; i += threads) {
+    const float4 a = *reinterpret_cast<const float4*>(in + 8 * i);
+    const float4 b = *reinterpret_cast<const float4*>(in + 8 * i + 4);
+    ushort4 lo, hi;
+    lo.x = to_operand<HALF>(a.x), lo.y = to_operand<HALF>(a.y), lo.z = to_operand<HALF>(a.z);
+    lo.w = to_operand<HALF>(a.w), hi.x = to_operand<HALF>(b.x), hi.y = to_operand<HALF>(b.y);
+    hi.z = to_operand<HALF>(b.z), hi.w = to_operand<HALF>(b.w);
+    *reinterpret_cast<ushort4*>(out + 8 * i) = lo;
+    *reinterpret_cast<ushort4*>(out + 8 * i + 4) = hi;
+  }
+  for (long long i = 8 * eights + index; i < total; i += threads) out[i] = to_operand<HALF>(in[i]);
+}
+
+// What a product needs converted, in one launch: the first blocks transpose the matrix
+// [rows, cols] to out [cols, rows] by tiles of 32, the rest convert the input.
+template <bool HALF>
 __global__ void __launch_bounds__(256)
-convert_kernel(const float* in, long long rows, int cols, uint16_t* out) {
-  if constexpr (!TRANSPOSE) {
-    const long long total = rows * cols;
-    for (long long i = blockIdx.x * 256LL + threadIdx.x; i < total; i += 256LL * gridDim.x)
-      out[i] = to_operand<HALF>(in[i]);
-  } else {
-    __shared__ uint16_t tile[32][33];
-    const int c0 = blockIdx.x * 32;
-    const long long r0 = blockIdx.y * 32LL;
-    const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
-    for (int j = ty; j < 32; j += 8) {
-      const long long r = r0 + j;
-      const int c = c0 + tx;
-      tile[j][tx] = (r < rows && c < cols) ? to_operand<HALF>(in[r * cols + c]) : 0;
-    }
-    __syncthreads();
-    for (int j = ty; j < 32; j += 8) {
-      const int c = c0 + j;
-      const long long r = r0 + tx;
-      if (c < cols && r < rows) out[c * rows + r] = tile[tx][j];
-    }
+convert_forward_kernel(const float* matrix, int rows, int cols, uint16_t* out, int tiles,
+                       const float* input, long long elements, uint16_t* input16) {
+  if (static_cast<int>(blockIdx.x) >= tiles) {
+    convert_elements<HALF>(input, elements, input16, (blockIdx.x - tiles) * 256LL + threadIdx.x,
+                           (gridDim.x - tiles) * 256LL);
+    return;
+  }
+  __shared__ uint16_t tile[32][33];
+  const int across = (cols + 31) / 32;
+  const int c0 = blockIdx.x % across * 32, r0 = blockIdx.x / across * 32;
+  const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+  for (int j = ty; j < 32; j += 8) {
+    const int r = r0 + j, c = c0 + tx;
+    tile[j][tx] = (r < rows && c < cols) ? to_operand<HALF>(matrix[static_cast<long long>(r) * cols + c]) : 0;
+  }
+  __syncthreads();
+  for (int j = ty; j < 32; j += 8) {
+    const int c = c0 + j, r = r0 + tx;
+    if (c < cols && r < rows) out[static_cast<long long>(c) * rows + r] = tile[tx][j];
   }
 }
 
@@ -209,19 +230,183 @@ product_rows_kernel(ProductArgs a) {
     }
 }
 
-// Short contractions take 128 x 128 tiles (more workgroups to overlap the
-// start-up and the stores); from 1536 elements on, 256 x 256 tiles of eight
-// waves, which halve the operand traffic from L2, are faster.
+// The same product with one wave a SIMD: four waves, arranged 2 x 2, each with a (32 JM) x
+// (32 JN) part of a (64 JM) x (64 JN) tile, which read each operand from LDS for JN or
+// JM matrix instructions.  Nothing but the wave itself fills the matrix pipe: a row of
+// the left operand is read again for the next 16-element step as soon as it has been
+// multiplied, the right operand a step ahead; the barrier of a stage stands before its
+// last step (whose operands are in registers), and the fills of the stage after
+// next, one every other instruction, follow it.
+template <bool HALF, int JM, int JN>
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(1, 1)))
+product_rows_wide_kernel(ProductArgs a) {
+  constexpr int KS = kDepth / 16;
+  constexpr int TM = 64 * JM, TN = 64 * JN;
+  constexpr int kLeftBytes = TM * kDepth * 2, kStageBytes = kLeftBytes + TN * kDepth * 2;
+  constexpr int LEFT_LOADS = TM * (kDepth / 8) / 256, RIGHT_LOADS = TN * (kDepth / 8) / 256;
+  constexpr int LOADS = LEFT_LOADS + RIGHT_LOADS;
+  static_assert(LOADS <= 3 * (JM * JN / 2), "the fills stand between the instructions of three steps");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int h = lane / 32, n = lane % 32;
+  const int n_tiles = (a.n_rows + TN - 1) / TN;
+  const int logical = xcd_logical_block();
+  const int m0 = __builtin_amdgcn_readfirstlane(logical / n_tiles * TM);
+  const int n0 = __builtin_amdgcn_readfirstlane(logical % n_tiles * TN);
+  const int wm = 32 * JM * (wave / 2), wn = 32 * JN * (wave % 2);
+  // loads of a wave are eight rows apart, which keeps the swizzle: one lane offset.
+  // Columns beyond the contraction are rows of their own to the descriptor; those of
+  // the last stages read zeros or another row's start into a stage nobody reads.
+  const int32x4 left = make_rsrc(a.left + static_cast<long long>(m0) * a.depth,
+                                 static_cast<uint32_t>(static_cast<long long>(a.m_rows - m0) * a.depth * 2));
+  const int32x4 right = make_rsrc(a.right + static_cast<long long>(n0) * a.depth,
+                                  static_cast<uint32_t>(static_cast<long long>(a.n_rows - n0) * a.depth * 2));
+  uint32_t fill_at[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i)
+    fill_at[i] = i < LEFT_LOADS ? tile_fill_offset<kDepth>((wave * LEFT_LOADS + i) * 64 + lane, a.depth)
+                                : tile_fill_offset<kDepth>((wave * RIGHT_LOADS + i - LEFT_LOADS) * 64 + lane, a.depth);
+  const uint32_t left_stage = lds_address(lds) + wave * LEFT_LOADS * 1024;
+  const uint32_t right_stage = lds_address(lds) + kLeftBytes + wave * RIGHT_LOADS * 1024;
+  auto fill = [&](int stage, int i) {
+    if (i < LEFT_LOADS)
+      lds_fill_at<16>(left, left_stage + stage * kStageBytes + i * 1024, fill_at[i]);
+    else
+      lds_fill_at<16>(right, right_stage + stage * kStageBytes + (i - LEFT_LOADS) * 1024, fill_at[i]);
+    fill_at[i] += kDepth * 2;
+  };
+  constexpr int kBlockStep = 32 * (kDepth / 8) * 16;
+  int left_read[KS], right_read[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    left_read[ks] = tile_row_read<kDepth>(wm + n, 2 * ks + h);
+    right_read[ks] = kLeftBytes + tile_row_read<kDepth>(wn + n, 2 * ks + h);
+  }
+  floatx16 acc[JM][JN];
+#pragma unroll
+  for (int jn = 0; jn < JN; ++jn) {
+    const int column = n0 + wn + 32 * jn + n;
+    const float start = (a.bias && column < a.n_rows) ? a.bias[column] : 0.0f;
+#pragma unroll
+    for (int jm = 0; jm < JM; ++jm)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[jm][jn][i] = start;
+  }
+  const int steps = a.depth / kDepth;
+  uint4 l[JM], r[2][JN];
+  auto read_left = [&](int stage, int ks, int j) {
+    l[j] = *reinterpret_cast<const uint4*>(lds + left_read[ks] + stage * kStageBytes + j * kBlockStep);
+  };
+  auto read_right = [&](int stage, int ks, int j) {
+    r[ks & 1][j] = *reinterpret_cast<const uint4*>(lds + right_read[ks] + stage * kStageBytes + j * kBlockStep);
+  };
+  // the products of step ks, the reads of step `next` of a stage behind their operands'
+  // last use, and fills first .. first + JM JN / 2 - 1 of a stage between
+  auto multiply = [&](int ks, int next_stage, int next, int fill_stage, int first) {
+#pragma unroll
+    for (int jm = 0; jm < JM; ++jm) {
+#pragma unroll
+      for (int jn = 0; jn < JN; ++jn) {
+        const int i = jm * JN + jn;
+        acc[jm][jn] = mma<HALF>(l[jm], r[ks & 1][jn], acc[jm][jn]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (first >= 0 && i % 2 == 1 && first + i / 2 < LOADS) {
+          fill(fill_stage, first + i / 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (jm == 0) read_right(next_stage, next, jn);
+      }
+      read_left(next_stage, next, jm);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr int PART = JM * JN / 2;
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) fill(0, i);
+  wait_loads<0>();
+  lds_barrier();
+#pragma unroll
+  for (int j = 0; j < JN; ++j) read_right(0, 0, j);
+#pragma unroll
+  for (int j = 0; j < JM; ++j) read_left(0, 0, j);
+#pragma unroll
+  for (int i = 0; i < PART && i < LOADS; ++i) fill(1, i);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int step = 0; step < steps; step += 2) {
+#pragma unroll
+    for (int stage = 0; stage < 2; ++stage) {
+      if (stage == 1 && step + 1 >= steps) break;
+      multiply(0, stage, 1, stage ^ 1, PART);
+      multiply(1, stage, 2, stage ^ 1, 2 * PART);
+      multiply(2, stage, 3, stage ^ 1, -1);
+      // the next stage has landed, and every wave has read the last of this one
+      wait_loads<0>();
+      lds_barrier();
+      multiply(3, stage ^ 1, 0, stage, 0);
+    }
+  }
+  wait_loads<0>();  // no fill may land after the workgroup has given its LDS back
+  // four rows of one column a lane -> four columns of one row: 128 (or 64) contiguous
+  // bytes of eight rows a store
+  const int row0 = m0 + wm + 4 * h + n % 4, column0 = n0 + wn + n / 4 * 4;
+#pragma unroll
+  for (int jm = 0; jm < JM; ++jm)
+#pragma unroll
+    for (int jn = 0; jn < JN; ++jn)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const floatx16& c = acc[jm][jn];
+        const float4 v = quad_transpose(make_float4(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]));
+        const int row = row0 + 32 * jm + 8 * q, column = column0 + 32 * jn;
+        if (row >= a.m_rows || column >= a.n_rows) continue;
+        const long long at = static_cast<long long>(row) * a.n_rows + column;
+        if (a.out_bf16)
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + at) =
+              make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w));
+        else
+          *reinterpret_cast<float4*>(static_cast<float*>(a.out) + at) = v;
+      }
+}
+
+// A tile of a product: its size, the time of a 64-element step of one workgroup when a
+// compute unit has it alone, and per workgroup when compute units are full, in units of
+// 10 ns.
+struct Tile {
+  int rows, columns, alone, full;
+};
+constexpr Tile kWideTile = {256, 192, 108, 125};   // product_rows_wide_kernel<4, 3>
+constexpr Tile kMediumTile = {64, 128, 58, 35};    // product_rows_kernel<1, 2>
+constexpr Tile kSmallTile = {64, 64, 50, 20};      // product_rows_kernel<1, 1>
+
+// The time of a product with one kind of tiles: its steps, and the filling of the first
+// stages and the stores at about five of them, as often as compute units take turns.
+long long product_time(const Tile& t, int rows, int columns, int slices, int steps) {
+  constexpr long long kComputeUnits = 256;
+  const long long tiles = 1LL * ((rows + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns) * slices;
+  const long long turns = (tiles + kComputeUnits - 1) / kComputeUnits;
+  return (steps + 5LL) * std::max<long long>(t.alone, turns * t.full);
+}
+
+// 16384 x 768 -> 2304 and its input gradient take 72 and 53 us in wide tiles (89 and 75 in
+// tiles of 128 x 128 or, with eight waves, 256 x 256); 4096 x 2304 -> 768 26 us in small
+// ones (33, 64) and 500 rows of it 16 (28, 58).
 template <bool HALF>
 void launch_product_rows(hipStream_t s, const ProductArgs& p) {
-  auto blocks = [&](int tm, int tn) {
-    return static_cast<unsigned>((p.m_rows + tm - 1) / tm) *
-           static_cast<unsigned>((p.n_rows + tn - 1) / tn);
+  auto blocks = [&](const Tile& t) {
+    return static_cast<unsigned>((p.m_rows + t.rows - 1) / t.rows) *
+           static_cast<unsigned>((p.n_rows + t.columns - 1) / t.columns);
   };
-  if (p.depth >= 1536)
-    product_rows_kernel<HALF, 4, 2, 2, 8><<<blocks(256, 256), 512, 0, s>>>(p);
+  auto time = [&](const Tile& t) { return product_time(t, p.m_rows, p.n_rows, 1, p.depth / kDepth); };
+  const long long wide = time(kWideTile), medium = time(kMediumTile), small = time(kSmallTile);
+  const bool aligned = reinterpret_cast<uintptr_t>(p.out) % 16 == 0;  // it stores whole quads
+  if (aligned && wide <= medium && wide <= small)
+    product_rows_wide_kernel<HALF, 4, 3><<<blocks(kWideTile), 256, 0, s>>>(p);
+  else if (medium <= small)
+    product_rows_kernel<HALF, 1, 2, 2, 4><<<blocks(kMediumTile), 256, 0, s>>>(p);
   else
-    product_rows_kernel<HALF, 2, 2, 2, 4><<<blocks(128, 128), 256, 0, s>>>(p);
+    product_rows_kernel<HALF, 1, 1, 2, 4><<<blocks(kSmallTile), 256, 0, s>>>(p);
 }
 
 struct GramArgs {
@@ -328,14 +513,162 @@ product_columns_kernel(GramArgs a) {
     }
 }
 
-// out[i] = sum over slices of partial[slice][i], ascending.
+// The same in (64 JM) x (64 JN) tiles with one wave a SIMD, as product_rows_wide_kernel.
+template <bool HALF, int JM, int JN>
 __global__ void __launch_bounds__(256)
-sum_slices_kernel(const float* partial, long long elements, int slices, float* out) {
-  const long long i = blockIdx.x * 256LL + threadIdx.x;
-  if (i >= elements) return;
-  float sum = 0.0f;
-  for (int s = 0; s < slices; ++s) sum += partial[s * elements + i];
-  out[i] = sum;
+__attribute__((amdgpu_waves_per_eu(1, 1)))
+product_columns_wide_kernel(GramArgs a) {
+  constexpr int kRows = 64, KS = kRows / 16;
+  constexpr int TM = 64 * JM, TN = 64 * JN;
+  constexpr int kLeftBytes = kRows * TM * 2, kStageBytes = kLeftBytes + kRows * TN * 2;
+  constexpr int LEFT_LOADS = kRows * (TM / 8) / 256, RIGHT_LOADS = kRows * (TN / 8) / 256;
+  constexpr int LOADS = LEFT_LOADS + RIGHT_LOADS;
+  static_assert(LOADS <= 3 * (JM * JN / 2), "the fills stand between the instructions of three steps");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int h = lane / 32, n = lane % 32;
+  const int n_tiles = (a.n_cols + TN - 1) / TN, m_tiles = (a.m_cols + TM - 1) / TM;
+  const int tile = blockIdx.x % (n_tiles * m_tiles);
+  const int slice = __builtin_amdgcn_readfirstlane(blockIdx.x / (n_tiles * m_tiles));
+  const int m0 = __builtin_amdgcn_readfirstlane(tile / n_tiles * TM);
+  const int n0 = __builtin_amdgcn_readfirstlane(tile % n_tiles * TN);
+  const int wm = 32 * JM * (wave / 2), wn = 32 * JN * (wave % 2);
+  const int per_slice = ((a.rows + a.slices - 1) / a.slices + kRows - 1) / kRows * kRows;
+  const int first = slice * per_slice, last = min(first + per_slice, a.rows);
+  const int steps = first < last ? (last - first + kRows - 1) / kRows : 0;
+  // Columns beyond a matrix are the start of its next row, which only reaches output
+  // elements that are not stored; rows beyond the slice read zeros.
+  auto source = [&](const uint16_t* matrix, int stride, int col0) {
+    const long long elements = static_cast<long long>(last - first) * stride - col0;
+    return make_rsrc(matrix + static_cast<long long>(first) * stride + col0,
+                     elements <= 0 ? 0u : static_cast<uint32_t>(elements * 2));
+  };
+  const int32x4 left = source(a.left, a.m_cols, m0), right = source(a.right, a.n_cols, n0);
+  uint32_t fill_at[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i)
+    fill_at[i] = i < LEFT_LOADS ? tile_fill_offset<TM>((wave * LEFT_LOADS + i) * 64 + lane, a.m_cols)
+                                : tile_fill_offset<TN>((wave * RIGHT_LOADS + i - LEFT_LOADS) * 64 + lane, a.n_cols);
+  const uint32_t left_stage = lds_address(lds) + wave * LEFT_LOADS * 1024;
+  const uint32_t right_stage = lds_address(lds) + kLeftBytes + wave * RIGHT_LOADS * 1024;
+  auto fill = [&](int stage, int i) {
+    if (i < LEFT_LOADS)
+      lds_fill_at<16>(left, left_stage + stage * kStageBytes + i * 1024, fill_at[i]);
+    else
+      lds_fill_at<16>(right, right_stage + stage * kStageBytes + (i - LEFT_LOADS) * 1024, fill_at[i]);
+    fill_at[i] += kRows * 2 * (i < LEFT_LOADS ? a.m_cols : a.n_cols);
+  };
+  // blocks of 32 columns two apart share the swizzle
+  int left_read[2], right_read[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    left_read[j] = tile_transpose_read<TM>(lane, wm / 32 + j);
+    right_read[j] = kLeftBytes + tile_transpose_read<TN>(lane, wn / 32 + j);
+  }
+  floatx16 acc[JM][JN];
+#pragma unroll
+  for (int jm = 0; jm < JM; ++jm)
+#pragma unroll
+    for (int jn = 0; jn < JN; ++jn)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[jm][jn][i] = 0.0f;
+  uint4 l[JM], r[2][JN];
+  auto read_left = [&](int stage, int ks, int j) {
+    l[j] = __builtin_bit_cast(uint4, tile_transposed_operand<TM>(lds + stage * kStageBytes + j / 2 * 128,
+                                                                 left_read[j % 2], ks));
+  };
+  auto read_right = [&](int stage, int ks, int j) {
+    r[ks & 1][j] = __builtin_bit_cast(uint4, tile_transposed_operand<TN>(lds + stage * kStageBytes + j / 2 * 128,
+                                                                         right_read[j % 2], ks));
+  };
+  auto multiply = [&](int ks, int next_stage, int next, int fill_stage, int first_fill) {
+#pragma unroll
+    for (int jm = 0; jm < JM; ++jm) {
+#pragma unroll
+      for (int jn = 0; jn < JN; ++jn) {
+        const int i = jm * JN + jn;
+        acc[jm][jn] = mma<HALF>(l[jm], r[ks & 1][jn], acc[jm][jn]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (first_fill >= 0 && i % 2 == 1 && first_fill + i / 2 < LOADS) {
+          fill(fill_stage, first_fill + i / 2);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (jm == 0) read_right(next_stage, next, jn);
+      }
+      read_left(next_stage, next, jm);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  constexpr int PART = JM * JN / 2;
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) fill(0, i);
+  wait_loads<0>();
+  lds_barrier();
+#pragma unroll
+  for (int j = 0; j < JN; ++j) read_right(0, 0, j);
+#pragma unroll
+  for (int j = 0; j < JM; ++j) read_left(0, 0, j);
+#pragma unroll
+  for (int i = 0; i < PART && i < LOADS; ++i) fill(1, i);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int step = 0; step < steps; step += 2) {
+#pragma unroll
+    for (int stage = 0; stage < 2; ++stage) {
+      if (stage == 1 && step + 1 >= steps) break;
+      multiply(0, stage, 1, stage ^ 1, PART);
+      multiply(1, stage, 2, stage ^ 1, 2 * PART);
+      multiply(2, stage, 3, stage ^ 1, -1);
+      wait_loads<0>();
+      lds_barrier();
+      multiply(3, stage ^ 1, 0, stage, 0);
+    }
+  }
+  wait_loads<0>();  // no fill may land after the workgroup has given its LDS back
+  float* out = a.out + static_cast<long long>(slice) * a.m_cols * a.n_cols;
+  const int row0 = m0 + wm + 4 * h + n % 4, column0 = n0 + wn + n / 4 * 4;
+#pragma unroll
+  for (int jm = 0; jm < JM; ++jm)
+#pragma unroll
+    for (int jn = 0; jn < JN; ++jn)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const floatx16& c = acc[jm][jn];
+        const float4 v = quad_transpose(make_float4(c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]));
+        const int row = row0 + 32 * jm + 8 * q, column = column0 + 32 * jn;
+        if (row < a.m_cols && column < a.n_cols)
+          *reinterpret_cast<float4*>(out + static_cast<long long>(row) * a.n_cols + column) = v;
+      }
+}
+
+// The ends of both weight gradients in one launch: the first blocks add the slices of the
+// matrix gradient (ascending), four elements a thread, the rest the partitions of the
+// bias gradient.
+template <bool ALIGNED>
+__global__ void __launch_bounds__(256)
+sum_partials_kernel(const float* slices, long long elements, int count, float* d_matrix, int matrix_blocks,
+                    const float* partitions, int parts, int width, float* d_bias) {
+  if (static_cast<int>(blockIdx.x) >= matrix_blocks) {
+    const int c = (blockIdx.x - matrix_blocks) * 256 + threadIdx.x;
+    if (c >= width) return;
+    float sum = 0.0f;
+#pragma unroll 16
+    for (int p = 0; p < parts; ++p) sum += partitions[static_cast<long long>(p) * width + c];
+    d_bias[c] = sum;
+    return;
+  }
+  const long long i = 4 * (blockIdx.x * 256LL + threadIdx.x);
+  if (i >= elements) return;  // widths are multiples of 64
+  float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 4
+  for (int s = 0; s < count; ++s) {
+    const float4 v = *reinterpret_cast<const float4*>(slices + s * elements + i);
+    sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
+  }
+  if constexpr (ALIGNED)
+    *reinterpret_cast<float4*>(d_matrix + i) = sum;
+  else
+    d_matrix[i] = sum.x, d_matrix[i + 1] = sum.y, d_matrix[i + 2] = sum.z, d_matrix[i + 3] = sum.w;
 }
 
 // Column sums of [rows, width] in two levels with a fixed order
@@ -343,14 +676,24 @@ sum_slices_kernel(const float* partial, long long elements, int slices, float* o
 // optionally the 16-bit copy of the same values: the gradient is read once
 // for both.  A workgroup takes 64 columns of a 256-row partition; thread
 // (lane, quad) = (tid / 16, tid % 16) adds rows lane, lane + 16, ... of four
-// adjacent columns, and the sixteen lanes' sums are added in ascending order.
+// adjacent columns, and the sixteen lanes' sums are added in ascending order.  The
+// blocks beyond `tiles` make the 16-bit copies of the matrix and of the input.
 template <bool HALF>
 __global__ void __launch_bounds__(256)
-column_partial_kernel(const float* in, int rows, int width, float* partial, uint16_t* copy) {
+column_partial_kernel(const float* in, int rows, int width, float* partial, uint16_t* copy, int tiles,
+                      const float* matrix, long long matrix_elements, uint16_t* matrix16,
+                      const float* input, long long input_elements, uint16_t* input16) {
+  if (static_cast<int>(blockIdx.x) >= tiles) {
+    const long long index = (blockIdx.x - tiles) * 256LL + threadIdx.x, threads = (gridDim.x - tiles) * 256LL;
+    convert_elements<HALF>(matrix, matrix_elements, matrix16, index, threads);
+    convert_elements<HALF>(input, input_elements, input16, index, threads);
+    return;
+  }
   __shared__ float lanes[16][64];
   const int quad = threadIdx.x % 16, lane = threadIdx.x / 16;
-  const int c = blockIdx.x * 64 + quad * 4;
-  const int r0 = blockIdx.y * kBiasRows, r1 = min(r0 + kBiasRows, rows);
+  const int across = (width + 63) / 64, column_block = blockIdx.x % across, part = blockIdx.x / across;
+  const int c = column_block * 64 + quad * 4;
+  const int r0 = part * kBiasRows, r1 = min(r0 + kBiasRows, rows);
   float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   if (width % 4 == 0 && c < width) {
 #pragma unroll 4
@@ -376,22 +719,12 @@ column_partial_kernel(const float* in, int rows, int width, float* partial, uint
   }
   for (int e = 0; e < 4; ++e) lanes[lane][quad * 4 + e] = sum[e];
   __syncthreads();
-  const int column = blockIdx.x * 64 + threadIdx.x;
+  const int column = column_block * 64 + threadIdx.x;
   if (threadIdx.x < 64 && column < width) {
     float total = lanes[0][threadIdx.x];
     for (int l = 1; l < 16; ++l) total += lanes[l][threadIdx.x];
-    partial[static_cast<long long>(blockIdx.y) * width + column] = total;
+    partial[static_cast<long long>(part) * width + column] = total;
   }
-}
-
-__global__ void __launch_bounds__(256)
-column_final_kernel(const float* partial, int parts, int width, float* out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= width) return;
-  float sum = 0.0f;
-#pragma unroll 16
-  for (int p = 0; p < parts; ++p) sum += partial[static_cast<long long>(p) * width + c];
-  out[c] = sum;
 }
 
 // Any shape: one thread per output element, operands rounded like the matrix
@@ -442,13 +775,27 @@ bool matrix_cores(int input_dim, int output_dim) {
   return input_dim % 64 == 0 && output_dim % 64 == 0;
 }
 
-int weight_slices(int rows, int input_dim, int output_dim) {
-  const long long tiles = ((input_dim + 127) / 128) * static_cast<long long>((output_dim + 127) / 128);
-  // two workgroups a compute unit: as many slices as still run in one round
-  long long slices = 512 / tiles;
-  const long long most = (rows + 255) / 256;     // at least 256 rows a slice
-  if (slices > most) slices = most;
-  return static_cast<int>(slices < 1 ? 1 : slices);
+// How the matrix gradient is computed: the kind of tiles and the slices of the rows, as
+// many as fill the compute units once (one wide tile each or two of 128 x 128) but of
+// at least 256 rows, whose partial sums are written and read again at about 5 TB/s.
+struct WeightPlan {
+  bool wide = false;
+  int slices = 1;
+};
+WeightPlan weight_plan(int rows, int input_dim, int output_dim) {
+  constexpr Tile kWide = {256, 192, 115, 130}, kSquare = {128, 128, 75, 60};
+  auto plan = [&](const Tile& t, int resident, long long* time) {
+    const long long tiles = 1LL * ((input_dim + t.rows - 1) / t.rows) * ((output_dim + t.columns - 1) / t.columns);
+    const long long slices =
+        std::max(1LL, std::min<long long>(resident / tiles, (rows + 255) / 256));
+    const int steps = static_cast<int>(((rows + slices - 1) / slices + 63) / 64);
+    *time = product_time(t, input_dim, output_dim, static_cast<int>(slices), steps) +
+            (slices > 1 ? 8LL * slices * input_dim * output_dim / 50000 : 0);
+    return static_cast<int>(slices);
+  };
+  long long wide_time = 0, square_time = 0;
+  const int wide = plan(kWide, 256, &wide_time), square = plan(kSquare, 512, &square_time);
+  return wide_time <= square_time ? WeightPlan{true, wide} : WeightPlan{false, square};
 }
 
 struct Layout {
@@ -467,19 +814,10 @@ Layout layout(int dtype, int rows, int input_dim, int output_dim) {
   l.matrix16 = take(in * out * 2);
   l.input16 = take(dtype == PLUTO_HIP_F32 ? r * in * 2 : 0);
   l.gradient16 = take(r * out * 2);
-  l.partial = take(static_cast<size_t>(weight_slices(rows, input_dim, output_dim)) * in * out * 4);
+  l.partial = take(static_cast<size_t>(weight_plan(rows, input_dim, output_dim).slices) * in * out * 4);
   l.bias_partial = take(static_cast<size_t>((rows + kBiasRows - 1) / kBiasRows) * out * 4);
   l.total = at;
   return l;
-}
-
-template <bool HALF, bool TRANSPOSE>
-void convert(hipStream_t s, const float* in, long long rows, int cols, uint16_t* out) {
-  if constexpr (TRANSPOSE)
-    convert_kernel<HALF, true><<<dim3((cols + 31) / 32, static_cast<unsigned>((rows + 31) / 32)),
-                                 256, 0, s>>>(in, rows, cols, out);
-  else
-    convert_kernel<HALF, false><<<blocks_for(rows * cols, 8192), 256, 0, s>>>(in, rows, cols, out);
 }
 
 template <bool HALF>
@@ -492,13 +830,13 @@ int forward(hipStream_t s, int dtype, const void* input, const float* matrix, co
   }
   const Layout l = layout(dtype, rows, input_dim, output_dim);
   uint16_t* matrix16 = reinterpret_cast<uint16_t*>(scratch + l.matrix16);  // w^T [out, in]
-  convert<HALF, true>(s, matrix, input_dim, output_dim, matrix16);
-  const uint16_t* input16 = static_cast<const uint16_t*>(input);
-  if (dtype == PLUTO_HIP_F32) {
-    uint16_t* copy = reinterpret_cast<uint16_t*>(scratch + l.input16);
-    convert<HALF, false>(s, static_cast<const float*>(input), rows, input_dim, copy);
-    input16 = copy;
-  }
+  const bool copied = dtype == PLUTO_HIP_F32;
+  uint16_t* copy = reinterpret_cast<uint16_t*>(scratch + l.input16);
+  const uint16_t* input16 = copied ? copy : static_cast<const uint16_t*>(input);
+  const int tiles = ((input_dim + 31) / 32) * ((output_dim + 31) / 32);
+  const long long elements = copied ? 1LL * rows * input_dim : 0;
+  convert_forward_kernel<HALF><<<tiles + (copied ? blocks_for(elements / 8, 2048) : 0), 256, 0, s>>>(
+      matrix, input_dim, output_dim, matrix16, tiles, static_cast<const float*>(input), elements, copy);
   ProductArgs p;
   p.left = input16;
   p.right = matrix16;
@@ -522,25 +860,28 @@ int backward(hipStream_t s, int dtype, const void* input, const float* matrix,
   const int parts = (rows + kBiasRows - 1) / kBiasRows;
   const bool cores = matrix_cores(input_dim, output_dim);
   uint16_t* gradient16 = reinterpret_cast<uint16_t*>(scratch + l.gradient16);  // dy [rows, out]
-  column_partial_kernel<HALF><<<dim3((output_dim + 63) / 64, parts), 256, 0, s>>>(
-      d_output, rows, output_dim, bias_partial, cores ? gradient16 : nullptr);
-  column_final_kernel<<<(output_dim + 63) / 64, 64, 0, s>>>(bias_partial, parts, output_dim,
-                                                            d_bias);
+  uint16_t* matrix16 = reinterpret_cast<uint16_t*>(scratch + l.matrix16);  // w [in, out]
+  const bool copied = cores && dtype == PLUTO_HIP_F32;
+  uint16_t* copy = reinterpret_cast<uint16_t*>(scratch + l.input16);
+  const long long elements = 1LL * input_dim * output_dim;
+  const long long matrix_elements = cores ? elements : 0, input_elements = copied ? 1LL * rows * input_dim : 0;
+  const int tiles = (output_dim + 63) / 64 * parts;
+  const long long converted = matrix_elements + input_elements;
+  column_partial_kernel<HALF>
+      <<<tiles + (converted > 0 ? blocks_for(converted / 8, 2048) : 0), 256, 0, s>>>(
+          d_output, rows, output_dim, bias_partial, cores ? gradient16 : nullptr, tiles, matrix, matrix_elements,
+          matrix16, static_cast<const float*>(input), input_elements, copy);
+  const int bias_blocks = (output_dim + 255) / 256;
   if (!cores) {
+    sum_partials_kernel<false><<<bias_blocks, 256, 0, s>>>(nullptr, 0, 0, nullptr, 0, bias_partial, parts,
+                                                           output_dim, d_bias);
     generic_dense_kernel<HALF><<<blocks_for(1LL * rows * input_dim), 256, 0, s>>>(
         1, dtype, input, matrix, d_output, nullptr, rows, input_dim, output_dim, d_input);
-    generic_dense_kernel<HALF><<<blocks_for(1LL * input_dim * output_dim), 256, 0, s>>>(
+    generic_dense_kernel<HALF><<<blocks_for(elements), 256, 0, s>>>(
         2, dtype, input, matrix, d_output, nullptr, rows, input_dim, output_dim, d_matrix);
     return launch_status();
   }
-  uint16_t* matrix16 = reinterpret_cast<uint16_t*>(scratch + l.matrix16);      // w [in, out]
-  convert<HALF, false>(s, matrix, input_dim, output_dim, matrix16);
-  const uint16_t* input16 = static_cast<const uint16_t*>(input);
-  if (dtype == PLUTO_HIP_F32) {
-    uint16_t* copy = reinterpret_cast<uint16_t*>(scratch + l.input16);
-    convert<HALF, false>(s, static_cast<const float*>(input), rows, input_dim, copy);
-    input16 = copy;
-  }
+  const uint16_t* input16 = copied ? copy : static_cast<const uint16_t*>(input);
   // dx[r, i] = sum_o dy[r, o] w[i, o]
   ProductArgs p;
   p.left = gradient16;
@@ -559,15 +900,27 @@ int backward(hipStream_t s, int dtype, const void* input, const float* matrix,
   g.rows = rows;
   g.m_cols = input_dim;
   g.n_cols = output_dim;
-  g.slices = weight_slices(rows, input_dim, output_dim);
+  const WeightPlan plan = weight_plan(rows, input_dim, output_dim);
+  g.slices = plan.slices;
   g.out = g.slices == 1 ? d_matrix : reinterpret_cast<float*>(scratch + l.partial);
-  const unsigned tiles = static_cast<unsigned>((input_dim + 127) / 128) *
-                         static_cast<unsigned>((output_dim + 127) / 128);
-  product_columns_kernel<HALF><<<tiles * g.slices, kThreads, 0, s>>>(g);
+  auto weight_tiles = [&](int m, int n) {
+    return static_cast<unsigned>((input_dim + m - 1) / m) * static_cast<unsigned>((output_dim + n - 1) / n);
+  };
+  const bool aligned = reinterpret_cast<uintptr_t>(d_matrix) % 16 == 0;
+  if (plan.wide && (aligned || g.slices > 1))
+    product_columns_wide_kernel<HALF, 4, 3><<<weight_tiles(256, 192) * g.slices, 256, 0, s>>>(g);
+  else
+    product_columns_kernel<HALF><<<weight_tiles(128, 128) * g.slices, kThreads, 0, s>>>(g);
   status = launch_status();
-  if (status != 0 || g.slices == 1) return status;
-  const long long elements = 1LL * input_dim * output_dim;
-  sum_slices_kernel<<<blocks_for(elements), 256, 0, s>>>(g.out, elements, g.slices, d_matrix);
+  if (status != 0) return status;
+  const int matrix_blocks = g.slices == 1 ? 0 : static_cast<int>((elements / 4 + 255) / 256);
+  const unsigned blocks = matrix_blocks + bias_blocks;
+  if (aligned)
+    sum_partials_kernel<true><<<blocks, 256, 0, s>>>(g.out, elements, g.slices, d_matrix, matrix_blocks,
+                                                     bias_partial, parts, output_dim, d_bias);
+  else
+    sum_partials_kernel<false><<<blocks, 256, 0, s>>>(g.out, elements, g.slices, d_matrix, matrix_blocks,
+                                                      bias_partial, parts, output_dim, d_bias);
   return launch_status();
 }
 

@@ -146,27 +146,6 @@ __device__ inline floatx4 mma16(floatx4 acc, float4 a, floatx4 b) {
   return mma16(acc, a, make_float4(b[0], b[1], b[2], b[3]));
 }
 
-// Lanes 4 i .. 4 i + 3 hold the rows of a 4 x 4 matrix; afterwards its columns.
-__device__ inline float4 quad_transpose(float4 v) {
-  auto swap = [](float& low, float& high, bool upper, auto exchange) {
-    const float other = exchange(upper ? low : high);
-    low = upper ? other : low;
-    high = upper ? high : other;
-  };
-  auto with_1 = [](float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));
-  };
-  auto with_2 = [](float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xf, 0xf, true));
-  };
-  const bool odd = threadIdx.x & 1, second = threadIdx.x & 2;
-  swap(v.x, v.y, odd, with_1);
-  swap(v.z, v.w, odd, with_1);
-  swap(v.x, v.z, second, with_2);
-  swap(v.y, v.w, second, with_2);
-  return v;
-}
-
 // One product of several tiles with the same left operand: their chains take turns.
 template <int TILES, class F>
 __device__ inline void mma16_tiles(floatx4 (&acc)[TILES], float4 a, F right) {

@@ -113,10 +113,8 @@ __device__ inline int32x4 make_rsrc(const void* base, uint32_t bytes) {
 // issued (the base is read at issue): whatever the compiler keeps in M0
 // survives.
 template <int BYTES>
-__device__ inline void lds_fill(int32x4 descriptor, const void* lds, uint32_t offset) {
+__device__ inline void lds_fill_at(int32x4 descriptor, uint32_t address, uint32_t offset) {
   static_assert(BYTES == 16 || BYTES == 4);
-  const uint32_t address = __builtin_amdgcn_readfirstlane(
-      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds)));
   uint32_t saved_m0;
   if constexpr (BYTES == 16)
     asm volatile(
@@ -132,6 +130,15 @@ __device__ inline void lds_fill(int32x4 descriptor, const void* lds, uint32_t of
         : "=&s"(saved_m0)
         : "s"(address), "v"(offset), "s"(descriptor)
         : "memory");
+}
+// The address of a place in LDS, uniform, as lds_fill_at takes it.
+__device__ inline uint32_t lds_address(const void* lds) {
+  return __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lds)));
+}
+template <int BYTES>
+__device__ inline void lds_fill(int32x4 descriptor, const void* lds, uint32_t offset) {
+  lds_fill_at<BYTES>(descriptor, lds_address(lds), offset);
 }
 
 // LDS transpose read (ds_read_b64_tr_b16).  Within every group of 16 lanes,
@@ -169,6 +176,27 @@ __device__ inline float half_swap_sum(float v) {
   float lower, upper;
   half_swap(v, lower, upper);
   return lower + upper;
+}
+
+// Lanes 4 i .. 4 i + 3 hold the rows of a 4 x 4 matrix; afterwards its columns.
+__device__ inline float4 quad_transpose(float4 v) {
+  auto swap = [](float& low, float& high, bool upper, auto exchange) {
+    const float other = exchange(upper ? low : high);
+    low = upper ? other : low;
+    high = upper ? high : other;
+  };
+  auto with_1 = [](float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, true));
+  };
+  auto with_2 = [](float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xf, 0xf, true));
+  };
+  const bool odd = threadIdx.x & 1, second = threadIdx.x & 2;
+  swap(v.x, v.y, odd, with_1);
+  swap(v.z, v.w, odd, with_1);
+  swap(v.x, v.z, second, with_2);
+  swap(v.y, v.w, second, with_2);
+  return v;
 }
 
 // Row-major bf16 tile [rows][D] in LDS whose 16-byte chunk c of row r sits at

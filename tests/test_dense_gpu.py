@@ -103,6 +103,40 @@ def test_bench_shape_matches_float64_products(capi, oracle):
     close(db, dy.double().sum(0), 1e-5, "db")
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("shape", [(9000, 832, 2176), (8170, 128, 768), (9000, 64, 192)])
+def test_large_tiles_match_products_of_the_rounded_operands(capi, dtype, shape):
+    # The products pick their tiles by size: the first shape takes 256 x 192 ones in all
+    # three products (ragged in every direction), the second 64 x 128 ones forward, the
+    # third one 64-element step.  Against FP32 products of the 16-bit operands; an output
+    # address that is not a multiple of 16 bytes takes the other tiles.
+    rows, n_in, n_out = shape
+    torch.manual_seed(sum(shape))
+    x = torch.randn(rows, n_in, device="cuda")
+    w = torch.randn(n_in, n_out, device="cuda") / n_in ** 0.5
+    b = torch.randn(n_out, device="cuda")
+    dy = torch.randn(rows, n_out, device="cuda")
+    half = torch.bfloat16 if dtype == "bf16" else torch.float16
+    x = x.to(half).float()
+    tx = x.to(torch.bfloat16) if dtype == "bf16" else x
+    w16, dy16 = w.to(half).float(), dy.to(half).float()
+    y = capi.dense_forward(tx, w, b)
+    dx, dw, db = capi.dense_backward(tx, w, dy)
+    storage = torch.empty(rows * n_out + 2, dtype=y.dtype, device="cuda")
+    shifted = capi.dense_forward(tx, w, b, out=storage[2:].view(rows, n_out))
+    torch.cuda.synchronize()
+
+    def check(got, want, tolerance, what):
+        error = (got.double() - want.double()).norm() / want.double().norm()
+        assert error < tolerance, "%s: relative error %.2e" % (what, error)
+
+    check(y, x @ w16 + b, 3e-3 if dtype == "bf16" else 2e-6, "y")
+    check(dx, dy16 @ w16.t().contiguous(), 2e-6, "dx")
+    check(dw, x.t().contiguous() @ dy16, 2e-6, "dw")
+    check(db, dy.sum(0, dtype=torch.float64), 2e-6, "db")
+    check(shifted, y, 2e-3 if dtype == "bf16" else 2e-6, "y at a shifted address")
+
+
 def test_gradients_are_overwritten_and_repeatable(capi, oracle):
     rows, n_in, n_out = 700, 128, 192
     x, w, b, dy = case(oracle, "bf16", rows, n_in, n_out, seed=1)
