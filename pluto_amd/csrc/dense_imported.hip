@@ -53,6 +53,10 @@ struct GroupQuantizer {
     const float corrected = __builtin_fmaf(__builtin_fmaf(-q, divisor, v), inverse, q);
     return fminf(fmaxf(corrected, -448.0f), 448.0f);
   }
+  // The FP8 code of the value nearest to the quotient.
+  __device__ int code(float v) const {
+    return __builtin_amdgcn_cvt_pk_fp8_f32(quotient(v), 0.0f, 0, false) & 0xff;
+  }
   // The FP8 values (unscaled) nearest to the two quotients, as floats.
   __device__ void round(float first, float second, float& a, float& b) const {
     const int codes = __builtin_amdgcn_cvt_pk_fp8_f32(quotient(first), quotient(second), 0, false);
@@ -340,59 +344,54 @@ __global__ void __launch_bounds__(256) imported_matvec_ragged_kernel(MatVecArgs 
 }
 
 // ---- more than eight tokens: the matrix cores --------------------------------
-// out[t, r] = sum_k w[r, k] x[t, k] as a 32-row x 32-token tile per wave on
-// v_mfma_f32_32x32x16_bf16.  bf16 weights and tokens are exact operands.  FP8
-// codes are exact in bf16 too, so FP8 weights are multiplied unscaled with the
-// FP8 values of the quantized tokens, and each block of 128 contraction
-// elements is scaled once by (weight block scale) x (token group scale):
-// the same products as (w s_w)(x s_x), summed in FP32 in a different order.
-// Lane (n, h) covers elements [64 h, 64 h + 64) of a 128-element block, for
-// weight row n (A operand) and for token n (B operand).  The eight waves of a
-// workgroup share a tile and take every eighth block; their partial tiles are
-// added in wave order through LDS.
+// out[t, r] = sum_k w[r, k] x[t, k], 32 rows x 32 tokens a tile.  bf16 weights and
+// tokens are exact operands of v_mfma_f32_32x32x16_bf16.  FP8 codes are exact in bf16
+// too, so FP8 weights are multiplied unscaled with the FP8 values of the quantized
+// tokens on v_mfma_f32_16x16x32_bf16, and each block of 128 contraction elements is
+// scaled once by (weight block scale) x (token group scale): the same products as (w
+// s_w)(x s_x), summed in FP32 in a different order.  (v_mfma_f32_16x16x32_fp8_fp8 would
+// take the codes as they are, but sums with fewer bits: 0.1 % of the results of 1024
+// columns were more than a bf16 rounding off.)  The eight waves of a workgroup share a
+// tile and take every eighth block; their partial tiles are added in wave order
+// through LDS.
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float floatx4;
 typedef __attribute__((ext_vector_type(16))) float floatx16;
 
-// Tokens as FP8 values in bf16 and their group scales [tokens, n / 128].  The
-// values are written in the order the matrix-core kernel reads them, so that
-// each of its loads is one contiguous KiB: [pass of 32 tokens][block of 128
-// columns][step j][lane = token % 32 + 32 h][8], the lane's elements being
-// columns 128 block + 64 h + 8 j .. + 7.
+// Tokens as FP8 codes and their group scales [tokens, n / 128].  The codes are written
+// in the order the matrix-core kernel reads them, so that each of its loads is one
+// contiguous KiB: [pass of 32 tokens][block of 128 columns][half of the block][half of
+// the tokens][lane = token % 16 + 16 q][16], the lane's elements being columns 128
+// block + 64 half + 16 q .. + 15.
 __global__ void __launch_bounds__(kGroup)
-imported_token_fp8_kernel(const uint16_t* x, int n, uint16_t* values, float* scales) {
+imported_token_fp8_kernel(const uint16_t* x, int n, unsigned char* codes, float* scales) {
   __shared__ float largest[2];
   const int token = blockIdx.y, block = blockIdx.x, c = threadIdx.x;
   x += static_cast<size_t>(token) * n;
-  const int i = block * kGroup + c;
-  const float v = i < n ? bf16_bits_to_float(x[i]) : 0.0f;
+  const float v = bf16_bits_to_float(x[block * kGroup + c]);  // n is a multiple of 128
   const float mine = wave_max(fabsf(v));
   if (threadIdx.x % 64 == 0) largest[threadIdx.x / 64] = mine;
   __syncthreads();
   const GroupQuantizer quantizer(fmaxf(largest[0], largest[1]));
-  float value, unused;
-  quantizer.round(v, 0.0f, value, unused);
-  const size_t pass = token / 32;
-  const int lane = token % 32 + 32 * (c / 64), step = (c % 64) / 8;
-  if (i < n)
-    values[(((pass * gridDim.x + block) * 8 + step) * 64 + lane) * 8 + c % 8] =
-        float_to_bf16_bits(value);
+  const size_t piece = ((static_cast<size_t>(token / 32) * gridDim.x + block) * 2 + c / 64) * 2 + token % 32 / 16;
+  codes[(piece * 64 + token % 16 + c % 64 / 16 * 16) * 16 + c % 16] =
+      static_cast<unsigned char>(quantizer.code(v));
   if (threadIdx.x == 0) scales[static_cast<size_t>(token) * gridDim.x + block] = quantizer.scale;
 }
 
-struct TileArgs {
-  const void* weights = nullptr;
-  const float* weight_scales = nullptr;  // FP8 only
-  const uint16_t* tokens = nullptr;      // bf16 [count, cols]; FP8: one pass in operand order
-  const float* token_scales = nullptr;   // FP8 only: [count, cols / 128]
-  uint16_t* out = nullptr;               // [count, rows]
-  int cols = 0, rows = 0, count = 0;     // count <= 32
-};
-
-template <bool HIGH>
-__device__ inline uint32_t fp8_pair_to_bf16(uint32_t word) {
-  const floatx2 v = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(word), HIGH);
-  return (__float_as_uint(v.y) & 0xffff0000u) | (__float_as_uint(v.x) >> 16);
+// Eight FP8 codes (the lower or the upper eight of sixteen) as bf16, exactly.
+__device__ inline bf16x8 fp8_to_bf16(const uint4& codes, int part) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  const uint32_t word[2] = {part == 0 ? codes.x : codes.z, part == 0 ? codes.y : codes.w};
+  bf16x8 out;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bf16x2 low = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word[i], 1.0f, false);
+    const bf16x2 high = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word[i], 1.0f, true);
+    out[4 * i] = low[0], out[4 * i + 1] = low[1], out[4 * i + 2] = high[0], out[4 * i + 3] = high[1];
+  }
+  return out;
 }
 
 constexpr int kTileWaves = 8;  // waves that split a tile's contraction
@@ -405,97 +404,51 @@ struct TileManyArgs {
   int rows[kManyMax];
   int first_block[kManyMax + 1];
   int matrices = 0;
-  const uint16_t* tokens = nullptr;
-  const float* token_scales = nullptr;
-  int cols = 0, count = 0;
+  const void* tokens = nullptr;         // bf16 [count, cols]; FP8: one pass in operand order
+  const float* token_scales = nullptr;  // FP8 only: [count, cols / 128]
+  int cols = 0, count = 0;              // count <= 32
 };
 
-// One tile: 32 rows of the matrix times up to 32 tokens, the contraction split
-// over the workgroup's waves.  AHEAD (FP8 only): blocks of a wave whose weight
-// loads are issued together.
-template <bool FP8, int AHEAD>
-__device__ __forceinline__ void imported_tile(const TileArgs& a, int tile,
-                                              float (*partial)[16][64]) {
+// The matrix of a tile and its first row there.
+struct TilePlace {
+  int which, row;
+};
+template <int ROWS>
+__device__ inline TilePlace tile_place(const TileManyArgs& m, int tile) {
+  int which = 0;
+  while (which + 1 < m.matrices && tile >= m.first_block[which + 1]) ++which;
+  return {which, (tile - m.first_block[which]) * ROWS};
+}
+
+// bf16: one tile a workgroup.  Lane (n, h) covers elements [64 h, 64 h + 64) of a
+// 128-element block, for weight row n (A operand) and for token n (B operand).
+__global__ void __launch_bounds__(64 * kTileWaves)
+imported_tile_kernel(TileManyArgs m) {
+  __shared__ float partial[kTileWaves - 1][16][64];
+  const TilePlace place = tile_place<32>(m, blockIdx.x);
+  const int rows = m.rows[place.which];
   const int lane = threadIdx.x % 64, n = lane % 32, h = lane / 32;
   const int wave = threadIdx.x / 64;
-  const int row_base = tile * 32;
-  const int row = min(row_base + n, a.rows - 1);   // rows and tokens past the end repeat
-  const int token = min(n, a.count - 1);           // the last one and are not stored
-  const int groups = a.cols / kGroup;
-  const unsigned char* w = static_cast<const unsigned char*>(a.weights) +
-                           (static_cast<size_t>(row) * a.cols + 64 * h) * (FP8 ? 1 : 2);
-  // FP8: operand order, 1 KiB a step; otherwise the token's own row
-  const uint16_t* x = FP8 ? a.tokens + lane * 8 : a.tokens + static_cast<size_t>(token) * a.cols + 64 * h;
-  const float* block_scale =
-      FP8 ? a.weight_scales + static_cast<size_t>(row_base / kGroup) * groups : nullptr;
-  const float* group_scale = FP8 ? a.token_scales + static_cast<size_t>(token) * groups : nullptr;
+  const int row = min(place.row + n, rows - 1);   // rows and tokens past the end repeat
+  const int token = min(n, m.count - 1);          // the last one and are not stored
+  const int groups = m.cols / kGroup;
+  const unsigned char* w = static_cast<const unsigned char*>(m.weights[place.which]) +
+                           (static_cast<size_t>(row) * m.cols + 64 * h) * 2;
+  const uint16_t* x = static_cast<const uint16_t*>(m.tokens) + static_cast<size_t>(token) * m.cols + 64 * h;
   floatx16 total;
 #pragma unroll
   for (int i = 0; i < 16; ++i) total[i] = 0.0f;
-  if constexpr (FP8) {
-    // A wave's weight rows are few bytes (64 a lane and block): the loads of
-    // AHEAD of its blocks (all of them for widths up to 8192) are issued before
-    // anything is waited for, so that the latency of HBM is paid once a batch
-    // and not once a block; the tokens (L2 hits) follow one block ahead of the
-    // products.  Blocks past the end repeat the last one (loads without
-    // branches) and are not added.
-    constexpr int kAhead = AHEAD;
-    for (int g0 = wave; g0 < groups; g0 += kTileWaves * kAhead) {
-      uint4 raw[kAhead][4];
+  for (int g = wave; g < groups; g += kTileWaves) {
+    uint4 xs[8];
 #pragma unroll
-      for (int b = 0; b < kAhead; ++b) {
-        const int g = min(g0 + b * kTileWaves, groups - 1);
+    for (int j = 0; j < 8; ++j) xs[j] = *reinterpret_cast<const uint4*>(x + g * kGroup + 8 * j);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          raw[b][j] = *reinterpret_cast<const uint4*>(w + static_cast<size_t>(g) * kGroup + 16 * j);
-      }
-      uint4 xs[2][8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        xs[0][j] = *reinterpret_cast<const uint4*>(x + (static_cast<size_t>(g0) * 8 + j) * 512);
-#pragma unroll
-      for (int b = 0; b < kAhead; ++b) {
-        const int g = g0 + b * kTileWaves;
-        if (b + 1 < kAhead) {
-          const int next = min(g + kTileWaves, groups - 1);
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            xs[(b + 1) % 2][j] =
-                *reinterpret_cast<const uint4*>(x + (static_cast<size_t>(next) * 8 + j) * 512);
-        }
-        floatx16 acc;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t lo = j % 2 == 0 ? raw[b][j / 2].x : raw[b][j / 2].z;
-          const uint32_t hi = j % 2 == 0 ? raw[b][j / 2].y : raw[b][j / 2].w;
-          const uint4 bits = make_uint4(fp8_pair_to_bf16<false>(lo), fp8_pair_to_bf16<true>(lo),
-                                        fp8_pair_to_bf16<false>(hi), fp8_pair_to_bf16<true>(hi));
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bits),
-                                                        __builtin_bit_cast(bf16x8, xs[b % 2][j]),
-                                                        acc, 0, 0, 0);
-        }
-        // a block past the end contributes nothing (its scale is read in range)
-        const int in_range = min(g, groups - 1);
-        const float scale = g < groups ? block_scale[in_range] * group_scale[in_range] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) total[i] += acc[i] * scale;
-      }
-    }
-  } else {
-    for (int g = wave; g < groups; g += kTileWaves) {
-      uint4 xs[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) xs[j] = *reinterpret_cast<const uint4*>(x + g * kGroup + 8 * j);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint4 bits =
-            *reinterpret_cast<const uint4*>(w + (static_cast<size_t>(g) * kGroup + 8 * j) * 2);
-        total = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bits),
-                                                        __builtin_bit_cast(bf16x8, xs[j]), total,
-                                                        0, 0, 0);
-      }
+    for (int j = 0; j < 8; ++j) {
+      const uint4 bits =
+          *reinterpret_cast<const uint4*>(w + (static_cast<size_t>(g) * kGroup + 8 * j) * 2);
+      total = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bits),
+                                                      __builtin_bit_cast(bf16x8, xs[j]), total,
+                                                      0, 0, 0);
     }
   }
   if (wave > 0) {
@@ -509,48 +462,190 @@ __device__ __forceinline__ void imported_tile(const TileArgs& a, int tile,
 #pragma unroll
     for (int w = 0; w < kTileWaves - 1; ++w) total[i] += partial[w][i][lane];
   // accumulator element 4 q + i = (row 8 q + 4 h + i, token n)
-  if (n >= a.count) return;
+  if (n >= m.count) return;
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = row_base + 8 * q + 4 * h + i;
-      if (r < a.rows)
-        a.out[static_cast<size_t>(n) * a.rows + r] = float_to_bf16_bits(total[4 * q + i]);
+      const int r = place.row + 8 * q + 4 * h + i;
+      if (r < rows)
+        m.out[place.which][static_cast<size_t>(n) * rows + r] = float_to_bf16_bits(total[4 * q + i]);
     }
 }
 
-template <bool FP8, int AHEAD = 1>
-__global__ void __launch_bounds__(64 * kTileWaves) imported_tile_kernel(TileManyArgs m) {
-  __shared__ float partial[kTileWaves - 1][16][64];
-  int which = 0;
-  while (which + 1 < m.matrices && static_cast<int>(blockIdx.x) >= m.first_block[which + 1])
-    ++which;
-  TileArgs a;
-  a.weights = m.weights[which];
-  a.weight_scales = m.weight_scales[which];
-  a.tokens = m.tokens;
-  a.token_scales = m.token_scales;
-  a.out = m.out[which];
-  a.cols = m.cols;
-  a.rows = m.rows[which];
-  a.count = m.count;
-  imported_tile<FP8, AHEAD>(a, blockIdx.x - m.first_block[which], partial);
+// FP8: one workgroup a compute unit that walks over tiles.  A wave's blocks of the
+// contraction are the same in every tile: their tokens stay in registers, and each
+// block of weights is requested for the next tile as soon as its registers have been
+// multiplied, so that HBM never waits for a tile's products and sums (one tile a
+// workgroup, the compute units went idle between 516 tiles of 5120 columns: 37 us
+// against 25).  BLOCKS: a wave's blocks, as many as its registers hold; wider matrices
+// take several passes a tile, for each of which the tokens are loaded again.  Lane (q,
+// n16) covers elements 16 q .. + 15 of each half block of weight row n16 of each of
+// PARTS 16-row parts (A operands) and of tokens n16 and 16 + n16 (B operands).
+template <int BLOCKS, int PARTS, bool ONE_PASS>
+__global__ void __launch_bounds__(64 * kTileWaves)
+imported_tile_fp8_kernel(TileManyArgs m, int passes) {
+  if constexpr (ONE_PASS) passes = 1;
+  __shared__ float partial[2][kTileWaves][8 * PARTS][64];
+  const int lane = threadIdx.x % 64, n = lane % 16, q = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int groups = m.cols / kGroup, tiles = m.first_block[m.matrices];
+  auto block_of = [&](int pass, int b) { return wave + kTileWaves * (pass * BLOCKS + b); };
+  const uint32_t lane_at = static_cast<uint32_t>(n) * m.cols + 16 * q;
+  uint4 raw[BLOCKS][2][PARTS], x[BLOCKS][2][2];  // [block][half][rows or tokens]
+  float group_scale[BLOCKS][2];
+  // rows past the end read zeros
+  auto request = [&](const __amdgpu_buffer_rsrc_t& rows, int pass, int b) {
+    const uint32_t at = min(block_of(pass, b), groups - 1) * kGroup;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int t = 0; t < PARTS; ++t)
+        raw[b][half][t] = __builtin_bit_cast(
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, lane_at + 16 * t * m.cols, at + 64 * half, 0));
+  };
+  auto rows_of = [&](int tile) {
+    const TilePlace place = tile_place<16 * PARTS>(m, tile);
+    const size_t first = static_cast<size_t>(place.row) * m.cols;
+    const int rows = min(16 * PARTS, m.rows[place.which] - place.row);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<unsigned char*>(static_cast<const unsigned char*>(m.weights[place.which]) + first), 0,
+        rows * m.cols, 0x00020000);
+  };
+  auto load_tokens = [&](int pass) {
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) {
+      const int g = min(block_of(pass, b), groups - 1);
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          x[b][half][t] = static_cast<const uint4*>(m.tokens)[((g * 2 + half) * 2 + t) * 64 + lane];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)  // tokens past the end are not stored
+        group_scale[b][t] = m.token_scales[static_cast<size_t>(min(16 * t + n, m.count - 1)) * groups + g];
+    }
+  };
+  load_tokens(0);
+  {
+    const __amdgpu_buffer_rsrc_t rows = rows_of(blockIdx.x);
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) request(rows, 0, b);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  int buffer = 0;
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, buffer ^= 1) {
+    const TilePlace place = tile_place<16 * PARTS>(m, tile);
+    const int rows = m.rows[place.which];
+    const float* block_scale = m.weight_scales[place.which] + static_cast<size_t>(place.row / kGroup) * groups;
+    floatx4 total[PARTS][2];
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) total[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int pass = 0; pass < passes; ++pass) {
+      if (!ONE_PASS && (pass > 0 || tile != static_cast<int>(blockIdx.x))) load_tokens(pass);
+      const int next_pass = pass + 1 < passes ? pass + 1 : 0;
+      const int next_tile = next_pass > 0 ? tile : min(tile + static_cast<int>(gridDim.x), tiles - 1);
+      const __amdgpu_buffer_rsrc_t next_rows = rows_of(next_tile);
+#pragma unroll
+      for (int b = 0; b < BLOCKS; ++b) {
+        // a block past the end contributes nothing (its scale is read in range)
+        const int g = block_of(pass, b);
+        const float weight_scale = g < groups ? block_scale[min(g, groups - 1)] : 0.0f;
+        floatx4 acc[PARTS][2];
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        // the tokens are converted here for every tile: converted once they would take
+        // twice the registers, which the compiler does not see
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            asm volatile("" : "+v"(x[b][half][j].x), "+v"(x[b][half][j].y), "+v"(x[b][half][j].z),
+                              "+v"(x[b][half][j].w));
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int part = 0; part < 2; ++part) {
+            bf16x8 w[PARTS], t[2];
+#pragma unroll
+            for (int i = 0; i < PARTS; ++i) w[i] = fp8_to_bf16(raw[b][half][i], part);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) t[j] = fp8_to_bf16(x[b][half][j], part);
+#pragma unroll
+            for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], t[j], acc[i][j], 0, 0, 0);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+        request(next_rows, next_pass, b);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) total[i][j] += acc[i][j] * (weight_scale * group_scale[b][j]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8 * PARTS; ++i) partial[buffer][wave][i][lane] = total[i / 8][i / 4 % 2][i % 4];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // requests stay in flight
+    // every wave adds one or two of the elements: element e is rows 16 (e / 8) + 4 q + e % 4,
+    // tokens 16 (e / 4 % 2) + n
+#pragma unroll
+    for (int k = 0; k < PARTS; ++k) {
+      const int e = PARTS * wave + k;
+      float sum = partial[buffer][0][e][lane];
+#pragma unroll
+      for (int w = 1; w < kTileWaves; ++w) sum += partial[buffer][w][e][lane];
+      const int row = place.row + 16 * (e / 8) + 4 * q + e % 4, token = 16 * (e / 4 % 2) + n;
+      if (row < rows && token < m.count)
+        m.out[place.which][static_cast<size_t>(token) * rows + row] = float_to_bf16_bits(sum);
+    }
+  }
 }
 
-// Picks AHEAD = blocks a wave owns, up to eight.
-void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t, int blocks) {
-  const int groups = t.cols / kGroup;
-  auto launch = [&](auto kernel) { kernel<<<blocks, 64 * kTileWaves, 0, s>>>(t); };
-  switch (std::min(8, (groups + kTileWaves - 1) / kTileWaves)) {
-    case 1: return launch(imported_tile_kernel<true, 1>);
-    case 2: return launch(imported_tile_kernel<true, 2>);
-    case 3: return launch(imported_tile_kernel<true, 3>);
-    case 4: return launch(imported_tile_kernel<true, 4>);
-    case 5: return launch(imported_tile_kernel<true, 5>);
-    case 6: return launch(imported_tile_kernel<true, 6>);
-    case 7: return launch(imported_tile_kernel<true, 7>);
-    default: return launch(imported_tile_kernel<true, 8>);
+// Where every compute unit walks over several tiles they have 16 rows (shorter ends: 516 x
+// 32 rows of 5120 columns 27.4 us in tiles of 32 rows, 24.7 in tiles of 16).  Fewer have
+// 32, for the tokens, as many bytes as a tile's weights, are loaded for one tile only
+// (160 x 32 rows of 6144 columns: 14.3 us, 15.5 in tiles of 16).
+int fp8_tile_rows(int matrices, const int* rows) {
+  long long tiles = 0;
+  for (int i = 0; i < matrices; ++i) tiles += (rows[i] + 31) / 32;
+  return tiles >= 256 ? 16 : 32;
+}
+
+void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t, int tile_rows) {
+  const int owned = (t.cols / kGroup + kTileWaves - 1) / kTileWaves;  // blocks of a wave
+  const int tiles = t.first_block[t.matrices];
+  int passes = 1;
+  auto launch = [&](auto kernel) { kernel<<<std::min(tiles, 256), 64 * kTileWaves, 0, s>>>(t, passes); };
+  if (tile_rows == 16) {
+    passes = (owned + 5) / 6;
+    if (passes > 1) return launch(imported_tile_fp8_kernel<6, 1, false>);
+    switch (owned) {
+      case 1: return launch(imported_tile_fp8_kernel<1, 1, true>);
+      case 2: return launch(imported_tile_fp8_kernel<2, 1, true>);
+      case 3: return launch(imported_tile_fp8_kernel<3, 1, true>);
+      case 4: return launch(imported_tile_fp8_kernel<4, 1, true>);
+      case 5: return launch(imported_tile_fp8_kernel<5, 1, true>);
+      default: return launch(imported_tile_fp8_kernel<6, 1, true>);
+    }
+  }
+  if (owned > 5) {
+    passes = (owned + 3) / 4;
+    return (owned + passes - 1) / passes == 3 ? launch(imported_tile_fp8_kernel<3, 2, false>)
+                                              : launch(imported_tile_fp8_kernel<4, 2, false>);
+  }
+  switch (owned) {
+    case 1: return launch(imported_tile_fp8_kernel<1, 2, true>);
+    case 2: return launch(imported_tile_fp8_kernel<2, 2, true>);
+    case 3: return launch(imported_tile_fp8_kernel<3, 2, true>);
+    case 4: return launch(imported_tile_fp8_kernel<4, 2, true>);
+    default: return launch(imported_tile_fp8_kernel<5, 2, true>);
   }
 }
 
@@ -628,13 +723,13 @@ bool matvec_prepares(int storage, const void* input, int tokens, int input_dim) 
 namespace {
 size_t tile_values_bytes(int tokens, int input_dim) {
   const size_t padded = (static_cast<size_t>(tokens) + 31) / 32 * 32;
-  return align_up(padded * input_dim * 2, 256);
+  return align_up(padded * input_dim, 256);
 }
 }  // namespace
 
 size_t dense_imported_workspace_bytes(int tokens, int input_dim) {
-  // FP32 tokens (vector path), or their FP8 values in bf16, in whole passes of
-  // 32 tokens, and the group scales (matrix-core path)
+  // FP32 tokens (vector path), or their FP8 codes, in whole passes of 32 tokens, and
+  // the group scales (matrix-core path)
   const size_t vector_path = align_up(static_cast<size_t>(tokens) * input_dim * sizeof(float), 256);
   const size_t groups = (static_cast<size_t>(input_dim) + kGroup - 1) / kGroup;
   const size_t tile_path = tile_values_bytes(tokens, input_dim) + align_up(tokens * groups * 4, 256);
@@ -689,25 +784,26 @@ int launch_dense_imported_forward(hipStream_t s, int storage, int matrices,
     return launch_status();
   }
   TileManyArgs t;
-  fill(t, t.weight_scales, 32);
-  t.tokens = static_cast<const uint16_t*>(input);
+  const int tile_rows = fp8 ? fp8_tile_rows(matrices, output_dims) : 32;
+  fill(t, t.weight_scales, tile_rows);
+  const unsigned char* token_bytes = static_cast<const unsigned char*>(input);
   if (fp8) {
-    uint16_t* values = static_cast<uint16_t*>(workspace);
+    unsigned char* codes = static_cast<unsigned char*>(workspace);
     float* token_scales = reinterpret_cast<float*>(static_cast<char*>(workspace) +
                                                    tile_values_bytes(tokens, input_dim));
     imported_token_fp8_kernel<<<groups, kGroup, 0, s>>>(static_cast<const uint16_t*>(input),
-                                                        input_dim, values, token_scales);
-    t.tokens = values;
+                                                        input_dim, codes, token_scales);
+    token_bytes = codes;
     t.token_scales = token_scales;
   }
   const int blocks = t.first_block[matrices];
   for (int done = 0; done < tokens; done += 32) {
     t.count = tokens - done < 32 ? tokens - done : 32;
+    t.tokens = token_bytes + static_cast<size_t>(done) * input_dim * (fp8 ? 1 : 2);
     if (fp8)
-      launch_fp8_tiles(s, t, blocks);
+      launch_fp8_tiles(s, t, tile_rows);
     else
-      imported_tile_kernel<false><<<blocks, 64 * kTileWaves, 0, s>>>(t);
-    t.tokens += static_cast<size_t>(32) * input_dim;
+      imported_tile_kernel<<<blocks, 64 * kTileWaves, 0, s>>>(t);
     if (fp8) t.token_scales += static_cast<size_t>(32) * (input_dim / kGroup);
     for (int i = 0; i < matrices; ++i) t.out[i] += static_cast<size_t>(32) * output_dims[i];
   }

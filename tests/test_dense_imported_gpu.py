@@ -174,6 +174,28 @@ def test_matrix_core_batch_matches_the_oracle(capi, oracle):
             assert np.mean(got[t] != want) <= 0.05, (storage, t)
 
 
+@pytest.mark.parametrize("cols,rows,tokens", [(128, 8200, 9), (5120, 8210, 32), (6144, 8192, 17), (7168, 8200, 32),
+                                              (4096, 100, 16), (6144, 33, 32), (9216, 130, 31)])
+def test_fp8_tiles_match_float64_products(capi, cols, rows, tokens):
+    """More than eight tokens of FP8 matrices: workgroups that walk over tiles of 16 rows
+    (8192 rows and more) or of 32, with one pass over the columns or several, partial
+    row tiles, columns that are no multiple of the eight waves' blocks.  Against float64
+    products of the FP8 values and the tokens quantized as one token is."""
+    torch.manual_seed(cols + rows)
+    weights = torch.randn(rows, cols, device="cuda").to(torch.float8_e4m3fn)
+    scales = torch.rand((rows + 127) // 128, cols // 128, device="cuda") + 0.5
+    # tokens that are FP8 values times a power of two are quantized exactly
+    x = torch.randn(tokens, cols, device="cuda").to(torch.float8_e4m3fn).float().clamp(-448, 448)
+    x.view(tokens, cols // 128, 128)[:, :, 0] = 448.0
+    x = (x * 0.25).to(torch.bfloat16)
+    got = capi.dense_imported_forward_batch(capi.MATRIX_FP8_E4M3, weights.view(torch.uint8), scales, x)
+    torch.cuda.synchronize()
+    full = scales.double().repeat_interleave(128, 0)[:rows].repeat_interleave(128, 1)
+    want = x.double() @ (weights.double() * full).t()
+    error = (got.double() - want).abs()
+    assert (error <= 0.004 * want.abs() + 2e-5 * want.abs().max()).all(), error.max().item()
+
+
 @pytest.mark.parametrize("cols,tokens", [(512, 32), (512, 40), (1024, 33), (512, 5), (263, 11)])
 def test_several_matrices_of_one_input_match_the_single_calls(capi, oracle, cols, tokens):
     """The query | gate, key and value projections of a block (qwen/model.cc:174-274)
