@@ -21,8 +21,10 @@ struct PrefillPrepareArgs {
   const void* v = nullptr;   // bf16 [T, kh, d]
   const float* q_norm = nullptr;
   const float* k_norm = nullptr;
-  const float* cosines = nullptr;  // [T, rotary/2]
-  const float* sines = nullptr;
+  float* cosines = nullptr;  // scratch for the rotation's table [T, rotary/2]
+  float* sines = nullptr;
+  bool keep_table = false;   // the caller reads the table afterwards
+  float theta = 10000.0f;
   void* q_out = nullptr;  // [T, qh, d], bf16 when rounding, else fp32
   int q_out_dtype = PLUTO_HIP_BF16;
   CacheView cache;
@@ -100,9 +102,6 @@ struct DecodeArgs {
   double inverse_frequency[128];
 };
 
-int launch_rope_table(hipStream_t stream, int start_position, int length,
-                      int rotary_dim, float theta, bool round, float* cosines,
-                      float* sines);
 int launch_prefill_prepare(hipStream_t stream, const PrefillPrepareArgs& args);
 int launch_decode_prepare(hipStream_t stream, const DecodePrepareArgs& args,
                           const DecodeBatch& batch);

@@ -274,9 +274,6 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   const bool round = p->round_to_bfloat16 != 0;
   const int qh = p->query_heads, kh = p->key_value_heads, d = p->head_dim;
 
-  status = launch_rope_table(s, start_position, length, p->rotary_dim, p->rope_theta, round,
-                             cosines, sines);
-  if (status != 0) return status;
   PrefillPrepareArgs prep;
   prep.qg = qg;
   prep.k = k;
@@ -295,6 +292,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   prep.key_value_heads = kh;
   prep.head_dim = d;
   prep.rotary_dim = p->rotary_dim;
+  prep.theta = p->rope_theta;
   prep.epsilon = p->rms_norm_epsilon;
   prep.round = round;
   status = launch_prefill_prepare(s, prep);
@@ -392,8 +390,6 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   // Recompute what the forward pass derived from the inputs: normalised,
   // rotated q and k (PrepareKernel, qwen_attention.cc:30-63), then -- unless
   // the forward pass saved them -- the attention core with its row statistics.
-  status = launch_rope_table(s, 0, length, p->rotary_dim, p->rope_theta, round, cosines, sines);
-  if (status != 0) return status;
   PrefillPrepareArgs prep;
   prep.qg = qg;
   prep.k = k;
@@ -411,6 +407,8 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   prep.key_value_heads = kh;
   prep.head_dim = d;
   prep.rotary_dim = p->rotary_dim;
+  prep.theta = p->rope_theta;
+  prep.keep_table = true;  // the gradients rotate back
   prep.epsilon = p->rms_norm_epsilon;
   prep.round = round;
   status = launch_prefill_prepare(s, prep);
@@ -774,6 +772,7 @@ static int decode_run(void* stream, const pluto_hip_attention_params* p, int bat
       prep.key_value_heads = kh;
       prep.head_dim = d;
       prep.rotary_dim = p->rotary_dim;
+  prep.theta = p->rope_theta;
       prep.epsilon = p->rms_norm_epsilon;
       prep.theta = p->rope_theta;
       prep.round = round;

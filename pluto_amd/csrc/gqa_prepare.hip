@@ -11,21 +11,46 @@
 #include "gqa_rotate.h"
 #include "mfma_tile.h"
 
+#include <cmath>
+#include <type_traits>
+
 namespace pluto_hip {
 namespace {
 
+// theta^(-2 i / rotary) for i < rotary/2, made once on the host.
+struct RopeFrequencies {
+  double value[128];
+};
+
+const RopeFrequencies& rope_frequencies(float theta, int rotary_dim) {
+  thread_local RopeFrequencies known;
+  thread_local float known_theta = 0.0f;
+  thread_local int known_dim = -1;
+  if (theta != known_theta || rotary_dim != known_dim) {
+    for (int f = 0; f < rotary_dim / 2; ++f)
+      known.value[f] = std::pow(static_cast<double>(theta), -2.0 * f / rotary_dim);
+    known_theta = theta;
+    known_dim = rotary_dim;
+  }
+  return known;
+}
+
+__device__ inline void rope_angle(int position, double frequency, bool round, float& cosine, float& sine) {
+  double s, c;
+  sincos(static_cast<double>(position) * frequency, &s, &c);
+  cosine = maybe_round(static_cast<float>(c), round);
+  sine = maybe_round(static_cast<float>(s), round);
+}
+
 // cos/sin of position * theta^(-2 i / rotary) for i < rotary/2, rounded.
 __global__ void __launch_bounds__(256)
-rope_table_kernel(int start_position, int length, int rotary_dim, float theta,
+rope_table_kernel(int start_position, int length, int rotary_dim, RopeFrequencies frequencies,
                   bool round, float* __restrict__ cosines, float* __restrict__ sines) {
   const int half = rotary_dim / 2;
   const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= static_cast<long long>(length) * half) return;
   const int row = static_cast<int>(i / half), f = static_cast<int>(i % half);
-  const double angle = static_cast<double>(start_position + row) *
-                       pow(static_cast<double>(theta), -2.0 * f / rotary_dim);
-  cosines[i] = maybe_round(static_cast<float>(cos(angle)), round);
-  sines[i] = maybe_round(static_cast<float>(sin(angle)), round);
+  rope_angle(start_position + row, frequencies.value[f], round, cosines[i], sines[i]);
 }
 
 // One wave per (row, head); heads [0, qh) are queries, [qh, qh + kh) keys
@@ -67,15 +92,19 @@ prefill_prepare_kernel(PrefillPrepareArgs a) {
 // 16-byte load and store), the D/8 threads of a (row, head) are neighbouring
 // lanes.  Requires rotary_dim/2 to be a multiple of 8 so that a thread's RoPE
 // partners all sit in one other thread.  Arithmetic and rounding points are
-// those of normalize_rotate above.
-template <int D>
+// those of normalize_rotate above.  ANGLES: the workgroup makes the cosines and sines of
+// its rows itself, while the rows travel, instead of reading the table.
+template <int D, bool ANGLES>
 __global__ void __launch_bounds__(256)
-prefill_prepare_bf16_kernel(PrefillPrepareArgs a) {
-  constexpr int LANES = D / 8;
+prefill_prepare_bf16_kernel(PrefillPrepareArgs a, std::conditional_t<ANGLES, RopeFrequencies, int> frequencies) {
+  constexpr int LANES = D / 8, UNITS = 256 / LANES;
+  __shared__ __attribute__((aligned(16))) float angles[2][ANGLES ? UNITS * (D / 2) : 4];
   const int heads = a.query_heads + a.key_value_heads;
   const long long thread = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  const long long unit = thread / LANES;
-  if (unit >= static_cast<long long>(a.length) * heads) return;  // whole groups drop out
+  const long long units = static_cast<long long>(a.length) * heads;
+  const long long unit = min(thread / LANES, units - 1);
+  const bool outside = thread / LANES >= units;  // whole groups
+  const int first_row = static_cast<int>(static_cast<long long>(blockIdx.x) * UNITS / heads);
   const int chunk = static_cast<int>(thread % LANES);
   const int row = static_cast<int>(unit / heads);
   const int head = static_cast<int>(unit % heads);
@@ -99,6 +128,15 @@ prefill_prepare_bf16_kernel(PrefillPrepareArgs a) {
     weight = a.k_norm;
   }
   const uint4 bits = *reinterpret_cast<const uint4*>(in + 8 * chunk);
+  if constexpr (ANGLES) {
+    const long long last_unit = min(static_cast<long long>(blockIdx.x + 1) * UNITS, units) - 1;
+    const int count = (static_cast<int>(last_unit / heads) - first_row + 1) * half;
+    for (int i = threadIdx.x; i < count; i += 256)
+      rope_angle(a.start_position + first_row + i / half, frequencies.value[i % half], a.round, angles[0][i],
+                 angles[1][i]);
+    __syncthreads();
+  }
+  if (outside) return;
   const uint32_t words[4] = {bits.x, bits.y, bits.z, bits.w};
   float x[8];
 #pragma unroll
@@ -136,11 +174,14 @@ prefill_prepare_bf16_kernel(PrefillPrepareArgs a) {
   for (int i = 0; i < 4; ++i) partner[i] = __shfl(normalized[i], partner_lane, 64);
   uint32_t result[4] = {normalized[0], normalized[1], normalized[2], normalized[3]};
   if (rotated) {
-    const long long table = static_cast<long long>(row) * half + (lower ? first : first - half);
-    const float4 c0 = *reinterpret_cast<const float4*>(a.cosines + table);
-    const float4 c1 = *reinterpret_cast<const float4*>(a.cosines + table + 4);
-    const float4 s0 = *reinterpret_cast<const float4*>(a.sines + table);
-    const float4 s1 = *reinterpret_cast<const float4*>(a.sines + table + 4);
+    const long long table =
+        static_cast<long long>(row - (ANGLES ? first_row : 0)) * half + (lower ? first : first - half);
+    const float* cosines = ANGLES ? angles[0] : a.cosines;
+    const float* sines = ANGLES ? angles[1] : a.sines;
+    const float4 c0 = *reinterpret_cast<const float4*>(cosines + table);
+    const float4 c1 = *reinterpret_cast<const float4*>(cosines + table + 4);
+    const float4 s0 = *reinterpret_cast<const float4*>(sines + table);
+    const float4 s1 = *reinterpret_cast<const float4*>(sines + table + 4);
     const float cosine[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
     const float sine[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
@@ -216,15 +257,10 @@ decode_prepare_kernel(DecodePrepareArgs a, DecodeBatch batch) {
 
 }  // namespace
 
-int launch_rope_table(hipStream_t stream, int start_position, int length,
-                      int rotary_dim, float theta, bool round, float* cosines,
-                      float* sines) {
-  const long long count = static_cast<long long>(length) * (rotary_dim / 2);
-  if (!kernel_enabled(kAuxiliaryKernel)) return 0;
-  rope_table_kernel<<<static_cast<unsigned>((count + 255) / 256), 256, 0, stream>>>(
-      start_position, length, rotary_dim, theta, round, cosines, sines);
-  return launch_status();
-}
+// Below, what is left of a table launch (5 us) is more than the angles cost when every
+// workgroup makes those of its rows: 19 rows of 24 + 4 heads of 256 channels took 20.0 us
+// in all with the table, 18.1 without.
+constexpr long long kOwnAnglesBlocks = 2048;
 
 int launch_prefill_prepare(hipStream_t stream, const PrefillPrepareArgs& a) {
   const long long units =
@@ -239,15 +275,32 @@ int launch_prefill_prepare(hipStream_t stream, const PrefillPrepareArgs& a) {
       aligned(a.k) && aligned(a.v) && aligned(a.q_out) && aligned(a.cache.keys) &&
       aligned(a.cache.values) && aligned(a.q_norm) && aligned(a.k_norm) && aligned(a.cosines) &&
       aligned(a.sines);
+  const long long blocks = (units * (d / 8) + 255) / 256;
+  const RopeFrequencies& frequencies = rope_frequencies(a.theta, a.rotary_dim);
+  const bool own_angles = vectorised && !a.keep_table && blocks <= kOwnAnglesBlocks;
+  if (!own_angles) {
+    const long long count = static_cast<long long>(a.length) * (a.rotary_dim / 2);
+    if (count > 0) {
+      rope_table_kernel<<<static_cast<unsigned>((count + 255) / 256), 256, 0, stream>>>(
+          a.start_position, a.length, a.rotary_dim, frequencies, a.round, a.cosines, a.sines);
+      const int status = launch_status();
+      if (status != 0) return status;
+    }
+  }
   if (vectorised) {
-    const long long threads = units * (d / 8);
-    const unsigned blocks = static_cast<unsigned>((threads + 255) / 256);
+    auto launch = [&](auto width) {
+      constexpr int D = decltype(width)::value;
+      if (own_angles)
+        prefill_prepare_bf16_kernel<D, true><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(a, frequencies);
+      else
+        prefill_prepare_bf16_kernel<D, false><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(a, 0);
+    };
     if (d == 64)
-      prefill_prepare_bf16_kernel<64><<<blocks, 256, 0, stream>>>(a);
+      launch(std::integral_constant<int, 64>());
     else if (d == 128)
-      prefill_prepare_bf16_kernel<128><<<blocks, 256, 0, stream>>>(a);
+      launch(std::integral_constant<int, 128>());
     else
-      prefill_prepare_bf16_kernel<256><<<blocks, 256, 0, stream>>>(a);
+      launch(std::integral_constant<int, 256>());
     return launch_status();
   }
   prefill_prepare_kernel<<<static_cast<unsigned>((units + 3) / 4), 256, 0, stream>>>(a);

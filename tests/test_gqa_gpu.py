@@ -291,6 +291,27 @@ def test_config3_prefill_8192(capi, oracle):
     assert_close_bf16(got, out2.float().cpu().numpy(), "config 3 vs fp32-arithmetic kernel")
 
 
+@pytest.mark.parametrize("d,rotary,rows", [(128, 64, 4096), (256, 64, 2048), (64, 32, 4096)])
+def test_angles_of_short_and_long_prefills_agree(capi, oracle, d, rotary, rows):
+    # Up to a size every workgroup of the preparation makes the rotation's angles
+    # itself (here exactly at it), beyond it they come from a table: the cached keys
+    # of the same rows must be the same bytes.
+    qh, kh = (6, 2) if d > 64 else (12, 4)
+    keys = []
+    for length in (rows, rows + 3):
+        p, _ = both_params(capi, oracle, query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=rotary,
+                           capacity=rows + 10)
+        torch.manual_seed(d)
+        qg = torch.randn(rows + 3, qh, 2, d, device="cuda").to(torch.bfloat16)[:length].contiguous()
+        k, v = (torch.randn(rows + 3, kh, d, device="cuda").to(torch.bfloat16)[:length].contiguous()
+                for _ in range(2))
+        cache = capi.KvCache(rows + 10, kh, d)
+        capi.gqa_prefill(p, qg, k, v, dev(values(d, 0.2, 0.3)), dev(values(d, 0.8, 0.4)), cache, start_position=5)
+        torch.cuda.synchronize()
+        keys.append(cache.keys[:, 5:5 + rows].clone())
+    assert torch.equal(keys[0], keys[1])
+
+
 @pytest.mark.parametrize("start,length,d", [(3999, 1, 256), (4032, 64, 256), (2000, 129, 256),
                                             (1023, 33, 128), (5037, 257, 128), (3000, 700, 128)])
 def test_prefill_behind_a_long_cache_splits_its_keys(capi, oracle, start, length, d):
