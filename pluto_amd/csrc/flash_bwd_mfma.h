@@ -36,9 +36,9 @@ FlashBackwardArgs packed_flash_backward(const GenericBackwardArgs& args, float* 
                                         uint16_t* d_out_bf16);
 bool flash_backward_supported(const FlashBackwardArgs& args);
 int launch_flash_backward(hipStream_t stream, const FlashBackwardArgs& args);
-// The key-owned kernel for heads of 64 channels with a hand-scheduled main loop
-// (flash_dkv_wide.hip); reads what the query-owned kernel left in lse2,
-// deltas and d_out_bf16.
+// The key-owned kernels with a hand-scheduled main loop, heads of 64 or 128 channels
+// (flash_dkv_wide.hip); they read what the query-owned kernel left in lse2, deltas
+// and d_out_bf16.
 int launch_flash_dkv_wide(hipStream_t stream, const FlashBackwardArgs& args);
 
 }  // namespace pluto_hip

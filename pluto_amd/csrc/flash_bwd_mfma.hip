@@ -11,8 +11,8 @@
 //         (attention.cc:283-291): delta = sum(dO * O) per (row, head), plus the
 //         row's log2-sum-exp and a bf16 copy of dO, all three left in the
 //         workspace for the second kernel.
-//   dkv   one workgroup per 128 keys, loops over query tiles in ascending
-//         order.
+//   dkv   heads of 64: one workgroup per 128 keys, loops over query tiles in
+//         ascending order (heads of 128: flash_dkv_wide.hip).
 // Streamed tiles are row major in LDS, filled by direct-to-LDS buffer loads;
 // the same tile feeds the score product through 16-byte row reads and the
 // gradient product through LDS transpose reads (mfma_tile.h).  All products
@@ -31,13 +31,12 @@ namespace {
 constexpr int kThreads = 256;
 // Schedules (see BackwardUnit).  The 64-wide dQ kernel keeps three
 // workgroups per CU resident, which holds the whole paired grid of the
-// training shape at once; the other three kernels hold two per CU and drain
-// faster unpaired (1554 -> 1177 us for dK/dV and 754 -> 644 us for dQ at
-// T = 8192, 24 heads of 128; 99 -> 94 us for dK/dV at T = 1024, 12 heads of
-// 64, 16 sequences; the 64-wide dQ kernel is 8 % slower unpaired).
+// training shape at once; the other kernels hold two per CU and drain
+// faster unpaired (754 -> 644 us for dQ at T = 8192, 24 heads of 128; 99 -> 94 us
+// for dK/dV at T = 1024, 12 heads of 64, 16 sequences; the 64-wide dQ kernel is 8 %
+// slower unpaired).
 constexpr int kWideFromRows = 4096;
 constexpr bool kDqPaired64 = true;
-constexpr bool kOtherPaired = false;
 
 // Which tile(s) a workgroup owns.  Paired: the workgroup takes tile `pair`
 // and tile tiles-1-pair, which together carry the same work for every pair
@@ -323,12 +322,11 @@ __device__ inline void dkv_fill_stage(unsigned char* stage, int wave, int lane,
 }
 
 // dK^T[d, key] = sum_q Q^T[d, q] dS[q, key];  dV^T[d, key] = sum_q dO^T[d, q] P[q, key]
-template <int D, bool PAIRED>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 flash_dkv_kernel(FlashBackwardArgs a) {
-  constexpr int BNK = 128;
-  constexpr int BQ = D == 64 ? 64 : 32;  // query rows per LDS tile
+  constexpr int D = 64, BNK = 128;
+  constexpr int BQ = 64;  // query rows per LDS tile
   constexpr int KCH = D / 8, KS = D / 16, DB = D / 32, QB = BQ / 32;
   constexpr int LOADS = BQ * KCH / kThreads;
   constexpr int kTileBytes = BQ * D * 2;
@@ -341,8 +339,8 @@ flash_dkv_kernel(FlashBackwardArgs a) {
   const int h = lane / 32, n = lane % 32;
   const int T = a.context_length, H = a.num_heads, E = H * D;
   const int key_tiles = (T + BNK - 1) / BNK;
-  const BackwardUnit unit = backward_unit<PAIRED>(key_tiles, H);
-  const int pair = unit.pair, head = unit.head, seq = unit.seq;
+  const BackwardUnit unit = backward_unit<false>(key_tiles, H);
+  const int head = unit.head, seq = unit.seq;
   const long long seq_row0 = static_cast<long long>(seq) * T;
   const long long stats_base = (static_cast<long long>(seq) * H + head) * T;
   const long long q_stride = a.q_row, kv_stride = a.kv_row;
@@ -367,164 +365,145 @@ flash_dkv_kernel(FlashBackwardArgs a) {
 #pragma unroll
   for (int db = 0; db < DB; ++db) tr_read[db] = tile_transpose_read<D>(lane, db);
 
-  // Key tiles (pair) and (key_tiles-1-pair) together visit the same number of
-  // query tiles for every pair.  Query tiles are visited in ascending order
-  // within each key tile (fixed reduction order).
-  for (int pass = 0; pass < (PAIRED ? 2 : 1); ++pass) {
-    const int key_tile = pass == 0 ? pair : key_tiles - 1 - pair;
-    if (pass == 1 && key_tile == pair) break;
-    const int k0 = key_tile * BNK;
-    const int first_tile = k0 / BQ;
-    if (first_tile < tiles)
-      dkv_fill_stage<D, BQ, LOADS>(lds + ((first_tile) & 1) * kStageBytes, wave, lane, q_base, g_base,
-                                   lse2_base, delta_base, q_stride, E, (first_tile) * BQ, T, q_fill, g_fill);
-    const int key_row = k0 + 32 * wave + n;
-    const int key_load = min(key_row, T - 1);
-    bf16x8 kf[KS], vf[KS];
+  // Query tiles are visited in ascending order (fixed reduction order).
+  const int k0 = unit.pair * BNK;
+  const int first_tile = k0 / BQ;
+  if (first_tile < tiles)
+    dkv_fill_stage<D, BQ, LOADS>(lds + ((first_tile) & 1) * kStageBytes, wave, lane, q_base, g_base,
+                                 lse2_base, delta_base, q_stride, E, (first_tile) * BQ, T, q_fill, g_fill);
+  const int key_row = k0 + 32 * wave + n;
+  const int key_load = min(key_row, T - 1);
+  bf16x8 kf[KS], vf[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      kf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-          k_base + key_load * kv_stride + 16 * ks + 8 * h));
-      vf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-          v_base + key_load * kv_stride + 16 * ks + 8 * h));
+  for (int ks = 0; ks < KS; ++ks) {
+    kf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
+        k_base + key_load * kv_stride + 16 * ks + 8 * h));
+    vf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
+        v_base + key_load * kv_stride + 16 * ks + 8 * h));
+  }
+  floatx16 dk_acc[DB], dv_acc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      dk_acc[db][i] = 0.0f;
+      dv_acc[db][i] = 0.0f;
     }
-    floatx16 dk_acc[DB], dv_acc[DB];
+  const int wave_first_key = k0 + 32 * wave;
+
+  for (int tile = first_tile; tile < tiles; ++tile) {
+    const int q0 = tile * BQ;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tile + 1 < tiles)
+      dkv_fill_stage<D, BQ, LOADS>(lds + ((tile + 1) & 1) * kStageBytes, wave, lane, q_base, g_base,
+                                   lse2_base, delta_base, q_stride, E, (tile + 1) * BQ, T, q_fill, g_fill);
+    const unsigned char* q_tile = lds + (tile & 1) * kStageBytes;
+    const unsigned char* g_tile = q_tile + kTileBytes;
+    const float* stat_lse2 = reinterpret_cast<const float*>(q_tile + 2 * kTileBytes);
+    const float* stat_delta = stat_lse2 + kStatBytes / 4;
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+    for (int qb = 0; qb < QB; ++qb) {
+      const int qb0 = q0 + 32 * qb;
+      if (qb0 + 31 < wave_first_key) continue;  // every query precedes my keys
+      const unsigned char* q_block = q_tile + qb * kBlockBytes;
+      const unsigned char* g_block = g_tile + qb * kBlockBytes;
+      bf16x8 qt[2][DB], gt[2][DB];  // transposed operands, requested up front
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          gt[s2][db] = tile_transposed_operand<D>(g_block, tr_read[db], s2);
+          qt[s2][db] = tile_transposed_operand<D>(q_block, tr_read[db], s2);
+        }
+      // accumulator register i = (query qb0 + 8(i/4) + 4h + i%4, key n); the
+      // score accumulator starts from -lse/scale of its query, the dP
+      // accumulator from -delta
+      floatx16 s, dp;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 l2 = *reinterpret_cast<const float4*>(&stat_lse2[32 * qb + 8 * j + 4 * h]);
+        const float4 dl = *reinterpret_cast<const float4*>(&stat_delta[32 * qb + 8 * j + 4 * h]);
+        s[4 * j + 0] = l2.x; s[4 * j + 1] = l2.y; s[4 * j + 2] = l2.z; s[4 * j + 3] = l2.w;
+        dp[4 * j + 0] = dl.x; dp[4 * j + 1] = dl.y; dp[4 * j + 2] = dl.z; dp[4 * j + 3] = dl.w;
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8 qa = as_bf16x8(*reinterpret_cast<const uint4*>(q_block + row_read[ks]));
+        const bf16x8 ga = as_bf16x8(*reinterpret_cast<const uint4*>(g_block + row_read[ks]));
+        s = mfma32(qa, kf[ks], s);
+        dp = mfma32(ga, vf[ks], dp);
+      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        dk_acc[db][i] = 0.0f;
-        dv_acc[db][i] = 0.0f;
+        const float p = __builtin_amdgcn_exp2f(s[i] * scale2);
+        s[i] = p;
+        dp[i] = p * dp[i];
       }
-    const int wave_first_key = k0 + 32 * wave;
-
-    for (int tile = first_tile; tile < tiles; ++tile) {
-      const int q0 = tile * BQ;
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (tile + 1 < tiles)
-        dkv_fill_stage<D, BQ, LOADS>(lds + ((tile + 1) & 1) * kStageBytes, wave, lane, q_base, g_base,
-                                     lse2_base, delta_base, q_stride, E, (tile + 1) * BQ, T, q_fill, g_fill);
-      const unsigned char* q_tile = lds + (tile & 1) * kStageBytes;
-      const unsigned char* g_tile = q_tile + kTileBytes;
-      const float* stat_lse2 = reinterpret_cast<const float*>(q_tile + 2 * kTileBytes);
-      const float* stat_delta = stat_lse2 + kStatBytes / 4;
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
-        const int qb0 = q0 + 32 * qb;
-        if (qb0 + 31 < wave_first_key) continue;  // every query precedes my keys
-        const unsigned char* q_block = q_tile + qb * kBlockBytes;
-        const unsigned char* g_block = g_tile + qb * kBlockBytes;
-        // transposed operands: requested up front when the register budget
-        // allows (64-wide heads), otherwise just before their products
-        constexpr bool kHoist = D == 64;
-        bf16x8 qt[2][DB], gt[2][DB];
-        if constexpr (kHoist) {
-#pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-            for (int db = 0; db < DB; ++db) {
-              gt[s2][db] = tile_transposed_operand<D>(g_block, tr_read[db], s2);
-              qt[s2][db] = tile_transposed_operand<D>(q_block, tr_read[db], s2);
-            }
-        }
-        // accumulator register i = (query qb0 + 8(i/4) + 4h + i%4, key n); the
-        // score accumulator starts from -lse/scale of its query, the dP
-        // accumulator from -delta
-        floatx16 s, dp;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float4 l2 = *reinterpret_cast<const float4*>(&stat_lse2[32 * qb + 8 * j + 4 * h]);
-          const float4 dl = *reinterpret_cast<const float4*>(&stat_delta[32 * qb + 8 * j + 4 * h]);
-          s[4 * j + 0] = l2.x; s[4 * j + 1] = l2.y; s[4 * j + 2] = l2.z; s[4 * j + 3] = l2.w;
-          dp[4 * j + 0] = dl.x; dp[4 * j + 1] = dl.y; dp[4 * j + 2] = dl.z; dp[4 * j + 3] = dl.w;
-        }
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8 qa = as_bf16x8(*reinterpret_cast<const uint4*>(q_block + row_read[ks]));
-          const bf16x8 ga = as_bf16x8(*reinterpret_cast<const uint4*>(g_block + row_read[ks]));
-          s = mfma32(qa, kf[ks], s);
-          dp = mfma32(ga, vf[ks], dp);
-        }
+      if (qb0 < wave_first_key + 31 || qb0 + 32 > T) {
+        // diagonal block (queries before this lane's key) or sequence tail
+        const int first = key_row - qb0 - 4 * h;   // visible: local query >= first
+        const int last = T - 1 - qb0 - 4 * h;      //          local query <= last
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const float p = __builtin_amdgcn_exp2f(s[i] * scale2);
-          s[i] = p;
-          dp[i] = p * dp[i];
+          const int local = 8 * (i / 4) + (i % 4);
+          const bool hidden = (local < first) | (local > last);
+          s[i] = hidden ? 0.0f : s[i];
+          dp[i] = hidden ? 0.0f : dp[i];
         }
-        if (qb0 < wave_first_key + 31 || qb0 + 32 > T) {
-          // diagonal block (queries before this lane's key) or sequence tail
-          const int first = key_row - qb0 - 4 * h;   // visible: local query >= first
-          const int last = T - 1 - qb0 - 4 * h;      //          local query <= last
+      }
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int local = 8 * (i / 4) + (i % 4);
-            const bool hidden = (local < first) | (local > last);
-            s[i] = hidden ? 0.0f : s[i];
-            dp[i] = hidden ? 0.0f : dp[i];
-          }
-        }
+      for (int s2 = 0; s2 < 2; ++s2) {
+        const bf16x8 pf = accumulator_to_operand(s, s2);
+        const bf16x8 dsf = accumulator_to_operand(dp, s2);
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const bf16x8 pf = accumulator_to_operand(s, s2);
-          const bf16x8 dsf = accumulator_to_operand(dp, s2);
-          if constexpr (!kHoist) {
-#pragma unroll
-            for (int db = 0; db < DB; ++db) {
-              gt[s2][db] = tile_transposed_operand<D>(g_block, tr_read[db], s2);
-              qt[s2][db] = tile_transposed_operand<D>(q_block, tr_read[db], s2);
-            }
-          }
-#pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            dv_acc[db] = mfma32(gt[s2][db], pf, dv_acc[db]);
-            dk_acc[db] = mfma32(qt[s2][db], dsf, dk_acc[db]);
-          }
+        for (int db = 0; db < DB; ++db) {
+          dv_acc[db] = mfma32(gt[s2][db], pf, dv_acc[db]);
+          dk_acc[db] = mfma32(qt[s2][db], dsf, dk_acc[db]);
         }
       }
     }
-    // dK and dV leave through LDS so that every store instruction writes whole
-    // rows (16 lanes x 16 bytes): written straight from the accumulators, a
-    // lane's 16-byte pieces lie 9 KiB apart and each store touches 32 lines.
-    // One tensor at a time, 32 keys x D floats a wave, pieces swizzled by row.
-    __syncthreads();  // every wave is done with the tile stages
-    {
-      // 64 columns of one tensor at a time: 32 keys x 64 floats a wave, 32 KiB
-      static_assert(4 * 32 * 64 * 4 <= 2 * kStageBytes, "the stages hold one step of the workgroup");
-      constexpr int kPieces = 16;  // 16-byte pieces in 64 columns
-      float4* area = reinterpret_cast<float4*>(lds) + wave * 32 * kPieces;
-      const int out_piece = lane % kPieces, out_row = lane / kPieces;
+  }
+  // dK and dV leave through LDS so that every store instruction writes whole
+  // rows (16 lanes x 16 bytes): written straight from the accumulators, a
+  // lane's 16-byte pieces lie 9 KiB apart and each store touches 32 lines.
+  // One tensor at a time, 32 keys x D floats a wave, pieces swizzled by row.
+  __syncthreads();  // every wave is done with the tile stages
+  {
+    // 64 columns of one tensor at a time: 32 keys x 64 floats a wave, 32 KiB
+    static_assert(4 * 32 * 64 * 4 <= 2 * kStageBytes, "the stages hold one step of the workgroup");
+    constexpr int kPieces = 16;  // 16-byte pieces in 64 columns
+    float4* area = reinterpret_cast<float4*>(lds) + wave * 32 * kPieces;
+    const int out_piece = lane % kPieces, out_row = lane / kPieces;
 #pragma unroll
-      for (int step = 0; step < 2 * (D / 64); ++step) {
-        const int tensor = step / (D / 64), half = step % (D / 64);
+    for (int step = 0; step < 2 * (D / 64); ++step) {
+      const int tensor = step / (D / 64), half = step % (D / 64);
 #pragma unroll
-        for (int d2 = 0; d2 < 2; ++d2)
+      for (int d2 = 0; d2 < 2; ++d2)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const floatx16& acc = tensor == 0 ? dk_acc[2 * half + d2] : dv_acc[2 * half + d2];
-            const float factor = tensor == 0 ? a.scale : 1.0f;
-            float4 value;
-            value.x = acc[4 * j + 0] * factor;
-            value.y = acc[4 * j + 1] * factor;
-            value.z = acc[4 * j + 2] * factor;
-            value.w = acc[4 * j + 3] * factor;
-            const int piece = 8 * d2 + 2 * j + h;
-            area[n * kPieces + (piece ^ (n % kPieces))] = value;
-          }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads what its own lanes wrote
-        float* dst = (tensor == 0 ? a.dk : a.dv) + (seq_row0 + k0 + 32 * wave) * a.dkv_row +
-                     head * D + 64 * half;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int row = 4 * i + out_row;
-          const float4 value = area[row * kPieces + (out_piece ^ (row % kPieces))];
-          if (k0 + 32 * wave + row < T)
-            *reinterpret_cast<float4*>(dst + row * a.dkv_row + 4 * out_piece) = value;
+        for (int j = 0; j < 4; ++j) {
+          const floatx16& acc = tensor == 0 ? dk_acc[2 * half + d2] : dv_acc[2 * half + d2];
+          const float factor = tensor == 0 ? a.scale : 1.0f;
+          float4 value;
+          value.x = acc[4 * j + 0] * factor;
+          value.y = acc[4 * j + 1] * factor;
+          value.z = acc[4 * j + 2] * factor;
+          value.w = acc[4 * j + 3] * factor;
+          const int piece = 8 * d2 + 2 * j + h;
+          area[n * kPieces + (piece ^ (n % kPieces))] = value;
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the area is overwritten
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads what its own lanes wrote
+      float* dst = (tensor == 0 ? a.dk : a.dv) + (seq_row0 + k0 + 32 * wave) * a.dkv_row +
+                   head * D + 64 * half;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int row = 4 * i + out_row;
+        const float4 value = area[row * kPieces + (out_piece ^ (row % kPieces))];
+        if (k0 + 32 * wave + row < T)
+          *reinterpret_cast<float4*>(dst + row * a.dkv_row + 4 * out_piece) = value;
       }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the area is overwritten
     }
-    __syncthreads();  // the next pass refills a stage
   }
 }
 
@@ -593,21 +572,20 @@ int launch_flash_backward(hipStream_t stream, const FlashBackwardArgs& a) {
   } else if (dim == 64) {
     launch_dq<64, kDqPaired64>(stream, a, kDqPaired64 ? paired : unpaired);
   } else {
-    launch_dq<128, kOtherPaired>(stream, a, kOtherPaired ? paired : unpaired);
+    launch_dq<128, false>(stream, a, unpaired);
   }
   const int status = launch_status();
   if (status != 0) return status;
   if (!kernel_enabled(kMainKernel)) return 0;
-  // The hand-scheduled kernel (one wave a SIMD, 64 keys a wave) gives the same
-  // bits; it is level with the kernel below at 2048 rows and 6 % ahead at 4096.
-  if (dim == 64 && kernel_enabled(kEightWave) &&
-      (a.context_length >= kWideFromRows || !kernel_enabled(kFromLength)))
+  // The hand-scheduled kernels (one wave a SIMD, 64 keys a wave) halve the LDS
+  // reads of a matrix instruction.  For 128 channels, where 32 keys a wave are
+  // bound by them, that is worth 7 % at 64 rows, 1.5 times at 1024 and twice at 8192.  For 64
+  // channels the vector work beside the products is the bound and the kernel
+  // below is level at 2048 rows, 6 % behind at 4096.
+  if (dim == 128 || (kernel_enabled(kEightWave) &&
+                     (a.context_length >= kWideFromRows || !kernel_enabled(kFromLength))))
     return launch_flash_dkv_wide(stream, a);
-  const unsigned grid = kOtherPaired ? paired : unpaired;
-  if (dim == 64)
-    flash_dkv_kernel<64, kOtherPaired><<<grid, kThreads, 0, stream>>>(a);
-  else
-    flash_dkv_kernel<128, kOtherPaired><<<grid, kThreads, 0, stream>>>(a);
+  flash_dkv_kernel<<<unpaired, kThreads, 0, stream>>>(a);
   return launch_status();
 }
 

@@ -264,6 +264,14 @@ def test_hand_scheduled_key_owned_backward_gives_the_same_bits(capi, oracle, T, 
         assert_close_bf16_gradient(wide.cpu().numpy(), want, "wide dK/dV T%d" % T)
 
 
+@pytest.mark.parametrize("T,H,B", [(1, 1, 1), (33, 1, 2), (64, 2, 1), (65, 1, 1), (96, 1, 2), (129, 2, 1),
+                                   (257, 3, 2), (450, 2, 2)])
+def test_hand_scheduled_backward_of_128_channels(capi, oracle, T, H, B):
+    """Lengths that end inside the first block of either wave, inside a block of 32, at
+    the edges of a wave's 64 and a workgroup's 128 keys."""
+    check(capi, oracle, T, H, 128 * H, B, True, seed=T + H)
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_probabilities_pass(capi, bf16):
     # attention_test.cc:41-146: rows sum to one, zeros above the diagonal, P.V = out
