@@ -61,7 +61,7 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E (published)
 MEASURED_TRAFFIC_BYTES = {
     # (workload, kernel group): (bytes read + written, commit the counters were read at)
     ("mha_train_bf16", "flash_forward_kernel<64>"): (99.1e6 + 26.7e6, "4f26c5a"),
-    ("mha_train_bf16", "flash_dq_kernel<64>"): (179.5e6 + 77.1e6, "4f26c5a"),
+    ("mha_train_bf16", "flash_dq_kernel"): (179.5e6 + 77.1e6, "4f26c5a"),
     ("mha_train_bf16", "flash_dkv_kernel"): (154.5e6 + 100.7e6, "4f26c5a"),
     ("gqa_prefill", "flash_forward_pipelined_kernel<128>"): (184.6e6 + 88.1e6, "4f26c5a"),
     ("gqa_prefill_d256", "flash_forward_pipelined_kernel<256>"): (444.8e6 + 100.9e6, "4f26c5a"),
@@ -141,7 +141,7 @@ def mha_train_bf16(torch, capi):
     # dP, dK, dV).  The 5 counted products are shared out in that proportion.
     return dict(step=step, graph_outputs=lambda: list(state["fwd"]) + [d_qkv],
                 kernels=[("flash_forward_kernel<64>", forward, None, fwd),
-                         ("flash_dq_kernel<64>", backward, capi.QUERY_KERNEL, bwd * 3 / 7),
+                         ("flash_dq_kernel", backward, capi.QUERY_KERNEL, bwd * 3 / 7),
                          ("flash_dkv_kernel", backward, capi.MAIN_KERNEL, bwd * 4 / 7)],
                 work=fwd + bwd, metric="attention_fwd_bwd_tflops", unit="TFLOP/s", dtype="bf16",
                 bound="mfma", peak=PEAK_BF16_TFLOPS,

@@ -40,5 +40,7 @@ int launch_flash_backward(hipStream_t stream, const FlashBackwardArgs& args);
 // (flash_dkv_wide.hip); they read what the query-owned kernel left in lse2, deltas
 // and d_out_bf16.
 int launch_flash_dkv_wide(hipStream_t stream, const FlashBackwardArgs& args);
+// The query-owned kernel for heads of 128 channels (flash_dq_wide.hip).
+int launch_flash_dq_wide(hipStream_t stream, const FlashBackwardArgs& args);
 
 }  // namespace pluto_hip

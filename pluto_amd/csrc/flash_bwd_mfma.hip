@@ -6,7 +6,8 @@
 // order and no atomics, hence bitwise repeatable.
 //
 // Two kernels:
-//   dq    one workgroup per 128 queries, loops over 64-key tiles.  Its
+//   dq    heads of 64 (of 128: flash_dq_wide.hip): one workgroup per 128
+//         queries, loops over 64-key tiles.  Its
 //         prologue also does what the reference's delta pass does
 //         (attention.cc:283-291): delta = sum(dO * O) per (row, head), plus the
 //         row's log2-sum-exp and a bf16 copy of dO, all three left in the
@@ -29,14 +30,11 @@ namespace pluto_hip {
 namespace {
 
 constexpr int kThreads = 256;
-// Schedules (see BackwardUnit).  The 64-wide dQ kernel keeps three
-// workgroups per CU resident, which holds the whole paired grid of the
-// training shape at once; the other kernels hold two per CU and drain
-// faster unpaired (754 -> 644 us for dQ at T = 8192, 24 heads of 128; 99 -> 94 us
-// for dK/dV at T = 1024, 12 heads of 64, 16 sequences; the 64-wide dQ kernel is 8 %
-// slower unpaired).
+// The dQ kernel keeps three workgroups per CU resident, which holds the whole
+// paired grid of the training shape at once (8 % slower unpaired); the dK/dV kernel
+// holds two per CU and drains faster unpaired (99 -> 94 us at T = 1024, 12 heads of
+// 64, 16 sequences).
 constexpr int kWideFromRows = 4096;
-constexpr bool kDqPaired64 = true;
 
 // Which tile(s) a workgroup owns.  Paired: the workgroup takes tile `pair`
 // and tile tiles-1-pair, which together carry the same work for every pair
@@ -71,27 +69,24 @@ __device__ inline BackwardUnit backward_unit(int tiles, int heads) {
 
 // dQ^T[d, query] = sum_keys K^T[d, key] dS^T[key, query]
 // PREPARED: dO arrives as bf16 with its row statistics, else the prologue makes them.
-template <int D, bool PAIRED, bool PREPARED>
-__global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
+template <bool PREPARED>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 flash_dq_kernel(FlashBackwardArgs a) {
-  constexpr int BM = 128, BN = 64;
+  constexpr int D = 64, BM = 128, BN = 64;
   constexpr int KCH = D / 8, KS = D / 16, DB = D / 32, KB = BN / 32;
   constexpr int LOADS = BN * KCH / kThreads;
   constexpr int kTileBytes = BN * D * 2, kStageBytes = 2 * kTileBytes;
   constexpr int kBlockBytes = 32 * D * 2;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
-  // 4 KiB a wave that no other wave touches (64-wide heads, where three
-  // workgroups of 48 KiB still share a compute unit): rows on their way out are
-  // reordered here without a barrier
-  constexpr bool kOwnArea = D == 64;
-  __shared__ __attribute__((aligned(16))) uint4 own_area[kOwnArea ? 4 * 256 : 1];
+  // 4 KiB a wave that no other wave touches (three workgroups of 48 KiB still
+  // share a compute unit): rows on their way out are reordered here without a barrier
+  __shared__ __attribute__((aligned(16))) uint4 own_area[4 * 256];
 
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
   const int T = a.context_length, H = a.num_heads, E = H * D;
   const int q_tiles = (T + BM - 1) / BM;
-  const BackwardUnit unit = backward_unit<PAIRED>(q_tiles, H);
+  const BackwardUnit unit = backward_unit<true>(q_tiles, H);
   const int pair = unit.pair, head = unit.head, seq = unit.seq;
   const long long seq_row0 = static_cast<long long>(seq) * T;
   const long long stats_base = (static_cast<long long>(seq) * H + head) * T;
@@ -115,7 +110,7 @@ flash_dq_kernel(FlashBackwardArgs a) {
 
   // Query tiles (q_tiles-1-pair) and (pair) together see the same number of
   // keys for every pair: equal work per workgroup under the causal mask.
-  for (int pass = 0; pass < (PAIRED ? 2 : 1); ++pass) {
+  for (int pass = 0; pass < 2; ++pass) {
     const int q_tile = pass == 0 ? q_tiles - 1 - pair : pair;
     if (pass == 1 && q_tile == q_tiles - 1 - pair) break;
     const int q0 = q_tile * BM;
@@ -126,8 +121,7 @@ flash_dq_kernel(FlashBackwardArgs a) {
 
     const int wave_first_row = q0 + 32 * wave;
     const int q_row = wave_first_row + n;
-    uint4* copy_area = kOwnArea ? own_area + wave * 256
-                                : reinterpret_cast<uint4*>(lds + kStageBytes) + wave * 32 * KCH;
+    uint4* copy_area = own_area + wave * 256;
     // Rows beyond the sequence are clamped to its last row and never stored.
     const int q_load = min(q_row, T - 1);
     bf16x8 qf[KS], gf[KS];
@@ -167,8 +161,7 @@ flash_dq_kernel(FlashBackwardArgs a) {
         gf[ks] = as_bf16x8(bits);
         copy_area[n * KCH + ((2 * ks + h) ^ (n & 7))] = bits;
       }
-      // The bf16 copy of dO leaves through LDS (the wave's slice of the stage
-      // that no fill has been issued into yet): a lane holds 16-byte pieces of its
+      // The bf16 copy of dO leaves through the wave's own area: a lane holds 16-byte pieces of its
       // own row, and stored from there a store instruction touches 32 lines;
       // from LDS it writes whole rows (25 MB in 17 us against 5 us).
 #pragma unroll
@@ -256,44 +249,29 @@ flash_dq_kernel(FlashBackwardArgs a) {
         }
       }
     }
-    if constexpr (kOwnArea) {
-      // dQ leaves through the wave's own area, 32 columns at a time: a store
-      // instruction then writes eight whole 128-byte half rows instead of
-      // 32-byte pieces of 32 rows
-      float4* area = reinterpret_cast<float4*>(own_area) + wave * 256;
-      float* dst = a.dq + (seq_row0 + wave_first_row) * a.dq_row + head * D;
+    // dQ leaves through the wave's own area, 32 columns at a time: a store
+    // instruction then writes eight whole 128-byte half rows instead of
+    // 32-byte pieces of 32 rows
+    float4* area = reinterpret_cast<float4*>(own_area) + wave * 256;
+    float* dst = a.dq + (seq_row0 + wave_first_row) * a.dq_row + head * D;
 #pragma unroll
-      for (int db = 0; db < DB; ++db) {
+    for (int db = 0; db < DB; ++db) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float4 value;
-          value.x = dq_acc[db][4 * j + 0] * a.scale;
-          value.y = dq_acc[db][4 * j + 1] * a.scale;
-          value.z = dq_acc[db][4 * j + 2] * a.scale;
-          value.w = dq_acc[db][4 * j + 3] * a.scale;
-          area[n * 8 + ((2 * j + h) ^ (n & 7))] = value;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = 8 * i + lane / 8, piece = lane % 8;
-          const float4 value = area[row * 8 + (piece ^ (row & 7))];
-          if (wave_first_row + row < T)
-            *reinterpret_cast<float4*>(dst + row * a.dq_row + 32 * db + 4 * piece) = value;
-        }
+      for (int j = 0; j < 4; ++j) {
+        float4 value;
+        value.x = dq_acc[db][4 * j + 0] * a.scale;
+        value.y = dq_acc[db][4 * j + 1] * a.scale;
+        value.z = dq_acc[db][4 * j + 2] * a.scale;
+        value.w = dq_acc[db][4 * j + 3] * a.scale;
+        area[n * 8 + ((2 * j + h) ^ (n & 7))] = value;
       }
-    } else if (q_row < T) {
-      float* dst = a.dq + (seq_row0 + q_row) * a.dq_row + head * D;
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float4 value;
-          value.x = dq_acc[db][4 * j + 0] * a.scale;
-          value.y = dq_acc[db][4 * j + 1] * a.scale;
-          value.z = dq_acc[db][4 * j + 2] * a.scale;
-          value.w = dq_acc[db][4 * j + 3] * a.scale;
-          *reinterpret_cast<float4*>(dst + 32 * db + 8 * j + 4 * h) = value;
-        }
+      for (int i = 0; i < 4; ++i) {
+        const int row = 8 * i + lane / 8, piece = lane % 8;
+        const float4 value = area[row * 8 + (piece ^ (row & 7))];
+        if (wave_first_row + row < T)
+          *reinterpret_cast<float4*>(dst + row * a.dq_row + 32 * db + 4 * piece) = value;
+      }
     }
     __syncthreads();  // the next pass refills stage 0
   }
@@ -551,16 +529,6 @@ bool flash_backward_supported(const FlashBackwardArgs& a) {
   return true;
 }
 
-namespace {
-template <int D, bool DQ_PAIRED>
-void launch_dq(hipStream_t stream, const FlashBackwardArgs& a, unsigned grid) {
-  if (a.d_out)
-    flash_dq_kernel<D, DQ_PAIRED, false><<<grid, kThreads, 0, stream>>>(a);
-  else
-    flash_dq_kernel<D, DQ_PAIRED, true><<<grid, kThreads, 0, stream>>>(a);
-}
-}  // namespace
-
 int launch_flash_backward(hipStream_t stream, const FlashBackwardArgs& a) {
   const int dim = a.head_dim;
   const long long tiles128 = (a.context_length + 127) / 128;
@@ -568,13 +536,17 @@ int launch_flash_backward(hipStream_t stream, const FlashBackwardArgs& a) {
   if (tiles128 * units > 0x7fffffffLL) return PLUTO_HIP_EINVAL;
   const unsigned paired = static_cast<unsigned>(((tiles128 + 1) / 2) * units);
   const unsigned unpaired = static_cast<unsigned>(tiles128 * units);
+  int status = 0;
   if (!kernel_enabled(kQueryKernel)) {
-  } else if (dim == 64) {
-    launch_dq<64, kDqPaired64>(stream, a, kDqPaired64 ? paired : unpaired);
+  } else if (dim == 128) {
+    status = launch_flash_dq_wide(stream, a);
   } else {
-    launch_dq<128, false>(stream, a, unpaired);
+    if (a.d_out)
+      flash_dq_kernel<false><<<paired, kThreads, 0, stream>>>(a);
+    else
+      flash_dq_kernel<true><<<paired, kThreads, 0, stream>>>(a);
+    status = launch_status();
   }
-  const int status = launch_status();
   if (status != 0) return status;
   if (!kernel_enabled(kMainKernel)) return 0;
   // The hand-scheduled kernels (one wave a SIMD, 64 keys a wave) halve the LDS
