@@ -14,8 +14,9 @@
 // float a lane along a row for the gradient products.  The orientation is the
 // one of attn_f32_mfma.hip: dq works on S^T (lane = query), dkv on S (lane = key),
 // so the score tile's accumulator is the B operand of the gradient product.
-// 4 sequences x 12 heads x 256 x 64: 19 us for the pair, where the kernels that
+// 4 sequences x 12 heads x 256 x 64: 40 us for the pair, where the kernels that
 // multiply one element at a time took 653 us.
+#include "attn_f32_tile.h"
 #include "attn_generic.h"
 #include "mfma_tile.h"
 
@@ -23,48 +24,6 @@ namespace pluto_hip {
 namespace {
 
 constexpr int kWaves = 4;  // per workgroup, each taking every fourth streamed tile
-
-// 32 rows of D floats in LDS, 16-byte piece c of row r at slot c ^ swizzle(r):
-// the lanes of a row read (32 rows, same piece) spread over the banks.
-template <int D>
-struct F32Tile {
-  static constexpr int kPieces = D / 4;
-  static constexpr int kBytes = 32 * D * 4;
-  __device__ static int swizzle(int row) { return row & (kPieces < 16 ? kPieces - 1 : 15); }
-  // Queues the fill from global rows `row_bytes` apart, `valid` of which exist
-  // (the rest read as zero).
-  __device__ static void fill(unsigned char* tile, const float* base, long long row_stride,
-                              int valid, int lane) {
-    const int32x4 rsrc = make_rsrc(
-        base, valid <= 0 ? 0u : static_cast<uint32_t>((min(valid, 32) - 1) * row_stride + D) * 4u);
-#pragma unroll
-    for (int i = 0; i < kBytes / 1024; ++i) {
-      const int at = i * 64 + lane, row = at / kPieces, slot = at % kPieces;
-      lds_fill<16>(rsrc, tile + i * 1024,
-                   static_cast<uint32_t>(row * row_stride * 4 + (slot ^ swizzle(row)) * 16));
-    }
-  }
-  __device__ static float4 row_piece(const unsigned char* tile, int row, int piece) {
-    return *reinterpret_cast<const float4*>(tile + (row * kPieces + (piece ^ swizzle(row))) * 16);
-  }
-  __device__ static float element(const unsigned char* tile, int row, int channel) {
-    return *reinterpret_cast<const float*>(
-        tile + (row * kPieces + ((channel / 4) ^ swizzle(row))) * 16 + (channel % 4) * 4);
-  }
-};
-
-// The lane's half (channels h D/2 ..) of one row.
-template <int HALF>
-__device__ inline void load_half_row(const float* row, float* out) {
-#pragma unroll
-  for (int j = 0; j < HALF / 4; ++j) {
-    const float4 v = reinterpret_cast<const float4*>(row)[j];
-    out[4 * j] = v.x; out[4 * j + 1] = v.y; out[4 * j + 2] = v.z; out[4 * j + 3] = v.w;
-  }
-}
-
-__device__ inline void wait_fills() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ inline void wait_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 struct F32Unit {
   int tile, head, seq;
@@ -120,6 +79,22 @@ f32_dq_kernel(GenericBackwardArgs a) {
   const float* q_base = static_cast<const float*>(a.qkv) + row0 * 3 * E + unit.head * D;
   const int query = q0 + n, query_load = min(query, T - 1);
 
+  // A wave's first tile is on its way while it reads its own rows, the others while the
+  // one before is worked on: V in place as soon as it has been read, K, which is
+  // needed to the end, through registers.
+  unsigned char* k_tile = lds + wave * kArea;
+  unsigned char* v_tile = k_tile + Tile::kBytes;
+  typename Tile::Held k_held;
+  auto rows_of = [&](int kt) { return kt <= q0 / 32 ? T - kt * 32 : 0; };
+  auto request_k = [&](int kt) {
+    Tile::request(k_held, q_base + E + kt * 32 * 3LL * E, 3LL * E, rows_of(kt), lane);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto request_v = [&](int kt) {
+    Tile::fill(v_tile, q_base + 2 * E + kt * 32 * 3LL * E, 3LL * E, rows_of(kt), lane);
+  };
+  request_k(wave);
+  request_v(wave);
   float qf[HALF], gf[HALF];
   load_half_row<HALF>(q_base + query_load * 3LL * E + h * HALF, qf);
   const long long out_at = (row0 + query_load) * E + unit.head * D + h * HALF;
@@ -141,15 +116,12 @@ f32_dq_kernel(GenericBackwardArgs a) {
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[db][i] = 0.0f;
-  unsigned char* k_tile = lds + wave * kArea;
-  unsigned char* v_tile = k_tile + Tile::kBytes;
   const int key_tiles = q0 / 32 + 1;
   for (int kt = wave; kt < key_tiles; kt += kWaves) {
     const int k0 = kt * 32;
-    wait_reads();  // of the tile before
-    Tile::fill(k_tile, q_base + E + k0 * 3LL * E, 3LL * E, T - k0, lane);
-    Tile::fill(v_tile, q_base + 2 * E + k0 * 3LL * E, 3LL * E, T - k0, lane);
+    Tile::place(k_tile, k_held, lane);
     wait_fills();
+    request_k(kt + kWaves);
     floatx16 s, dp;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
@@ -166,6 +138,8 @@ f32_dq_kernel(GenericBackwardArgs a) {
       s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[4 * j + 3], s, 0, 0, 0);
       dp = __builtin_amdgcn_mfma_f32_32x32x2f32(v4.w, gf[4 * j + 3], dp, 0, 0, 0);
     }
+    wait_reads();
+    request_v(kt + kWaves);
     // register i = (key k0 + 8(i/4) + 4h + i%4, query n)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -180,7 +154,7 @@ f32_dq_kernel(GenericBackwardArgs a) {
         acc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(
             Tile::element(k_tile, 8 * (i / 4) + 4 * h + (i % 4), 32 * db + n), s[i], acc[db], 0, 0, 0);
   }
-  wait_reads();
+  wait_fills();
   float4 own[4 * DB];
 #pragma unroll
   for (int g = 0; g < 4 * DB; ++g)
@@ -211,6 +185,16 @@ f32_dkv_kernel(GenericBackwardArgs a) {
   const float* g_base = a.d_out + row0 * E + unit.head * D;
   const int key = k0 + n, key_load = min(key, T - 1);
 
+  // the first tile is on its way before the wave's own rows; registers to hold
+  // another are not left (21.5 us at 256 rows, 23.8 with the request in the loop)
+  unsigned char* q_tile = lds + wave * kArea;
+  unsigned char* g_tile = q_tile + Tile::kBytes;
+  auto request = [&](int qt) {
+    const int q0 = qt * 32;
+    Tile::fill(q_tile, q_base + q0 * 3LL * E, 3LL * E, T - q0, lane);
+    Tile::fill(g_tile, g_base + q0 * 1LL * E, E, T - q0, lane);
+  };
+  request(k0 / 32 + wave);
   float kf[HALF], vf[HALF];
   load_half_row<HALF>(q_base + E + key_load * 3LL * E + h * HALF, kf);
   load_half_row<HALF>(q_base + 2 * E + key_load * 3LL * E + h * HALF, vf);
@@ -219,14 +203,9 @@ f32_dkv_kernel(GenericBackwardArgs a) {
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
-  unsigned char* q_tile = lds + wave * kArea;
-  unsigned char* g_tile = q_tile + Tile::kBytes;
   const int query_tiles = (T + 31) / 32;
   for (int qt = k0 / 32 + wave; qt < query_tiles; qt += kWaves) {
     const int q0 = qt * 32;
-    wait_reads();  // of the tile before
-    Tile::fill(q_tile, q_base + q0 * 3LL * E, 3LL * E, T - q0, lane);
-    Tile::fill(g_tile, g_base + q0 * 1LL * E, E, T - q0, lane);
     if (h == 0) {
       const int row = min(q0 + n, T - 1);
       const float normalizer = a.normalizers[stats + row];
@@ -280,8 +259,10 @@ f32_dkv_kernel(GenericBackwardArgs a) {
         dk[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(Tile::element(q_tile, row, 32 * db + n), dp[i],
                                                       dk[db], 0, 0, 0);
       }
+    wait_reads();
+    if (qt + kWaves < query_tiles) request(qt + kWaves);
   }
-  wait_reads();
+  wait_fills();
   float4 own[8 * DB];
 #pragma unroll
   for (int g = 0; g < 4 * DB; ++g) {

@@ -8,7 +8,11 @@
 // maximum, sum and output, and wave 0 merges the four partial results through
 // LDS in wave order.  The FP32 matrix instruction is slow (64 cycles for
 // 32x32x2), a row block near the end of a sequence has many tiles and there
-// are few row blocks, so splitting the keys is what fills the machine.  As in
+// are few row blocks, so splitting the keys is what fills the machine; the row
+// blocks are handed out heaviest first, and a wave's tiles arrive in LDS while it
+// works on what is there.  Against lightest first with operands read from memory row
+// by row: 4 sequences x 12 heads x 256 x 64 19.4 -> 12.8 us, 2 x 12 x 1000 x 64
+// 75 -> 47, 2 x 6 x 1000 x 128 104 -> 50.  As in
 // the bf16 kernels the products are transposed,
 // S^T = K Q^T and O^T = V^T P^T, so that a lane owns one query column: its row
 // maximum and sum are lane-local up to one exchange between the two lane
@@ -18,6 +22,7 @@
 //        contiguous half row [h D/2, (h+1) D/2) of its key and of its query;
 //   O^T  step i contracts keys (8(i/4) + i%4, that + 4): exactly the keys
 //        accumulator register i holds in the two lane halves.
+#include "attn_f32_tile.h"
 #include "attn_generic.h"
 #include "mfma_tile.h"
 
@@ -27,14 +32,21 @@ namespace {
 constexpr int kKeySplit = 4;  // waves per workgroup, each taking every fourth key tile
 
 template <int D>
-__global__ void __launch_bounds__(64 * kKeySplit)
+__global__ void __launch_bounds__(64 * kKeySplit, D == 128 ? 1 : 2)
 f32_forward_kernel(GenericForwardArgs a) {
-  constexpr int HALF = D / 2, DB = D / 32;
-  __shared__ float part_o[kKeySplit - 1][DB * 16][64];
+  using Tile = F32Tile<D>;
+  constexpr int HALF = D / 2, DB = D / 32, kArea = 2 * Tile::kBytes, kFill = Tile::kFillOps;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kKeySplit * kArea];
+  // after the last tile: the partial results of waves 1 and up
+  auto part_o = reinterpret_cast<float(*)[DB * 16][64]>(lds);
+  static_assert((kKeySplit - 1) * DB * 16 * 64 * 4 <= kKeySplit * kArea);
   __shared__ float part_max[kKeySplit - 1][64], part_sum[kKeySplit - 1][64];
   const int lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
-  const int wave = threadIdx.x / 64;
-  const int q0 = blockIdx.x * 32, head = blockIdx.y, seq = blockIdx.z;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  // the row blocks that see the most keys first, of every (sequence, head)
+  const int q_tiles = (a.q_rows + 31) / 32, units = gridDim.x / q_tiles;
+  const int q0 = (q_tiles - 1 - static_cast<int>(blockIdx.x / units)) * 32;
+  const int head = (blockIdx.x % units) % a.query_heads, seq = (blockIdx.x % units) / a.query_heads;
   const int kv_head = head / a.group;
   const float* q_base = static_cast<const float*>(a.q.base) + seq * a.q.seq_stride +
                         head * a.q.head_stride;
@@ -46,15 +58,22 @@ f32_forward_kernel(GenericForwardArgs a) {
   const int query_load = min(query, a.q_rows - 1);
   const float scale2 = a.scale * kLog2e;
 
+  const int last_query = min(q0 + 32, a.q_rows) - 1;
+  const int visible_keys = min(a.kv_rows, a.start_position + last_query + 1);
+  const int key_tiles = (visible_keys + 31) / 32;
+  // K's tile is filled again as soon as the scores have been made and V's once it
+  // has been used, so that each has the other's products to arrive in.  The
+  // order of requests is K, V, K, V ...: waiting for one leaves the other on its way.
+  unsigned char* k_tile = lds + wave * kArea;
+  unsigned char* v_tile = k_tile + Tile::kBytes;
+  auto fill = [&](unsigned char* tile, const float* base, long long row_stride, int kt) {
+    const int k0 = kt < key_tiles ? kt * 32 : 0;
+    Tile::fill(tile, base + k0 * row_stride, row_stride, kt < key_tiles ? a.kv_rows - k0 : 0, lane);
+  };
+  fill(k_tile, k_base, a.k.row_stride, wave);
+  fill(v_tile, v_base, a.v.row_stride, wave);
   float qf[HALF];
-  {
-    const float4* row = reinterpret_cast<const float4*>(q_base + query_load * a.q.row_stride + h * HALF);
-#pragma unroll
-    for (int j = 0; j < HALF / 4; ++j) {
-      const float4 piece = row[j];
-      qf[4 * j] = piece.x; qf[4 * j + 1] = piece.y; qf[4 * j + 2] = piece.z; qf[4 * j + 3] = piece.w;
-    }
-  }
+  load_half_row<HALF>(q_base + query_load * a.q.row_stride + h * HALF, qf);
   floatx16 o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -62,47 +81,22 @@ f32_forward_kernel(GenericForwardArgs a) {
     for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
   float running_max = kMasked, running_sum = 0.0f;  // base-2 scaled scores
 
-  const int last_query = min(q0 + 32, a.q_rows) - 1;
-  const int visible_keys = min(a.kv_rows, a.start_position + last_query + 1);
-  const int key_tiles = (visible_keys + 31) / 32;
   const int my_last_key = a.start_position + query;  // keys beyond it are masked
-  // The key rows of a tile are requested one tile ahead and its value rows
-  // before its softmax: a wave runs alone on its SIMD, so nothing else hides
-  // the latency of these loads.
-  float4 k_next[HALF / 4];
-  {
-    const float4* row = reinterpret_cast<const float4*>(
-        k_base + min(wave * 32 + n, a.kv_rows - 1) * a.k.row_stride + h * HALF);
-#pragma unroll
-    for (int j = 0; j < HALF / 4; ++j) k_next[j] = row[j];
-  }
   for (int kt = wave; kt < key_tiles; kt += kKeySplit) {
-    float kf[HALF];
-#pragma unroll
-    for (int j = 0; j < HALF / 4; ++j) {
-      kf[4 * j] = k_next[j].x; kf[4 * j + 1] = k_next[j].y;
-      kf[4 * j + 2] = k_next[j].z; kf[4 * j + 3] = k_next[j].w;
-    }
-    if (kt + kKeySplit < key_tiles) {
-      const float4* row = reinterpret_cast<const float4*>(
-          k_base + min((kt + kKeySplit) * 32 + n, a.kv_rows - 1) * a.k.row_stride + h * HALF);
-#pragma unroll
-      for (int j = 0; j < HALF / 4; ++j) k_next[j] = row[j];
-    }
-    float values[DB][16];
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = min(kt * 32 + 8 * (i / 4) + 4 * h + (i % 4), a.kv_rows - 1);
-        values[db][i] = v_base[key * a.v.row_stride + 32 * db + n];
-      }
+    wait_fills<kFill>();  // K
     floatx16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < HALF; ++j)
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j], qf[j], s, 0, 0, 0);
+    for (int j = 0; j < HALF / 4; ++j) {
+      const float4 k4 = Tile::row_piece(k_tile, n, h * (HALF / 4) + j);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, qf[4 * j], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qf[4 * j + 1], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, qf[4 * j + 2], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[4 * j + 3], s, 0, 0, 0);
+    }
+    wait_reads();
+    fill(k_tile, k_base, a.k.row_stride, kt + kKeySplit);
     // register i = (key kt*32 + 8(i/4) + 4h + i%4, query n)
     float tile_max = kMasked;
 #pragma unroll
@@ -125,14 +119,21 @@ f32_forward_kernel(GenericForwardArgs a) {
     }
     running_sum = running_sum * correction + half_swap_sum(tile_sum);
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[db][i] *= correction;
+    wait_fills<kFill>();  // V
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(values[db][i], s[i], o[db], 0, 0, 0);
-    }
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+        o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+            Tile::element(v_tile, 8 * (i / 4) + 4 * h + (i % 4), 32 * db + n), s[i], o[db], 0, 0, 0);
+    wait_reads();
+    fill(v_tile, v_base, a.v.row_stride, kt + kKeySplit);
   }
+  wait_fills();
+  __syncthreads();  // every wave is done with its tiles
   // ---- merge: every wave's result is relative to its own maximum ------------
   if (wave > 0) {
     part_max[wave - 1][lane] = running_max;
@@ -204,6 +205,8 @@ bool f32_forward_supported(const GenericForwardArgs& a) {
       a.o_dtype != PLUTO_HIP_F32 || a.gate.base != nullptr)
     return false;
   if (a.q_rows <= 0 || a.kv_rows <= 0) return false;
+  // a tile's rows are addressed through 32-bit buffer offsets
+  if (32 * a.k.row_stride * 4 >= (1LL << 31) || 32 * a.v.row_stride * 4 >= (1LL << 31)) return false;
   auto mult4 = [](long long s) { return (s % 4) == 0; };
   return aligned16(a.q.base) && aligned16(a.k.base) && aligned16(a.v.base) && aligned16(a.out) &&
          mult4(a.q.seq_stride) && mult4(a.q.row_stride) && mult4(a.q.head_stride) &&
@@ -213,8 +216,9 @@ bool f32_forward_supported(const GenericForwardArgs& a) {
 }
 
 int launch_f32_forward(hipStream_t stream, const GenericForwardArgs& a, int sequences) {
-  const dim3 grid((a.q_rows + 31) / 32, a.query_heads, sequences);
-  if (grid.y > 65535u || grid.z > 65535u) return PLUTO_HIP_EUNSUPPORTED;
+  const long long blocks = (a.q_rows + 31LL) / 32 * a.query_heads * sequences;
+  if (blocks > 0x7fffffffLL) return PLUTO_HIP_EUNSUPPORTED;
+  const unsigned grid = static_cast<unsigned>(blocks);
   if (!kernel_enabled(kMainKernel)) return 0;
   switch (a.head_dim) {
     case 32: f32_forward_kernel<32><<<grid, 64 * kKeySplit, 0, stream>>>(a); break;
