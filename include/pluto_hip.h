@@ -280,11 +280,14 @@ int pluto_hip_gqa_prefill_probabilities(void* stream,
  *             be NULL), each fp32 [qh, positions[b] + 1]
  *             (AttentionProbabilitiesKernel, cached_attention_ops.cc:131-178)
  *   split_tokens: cache rows per split-K block: a multiple of 64 up to 512, or
- *             1024 at head width 256; 0 lets the library choose by the batch
- *             and its positions: 512 (1024 at head width 256), or less where
- *             such blocks would leave compute units idle.  Anything else is
+ *             1024 at head width 256; 0 lets the library choose for every
+ *             sequence by its own position, so that its result does not depend
+ *             on what else the batch holds.  Anything else is
  *             PLUTO_HIP_EINVAL, and the workspace size is then reported as 0.
- *             A workspace for given positions also serves smaller ones.
+ *             A workspace for given positions also serves smaller ones.  One
+ *             sized for 512 (1024 at head width 256) also serves a call with 0,
+ *             which takes blocks of that size if its own do not fit (the same
+ *             results up to the order of FP32 sums).
  * Returns PLUTO_HIP_ERANGE if any positions[b] >= capacity; nothing is
  * queued in that case. */
 size_t pluto_hip_gqa_decode_workspace_bytes(const pluto_hip_attention_params* p,
@@ -302,13 +305,14 @@ int pluto_hip_gqa_decode(void* stream, const pluto_hip_attention_params* p,
  * pass a workspace: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  No counterpart in the reference.  Same
  * arguments, results and errors as pluto_hip_gqa_decode (bit for bit), but the
- * scratch (prepared queries and split-K partial results) is a fixed array of
- * PLUTO_HIP_GQA_DECODE_STATIC_BYTES that the library keeps on every GPU it
- * runs on, and the call allocates nothing.  A call that would need more than
- * that (pluto_hip_gqa_decode_workspace_bytes says how much) returns
- * PLUTO_HIP_ELIMIT and queues nothing; the decode configuration (batch 32,
- * contexts up to 32768, 24 query heads of 128, 512-token blocks) needs about
- * 13 MiB.  All calls on one GPU share the array: calls that overlap there, on
+ * scratch (prepared queries and split-K partial results) is a fixed array
+ * that the library keeps on every GPU it runs on, and the call allocates
+ * nothing.  A call that would need more than PLUTO_HIP_GQA_DECODE_STATIC_BYTES
+ * (pluto_hip_gqa_decode_workspace_bytes says how much; split_tokens 0 counts
+ * as 512, or 1024 at head width 256, and the array has room for the smaller
+ * blocks it takes) returns PLUTO_HIP_ELIMIT and queues nothing; the decode
+ * configuration (batch 32, contexts up to 32768, 24 query heads of 128,
+ * 512-token blocks) needs about 13 MiB.  All calls on one GPU share the array: calls that overlap there, on
  * whatever streams, race on it.  pluto_hip_gqa_decode_static_prepare looks
  * the array's device address up for the calling thread's current device (the
  * entry point does it itself on its first call there).

@@ -42,6 +42,7 @@ struct DecodeBatch {
   void* keys[kDecodeBatchMax];
   void* values[kDecodeBatchMax];
   int block_start[kDecodeBatchMax + 1];  // prefix sum of split-K blocks
+  uint16_t split[kDecodeBatchMax];       // cache rows a block
 };
 
 struct DecodePrepareArgs {
@@ -72,6 +73,43 @@ constexpr bool decode_split_valid(int head_dim, int split) {
   return split >= 64 && split % 64 == 0 &&
          (split <= 512 || split == decode_split_default(head_dim));
 }
+// The block size of a sequence of `rows` rows where the caller leaves it to the
+// library.  It depends on nothing but the sequence itself, so that a sequence's result
+// does not change with the batch it is decoded in.  A block's rows are read one after
+// the other and a sequence's blocks are added up one after the other, so the best size
+// for a sequence alone grows with the square root of its length (head width 256: 128
+// rows at 777, 18 us against 35 in one block of 1024; 256 at 4096, 26 against 39), and
+// a full chip wants larger blocks, of which it starts fewer (32 sequences of 777 rows:
+// 45 us in blocks of 128, 42 of 192, 36 of 256).  8 sqrt(rows) at head width 256 and 10
+// sqrt(rows) below, to the nearest 64, lie between: batches of 1 to 32 with lengths
+// spread to 32768 take 3.5 % longer on average than with a size picked for the whole
+// batch, between 9 % less and 14 % more.  The default sizes have loops of their own: at the narrower widths they are faster
+// than anything from 320 up (64 sequences of 2048 rows at width 64: 27 us, 34 in blocks of
+// 448), at 256 beyond 16384 rows for all but a sequence or two.
+constexpr int decode_split_for(int head_dim, int rows) {
+  const long long factor = head_dim == 256 ? 8 : 10;
+  if (head_dim == 256 && rows > 16384) return decode_split_default(head_dim);
+  long long split = 64;
+  while (split < 512 && factor * factor * rows > (split + 32) * (split + 32)) split += 64;
+  return head_dim != 256 && split > 256 ? decode_split_default(head_dim) : static_cast<int>(split);
+}
+// The blocks of such a sequence.
+constexpr int decode_blocks_for(int head_dim, int rows) {
+  const int split = decode_split_for(head_dim, rows);
+  return static_cast<int>((static_cast<long long>(rows) + split - 1) / split);
+}
+// The most blocks a sequence of up to `rows` rows has: where the size steps up, the
+// blocks become fewer.
+constexpr int decode_blocks_up_to(int head_dim, int rows) {
+  int most = decode_blocks_for(head_dim, rows);
+  const int factor = head_dim == 256 ? 8 : 10;
+  for (int split = 64; split < 512; split += 64) {
+    const int last = (split + 32) * (split + 32) / (factor * factor);  // longest with this size
+    if (last < rows) most = most > decode_blocks_for(head_dim, last) ? most : decode_blocks_for(head_dim, last);
+  }
+  if (head_dim == 256 && rows > 16384) most = most > 32 ? most : 32;
+  return most;
+}
 
 // The fused decode step (preparation of the new token, split-K attention over
 // the cache, combine and gate in the workgroup that finishes a (sequence, kv
@@ -87,7 +125,6 @@ struct DecodeArgs {
   long long token_stride = 0, head_stride = 0;  // of the bf16 caches
   int query_heads = 0, key_value_heads = 0, head_dim = 0, rotary_dim = 0;
   float epsilon = 1e-6f;
-  int split_tokens = 512;
   float scale = 1.0f;
   // partial results of split-K block i (global index block_start[b] + j,
   // kv head g): o [block, kh, group, d], m and l [block, kh, group]

@@ -16,7 +16,11 @@
 // holds its own copy of the array until the process ends.  In host code the
 // array's name is only a handle for hipGetSymbolAddress: kernels and copies
 // take the per-device address kept in static_scratch_address.
-constexpr size_t kStaticScratchBytes = PLUTO_HIP_GQA_DECODE_STATIC_BYTES;
+// What a call may need is counted in blocks of the caller's size or the default's; with
+// block sizes of their own the sequences have up to five times as many (784 rows of
+// 256 channels: five of 192 instead of one of 1024), which with the queries is up to
+// (5 x 258 + 256) / (258 + 256) = 3.01 times the bytes.
+constexpr size_t kStaticScratchBytes = PLUTO_HIP_GQA_DECODE_STATIC_BYTES / 16 * 52;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace pluto_hip {
@@ -156,54 +160,36 @@ PrefillBackwardLayout prefill_backward_layout(const pluto_hip_attention_params* 
 }
 
 
-long long decode_blocks(int batch, const int* positions, int split) {
+// Whether a decode call that leaves the block size to the library gives every sequence
+// a size of its own: only the fused kernel reads the blocks, and it alone is faster
+// for them.  A call whose caches then turn out to need the any-shape kernels has room it
+// does not use.
+bool decode_own_sizes(const pluto_hip_attention_params* p, int split_tokens) {
+  return split_tokens == 0 && p->round_to_bfloat16 &&
+         decode_fast_supported(p->head_dim, p->query_heads / p->key_value_heads);
+}
+// The block size of one sequence; split_tokens as the caller gave it.
+int decode_split(const pluto_hip_attention_params* p, int position, int split_tokens) {
+  if (split_tokens != 0) return split_tokens;
+  return decode_own_sizes(p, split_tokens) ? decode_split_for(p->head_dim, position + 1)
+                                           : decode_split_default(p->head_dim);
+}
+long long decode_blocks(const pluto_hip_attention_params* p, int batch, const int* positions,
+                        int split_tokens) {
   long long blocks = 0;
-  for (int b = 0; b < batch; ++b) blocks += (static_cast<long long>(positions[b]) + split) / split;
+  for (int b = 0; b < batch; ++b) {
+    const int split = decode_split(p, positions[b], split_tokens);
+    blocks += (static_cast<long long>(positions[b]) + split) / split;
+  }
   return blocks;
 }
-
-// The block size of a call that leaves it to the library: of the default and its
-// halves the one whose estimated time is least.  What the estimate is made of was
-// fitted to calls of 1 to 32 sequences of 100 to 32000 rows: a workgroup takes a
-// fixed time whatever it does and some more for every 64 rows of its block; the
-// chip holds two (head width 256) or three a compute unit at once, and a call
-// takes as many rounds of them as it needs; the workgroup that ends a sequence
-// adds up its blocks.  (One sequence of 777 rows at width 256: 34 us with one block
-// of 1024 rows, 18 with blocks of 128.)  Sizes below the default are taken only
-// up to two rounds, which bounds the scratch such a call needs.
-long long decode_resident(int head_dim) { return head_dim == 256 ? 512 : 768; }
-int decode_split(const pluto_hip_attention_params* p, int batch, const int* positions,
-                 int split_tokens) {
-  if (split_tokens != 0) return split_tokens;
-  const bool wide = p->head_dim == 256;
-  const double fixed = wide ? 12.0 : 11.0, rows64 = wide ? 1.2 : 0.45, combine = wide ? 0.25 : 0.19;
-  const long long resident = decode_resident(p->head_dim);
-  const int standard = decode_split_default(p->head_dim);
-  int longest = 0;
-  for (int b = 0; b < batch; ++b) longest = positions[b] > longest ? positions[b] : longest;
-  int best = standard;
-  double least = 0.0;
-  for (int split = standard; split >= 64; split /= 2) {
-    const long long workgroups = decode_blocks(batch, positions, split) * p->key_value_heads;
-    if (split < standard && workgroups > 2 * resident) break;
-    const double rounds = static_cast<double>((workgroups + resident - 1) / resident);
-    const double estimate = rounds * (fixed + rows64 * (split / 64)) +
-                            combine * static_cast<double>(longest / split + 1);
-    if (split == standard || estimate < least) {
-      best = split;
-      least = estimate;
-    }
-  }
-  return best;
-}
-// An upper bound of the blocks of such a call that also holds for every call at
-// smaller positions.
+// The most blocks of a call at these or smaller positions.
 long long decode_blocks_bound(const pluto_hip_attention_params* p, int batch, const int* positions,
                               int split_tokens) {
-  if (split_tokens != 0) return decode_blocks(batch, positions, split_tokens);
-  const long long standard = decode_blocks(batch, positions, decode_split_default(p->head_dim));
-  const long long smaller = 2 * decode_resident(p->head_dim) / p->key_value_heads;
-  return standard > smaller ? standard : smaller;
+  if (!decode_own_sizes(p, split_tokens)) return decode_blocks(p, batch, positions, split_tokens);
+  long long blocks = 0;
+  for (int b = 0; b < batch; ++b) blocks += decode_blocks_up_to(p->head_dim, positions[b] + 1);
+  return blocks;
 }
 
 // What the forward pass can leave for the backward pass: the attention output
@@ -619,7 +605,7 @@ static int decode_run(void* stream, const pluto_hip_attention_params* p, int bat
                       const void* q_gate, const void* k, const void* v, const float* q_norm,
                       const float* k_norm, const int* positions,
                       const pluto_hip_kv_cache_view* caches, void* out,
-                      float* const* probabilities, int split, void* workspace,
+                      float* const* probabilities, int split_tokens, void* workspace,
                       const DecodeLayout& layout, bool clear_arrivals);
 
 int pluto_hip_gqa_decode(void* stream, const pluto_hip_attention_params* p, int batch,
@@ -631,17 +617,23 @@ int pluto_hip_gqa_decode(void* stream, const pluto_hip_attention_params* p, int 
   const int status = decode_check(p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions,
                                   caches, out, split_tokens);
   if (status != 0) return status;
-  const int split = decode_split(p, batch, positions, split_tokens);
-  const DecodeLayout layout =
-      decode_layout(p, batch, decode_blocks(batch, positions, split),
-                    static_cast<size_t>(batch) * p->key_value_heads * sizeof(unsigned));
+  auto layout_of = [&](int split) {
+    return decode_layout(p, batch, decode_blocks(p, batch, positions, split),
+                         static_cast<size_t>(batch) * p->key_value_heads * sizeof(unsigned));
+  };
+  DecodeLayout layout = layout_of(split_tokens);
+  if (split_tokens == 0 && workspace_bytes < layout.total) {
+    // room for blocks of the default size at least
+    split_tokens = decode_split_default(p->head_dim);
+    layout = layout_of(split_tokens);
+  }
   if (!workspace || workspace_bytes < layout.total) return PLUTO_HIP_EWORKSPACE;
   // whatever the workspace held: the counters are cleared by a launch of their own
   return decode_run(stream, p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions, caches,
-                    out, probabilities, split, workspace, layout, true);
+                    out, probabilities, split_tokens, workspace, layout, true);
 }
 
-size_t pluto_hip_gqa_decode_static_bytes(void) { return kStaticScratchBytes; }
+size_t pluto_hip_gqa_decode_static_bytes(void) { return PLUTO_HIP_GQA_DECODE_STATIC_BYTES; }
 
 int pluto_hip_gqa_decode_static_prepare(void) {
   void* address = nullptr;
@@ -656,12 +648,16 @@ int pluto_hip_gqa_decode_static(void* stream, const pluto_hip_attention_params* 
   int status = decode_check(p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions, caches,
                             out, split_tokens);
   if (status != 0) return status;
-  const int split = decode_split(p, batch, positions, split_tokens);
   if (static_cast<size_t>(batch) * p->key_value_heads * sizeof(unsigned) > kStaticArrivalBytes)
     return PLUTO_HIP_ELIMIT;
-  const DecodeLayout layout =
-      decode_layout(p, batch, decode_blocks(batch, positions, split), kStaticArrivalBytes);
-  if (layout.total > kStaticScratchBytes) return PLUTO_HIP_ELIMIT;
+  auto layout_of = [&](int split) {
+    return decode_layout(p, batch, decode_blocks(p, batch, positions, split), kStaticArrivalBytes);
+  };
+  const int counted = split_tokens != 0 ? split_tokens : decode_split_default(p->head_dim);
+  const DecodeLayout layout = layout_of(split_tokens);
+  if (layout_of(counted).total > PLUTO_HIP_GQA_DECODE_STATIC_BYTES ||
+      layout.total > kStaticScratchBytes)
+    return PLUTO_HIP_ELIMIT;
   void* address = nullptr;
   int device = 0;
   status = static_scratch(&address, &device);
@@ -680,7 +676,7 @@ int pluto_hip_gqa_decode_static(void* stream, const pluto_hip_attention_params* 
     }
   }
   status = decode_run(stream, p, batch, io_dtype, q_gate, k, v, q_norm, k_norm, positions, caches,
-                      out, probabilities, split, address, layout, false);
+                      out, probabilities, split_tokens, address, layout, false);
   if (status != 0) static_scratch_dirty[device].store(true, std::memory_order_release);
   return status;
 }
@@ -702,7 +698,7 @@ static int decode_run(void* stream, const pluto_hip_attention_params* p, int bat
                       const void* q_gate, const void* k, const void* v, const float* q_norm,
                       const float* k_norm, const int* positions,
                       const pluto_hip_kv_cache_view* caches, void* out,
-                      float* const* probabilities, int split, void* workspace,
+                      float* const* probabilities, int split_tokens, void* workspace,
                       const DecodeLayout& layout, bool clear_arrivals) {
   int status = 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -751,7 +747,10 @@ static int decode_run(void* stream, const pluto_hip_attention_params* p, int bat
       slice.positions[i] = positions[b];
       slice.keys[i] = caches[b].keys;
       slice.values[i] = caches[b].values;
-      slice.block_start[i + 1] = slice.block_start[i] + (positions[b] + split) / split;
+      const int split = decode_split(p, positions[b], split_tokens);
+      slice.split[i] = static_cast<uint16_t>(split);
+      slice.block_start[i + 1] =
+          slice.block_start[i] + static_cast<int>((static_cast<long long>(positions[b]) + split) / split);
     }
     if (!fast || probabilities) {
       // the any-shape kernels and the probabilities pass read prepared queries
@@ -795,7 +794,6 @@ static int decode_run(void* stream, const pluto_hip_attention_params* p, int bat
       a.head_dim = d;
       a.rotary_dim = p->rotary_dim;
       a.epsilon = p->rms_norm_epsilon;
-      a.split_tokens = split;
       a.scale = scale;
       a.part_o = reinterpret_cast<float*>(area + layout.part_o);
       a.part_m = reinterpret_cast<float*>(area + layout.part_m);

@@ -4,7 +4,7 @@
 // Semantics: CachedAttentionStep (src/llm/layers/util/cached_attention_ops.cc:
 // 308-353: PrepareAttentionKernel :30-79, FullAttentionKernel :83-126) for
 // every sequence of the batch.  One workgroup owns one (sequence, kv head,
-// block of `split_tokens` cache rows) and serves ALL query heads of the group,
+// block of the sequence's `split` cache rows) and serves ALL query heads of the group,
 // so every K and V byte is read from HBM exactly once (the reference launches
 // one program per query head and streams the cache once per head of the
 // group).
@@ -629,14 +629,15 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
   ctx.seq = seq;
   ctx.position = batch.positions[b];
   ctx.length = ctx.position + 1;
-  ctx.t0 = j * a.split_tokens;
-  ctx.per_wave = a.split_tokens / 4;
+  const int split = batch.split[b];
+  ctx.t0 = j * split;
+  ctx.per_wave = split / 4;
   ctx.keys = static_cast<uint16_t*>(batch.keys[b]) + g * a.head_stride;
   ctx.values = static_cast<uint16_t*>(batch.values[b]) + g * a.head_stride;
   ctx.slot = (a.block_base + block) * kh + g;
   const bool is_last = j == blocks_here - 1;  // this block holds row `position`
   constexpr int kFixed = decode_split_default(D);
-  if (a.split_tokens == kFixed) {
+  if (split == kFixed) {
     if (is_last)
       decode_block<D, GROUP, kFixed, true>(a, ctx, value_area, wave_max, wave_sum_lds, q_lds, new_row);
     else
@@ -846,7 +847,8 @@ int launch_decode_fast(hipStream_t stream, const DecodeArgs& a, const DecodeBatc
   const long long blocks =
       static_cast<long long>(batch.block_start[batch.count]) * a.key_value_heads;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return PLUTO_HIP_EINVAL;
-  if (!decode_split_valid(a.head_dim, a.split_tokens)) return PLUTO_HIP_EINVAL;
+  for (int i = 0; i < batch.count; ++i)
+    if (!decode_split_valid(a.head_dim, batch.split[i])) return PLUTO_HIP_EINVAL;
   if (a.rotary_dim / 2 > 128) return PLUTO_HIP_EUNSUPPORTED;
   if (!kernel_enabled(kMainKernel)) return 0;
   switch (a.head_dim) {

@@ -403,7 +403,7 @@ def test_config4_batched_decode(capi, oracle, d, rotary, split):
     # batch 32, context length ~ U[1024, 32768] (seed 3), 24 query heads, 4 KV
     # heads, D=128, bf16 cache, split-K over 512-token blocks; and the same
     # batch at the model's own head width (cached_attention_ops.h:13-22: 256,
-    # 64 rotated channels) with the default blocks of 1024 rows.
+    # 64 rotated channels) with the block sizes the library picks a sequence.
     batch, qh, kh, capacity = 32, 24, 4, 32768
     kw = dict(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=rotary, capacity=capacity)
     p, po = both_params(capi, oracle, **kw)
@@ -457,14 +457,14 @@ def test_config4_batched_decode(capi, oracle, d, rotary, split):
 
 @pytest.mark.parametrize("d,qh,kh,rotary,split", [
     (256, 12, 2, 64, 0), (256, 12, 2, 64, 1024), (256, 12, 2, 64, 512), (256, 12, 2, 64, 192),
-    (256, 8, 1, 256, 0), (64, 8, 2, 16, 0), (64, 2, 2, 64, 512), (64, 4, 2, 32, 320),
+    (256, 8, 1, 256, 0), (256, 8, 1, 256, 1024), (64, 8, 2, 16, 0), (64, 2, 2, 64, 512), (64, 4, 2, 32, 320),
     (128, 8, 1, 32, 0), (128, 4, 4, 128, 0)])
 def test_batched_decode_block_sizes_and_head_widths(capi, oracle, d, qh, kh, rotary, split):
     # cached_attention_ops.h:13-22: the model's heads are 256 wide with 64
     # rotated channels.  The fused kernel is specialised for blocks of 1024
-    # cache rows there and of 512 at the narrower widths (the defaults, split
-    # 0), with a request order fixed at compile time, and takes any other
-    # multiple of 64 up to 512 with its run-time loops; groups of 1, 2, 4, 6
+    # cache rows there and of 512 at the narrower widths, with a request order
+    # fixed at compile time, and takes any other multiple of 64 up to 512 with
+    # its run-time loops (split 0: each sequence its own size); groups of 1, 2, 4, 6
     # and 8 query heads; lengths on both sides of the block boundaries.
     capacity = 5120
     kw = dict(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=rotary, capacity=capacity)
@@ -535,6 +535,47 @@ def test_decode_block_size_chosen_by_the_library(capi, d, batch):
         want = capi.gqa_decode(p, q_gate, k, v, w, w, caches, positions=positions, split_tokens=512,
                                advance=False).float()
         assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-4), length
+
+
+@pytest.mark.parametrize("d,batch", [(64, 70), (128, 40), (256, 40)])
+def test_a_sequence_decodes_alone_as_in_any_batch(capi, d, batch):
+    """With the block sizes left to the library a sequence's result has the same bits
+    whatever else is decoded beside it.  A workspace that only holds blocks of the
+    default size still serves the call, with the bits those blocks give."""
+    qh, kh, longest = 12, 2, 18000 if d == 256 else 5000
+    default = 1024 if d == 256 else 512
+    p = capi.attention_params(qh, kh, d, 32, capacity=longest)
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    rng = np.random.default_rng(d)
+    bf = torch.bfloat16
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(bf)
+    lengths = [777, 1, 64, 145, 400, 401, 784, 785, 1024, 1300, longest]
+    lengths += [int(n) for n in rng.integers(1, 2500, batch - len(lengths))]
+    positions = [n - 1 for n in lengths]
+    q_gate, k, v = values(batch, qh, 2, d), values(batch, kh, d), values(batch, kh, d)
+    w = torch.zeros(d, device="cuda")
+    shared = (values(kh, longest, d), values(kh, longest, d))
+    caches = []
+    for _ in range(batch):
+        c = capi.KvCache(longest, kh, d)
+        c.keys.copy_(shared[0])
+        c.values.copy_(shared[1])
+        caches.append(c)
+
+    def decode(which, **kw):
+        index = torch.tensor(which, device="cuda")
+        return capi.gqa_decode(p, q_gate[index], k[index], v[index], w, w, [caches[i] for i in which],
+                               positions=[positions[i] for i in which], advance=False, **kw)
+
+    everyone = list(range(batch))
+    together = decode(everyone)
+    assert capi.last_path() == capi.PATH_SPLIT_K
+    for some in ([0], [10], [0, 10], list(range(11)), everyone[5:]):
+        assert torch.equal(decode(some), together[torch.tensor(some, device="cuda")]), some
+    small = capi.gqa_decode_workspace(p, positions, default)
+    assert small.numel() < capi.gqa_decode_workspace(p, positions).numel()
+    assert torch.equal(decode(everyone, workspace=small), decode(everyone, split_tokens=default))
 
 
 def test_decode_more_than_one_launch_slice(capi, oracle):

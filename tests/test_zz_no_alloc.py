@@ -173,3 +173,37 @@ def test_rejects_what_does_not_fit(capi):
     assert b"fixed scratch" in handle.pluto_hip_error_string(capi.ELIMIT)
     torch.cuda.synchronize()
     assert (out == 7.0).all()
+
+
+@pytest.mark.parametrize("batch,qh,kh,d,length", [(32, 32, 1, 256, 4096), (32, 12, 1, 64, 5000),
+                                                  (330, 24, 4, 256, 777), (300, 24, 4, 128, 900)])
+def test_the_limit_is_counted_in_default_blocks(capi, batch, qh, kh, d, length):
+    """Block sizes left to the library do not narrow what the fixed scratch takes: heads
+    that share a kv head twelve or thirty-two at a time (any-shape kernels), and sequences that
+    just fit in default blocks and take more of their own size.  The results are
+    those of the workspace entry point, bit for bit."""
+    p = capi.attention_params(qh, kh, d, 32, capacity=length)
+    gen = torch.Generator(device="cuda").manual_seed(batch + d)
+    bf = torch.bfloat16
+    def draw(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(bf)
+    # a few caches stand in for all: every sequence of a cache appends the same row to it
+    made = [capi.KvCache(length, kh, d) for _ in range(4)]
+    for c in made:
+        c.keys.copy_(draw(kh, length, d))
+        c.values.copy_(draw(kh, length, d))
+    q_gate = draw(batch, qh, 2, d)
+    k, v = draw(4, kh, d).repeat(batch // 4 + 1, 1, 1)[:batch].contiguous(), draw(1, kh, d).repeat(batch, 1, 1)
+    w = torch.zeros(d, device="cuda")
+    caches = [made[i % 4] for i in range(batch)]
+    positions = [length - 1] * batch
+    pos = (ctypes.c_int * batch)(*positions)
+    default = 1024 if d == 256 else 512
+    needed = capi.lib().pluto_hip_gqa_decode_workspace_bytes(ctypes.byref(p), batch, pos, default)
+    assert needed < capi.lib().pluto_hip_gqa_decode_static_bytes()
+    want = capi.gqa_decode(p, q_gate, k, v, w, w, caches, positions=positions, advance=False)
+    got = torch.full_like(want, float("nan"))
+    capi.gqa_decode_static(p, q_gate, k, v, w, w, caches, positions, got)
+    torch.cuda.synchronize()
+    assert torch.isfinite(want.float()).all()
+    assert torch.equal(got, want)
