@@ -206,6 +206,12 @@ int pluto_hip_attention_params_validate(const pluto_hip_attention_params* p);
  *        qwen_attention.cc:445-447, without its quadratic tensors).  Only for
  *        start_position 0 and where that size is not 0: round_to_bfloat16, a
  *        BF16 cache and head_dim 64 or 128; PLUTO_HIP_EUNSUPPORTED otherwise.
+ *   workspace  pluto_hip_gqa_prefill_workspace_bytes(...) bytes.  Where `length`
+ *        is at most half of the capacity (head_dim 128 and 256,
+ *        round_to_bfloat16) that includes room for sharing the keys of a query
+ *        tile out to several workgroups; a workspace that ends before that
+ *        room is accepted too, and the call then does without (the same
+ *        results up to the order of FP32 sums).
  * The quadratic probability tensor of the reference is not produced. */
 size_t pluto_hip_gqa_prefill_workspace_bytes(const pluto_hip_attention_params* p,
                                              int length);

@@ -345,14 +345,14 @@ def gqa_prefill(p, qg, k, v, q_norm, k_norm, cache, start_position=0, want_lse=F
         out = torch.empty((T, p.query_heads, p.head_dim), dtype=torch.bfloat16, device=qg.device)
     lse = (torch.empty((T, p.query_heads), dtype=torch.float32, device=qg.device)
            if want_lse else None)
-    size = lib().pluto_hip_gqa_prefill_workspace_bytes(ctypes.byref(p), T)
     if workspace is None:
+        size = lib().pluto_hip_gqa_prefill_workspace_bytes(ctypes.byref(p), T)
         workspace = torch.empty(max(size, 1), dtype=torch.uint8, device=qg.device)
     view = cache.view()
     check(lib().pluto_hip_gqa_prefill(stream or current_stream(), ctypes.byref(p), T,
                                       start_position, ptr(qg), ptr(k), ptr(v), ptr(q_norm),
                                       ptr(k_norm), ctypes.byref(view), ptr(out), ptr(lse),
-                                      ptr(saved), ptr(workspace), size))
+                                      ptr(saved), ptr(workspace), workspace.numel()))
     cache.position = start_position + T
     result = (out, lse) if want_lse else out
     if want_probabilities:
@@ -360,7 +360,7 @@ def gqa_prefill(p, qg, k, v, q_norm, k_norm, cache, start_position=0, want_lse=F
                                     device=qg.device)
         check(lib().pluto_hip_gqa_prefill_probabilities(
             stream or current_stream(), ctypes.byref(p), T, start_position, ctypes.byref(view),
-            ptr(workspace), size, ptr(probabilities)))
+            ptr(workspace), workspace.numel(), ptr(probabilities)))
         result = (result + (probabilities,)) if want_lse else (result, probabilities)
     return result
 

@@ -35,7 +35,7 @@ struct FlashForwardArgs {
 
 // Scratch for the partial results of any call with these rows and at most kv_rows
 // keys; 0: never split.
-size_t flash_forward_split_bytes(int head_dim, int q_rows, int kv_rows);
+size_t flash_forward_split_bytes(int head_dim, int q_rows, int kv_rows, int query_heads, int group);
 
 bool flash_forward_supported(const FlashForwardArgs& args, int head_dim);
 int launch_flash_forward(hipStream_t stream, const FlashForwardArgs& args,

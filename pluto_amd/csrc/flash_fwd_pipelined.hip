@@ -836,16 +836,24 @@ bool share_out(const std::vector<int>& cost, const std::vector<int>& order, int 
   return true;
 }
 
+int split_partitions(int kv_heads) {
+  return kv_heads % 8 == 0 ? 8 : 8 % kv_heads == 0 ? kv_heads : 1;
+}
+// Tiles of a partition.
+long long split_items(int q_rows, int tile_rows, int query_heads, int group) {
+  return 1LL * ((q_rows + tile_rows - 1) / tile_rows) * query_heads / split_partitions(query_heads / group);
+}
+// Rows that are more than half of the keys have light tiles that fill the gaps the
+// heavy ones leave, and their results stay those of the other kernels to the bit.
+bool split_rows(int q_rows, int kv_rows) { return q_rows <= kv_rows / 2; }
+
 void build_split(const ScheduleKey& k, SplitPlan* plan) {
   plan->useful = false;
   const int q_tiles = (k.q_rows + k.tile_rows - 1) / k.tile_rows;
-  const int kv_heads = k.query_heads / k.group;
-  // Rows that are more than half of the keys have light tiles that fill the gaps the
-  // heavy ones leave, and their results stay those of the other kernels to the bit.
-  if (k.workgroups != kSplitLists || k.kv_rows > BN * 0xffff || k.q_rows > k.kv_rows / 2) return;
-  const int partitions = kv_heads % 8 == 0 ? 8 : 8 % kv_heads == 0 ? kv_heads : 1;
+  if (k.workgroups != kSplitLists || k.kv_rows > BN * 0xffff || !split_rows(k.q_rows, k.kv_rows)) return;
+  const int partitions = split_partitions(k.query_heads / k.group);
   const int lists = kSplitLists / partitions;
-  const long long items = 1LL * q_tiles * k.query_heads / partitions;
+  const long long items = split_items(k.q_rows, k.tile_rows, k.query_heads, k.group);
   if (items > kSplitEntries) return;
   std::vector<int> cost(items), order(items);
   long long total = 0;
@@ -878,9 +886,11 @@ void build_split(const ScheduleKey& k, SplitPlan* plan) {
 
 }  // namespace
 
-size_t flash_forward_split_bytes(int head_dim, int q_rows, int kv_rows) {
+size_t flash_forward_split_bytes(int head_dim, int q_rows, int kv_rows, int query_heads, int group) {
   if ((head_dim != 128 && head_dim != 256) || kv_rows < 2 * kShortestPart * BN) return 0;
   const int tile_rows = 32 * (head_dim == 256 ? kWaves<256> : kWaves<128>);
+  if (!split_rows(q_rows, kv_rows) || split_items(q_rows, tile_rows, query_heads, group) > kSplitEntries)
+    return 0;
   return 1ull * kSplitEntries * std::min(tile_rows, q_rows) * (head_dim + 2) * 4;
 }
 

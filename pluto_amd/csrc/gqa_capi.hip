@@ -86,6 +86,8 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 size_t element_bytes(int dtype) { return dtype == PLUTO_HIP_BF16 ? 2 : 4; }
 
+// The partial results come last: a workspace that ends before them serves a call whose
+// keys are then not shared out in parts.
 struct PrefillLayout {
   size_t cosines, sines, queries, partial, partial_bytes, total;
 };
@@ -100,8 +102,10 @@ PrefillLayout prefill_layout(const pluto_hip_attention_params* p, int length) {
                                        (p->round_to_bfloat16 ? 2 : 4),
                                    256);
   // whatever the start position: a sequence has at most `capacity` keys
-  l.partial_bytes =
-      p->round_to_bfloat16 ? flash_forward_split_bytes(p->head_dim, length, p->capacity) : 0;
+  l.partial_bytes = p->round_to_bfloat16
+                        ? flash_forward_split_bytes(p->head_dim, length, p->capacity, p->query_heads,
+                                                    p->query_heads / p->key_value_heads)
+                        : 0;
   l.total = l.partial + align_up(l.partial_bytes, 256);
   return l;
 }
@@ -251,7 +255,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   if (saved && (start_position != 0 || !saved_supported(p, cache->dtype)))
     return PLUTO_HIP_EUNSUPPORTED;
   const PrefillLayout layout = prefill_layout(p, length);
-  if (!workspace || workspace_bytes < layout.total) return PLUTO_HIP_EWORKSPACE;
+  if (!workspace || workspace_bytes < layout.partial) return PLUTO_HIP_EWORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   char* scratch = static_cast<char*>(workspace);
   float* cosines = reinterpret_cast<float*>(scratch + layout.cosines);
@@ -314,7 +318,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
     f.query_heads = qh;
     f.group = qh / kh;
     f.scale = scale;
-    if (layout.partial_bytes > 0) f.partial = scratch + layout.partial;
+    if (layout.partial_bytes > 0 && workspace_bytes >= layout.total) f.partial = scratch + layout.partial;
     if (flash_forward_supported(f, d)) {
       note_path(PLUTO_HIP_PATH_FLASH);
       return launch_flash_forward(s, f, d, 1);
@@ -517,7 +521,7 @@ int pluto_hip_gqa_prefill_probabilities(void* stream, const pluto_hip_attention_
   if (status != 0) return status;
   if (static_cast<long long>(start_position) + length > p->capacity) return PLUTO_HIP_ERANGE;
   const PrefillLayout layout = prefill_layout(p, length);
-  if (!workspace || workspace_bytes < layout.total) return PLUTO_HIP_EWORKSPACE;
+  if (!workspace || workspace_bytes < layout.partial) return PLUTO_HIP_EWORKSPACE;
   const CacheView view{cache->keys, cache->values, cache->dtype, cache->token_stride,
                        cache->head_stride};
   const float scale = 1.0f / std::sqrt(static_cast<float>(p->head_dim));

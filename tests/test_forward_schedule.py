@@ -111,3 +111,25 @@ def test_rejections(library):
     assert call(96, 100, 100, 0, 4, 1, 1, 256, items, 4, ctypes.byref(w), ctypes.byref(s)) == capi.EINVAL
     assert call(128, 100, 100, 0, 4, 3, 1, 256, items, 4, ctypes.byref(w), ctypes.byref(s)) == capi.EINVAL
     assert call(128, 8192, 8192, 0, 24, 6, 1, 256, items, 4, ctypes.byref(w), ctypes.byref(s)) == capi.ELIMIT
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+def test_the_prefill_workspace_has_room_for_parts_only_where_tiles_are_split(library, head_dim):
+    """Angles and queries, and behind them the partial results of tiles whose keys are
+    shared out: never for rows that are more than half of the keys a sequence can have,
+    nor for more tiles than the lists hold."""
+    def aligned(n):
+        return -(-n // 256) * 256
+    rotary, heads, kv_heads = 32, 24, 4
+    def parts(length, capacity):
+        p = capi.attention_params(heads, kv_heads, head_dim, rotary, capacity=capacity)
+        base = 2 * aligned(length * rotary // 2 * 4) + aligned(length * heads * head_dim * 2)
+        return library.pluto_hip_gqa_prefill_workspace_bytes(ctypes.byref(p), length) - base
+    for length, capacity in [(8192, 8192), (1024, 1024), (1024, 2047), (513, 1025), (20, 1000), (20, 20),
+                             (20000, 200000)]:
+        assert parts(length, capacity) == 0, (length, capacity)
+    for length, capacity in [(1024, 2048), (20, 1024), (1531, 3840)]:
+        # at most 384 parts, each a tile's rows of outputs and two numbers a row
+        rows = min(length, tile_rows(head_dim))
+        want = 0 if head_dim == 64 else aligned(384 * rows * (head_dim + 2) * 4)
+        assert parts(length, capacity) == want, (length, capacity)

@@ -537,6 +537,41 @@ def test_decode_block_size_chosen_by_the_library(capi, d, batch):
         assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-4), length
 
 
+@pytest.mark.parametrize("d,rows,start", [(256, 34, 7336), (128, 61, 4000)])
+def test_prefill_without_room_for_parts(capi, d, rows, start):
+    """A workspace that ends before the partial results is accepted: the call does not
+    share keys out then, writes nothing behind the workspace, and agrees with the call that
+    does to the order of FP32 sums; probabilities only need the queries either."""
+    qh, kh = 24, 4
+    p = capi.attention_params(qh, kh, d, 32, capacity=start + rows)
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    bf = torch.bfloat16
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(bf)
+    qg, k, v = values(rows, qh, 2, d), values(rows, kh, d), values(rows, kh, d)
+    w = torch.zeros(d, device="cuda")
+    cache = capi.KvCache(start + rows, kh, d)
+    cache.keys.copy_(values(*cache.keys.shape))
+    cache.values.copy_(values(*cache.values.shape))
+    whole = capi.gqa_prefill(p, qg, k, v, w, w, cache, start_position=start)
+    # angles and queries, each rounded up to 256 bytes
+    base = 2 * (-(-rows * 16 * 4 // 256) * 256) + rows * qh * d * 2
+    assert base % 256 == 0
+    import ctypes
+    assert base < capi.lib().pluto_hip_gqa_prefill_workspace_bytes(ctypes.byref(p), rows)
+    space = torch.full((base + (1 << 16),), 0x5a, dtype=torch.uint8, device="cuda")
+    out, probabilities = capi.gqa_prefill(p, qg, k, v, w, w, cache, start_position=start,
+                                          workspace=space[:base], want_probabilities=True)
+    torch.cuda.synchronize()
+    assert torch.all(space[base:] == 0x5a)
+    difference = (out.float() - whole.float()).abs()
+    assert torch.all(difference <= 2.0 ** -7 * whole.float().abs() + 1e-4)
+    np.testing.assert_allclose(probabilities.double().sum(-1).cpu().numpy(), 1.0, atol=1e-5)
+    with pytest.raises(capi.PlutoHipError) as info:
+        capi.gqa_prefill(p, qg, k, v, w, w, cache, start_position=start, workspace=space[:base - 256])
+    assert info.value.code == capi.EWORKSPACE
+
+
 @pytest.mark.parametrize("d,batch", [(64, 70), (128, 40), (256, 40)])
 def test_a_sequence_decodes_alone_as_in_any_batch(capi, d, batch):
     """With the block sizes left to the library a sequence's result has the same bits
