@@ -541,7 +541,7 @@ def test_decode_block_size_chosen_by_the_library(capi, d, batch):
 def test_prefill_without_room_for_parts(capi, d, rows, start):
     """A workspace that ends before the partial results is accepted: the call does not
     share keys out then, writes nothing behind the workspace, and agrees with the call that
-    does to the order of FP32 sums; probabilities only need the queries either."""
+    does; probabilities only need the queries either."""
     qh, kh = 24, 4
     p = capi.attention_params(qh, kh, d, 32, capacity=start + rows)
     gen = torch.Generator(device="cuda").manual_seed(d)
@@ -564,8 +564,13 @@ def test_prefill_without_room_for_parts(capi, d, rows, start):
                                           workspace=space[:base], want_probabilities=True)
     torch.cuda.synchronize()
     assert torch.all(space[base:] == 0x5a)
-    difference = (out.float() - whole.float()).abs()
-    assert torch.all(difference <= 2.0 ** -7 * whole.float().abs() + 1e-4)
+    # The two round the same probabilities to bf16 against different references, and then
+    # the outputs: independent errors of at most 2^-9 relative, 2^-9 / sqrt(3) root mean square.
+    # A sum of n terms p v with such errors in p is off by that much of sqrt(sum p^2 v^2),
+    # which is its own size for values of mean zero; so 2^-9 / sqrt(3) for the probabilities
+    # and as much for the output, of each call: 2.3e-3 of the norm in all, and twice that allowed.
+    difference = (out.float() - whole.float()).norm() / whole.float().norm()
+    assert difference <= 4.6e-3
     np.testing.assert_allclose(probabilities.double().sum(-1).cpu().numpy(), 1.0, atol=1e-5)
     with pytest.raises(capi.PlutoHipError) as info:
         capi.gqa_prefill(p, qg, k, v, w, w, cache, start_position=start, workspace=space[:base - 256])
