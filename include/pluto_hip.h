@@ -515,7 +515,8 @@ int pluto_hip_dense_backward(void* stream, int dtype, const void* input,
  * [ceil(output_dim/128), ceil(input_dim/128)], times ONE bf16 token
  * [input_dim] -> bf16 [output_dim].  All arithmetic is FP32.  With FP8 weights
  * the token is quantized first, in independent groups of 128 elements:
- * scale = max|x| / 448, x -> fp8(x / max(scale, 1e-12)) * scale.  `scales`
+ * scale = max|x| / 448, x -> fp8(x / max(scale, 1e-12)) * scale; a token with
+ * a NaN or an infinity gives NaN in every output.  `scales`
  * must be non-NULL exactly for FP8 storage; dimensions in [1, 1048576] (:271).
  * workspace: pluto_hip_dense_imported_workspace_bytes(input_dim) bytes. */
 #define PLUTO_HIP_MATRIX_BF16 0

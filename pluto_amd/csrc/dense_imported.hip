@@ -40,11 +40,15 @@ __device__ inline float fp8_value(uint32_t bits) {
 // group's reciprocal with one correction step, which rounds as the division
 // does, and the rounding is the hardware conversion: six instructions a value
 // where a divide and a rounding by parts took sixty, 9 us of a one-token
-// projection whose workgroups each prepare the token.
+// projection whose workgroups each prepare the token.  The largest magnitude comes as
+// the bits of its bf16 value, of which a maximum keeps a NaN where that of floats loses
+// it.  A group with a NaN or an infinity makes every sum it enters NaN (fp8(NaN) is NaN
+// and fp8(v / inf) * inf is 0 * inf or NaN); its scale says so for all of its values,
+// and the quotients, which the clamp keeps finite, need not be looked at.
 struct GroupQuantizer {
   float scale, divisor, inverse;
-  __device__ explicit GroupQuantizer(float largest) {
-    scale = largest / 448.0f;
+  __device__ explicit GroupQuantizer(uint32_t largest) {
+    scale = largest < 0x7f80u ? __uint_as_float(largest << 16) / 448.0f : __builtin_nanf("");
     divisor = fmaxf(scale, 1e-12f);
     inverse = 1.0f / divisor;
   }
@@ -66,22 +70,30 @@ struct GroupQuantizer {
   }
 };
 
+// Largest of `lanes` neighbouring lanes' values.
+__device__ inline uint32_t lanes_max(uint32_t v, int lanes) {
+  for (int offset = lanes / 2; offset > 0; offset >>= 1)
+    v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), offset, 64)));
+  return v;
+}
+
 // token[i] = float(x[i]), for FP8 storage quantized per group of 128.
 template <bool FP8>
 __global__ void __launch_bounds__(kGroup)
 imported_token_kernel(const uint16_t* x, int n, float* token) {
-  __shared__ float largest[2];
+  __shared__ uint32_t largest[2];
   x += static_cast<size_t>(blockIdx.y) * n;      // one token per grid row
   token += static_cast<size_t>(blockIdx.y) * n;
   const int i = blockIdx.x * kGroup + threadIdx.x;
-  const float v = i < n ? bf16_bits_to_float(x[i]) : 0.0f;
+  const uint16_t bits = i < n ? x[i] : 0;
+  const float v = bf16_bits_to_float(bits);
   if constexpr (!FP8) {
     if (i < n) token[i] = v;
   } else {
-    const float mine = wave_max(fabsf(v));
+    const uint32_t mine = lanes_max(bits & 0x7fffu, 64);
     if (threadIdx.x % 64 == 0) largest[threadIdx.x / 64] = mine;
     __syncthreads();
-    const GroupQuantizer quantizer(fmaxf(largest[0], largest[1]));
+    const GroupQuantizer quantizer(max(largest[0], largest[1]));
     float value, unused;
     quantizer.round(v, 0.0f, value, unused);
     if (i < n) token[i] = value * quantizer.scale;
@@ -184,13 +196,11 @@ imported_matvec_kernel(MatVecArgs a) {
       for (int e = 0; e < 8; ++e)
         v[e] = __uint_as_float(e % 2 ? words[e / 2] & 0xffff0000u : words[e / 2] << 16);
       if constexpr (STORAGE == 2) {
-        float largest = 0.0f;
+        uint32_t largest = 0;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) largest = fmaxf(largest, fabsf(v[e]));
-#pragma unroll
-        for (int offset = 8; offset > 0; offset >>= 1)
-          largest = fmaxf(largest, __shfl_xor(largest, offset, 64));
-        const GroupQuantizer quantizer(largest);
+        for (int i = 0; i < 4; ++i)
+          largest = max(largest, max(words[i] & 0x7fffu, words[i] >> 16 & 0x7fffu));
+        const GroupQuantizer quantizer(lanes_max(largest, 16));
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
           quantizer.round(v[e], v[e + 1], v[e], v[e + 1]);
@@ -366,14 +376,15 @@ typedef __attribute__((ext_vector_type(16))) float floatx16;
 // block + 64 half + 16 q .. + 15.
 __global__ void __launch_bounds__(kGroup)
 imported_token_fp8_kernel(const uint16_t* x, int n, unsigned char* codes, float* scales) {
-  __shared__ float largest[2];
+  __shared__ uint32_t largest[2];
   const int token = blockIdx.y, block = blockIdx.x, c = threadIdx.x;
   x += static_cast<size_t>(token) * n;
-  const float v = bf16_bits_to_float(x[block * kGroup + c]);  // n is a multiple of 128
-  const float mine = wave_max(fabsf(v));
+  const uint16_t bits = x[block * kGroup + c];  // n is a multiple of 128
+  const float v = bf16_bits_to_float(bits);
+  const uint32_t mine = lanes_max(bits & 0x7fffu, 64);
   if (threadIdx.x % 64 == 0) largest[threadIdx.x / 64] = mine;
   __syncthreads();
-  const GroupQuantizer quantizer(fmaxf(largest[0], largest[1]));
+  const GroupQuantizer quantizer(max(largest[0], largest[1]));
   const size_t piece = ((static_cast<size_t>(token / 32) * gridDim.x + block) * 2 + c / 64) * 2 + token % 32 / 16;
   codes[(piece * 64 + token % 16 + c % 64 / 16 * 16) * 16 + c % 16] =
       static_cast<unsigned char>(quantizer.code(v));

@@ -309,3 +309,30 @@ def test_one_token_is_prepared_as_for_several(capi, storage, cols, rows):
     both = capi.dense_imported_forward_batch(code, w, scales, x)
     for t in range(2):
         assert torch.equal(capi.dense_imported_forward(code, w, scales, x[t].contiguous()), both[t]), t
+
+
+@pytest.mark.parametrize("tokens", [1, 2, 5, 40])
+@pytest.mark.parametrize("cols,rows", [(128, 33), (144, 17), (263, 20), (5120, 130)])
+def test_a_non_finite_token_gives_nan_and_touches_no_other(capi, oracle, tokens, cols, rows):
+    """FP8 weights: a NaN or an infinity anywhere in a token makes all of its outputs
+    NaN, as the scalar specification's do, on every way a token is prepared; the other
+    tokens keep their bits."""
+    gen = torch.Generator(device="cuda").manual_seed(cols + tokens)
+    clean = torch.randn((tokens, cols), generator=gen, device="cuda").to(torch.bfloat16)
+    w = torch.randint(0, 0x7f, (rows, cols), generator=gen, device="cuda", dtype=torch.uint8)
+    scales = torch.rand(((rows + 127) // 128, (cols + 127) // 128), generator=gen, device="cuda")
+    code = capi.MATRIX_FP8_E4M3
+    expected = capi.dense_imported_forward_batch(code, w, scales, clean)
+    assert torch.isfinite(expected.float()).all()
+    for value in (float("nan"), -float("nan"), float("inf"), -float("inf")):
+        for column in (0, 127, cols - 1):
+            x = clean.clone()
+            bad = list(range(0, tokens, 3))
+            x[bad, column] = value
+            got = capi.dense_imported_forward_batch(code, w, scales, x)
+            good = [t for t in range(tokens) if t not in bad]
+            assert torch.isnan(got[bad].float()).all(), (value, column)
+            assert torch.equal(got[good], expected[good]), (value, column)
+    want = oracle.imported_matvec(oracle.MATRIX_FP8_E4M3, w.cpu().numpy(), scales.cpu().numpy(),
+                                  x[0].float().cpu().numpy())
+    assert np.isnan(want).all()
