@@ -230,14 +230,26 @@ product_rows_kernel(ProductArgs a) {
     }
 }
 
+// Four neighbouring results in one store at any address of their type: global memory
+// takes wide accesses unaligned, the types keep the compiler from assuming more.
+struct __attribute__((packed, aligned(4))) FourFloats {
+  float x, y, z, w;
+};
+struct __attribute__((packed, aligned(2))) FourHalves {
+  uint32_t low, high;
+};
+
 // The same product with one wave a SIMD: four waves, arranged 2 x 2, each with a (32 JM) x
 // (32 JN) part of a (64 JM) x (64 JN) tile, which read each operand from LDS for JN or
 // JM matrix instructions.  Nothing but the wave itself fills the matrix pipe: a row of
 // the left operand is read again for the next 16-element step as soon as it has been
 // multiplied, the right operand a step ahead; the barrier of a stage stands before its
 // last step (whose operands are in registers), and the fills of the stage after
-// next, one every other instruction, follow it.
-template <bool HALF, int JM, int JN>
+// next, one every other instruction, follow it.  WORDS: the output starts at a word;
+// between two words a store of four bf16 values is slower than four stores of one (16384
+// x 768 -> 3072: 131 us, 116 so, 104 at a word; the choice is not made in the kernel, where
+// it cost the others 5 %).
+template <bool HALF, int JM, int JN, bool WORDS>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(1, 1)))
 product_rows_wide_kernel(ProductArgs a) {
@@ -348,6 +360,23 @@ product_rows_wide_kernel(ProductArgs a) {
     }
   }
   wait_loads<0>();  // no fill may land after the workgroup has given its LDS back
+  if constexpr (!WORDS) {
+#pragma unroll
+    for (int jm = 0; jm < JM; ++jm)
+#pragma unroll
+      for (int jn = 0; jn < JN; ++jn) {
+        const int column = n0 + wn + 32 * jn + n;
+        if (column >= a.n_rows) continue;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int row = m0 + wm + 32 * jm + 8 * (i / 4) + 4 * h + i % 4;
+          if (row < a.m_rows)
+            static_cast<uint16_t*>(a.out)[static_cast<long long>(row) * a.n_rows + column] =
+                float_to_bf16_bits(acc[jm][jn][i]);
+        }
+      }
+    return;
+  }
   // four rows of one column a lane -> four columns of one row: 128 (or 64) contiguous
   // bytes of eight rows a store
   const int row0 = m0 + wm + 4 * h + n % 4, column0 = n0 + wn + n / 4 * 4;
@@ -363,10 +392,10 @@ product_rows_wide_kernel(ProductArgs a) {
         if (row >= a.m_rows || column >= a.n_rows) continue;
         const long long at = static_cast<long long>(row) * a.n_rows + column;
         if (a.out_bf16)
-          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + at) =
-              make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w));
+          *reinterpret_cast<FourHalves*>(static_cast<uint16_t*>(a.out) + at) = {pack_bf16(v.x, v.y),
+                                                                               pack_bf16(v.z, v.w)};
         else
-          *reinterpret_cast<float4*>(static_cast<float*>(a.out) + at) = v;
+          *reinterpret_cast<FourFloats*>(static_cast<float*>(a.out) + at) = {v.x, v.y, v.z, v.w};
       }
 }
 
@@ -376,7 +405,7 @@ product_rows_wide_kernel(ProductArgs a) {
 struct Tile {
   int rows, columns, alone, full;
 };
-constexpr Tile kWideTile = {256, 192, 108, 125};   // product_rows_wide_kernel<4, 3>
+constexpr Tile kWideTile = {256, 192, 108, 125};   // product_rows_wide_kernel
 constexpr Tile kMediumTile = {64, 128, 58, 35};    // product_rows_kernel<1, 2>
 constexpr Tile kSmallTile = {64, 64, 50, 20};      // product_rows_kernel<1, 1>
 
@@ -400,13 +429,19 @@ void launch_product_rows(hipStream_t s, const ProductArgs& p) {
   };
   auto time = [&](const Tile& t) { return product_time(t, p.m_rows, p.n_rows, 1, p.depth / kDepth); };
   const long long wide = time(kWideTile), medium = time(kMediumTile), small = time(kSmallTile);
-  const bool aligned = reinterpret_cast<uintptr_t>(p.out) % 16 == 0;  // it stores whole quads
-  if (aligned && wide <= medium && wide <= small)
-    product_rows_wide_kernel<HALF, 4, 3><<<blocks(kWideTile), 256, 0, s>>>(p);
-  else if (medium <= small)
+  if (wide <= medium && wide <= small) {
+    if constexpr (!HALF) {  // FP32 activations have FP32 results
+      if (p.out_bf16 && reinterpret_cast<uintptr_t>(p.out) % 4 != 0) {
+        product_rows_wide_kernel<HALF, 4, 3, false><<<blocks(kWideTile), 256, 0, s>>>(p);
+        return;
+      }
+    }
+    product_rows_wide_kernel<HALF, 4, 3, true><<<blocks(kWideTile), 256, 0, s>>>(p);
+  } else if (medium <= small) {
     product_rows_kernel<HALF, 1, 2, 2, 4><<<blocks(kMediumTile), 256, 0, s>>>(p);
-  else
+  } else {
     product_rows_kernel<HALF, 1, 1, 2, 4><<<blocks(kSmallTile), 256, 0, s>>>(p);
+  }
 }
 
 struct GramArgs {

@@ -108,8 +108,8 @@ def test_bench_shape_matches_float64_products(capi, oracle):
 def test_large_tiles_match_products_of_the_rounded_operands(capi, dtype, shape):
     # The products pick their tiles by size: the first shape takes 256 x 192 ones in all
     # three products (ragged in every direction), the second 64 x 128 ones forward, the
-    # third one 64-element step.  Against FP32 products of the 16-bit operands; an output
-    # address that is not a multiple of 16 bytes takes the other tiles.
+    # third one 64-element step.  Against FP32 products of the 16-bit operands; at an output
+    # address of any element the tiles, and with them the bits, are the same.
     rows, n_in, n_out = shape
     torch.manual_seed(sum(shape))
     x = torch.randn(rows, n_in, device="cuda")
@@ -122,9 +122,13 @@ def test_large_tiles_match_products_of_the_rounded_operands(capi, dtype, shape):
     w16, dy16 = w.to(half).float(), dy.to(half).float()
     y = capi.dense_forward(tx, w, b)
     dx, dw, db = capi.dense_backward(tx, w, dy)
-    storage = torch.empty(rows * n_out + 2, dtype=y.dtype, device="cuda")
-    shifted = capi.dense_forward(tx, w, b, out=storage[2:].view(rows, n_out))
-    torch.cuda.synchronize()
+    storage = torch.full((rows * n_out + 4,), 7.0, dtype=y.dtype, device="cuda")
+    for shift in (1, 2, 3):
+        shifted = capi.dense_forward(tx, w, b, out=storage[shift:shift + rows * n_out].view(rows, n_out))
+        torch.cuda.synchronize()
+        assert torch.equal(shifted, y), shift
+        assert torch.all(storage[:shift] == 7.0) and torch.all(storage[shift + rows * n_out:] == 7.0)
+        storage.fill_(7.0)
 
     def check(got, want, tolerance, what):
         error = (got.double() - want.double()).norm() / want.double().norm()
@@ -134,7 +138,6 @@ def test_large_tiles_match_products_of_the_rounded_operands(capi, dtype, shape):
     check(dx, dy16 @ w16.t().contiguous(), 2e-6, "dx")
     check(dw, x.t().contiguous() @ dy16, 2e-6, "dw")
     check(db, dy.sum(0, dtype=torch.float64), 2e-6, "db")
-    check(shifted, y, 2e-3 if dtype == "bf16" else 2e-6, "y at a shifted address")
 
 
 def test_gradients_are_overwritten_and_repeatable(capi, oracle):
