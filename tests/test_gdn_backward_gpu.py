@@ -205,6 +205,80 @@ def test_benchmarked_shape_against_token_by_token_kernels(capi):
         assert_close(chunked[name], sequential[name], 2e-4, name)
 
 
+@pytest.mark.parametrize("T,kh,vh", [(200, 16, 48), (65, 11, 33), (321, 18, 36), (64, 40, 40), (130, 8, 32)])
+def test_many_value_heads_against_token_by_token_kernels(capi, T, kh, vh):
+    """Beyond 32 value heads a workgroup of the sequential chunk kernels takes two column
+    tiles: the decoder's own 16 key and 48 value heads (three to a key head), counts
+    that are and are not multiples of eight (the two numberings of the workgroups), one
+    chunk, a ragged one and several; 32 heads are the last with one tile."""
+    kw = dict(key_heads=kh, value_heads=vh, key_head_dim=128, value_head_dim=128, conv_kernel_dim=4,
+              round_to_bfloat16=False)
+    p = capi.delta_params(**kw)
+    c = make_case(T, kh, vh, 128, 128, 4, seed=T + vh)
+    bf = torch.bfloat16
+    args = (p, dev(c["qkv"], bf), dev(c["z"], bf), dev(c["a"], bf), dev(c["b"], bf), dev(c["conv"]),
+            dev(c["a_log"]), dev(c["dt_bias"]), dev(c["norm"]), dev(c["dy"]))
+
+    def once():
+        grads = dict(conv_weight=torch.zeros((2 * kh + vh) * 128, 4, device="cuda"),
+                     a_log=torch.zeros(vh, device="cuda"), dt_bias=torch.zeros(vh, device="cuda"),
+                     norm=torch.zeros(128, device="cuda"))
+        out = capi.gdn_layer_backward(*args, parameter_grads=grads)
+        torch.cuda.synchronize()
+        named = dict(zip(("dqkv", "dz", "da", "db"), out))
+        named.update(grads)
+        return {k: v.cpu().numpy() for k, v in named.items()}
+
+    chunked = once()
+    assert capi.last_path() == capi.PATH_CHUNKED
+    with capi.force_generic():
+        sequential = once()
+        assert capi.last_path() == capi.PATH_RECURRENCE
+    for name in sequential:
+        assert_close(chunked[name], sequential[name], 2e-4, name)
+
+
+@pytest.mark.parametrize("rounding", [False, True])
+def test_tensors_off_sixteen_bytes_give_the_same_bits(capi, rounding):
+    """Every tensor one element past a 16-byte boundary: the passes with wide accesses
+    (four-tap convolution forward and backward, output backward of rows of 128) take
+    their narrow variants, which do the same arithmetic.  Two sequences, whose second
+    starts at an odd multiple of the row's bytes."""
+    import ctypes
+    T, kh, vh, batch = 71, 2, 6, 2
+    p = capi.delta_params(key_heads=kh, value_heads=vh, key_head_dim=128, value_head_dim=128,
+                          conv_kernel_dim=4, round_to_bfloat16=rounding)
+    c = make_case(T, kh, vh, 128, 128, 4, seed=9, batch=batch)
+    bf = torch.bfloat16
+    inputs = [dev(c["qkv"], bf), dev(c["z"], bf), dev(c["a"], bf), dev(c["b"], bf), dev(c["conv"]),
+              dev(c["a_log"]), dev(c["dt_bias"]), dev(c["norm"]), dev(c["dy"])]
+    channels = (2 * kh + vh) * 128
+    shapes = [inputs[0].shape, inputs[1].shape, inputs[2].shape, inputs[3].shape, (channels, 4), (vh,),
+              (vh,), (128,)]  # gradients of the inputs, then of the parameters
+
+    def once(shift):
+        def moved(x):
+            space = torch.zeros(x.numel() + 8, dtype=x.dtype, device="cuda")
+            view = space[shift:shift + x.numel()].view(x.shape)
+            view.copy_(x)
+            assert view.data_ptr() % 16 == (shift * x.element_size()) % 16
+            return view
+        given = [moved(x) for x in inputs]
+        out = [moved(torch.zeros(s, device="cuda")) for s in shapes]
+        size = capi.lib().pluto_hip_gdn_layer_backward_workspace_bytes(ctypes.byref(p), T, 1)
+        workspace = torch.empty(size, dtype=torch.uint8, device="cuda")
+        capi.check(capi.lib().pluto_hip_gdn_layer_backward(
+            capi.current_stream(), ctypes.byref(p), batch, T, *[capi.ptr(x) for x in given],
+            *[capi.ptr(x) for x in out], capi.ptr(workspace), size))
+        torch.cuda.synchronize()
+        assert capi.last_path() == capi.PATH_CHUNKED
+        return out
+
+    for name, a, b in zip(("dqkv", "dz", "da", "db", "conv", "a_log", "dt_bias", "norm"), once(0), once(1)):
+        assert torch.isfinite(a).all() and a.abs().max() > 0, name
+        assert torch.equal(a, b), name
+
+
 def test_rejects_bad_arguments(capi):
     import ctypes
     p = capi.delta_params(key_heads=1, value_heads=2, key_head_dim=4, value_head_dim=6,

@@ -284,3 +284,57 @@ def test_split_operand_kernels_keep_fp32_accuracy(capi, T, qh, kh, rot):
         error = np.linalg.norm(got[name] - w) / max(np.linalg.norm(w), 0.1 * float(dv.norm()))
         print("%s T%d: %.2e" % (name, T, error))
         assert error <= 2e-5, name
+
+
+@pytest.mark.parametrize("T,qh,kh,d,rot,with_saved", [(70, 4, 2, 64, 32, True), (70, 4, 2, 64, 32, False),
+                                                      (131, 6, 2, 128, 32, True), (65, 6, 2, 256, 64, False)])
+def test_tensors_off_sixteen_bytes(capi, T, qh, kh, d, rot, with_saved):
+    """The gate's pass and the norm's have wide accesses where every tensor allows it.
+    With dy alone moved by one element the gate's narrow variant does the same arithmetic,
+    bit for bit; with the gradients moved too the norm's any-width kernel adds up in another
+    order (FP32 rounding); with the bf16 inputs moved the preparation's does as well, and an
+    element of q or k next to a rounding tie may fall to its other side."""
+    import ctypes
+    p = capi.attention_params(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=rot, capacity=T,
+                              round_to_bfloat16=True)
+    gen = torch.Generator(device="cuda").manual_seed(T + d)
+    bf = torch.bfloat16
+    def normal(*shape):
+        return torch.randn(shape, generator=gen, device="cuda")
+    qg, k, v = (0.5 * normal(T, qh, 2, d)).to(bf), (0.5 * normal(T, kh, d)).to(bf), (0.5 * normal(T, kh, d)).to(bf)
+    q_norm, k_norm, dy = 0.1 * normal(d), 0.1 * normal(d), normal(T, qh, d)
+    saved = None
+    if with_saved:
+        cache = capi.KvCache(T, kh, d)
+        saved = capi.gqa_prefill_saved(p, T, cache)
+        capi.gqa_prefill(p, qg, k, v, q_norm, k_norm, cache, saved=saved)
+
+    def once(inputs, upstream, outputs):
+        def moved(x, shift):
+            space = torch.zeros(x.numel() + 8, dtype=x.dtype, device="cuda")
+            view = space[shift:shift + x.numel()].view(x.shape)
+            view.copy_(x)
+            return view
+        given = [moved(x, inputs) for x in (qg, k, v)] + [q_norm, k_norm, moved(dy, upstream)]
+        out = [moved(torch.zeros(s, device="cuda"), outputs)
+               for s in ((T, qh, 2, d), (T, kh, d), (T, kh, d), (d,), (d,))]
+        size = capi.lib().pluto_hip_gqa_prefill_backward_workspace_bytes(ctypes.byref(p), T, 1, 1)
+        workspace = torch.empty(size, dtype=torch.uint8, device="cuda")
+        capi.check(capi.lib().pluto_hip_gqa_prefill_backward(
+            capi.current_stream(), ctypes.byref(p), T, *[capi.ptr(x) for x in given], capi.ptr(saved),
+            *[capi.ptr(x) for x in out], capi.ptr(workspace), size))
+        torch.cuda.synchronize()
+        assert capi.last_path() == (capi.PATH_MATRIX_F32 if d == 256 else capi.PATH_FLASH)
+        return out
+
+    names = ("dqg", "dk", "dv", "dq_norm", "dk_norm")
+    want = once(0, 0, 0)
+    for name, a, b in zip(names, want, once(0, 1, 0)):
+        assert torch.isfinite(a).all() and a.abs().max() > 0, name
+        assert torch.equal(a, b), name
+    for name, a, b in zip(names, want, once(0, 1, 1)):
+        # sums of d and of T * heads FP32 terms in two orders: about sqrt(terms) 2^-24 each
+        assert (a - b).norm() <= 1e-5 * a.norm(), name
+    for name, a, b in zip(names, want, once(1, 1, 1)):
+        # a bf16 ulp (2^-8) in one element of a thousand: 2^-8 sqrt(1e-3) of the norm
+        assert (a - b).norm() <= 2.0 ** -8 * 1e-3 ** 0.5 * a.norm(), name
