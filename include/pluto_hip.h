@@ -627,6 +627,21 @@ int pluto_hip_test_forward_schedule(int head_dim, int q_rows, int kv_rows, int s
                                     int workgroups_resident, uint16_t* items, int capacity,
                                     int* workgroups, int* slots);
 
+/* The same for one sequence whose query tiles share their keys out in parts.
+ * The kv heads congruent to p modulo *partitions are partition p, and every
+ * partition has the same 256 / *partitions lists: list j is entries first[j] ..
+ * first[j + 1] - 1.  An entry is four numbers: the tile, (query head within the
+ * partition) * q_tiles + q_tile, the key tiles of 64 it begins and ends at, and
+ * the slot of its partial result, 0xffff where it is the whole tile.  `tiles`
+ * are the tiles in parts, three numbers each: tile, first slot, parts.
+ * `entries` has room for 4 * capacity numbers, `tiles` for 3 * capacity / 2,
+ * `first` for 257, and capacity is 384 at least (PLUTO_HIP_ELIMIT).
+ * *partitions is 0 where the tiles are not split. */
+int pluto_hip_test_forward_split(int head_dim, int q_rows, int kv_rows, int start_position,
+                                 int query_heads, int group, int workgroups_resident,
+                                 uint16_t* entries, uint16_t* first, uint16_t* tiles,
+                                 int capacity, int* partitions, int* tile_count);
+
 #ifdef __cplusplus
 }
 #endif

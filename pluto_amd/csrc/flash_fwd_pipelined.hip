@@ -963,3 +963,38 @@ extern "C" int pluto_hip_test_forward_schedule(int head_dim, int q_rows, int kv_
   for (long long i = 0; i < entries; ++i) items[i] = schedule.item[i];
   return 0;
 }
+
+extern "C" int pluto_hip_test_forward_split(int head_dim, int q_rows, int kv_rows, int start_position,
+                                            int query_heads, int group, int workgroups_resident,
+                                            uint16_t* entries, uint16_t* first, uint16_t* tiles,
+                                            int capacity, int* partitions, int* tile_count) {
+  using namespace pluto_hip;
+  if ((head_dim != 128 && head_dim != 256) || q_rows <= 0 || kv_rows <= 0 || start_position < 0 ||
+      query_heads <= 0 || group <= 0 || query_heads % group != 0 || workgroups_resident < 0 ||
+      !entries || !first || !tiles || !partitions || !tile_count)
+    return PLUTO_HIP_EINVAL;
+  if (capacity < kSplitEntries) return PLUTO_HIP_ELIMIT;
+  ScheduleKey key;
+  key.q_rows = q_rows, key.kv_rows = kv_rows, key.start_position = start_position;
+  key.query_heads = query_heads, key.group = group, key.sequences = 1;
+  key.tile_rows = 32 * (head_dim == 256 ? kWaves<256> : kWaves<128>);
+  key.workgroups = workgroups_resident;
+  static thread_local SplitPlan plan;
+  build_split(key, &plan);
+  *partitions = plan.useful ? plan.split.partitions : 0;
+  *tile_count = 0;
+  if (!plan.useful) return 0;
+  const int lists = kSplitLists / plan.split.partitions;
+  for (int j = 0; j <= lists; ++j) first[j] = plan.split.first[j];
+  for (int e = 0; e < plan.split.first[lists]; ++e) {
+    const SplitEntry& part = plan.split.entry[e];
+    entries[4 * e] = part.tile, entries[4 * e + 1] = part.begin;
+    entries[4 * e + 2] = part.end, entries[4 * e + 3] = part.slot;
+  }
+  *tile_count = plan.tiles.count;
+  for (int i = 0; i < plan.tiles.count; ++i) {
+    tiles[3 * i] = plan.tiles.tile[i].tile, tiles[3 * i + 1] = plan.tiles.tile[i].slot;
+    tiles[3 * i + 2] = plan.tiles.tile[i].parts;
+  }
+  return 0;
+}

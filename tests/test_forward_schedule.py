@@ -2,7 +2,8 @@
 host alone: whatever the shape, every (sequence, head, query tile) is launched
 exactly once, lists never exceed the table, and the heads that share a kv head
 stay on as few XCDs as the partitioning promises (workgroup i runs on XCD i mod
-8).  No GPU is needed: the packing is host code behind a test-support export."""
+8); tiles whose keys are shared out have every key in one part.  No GPU is
+needed: the packing is host code behind test-support exports."""
 import ctypes
 import random
 
@@ -133,3 +134,101 @@ def test_the_prefill_workspace_has_room_for_parts_only_where_tiles_are_split(lib
         rows = min(length, tile_rows(head_dim))
         want = 0 if head_dim == 64 else aligned(384 * rows * (head_dim + 2) * 4)
         assert parts(length, capacity) == want, (length, capacity)
+
+
+PARTS = 384
+
+
+def split(library, head_dim, q_rows, start, query_heads, group, resident=256):
+    """(partitions, lists of (tile, begin, end, slot), tiles in parts) or None."""
+    entries, first = (ctypes.c_uint16 * (4 * PARTS))(), (ctypes.c_uint16 * 257)()
+    tiles = (ctypes.c_uint16 * (3 * PARTS // 2))()
+    partitions, count = ctypes.c_int(-1), ctypes.c_int(-1)
+    status = library.pluto_hip_test_forward_split(
+        head_dim, q_rows, start + q_rows, start, query_heads, group, resident, entries, first, tiles,
+        PARTS, ctypes.byref(partitions), ctypes.byref(count))
+    assert status == 0
+    if partitions.value == 0:
+        return None
+    lists = [[tuple(entries[4 * e:4 * e + 4]) for e in range(first[j], first[j + 1])]
+             for j in range(256 // partitions.value)]
+    return partitions.value, lists, [tuple(tiles[3 * i:3 * i + 3]) for i in range(count.value)]
+
+
+def check_split(library, head_dim, q_rows, start, query_heads, group):
+    made = split(library, head_dim, q_rows, start, query_heads, group)
+    if made is None:
+        return False
+    partitions, lists, tiles = made
+    kv_heads, q_tiles = query_heads // group, -(-q_rows // tile_rows(head_dim))
+    assert partitions in (1, 2, 4, 8) and kv_heads % partitions == 0
+    assert q_rows <= (start + q_rows) // 2
+    items = q_tiles * query_heads // partitions
+    entries = [e for part in lists for e in part]
+    assert len(entries) <= PARTS
+
+    def key_tiles(tile):
+        last = min((tile % q_tiles + 1) * tile_rows(head_dim), q_rows) - 1
+        return -(-(start + last + 1) // 64)
+
+    # every key tile of every query tile once, whole tiles without a slot
+    ranges = {}
+    for tile, begin, end, slot in entries:
+        assert tile < items and begin < end
+        ranges.setdefault(tile, []).append((begin, end, slot))
+    assert sorted(ranges) == list(range(items))
+    parts = {tile: (slot, count) for tile, slot, count in tiles}
+    assert len(parts) == len(tiles)
+    used = []
+    for tile, pieces in ranges.items():
+        pieces.sort()
+        assert pieces[0][0] == 0 and pieces[-1][1] == key_tiles(tile)
+        assert all(a[1] == b[0] for a, b in zip(pieces, pieces[1:]))
+        if pieces[0][2] == NO_ITEM:
+            assert len(pieces) == 1 and tile not in parts
+            continue
+        # the parts' slots follow each other in the order of their keys
+        assert [p[2] for p in pieces] == list(range(parts[tile][0], parts[tile][0] + parts[tile][1]))
+        used += [p[2] for p in pieces]
+        # all rows of the tile see all keys of every part but the last
+        first_row = tile % q_tiles * tile_rows(head_dim)
+        assert all(end * 64 <= start + first_row + 1 for _, end, _ in pieces[:-1])
+    assert sorted(used) == list(range(len(used))) and 0 < len(used) * partitions <= PARTS
+    assert len(parts) == sum(1 for pieces in ranges.values() if pieces[0][2] != NO_ITEM)
+    # what the split is for: the fullest list carries less than it would with whole tiles
+    def load(part):
+        return sum(end - begin + 8 + (3 if slot != NO_ITEM else 0) for _, begin, end, slot in part)
+    whole = [0] * len(lists)
+    for tile in sorted(range(items), key=key_tiles, reverse=True):
+        at = whole.index(min(whole))
+        whole[at] += key_tiles(tile) + 8
+    assert max(load(part) for part in lists) < max(whole)
+    return True
+
+
+def test_tiles_in_parts_cover_every_key_once(library):
+    assert check_split(library, 256, 34, 7336, 24, 6)
+    assert check_split(library, 256, 1531, 2309, 24, 6)
+    rng = random.Random(11)
+    made = 0
+    for _ in range(600):
+        group = rng.choice([1, 2, 3, 6, 8])
+        kv_heads = rng.choice([1, 2, 4, 8, 16, 3, 5, 12])
+        q_rows = rng.choice([rng.randint(1, 64), rng.randint(1, 600), rng.randint(1, 3000)])
+        start = rng.choice([q_rows, rng.randint(0, 3000), rng.randint(3000, 60000)])
+        made += bool(check_split(library, rng.choice([128, 256]), q_rows, start, group * kv_heads, group))
+    assert made > 150    # the sample does split
+
+
+def test_when_tiles_are_not_split(library):
+    assert split(library, 256, 1024, 0, 24, 6) is None            # rows are all the keys
+    assert split(library, 256, 1024, 1023, 24, 6) is None         # more than half of them
+    assert split(library, 256, 34, 7336, 24, 6, resident=250) is None   # not the chip the lists are for
+    assert split(library, 128, 20000, 200000, 24, 6) is None      # more tiles than the lists hold
+    buffers = [(ctypes.c_uint16 * n)() for n in (4 * PARTS, 257, 3 * PARTS // 2)]
+    a, b = ctypes.c_int(), ctypes.c_int()
+    def call(head_dim, heads, group, capacity):
+        return library.pluto_hip_test_forward_split(head_dim, 34, 7370, 7336, heads, group, 256, *buffers,
+                                                    capacity, ctypes.byref(a), ctypes.byref(b))
+    assert call(64, 24, 6, PARTS) == capi.EINVAL and call(256, 24, 5, PARTS) == capi.EINVAL
+    assert call(256, 24, 6, PARTS - 1) == capi.ELIMIT
