@@ -126,27 +126,25 @@ __device__ inline void wait_loads() {
 }
 
 // out[m, n] = bias[n] + sum_k left[m, k] right[n, k]; depth % 64 == 0.  A
-// workgroup of NWAVES waves, arranged 2 x (NWAVES / 2), owns a
-// (64 JM) x (16 NWAVES JN) tile and each wave a (32 JM) x (32 JN) part of it.
-// STAGES LDS stages of 64 contraction elements are filled STAGES - 1 steps
-// ahead.
-template <bool HALF, int JM, int JN, int STAGES, int NWAVES>
-__global__ void __launch_bounds__(64 * NWAVES)
+// workgroup of four waves, arranged 2 x 2, owns a 64 x (64 JN) tile and each wave
+// a 32 x (32 JN) part of it.  Two LDS stages of 64 contraction elements: one is
+// filled while the other is multiplied.
+template <bool HALF, int JN>
+__global__ void __launch_bounds__(kThreads)
 product_rows_kernel(ProductArgs a) {
-  constexpr int THREADS = 64 * NWAVES;
   constexpr int KS = kDepth / 16;  // matrix instructions along the contraction per stage
-  constexpr int TM = 64 * JM, TN = 32 * (NWAVES / 2) * JN;
+  constexpr int TM = 64, TN = 64 * JN;
   constexpr int kLeftBytes = TM * kDepth * 2, kRightBytes = TN * kDepth * 2;
   constexpr int kStageBytes = kLeftBytes + kRightBytes;
-  constexpr int LEFT_LOADS = TM * (kDepth / 8) / THREADS;
-  constexpr int RIGHT_LOADS = TN * (kDepth / 8) / THREADS;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[STAGES * kStageBytes];
+  constexpr int LEFT_LOADS = TM * (kDepth / 8) / kThreads;
+  constexpr int RIGHT_LOADS = TN * (kDepth / 8) / kThreads;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
   const int n_tiles = (a.n_rows + TN - 1) / TN;
   const int logical = xcd_logical_block();
   const int m0 = (logical / n_tiles) * TM, n0 = (logical % n_tiles) * TN;
-  const int wm = 32 * JM * (wave / (NWAVES / 2)), wn = 32 * JN * (wave % (NWAVES / 2));
+  const int wm = 32 * (wave / 2), wn = 32 * JN * (wave % 2);
   uint32_t left_fill[LEFT_LOADS], right_fill[RIGHT_LOADS];
 #pragma unroll
   for (int i = 0; i < LEFT_LOADS; ++i)
@@ -162,72 +160,60 @@ product_rows_kernel(ProductArgs a) {
     left_read[ks] = tile_row_read<kDepth>(wm + n, 2 * ks + h);
     right_read[ks] = tile_row_read<kDepth>(wn + n, 2 * ks + h);
   }
-  // acc[jm][jn]: a lane holds output column n0 + wn + 32 jn + n of rows
-  // m0 + wm + 32 jm + 8 q + 4 h + i (element 4 q + i)
-  floatx16 acc[JM][JN];
+  // acc[jn]: a lane holds output column n0 + wn + 32 jn + n of rows
+  // m0 + wm + 8 q + 4 h + i (element 4 q + i)
+  floatx16 acc[JN];
 #pragma unroll
   for (int jn = 0; jn < JN; ++jn) {
     const int column = n0 + wn + 32 * jn + n;
     const float start = (a.bias && column < a.n_rows) ? a.bias[column] : 0.0f;
 #pragma unroll
-    for (int jm = 0; jm < JM; ++jm)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[jm][jn][i] = start;
+    for (int i = 0; i < 16; ++i) acc[jn][i] = start;
   }
   const uint16_t* left = a.left + static_cast<long long>(m0) * a.depth;
   const uint16_t* right = a.right + static_cast<long long>(n0) * a.depth;
   const int steps = a.depth / kDepth;
   auto fill_stage = [&](int step) {
-    unsigned char* stage = lds + (step % STAGES) * kStageBytes;
+    unsigned char* stage = lds + (step % 2) * kStageBytes;
     tile_fill<kDepth, LEFT_LOADS>(stage, wave, left + step * kDepth, a.depth, m0, a.m_rows,
                                   left_fill);
     tile_fill<kDepth, RIGHT_LOADS>(stage + kLeftBytes, wave, right + step * kDepth, a.depth, n0,
                                    a.n_rows, right_fill);
   };
-  for (int step = 0; step < STAGES - 1 && step < steps; ++step) fill_stage(step);
+  fill_stage(0);
   for (int step = 0; step < steps; ++step) {
-    // stage `step` has landed once at most the STAGES - 2 later fills remain
-    if (step + STAGES - 2 < steps)
-      wait_loads<(STAGES - 2) * (LEFT_LOADS + RIGHT_LOADS)>();
-    else
-      wait_loads<0>();
+    wait_loads<0>();
     lds_barrier();
-    if (step + STAGES - 1 < steps) fill_stage(step + STAGES - 1);
-    const unsigned char* left_tile = lds + (step % STAGES) * kStageBytes;
+    if (step + 1 < steps) fill_stage(step + 1);
+    const unsigned char* left_tile = lds + (step % 2) * kStageBytes;
     const unsigned char* right_tile = left_tile + kLeftBytes;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      uint4 l[JM], r[JN];
-#pragma unroll
-      for (int j = 0; j < JM; ++j)
-        l[j] = *reinterpret_cast<const uint4*>(left_tile + left_read[ks] + j * kBlockStep);
+      uint4 r[JN];
+      const uint4 l = *reinterpret_cast<const uint4*>(left_tile + left_read[ks]);
 #pragma unroll
       for (int j = 0; j < JN; ++j)
         r[j] = *reinterpret_cast<const uint4*>(right_tile + right_read[ks] + j * kBlockStep);
 #pragma unroll
-      for (int jm = 0; jm < JM; ++jm)
-#pragma unroll
-        for (int jn = 0; jn < JN; ++jn) acc[jm][jn] = mma<HALF>(l[jm], r[jn], acc[jm][jn]);
+      for (int jn = 0; jn < JN; ++jn) acc[jn] = mma<HALF>(l, r[jn], acc[jn]);
     }
   }
   // 32 lanes store 32 consecutive columns of a row: 64 or 128 contiguous bytes
 #pragma unroll
-  for (int jm = 0; jm < JM; ++jm)
+  for (int jn = 0; jn < JN; ++jn) {
+    const int column = n0 + wn + 32 * jn + n;
+    if (column >= a.n_rows) continue;
 #pragma unroll
-    for (int jn = 0; jn < JN; ++jn) {
-      const int column = n0 + wn + 32 * jn + n;
-      if (column >= a.n_rows) continue;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = m0 + wm + 32 * jm + 8 * (i / 4) + 4 * h + i % 4;
-        if (row >= a.m_rows) continue;
-        const long long at = static_cast<long long>(row) * a.n_rows + column;
-        if (a.out_bf16)
-          static_cast<uint16_t*>(a.out)[at] = float_to_bf16_bits(acc[jm][jn][i]);
-        else
-          static_cast<float*>(a.out)[at] = acc[jm][jn][i];
-      }
+    for (int i = 0; i < 16; ++i) {
+      const int row = m0 + wm + 8 * (i / 4) + 4 * h + i % 4;
+      if (row >= a.m_rows) continue;
+      const long long at = static_cast<long long>(row) * a.n_rows + column;
+      if (a.out_bf16)
+        static_cast<uint16_t*>(a.out)[at] = float_to_bf16_bits(acc[jn][i]);
+      else
+        static_cast<float*>(a.out)[at] = acc[jn][i];
     }
+  }
 }
 
 // Four neighbouring results in one store at any address of their type: global memory
@@ -406,8 +392,8 @@ struct Tile {
   int rows, columns, alone, full;
 };
 constexpr Tile kWideTile = {256, 192, 108, 125};   // product_rows_wide_kernel
-constexpr Tile kMediumTile = {64, 128, 58, 35};    // product_rows_kernel<1, 2>
-constexpr Tile kSmallTile = {64, 64, 50, 20};      // product_rows_kernel<1, 1>
+constexpr Tile kMediumTile = {64, 128, 58, 35};    // product_rows_kernel<2>
+constexpr Tile kSmallTile = {64, 64, 50, 20};      // product_rows_kernel<1>
 
 // The time of a product with one kind of tiles: its steps, and the filling of the first
 // stages and the stores at about five of them, as often as compute units take turns.
@@ -438,9 +424,9 @@ void launch_product_rows(hipStream_t s, const ProductArgs& p) {
     }
     product_rows_wide_kernel<HALF, 4, 3, true><<<blocks(kWideTile), 256, 0, s>>>(p);
   } else if (medium <= small) {
-    product_rows_kernel<HALF, 1, 2, 2, 4><<<blocks(kMediumTile), 256, 0, s>>>(p);
+    product_rows_kernel<HALF, 2><<<blocks(kMediumTile), kThreads, 0, s>>>(p);
   } else {
-    product_rows_kernel<HALF, 1, 1, 2, 4><<<blocks(kSmallTile), 256, 0, s>>>(p);
+    product_rows_kernel<HALF, 1><<<blocks(kSmallTile), kThreads, 0, s>>>(p);
   }
 }
 

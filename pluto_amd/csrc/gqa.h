@@ -161,12 +161,10 @@ int launch_attention_probabilities(hipStream_t stream, const void* q, int q_dtyp
                                    float* probabilities);
 
 // Pieces of the whole-sequence backward (gqa_backward.hip).
-int launch_pack_heads(hipStream_t stream, const void* q, const void* k, const void* v, int dtype,
-                      int length, int query_heads, int key_value_heads, int head_dim,
-                      void* packed);
-int launch_gate_backward(hipStream_t stream, const void* qg, const void* core, int core_dtype,
-                         const float* dy, int length, int query_heads, int head_dim, bool round,
-                         float* dc, float* dqg);
+int launch_pack_heads(hipStream_t stream, const float* q, const float* k, const float* v, int length,
+                      int query_heads, int key_value_heads, int head_dim, float* packed);
+int launch_gate_backward(hipStream_t stream, const void* qg, const float* core, const float* dy,
+                         int length, int query_heads, int head_dim, bool round, float* dc, float* dqg);
 // The same for the matrix-core backward (head widths 64 and 128).
 int launch_gate_rows(hipStream_t stream, const void* qg, const void* core, const float* dy,
                      const float* maxima, const float* normalizers, int length, int query_heads,

@@ -23,12 +23,12 @@ namespace {
 // [T, qh, d] prepared queries, [T, kh, d] prepared keys and values ->
 // packed [T, 3E] (E = qh * d): Q | K of the head's kv head | V of it.  Moved in
 // pieces of PIECE elements (16 bytes when the head width allows).
-template <typename Element, int PIECE>
+template <int PIECE>
 __global__ void __launch_bounds__(256)
-pack_heads_kernel(const Element* q, const Element* k, const Element* v, int length, int qh,
-                  int kh, int d, Element* packed) {
-  struct alignas(sizeof(Element) * PIECE) Piece {
-    Element e[PIECE];
+pack_heads_kernel(const float* q, const float* k, const float* v, int length, int qh, int kh, int d,
+                  float* packed) {
+  struct alignas(sizeof(float) * PIECE) Piece {
+    float e[PIECE];
   };
   const int pieces_per_head = d / PIECE;
   const long long pieces_per_part = 1LL * qh * pieces_per_head;
@@ -40,23 +40,23 @@ pack_heads_kernel(const Element* q, const Element* k, const Element* v, int leng
     const int part = static_cast<int>(within / pieces_per_part);
     const int h = static_cast<int>((within % pieces_per_part) / pieces_per_head);
     const int c = static_cast<int>(within % pieces_per_head) * PIECE;
-    const Element* source = part == 0 ? q + (t * qh + h) * d + c
-                                      : (part == 1 ? k : v) + (t * kh + h / group) * d + c;
+    const float* source = part == 0 ? q + (t * qh + h) * d + c
+                                    : (part == 1 ? k : v) + (t * kh + h / group) * d + c;
     *reinterpret_cast<Piece*>(packed + i * PIECE) = *reinterpret_cast<const Piece*>(source);
   }
 }
 
 // dC = dy * Round(sigmoid(gate)); d gate = dy * Round(core) * s (1 - s).
 __global__ void __launch_bounds__(256)
-gate_backward_kernel(const uint16_t* qg, const void* core, int core_dtype, const float* dy,
-                     long long elements, int d, bool round, float* dc, float* dqg) {
+gate_backward_kernel(const uint16_t* qg, const float* core, const float* dy, long long elements,
+                     int d, bool round, float* dc, float* dqg) {
   for (long long i = blockIdx.x * 256LL + threadIdx.x; i < elements; i += 256LL * gridDim.x) {
     const long long unit = i / d;  // (row, head)
     const int c = static_cast<int>(i % d);
     const float gate = bf16_bits_to_float(qg[(unit * 2 + 1) * d + c]);
     const float sigmoid = 1.0f / (1.0f + expf(-gate));
     const float grad = dy[i];
-    float value = load_element(core, i, core_dtype);
+    float value = core[i];
     if (round) value = round_to_bf16(value);
     dc[i] = grad * (round ? round_to_bf16(sigmoid) : sigmoid);
     dqg[(unit * 2 + 1) * d + c] = grad * value * sigmoid * (1.0f - sigmoid);
@@ -353,41 +353,21 @@ int grid_for(long long elements) {
 
 }  // namespace
 
-int launch_pack_heads(hipStream_t stream, const void* q, const void* k, const void* v, int dtype,
-                      int length, int qh, int kh, int d, void* packed) {
+int launch_pack_heads(hipStream_t stream, const float* q, const float* k, const float* v, int length,
+                      int qh, int kh, int d, float* packed) {
   const long long elements = 3LL * length * qh * d;
-  if (dtype == PLUTO_HIP_BF16) {
-    auto* qs = static_cast<const uint16_t*>(q);
-    auto* ks = static_cast<const uint16_t*>(k);
-    auto* vs = static_cast<const uint16_t*>(v);
-    auto* out = static_cast<uint16_t*>(packed);
-    if (d % 8 == 0)
-      pack_heads_kernel<uint16_t, 8><<<grid_for(elements / 8), 256, 0, stream>>>(qs, ks, vs, length,
-                                                                                 qh, kh, d, out);
-    else
-      pack_heads_kernel<uint16_t, 1><<<grid_for(elements), 256, 0, stream>>>(qs, ks, vs, length, qh,
-                                                                             kh, d, out);
-  } else {
-    auto* qs = static_cast<const float*>(q);
-    auto* ks = static_cast<const float*>(k);
-    auto* vs = static_cast<const float*>(v);
-    auto* out = static_cast<float*>(packed);
-    if (d % 4 == 0)
-      pack_heads_kernel<float, 4><<<grid_for(elements / 4), 256, 0, stream>>>(qs, ks, vs, length, qh,
-                                                                              kh, d, out);
-    else
-      pack_heads_kernel<float, 1><<<grid_for(elements), 256, 0, stream>>>(qs, ks, vs, length, qh, kh,
-                                                                          d, out);
-  }
+  if (d % 4 == 0)
+    pack_heads_kernel<4><<<grid_for(elements / 4), 256, 0, stream>>>(q, k, v, length, qh, kh, d, packed);
+  else
+    pack_heads_kernel<1><<<grid_for(elements), 256, 0, stream>>>(q, k, v, length, qh, kh, d, packed);
   return launch_status();
 }
 
-int launch_gate_backward(hipStream_t stream, const void* qg, const void* core, int core_dtype,
-                         const float* dy, int length, int qh, int d, bool round, float* dc,
-                         float* dqg) {
+int launch_gate_backward(hipStream_t stream, const void* qg, const float* core, const float* dy,
+                         int length, int qh, int d, bool round, float* dc, float* dqg) {
   const long long elements = 1LL * length * qh * d;
-  gate_backward_kernel<<<grid_for(elements), 256, 0, stream>>>(
-      static_cast<const uint16_t*>(qg), core, core_dtype, dy, elements, d, round, dc, dqg);
+  gate_backward_kernel<<<grid_for(elements), 256, 0, stream>>>(static_cast<const uint16_t*>(qg), core, dy,
+                                                              elements, d, round, dc, dqg);
   return launch_status();
 }
 

@@ -490,16 +490,17 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
     status = launch_split_backward(s, a);
   } else {
     grads = {d_heads, d_heads + E, d_heads + 2LL * E, 3LL * E, 3LL * E};
-    status = launch_pack_heads(s, scratch + l.queries, scratch + l.keys, scratch + l.values,
-                               l.dtype, length, qh, kh, d, scratch + l.packed);
+    auto floats = [&](size_t offset) { return reinterpret_cast<float*>(scratch + offset); };
+    status = launch_pack_heads(s, floats(l.queries), floats(l.keys), floats(l.values), length, qh, kh, d,
+                               floats(l.packed));
     if (status != 0) return status;
-    status = pluto_hip_mha_forward(stream, l.dtype, scratch + l.packed, length, length, qh, E,
+    status = pluto_hip_mha_forward(stream, PLUTO_HIP_F32, scratch + l.packed, length, length, qh, E,
                                    scratch + l.core, maxima, normalizers);
     if (status != 0) return status;
-    float* dc = reinterpret_cast<float*>(scratch + l.dc);
-    status = launch_gate_backward(s, qg, core, l.dtype, dy, length, qh, d, round, dc, dqg);
+    float* dc = floats(l.dc);
+    status = launch_gate_backward(s, qg, floats(l.core), dy, length, qh, d, round, dc, dqg);
     if (status != 0) return status;
-    status = pluto_hip_mha_backward(stream, l.dtype, scratch + l.packed, core, dc, maxima,
+    status = pluto_hip_mha_backward(stream, PLUTO_HIP_F32, scratch + l.packed, core, dc, maxima,
                                     normalizers, length, length, qh, E, d_heads,
                                     scratch + l.attention, l.attention_bytes);
   }
@@ -775,7 +776,6 @@ static int decode_run(void* stream, const pluto_hip_attention_params* p, int bat
       prep.key_value_heads = kh;
       prep.head_dim = d;
       prep.rotary_dim = p->rotary_dim;
-  prep.theta = p->rope_theta;
       prep.epsilon = p->rms_norm_epsilon;
       prep.theta = p->rope_theta;
       prep.round = round;
