@@ -235,16 +235,17 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p,
  *   dy       fp32 [length, qh, d]     gradient of the layer output
  *   saved    optional: the block pluto_hip_gqa_prefill filled for the same
  *            inputs and parameters; the attention forward is then not repeated
- *            (a quarter of the call at length 8192).  NULL recomputes.
+ *            (a fifth of the call at length 8192).  NULL recomputes.
  *   dqg      fp32 [length, qh, 2, d]  query gradients at [..,0,:], gate at [..,1,:]
  *   dk, dv   fp32 [length, kh, d]
  *   dq_norm, dk_norm  optional fp32 [d]: the norm weights' gradients are ADDED
  *            to them (shared weights accumulate over calls, as in the
  *            reference); NULL skips that work.
  * Rounding points are treated as identities, with the rounded forward values
- * as operands where the reference uses them.  With round_to_bfloat16 set and
- * head_dim 64 or 128 the attention part runs on the matrix cores with bf16
- * operands; all other cases run FP32 kernels. */
+ * as operands where the reference uses them.  With round_to_bfloat16 set the
+ * attention part runs on the matrix cores: with bf16 operands at head_dim 64 and
+ * 128, to FP32 accuracy (factors as sums of three bf16 numbers) at 256; all
+ * other cases run FP32 kernels. */
 size_t pluto_hip_gqa_prefill_backward_workspace_bytes(const pluto_hip_attention_params* p,
                                                       int length, int q_weight_grad,
                                                       int k_weight_grad);

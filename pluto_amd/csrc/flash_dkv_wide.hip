@@ -186,10 +186,11 @@ flash_dkv_wide_kernel(FlashBackwardArgs a) {
 }
 
 // The same for 128 channels (gen_flash_dkv_loop128.py): the accumulators fill the
-// AGPRs, the loop statement also stores them.  Bound by the matrix pipe at the
-// clock the card keeps under it: 24 heads of 8192 rows 1313 -> 656 us (0.82
-// TFLOP, 1.26 PFLOP/s), where a wave of 32 keys with operands straight from LDS
-// was bound by the LDS reads.
+// AGPRs, the loop statement also stores them.  The matrix pipe is busy 67 % of the
+// time at the 1.86 GHz the card holds under it, with 2.4 other vector instructions to
+// a matrix instruction: 24 heads of 8192 rows 1313 -> 656 us (0.83 TFLOP, 1.27
+// PFLOP/s), where a wave of 32 keys with operands straight from LDS was bound by the
+// LDS reads.
 __global__ void __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 flash_dkv_wide128_kernel(FlashBackwardArgs a) {
   constexpr int D = 128, BNK = 128, KS = D / 16;

@@ -925,8 +925,6 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
   float* conv_partials = take(static_cast<size_t>(kConvSlices) * channels * kernel * 4);
 
   const long long elements = 1LL * length * channels;
-  // one channel a thread: four a thread (one wide access instead of four) was
-  // measured slower for the two kernels that also read the weights
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   const bool rows_aligned = aligned(qkv) && aligned(conv_weight) && aligned(dqkv);
   if (taps4) {
@@ -937,6 +935,8 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     else
       conv_train4_kernel<false><<<grid, 256, 0, stream>>>(input, conv_weight, length, channels, round, post);
   } else {
+    // one channel a thread: four (one wide access instead of four) were slower in the
+    // kernels for any number of taps that also read the weights
     conv_train_kernel<1><<<blocks_for(elements), 256, 0, stream>>>(
         static_cast<const uint16_t*>(qkv), conv_weight, length, channels, kernel, round, pre, post);
   }
