@@ -354,6 +354,46 @@ def test_layer_forward_matches_scalar_specification(capi, oracle, kh, vh, kd, vd
             assert_close(state[i].cpu().numpy(), want["state"], 2e-3, "delta-net layer state")
 
 
+def test_every_activation_rounds_as_the_scalar_kernel_rounds_it(capi):
+    """The convolution's wide kernel makes SiLU from the hardware's exponential and
+    reciprocal, the one for tensors off a 16-byte boundary from expf and a division.
+    Every bf16 argument between -80 and 80 goes through both (one token a sequence,
+    taps 0, 0, 0, 1, so that the convolution passes it on) and arrives in the state with
+    the same bits: decay and beta are the same in both calls, keys and queries too."""
+    kh, vh, d = 16, 48, 128
+    codes = torch.arange(0, 1 << 16, dtype=torch.int32, device="cuda").to(torch.int16).view(torch.bfloat16)
+    codes = codes[(codes.float().abs() <= 80) & (codes.float().abs() >= 1e-30)]
+    B = -(-codes.numel() // (vh * d))
+    channels = 2 * kh * d + vh * d
+    qkv = torch.ones(B, 1, channels, dtype=torch.bfloat16, device="cuda")
+    values = torch.ones(B * vh * d, dtype=torch.bfloat16, device="cuda")
+    values[:codes.numel()] = codes
+    qkv[:, 0, 2 * kh * d:] = values.view(B, vh * d)
+    conv = torch.zeros(channels, 4, device="cuda")
+    conv[:, 3] = 1.0
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    z = torch.randn(B, 1, vh * d, generator=gen, device="cuda").to(torch.bfloat16)
+    b = torch.full((B, 1, vh), 40.0, dtype=torch.bfloat16, device="cuda")  # beta is 1
+    zeros = torch.zeros(vh, device="cuda")
+    p = capi.delta_params(kh, vh, d, d)
+
+    def run(x):
+        state = torch.zeros(B, vh, d, d, device="cuda")
+        out = capi.gdn_layer_forward(p, x, z, torch.zeros_like(b), b, conv, zeros, zeros,
+                                     torch.ones(d, device="cuda"), state)
+        torch.cuda.synchronize()
+        return state, out
+
+    space = torch.empty(qkv.numel() + 8, dtype=torch.bfloat16, device="cuda")
+    shifted = space[1:1 + qkv.numel()].view(qkv.shape)
+    shifted.copy_(qkv)
+    wide, narrow = run(qkv), run(shifted)
+    # a row of the state holds each value once, times what all have in common
+    different = (wide[0][:, :, 0, :] != narrow[0][:, :, 0, :]).reshape(-1)
+    assert not different.any(), values[different].float().tolist()
+    assert torch.equal(wide[0], narrow[0]) and torch.equal(wide[1], narrow[1])
+
+
 @pytest.mark.parametrize("T", [1, 3, 4, 5, 15, 17, 70])
 def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T):
     """The convolution walks sixteen rows a thread where there are enough of them and
