@@ -37,8 +37,8 @@ def case(oracle, dtype, rows, n_in, n_out, seed):
 # kernels do not take (fully_connected.h:18: any positive width)
 SHAPES = [(128, 64, 64), (200, 128, 192), (77, 192, 64), (300, 64, 320), (1, 128, 128),
           (5, 7, 3), (70, 65, 129), (33, 128, 66),
-          # contractions of 1536 and more take the 256 x 256 tiles (forward:
-          # input_dim, input gradient: output_dim), here with ragged tiles
+          # long contractions (forward: input_dim, input gradient: output_dim)
+          # with ragged tiles
           (300, 1536, 64), (260, 64, 1536)]
 
 
@@ -77,7 +77,7 @@ def test_bench_shape_matches_float64_products(capi, oracle):
     """The GPT-2-small QKV projection at its full size (16384 rows, 768 ->
     2304, bf16): every output against float64 matrix products of the same
     rounded operands, computed by the library on the GPU; the weight gradient
-    there runs in four row slices and the bias gradient in 64 partitions."""
+    there runs in several row slices and the bias gradient in 64 partitions."""
     rows, n_in, n_out = 16384, 768, 2304
     g = torch.Generator(device="cuda").manual_seed(7)
     x = torch.randn(rows, n_in, device="cuda", generator=g).to(torch.bfloat16)
