@@ -18,6 +18,11 @@ struct SplitArgs {
   float* core = nullptr;      // [T, heads, 256] attention output
   float* maxima = nullptr;    // [heads, T] of the scaled scores
   float* inverses = nullptr;  // [heads, T] 1 / normalizer
+  // forward, optional: out = bf16(bf16(core) * bf16(sigmoid(gate))), [T, heads, 256], gate
+  // at [T, heads, 2, 256] + 256 of qg; lse [T, heads], maximum + log(normalizer)
+  uint16_t* out = nullptr;
+  const uint16_t* qg = nullptr;
+  float* lse = nullptr;
   // backward: the gradient of core as three bf16 tensors [T, heads, 256] whose sum
   // it is, `piece` elements apart, and its row products with core
   uint16_t* d_core = nullptr;

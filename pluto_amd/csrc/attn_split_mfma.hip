@@ -10,9 +10,12 @@
 // are 2^-24 of the product, what one FP32 rounding costs.  Per 32 x 32 block of
 // scores in products of depth 256: S 1, P V 3 (forward); S 1, dP 3, dQ 3; and
 // S 1, dP 3, dK 3, dV 6.  At sixteen times the rate of the FP32 matrix
-// instruction that is a third of its time.  T = 1024, 24/4 heads: 0.05, 0.07
-// and 0.12 ms for the three kernels, where the kernels that multiply one element
-// at a time took 3.9, 5.0 and 7.4 ms.
+// instruction that is a third of its time.  T = 1024, 24/4 heads: 0.043 (0.050
+// with the gated output), 0.065 and 0.108 ms for the three kernels, where the kernels that
+// multiply one element at a time took 3.9, 5.0 and 7.4 ms.  What bounds them: one wave a
+// SIMD in the longest workgroup's chain of tiles (16 steps of 112 matrix instructions for
+// dQ, half of whose time is softmax arithmetic, splits and waits beside an idle matrix
+// pipe), and 384 workgroups of lengths 1 to 16 on 256 compute units.
 //
 // Shape of the kernels as in flash_bwd_mfma.hip: four waves of 32 queries (keys)
 // each, tiles of 32 rows of the other side through two LDS stages filled by
@@ -21,6 +24,8 @@
 #include "attn_split_mfma.h"
 
 #include "mfma_tile.h"
+
+#include <type_traits>
 
 namespace pluto_hip {
 namespace {
@@ -94,11 +99,15 @@ struct TileAccess {
   }
 };
 
-// Nothing moves across: the operands of a step are requested before the matrix
-// instructions of the step before it, one step ahead of their use.  (Left to
-// itself the compiler requests an operand and waits for it before every one to
-// three matrix instructions: 282 us for dK/dV at T = 1024, 24 heads.)
+// Nothing moves across.  Operands are requested two or three steps ahead of their use
+// and what a step requests stands between its matrix instructions: one wave a SIMD
+// issues in order, so whatever stands before them in a burst runs beside none.  (Left to
+// itself the compiler requests an operand and waits for it before every one to three
+// matrix instructions: 282 us for dK/dV at T = 1024, 24 heads.)
 __device__ inline void fence_schedule() { __builtin_amdgcn_sched_barrier(0); }
+
+// Barrier for data exchanged through LDS: requests from memory stay under way.
+__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 __device__ inline void stage_ready() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -106,10 +115,11 @@ __device__ inline void stage_ready() {
 }
 
 // The two query-owned kernels: a workgroup owns 64 queries, waves 0 and 1 the two
-// halves at even key tiles, waves 2 and 3 the same at odd ones, and the upper
-// waves' results are added in at the end.  One wave a SIMD has nothing to cover
+// halves at even key tiles, waves 2 and 3 the same at odd ones, and the waves of a
+// half add up what they have at the end.  One wave a SIMD has nothing to cover
 // the chain scores -> softmax -> products of a tile; at T = 1024 the longest chain
-// is what the kernel takes, and this halves it (forward 79 -> 52 us, dQ 103 -> 70).
+// is what the kernel takes, and this halves it (forward 79 -> 52 us, dQ 103 -> 70
+// when it was made).
 constexpr int kQueries = 64;
 constexpr int kQueryStageBytes = 4 * kTileBytes;  // K and V of two tiles
 struct QueryWave {
@@ -125,45 +135,81 @@ struct QueryWave {
     query_load = min(query, a.length - 1);
   }
 };
-// Queues the fill of step's two tiles: K, V of the even one, K, V of the odd one.
-__device__ inline void fill_query_stage(const SplitArgs& a, unsigned char* lds, int step, int wave,
-                                        int head, const uint32_t* offsets) {
-  const long long kv_row = 1LL * (a.heads / a.group) * D;
-  const long long column = head / a.group * D;
-  unsigned char* stage = lds + (step & 1) * kQueryStageBytes;
+// The fill of a step's two tiles, K, V of the even one, then of the odd one: sixteen
+// requests a wave, dealt out between its products.  Issued together behind the barrier
+// they queue at the compute unit's one address path (16 cycles each, four waves) while no
+// wave computes (T = 1024, 24 heads: forward 50, dQ 67, dK/dV 118 us that way).  The
+// descriptors stay, the lanes' offsets move from step to step; rows beyond the tensor read
+// zero.
+struct QueryFill {
+  int32x4 rsrc[4];
+  uint32_t stage, advance, offsets[kLoads];
+  __device__ QueryFill(const SplitArgs& a, unsigned char* lds, int wave, int head, const TileAccess& at) {
+    const long long kv_row = 1LL * (a.heads / a.group) * D;
+    const long long column = head / a.group * D;
+    stage = lds_address(lds + wave * kLoads * 1024);
 #pragma unroll
-  for (int tile = 0; tile < 2; ++tile) {
-    const int k0 = (2 * step + tile) * kRows;
-    tile_fill<D, kLoads>(stage + 2 * tile * kTileBytes, wave, a.k + column + k0 * kv_row, kv_row, k0,
-                         a.length, offsets);
-    tile_fill<D, kLoads>(stage + (2 * tile + 1) * kTileBytes, wave, a.v + column + k0 * kv_row,
-                         kv_row, k0, a.length, offsets);
+    for (int tile = 0; tile < 2; ++tile) {
+      const uint32_t bytes = tile_bytes<D>(tile * kRows, a.length, kv_row);
+      rsrc[2 * tile] = make_rsrc(a.k + column + tile * kRows * kv_row, bytes);
+      rsrc[2 * tile + 1] = make_rsrc(a.v + column + tile * kRows * kv_row, bytes);
+    }
+    advance = static_cast<uint32_t>(2 * kRows * kv_row * 2);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) offsets[i] = at.fill[i];
   }
-}
-// The accumulators of the upper waves into LDS, 32 KiB each.
-__device__ inline void store_upper(unsigned char* lds, int half, int lane, const floatx16 (&acc)[DB]) {
-  float4* area = reinterpret_cast<float4*>(lds + half * 2 * kTileBytes);
+  __device__ void next_step() {
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+    for (int i = 0; i < kLoads; ++i) offsets[i] += advance;
+  }
+  __device__ void request(int step, int i) const {
+    const uint32_t at = __builtin_amdgcn_readfirstlane(stage + (step & 1) * kQueryStageBytes);
+    lds_fill_at<16>(rsrc[i / kLoads], at + i / kLoads * kTileBytes + i % kLoads * 1024, offsets[i % kLoads]);
+  }
+  __device__ void request_all(int step) const {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      area[(4 * db + j) * 64 + lane] =
-          make_float4(acc[db][4 * j], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]);
+    for (int i = 0; i < 4 * kLoads; ++i) request(step, i);
+  }
+};
+// The end of the query-owned kernels: of the two waves of a half, which hold sums of the
+// even and of the odd key tiles, the lower finishes channels 0..127 and the upper the
+// others (with one wave finishing all of them the gated forward took 61 us instead of
+// 50-55).
+constexpr int kHalfBlocks = DB / 2;
+template <int FIRST>
+__device__ inline void hand_over(unsigned char* lds, int half, int lane, const floatx16 (&acc)[DB]) {
+  float4* area = reinterpret_cast<float4*>(lds + (2 * half + FIRST / kHalfBlocks) * kTileBytes);
+#pragma unroll
+  for (int i = 0; i < kHalfBlocks; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const floatx16& from = acc[FIRST + i];
+      area[(4 * i + j) * 64 + lane] = make_float4(from[4 * j], from[4 * j + 1], from[4 * j + 2], from[4 * j + 3]);
+    }
 }
-__device__ inline float4 load_upper(const unsigned char* lds, int half, int lane, int piece) {
-  return reinterpret_cast<const float4*>(lds + half * 2 * kTileBytes)[piece * 64 + lane];
+// Four channels of block FIRST + i, registers 4 j .. 4 j + 3, of the other wave.
+template <int FIRST>
+__device__ inline float4 handed_over(const unsigned char* lds, int half, int lane, int i, int j) {
+  return reinterpret_cast<const float4*>(lds + (2 * half + FIRST / kHalfBlocks) * kTileBytes)[(4 * i + j) * 64 + lane];
 }
 
+// What the forward leaves beside core and its statistics: the backward's own forward
+// nothing, a layer's forward the gated output, stored eight bytes at a time where the
+// caller's tensors allow that.
+enum class Gated { kNone, kWide, kNarrow };
+
+template <Gated OUTPUT>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 split_forward_kernel(SplitArgs a) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQueryStageBytes];
-  __shared__ float upper_stats[2][2][64];
+  __shared__ float wave_stats[2][2][2][64];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
   const QueryWave w(a, wave, n);
   const int T = a.length, query = w.query, query_load = w.query_load, head = w.head;
   const long long q_row = 1LL * a.heads * D;
   const TileAccess at(wave, lane, 1LL * (a.heads / a.group) * D);
-  fill_query_stage(a, lds, 0, wave, head, at.fill);
+  QueryFill fill(a, lds, wave, head, at);
+  fill.request_all(0);
   bf16x8 qf[KS];
   load_row_operand(a.q + query_load * q_row + head * D, h, qf);
   floatx16 o[DB];
@@ -173,25 +219,27 @@ split_forward_kernel(SplitArgs a) {
   for (int step = 0; step < w.steps; ++step) {
     const int k0 = (2 * step + w.parity) * kRows;
     stage_ready();
-    if (step + 1 < w.steps) fill_query_stage(a, lds, step + 1, wave, head, at.fill);
-    if (k0 > w.first_query + 31) continue;  // every key follows my queries
+    fill.next_step();
+    if (k0 > w.first_query + 31) {  // every key follows my queries
+      fill.request_all(step + 1);
+      continue;
+    }
     const unsigned char* k_tile = lds + (step & 1) * kQueryStageBytes + w.parity * 2 * kTileBytes;
     const unsigned char* v_tile = k_tile + kTileBytes;
     floatx16 s = zero16();
     {
-      bf16x8 kf[2][4];
+      bf16x8 kf[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) kf[0][i] = at.row(k_tile, i);
+      for (int ks = 0; ks < 3; ++ks) kf[ks] = at.row(k_tile, ks);
 #pragma unroll
-      for (int g = 0; g < KS / 4; ++g) {
-        if (g + 1 < KS / 4)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) kf[(g + 1) % 2][i] = at.row(k_tile, 4 * (g + 1) + i);
+      for (int ks = 0; ks < KS; ++ks) {
         fence_schedule();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s = mfma32(kf[g % 2][i], qf[4 * g + i], s);
+        s = mfma32(kf[ks % 4], qf[ks], s);
         fence_schedule();
+        if (ks + 3 < KS) kf[(ks + 3) % 4] = at.row(k_tile, ks + 3);
+        if (ks % 2 == 1) fill.request(step + 1, ks / 2);
       }
+      fence_schedule();
     }
     bf16x8 vt[3];
     vt[0] = at.transposed(v_tile, 0, 0);
@@ -227,46 +275,91 @@ split_forward_kernel(SplitArgs a) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         const int at_step = s2 * DB + db;
-        if (at_step + 2 < 2 * DB)
-          vt[(at_step + 2) % 3] = at.transposed(v_tile, (at_step + 2) % DB, (at_step + 2) / DB);
-        fence_schedule();
 #pragma unroll
-        for (int part = 2; part >= 0; --part) o[db] = mfma32(vt[at_step % 3], p.part[part], o[db]);
-        fence_schedule();
+        for (int part = 2; part >= 0; --part) {
+          fence_schedule();
+          o[db] = mfma32(vt[at_step % 3], p.part[part], o[db]);
+          fence_schedule();
+          if (part == 2 && at_step + 2 < 2 * DB)
+            vt[(at_step + 2) % 3] = at.transposed(v_tile, (at_step + 2) % DB, (at_step + 2) / DB);
+          if (part == 1 && at_step < 2 * kLoads) fill.request(step + 1, 2 * kLoads + at_step);
+        }
       }
     }
   }
-  __syncthreads();  // nobody reads the stages any more
-  if (w.parity == 1) {
-    store_upper(lds, w.half, lane, o);
-    upper_stats[w.half][0][lane] = running_max;
-    upper_stats[w.half][1][lane] = running_sum;
-  }
-  __syncthreads();
-  if (w.parity == 1 || query >= T) return;
-  // a wave without tiles contributes weight 2^(kMasked - maximum) = 0
-  const float upper_max = upper_stats[w.half][0][lane];
-  const float maximum = fmaxf(running_max, upper_max);
-  const float own = __builtin_amdgcn_exp2f((running_max - maximum) * kLog2e);
-  const float other = __builtin_amdgcn_exp2f((upper_max - maximum) * kLog2e);
-  const float sum = running_sum * own + upper_stats[w.half][1][lane] * other;
-  const float inverse = 1.0f / (sum > 0.0f ? sum : 1.0f);
-  float* out = a.core + query * q_row + head * D + 4 * h;
+  stage_ready();  // nobody reads the stages any more, or fills one
+  if (w.parity == 0)
+    hand_over<kHalfBlocks>(lds, w.half, lane, o);
+  else
+    hand_over<0>(lds, w.half, lane, o);
+  wave_stats[w.half][w.parity][0][lane] = running_max;
+  wave_stats[w.half][w.parity][1][lane] = running_sum;
+  const long long unit = 1LL * query_load * a.heads + head;
+  auto finish = [&](auto first) {
+    constexpr int FIRST = decltype(first)::value;
+    const long long at_channel = 32 * FIRST + 4 * h;
+    // the gates travel while the waves meet
+    [[maybe_unused]] uint2 gates[kHalfBlocks][4];
+    [[maybe_unused]] const uint16_t* gate = a.qg + (2 * unit + 1) * D + at_channel;
+    if constexpr (OUTPUT == Gated::kWide) {
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+      for (int i = 0; i < kHalfBlocks; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float4 u = load_upper(lds, w.half, lane, 4 * db + j);
-      *reinterpret_cast<float4*>(out + 32 * db + 8 * j) =
-          make_float4((o[db][4 * j] * own + u.x * other) * inverse,
-                      (o[db][4 * j + 1] * own + u.y * other) * inverse,
-                      (o[db][4 * j + 2] * own + u.z * other) * inverse,
-                      (o[db][4 * j + 3] * own + u.w * other) * inverse);
+        for (int j = 0; j < 4; ++j) gates[i][j] = *reinterpret_cast<const uint2*>(gate + 32 * i + 8 * j);
     }
-  if (h == 0) {
-    a.maxima[1LL * head * T + query] = maximum;
-    a.inverses[1LL * head * T + query] = inverse;
-  }
+    lds_barrier();
+    if (query >= T) return;
+    // a wave without tiles has weight 2^(kMasked - maximum) = 0
+    const float other_max = wave_stats[w.half][1 - w.parity][0][lane];
+    const float maximum = fmaxf(running_max, other_max);
+    const float own = __builtin_amdgcn_exp2f((running_max - maximum) * kLog2e);
+    const float other = __builtin_amdgcn_exp2f((other_max - maximum) * kLog2e);
+    const float own_sum = running_sum * own, other_sum = wave_stats[w.half][1 - w.parity][1][lane] * other;
+    const float sum = own_sum + other_sum;
+    const float inverse = 1.0f / (sum > 0.0f ? sum : 1.0f);
+    float* out = a.core + unit * D + at_channel;
+#pragma unroll
+    for (int i = 0; i < kHalfBlocks; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 u = handed_over<FIRST>(lds, w.half, lane, i, j);
+        const floatx16& from = o[FIRST + i];
+        const float c[4] = {(from[4 * j] * own + u.x * other) * inverse, (from[4 * j + 1] * own + u.y * other) * inverse,
+                            (from[4 * j + 2] * own + u.z * other) * inverse,
+                            (from[4 * j + 3] * own + u.w * other) * inverse};
+        *reinterpret_cast<float4*>(out + 32 * i + 8 * j) = make_float4(c[0], c[1], c[2], c[3]);
+        if constexpr (OUTPUT != Gated::kNone) {
+          // qwen_attention.cc:103-108
+          uint16_t* gated = a.out + unit * D + at_channel + 32 * i + 8 * j;
+          float logits[4], g[4];
+          if constexpr (OUTPUT == Gated::kWide) {
+            const uint2 bits = gates[i][j];
+            logits[0] = __uint_as_float(bits.x << 16), logits[1] = __uint_as_float(bits.x & 0xffff0000u);
+            logits[2] = __uint_as_float(bits.y << 16), logits[3] = __uint_as_float(bits.y & 0xffff0000u);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) logits[e] = bf16_bits_to_float(gate[32 * i + 8 * j + e]);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) g[e] = round_to_bf16(c[e]) * round_to_bf16(gate_sigmoid(logits[e]));
+          if constexpr (OUTPUT == Gated::kWide) {
+            *reinterpret_cast<uint2*>(gated) = make_uint2(pack_bf16(g[0], g[1]), pack_bf16(g[2], g[3]));
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gated[e] = float_to_bf16_bits(g[e]);
+          }
+        }
+      }
+    if (FIRST == 0 && h == 0) {
+      a.maxima[1LL * head * T + query] = maximum;
+      a.inverses[1LL * head * T + query] = inverse;
+      if (OUTPUT != Gated::kNone && a.lse) a.lse[unit] = maximum + logf(sum > 0.0f ? sum : 1.0f);
+    }
+  };
+  if (w.parity == 0)
+    finish(std::integral_constant<int, 0>());
+  else
+    finish(std::integral_constant<int, kHalfBlocks>());
 }
 
 // 32 lanes a row, eight channels a lane; a workgroup walks 64 rows of one head.
@@ -319,7 +412,8 @@ split_dq_kernel(SplitArgs a) {
   const int T = a.length, query = w.query, query_load = w.query_load, head = w.head;
   const long long q_row = 1LL * a.heads * D;
   const TileAccess at(wave, lane, 1LL * (a.heads / a.group) * D);
-  fill_query_stage(a, lds, 0, wave, head, at.fill);
+  QueryFill fill(a, lds, wave, head, at);
+  fill.request_all(0);
   bf16x8 qf[KS], gf[3][KS];
   load_row_operand(a.q + query_load * q_row + head * D, h, qf);
 #pragma unroll
@@ -333,8 +427,11 @@ split_dq_kernel(SplitArgs a) {
   for (int step = 0; step < w.steps; ++step) {
     const int k0 = (2 * step + w.parity) * kRows;
     stage_ready();
-    if (step + 1 < w.steps) fill_query_stage(a, lds, step + 1, wave, head, at.fill);
-    if (k0 > w.first_query + 31) continue;  // every key follows my queries
+    fill.next_step();
+    if (k0 > w.first_query + 31) {  // every key follows my queries
+      fill.request_all(step + 1);
+      continue;
+    }
     const unsigned char* k_tile = lds + (step & 1) * kQueryStageBytes + w.parity * 2 * kTileBytes;
     const unsigned char* v_tile = k_tile + kTileBytes;
     floatx16 s = zero16(), dp = zero16();
@@ -346,14 +443,17 @@ split_dq_kernel(SplitArgs a) {
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      if (ks + 2 < KS) {
-        kf[(ks + 2) % 3] = at.row(k_tile, ks + 2);
-        vf[(ks + 2) % 3] = at.row(v_tile, ks + 2);
-      }
       fence_schedule();
       s = mfma32(kf[ks % 3], qf[ks], s);
 #pragma unroll
-      for (int part = 2; part >= 0; --part) dp = mfma32(vf[ks % 3], gf[part][ks], dp);
+      for (int part = 2; part >= 0; --part) {
+        fence_schedule();
+        if (part == 2 && ks + 2 < KS) kf[(ks + 2) % 3] = at.row(k_tile, ks + 2);
+        if (part == 1 && ks + 2 < KS) vf[(ks + 2) % 3] = at.row(v_tile, ks + 2);
+        if (part == 0) fill.request(step + 1, ks);
+        fence_schedule();
+        dp = mfma32(vf[ks % 3], gf[part][ks], dp);
+      }
       fence_schedule();
     }
     bf16x8 kt[3];
@@ -365,7 +465,9 @@ split_dq_kernel(SplitArgs a) {
     for (int i = 0; i < 16; ++i) {
       const float p =
           __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale, -maximum) * kLog2e) * inverse;
-      s[i] = 8 * (i / 4) + (i % 4) > limit ? 0.0f : p * (dp[i] - delta);
+      float ds = p * (dp[i] - delta);
+      asm("" : "+v"(ds));  // in every lane: no branch around it
+      s[i] = 8 * (i / 4) + (i % 4) > limit ? 0.0f : ds;
     }
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
@@ -373,29 +475,42 @@ split_dq_kernel(SplitArgs a) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         const int at_step = s2 * DB + db;
-        if (at_step + 2 < 2 * DB)
-          kt[(at_step + 2) % 3] = at.transposed(k_tile, (at_step + 2) % DB, (at_step + 2) / DB);
-        fence_schedule();
 #pragma unroll
-        for (int part = 2; part >= 0; --part) dq[db] = mfma32(kt[at_step % 3], ds.part[part], dq[db]);
-        fence_schedule();
+        for (int part = 2; part >= 0; --part) {
+          fence_schedule();
+          dq[db] = mfma32(kt[at_step % 3], ds.part[part], dq[db]);
+          fence_schedule();
+          if (part == 2 && at_step + 2 < 2 * DB)
+            kt[(at_step + 2) % 3] = at.transposed(k_tile, (at_step + 2) % DB, (at_step + 2) / DB);
+        }
       }
     }
   }
-  __syncthreads();  // nobody reads the stages any more
-  if (w.parity == 1) store_upper(lds, w.half, lane, dq);
+  stage_ready();  // nobody reads the stages any more, or fills one
+  if (w.parity == 0)
+    hand_over<kHalfBlocks>(lds, w.half, lane, dq);
+  else
+    hand_over<0>(lds, w.half, lane, dq);
   __syncthreads();
-  if (w.parity == 1 || query >= T) return;
-  float* out = a.dq + query * q_row + head * D + 4 * h;
+  if (query >= T) return;
+  auto finish = [&](auto first) {
+    constexpr int FIRST = decltype(first)::value;
+    float* out = a.dq + query * q_row + head * D + 32 * FIRST + 4 * h;
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+    for (int i = 0; i < kHalfBlocks; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float4 u = load_upper(lds, w.half, lane, 4 * db + j);
-      *reinterpret_cast<float4*>(out + 32 * db + 8 * j) =
-          make_float4((dq[db][4 * j] + u.x) * a.scale, (dq[db][4 * j + 1] + u.y) * a.scale,
-                      (dq[db][4 * j + 2] + u.z) * a.scale, (dq[db][4 * j + 3] + u.w) * a.scale);
-    }
+      for (int j = 0; j < 4; ++j) {
+        const float4 u = handed_over<FIRST>(lds, w.half, lane, i, j);
+        const floatx16& from = dq[FIRST + i];
+        *reinterpret_cast<float4*>(out + 32 * i + 8 * j) =
+            make_float4((from[4 * j] + u.x) * a.scale, (from[4 * j + 1] + u.y) * a.scale,
+                        (from[4 * j + 2] + u.z) * a.scale, (from[4 * j + 3] + u.w) * a.scale);
+      }
+  };
+  if (w.parity == 0)
+    finish(std::integral_constant<int, 0>());
+  else
+    finish(std::integral_constant<int, kHalfBlocks>());
 }
 
 constexpr int kKeys = 128;  // of a workgroup of the key-owned kernel
@@ -416,21 +531,31 @@ __device__ __forceinline__ void split_key_owned(const SplitArgs& a, unsigned cha
   const int first_key = k0 + 32 * wave, key = first_key + n, key_load = min(key, T - 1);
   const TileAccess at(wave, lane, q_row);
   const int first_tile = k0 / kRows, tiles = (T + kRows - 1) / kRows;
-  auto fill = [&](int tile) {
-    unsigned char* stage = lds + (tile & 1) * kDkvStageBytes;
-    const int q0 = tile * kRows;
-    tile_fill<D, kLoads>(stage, wave, a.q + head * D + q0 * q_row, q_row, q0, T, at.fill);
+  // A tile's requests, as in QueryFill; the first brings the rows' statistics as well.
+  const uint32_t bytes = tile_bytes<D>(0, T, q_row);
+  int32x4 rsrc[4];
+  rsrc[0] = make_rsrc(a.q + head * D, bytes);
 #pragma unroll
-    for (int part = 0; part < 3; ++part)
-      tile_fill<D, kLoads>(stage + (1 + part) * kTileBytes, wave,
-                           a.d_core + part * a.piece + head * D + q0 * q_row, q_row, q0, T, at.fill);
-    if (wave < 3) {
-      const float* source = wave == 0 ? a.maxima : wave == 1 ? a.inverses : a.deltas;
-      const int32x4 rsrc = make_rsrc(source + 1LL * head * T + q0, static_cast<uint32_t>(T - q0) * 4u);
-      lds_fill<4>(rsrc, stage + 4 * kTileBytes + wave * 256, lane * 4);
-    }
+  for (int part = 0; part < 3; ++part) rsrc[1 + part] = make_rsrc(a.d_core + part * a.piece + head * D, bytes);
+  const float* stats_of_wave = wave == 0 ? a.maxima : wave == 1 ? a.inverses : a.deltas;
+  const int32x4 stats_rsrc = make_rsrc(stats_of_wave + 1LL * head * T, static_cast<uint32_t>(T) * 4u);
+  const uint32_t tile_stage = lds_address(lds + wave * kLoads * 1024),
+                 stats_stage = lds_address(lds + 4 * kTileBytes + wave * 256);
+  const uint32_t advance = static_cast<uint32_t>(kRows * q_row * 2);
+  uint32_t offsets[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) offsets[i] = at.fill[i] + first_tile * advance;
+  auto request = [&](int tile, int i) {
+    const uint32_t stage = __builtin_amdgcn_readfirstlane((tile & 1) * kDkvStageBytes);
+    lds_fill_at<16>(rsrc[i / kLoads], tile_stage + stage + i / kLoads * kTileBytes + i % kLoads * 1024,
+                    offsets[i % kLoads]);
+    if (i == 0 && wave < 3) lds_fill_at<4>(stats_rsrc, stats_stage + stage, lane * 4 + tile * (kRows * 4));
   };
-  fill(first_tile);
+  auto request_all = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < 4 * kLoads; ++i) request(tile, i);
+  };
+  request_all(first_tile);
   bf16x8 kf[KS], vf[VALUES ? 1 : KS];
   load_row_operand(a.k + key_load * kv_row + head / a.group * D, h, kf);
   if constexpr (!VALUES) load_row_operand(a.v + key_load * kv_row + head / a.group * D, h, vf);
@@ -440,57 +565,65 @@ __device__ __forceinline__ void split_key_owned(const SplitArgs& a, unsigned cha
   for (int tile = first_tile; tile < tiles; ++tile) {
     const int q0 = tile * kRows;
     stage_ready();
-    if (tile + 1 < tiles) fill(tile + 1);
-    if (q0 + 31 < first_key) continue;  // every query precedes my keys
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) offsets[i] += advance;
+    if (q0 + 31 < first_key) {  // every query precedes my keys
+      request_all(tile + 1);
+      continue;
+    }
     const unsigned char* q_tile = lds + (tile & 1) * kDkvStageBytes;
     const unsigned char* g_tile = q_tile + kTileBytes;
     const float* stats = reinterpret_cast<const float*>(q_tile + 4 * kTileBytes);
     floatx16 s = zero16(), dp = zero16();
     if constexpr (VALUES) {
-      bf16x8 qa[2][4];
+      bf16x8 qa[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) qa[0][i] = at.row(q_tile, i);
-#pragma unroll
-      for (int g = 0; g < KS / 4; ++g) {
-        if (g + 1 < KS / 4)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) qa[(g + 1) % 2][i] = at.row(q_tile, 4 * (g + 1) + i);
-        fence_schedule();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s = mfma32(qa[g % 2][i], kf[4 * g + i], s);
-        fence_schedule();
-      }
-    } else {
-      bf16x8 qa[3], ga[3][3];
-      auto request = [&](int ks) {
-        qa[ks % 3] = at.row(q_tile, ks);
-#pragma unroll
-        for (int part = 0; part < 3; ++part)
-          ga[ks % 3][part] = at.row(g_tile + part * kTileBytes, ks);
-      };
-      request(0);
-      request(1);
+      for (int ks = 0; ks < 3; ++ks) qa[ks] = at.row(q_tile, ks);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 2 < KS) request(ks + 2);
+        fence_schedule();
+        s = mfma32(qa[ks % 4], kf[ks], s);
+        fence_schedule();
+        if (ks + 3 < KS) qa[(ks + 3) % 4] = at.row(q_tile, ks + 3);
+        if (ks % 2 == 1) request(tile + 1, ks / 2);
+      }
+      fence_schedule();
+    } else {
+      bf16x8 qa[3], ga[3][3];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        qa[ks] = at.row(q_tile, ks);
+#pragma unroll
+        for (int part = 0; part < 3; ++part) ga[ks][part] = at.row(g_tile + part * kTileBytes, ks);
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
         fence_schedule();
         s = mfma32(qa[ks % 3], kf[ks], s);
-#pragma unroll
-        for (int part = 2; part >= 0; --part) dp = mfma32(ga[ks % 3][part], vf[ks], dp);
         fence_schedule();
+        if (ks + 2 < KS) qa[(ks + 2) % 3] = at.row(q_tile, ks + 2);
+        request(tile + 1, ks);
+#pragma unroll
+        for (int part = 2; part >= 0; --part) {
+          fence_schedule();
+          dp = mfma32(ga[ks % 3][part], vf[ks], dp);
+          fence_schedule();
+          if (ks + 2 < KS) ga[(ks + 2) % 3][part] = at.row(g_tile + part * kTileBytes, ks + 2);
+        }
       }
+      fence_schedule();
     }
     // transposed operands of step (s2, db): dC's pieces for dV, Q for dK
     constexpr int kAhead = VALUES ? 1 : 2, kParts = VALUES ? 3 : 1;
     bf16x8 t[kAhead + 1][kParts];
-    auto request_transposed = [&](int step) {
-#pragma unroll
-      for (int part = 0; part < kParts; ++part)
-        t[step % (kAhead + 1)][part] = at.transposed(VALUES ? g_tile + part * kTileBytes : q_tile,
-                                                     step % DB, step / DB);
+    auto read_transposed = [&](int step, int part) {
+      t[step % (kAhead + 1)][part] =
+          at.transposed(VALUES ? g_tile + part * kTileBytes : q_tile, step % DB, step / DB);
     };
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) request_transposed(i);
+    for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+      for (int part = 0; part < kParts; ++part) read_transposed(i, part);
     fence_schedule();
     // register i = (query q0 + 8(i/4) + 4h + i%4, key n)
     const int first = key - q0 - 4 * h, last = T - 1 - q0 - 4 * h;
@@ -516,17 +649,20 @@ __device__ __forceinline__ void split_key_owned(const SplitArgs& a, unsigned cha
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         const int step = s2 * DB + db;
-        if (step + kAhead < 2 * DB) request_transposed(step + kAhead);
-        fence_schedule();
 #pragma unroll
         for (int gp = kParts - 1; gp >= 0; --gp)
 #pragma unroll
-          for (int part = 2 - gp; part >= 0; --part)
+          for (int part = 2 - gp; part >= 0; --part) {
+            fence_schedule();
             acc[db] = mfma32(t[step % (kAhead + 1)][gp], p.part[part], acc[db]);
-        fence_schedule();
+            fence_schedule();
+            if (part == 2 - gp && step + kAhead < 2 * DB) read_transposed(step + kAhead, gp);
+            if (VALUES && gp == 0 && part == 1 && step < 2 * kLoads) request(tile + 1, 2 * kLoads + step);
+          }
       }
     }
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the requests beyond the last tile
   if (key >= T) return;
   const float factor = VALUES ? 1.0f : a.scale;
   float* out = (VALUES ? a.dv : a.dk) + key * q_row + head * D + 4 * h;
@@ -561,7 +697,14 @@ bool split_attention_supported(int length, int heads, int head_dim) {
 }
 
 int launch_split_forward(hipStream_t stream, const SplitArgs& a) {
-  split_forward_kernel<<<tile_grid(a, kQueries), kThreads, 0, stream>>>(a);
+  auto launch = [&](auto kernel) { kernel<<<tile_grid(a, kQueries), kThreads, 0, stream>>>(a); };
+  const bool wide = ((reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.qg)) & 7u) == 0;
+  if (!a.out)
+    launch(split_forward_kernel<Gated::kNone>);
+  else if (wide)
+    launch(split_forward_kernel<Gated::kWide>);
+  else
+    launch(split_forward_kernel<Gated::kNarrow>);
   return launch_status();
 }
 

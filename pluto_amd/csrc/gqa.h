@@ -28,6 +28,11 @@ struct PrefillPrepareArgs {
   void* q_out = nullptr;  // [T, qh, d], bf16 when rounding, else fp32
   int q_out_dtype = PLUTO_HIP_BF16;
   CacheView cache;
+  // optional second copies for the backward pass, 16-byte aligned: the prepared queries
+  // [T, qh, d] as q_out, keys and values [T, kh, d] in the cache's storage
+  void* q_copy = nullptr;
+  void* k_copy = nullptr;
+  void* v_copy = nullptr;
   int length = 0, start_position = 0;
   int query_heads = 0, key_value_heads = 0, head_dim = 0, rotary_dim = 0;
   float epsilon = 1e-6f;

@@ -196,24 +196,44 @@ long long decode_blocks_bound(const pluto_hip_attention_params* p, int batch, co
   return blocks;
 }
 
-// What the forward pass can leave for the backward pass: the attention output
-// before the gate (bf16 [length, qh * d]) and the two row statistics (fp32
-// [qh, length] each), as the matrix-core backward kernels read them.
+// What the forward pass can leave for the backward pass, from the block's first multiple of
+// 256 bytes on: the attention output before the gate (bf16 at head width 64 and 128, FP32
+// at 256, [length, qh * d]) and the two row statistics (fp32 [qh, length] each), as the
+// matrix-core backward kernels read them, and what the preparation made: the normalised
+// and rotated heads (bf16) and the rotation's table.  The copies cost the forward 4 us at
+// 8192 rows of 24 + 4 heads of 128, making them again took the backward 42.
 struct SavedLayout {
-  size_t core, maxima, normalizers, total;
+  size_t core, maxima, normalizers, queries, keys, values, cosines, sines, total;
 };
 SavedLayout saved_layout(const pluto_hip_attention_params* p, int length) {
   SavedLayout l{};
-  const size_t rows = static_cast<size_t>(length) * p->query_heads;
-  l.core = 0;
-  l.maxima = align_up(rows * p->head_dim * 2, 256);
-  l.normalizers = l.maxima + align_up(rows * 4, 256);
-  l.total = l.normalizers + align_up(rows * 4, 256);
+  const size_t T = static_cast<size_t>(length), d = p->head_dim;
+  const size_t rows = T * p->query_heads, kv_rows = T * p->key_value_heads;
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t offset = at;
+    at += align_up(bytes, 256);
+    return offset;
+  };
+  l.core = take(rows * d * (d == kSplitHeadDim ? 4 : 2));
+  l.maxima = take(rows * 4);
+  l.normalizers = take(rows * 4);
+  l.queries = take(rows * d * 2);
+  l.keys = take(kv_rows * d * 2);
+  l.values = take(kv_rows * d * 2);
+  l.cosines = take(T * (p->rotary_dim / 2) * 4);
+  l.sines = take(T * (p->rotary_dim / 2) * 4);
+  l.total = at + 256;
   return l;
 }
-bool saved_supported(const pluto_hip_attention_params* p, int cache_dtype) {
+char* saved_base(const void* saved) {
+  return reinterpret_cast<char*>(align_up(reinterpret_cast<size_t>(saved), 256));
+}
+bool saved_supported(const pluto_hip_attention_params* p, int length, int cache_dtype) {
   return p->round_to_bfloat16 && cache_dtype == PLUTO_HIP_BF16 &&
-         (p->head_dim == 64 || p->head_dim == 128) && !force_generic();
+         (p->head_dim == 64 || p->head_dim == 128 ||
+          split_attention_supported(length, p->query_heads, p->head_dim)) &&
+         !force_generic();
 }
 
 }  // namespace
@@ -234,7 +254,8 @@ size_t pluto_hip_gqa_prefill_workspace_bytes(const pluto_hip_attention_params* p
 
 size_t pluto_hip_gqa_prefill_saved_bytes(const pluto_hip_attention_params* p, int length,
                                          int cache_dtype) {
-  if (validate_params(p) != 0 || length <= 0 || !saved_supported(p, cache_dtype)) return 0;
+  if (validate_params(p) != 0 || length <= 0 || !saved_supported(p, length, cache_dtype))
+    return 0;
   return saved_layout(p, length).total;
 }
 
@@ -252,7 +273,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   // cached_attention_ops.cc:318-320: appending beyond capacity fails first.
   if (static_cast<long long>(start_position) + length > p->capacity) return PLUTO_HIP_ERANGE;
   // the saved state describes a whole sequence attended from position 0
-  if (saved && (start_position != 0 || !saved_supported(p, cache->dtype)))
+  if (saved && (start_position != 0 || !saved_supported(p, length, cache->dtype)))
     return PLUTO_HIP_EUNSUPPORTED;
   const PrefillLayout layout = prefill_layout(p, length);
   if (!workspace || workspace_bytes < layout.partial) return PLUTO_HIP_EWORKSPACE;
@@ -285,11 +306,42 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   prep.theta = p->rope_theta;
   prep.epsilon = p->rms_norm_epsilon;
   prep.round = round;
+  const SavedLayout sl = saved ? saved_layout(p, length) : SavedLayout{};
+  char* kept = saved ? saved_base(saved) : nullptr;
+  if (saved) {
+    prep.q_copy = kept + sl.queries;
+    prep.k_copy = kept + sl.keys;
+    prep.v_copy = kept + sl.values;
+    prep.cosines = reinterpret_cast<float*>(kept + sl.cosines);
+    prep.sines = reinterpret_cast<float*>(kept + sl.sines);
+    prep.keep_table = true;
+  }
   status = launch_prefill_prepare(s, prep);
   if (status != 0) return status;
 
   const float scale = 1.0f / std::sqrt(static_cast<float>(d));
   const uint16_t* gate = static_cast<const uint16_t*>(qg) + d;
+  if (saved && d == kSplitHeadDim) {
+    // The backward at this width starts from FP32 factors: the forward makes them, and its
+    // output from them.  1024 rows of 24 / 4 heads: 44 us here, where the bf16 kernel took
+    // 36 and the backward repeated the forward in another 42.
+    SplitArgs a;
+    a.q = reinterpret_cast<const uint16_t*>(kept + sl.queries);
+    a.k = reinterpret_cast<const uint16_t*>(kept + sl.keys);
+    a.v = reinterpret_cast<const uint16_t*>(kept + sl.values);
+    a.length = length;
+    a.heads = qh;
+    a.group = qh / kh;
+    a.scale = scale;
+    a.core = reinterpret_cast<float*>(kept + sl.core);
+    a.maxima = reinterpret_cast<float*>(kept + sl.maxima);
+    a.inverses = reinterpret_cast<float*>(kept + sl.normalizers);
+    a.out = static_cast<uint16_t*>(out);
+    a.qg = static_cast<const uint16_t*>(qg);
+    a.lse = lse;
+    note_path(PLUTO_HIP_PATH_MATRIX_F32);
+    return launch_split_forward(s, a);
+  }
   if (round && cache->dtype == PLUTO_HIP_BF16 && !force_generic()) {
     FlashForwardArgs f;
     f.q = static_cast<const uint16_t*>(queries);
@@ -307,10 +359,9 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
     f.gate_head_stride = 2LL * d;
     f.lse = lse;
     if (saved) {
-      const SavedLayout sl = saved_layout(p, length);
-      f.core = reinterpret_cast<uint16_t*>(static_cast<char*>(saved) + sl.core);
-      f.maxima = reinterpret_cast<float*>(static_cast<char*>(saved) + sl.maxima);
-      f.normalizers = reinterpret_cast<float*>(static_cast<char*>(saved) + sl.normalizers);
+      f.core = reinterpret_cast<uint16_t*>(kept + sl.core);
+      f.maxima = reinterpret_cast<float*>(kept + sl.maxima);
+      f.normalizers = reinterpret_cast<float*>(kept + sl.normalizers);
     }
     f.q_rows = length;
     f.kv_rows = start_position + length;
@@ -368,53 +419,68 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
       prefill_backward_layout(p, length, dq_norm != nullptr || dk_norm != nullptr);
   if (l.attention_bytes == 0) return PLUTO_HIP_EINVAL;
   if (!workspace || workspace_bytes < l.total) return PLUTO_HIP_EWORKSPACE;
-  if (saved && !saved_supported(p, PLUTO_HIP_BF16)) return PLUTO_HIP_EUNSUPPORTED;
+  if (saved && !saved_supported(p, length, PLUTO_HIP_BF16)) return PLUTO_HIP_EUNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
   char* scratch = reinterpret_cast<char*>(align_up(reinterpret_cast<size_t>(workspace), 256));
-  float* cosines = reinterpret_cast<float*>(scratch + l.cosines);
-  float* sines = reinterpret_cast<float*>(scratch + l.sines);
+  const float* cosines = reinterpret_cast<float*>(scratch + l.cosines);
+  const float* sines = reinterpret_cast<float*>(scratch + l.sines);
   const bool round = p->round_to_bfloat16 != 0;
   const int qh = p->query_heads, kh = p->key_value_heads, d = p->head_dim;
   const int E = qh * d;
+  char *queries = scratch + l.queries, *keys = scratch + l.keys, *values = scratch + l.values;
 
-  // Recompute what the forward pass derived from the inputs: normalised,
-  // rotated q and k (PrepareKernel, qwen_attention.cc:30-63), then -- unless
-  // the forward pass saved them -- the attention core with its row statistics.
-  PrefillPrepareArgs prep;
-  prep.qg = qg;
-  prep.k = k;
-  prep.v = v;
-  prep.q_norm = q_norm;
-  prep.k_norm = k_norm;
-  prep.cosines = cosines;
-  prep.sines = sines;
-  prep.q_out = scratch + l.queries;
-  prep.q_out_dtype = l.dtype;
-  prep.cache = {scratch + l.keys, scratch + l.values, l.dtype, 1LL * kh * d, d};
-  prep.length = length;
-  prep.start_position = 0;
-  prep.query_heads = qh;
-  prep.key_value_heads = kh;
-  prep.head_dim = d;
-  prep.rotary_dim = p->rotary_dim;
-  prep.theta = p->rope_theta;
-  prep.keep_table = true;  // the gradients rotate back
-  prep.epsilon = p->rms_norm_epsilon;
-  prep.round = round;
-  status = launch_prefill_prepare(s, prep);
-  if (status != 0) return status;
-  const void* core = scratch + l.core;
+  // What the forward pass derived from the inputs -- normalised, rotated q and k
+  // (PrepareKernel, qwen_attention.cc:30-63), the attention core with its row statistics --
+  // is taken from the saved block or made again.
+  void* core = scratch + l.core;
   float* maxima = reinterpret_cast<float*>(scratch + l.maxima);
   float* normalizers = reinterpret_cast<float*>(scratch + l.normalizers);
   float* d_heads = reinterpret_cast<float*>(scratch + l.d_heads);
+  const bool kept = saved && (l.flash || l.split);
+  if (kept) {
+    const SavedLayout sl = saved_layout(p, length);
+    char* base = saved_base(saved);
+    core = base + sl.core;
+    maxima = reinterpret_cast<float*>(base + sl.maxima);
+    normalizers = reinterpret_cast<float*>(base + sl.normalizers);
+    queries = base + sl.queries;
+    keys = base + sl.keys;
+    values = base + sl.values;
+    cosines = reinterpret_cast<float*>(base + sl.cosines);
+    sines = reinterpret_cast<float*>(base + sl.sines);
+  } else {
+    PrefillPrepareArgs prep;
+    prep.qg = qg;
+    prep.k = k;
+    prep.v = v;
+    prep.q_norm = q_norm;
+    prep.k_norm = k_norm;
+    prep.cosines = reinterpret_cast<float*>(scratch + l.cosines);
+    prep.sines = reinterpret_cast<float*>(scratch + l.sines);
+    prep.q_out = queries;
+    prep.q_out_dtype = l.dtype;
+    prep.cache = {keys, values, l.dtype, 1LL * kh * d, d};
+    prep.length = length;
+    prep.start_position = 0;
+    prep.query_heads = qh;
+    prep.key_value_heads = kh;
+    prep.head_dim = d;
+    prep.rotary_dim = p->rotary_dim;
+    prep.theta = p->rope_theta;
+    prep.keep_table = true;  // the gradients rotate back
+    prep.epsilon = p->rms_norm_epsilon;
+    prep.round = round;
+    status = launch_prefill_prepare(s, prep);
+    if (status != 0) return status;
+  }
   NormBackwardGrads grads;
   if (l.flash) {
     const long long head_rows = 1LL * length * E;
     grads = {d_heads, d_heads + head_rows, d_heads + 2 * head_rows, E, E};
     FlashBackwardArgs f;
-    f.q = reinterpret_cast<const uint16_t*>(scratch + l.queries);
-    f.k = reinterpret_cast<const uint16_t*>(scratch + l.keys);
-    f.v = reinterpret_cast<const uint16_t*>(scratch + l.values);
+    f.q = reinterpret_cast<const uint16_t*>(queries);
+    f.k = reinterpret_cast<const uint16_t*>(keys);
+    f.v = reinterpret_cast<const uint16_t*>(values);
     f.q_row = E;
     f.kv_row = 1LL * kh * d;
     f.group = qh / kh;
@@ -430,13 +496,7 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
     f.num_heads = qh;
     f.head_dim = d;
     f.scale = 1.0f / std::sqrt(static_cast<float>(d));
-    if (saved) {
-      const SavedLayout sl = saved_layout(p, length);
-      const char* base = static_cast<const char*>(saved);
-      core = base + sl.core;
-      maxima = reinterpret_cast<float*>(const_cast<char*>(base) + sl.maxima);
-      normalizers = reinterpret_cast<float*>(const_cast<char*>(base) + sl.normalizers);
-    } else {
+    if (!kept) {
       FlashForwardArgs forward;
       forward.q = f.q;
       forward.k = f.k;
@@ -466,14 +526,14 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
     const long long head_rows = 1LL * length * E;
     grads = {d_heads, d_heads + head_rows, d_heads + 2 * head_rows, E, E};
     SplitArgs a;
-    a.q = reinterpret_cast<const uint16_t*>(scratch + l.queries);
-    a.k = reinterpret_cast<const uint16_t*>(scratch + l.keys);
-    a.v = reinterpret_cast<const uint16_t*>(scratch + l.values);
+    a.q = reinterpret_cast<const uint16_t*>(queries);
+    a.k = reinterpret_cast<const uint16_t*>(keys);
+    a.v = reinterpret_cast<const uint16_t*>(values);
     a.length = length;
     a.heads = qh;
     a.group = qh / kh;
     a.scale = 1.0f / std::sqrt(static_cast<float>(d));
-    a.core = reinterpret_cast<float*>(scratch + l.core);
+    a.core = static_cast<float*>(core);
     a.maxima = maxima;
     a.inverses = normalizers;
     a.d_core = reinterpret_cast<uint16_t*>(scratch + l.dc);
@@ -483,8 +543,10 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
     a.dk = d_heads + head_rows;
     a.dv = d_heads + 2 * head_rows;
     note_path(PLUTO_HIP_PATH_MATRIX_F32);
-    status = launch_split_forward(s, a);
-    if (status != 0) return status;
+    if (!kept) {
+      status = launch_split_forward(s, a);
+      if (status != 0) return status;
+    }
     status = launch_split_gate(s, a, qg, dy, dqg);
     if (status != 0) return status;
     status = launch_split_backward(s, a);

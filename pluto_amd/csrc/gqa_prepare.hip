@@ -71,7 +71,10 @@ prefill_prepare_kernel(PrefillPrepareArgs a) {
                       PLUTO_HIP_BF16};
     const long long out = (static_cast<long long>(row) * a.query_heads + head) * d;
     normalize_rotate(x, a.q_norm, d, a.rotary_dim, a.epsilon, a.round, cos_row, sin_row,
-                     [&](int c, float v) { store_element(a.q_out, out + c, a.q_out_dtype, v); });
+                     [&](int c, float v) {
+                       store_element(a.q_out, out + c, a.q_out_dtype, v);
+                       if (a.q_copy) store_element(a.q_copy, out + c, a.q_out_dtype, v);
+                     });
   } else {
     const int kv = head - a.query_heads;
     const long long in = (static_cast<long long>(row) * a.key_value_heads + kv) * d;
@@ -79,10 +82,14 @@ prefill_prepare_kernel(PrefillPrepareArgs a) {
     const long long out = static_cast<long long>(a.start_position + row) * a.cache.token_stride +
                           kv * a.cache.head_stride;
     normalize_rotate(x, a.k_norm, d, a.rotary_dim, a.epsilon, a.round, cos_row, sin_row,
-                     [&](int c, float v) { store_element(a.cache.keys, out + c, a.cache.dtype, v); });
+                     [&](int c, float v) {
+                       store_element(a.cache.keys, out + c, a.cache.dtype, v);
+                       if (a.k_copy) store_element(a.k_copy, in + c, a.cache.dtype, v);
+                     });
     for (int c = lane; c < d; c += 64) {
-      const float v = load_element(a.v, in + c, PLUTO_HIP_BF16);
-      store_element(a.cache.values, out + c, a.cache.dtype, maybe_round(v, a.round));
+      const float v = maybe_round(load_element(a.v, in + c, PLUTO_HIP_BF16), a.round);
+      store_element(a.cache.values, out + c, a.cache.dtype, v);
+      if (a.v_copy) store_element(a.v_copy, in + c, a.cache.dtype, v);
     }
   }
 }
@@ -113,15 +120,19 @@ prefill_prepare_bf16_kernel(PrefillPrepareArgs a, std::conditional_t<ANGLES, Rop
   const int kv = head - a.query_heads;
   const uint16_t* in;
   uint16_t* out;
+  uint16_t* copy;
   const float* weight;
+  // the unit's place among the heads of its side
+  const long long at = (is_query ? static_cast<long long>(row) * a.query_heads + head
+                                 : static_cast<long long>(row) * a.key_value_heads + kv) * D;
   if (is_query) {
-    in = static_cast<const uint16_t*>(a.qg) +
-         (static_cast<long long>(row) * a.query_heads + head) * 2 * D;
-    out = static_cast<uint16_t*>(a.q_out) + (static_cast<long long>(row) * a.query_heads + head) * D;
+    in = static_cast<const uint16_t*>(a.qg) + 2 * at;
+    out = static_cast<uint16_t*>(a.q_out) + at;
+    copy = static_cast<uint16_t*>(a.q_copy);
     weight = a.q_norm;
   } else {
-    in = static_cast<const uint16_t*>(a.k) +
-         (static_cast<long long>(row) * a.key_value_heads + kv) * D;
+    in = static_cast<const uint16_t*>(a.k) + at;
+    copy = static_cast<uint16_t*>(a.k_copy);
     out = static_cast<uint16_t*>(a.cache.keys) +
           static_cast<long long>(a.start_position + row) * a.cache.token_stride +
           kv * a.cache.head_stride;
@@ -197,14 +208,17 @@ prefill_prepare_bf16_kernel(PrefillPrepareArgs a, std::conditional_t<ANGLES, Rop
       result[i] = lower ? pack_bf16(a0 - b0, a1 - b1) : pack_bf16(a0 + b0, a1 + b1);
     }
   }
-  *reinterpret_cast<uint4*>(out + 8 * chunk) = make_uint4(result[0], result[1], result[2], result[3]);
+  const uint4 stored = make_uint4(result[0], result[1], result[2], result[3]);
+  *reinterpret_cast<uint4*>(out + 8 * chunk) = stored;
+  if (copy) *reinterpret_cast<uint4*>(copy + at + 8 * chunk) = stored;
   if (!is_query) {
-    const uint16_t* v_in = static_cast<const uint16_t*>(a.v) +
-                           (static_cast<long long>(row) * a.key_value_heads + kv) * D;
+    const uint16_t* v_in = static_cast<const uint16_t*>(a.v) + at;
     uint16_t* v_out = static_cast<uint16_t*>(a.cache.values) +
                       static_cast<long long>(a.start_position + row) * a.cache.token_stride +
                       kv * a.cache.head_stride;
-    *reinterpret_cast<uint4*>(v_out + 8 * chunk) = *reinterpret_cast<const uint4*>(v_in + 8 * chunk);
+    const uint4 value = *reinterpret_cast<const uint4*>(v_in + 8 * chunk);
+    *reinterpret_cast<uint4*>(v_out + 8 * chunk) = value;
+    if (a.v_copy) *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.v_copy) + at + 8 * chunk) = value;
   }
 }
 

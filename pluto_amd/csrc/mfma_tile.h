@@ -206,6 +206,13 @@ __device__ inline float4 quad_transpose(float4 v) {
 // reads (four consecutive rows x two adjacent chunks -> eight different slots).
 __device__ inline int tile_swizzle(int row) { return 2 * (row & 3) + ((row >> 2) & 1); }
 
+// Bytes from row `row0` of D elements to the end of a tensor of `rows` rows.
+template <int D>
+__device__ inline uint32_t tile_bytes(int row0, int rows, long long row_stride) {
+  const long long rows_left = rows - 1 - row0;
+  return rows_left < 0 ? 0u : static_cast<uint32_t>((rows_left * row_stride + D) * 2);
+}
+
 // Queues the fill of a ROWS x D tile by direct-to-LDS buffer loads.  Load i of
 // a lane writes 16 bytes at chunk (wave*LOADS + i)*64 + lane of the tile;
 // offsets[i] = byte offset, from the tile's first row, of the chunk that
@@ -215,9 +222,7 @@ template <int D, int LOADS>
 __device__ inline void tile_fill(unsigned char* tile, int wave, const uint16_t* base,
                                  long long row_stride, int row0, int rows,
                                  const uint32_t* offsets) {
-  const long long rows_left = rows - 1 - row0;
-  const int32x4 rsrc = make_rsrc(
-      base, rows_left < 0 ? 0u : static_cast<uint32_t>((rows_left * row_stride + D) * 2));
+  const int32x4 rsrc = make_rsrc(base, tile_bytes<D>(row0, rows, row_stride));
 #pragma unroll
   for (int i = 0; i < LOADS; ++i)
     lds_fill<16>(rsrc, tile + (wave * LOADS + i) * 1024, offsets[i]);

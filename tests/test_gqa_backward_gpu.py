@@ -122,6 +122,44 @@ def test_state_saved_by_forward_gives_the_recomputed_gradients(capi, shape):
         assert_close_bf16_gradient(value.cpu().numpy(), want[name], "%s T%d d%d" % (name, T, d))
 
 
+@pytest.mark.parametrize("T,qh,kh,d,rot", [(1, 2, 1, 256, 64), (31, 4, 2, 256, 64), (65, 6, 2, 256, 64),
+                                           (130, 6, 1, 256, 128), (97, 4, 2, 128, 32), (97, 4, 2, 64, 32)])
+def test_saved_block_holds_what_both_passes_need(capi, T, qh, kh, d, rot):
+    """The block is filled where it starts (also off a multiple of 256 bytes), whatever the
+    output's alignment, and the backward makes of it, bit for bit, what it makes of the
+    inputs.  Head width 256: the forward that fills it keeps its softmax weights in FP32, so
+    its output is within the rounding of bf16 weights of the other forward's (2^-9 a
+    weight, sums of weighted values: 1e-2 of the norm is generous) and its cache the same."""
+    import ctypes
+    got, _, args, _ = run_case(capi, T, qh, kh, d, rot, True, seed=T + d)
+    p, qg, k, v, qw, kw_, dy = args
+    plain_cache = capi.KvCache(T, kh, d)
+    plain, plain_lse = capi.gqa_prefill(p, qg, k, v, qw, kw_, plain_cache, want_lse=True)
+    size = capi.lib().pluto_hip_gqa_prefill_saved_bytes(ctypes.byref(p), T, capi.BF16)
+    assert size > 0
+    for shift in (0, 2 if d == 256 else 0):
+        block = torch.full((size + 64,), 0x7f, dtype=torch.uint8, device="cuda")[48:48 + size]
+        space = torch.zeros(T * qh * d + 8, dtype=torch.bfloat16, device="cuda")
+        out = space[shift:shift + T * qh * d].view(T, qh, d)
+        cache = capi.KvCache(T, kh, d)
+        made, lse = capi.gqa_prefill(p, qg, k, v, qw, kw_, cache, saved=block, out=out, want_lse=True)
+        torch.cuda.synchronize()
+        assert torch.equal(cache.keys, plain_cache.keys) and torch.equal(cache.values, plain_cache.values)
+        if d == 256:
+            assert capi.last_path() == capi.PATH_MATRIX_F32
+            assert (made.float() - plain.float()).norm() <= 1e-2 * plain.float().norm()
+            # the bf16 kernel adds up rounded weights: each, and so the sum, is off by at
+            # most 2^-9 of itself, and the logarithm by as much
+            assert (lse - plain_lse).abs().max() <= 2.0 ** -9 + 1e-5 * (1 + plain_lse.abs().max())
+        else:
+            assert torch.equal(made, plain) and torch.equal(lse, plain_lse)
+        dq_norm, dk_norm = torch.zeros(d, device="cuda"), torch.zeros(d, device="cuda")
+        grads = capi.gqa_prefill_backward(p, qg, k, v, qw, kw_, dy, dq_norm=dq_norm, dk_norm=dk_norm, saved=block)
+        torch.cuda.synchronize()
+        for name, value in zip(("dqg", "dk", "dv", "dq_norm", "dk_norm"), grads + (dq_norm, dk_norm)):
+            assert np.array_equal(value.cpu().numpy(), got[name]), name
+
+
 def test_long_sequence_with_saved_state_matches_oracle(capi):
     """T=1024, one kv group of six 128-wide heads (the grouping of the benchmarked
     shape): eight query tiles, so the unpaired heaviest-first grid, with the block
