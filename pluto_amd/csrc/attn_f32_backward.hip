@@ -1,24 +1,26 @@
-// Causal attention backward with FP32 storage on the FP32 matrix cores
-// (v_mfma_f32_32x32x2_f32): the two backward kernels of the reference's FP32
-// mode (src/llm/layers/attention.cc:235-396), every product and sum in FP32.
+// Causal attention backward with FP32 storage: the two backward kernels of the
+// reference's FP32 mode (src/llm/layers/attention.cc:235-396), every factor in three bf16
+// pieces and every sum in FP32 (attn_f32_split.h).
 //
 //   dq    a workgroup owns 32 query rows of one (sequence, head); also does the
 //         reference's delta pass (attention.cc:283-291) for them
 //   dkv   a workgroup owns 32 keys
 // In both, the four waves take every fourth tile of the other side (32 rows
-// each) and their results are added in wave order through LDS: the matrix
-// instruction is slow (64 cycles), a sequence of 256 rows has 8 tiles a head, and
-// splitting the streamed side is what fills the machine there.  A tile is filled
-// by direct-to-LDS loads into the wave's own area (no barrier in the loop) and
-// read both ways: 16-byte pieces of a lane's row for the score products, one
-// float a lane along a row for the gradient products.  The orientation is the
-// one of attn_f32_mfma.hip: dq works on S^T (lane = query), dkv on S (lane = key),
-// so the score tile's accumulator is the B operand of the gradient product.
-// 4 sequences x 12 heads x 256 x 64: 40 us for the pair, where the kernels that
-// multiply one element at a time took 653 us.
-#include "attn_f32_tile.h"
+// each) and their results are added in wave order through LDS: a sequence of 256 rows has
+// 8 tiles a head, and splitting the streamed side is what fills the machine there.  A
+// wave's area holds one tile at a time and takes them in turn (dq: V, K; dkv: Q, dO, Q),
+// so that two workgroups share a compute unit.  The orientation is the one of
+// attn_f32_mfma.hip: dq works on S^T (lane = query), dkv on S (lane = key), so the score
+// tile's accumulator is the B operand of the gradient product.
+//
+// 4 sequences x 12 heads x 256 x 64: dq 11.6, dkv 15.2 us (18.9 and 21.1 on the FP32
+// matrix instructions); 16 x 12 x 512 x 64 88 and 117.  Small calls are bound by the
+// chain of a wave (its first tile's way from memory, the pieces, two products after each
+// other, the merge: 7 us with one tile), large ones by streaming every tile once for 32
+// rows.  Against 64-bit arithmetic the gradients are 2.4e-7 off for standard normal
+// inputs of 256 rows, 3.0e-7 with the FP32 matrix instructions.
+#include "attn_f32_split.h"
 #include "attn_generic.h"
-#include "mfma_tile.h"
 
 namespace pluto_hip {
 namespace {
@@ -29,23 +31,44 @@ struct F32Unit {
   int tile, head, seq;
 };
 // Tiles are numbered heaviest first over the whole grid.
-__device__ inline F32Unit f32_unit(const GenericBackwardArgs& a) {
+__device__ inline F32Unit f32_unit(const GenericBackwardArgs& a, int block) {
   const int sequences = a.rows / a.context_length;
   const int units = sequences * a.num_heads;
   F32Unit u;
-  u.tile = blockIdx.x / units;
-  u.head = (blockIdx.x % units) % a.num_heads;
-  u.seq = (blockIdx.x % units) / a.num_heads;
+  u.tile = block / units;
+  u.head = (block % units) % a.num_heads;
+  u.seq = (block % units) / a.num_heads;
   return u;
 }
 
+// LDS of a workgroup: its own rows of two tensors, the waves' areas, the statistics of a
+// streamed tile's rows; at the end the waves' results, `groups` KiB each.
+constexpr int kOwnDeltaRows = 512;
+template <int D, int GROUPS>
+struct F32BackwardLds {
+  static constexpr int kTiles = 2 * F32Rows<D>::kOwnBytes + kWaves * F32Rows<D>::kAreaBytes;
+  static constexpr int kMerge = kWaves * GROUPS * 1024;
+  __attribute__((aligned(1024))) unsigned char bytes[kTiles > kMerge ? kTiles : kMerge];
+  __attribute__((aligned(16))) float row_stats[kWaves][3][32];
+  float part_deltas[kWaves][64];
+  __device__ unsigned char* own(int tensor) { return bytes + tensor * F32Rows<D>::kOwnBytes; }
+  __device__ unsigned char* area(int wave) {
+    return bytes + 2 * F32Rows<D>::kOwnBytes + wave * F32Rows<D>::kAreaBytes;
+  }
+};
+template <int D>
+using DqLds = F32BackwardLds<D, D / 8>;
+template <int D>
+using DkvLds = F32BackwardLds<D, D / 4>;
+
+__device__ inline float dot4(float4 a, float4 b) { return (a.x * b.x + a.y * b.y) + (a.z * b.z + a.w * b.w); }
+
 // Adds the waves' accumulators (COUNT groups of four registers a lane) in wave
-// order.  The waves take turns at the groups; `store(group, lane, sum)` gets each
-// total once.  Every wave's area holds its COUNT * 1 KiB.
+// order.  The waves take turns at the groups; `store(group, sum)` gets each total once.
 template <int COUNT, typename Store>
-__device__ inline void merge_waves(unsigned char* areas, int area_bytes, int wave, int lane,
-                                   const float4 (&own)[COUNT], Store store) {
-  float4* mine = reinterpret_cast<float4*>(areas + wave * area_bytes);
+__device__ inline void merge_waves(unsigned char* lds, int wave, int lane, const float4 (&own)[COUNT], Store store) {
+  __syncthreads();  // nobody reads tiles any more
+  float4* mine = reinterpret_cast<float4*>(lds + wave * COUNT * 1024);
 #pragma unroll
   for (int g = 0; g < COUNT; ++g) mine[g * 64 + lane] = own[g];
   __syncthreads();
@@ -53,93 +76,82 @@ __device__ inline void merge_waves(unsigned char* areas, int area_bytes, int wav
 #pragma unroll
   for (int k = 0; k < COUNT / kWaves; ++k) {
     const int g = k * kWaves + wave;
-    float4 sum = reinterpret_cast<const float4*>(areas)[g * 64 + lane];
+    float4 sum = reinterpret_cast<const float4*>(lds)[g * 64 + lane];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) {
-      const float4 v = reinterpret_cast<const float4*>(areas + w * area_bytes)[g * 64 + lane];
+      const float4 v = reinterpret_cast<const float4*>(lds + w * COUNT * 1024)[g * 64 + lane];
       sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
     }
     store(g, sum);
   }
 }
 
-template <int D>
-__global__ void __launch_bounds__(64 * kWaves, D == 128 ? 1 : 2)
-f32_dq_kernel(GenericBackwardArgs a) {
-  using Tile = F32Tile<D>;
-  constexpr int HALF = D / 2, DB = D / 32, kArea = 2 * Tile::kBytes;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kWaves * kArea];
+template <int D, class Lds>
+__device__ __forceinline__ void f32_dq(const GenericBackwardArgs& a, const F32Unit& unit, Lds& sm) {
+  using Rows = F32Rows<D>;
+  constexpr int KS = Rows::KS, DB = Rows::DB;
   const int lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int T = a.context_length, E = a.embedding_dim;
-  const F32Unit unit = f32_unit(a);
   const int q0 = ((T + 31) / 32 - 1 - unit.tile) * 32;
   const long long row0 = static_cast<long long>(unit.seq) * T;
   const long long stats = (static_cast<long long>(unit.seq) * a.num_heads + unit.head) * T;
   const float* q_base = static_cast<const float*>(a.qkv) + row0 * 3 * E + unit.head * D;
   const int query = q0 + n, query_load = min(query, T - 1);
+  const int key_tiles = q0 / 32 + 1;
 
-  // A wave's first tile is on its way while it reads its own rows, the others while the
-  // one before is worked on: V in place as soon as it has been read, K, which is
-  // needed to the end, through registers.
-  unsigned char* k_tile = lds + wave * kArea;
-  unsigned char* v_tile = k_tile + Tile::kBytes;
-  typename Tile::Held k_held;
-  auto rows_of = [&](int kt) { return kt <= q0 / 32 ? T - kt * 32 : 0; };
-  auto request_k = [&](int kt) {
-    Tile::request(k_held, q_base + E + kt * 32 * 3LL * E, 3LL * E, rows_of(kt), lane);
-    __builtin_amdgcn_sched_barrier(0);
+  // a tile is requested as soon as the one before has been split
+  unsigned char* area = sm.area(wave);
+  typename Rows::Raw k_raw, v_raw;
+  auto request = [&](typename Rows::Raw& raw, int tensor, int kt) {
+    Rows::request(raw, q_base + tensor * E + (kt < key_tiles ? kt * 32 * 3LL * E : 0), 3LL * E,
+                  kt < key_tiles ? T - kt * 32 : 0, lane);
   };
-  auto request_v = [&](int kt) {
-    Tile::fill(v_tile, q_base + 2 * E + kt * 32 * 3LL * E, 3LL * E, rows_of(kt), lane);
-  };
-  request_k(wave);
-  request_v(wave);
-  float qf[HALF], gf[HALF];
-  load_half_row<HALF>(q_base + query_load * 3LL * E + h * HALF, qf);
-  const long long out_at = (row0 + query_load) * E + unit.head * D + h * HALF;
-  load_half_row<HALF>(a.d_out + out_at, gf);
-  float delta = 0.0f;
-#pragma unroll
-  for (int j = 0; j < HALF / 4; ++j) {
-    const float4 o = reinterpret_cast<const float4*>(static_cast<const float*>(a.out) + out_at)[j];
-    delta += gf[4 * j] * o.x + gf[4 * j + 1] * o.y + gf[4 * j + 2] * o.z + gf[4 * j + 3] * o.w;
-  }
-  delta = half_swap_sum(delta);
-  if (wave == 0 && h == 0 && query < T) a.deltas[stats + query] = delta;
+  request(k_raw, 1, wave);
+  request(v_raw, 2, wave);
   const float maximum = a.maxima[stats + query_load];
   const float normalizer = a.normalizers[stats + query_load];
   const float inverse = 1.0f / (normalizer > 0.0f ? normalizer : 1.0f);
-
+  float part_delta = 0.0f;
+  for (int ks = wave; ks < KS; ks += kWaves) {
+    const int c = 16 * ks + 8 * h;
+    const long long at = (row0 + query_load) * E + unit.head * D + c;
+    const float4* q = reinterpret_cast<const float4*>(q_base + query_load * 3LL * E + c);
+    const float4* g = reinterpret_cast<const float4*>(a.d_out + at);
+    const float4* o = reinterpret_cast<const float4*>(static_cast<const float*>(a.out) + at);
+    const float4 g0 = g[0], g1 = g[1];
+    Rows::keep_own(sm.own(0), ks, lane, split_eight(q[0], q[1]));
+    Rows::keep_own(sm.own(1), ks, lane, split_eight(g0, g1));
+    part_delta += dot4(g0, o[0]) + dot4(g1, o[1]);
+  }
+  sm.part_deltas[wave][lane] = part_delta;
   floatx16 acc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[db][i] = 0.0f;
-  const int key_tiles = q0 / 32 + 1;
+  __syncthreads();
+  float delta = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) delta += sm.part_deltas[w][lane];
+  delta = half_swap_sum(delta);
+  if (wave == 0 && h == 0 && query < T) a.deltas[stats + query] = delta;
+
   for (int kt = wave; kt < key_tiles; kt += kWaves) {
     const int k0 = kt * 32;
-    Tile::place(k_tile, k_held, lane);
-    wait_fills();
-    request_k(kt + kWaves);
     floatx16 s, dp;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
+    Rows::keep(area, v_raw, lane);
+    request(v_raw, 2, kt + kWaves);
 #pragma unroll
-    for (int j = 0; j < HALF / 4; ++j) {
-      const float4 k4 = Tile::row_piece(k_tile, n, h * (HALF / 4) + j);
-      const float4 v4 = Tile::row_piece(v_tile, n, h * (HALF / 4) + j);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, qf[4 * j], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(v4.x, gf[4 * j], dp, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qf[4 * j + 1], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(v4.y, gf[4 * j + 1], dp, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, qf[4 * j + 2], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(v4.z, gf[4 * j + 2], dp, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[4 * j + 3], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(v4.w, gf[4 * j + 3], dp, 0, 0, 0);
-    }
-    wait_reads();
-    request_v(kt + kWaves);
+    for (int ks = 0; ks < KS; ++ks)
+      dp = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(1), ks, lane), dp);
+    Rows::keep(area, k_raw, lane);  // in V's place
+    request(k_raw, 1, kt + kWaves);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(0), ks, lane), s);
     // register i = (key k0 + 8(i/4) + 4h + i%4, query n)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -148,13 +160,12 @@ f32_dq_kernel(GenericBackwardArgs a) {
       s[i] = key <= query_load ? p * (dp[i] - delta) * a.scale : 0.0f;
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const Pieces ds = split_accumulator(s, s2);
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
-        acc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-            Tile::element(k_tile, 8 * (i / 4) + 4 * h + (i % 4), 32 * db + n), s[i], acc[db], 0, 0, 0);
+      for (int db = 0; db < DB; ++db) acc[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), ds, acc[db]);
+    }
   }
-  wait_fills();
   float4 own[4 * DB];
 #pragma unroll
   for (int g = 0; g < 4 * DB; ++g)
@@ -162,48 +173,66 @@ f32_dq_kernel(GenericBackwardArgs a) {
                          acc[g / 4][4 * (g % 4) + 2], acc[g / 4][4 * (g % 4) + 3]);
   float* out = a.d_qkv + (row0 + query_load) * 3 * E + unit.head * D + 4 * h;
   // group g = channels 32 (g / 4) + 8 (g % 4) + 4 h .. + 3 of query n
-  merge_waves(lds, kArea, wave, lane, own, [&](int g, float4 sum) {
+  merge_waves(sm.bytes, wave, lane, own, [&](int g, float4 sum) {
     if (query < T) *reinterpret_cast<float4*>(out + 8 * g) = sum;
   });
 }
 
-template <int D>
-__global__ void __launch_bounds__(64 * kWaves, D == 128 ? 1 : 2)
-f32_dkv_kernel(GenericBackwardArgs a) {
-  using Tile = F32Tile<D>;
-  constexpr int HALF = D / 2, DB = D / 32, kArea = 2 * Tile::kBytes;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kWaves * kArea];
-  __shared__ __attribute__((aligned(16))) float row_stats[kWaves][3][32];
+// own_deltas: [kOwnDeltaRows] in LDS, or null where the dq kernel has left the row sums.
+template <int D, bool OWN_DELTAS, class Lds>
+__device__ __forceinline__ void f32_dkv(const GenericBackwardArgs& a, const F32Unit& unit, Lds& sm, float* own_deltas) {
+  using Rows = F32Rows<D>;
+  constexpr int KS = Rows::KS, DB = Rows::DB;
+  auto& row_stats = sm.row_stats;
   const int lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int T = a.context_length, E = a.embedding_dim;
-  const F32Unit unit = f32_unit(a);
   const int k0 = unit.tile * 32;
   const long long row0 = static_cast<long long>(unit.seq) * T;
   const long long stats = (static_cast<long long>(unit.seq) * a.num_heads + unit.head) * T;
   const float* q_base = static_cast<const float*>(a.qkv) + row0 * 3 * E + unit.head * D;
   const float* g_base = a.d_out + row0 * E + unit.head * D;
   const int key = k0 + n, key_load = min(key, T - 1);
+  const int query_tiles = (T + 31) / 32;
 
-  // the first tile is on its way before the wave's own rows; registers to hold
-  // another are not left (21.5 us at 256 rows, 23.8 with the request in the loop)
-  unsigned char* q_tile = lds + wave * kArea;
-  unsigned char* g_tile = q_tile + Tile::kBytes;
-  auto request = [&](int qt) {
-    const int q0 = qt * 32;
-    Tile::fill(q_tile, q_base + q0 * 3LL * E, 3LL * E, T - q0, lane);
-    Tile::fill(g_tile, g_base + q0 * 1LL * E, E, T - q0, lane);
+  unsigned char* area = sm.area(wave);
+  typename Rows::Raw q_raw, g_raw;
+  auto request_q = [&](int qt) {
+    const bool exists = qt < query_tiles;
+    Rows::request(q_raw, q_base + (exists ? qt * 32 * 3LL * E : 0), 3LL * E, exists ? T - qt * 32 : 0, lane);
   };
-  request(k0 / 32 + wave);
-  float kf[HALF], vf[HALF];
-  load_half_row<HALF>(q_base + E + key_load * 3LL * E + h * HALF, kf);
-  load_half_row<HALF>(q_base + 2 * E + key_load * 3LL * E + h * HALF, vf);
+  auto request_g = [&](int qt) {
+    const bool exists = qt < query_tiles;
+    Rows::request(g_raw, g_base + (exists ? qt * 32 * 1LL * E : 0), E, exists ? T - qt * 32 : 0, lane);
+  };
+  request_q(k0 / 32 + wave);
+  request_g(k0 / 32 + wave);
+  for (int ks = wave; ks < KS; ks += kWaves) {
+    const float4* k = reinterpret_cast<const float4*>(q_base + E + key_load * 3LL * E + 16 * ks + 8 * h);
+    const float4* v = reinterpret_cast<const float4*>(q_base + 2 * E + key_load * 3LL * E + 16 * ks + 8 * h);
+    Rows::keep_own(sm.own(0), ks, lane, split_eight(k[0], k[1]));
+    Rows::keep_own(sm.own(1), ks, lane, split_eight(v[0], v[1]));
+  }
+  if constexpr (OWN_DELTAS) {
+    // those of the wave's own tiles: nobody else reads them
+    for (int qt = k0 / 32 + wave; qt < query_tiles; qt += kWaves) {
+      const int row = min(qt * 32 + n, T - 1);
+      const float4* g = reinterpret_cast<const float4*>(g_base + row * 1LL * E + 8 * h);
+      const float4* o = reinterpret_cast<const float4*>(static_cast<const float*>(a.out) + (row0 + row) * E +
+                                                        unit.head * D + 8 * h);
+      float delta = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) delta += dot4(g[4 * ks], o[4 * ks]) + dot4(g[4 * ks + 1], o[4 * ks + 1]);
+      delta = half_swap_sum(delta);
+      if (h == 0) own_deltas[qt * 32 + n] = delta;
+    }
+  }
   floatx16 dk[DB], dv[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
-  const int query_tiles = (T + 31) / 32;
+  __syncthreads();
   for (int qt = k0 / 32 + wave; qt < query_tiles; qt += kWaves) {
     const int q0 = qt * 32;
     if (h == 0) {
@@ -211,25 +240,21 @@ f32_dkv_kernel(GenericBackwardArgs a) {
       const float normalizer = a.normalizers[stats + row];
       row_stats[wave][0][n] = a.maxima[stats + row];
       row_stats[wave][1][n] = 1.0f / (normalizer > 0.0f ? normalizer : 1.0f);
-      row_stats[wave][2][n] = a.deltas[stats + row];
+      row_stats[wave][2][n] = OWN_DELTAS ? own_deltas[q0 + n] : a.deltas[stats + row];
     }
-    wait_fills();
     floatx16 s, dp;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
+    // one area for Q, dO and Q again: two would leave room for one workgroup a compute unit
+    Rows::keep(area, q_raw, lane);
 #pragma unroll
-    for (int j = 0; j < HALF / 4; ++j) {
-      const float4 q4 = Tile::row_piece(q_tile, n, h * (HALF / 4) + j);
-      const float4 g4 = Tile::row_piece(g_tile, n, h * (HALF / 4) + j);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(q4.x, kf[4 * j], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.x, vf[4 * j], dp, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(q4.y, kf[4 * j + 1], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.y, vf[4 * j + 1], dp, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(q4.z, kf[4 * j + 2], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.z, vf[4 * j + 2], dp, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(q4.w, kf[4 * j + 3], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.w, vf[4 * j + 3], dp, 0, 0, 0);
-    }
+    for (int ks = 0; ks < KS; ++ks)
+      s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(0), ks, lane), s);
+    Rows::keep(area, g_raw, lane);
+    request_g(qt + kWaves);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      dp = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(1), ks, lane), dp);
     // register i = (query q0 + 8(i/4) + 4h + i%4, key n)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -250,19 +275,20 @@ f32_dkv_kernel(GenericBackwardArgs a) {
       }
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const Pieces p = split_accumulator(s, s2);
 #pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const int row = 8 * (i / 4) + 4 * h + (i % 4);
-        dv[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(Tile::element(g_tile, row, 32 * db + n), s[i],
-                                                      dv[db], 0, 0, 0);
-        dk[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(Tile::element(q_tile, row, 32 * db + n), dp[i],
-                                                      dk[db], 0, 0, 0);
-      }
-    wait_reads();
-    if (qt + kWaves < query_tiles) request(qt + kWaves);
+      for (int db = 0; db < DB; ++db) dv[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), p, dv[db]);
+    }
+    Rows::keep(area, q_raw, lane);
+    request_q(qt + kWaves);
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const Pieces ds = split_accumulator(dp, s2);
+#pragma unroll
+      for (int db = 0; db < DB; ++db) dk[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), ds, dk[db]);
+    }
   }
-  wait_fills();
   float4 own[8 * DB];
 #pragma unroll
   for (int g = 0; g < 4 * DB; ++g) {
@@ -272,14 +298,59 @@ f32_dkv_kernel(GenericBackwardArgs a) {
                                   dv[g / 4][4 * (g % 4) + 2], dv[g / 4][4 * (g % 4) + 3]);
   }
   float* out = a.d_qkv + (row0 + key_load) * 3 * E + E + unit.head * D + 4 * h;
-  merge_waves(lds, kArea, wave, lane, own, [&](int g, float4 sum) {
+  merge_waves(sm.bytes, wave, lane, own, [&](int g, float4 sum) {
     const int tensor = g / (4 * DB);
     if (key < T) *reinterpret_cast<float4*>(out + tensor * E + 8 * (g % (4 * DB))) = sum;
   });
 }
 
 template <int D>
+__global__ void __launch_bounds__(64 * kWaves, D == 128 ? 1 : 2)
+f32_dq_kernel(GenericBackwardArgs a) {
+  __shared__ DqLds<D> sm;
+  f32_dq<D>(a, f32_unit(a, blockIdx.x), sm);
+}
+
+template <int D>
+__global__ void __launch_bounds__(64 * kWaves, D == 128 ? 1 : 2)
+f32_dkv_kernel(GenericBackwardArgs a) {
+  __shared__ DkvLds<D> sm;
+  f32_dkv<D, false>(a, f32_unit(a, blockIdx.x), sm, nullptr);
+}
+
+// Both in one launch: every dkv workgroup makes the row sums of the queries it streams.
+// The halves of a level (tiles of equal length) follow each other.
+template <int D>
+__global__ void __launch_bounds__(64 * kWaves, D == 128 ? 1 : 2)
+f32_pair_kernel(GenericBackwardArgs a) {
+  __shared__ DkvLds<D> sm;
+  __shared__ float own_deltas[kOwnDeltaRows];
+  const int units = a.rows / a.context_length * a.num_heads;
+  const int level = blockIdx.x / units, block = level / 2 * units + blockIdx.x % units;
+  if (level % 2 == 0)
+    f32_dkv<D, true>(a, f32_unit(a, block), sm, own_deltas);
+  else
+    f32_dq<D>(a, f32_unit(a, block), sm);
+}
+
+// One launch where the workgroups of both kernels fit on the chip together, or nearly so
+// (two a compute unit, one at D = 128), and for short sequences, of which a workgroup sees
+// little, to several times that.  Beyond, the row sums made more than once cost more than
+// the launch.  Two launches against one, us: 1 x 12 x 48 x 64 14.8, 8.9; 4 x 12 x 200 24.2,
+// 20.6; 16 x 12 x 100 32.5, 29.9; 4 x 12 x 256 (384 workgroups each) 25.1, 26.7; 8 x 12 x
+// 512 104, 120; 4 x 6 x 256 x 128 41.7, 34.3; 8 x 6 x 512 x 128 145, 179.
+template <int D>
+bool one_launch(const GenericBackwardArgs& a, unsigned grid) {
+  constexpr unsigned kResident = D == 128 ? 192 : 352, kShort = D == 128 ? 576 : 1152;
+  return a.context_length <= kOwnDeltaRows && (grid <= kResident || (a.context_length <= 128 && grid <= kShort));
+}
+
+template <int D>
 int launch(hipStream_t stream, const GenericBackwardArgs& a, unsigned grid) {
+  if (one_launch<D>(a, grid) && kernel_enabled(kQueryKernel) && kernel_enabled(kMainKernel)) {
+    f32_pair_kernel<D><<<2 * grid, 64 * kWaves, 0, stream>>>(a);
+    return launch_status();
+  }
   if (kernel_enabled(kQueryKernel)) f32_dq_kernel<D><<<grid, 64 * kWaves, 0, stream>>>(a);
   int status = launch_status();
   if (status != 0) return status;

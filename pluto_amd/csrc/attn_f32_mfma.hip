@@ -1,30 +1,23 @@
-// Causal attention forward with FP32 storage and FP32 matrix-core arithmetic
-// (v_mfma_f32_32x32x2_f32): the reference's FP32 mode of
-// FlashAttentionForwardKernel (src/llm/layers/attention.cc:98-170), where
-// products and sums stay in FP32.
+// Causal attention forward with FP32 storage: the reference's FP32 mode of
+// FlashAttentionForwardKernel (src/llm/layers/attention.cc:98-170), every factor in three
+// bf16 pieces and every sum in FP32 (attn_f32_split.h).
 //
 // A workgroup of four waves owns 32 query rows of one (sequence, head); wave w
 // walks the visible key tiles (32 keys each) w, w + 4, ... with its own running
-// maximum, sum and output, and wave 0 merges the four partial results through
-// LDS in wave order.  The FP32 matrix instruction is slow (64 cycles for
-// 32x32x2), a row block near the end of a sequence has many tiles and there
+// maximum, sum and output, and the waves merge the four partial results through
+// LDS in wave order.  A row block near the end of a sequence has many tiles and there
 // are few row blocks, so splitting the keys is what fills the machine; the row
-// blocks are handed out heaviest first, and a wave's tiles arrive in LDS while it
-// works on what is there.  Against lightest first with operands read from memory row
-// by row: 4 sequences x 12 heads x 256 x 64 19.4 -> 12.8 us, 2 x 12 x 1000 x 64
-// 75 -> 47, 2 x 6 x 1000 x 128 104 -> 50.  As in
+// blocks are handed out heaviest first, and a wave's next tiles travel while it
+// works on the ones it has.  4 sequences x 12 heads x 256 x 64 10.0 us (12.3 on the FP32
+// matrix instructions), 16 x 12 x 512 x 64 77; outputs 1.7e-7 off 64-bit arithmetic for
+// standard normal inputs, 2.2e-7 with those instructions.  As in
 // the bf16 kernels the products are transposed,
 // S^T = K Q^T and O^T = V^T P^T, so that a lane owns one query column: its row
 // maximum and sum are lane-local up to one exchange between the two lane
-// halves, and P^T leaves the accumulator in B-operand order.  The contraction
-// order of a matrix instruction is free as long as both operands agree:
-//   S^T  step j contracts channels (j, j + D/2): lane half h reads the
-//        contiguous half row [h D/2, (h+1) D/2) of its key and of its query;
-//   O^T  step i contracts keys (8(i/4) + i%4, that + 4): exactly the keys
-//        accumulator register i holds in the two lane halves.
-#include "attn_f32_tile.h"
+// halves, and P^T leaves the accumulator in B-operand order.  K and V take turns in the
+// wave's area: with one each a compute unit would hold one workgroup.
+#include "attn_f32_split.h"
 #include "attn_generic.h"
-#include "mfma_tile.h"
 
 namespace pluto_hip {
 namespace {
@@ -34,13 +27,11 @@ constexpr int kKeySplit = 4;  // waves per workgroup, each taking every fourth k
 template <int D>
 __global__ void __launch_bounds__(64 * kKeySplit, D == 128 ? 1 : 2)
 f32_forward_kernel(GenericForwardArgs a) {
-  using Tile = F32Tile<D>;
-  constexpr int HALF = D / 2, DB = D / 32, kArea = 2 * Tile::kBytes, kFill = Tile::kFillOps;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kKeySplit * kArea];
-  // after the last tile: the partial results of waves 1 and up
-  auto part_o = reinterpret_cast<float(*)[DB * 16][64]>(lds);
-  static_assert((kKeySplit - 1) * DB * 16 * 64 * 4 <= kKeySplit * kArea);
-  __shared__ float part_max[kKeySplit - 1][64], part_sum[kKeySplit - 1][64];
+  using Rows = F32Rows<D>;
+  constexpr int KS = Rows::KS, DB = Rows::DB;
+  constexpr int kMergeBytes = kKeySplit * 4 * DB * 1024, kTileBytes = Rows::kOwnBytes + kKeySplit * Rows::kAreaBytes;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kTileBytes > kMergeBytes ? kTileBytes : kMergeBytes];
+  __shared__ float part_max[kKeySplit][64], part_sum[kKeySplit][64];
   const int lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   // the row blocks that see the most keys first, of every (sequence, head)
@@ -61,49 +52,45 @@ f32_forward_kernel(GenericForwardArgs a) {
   const int last_query = min(q0 + 32, a.q_rows) - 1;
   const int visible_keys = min(a.kv_rows, a.start_position + last_query + 1);
   const int key_tiles = (visible_keys + 31) / 32;
-  // K's tile is filled again as soon as the scores have been made and V's once it
-  // has been used, so that each has the other's products to arrive in.  The
-  // order of requests is K, V, K, V ...: waiting for one leaves the other on its way.
-  unsigned char* k_tile = lds + wave * kArea;
-  unsigned char* v_tile = k_tile + Tile::kBytes;
-  auto fill = [&](unsigned char* tile, const float* base, long long row_stride, int kt) {
+  unsigned char* own = lds;
+  unsigned char* area = lds + Rows::kOwnBytes + wave * Rows::kAreaBytes;
+  // a tile is requested as soon as the one before has been split
+  typename Rows::Raw k_raw, v_raw;
+  auto request = [&](typename Rows::Raw& raw, const float* base, long long row_stride, int kt) {
     const int k0 = kt < key_tiles ? kt * 32 : 0;
-    Tile::fill(tile, base + k0 * row_stride, row_stride, kt < key_tiles ? a.kv_rows - k0 : 0, lane);
+    Rows::request(raw, base + k0 * row_stride, row_stride, kt < key_tiles ? a.kv_rows - k0 : 0, lane);
   };
-  fill(k_tile, k_base, a.k.row_stride, wave);
-  fill(v_tile, v_base, a.v.row_stride, wave);
-  float qf[HALF];
-  load_half_row<HALF>(q_base + query_load * a.q.row_stride + h * HALF, qf);
+  request(k_raw, k_base, a.k.row_stride, wave);
+  request(v_raw, v_base, a.v.row_stride, wave);
+  for (int ks = wave; ks < KS; ks += kKeySplit) {
+    const float4* row = reinterpret_cast<const float4*>(q_base + query_load * a.q.row_stride + 16 * ks + 8 * h);
+    Rows::keep_own(own, ks, lane, split_eight(row[0], row[1]));
+  }
   floatx16 o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
   float running_max = kMasked, running_sum = 0.0f;  // base-2 scaled scores
+  __syncthreads();
 
-  const int my_last_key = a.start_position + query;  // keys beyond it are masked
+  const int last_key = min(a.start_position + query, a.kv_rows - 1);  // keys beyond it are masked
   for (int kt = wave; kt < key_tiles; kt += kKeySplit) {
-    wait_fills<kFill>();  // K
+    Rows::keep(area, k_raw, lane);
+    request(k_raw, k_base, a.k.row_stride, kt + kKeySplit);
     floatx16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < HALF / 4; ++j) {
-      const float4 k4 = Tile::row_piece(k_tile, n, h * (HALF / 4) + j);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, qf[4 * j], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qf[4 * j + 1], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, qf[4 * j + 2], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[4 * j + 3], s, 0, 0, 0);
-    }
-    wait_reads();
-    fill(k_tile, k_base, a.k.row_stride, kt + kKeySplit);
+    for (int ks = 0; ks < KS; ++ks) s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(own, ks, lane), s);
+    Rows::keep(area, v_raw, lane);  // in K's place
+    request(v_raw, v_base, a.v.row_stride, kt + kKeySplit);
     // register i = (key kt*32 + 8(i/4) + 4h + i%4, query n)
+    const int last = last_key - kt * 32 - 4 * h;
     float tile_max = kMasked;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int key = kt * 32 + 8 * (i / 4) + 4 * h + (i % 4);
-      const bool visible = key <= my_last_key && key < a.kv_rows;
-      s[i] = visible ? s[i] * scale2 : kMasked;
+      s[i] = 8 * (i / 4) + i % 4 <= last ? s[i] * scale2 : kMasked;
       tile_max = fmaxf(tile_max, s[i]);
     }
     tile_max = half_swap_max(tile_max);
@@ -118,74 +105,63 @@ f32_forward_kernel(GenericForwardArgs a) {
       tile_sum += p;
     }
     running_sum = running_sum * correction + half_swap_sum(tile_sum);
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[db][i] *= correction;
-    wait_fills<kFill>();  // V
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-        o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-            Tile::element(v_tile, 8 * (i / 4) + 4 * h + (i % 4), 32 * db + n), s[i], o[db], 0, 0, 0);
-    wait_reads();
-    fill(v_tile, v_base, a.v.row_stride, kt + kKeySplit);
-  }
-  wait_fills();
-  __syncthreads();  // every wave is done with its tiles
-  // ---- merge: every wave's result is relative to its own maximum ------------
-  if (wave > 0) {
-    part_max[wave - 1][lane] = running_max;
-    part_sum[wave - 1][lane] = running_sum;
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) part_o[wave - 1][db * 16 + i][lane] = o[db][i];
-  }
-  __syncthreads();
-  if (wave > 0) return;
-  {
-    float maximum = running_max;
-#pragma unroll
-    for (int w = 0; w < kKeySplit - 1; ++w) maximum = fmaxf(maximum, part_max[w][lane]);
-    // a wave without tiles contributes weight 2^(kMasked - maximum) = 0
-    const float own = __builtin_amdgcn_exp2f(running_max - maximum);
-    running_sum *= own;
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[db][i] *= own;
-#pragma unroll
-    for (int w = 0; w < kKeySplit - 1; ++w) {
-      const float weight = __builtin_amdgcn_exp2f(part_max[w][lane] - maximum);
-      running_sum += part_sum[w][lane] * weight;
+    if (__any(correction != 1.0f)) {
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[db][i] += part_o[w][db * 16 + i][lane] * weight;
+        for (int i = 0; i < 16; ++i) o[db][i] *= correction;
     }
-    running_max = maximum;
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const Pieces p = split_accumulator(s, s2);
+#pragma unroll
+      for (int db = 0; db < DB; ++db) o[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), p, o[db]);
+    }
+  }
+  // ---- merge: every wave's result is relative to its own maximum; the waves take turns at
+  // the groups of four channels
+  __syncthreads();  // nobody reads tiles any more
+  constexpr int kGroups = 4 * DB;
+  static_assert(kGroups % kKeySplit == 0, "the groups divide over the waves");
+  float4* mine = reinterpret_cast<float4*>(lds + wave * kGroups * 1024);
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g)
+    mine[g * 64 + lane] = make_float4(o[g / 4][4 * (g % 4)], o[g / 4][4 * (g % 4) + 1], o[g / 4][4 * (g % 4) + 2],
+                                      o[g / 4][4 * (g % 4) + 3]);
+  part_max[wave][lane] = running_max;
+  part_sum[wave][lane] = running_sum;
+  __syncthreads();
+  float maximum = part_max[0][lane];
+#pragma unroll
+  for (int w = 1; w < kKeySplit; ++w) maximum = fmaxf(maximum, part_max[w][lane]);
+  // a wave without tiles has weight 2^(kMasked - maximum) = 0
+  float weight[kKeySplit], sum = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kKeySplit; ++w) {
+    weight[w] = __builtin_amdgcn_exp2f(part_max[w][lane] - maximum);
+    sum += part_sum[w][lane] * weight[w];
   }
   if (query >= a.q_rows) return;
-  const float normalizer = running_sum > 0.0f ? running_sum : 1.0f;
+  const float normalizer = sum > 0.0f ? sum : 1.0f;
   const float inverse = 1.0f / normalizer;
   float* out = static_cast<float*>(a.out) + seq * a.o_seq_stride + query * a.o_row_stride +
-               head * a.o_head_stride;
-  // O^T register i of block db = (channel 32 db + 8(i/4) + 4h + i%4, query n)
+               head * a.o_head_stride + 4 * h;
+  // group g = channels 8 g + 4 h .. + 3 of query n
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+  for (int k = 0; k < kGroups / kKeySplit; ++k) {
+    const int g = k * kKeySplit + wave;
+    float4 total = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float4 piece;
-      piece.x = o[db][4 * j] * inverse;
-      piece.y = o[db][4 * j + 1] * inverse;
-      piece.z = o[db][4 * j + 2] * inverse;
-      piece.w = o[db][4 * j + 3] * inverse;
-      *reinterpret_cast<float4*>(out + 32 * db + 8 * j + 4 * h) = piece;
+    for (int w = 0; w < kKeySplit; ++w) {
+      const float4 v = reinterpret_cast<const float4*>(lds + w * kGroups * 1024)[g * 64 + lane];
+      total.x += v.x * weight[w]; total.y += v.y * weight[w];
+      total.z += v.z * weight[w]; total.w += v.w * weight[w];
     }
-  if (h == 0) {
-    const float maximum = running_max * (1.0f / kLog2e);
+    *reinterpret_cast<float4*>(out + 8 * g) =
+        make_float4(total.x * inverse, total.y * inverse, total.z * inverse, total.w * inverse);
+  }
+  if (wave == 0 && h == 0) {
+    maximum *= 1.0f / kLog2e;
     const long long stat = (static_cast<long long>(seq) * a.query_heads + head) * a.q_rows + query;
     if (a.maxima) a.maxima[stat] = maximum;
     if (a.normalizers) a.normalizers[stat] = normalizer;

@@ -1,0 +1,141 @@
+// FP32 attention on the bf16 matrix cores: what the forward and backward kernels share.
+//
+// An FP32 number is the sum of three bf16 numbers (8 + 8 + 8 mantissa bits), and a
+// product of two such sums is six bf16 matrix products with FP32 sums: the three left
+// out are 2^-25 of the product, less than one FP32 rounding.  Six v_mfma_f32_32x32x16_bf16
+// take 192 cycles where the FP32 instruction needs 512 for the same depth; making the
+// pieces costs 44 cycles of vector instructions a pair of numbers.
+//
+// A workgroup of four waves owns 32 rows of one side, kept in LDS as pieces in operand
+// order; every wave streams tiles of 32 rows of the other side of its own through an area
+// of LDS, where a tile lies as pieces and is read both ways: by rows for the score
+// products, transposed for those that contract over rows.
+#pragma once
+
+#include "mfma_tile.h"
+
+namespace pluto_hip {
+
+struct Pieces {
+  bf16x8 part[3];
+};
+
+// acc + a b, smallest products first.
+__device__ inline floatx16 mma_pieces(const Pieces& a, const Pieces& b, floatx16 acc) {
+#pragma unroll
+  for (int i = 2; i >= 0; --i)
+#pragma unroll
+    for (int j = 2 - i; j >= 0; --j) acc = mfma32(a.part[i], b.part[j], acc);
+  return acc;
+}
+
+// Two numbers as the packed words of their pieces.
+__device__ inline void split_pair(float first, float second, uint32_t& high, uint32_t& middle, uint32_t& low) {
+  high = pack_bf16(first, second);
+  first -= __uint_as_float(high << 16);
+  second -= __uint_as_float(high & 0xffff0000u);
+  middle = pack_bf16(first, second);
+  first -= __uint_as_float(middle << 16);
+  second -= __uint_as_float(middle & 0xffff0000u);
+  low = pack_bf16(first, second);
+}
+__device__ inline Pieces split_eight(const float (&x)[8]) {
+  uint32_t words[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) split_pair(x[2 * i], x[2 * i + 1], words[0][i], words[1][i], words[2][i]);
+  Pieces out;
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+    out.part[p] = as_bf16x8(make_uint4(words[p][0], words[p][1], words[p][2], words[p][3]));
+  return out;
+}
+__device__ inline Pieces split_eight(float4 a, float4 b) {
+  const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  return split_eight(x);
+}
+// Accumulator registers 8 s2 .. 8 s2 + 7 as a B operand.
+__device__ inline Pieces split_accumulator(const floatx16& acc, int s2) {
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = acc[8 * s2 + e];
+  return split_eight(x);
+}
+
+template <int D>
+struct F32Rows {
+  static constexpr int KS = D / 16, DB = D / 32;
+  static constexpr int kWidth = D < 64 ? 64 : D;  // of a row in LDS: the swizzle permutes eight pieces
+  static constexpr int kOwnBytes = 3 * KS * 1024;
+  static constexpr int kPartBytes = 32 * kWidth * 2, kAreaBytes = 3 * kPartBytes;
+
+  // A tile as it arrives: four channels a lane, whole rows next to each other (a lane's
+  // channels of an operand at a time, 32 rows an access, the loads took twice as long as
+  // everything else).
+  static constexpr int kLanes = D / 4, kLoads = 32 * kLanes / 64;
+  struct Raw {
+    float4 v[kLoads];
+  };
+  // Rows `row_stride` floats apart, `valid` of which exist; the others read as zero.
+  __device__ static void request(Raw& raw, const float* base, long long row_stride, int valid, int lane) {
+    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(base), 0,
+        valid <= 0 ? 0 : static_cast<int>(((min(valid, 32) - 1) * row_stride + D) * 4), 0x00020000);
+    const int bytes = static_cast<int>(row_stride * 4);
+    int at = lane / kLanes * bytes + lane % kLanes * 16;
+    asm volatile("" : "+v"(at));  // one register kept over a loop, not one a load
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      raw.v[i] = __builtin_bit_cast(
+          float4, __builtin_amdgcn_raw_buffer_load_b128(rows, at + i * (64 / kLanes) * bytes, 0, 0));
+  }
+
+  // The workgroup's own rows: operand (part, ks) is 1 KiB, a lane's eight channels together.
+  __device__ static void keep_own(unsigned char* own, int ks, int lane, const Pieces& p) {
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+      *reinterpret_cast<bf16x8*>(own + ((part * KS + ks) * 64 + lane) * 16) = p.part[part];
+  }
+  __device__ static Pieces read_own(const unsigned char* own, int ks, int lane) {
+    Pieces p;
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+      p.part[part] = *reinterpret_cast<const bf16x8*>(own + ((part * KS + ks) * 64 + lane) * 16);
+    return p;
+  }
+
+  // The wave's area: row-major tiles of the three pieces.  A wave's accesses to LDS are
+  // carried out in order, so a tile may follow another without a wait.
+  __device__ static void keep(unsigned char* area, const Raw& raw, int lane) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int row = i * (64 / kLanes) + lane / kLanes, piece = lane % kLanes;
+      const int at = tile_row_read<kWidth>(row, piece / 2) + piece % 2 * 8;
+      uint32_t words[3][2];
+      split_pair(raw.v[i].x, raw.v[i].y, words[0][0], words[1][0], words[2][0]);
+      split_pair(raw.v[i].z, raw.v[i].w, words[0][1], words[1][1], words[2][1]);
+#pragma unroll
+      for (int part = 0; part < 3; ++part)
+        *reinterpret_cast<uint2*>(area + part * kPartBytes + at) = make_uint2(words[part][0], words[part][1]);
+    }
+  }
+  // A operand: row n, channels 16 ks + 8 h .. + 7
+  __device__ static Pieces read_rows(const unsigned char* area, int ks, int lane) {
+    const int at = tile_row_read<kWidth>(lane % 32, 2 * ks + lane / 32);
+    Pieces p;
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+      p.part[part] = *reinterpret_cast<const bf16x8*>(area + part * kPartBytes + at);
+    return p;
+  }
+  // A operand: channels 32 db + n of rows 16 s2 .. in accumulator order
+  __device__ static Pieces read_transposed(const unsigned char* area, int db, int s2, int lane) {
+    Pieces p;
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+      p.part[part] =
+          tile_transposed_operand<kWidth>(area + part * kPartBytes, tile_transpose_read<kWidth>(lane, db), s2);
+    return p;
+  }
+};
+
+}  // namespace pluto_hip

@@ -23,6 +23,7 @@
 // accumulator is the B operand of the product that follows.
 #include "attn_split_mfma.h"
 
+#include "attn_f32_split.h"
 #include "mfma_tile.h"
 
 #include <type_traits>
@@ -35,31 +36,6 @@ constexpr int kThreads = 256, kRows = 32;
 constexpr int KCH = D / 8, KS = D / 16, DB = D / 32;
 constexpr int kLoads = kRows * KCH / kThreads;
 constexpr int kTileBytes = kRows * D * 2;
-
-struct Pieces {
-  bf16x8 part[3];
-};
-
-// Accumulator registers 8 s2 .. 8 s2 + 7 as three B operands that add up to them.
-__device__ inline Pieces split_accumulator(const floatx16& acc, int s2) {
-  uint32_t words[3][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float first = acc[8 * s2 + 2 * i], second = acc[8 * s2 + 2 * i + 1];
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      const uint32_t bits = pack_bf16(first, second);
-      words[p][i] = bits;
-      first -= __uint_as_float(bits << 16);
-      second -= __uint_as_float(bits & 0xffff0000u);
-    }
-  }
-  Pieces out;
-#pragma unroll
-  for (int p = 0; p < 3; ++p)
-    out.part[p] = as_bf16x8(make_uint4(words[p][0], words[p][1], words[p][2], words[p][3]));
-  return out;
-}
 
 __device__ inline floatx16 zero16() {
   floatx16 z;

@@ -100,6 +100,62 @@ def test_fp32_matrix_core_backward_at_tile_edges(capi, oracle, T, D):
     assert capi.last_path() == capi.PATH_MATRIX_F32
 
 
+@pytest.mark.parametrize("T,H,D,B", [(1, 1, 64, 1), (33, 2, 32, 2), (128, 3, 64, 3), (129, 2, 128, 2),
+                                     (500, 2, 64, 2), (512, 1, 128, 1), (513, 1, 64, 1), (128, 13, 64, 23)])
+def test_fp32_backward_in_one_launch_and_in_two(capi, T, H, D, B):
+    """Small calls run both backward kernels in one launch, where the key-owned half makes
+    the row sums of dO * O itself, in another order: dQ bit for bit, dK and dV to FP32
+    rounding of those sums (D terms, 2^-24 sqrt(D) of the score gradients)."""
+    gen = torch.Generator(device="cuda").manual_seed(T + D)
+    x = torch.randn((B * T, 3 * H * D), generator=gen, device="cuda")
+    d_out = torch.randn((B * T, H * D), generator=gen, device="cuda")
+    out, maxima, normalizers = capi.mha_forward(x, T, H)
+    workspace = capi.mha_backward_workspace(x, T, H)
+    one = capi.mha_backward(x, out, d_out, maxima, normalizers, T, H, workspace)
+    assert capi.last_path() == capi.PATH_MATRIX_F32
+    two = torch.empty_like(one)
+    everything = capi.lib().pluto_hip_test_kernel_classes(0)
+    try:
+        for half in (2, 1):  # the query-owned kernel, then the other
+            capi.lib().pluto_hip_test_kernel_classes(everything & ~3 | half)
+            capi.mha_backward(x, out, d_out, maxima, normalizers, T, H, workspace, two)
+    finally:
+        capi.lib().pluto_hip_test_kernel_classes(everything)
+    torch.cuda.synchronize()
+    a, b = one.view(B * T, 3, H * D), two.view(B * T, 3, H * D)
+    assert torch.equal(a[:, 0], b[:, 0])
+    assert (a - b).norm() <= 2.0 ** -24 * D ** 0.5 * 8 * b.norm()
+
+
+def test_fp32_non_finite_rows_stay_in_their_tile(capi):
+    """Whatever a key or a gradient row holds, queries of earlier tiles of 32 rows, and the
+    gradients that do not see it, are what they are without it; what sees it is not finite."""
+    T, H, D = 160, 2, 64
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((T, 3 * H * D), generator=gen, device="cuda")
+    d_out = torch.randn((T, H * D), generator=gen, device="cuda")
+
+    def once(x, d_out):
+        out, maxima, normalizers = capi.mha_forward(x, T, H)
+        grads = capi.mha_backward(x, out, d_out, maxima, normalizers, T, H)
+        torch.cuda.synchronize()
+        return out, grads.view(T, 3, H * D)
+
+    out, grads = once(x, d_out)
+    for bad in (float("inf"), float("-inf"), float("nan")):
+        changed = x.clone()
+        changed[100, 2 * H * D + 5] = bad  # a value of head 0
+        out2, _ = once(changed, d_out)
+        assert torch.equal(out2[:96], out[:96]) and torch.equal(out2[:, D:], out[:, D:])
+        assert not torch.isfinite(out2[100:, 5]).any()
+        changed = d_out.clone()
+        changed[40, 5] = bad
+        _, grads2 = once(x, changed)
+        assert torch.equal(grads2[64:, 1:], grads[64:, 1:])  # keys after the query's tile
+        assert torch.equal(grads2[:32, 0], grads[:32, 0]) and torch.equal(grads2[64:, 0], grads[64:, 0])
+        assert not torch.isfinite(grads2[:41, 2, 5]).any()
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_peaked_scores(capi, oracle, bf16):
     check(capi, oracle, 65, 1, 64, 2, bf16, seed=5, qk_scale=20.0 if not bf16 else 4.0)
