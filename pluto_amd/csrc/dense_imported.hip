@@ -5,13 +5,16 @@
 //   ImportedForward               :295-341 bf16 token -> fp32 -> (quantize) ->
 //                                          mat-vec -> bf16
 // One frozen checkpoint matrix [output_dim, input_dim] in bf16, fp32 or OCP
-// FP8 E4M3 with FP32 scales [ceil(out/128), ceil(in/128)] times one bf16
-// token.  Byte-bound: every weight is read once.  A wave owns four output
-// rows and reads them in 16-byte pieces (whenever rows start 16-byte aligned),
-// a single token is prepared by the workgroups themselves, several come from the
-// FP32 copy a kernel of their own leaves in the workspace; all arithmetic is
-// FP32, the 64 lane sums are added by a butterfly.
+// FP8 E4M3 with FP32 scales [ceil(out/128), ceil(in/128)] times bf16 tokens.
+// Byte-bound for few tokens: every weight is read once.  Three families of kernels:
+//   vector        any storage, width and alignment; up to eight tokens a pass over the
+//                 weights, FP32 arithmetic
+//   few tokens    bf16 and FP8 weights of whole 128-element blocks, up to eight tokens:
+//                 4 x 4 blocks on the matrix cores, tokens prepared by the workgroups
+//   tiles         the same weights, more tokens: 16 x 16 blocks, 32 tokens a pass
+// All sums are FP32.
 #include <algorithm>
+#include <type_traits>
 
 #include "dense.h"
 
@@ -117,6 +120,18 @@ struct MatVecArgs {
 
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
+// Largest of sixteen neighbouring lanes' values.
+__device__ inline uint32_t row_max(uint32_t v) {
+  auto step = [&](auto control) {
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), decltype(control)::value, 0xf, 0xf, true)));
+  };
+  step(std::integral_constant<int, 0xB1>());   // quad_perm 1, 0, 3, 2
+  step(std::integral_constant<int, 0x4E>());   // quad_perm 2, 3, 0, 1
+  step(std::integral_constant<int, 0x141>());  // row_half_mirror
+  step(std::integral_constant<int, 0x140>());  // row_mirror
+  return v;
+}
+
 // Four FP8 E4M3 codes of a word as floats, by the hardware conversion.
 __device__ inline void fp8_word(uint32_t word, float* out) {
   const floatx2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(word), false);
@@ -150,8 +165,7 @@ __device__ inline MatVecTarget matvec_target(const MatVecArgs& a) {
 // workgroup converts (FP8: quantizes) the token itself while its first weights
 // travel, instead of reading what a launch of its own left in memory; in LDS the
 // quarters of a piece lie apart, so that the lanes read consecutive 16 bytes.
-// 5120 -> 12288 + 1024 + 1024 in FP8, one token: 41 us as a token and a mat-vec
-// launch a matrix, 17 us as one launch.
+// (Rows of whole 128-element blocks have kernels of their own, see below.)
 template <int STORAGE, int TOKENS, int STEPS, bool PREPARE>
 __global__ void __launch_bounds__(256, TOKENS > 1 ? 1 : PREPARE && STORAGE == 2 && STEPS < 8 ? 4 : 3)
 imported_matvec_kernel(MatVecArgs a) {
@@ -353,9 +367,446 @@ __global__ void __launch_bounds__(256) imported_matvec_ragged_kernel(MatVecArgs 
     }
 }
 
+// ---- up to eight tokens of whole 128-element blocks ---------------------------
+// v_mfma_f32_4x4x4_16b_bf16 multiplies sixteen independent pairs of 4 x 4 blocks: lane i of
+// a block gives four elements of row i and of column i and finds element (j, i) of the
+// product in register j.  Two kernels use it, both with persistent waves that own four
+// rows of weights at a time, request a step's weights for the next four as soon as they
+// have been multiplied, and find the tokens in LDS, put there by the workgroup while its
+// first weights travel:
+//   one      lanes are 64 pieces of sixteen bytes of one row, as in a mat-vec, and a lane
+//            takes the product of its own piece and its own piece of the token: one of
+//            sixteen products, but every weight is read in contiguous KiB
+//   several  the rows of a block are four rows of weights, its columns four tokens: all
+//            products are used, and a load instruction reads 256 bytes of each row
+// A piece's product is the same in both, and both add up pieces in the order of a lane
+// that takes every 64th and then of wave_sum, so that a token's results do not depend on
+// how many there are.  FP8: codes are exact in bf16, and the sixteen elements of a piece lie
+// in one block of scales, which multiply their sum (see below).
+// On the vector units every token is another FMA a weight and another read of its values.
+// Hot weights (in the memory-side cache), us for 1, 2, 4, 8 tokens, before and now:
+// 5120 -> 16480 in FP8 19.0, 34.1, 50.1, 84.2 and 17.5, 19.7, 20.8, 24.5; 6144 -> 5120
+// in FP8 8.5, 13.8, 20.9, 35.4 and 9.3, 11.8, 13.2, 18.4; 5120 -> 16480 in bf16 26.4,
+// 31.7, 47.3, 70.3 and 26.2, 26.6, 29.1, 30.0 (169 MB: 6.3 TB/s).
+typedef __attribute__((ext_vector_type(4))) short shortx4;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float floatx4;
+
+constexpr int kFewTokens = 8, kFewWaves = 8;
+constexpr int kFewColumns = 9216;  // 8 tokens as bf16 in LDS: 144 KiB
+
+// Eight FP8 codes (the lower or the upper eight of sixteen) as bf16, exactly.
+__device__ inline bf16x8 fp8_to_bf16(const uint4& codes, int part) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  const uint32_t word[2] = {part == 0 ? codes.x : codes.z, part == 0 ? codes.y : codes.w};
+  bf16x8 out;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bf16x2 low = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word[i], 1.0f, false);
+    const bf16x2 high = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word[i], 1.0f, true);
+    out[4 * i] = low[0], out[4 * i + 1] = low[1], out[4 * i + 2] = high[0], out[4 * i + 3] = high[1];
+  }
+  return out;
+}
+
+// acc += the products of eight elements a lane: column i of a block's lanes is lane i's
+// piece of a token, row i lane i's piece of a row, so that lane i finds the product of its
+// own two pieces in register i.
+__device__ inline floatx4 mma_few(uint4 weights, uint4 tokens, floatx4 acc) {
+  typedef __attribute__((ext_vector_type(2))) uint32_t uint32x2;
+  const uint32x2 w[2] = {{weights.x, weights.y}, {weights.z, weights.w}}, t[2] = {{tokens.x, tokens.y}, {tokens.z, tokens.w}};
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    acc = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(shortx4, w[i]), __builtin_bit_cast(shortx4, t[i]), acc,
+                                                 0, 0, 0);
+  return acc;
+}
+
+// Sums of N values over the 64 lanes: lanes l / (64 / N) end with value l, added in the
+// order of wave_sum.
+template <int N>
+__device__ inline float sums_of(float (&v)[N]) {
+  int offset = 32;
+#pragma unroll
+  for (int n = N; n > 1; n /= 2, offset /= 2) {
+    const bool upper = threadIdx.x & offset;
+#pragma unroll
+    for (int i = 0; i < n / 2; ++i) {
+      float low = v[i], high = v[i + n / 2];
+      asm("" : "+v"(low), "+v"(high));  // values: the compiler would choose between addresses
+      const float kept = upper ? high : low, sent = upper ? low : high;
+      v[i] = kept + __shfl_xor(sent, offset, 64);
+    }
+  }
+  float sum = v[0];
+#pragma unroll
+  for (; offset > 0; offset /= 2) sum += __shfl_xor(sum, offset, 64);
+  return sum;
+}
+
+struct FewArgs {
+  const void* weights[kManyMax];
+  const float* scales[kManyMax];  // FP8 only
+  uint16_t* out[kManyMax];        // [tokens, rows]
+  int rows[kManyMax];
+  int first_block[kManyMax + 1];  // of quadruples of rows
+  int matrices = 0;
+  const uint16_t* tokens = nullptr;  // bf16 [count, cols]
+  int cols = 0, count = 0;
+};
+
+constexpr int kFewRows = 4;
+constexpr int kFewThreads = 64 * kFewWaves;
+
+// Four rows of a matrix.
+struct FewUnit {
+  int which, row;
+  __amdgpu_buffer_rsrc_t weights;  // those past the end read zeros
+  const float* scales;
+};
+template <bool FP8>
+__device__ inline FewUnit few_unit(const FewArgs& m, int unit) {
+  const int row_bytes = m.cols * (FP8 ? 1 : 2);
+  FewUnit u;
+  u.which = 0;
+#pragma unroll
+  for (int i = 1; i < kManyMax; ++i) u.which += unit >= m.first_block[i];  // unused ones start at the end
+  u.row = (unit - m.first_block[u.which]) * kFewRows;
+  u.weights = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<unsigned char*>(static_cast<const unsigned char*>(m.weights[u.which]) +
+                                 static_cast<size_t>(u.row) * row_bytes),
+      0, min(kFewRows, m.rows[u.which] - u.row) * row_bytes, 0x00020000);
+  u.scales = FP8 ? m.scales[u.which] + static_cast<size_t>(u.row / kGroup) * (m.cols / kGroup) : nullptr;
+  return u;
+}
+
+// The tokens' way into LDS, eight values a thread and load.
+template <bool FP8, int TOKENS>
+struct FewTokens {
+  static constexpr int kPieces = TOKENS * kFewColumns / 8;
+  static constexpr int kLoads = (kPieces + kFewThreads - 1) / kFewThreads;
+  typedef uint4 Values[kLoads];
+  static __device__ __forceinline__ void request(const FewArgs& m, Values& values) {
+    const int pieces = m.count * (m.cols / 8);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      if (i * kFewThreads >= pieces) break;
+      values[i] = reinterpret_cast<const uint4*>(
+          m.tokens)[min(i * kFewThreads + static_cast<int>(threadIdx.x), pieces - 1)];
+    }
+  }
+  // place(token, column, eight bf16 values), scale(token, group, scale)
+  template <class Place, class Scale>
+  static __device__ __forceinline__ void store(const FewArgs& m, const Values& values, Place place, Scale scale) {
+    const int pieces = m.count * (m.cols / 8);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      if (i * kFewThreads >= pieces) break;
+      const int piece = i * kFewThreads + static_cast<int>(threadIdx.x);
+      const int token = TOKENS == 1 ? 0 : piece / (m.cols / 8), c = (piece - token * (m.cols / 8)) * 8;
+      uint4 v = values[i];
+      if constexpr (FP8) {
+        const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+        uint32_t largest = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) largest = max(largest, max(words[e] & 0x7fffu, words[e] >> 16 & 0x7fffu));
+        const GroupQuantizer quantizer(row_max(largest));  // sixteen lanes hold a group
+        uint32_t rounded[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float first, second;
+          quantizer.round(__uint_as_float(words[e] << 16), __uint_as_float(words[e] & 0xffff0000u), first, second);
+          rounded[e] = (__float_as_uint(first) >> 16) | (__float_as_uint(second) & 0xffff0000u);  // exact in bf16
+        }
+        v = make_uint4(rounded[0], rounded[1], rounded[2], rounded[3]);
+        if (piece < pieces && c % kGroup == 0) scale(token, c / kGroup, quantizer.scale);
+      }
+      if (piece >= pieces) break;  // whole groups of sixteen lanes
+      place(token, c, v);
+    }
+  }
+};
+
+// Barrier for LDS: weights stay in flight.
+__device__ inline void few_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// STEPS: of a panel, as many steps of 1 KiB of each row as the registers hold; rows longer
+// than that are several panels.
+template <bool FP8, int STEPS, int TOKENS>
+__global__ void __launch_bounds__(kFewThreads)
+imported_one_kernel(FewArgs m, int panels) {
+  constexpr int R = kFewRows, kElements = FP8 ? 16 : 8;  // of a lane's piece
+  constexpr int kStepColumns = 64 * kElements, kReads = kElements / 8;
+  extern __shared__ uint4 few_lds[];  // [steps][TOKENS][kReads][64], then FP8: scales [steps][TOKENS][8]
+  const int lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int steps = STEPS * panels, groups = m.cols / kGroup, units = m.first_block[m.matrices];
+  const int row_bytes = m.cols * (FP8 ? 1 : 2);
+  const bool whole = steps * kStepColumns == m.cols;
+  float* token_scales = reinterpret_cast<float*>(few_lds + TOKENS * steps * kReads * 64);
+  uint4 raw[STEPS][R];
+  float scale[STEPS];
+  auto request = [&](const FewUnit& u, int panel, int step) {
+    const int at = (panel * STEPS + step) * 1024 + lane * 16;
+    const bool exists = whole || at < row_bytes;
+    if (FP8) scale[step] = u.scales[min(at / kGroup, groups - 1)];
+#pragma unroll
+    for (int r = 0; r < R; ++r)  // what lies past the end of a row reads zero
+      raw[step][r] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(u.weights, exists ? r * row_bytes + at : -1, 0, 0));
+    if (FP8 && !whole) scale[step] = exists ? scale[step] : 0.0f;
+  };
+
+  // The tokens first (requests are answered in order), the weights behind them.
+  using Tokens = FewTokens<FP8, TOKENS>;
+  typename Tokens::Values values;
+  Tokens::request(m, values);
+  __builtin_amdgcn_sched_barrier(0);
+  // a compute unit's waves lie far apart in the rows: where there are few, all of them
+  // have work
+  int unit = wave * gridDim.x + blockIdx.x;
+  FewUnit now = few_unit<FP8>(m, min(unit, units - 1));
+#pragma unroll
+  for (int step = 0; step < STEPS; ++step) request(now, 0, step);
+  __builtin_amdgcn_sched_barrier(0);
+  if (!whole) {  // the pieces past the end, and their scales
+    for (int i = threadIdx.x; i < TOKENS * steps * kReads * 64; i += kFewThreads) {
+      const int step = i / (TOKENS * kReads * 64);
+      if ((step * 64 + i % 64) * kElements >= m.cols) few_lds[i] = make_uint4(0, 0, 0, 0);
+    }
+    if (FP8)
+      for (int i = threadIdx.x; i < TOKENS * steps * 8; i += kFewThreads)
+        if (i / (TOKENS * 8) * 8 + i % 8 >= groups) token_scales[i] = 0.0f;
+  }
+  Tokens::store(
+      m, values,
+      [&](int token, int c, uint4 v) {
+        const int at = c / kElements;  // the piece of the row
+        few_lds[((at / 64 * TOKENS + token) * kReads + c % kElements / 8) * 64 + at % 64] = v;
+      },
+      [&](int token, int group, float s) { token_scales[(group / 8 * TOKENS + token) * 8 + group % 8] = s; });
+  few_barrier();
+
+  const bool odd = lane & 1, second = lane & 2;
+  uint4 x[2][kReads];
+  float x_scale[2] = {1.0f, 1.0f};
+  // the lane's places in LDS move with the steps, a token's offset is part of the read
+  constexpr int kStride = TOKENS * kReads * 64, kScaleStride = TOKENS * 8;
+  const uint4* x_at = few_lds + lane;
+  const float* scale_at = token_scales + lane / 8;
+  auto read_token = [&](int slot, int t) {
+#pragma unroll
+    for (int k = 0; k < kReads; ++k) x[slot][k] = x_at[(t * kReads + k) * 64];
+    if (FP8) x_scale[slot] = scale_at[t * 8];
+  };
+  read_token(0, 0);
+  while (unit < units) {
+    const int next_unit = unit + kFewWaves * gridDim.x;
+    float sums[TOKENS * R];
+#pragma unroll
+    for (int i = 0; i < TOKENS * R; ++i) sums[i] = 0.0f;
+    const int own_row = now.row, own_which = now.which;
+    for (int panel = 0; panel < panels; ++panel) {
+      const bool last = panel + 1 == panels;
+      if (last) now = few_unit<FP8>(m, min(next_unit, units - 1));
+      const int next_panel = last ? 0 : panel + 1;
+#pragma unroll
+      for (int step = 0; step < STEPS; ++step) {
+        uint4 w[R][kReads];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int k = 0; k < kReads; ++k)
+            w[r][k] = FP8 ? __builtin_bit_cast(uint4, fp8_to_bf16(raw[step][r], k)) : raw[step][r];
+        const float weight_scale = FP8 ? scale[step] : 1.0f;
+        __builtin_amdgcn_sched_barrier(0);
+        request(now, next_panel, step);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < TOKENS; ++t) {
+          // a token's values are read while the one before is multiplied
+          const int slot = (step * TOKENS + t) % 2;
+          if (t + 1 == TOKENS) {
+            const bool first = step + 1 == STEPS && last;
+            x_at = first ? few_lds + lane : x_at + kStride;
+            scale_at = first ? token_scales + lane / 8 : scale_at + kScaleStride;
+          }
+          read_token(1 - slot, t + 1 < TOKENS ? t + 1 : 0);
+          __builtin_amdgcn_sched_barrier(0);
+          const float factor = weight_scale * x_scale[slot];
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int k = 0; k < kReads; ++k) acc = mma_few(w[r][k], x[slot][k], acc);
+            const float low = odd ? acc[1] : acc[0], high = odd ? acc[3] : acc[2];
+            const float product = second ? high : low;
+            sums[t * R + r] = FP8 ? __builtin_fmaf(product, factor, sums[t * R + r]) : sums[t * R + r] + product;
+            asm volatile("" : "+v"(sums[t * R + r]));  // here: the compiler would keep every acc to the end
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // the last slot read is the first of the next panel
+        if (STEPS * TOKENS % 2 == 1 && step + 1 == STEPS) {
+#pragma unroll
+          for (int k = 0; k < kReads; ++k) x[0][k] = x[1][k];
+          x_scale[0] = x_scale[1];
+        }
+      }
+    }
+    const float sum = sums_of(sums);
+    constexpr int kLanes = 64 / (TOKENS * R);
+    const int index = lane / kLanes, token = index / R, row = own_row + index % R, rows = m.rows[own_which];
+    if (lane % kLanes == 0 && row < rows && token < m.count)
+      m.out[own_which][static_cast<size_t>(token) * rows + row] = float_to_bf16_bits(sum);
+    unit = next_unit;
+  }
+}
+
+// A step is 256 bytes of each of the four rows: lane 4 p + i holds piece p of row i and, of
+// the tokens, piece p of token i (of tokens i and 4 + i where QUADS is two).  STEPS: of a
+// panel, a multiple of four; step s belongs to the lanes 16 (s % 4) + p of the order of
+// sums above.
+template <bool FP8, int STEPS, int QUADS>
+__global__ void __launch_bounds__(kFewThreads)
+imported_several_kernel(FewArgs m, int panels) {
+  static_assert(STEPS % 4 == 0);
+  constexpr int kElements = FP8 ? 16 : 8;           // of a lane's piece
+  constexpr int kStepColumns = 16 * kElements, kReads = kElements / 8;
+  extern __shared__ uint4 few_lds[];  // [QUADS][steps][kReads][64], then FP8: scales [2 steps][8]
+  const int lane = threadIdx.x % 64, i4 = lane % 4, block = lane / 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int steps = STEPS * panels, groups = m.cols / kGroup, units = m.first_block[m.matrices];
+  const uint32_t row_bytes = m.cols * (FP8 ? 1 : 2);
+  const bool whole = steps * kStepColumns == m.cols;
+  float* token_scales = reinterpret_cast<float*>(few_lds + QUADS * steps * kReads * 64);
+  const uint32_t lane_at = i4 * row_bytes + block * 16;
+  uint4 raw[STEPS];
+  auto request = [&](const FewUnit& u, int panel, int step) {
+    const uint32_t at = (panel * STEPS + step) * 256;
+    // what lies past the end of a row reads zero
+    const uint32_t mine = whole || at + block * 16 < row_bytes ? lane_at : 0x80000000u;
+    raw[step] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(u.weights, mine, at, 0));
+  };
+  // a panel's scales: lane l holds that of group l of it
+  auto request_scales = [&](const FewUnit& u, int panel) {
+    const int group = panel * STEPS * 2 + lane;
+    return FP8 ? u.scales[min(group, groups - 1)] : 0.0f;
+  };
+
+  using Tokens = FewTokens<FP8, 4 * QUADS>;
+  typename Tokens::Values values;
+  Tokens::request(m, values);
+  __builtin_amdgcn_sched_barrier(0);
+  int unit = wave * gridDim.x + blockIdx.x;
+  FewUnit now = few_unit<FP8>(m, min(unit, units - 1));
+  float scales = request_scales(now, 0);  // before the weights, which it would have to wait for
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int step = 0; step < STEPS; ++step) request(now, 0, step);
+  __builtin_amdgcn_sched_barrier(0);
+  if (!whole) {  // the pieces past the end, and their scales
+    for (int i = threadIdx.x; i < QUADS * steps * kReads * 64; i += kFewThreads) {
+      const int step = i / (kReads * 64) % steps;
+      if ((step * 16 + i % 64 / 4) * kElements >= m.cols) few_lds[i] = make_uint4(0, 0, 0, 0);
+    }
+    if (FP8)
+      for (int i = threadIdx.x; i < 2 * steps * kFewTokens; i += kFewThreads)
+        if (i / kFewTokens >= groups) token_scales[i] = 0.0f;
+  }
+  Tokens::store(
+      m, values,
+      [&](int token, int c, uint4 v) {
+        const int at = c / kElements;  // the piece of the row
+        few_lds[((token / 4 * steps + at / 16) * kReads + c % kElements / 8) * 64 + at % 16 * 4 + token % 4] = v;
+      },
+      [&](int token, int group, float s) { token_scales[group * kFewTokens + token] = s; });
+  few_barrier();
+
+  // a step's tokens are read a step ahead
+  uint4 t[2][QUADS][kReads];
+  float token_scale[2][QUADS];
+  auto read_tokens = [&](int slot, int panel, int step) {
+    const int at = panel * STEPS + step;
+#pragma unroll
+    for (int j = 0; j < QUADS; ++j) {
+#pragma unroll
+      for (int k = 0; k < kReads; ++k) t[slot][j][k] = few_lds[((j * steps + at) * kReads + k) * 64 + lane];
+      if (FP8) token_scale[slot][j] = token_scales[(2 * at + block / 8) * kFewTokens + 4 * j + i4];
+    }
+  };
+  read_tokens(0, 0, 0);
+  while (unit < units) {
+    const int next_unit = unit + kFewWaves * gridDim.x;
+    floatx4 total[QUADS][4];
+#pragma unroll
+    for (int j = 0; j < QUADS; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) total[j][u] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    const FewUnit own = now;
+    for (int panel = 0; panel < panels; ++panel) {
+      const bool last = panel + 1 == panels;
+      if (last) now = few_unit<FP8>(m, min(next_unit, units - 1));
+      const int next_panel = last ? 0 : panel + 1;
+      const float next_scales = request_scales(now, next_panel);
+#pragma unroll
+      for (int step = 0; step < STEPS; ++step) {
+        const int slot = step % 2, u = step % 4;
+        read_tokens(1 - slot, step + 1 < STEPS ? panel : next_panel, step + 1 < STEPS ? step + 1 : 0);
+        __builtin_amdgcn_sched_barrier(0);
+        uint4 w[kReads];
+#pragma unroll
+        for (int k = 0; k < kReads; ++k)
+          w[k] = FP8 ? __builtin_bit_cast(uint4, fp8_to_bf16(raw[step], k)) : raw[step];
+        // pieces 0 .. 7 of a step of FP8 are one group, 8 .. 15 the next
+        float weight_scale = 1.0f;
+        if constexpr (FP8) {
+          const float low = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(scales), 2 * step));
+          const float high = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(scales), 2 * step + 1));
+          weight_scale = block < 8 ? low : high;
+          if (!whole) weight_scale = ((panel * STEPS + step) * 16 + block) * kElements < m.cols ? weight_scale : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < QUADS; ++j) {
+          floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int k = 0; k < kReads; ++k) acc = mma_few(w[k], t[slot][j][k], acc);
+          const float factor = FP8 ? weight_scale * token_scale[slot][j] : 1.0f;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            total[j][u][i] = FP8 ? __builtin_fmaf(acc[i], factor, total[j][u][i]) : total[j][u][i] + acc[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        request(now, next_panel, step);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      scales = next_scales;
+    }
+    // over the pieces; lanes 16 k + i end with row k of token i
+    const int row = own.row + lane / 16;
+#pragma unroll
+    for (int j = 0; j < QUADS; ++j) {
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = (total[j][0][i] + total[j][2][i]) + (total[j][1][i] + total[j][3][i]);
+      const bool upper = lane & 32, odd = lane & 16;
+      const float a = (upper ? v[2] : v[0]) + __shfl_xor(upper ? v[0] : v[2], 32, 64);
+      const float b = (upper ? v[3] : v[1]) + __shfl_xor(upper ? v[1] : v[3], 32, 64);
+      float sum = (odd ? b : a) + __shfl_xor(odd ? a : b, 16, 64);
+      sum += __shfl_xor(sum, 8, 64);
+      sum += __shfl_xor(sum, 4, 64);
+      const int token = 4 * j + i4, rows = m.rows[own.which];
+      if (lane % 16 < 4 && row < rows && token < m.count)
+        m.out[own.which][static_cast<size_t>(token) * rows + row] = float_to_bf16_bits(sum);
+    }
+    unit = next_unit;
+  }
+}
+
 // ---- more than eight tokens: the matrix cores --------------------------------
-// out[t, r] = sum_k w[r, k] x[t, k], 32 rows x 32 tokens a tile.  bf16 weights and
-// tokens are exact operands of v_mfma_f32_32x32x16_bf16.  FP8 codes are exact in bf16
+// out[t, r] = sum_k w[r, k] x[t, k], 16 or 32 rows x 16 or 32 tokens a tile.  bf16 weights and
+// tokens are exact operands of v_mfma_f32_16x16x32_bf16.  FP8 codes are exact in bf16
 // too, so FP8 weights are multiplied unscaled with the FP8 values of the quantized
 // tokens on v_mfma_f32_16x16x32_bf16, and each block of 128 contraction elements is
 // scaled once by (weight block scale) x (token group scale): the same products as (w
@@ -364,10 +815,6 @@ __global__ void __launch_bounds__(256) imported_matvec_ragged_kernel(MatVecArgs 
 // columns were more than a bf16 rounding off.)  The eight waves of a workgroup share a
 // tile and take every eighth block; their partial tiles are added in wave order
 // through LDS.
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float floatx4;
-typedef __attribute__((ext_vector_type(16))) float floatx16;
 
 // Tokens as FP8 codes and their group scales [tokens, n / 128].  The codes are written
 // in the order the matrix-core kernel reads them, so that each of its loads is one
@@ -389,20 +836,6 @@ imported_token_fp8_kernel(const uint16_t* x, int n, unsigned char* codes, float*
   codes[(piece * 64 + token % 16 + c % 64 / 16 * 16) * 16 + c % 16] =
       static_cast<unsigned char>(quantizer.code(v));
   if (threadIdx.x == 0) scales[static_cast<size_t>(token) * gridDim.x + block] = quantizer.scale;
-}
-
-// Eight FP8 codes (the lower or the upper eight of sixteen) as bf16, exactly.
-__device__ inline bf16x8 fp8_to_bf16(const uint4& codes, int part) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-  const uint32_t word[2] = {part == 0 ? codes.x : codes.z, part == 0 ? codes.y : codes.w};
-  bf16x8 out;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const bf16x2 low = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word[i], 1.0f, false);
-    const bf16x2 high = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(word[i], 1.0f, true);
-    out[4 * i] = low[0], out[4 * i + 1] = low[1], out[4 * i + 2] = high[0], out[4 * i + 3] = high[1];
-  }
-  return out;
 }
 
 constexpr int kTileWaves = 8;  // waves that split a tile's contraction
@@ -431,57 +864,118 @@ __device__ inline TilePlace tile_place(const TileManyArgs& m, int tile) {
   return {which, (tile - m.first_block[which]) * ROWS};
 }
 
-// bf16: one tile a workgroup.  Lane (n, h) covers elements [64 h, 64 h + 64) of a
-// 128-element block, for weight row n (A operand) and for token n (B operand).
+// The partial tiles of the waves (`elements` of 64 lanes each) added in wave order; element
+// e belongs to rows .. of the store.  Requests stay in flight across the barrier.
+template <int ELEMENTS, typename Store>
+__device__ inline void add_waves(float (&partial)[kTileWaves][ELEMENTS][64], const float (&own)[ELEMENTS], int wave,
+                                 int lane, Store store) {
+#pragma unroll
+  for (int i = 0; i < ELEMENTS; ++i) partial[wave][i][lane] = own[i];
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int k = 0; k < (ELEMENTS + kTileWaves - 1) / kTileWaves; ++k) {
+    const int e = k * kTileWaves + wave;
+    if (ELEMENTS % kTileWaves != 0 && e >= ELEMENTS) break;
+    float sum = partial[0][e][lane];
+#pragma unroll
+    for (int w = 1; w < kTileWaves; ++w) sum += partial[w][e][lane];
+    store(e, sum);
+  }
+}
+
+// bf16, the same walk over tiles of 16 rows as below.  Lane (q, n16) covers elements 32 s +
+// 8 q .. + 7 of each block of weight row n16 and of tokens n16 (and 16 + n16): operands of
+// v_mfma_f32_16x16x32_bf16 as they lie in memory, four lanes a 64-byte piece of a row.
+// Bound by the addresses of those pieces, sixteen rows a load.  5120 -> 16480, 9, 16 and 32
+// tokens: 62.7, 75.1 and 98.3 us with one tile of 32 rows a workgroup, 36.7, 37.7 and 75.5
+// so (32 tokens take twice the registers, so that the rows travel in several passes).
+template <int BLOCKS, int TOKEN_PARTS, bool ONE_PASS>
 __global__ void __launch_bounds__(64 * kTileWaves)
-imported_tile_kernel(TileManyArgs m) {
-  __shared__ float partial[kTileWaves - 1][16][64];
-  const TilePlace place = tile_place<32>(m, blockIdx.x);
-  const int rows = m.rows[place.which];
-  const int lane = threadIdx.x % 64, n = lane % 32, h = lane / 32;
-  const int wave = threadIdx.x / 64;
-  const int row = min(place.row + n, rows - 1);   // rows and tokens past the end repeat
-  const int token = min(n, m.count - 1);          // the last one and are not stored
-  const int groups = m.cols / kGroup;
-  const unsigned char* w = static_cast<const unsigned char*>(m.weights[place.which]) +
-                           (static_cast<size_t>(row) * m.cols + 64 * h) * 2;
-  const uint16_t* x = static_cast<const uint16_t*>(m.tokens) + static_cast<size_t>(token) * m.cols + 64 * h;
-  floatx16 total;
+imported_tile_bf16_kernel(TileManyArgs m, int passes) {
+  if constexpr (ONE_PASS) passes = 1;
+  constexpr int STEPS = kGroup / 32;
+  __shared__ float partial[2][kTileWaves][4 * TOKEN_PARTS][64];
+  const int lane = threadIdx.x % 64, n = lane % 16, q = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int groups = m.cols / kGroup, tiles = m.first_block[m.matrices];
+  auto block_of = [&](int pass, int b) { return wave + kTileWaves * (pass * BLOCKS + b); };
+  const uint32_t lane_at = (static_cast<uint32_t>(n) * m.cols + 8 * q) * 2;
+  uint4 raw[BLOCKS][STEPS], x[BLOCKS][STEPS][TOKEN_PARTS];
+  auto request = [&](const __amdgpu_buffer_rsrc_t& rows, int pass, int b) {
+    const uint32_t at = min(block_of(pass, b), groups - 1) * (kGroup * 2);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) total[i] = 0.0f;
-  for (int g = wave; g < groups; g += kTileWaves) {
-    uint4 xs[8];
+    for (int s = 0; s < STEPS; ++s)
+      raw[b][s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, lane_at, at + 64 * s, 0));
+  };
+  // rows past the end read zeros
+  auto rows_of = [&](int tile) {
+    const TilePlace place = tile_place<16>(m, tile);
+    const size_t first = static_cast<size_t>(place.row) * m.cols * 2;
+    const int rows = min(16, m.rows[place.which] - place.row);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<unsigned char*>(static_cast<const unsigned char*>(m.weights[place.which]) + first), 0,
+        rows * m.cols * 2, 0x00020000);
+  };
+  auto load_tokens = [&](int pass) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) xs[j] = *reinterpret_cast<const uint4*>(x + g * kGroup + 8 * j);
+    for (int j = 0; j < TOKEN_PARTS; ++j) {
+      // tokens past the end repeat the last one and are not stored
+      const uint16_t* token = static_cast<const uint16_t*>(m.tokens) +
+                              static_cast<size_t>(min(16 * j + n, m.count - 1)) * m.cols + 8 * q;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint4 bits =
-          *reinterpret_cast<const uint4*>(w + (static_cast<size_t>(g) * kGroup + 8 * j) * 2);
-      total = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bits),
-                                                      __builtin_bit_cast(bf16x8, xs[j]), total,
-                                                      0, 0, 0);
+      for (int b = 0; b < BLOCKS; ++b) {
+        const int g = block_of(pass, b);
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+          x[b][s][j] = *reinterpret_cast<const uint4*>(token + min(g, groups - 1) * kGroup + 32 * s);
+          if (g >= groups) x[b][s][j] = make_uint4(0, 0, 0, 0);  // a block past the end
+        }
+      }
     }
+  };
+  load_tokens(0);
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    const __amdgpu_buffer_rsrc_t rows = rows_of(blockIdx.x);
+#pragma unroll
+    for (int b = 0; b < BLOCKS; ++b) request(rows, 0, b);
   }
-  if (wave > 0) {
+  __builtin_amdgcn_sched_barrier(0);
+  int buffer = 0;
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, buffer ^= 1) {
+    const TilePlace place = tile_place<16>(m, tile);
+    const int rows = m.rows[place.which];
+    floatx4 total[TOKEN_PARTS];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) partial[wave - 1][i][lane] = total[i];
-  }
-  __syncthreads();
-  if (wave > 0) return;
+    for (int j = 0; j < TOKEN_PARTS; ++j) total[j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int pass = 0; pass < passes; ++pass) {
+      if (!ONE_PASS && (pass > 0 || tile != static_cast<int>(blockIdx.x))) load_tokens(pass);
+      const int next_pass = pass + 1 < passes ? pass + 1 : 0;
+      const int next_tile = next_pass > 0 ? tile : min(tile + static_cast<int>(gridDim.x), tiles - 1);
+      const __amdgpu_buffer_rsrc_t next_rows = rows_of(next_tile);
 #pragma unroll
-  for (int i = 0; i < 16; ++i)
+      for (int b = 0; b < BLOCKS; ++b) {
 #pragma unroll
-    for (int w = 0; w < kTileWaves - 1; ++w) total[i] += partial[w][i][lane];
-  // accumulator element 4 q + i = (row 8 q + 4 h + i, token n)
-  if (n >= m.count) return;
+        for (int s = 0; s < STEPS; ++s)
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = place.row + 8 * q + 4 * h + i;
-      if (r < rows)
-        m.out[place.which][static_cast<size_t>(n) * rows + r] = float_to_bf16_bits(total[4 * q + i]);
+          for (int j = 0; j < TOKEN_PARTS; ++j)
+            total[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, raw[b][s]),
+                                                               __builtin_bit_cast(bf16x8, x[b][s][j]), total[j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        request(next_rows, next_pass, b);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
+    float own[4 * TOKEN_PARTS];
+#pragma unroll
+    for (int i = 0; i < 4 * TOKEN_PARTS; ++i) own[i] = total[i / 4][i % 4];
+    // element e is row 4 q + e % 4, token 16 (e / 4) + n
+    add_waves(partial[buffer], own, wave, lane, [&](int e, float sum) {
+      const int row = place.row + 4 * q + e % 4, token = 16 * (e / 4) + n;
+      if (row < rows && token < m.count)
+        m.out[place.which][static_cast<size_t>(token) * rows + row] = float_to_bf16_bits(sum);
+    });
+  }
 }
 
 // FP8: one workgroup a compute unit that walks over tiles.  A wave's blocks of the
@@ -493,18 +987,19 @@ imported_tile_kernel(TileManyArgs m) {
 // take several passes a tile, for each of which the tokens are loaded again.  Lane (q,
 // n16) covers elements 16 q .. + 15 of each half block of weight row n16 of each of
 // PARTS 16-row parts (A operands) and of tokens n16 and 16 + n16 (B operands).
-template <int BLOCKS, int PARTS, bool ONE_PASS>
+// TOKEN_PARTS: one for up to sixteen tokens.
+template <int BLOCKS, int PARTS, int TOKEN_PARTS, bool ONE_PASS>
 __global__ void __launch_bounds__(64 * kTileWaves)
 imported_tile_fp8_kernel(TileManyArgs m, int passes) {
   if constexpr (ONE_PASS) passes = 1;
-  __shared__ float partial[2][kTileWaves][8 * PARTS][64];
+  __shared__ float partial[2][kTileWaves][4 * TOKEN_PARTS * PARTS][64];
   const int lane = threadIdx.x % 64, n = lane % 16, q = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int groups = m.cols / kGroup, tiles = m.first_block[m.matrices];
   auto block_of = [&](int pass, int b) { return wave + kTileWaves * (pass * BLOCKS + b); };
   const uint32_t lane_at = static_cast<uint32_t>(n) * m.cols + 16 * q;
-  uint4 raw[BLOCKS][2][PARTS], x[BLOCKS][2][2];  // [block][half][rows or tokens]
-  float group_scale[BLOCKS][2];
+  uint4 raw[BLOCKS][2][PARTS], x[BLOCKS][2][TOKEN_PARTS];  // [block][half][rows or tokens]
+  float group_scale[BLOCKS][TOKEN_PARTS];
   // rows past the end read zeros
   auto request = [&](const __amdgpu_buffer_rsrc_t& rows, int pass, int b) {
     const uint32_t at = min(block_of(pass, b), groups - 1) * kGroup;
@@ -530,10 +1025,10 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
 #pragma unroll
       for (int half = 0; half < 2; ++half)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < TOKEN_PARTS; ++t)
           x[b][half][t] = static_cast<const uint4*>(m.tokens)[((g * 2 + half) * 2 + t) * 64 + lane];
 #pragma unroll
-      for (int t = 0; t < 2; ++t)  // tokens past the end are not stored
+      for (int t = 0; t < TOKEN_PARTS; ++t)  // tokens past the end are not stored
         group_scale[b][t] = m.token_scales[static_cast<size_t>(min(16 * t + n, m.count - 1)) * groups + g];
     }
   };
@@ -549,11 +1044,11 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
     const TilePlace place = tile_place<16 * PARTS>(m, tile);
     const int rows = m.rows[place.which];
     const float* block_scale = m.weight_scales[place.which] + static_cast<size_t>(place.row / kGroup) * groups;
-    floatx4 total[PARTS][2];
+    floatx4 total[PARTS][TOKEN_PARTS];
 #pragma unroll
     for (int i = 0; i < PARTS; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) total[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < TOKEN_PARTS; ++j) total[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     for (int pass = 0; pass < passes; ++pass) {
       if (!ONE_PASS && (pass > 0 || tile != static_cast<int>(blockIdx.x))) load_tokens(pass);
       const int next_pass = pass + 1 < passes ? pass + 1 : 0;
@@ -564,32 +1059,32 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
         // a block past the end contributes nothing (its scale is read in range)
         const int g = block_of(pass, b);
         const float weight_scale = g < groups ? block_scale[min(g, groups - 1)] : 0.0f;
-        floatx4 acc[PARTS][2];
+        floatx4 acc[PARTS][TOKEN_PARTS];
 #pragma unroll
         for (int i = 0; i < PARTS; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+          for (int j = 0; j < TOKEN_PARTS; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
         // the tokens are converted here for every tile: converted once they would take
         // twice the registers, which the compiler does not see
 #pragma unroll
         for (int half = 0; half < 2; ++half)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
+          for (int j = 0; j < TOKEN_PARTS; ++j)
             asm volatile("" : "+v"(x[b][half][j].x), "+v"(x[b][half][j].y), "+v"(x[b][half][j].z),
                               "+v"(x[b][half][j].w));
 #pragma unroll
         for (int half = 0; half < 2; ++half)
 #pragma unroll
           for (int part = 0; part < 2; ++part) {
-            bf16x8 w[PARTS], t[2];
+            bf16x8 w[PARTS], t[TOKEN_PARTS];
 #pragma unroll
             for (int i = 0; i < PARTS; ++i) w[i] = fp8_to_bf16(raw[b][half][i], part);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) t[j] = fp8_to_bf16(x[b][half][j], part);
+            for (int j = 0; j < TOKEN_PARTS; ++j) t[j] = fp8_to_bf16(x[b][half][j], part);
 #pragma unroll
             for (int i = 0; i < PARTS; ++i)
 #pragma unroll
-              for (int j = 0; j < 2; ++j)
+              for (int j = 0; j < TOKEN_PARTS; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], t[j], acc[i][j], 0, 0, 0);
           }
         __builtin_amdgcn_sched_barrier(0);
@@ -598,24 +1093,20 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
 #pragma unroll
         for (int i = 0; i < PARTS; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) total[i][j] += acc[i][j] * (weight_scale * group_scale[b][j]);
+          for (int j = 0; j < TOKEN_PARTS; ++j) total[i][j] += acc[i][j] * (weight_scale * group_scale[b][j]);
       }
     }
+    constexpr int kElements = 4 * TOKEN_PARTS * PARTS;
+    float own[kElements];
 #pragma unroll
-    for (int i = 0; i < 8 * PARTS; ++i) partial[buffer][wave][i][lane] = total[i / 8][i / 4 % 2][i % 4];
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // requests stay in flight
-    // every wave adds one or two of the elements: element e is rows 16 (e / 8) + 4 q + e % 4,
-    // tokens 16 (e / 4 % 2) + n
-#pragma unroll
-    for (int k = 0; k < PARTS; ++k) {
-      const int e = PARTS * wave + k;
-      float sum = partial[buffer][0][e][lane];
-#pragma unroll
-      for (int w = 1; w < kTileWaves; ++w) sum += partial[buffer][w][e][lane];
-      const int row = place.row + 16 * (e / 8) + 4 * q + e % 4, token = 16 * (e / 4 % 2) + n;
+    for (int i = 0; i < kElements; ++i) own[i] = total[i / (4 * TOKEN_PARTS)][i / 4 % TOKEN_PARTS][i % 4];
+    // element e is row 16 (e / (4 TOKEN_PARTS)) + 4 q + e % 4, token 16 (e / 4 % TOKEN_PARTS) + n
+    add_waves(partial[buffer], own, wave, lane, [&](int e, float sum) {
+      const int row = place.row + 16 * (e / (4 * TOKEN_PARTS)) + 4 * q + e % 4;
+      const int token = 16 * (e / 4 % TOKEN_PARTS) + n;
       if (row < rows && token < m.count)
         m.out[place.which][static_cast<size_t>(token) * rows + row] = float_to_bf16_bits(sum);
-    }
+    });
   }
 }
 
@@ -629,41 +1120,110 @@ int fp8_tile_rows(int matrices, const int* rows) {
   return tiles >= 256 ? 16 : 32;
 }
 
-void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t, int tile_rows) {
-  const int owned = (t.cols / kGroup + kTileWaves - 1) / kTileWaves;  // blocks of a wave
-  const int tiles = t.first_block[t.matrices];
+template <int PARTS, int TOKEN_PARTS>
+void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t) {
+  const int groups = t.cols / kGroup, owned = (groups + kTileWaves - 1) / kTileWaves;  // blocks of a wave
+  const unsigned grid = std::min(t.first_block[t.matrices], 256);
   int passes = 1;
-  auto launch = [&](auto kernel) { kernel<<<std::min(tiles, 256), 64 * kTileWaves, 0, s>>>(t, passes); };
-  if (tile_rows == 16) {
-    passes = (owned + 5) / 6;
-    if (passes > 1) return launch(imported_tile_fp8_kernel<6, 1, false>);
-    switch (owned) {
-      case 1: return launch(imported_tile_fp8_kernel<1, 1, true>);
-      case 2: return launch(imported_tile_fp8_kernel<2, 1, true>);
-      case 3: return launch(imported_tile_fp8_kernel<3, 1, true>);
-      case 4: return launch(imported_tile_fp8_kernel<4, 1, true>);
-      case 5: return launch(imported_tile_fp8_kernel<5, 1, true>);
-      default: return launch(imported_tile_fp8_kernel<6, 1, true>);
-    }
-  }
-  if (owned > 5) {
+  auto launch = [&](auto kernel) { kernel<<<grid, 64 * kTileWaves, 0, s>>>(t, passes); };
+  // as many blocks as a wave's registers hold
+  constexpr int kMost = PARTS * TOKEN_PARTS == 4 ? 5 : 6;
+  if (owned > kMost) {
     passes = (owned + 3) / 4;
-    return (owned + passes - 1) / passes == 3 ? launch(imported_tile_fp8_kernel<3, 2, false>)
-                                              : launch(imported_tile_fp8_kernel<4, 2, false>);
+    return (owned + passes - 1) / passes == 3 ? launch(imported_tile_fp8_kernel<3, PARTS, TOKEN_PARTS, false>)
+                                              : launch(imported_tile_fp8_kernel<4, PARTS, TOKEN_PARTS, false>);
   }
   switch (owned) {
-    case 1: return launch(imported_tile_fp8_kernel<1, 2, true>);
-    case 2: return launch(imported_tile_fp8_kernel<2, 2, true>);
-    case 3: return launch(imported_tile_fp8_kernel<3, 2, true>);
-    case 4: return launch(imported_tile_fp8_kernel<4, 2, true>);
-    default: return launch(imported_tile_fp8_kernel<5, 2, true>);
+    case 1: return launch(imported_tile_fp8_kernel<1, PARTS, TOKEN_PARTS, true>);
+    case 2: return launch(imported_tile_fp8_kernel<2, PARTS, TOKEN_PARTS, true>);
+    case 3: return launch(imported_tile_fp8_kernel<3, PARTS, TOKEN_PARTS, true>);
+    case 4: return launch(imported_tile_fp8_kernel<4, PARTS, TOKEN_PARTS, true>);
+    case 5: return launch(imported_tile_fp8_kernel<5, PARTS, TOKEN_PARTS, true>);
+    default:
+      if constexpr (kMost == 6) launch(imported_tile_fp8_kernel<6, PARTS, TOKEN_PARTS, true>);
   }
 }
 
-// The matrix-core path takes bf16 and FP8 weights whose rows are whole
-// 128-element blocks; fewer than nine tokens are cheaper on the vector path.
-bool tile_path(int storage, int tokens, int input_dim) {
-  return storage != PLUTO_HIP_MATRIX_F32 && tokens > 8 && input_dim % kGroup == 0;
+template <int TOKEN_PARTS>
+void launch_bf16_tiles(hipStream_t s, const TileManyArgs& t) {
+  const int owned = (t.cols / kGroup + kTileWaves - 1) / kTileWaves;
+  const unsigned grid = std::min(t.first_block[t.matrices], 256);
+  int passes = 1;
+  auto launch = [&](auto kernel) { kernel<<<grid, 64 * kTileWaves, 0, s>>>(t, passes); };
+  constexpr int kMost = TOKEN_PARTS == 1 ? 6 : 3;
+  if (owned > kMost) {
+    passes = (owned + kMost - 1) / kMost;
+    return launch(imported_tile_bf16_kernel<kMost, TOKEN_PARTS, false>);
+  }
+  switch (owned) {
+    case 1: return launch(imported_tile_bf16_kernel<1, TOKEN_PARTS, true>);
+    case 2: return launch(imported_tile_bf16_kernel<2, TOKEN_PARTS, true>);
+    case 3: return launch(imported_tile_bf16_kernel<3, TOKEN_PARTS, true>);
+    case 4: if constexpr (kMost == 6) return launch(imported_tile_bf16_kernel<4, TOKEN_PARTS, true>);
+    case 5: if constexpr (kMost == 6) return launch(imported_tile_bf16_kernel<5, TOKEN_PARTS, true>);
+    default: if constexpr (kMost == 6) return launch(imported_tile_bf16_kernel<6, TOKEN_PARTS, true>);
+  }
+}
+
+template <bool FP8, int TOKENS>
+void launch_one(hipStream_t s, const FewArgs& a) {
+  const int steps = (a.cols + (FP8 ? 1023 : 511)) / (FP8 ? 1024 : 512);
+  const int panels = (steps + 5) / 6, of_panel = (steps + panels - 1) / panels;
+  const unsigned grid = std::min(a.first_block[a.matrices], 256);
+  const size_t lds = static_cast<size_t>(TOKENS) * of_panel * panels * (FP8 ? 2048 + 32 : 1024);
+  auto launch = [&](auto kernel) { kernel<<<grid, kFewThreads, lds, s>>>(a, panels); };
+  switch (of_panel) {
+    case 1: return launch(imported_one_kernel<FP8, 1, TOKENS>);
+    case 2: return launch(imported_one_kernel<FP8, 2, TOKENS>);
+    case 3: return launch(imported_one_kernel<FP8, 3, TOKENS>);
+    case 4: return launch(imported_one_kernel<FP8, 4, TOKENS>);
+    case 5: return launch(imported_one_kernel<FP8, 5, TOKENS>);
+    default: return launch(imported_one_kernel<FP8, 6, TOKENS>);
+  }
+}
+template <bool FP8, int QUADS>
+void launch_several(hipStream_t s, const FewArgs& a) {
+  const int steps = (a.cols + (FP8 ? 255 : 127)) / (FP8 ? 256 : 128);
+  int panels = (steps + 23) / 24;
+  auto panel_steps = [&] { return ((steps + panels - 1) / panels + 3) / 4 * 4; };
+  // what the panels hold past the end must not take more LDS than the widest rows do
+  while (panel_steps() * panels > kFewColumns / (FP8 ? 256 : 128)) ++panels;
+  const int of_panel = panel_steps();
+  const unsigned grid = std::min(a.first_block[a.matrices], 256);
+  const size_t lds = static_cast<size_t>(of_panel) * panels * (QUADS * (FP8 ? 2048 : 1024) + (FP8 ? 2 * kFewTokens * 4 : 0));
+  auto launch = [&](auto kernel) { kernel<<<grid, kFewThreads, lds, s>>>(a, panels); };
+  switch (of_panel) {
+    case 4: return launch(imported_several_kernel<FP8, 4, QUADS>);
+    case 8: return launch(imported_several_kernel<FP8, 8, QUADS>);
+    case 12: return launch(imported_several_kernel<FP8, 12, QUADS>);
+    case 16: return launch(imported_several_kernel<FP8, 16, QUADS>);
+    case 20: return launch(imported_several_kernel<FP8, 20, QUADS>);
+    default: return launch(imported_several_kernel<FP8, 24, QUADS>);
+  }
+}
+// Two tokens of FP8 weights take 21.7 us in the kernel for one and 19.6 in the other (5120
+// -> 16480), two of bf16 weights, which need no conversion, 27.6 and 29.0.
+template <bool FP8>
+void launch_few(hipStream_t s, const FewArgs& a) {
+  if (a.count == 1) return launch_one<FP8, 1>(s, a);
+  if constexpr (!FP8)
+    if (a.count == 2) return launch_one<FP8, 2>(s, a);
+  return a.count <= 4 ? launch_several<FP8, 1>(s, a) : launch_several<FP8, 2>(s, a);
+}
+
+// The matrix cores take bf16 and FP8 weights whose rows are whole 128-element blocks: up
+// to eight tokens of rows that fit in LDS, and more.  Everything else, and up to eight
+// tokens of longer rows, is the vector path's; what up to eight tokens take does not
+// depend on their number, so that a token's results do not either.  Weights are read by
+// buffer loads, which take whole words; tokens in pieces of sixteen bytes, but for the
+// kernel that makes FP8 codes of more than eight, which takes elements.
+bool matrix_cores(int storage, int matrices, const void* const* weights, const void* input, int tokens, int input_dim) {
+  if (storage == PLUTO_HIP_MATRIX_F32 || input_dim % kGroup != 0) return false;
+  auto aligned = [](const void* p, unsigned bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; };
+  for (int i = 0; i < matrices; ++i)
+    if (!aligned(weights[i], 4)) return false;
+  if (tokens <= kFewTokens && input_dim > kFewColumns) return false;
+  return aligned(input, 16) || (tokens > kFewTokens && storage == PLUTO_HIP_MATRIX_FP8_E4M3);
 }
 
 template <int STORAGE, int TOKENS, bool PREPARE>
@@ -771,7 +1331,16 @@ int launch_dense_imported_forward(hipStream_t s, int storage, int matrices,
           args.first_block[i] + (used ? (output_dims[i] + rows_per_block - 1) / rows_per_block : 0);
     }
   };
-  if (!tile_path(storage, tokens, input_dim)) {
+  const bool matrix = matrix_cores(storage, matrices, weights, input, tokens, input_dim);
+  if (matrix && tokens <= kFewTokens) {
+    FewArgs a;
+    fill(a, a.scales, 4);
+    a.tokens = static_cast<const uint16_t*>(input);
+    a.count = tokens;
+    fp8 ? launch_few<true>(s, a) : launch_few<false>(s, a);
+    return launch_status();
+  }
+  if (!matrix) {
     MatVecArgs a;
     fill(a, a.scales, 4 * kRowsPerWave);
     if (matvec_prepares(storage, input, tokens, input_dim)) {
@@ -795,7 +1364,7 @@ int launch_dense_imported_forward(hipStream_t s, int storage, int matrices,
     return launch_status();
   }
   TileManyArgs t;
-  const int tile_rows = fp8 ? fp8_tile_rows(matrices, output_dims) : 32;
+  const int tile_rows = fp8 ? fp8_tile_rows(matrices, output_dims) : 16;
   fill(t, t.weight_scales, tile_rows);
   const unsigned char* token_bytes = static_cast<const unsigned char*>(input);
   if (fp8) {
@@ -807,14 +1376,15 @@ int launch_dense_imported_forward(hipStream_t s, int storage, int matrices,
     token_bytes = codes;
     t.token_scales = token_scales;
   }
-  const int blocks = t.first_block[matrices];
   for (int done = 0; done < tokens; done += 32) {
     t.count = tokens - done < 32 ? tokens - done : 32;
     t.tokens = token_bytes + static_cast<size_t>(done) * input_dim * (fp8 ? 1 : 2);
-    if (fp8)
-      launch_fp8_tiles(s, t, tile_rows);
+    if (!fp8)
+      t.count <= 16 ? launch_bf16_tiles<1>(s, t) : launch_bf16_tiles<2>(s, t);
+    else if (tile_rows == 16)
+      t.count <= 16 ? launch_fp8_tiles<1, 1>(s, t) : launch_fp8_tiles<1, 2>(s, t);
     else
-      imported_tile_kernel<<<blocks, 64 * kTileWaves, 0, s>>>(t);
+      t.count <= 16 ? launch_fp8_tiles<2, 1>(s, t) : launch_fp8_tiles<2, 2>(s, t);
     if (fp8) t.token_scales += static_cast<size_t>(32) * (input_dim / kGroup);
     for (int i = 0; i < matrices; ++i) t.out[i] += static_cast<size_t>(32) * output_dims[i];
   }

@@ -336,3 +336,59 @@ def test_a_non_finite_token_gives_nan_and_touches_no_other(capi, oracle, tokens,
     want = oracle.imported_matvec(oracle.MATRIX_FP8_E4M3, w.cpu().numpy(), scales.cpu().numpy(),
                                   x[0].float().cpu().numpy())
     assert np.isnan(want).all()
+
+
+@pytest.mark.parametrize("storage", ["bf16", "fp8"])
+@pytest.mark.parametrize("cols,heights", [(128, [1]), (256, [3, 4]), (384, [130]), (1152, [5, 1, 2050]),
+                                          (5120, [129, 7]), (8448, [6]), (9216, [9, 64]), (9344, [5])])
+def test_few_and_many_tokens_of_whole_blocks(capi, storage, cols, heights):
+    """The matrix-core kernels for one, several and more than eight tokens at the edges
+    of their panels (and one width past them): row quadruples that end early, more than
+    one matrix, weights and tokens that do not start 16-byte aligned.  Up to eight tokens
+    give one token's bits; every result lies within the rounding of a bf16 result (eight bits: 2^-8)
+    and of up to 128 FP32 additions on a term's way (2^-17 of the products' magnitudes)
+    of the float64 sum."""
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    # tokens that are FP8 values times a power of two are quantized exactly
+    x = torch.randn((33, cols), generator=gen, device="cuda").to(torch.float8_e4m3fn).float()
+    x.view(33, cols // 128, 128)[:, :, 5] = 448.0
+    x = (x * 0.25).to(torch.bfloat16)
+    code = {"bf16": capi.MATRIX_BF16, "fp8": capi.MATRIX_FP8_E4M3}[storage]
+    weights, scales, full = [], [], []
+    for rows in heights:
+        w = torch.randn((rows, cols), generator=gen, device="cuda")
+        s = torch.rand(((rows + 127) // 128, cols // 128), generator=gen, device="cuda") + 0.5
+        if storage == "bf16":
+            weights.append(w.to(torch.bfloat16))
+            full.append(weights[-1].double())
+        else:
+            w = w.to(torch.float8_e4m3fn)
+            weights.append(w.view(torch.uint8))
+            scales.append(s)
+            full.append(w.double() * s.double().repeat_interleave(128, 0)[:rows].repeat_interleave(128, 1))
+    scales = scales or None
+    single = [capi.dense_imported_forward_many(code, weights, scales, x[t:t + 1].clone()) for t in range(8)]
+
+    def check(got, count, i):
+        want = x[:count].double() @ full[i].t()
+        bound = 2.0 ** -8 * want.abs() + 2.0 ** -17 * (x[:count].double().abs() @ full[i].abs().t())
+        assert ((got.double() - want).abs() <= bound).all(), (count, i)
+
+    for count in (1, 2, 3, 4, 5, 8, 9, 16, 17, 33):
+        got = capi.dense_imported_forward_many(code, weights, scales, x[:count].clone())
+        for i in range(len(heights)):
+            check(got[i], count, i)
+            for t in range(count if count <= 8 else 0):
+                assert torch.equal(got[i][t], single[t][i][0]), (count, t)
+
+    def shifted(tensor, elements):
+        room = torch.empty(tensor.numel() + elements, dtype=tensor.dtype, device="cuda")[elements:].view(tensor.shape)
+        return room.copy_(tensor)
+
+    for count in (1, 3, 17):
+        for elements in (1, 2, 4):
+            inputs = shifted(x[:count], elements)
+            moved = [shifted(w, 4 * elements // w.element_size()) for w in weights]
+            got = capi.dense_imported_forward_many(code, moved, scales, inputs)
+            for i in range(len(heights)):
+                check(got[i], count, i)
