@@ -1,58 +1,15 @@
 // FP32 attention on the bf16 matrix cores: what the forward and backward kernels share.
 //
-// An FP32 number is the sum of three bf16 numbers (8 + 8 + 8 mantissa bits), and a
-// product of two such sums is six bf16 matrix products with FP32 sums: the three left
-// out are 2^-25 of the product, less than one FP32 rounding.  Six v_mfma_f32_32x32x16_bf16
-// take 192 cycles where the FP32 instruction needs 512 for the same depth; making the
-// pieces costs 44 cycles of vector instructions a pair of numbers.
-//
 // A workgroup of four waves owns 32 rows of one side, kept in LDS as pieces in operand
 // order; every wave streams tiles of 32 rows of the other side of its own through an area
 // of LDS, where a tile lies as pieces and is read both ways: by rows for the score
 // products, transposed for those that contract over rows.
 #pragma once
 
-#include "mfma_tile.h"
+#include "bf16_pieces.h"
 
 namespace pluto_hip {
 
-struct Pieces {
-  bf16x8 part[3];
-};
-
-// acc + a b, smallest products first.
-__device__ inline floatx16 mma_pieces(const Pieces& a, const Pieces& b, floatx16 acc) {
-#pragma unroll
-  for (int i = 2; i >= 0; --i)
-#pragma unroll
-    for (int j = 2 - i; j >= 0; --j) acc = mfma32(a.part[i], b.part[j], acc);
-  return acc;
-}
-
-// Two numbers as the packed words of their pieces.
-__device__ inline void split_pair(float first, float second, uint32_t& high, uint32_t& middle, uint32_t& low) {
-  high = pack_bf16(first, second);
-  first -= __uint_as_float(high << 16);
-  second -= __uint_as_float(high & 0xffff0000u);
-  middle = pack_bf16(first, second);
-  first -= __uint_as_float(middle << 16);
-  second -= __uint_as_float(middle & 0xffff0000u);
-  low = pack_bf16(first, second);
-}
-__device__ inline Pieces split_eight(const float (&x)[8]) {
-  uint32_t words[3][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) split_pair(x[2 * i], x[2 * i + 1], words[0][i], words[1][i], words[2][i]);
-  Pieces out;
-#pragma unroll
-  for (int p = 0; p < 3; ++p)
-    out.part[p] = as_bf16x8(make_uint4(words[p][0], words[p][1], words[p][2], words[p][3]));
-  return out;
-}
-__device__ inline Pieces split_eight(float4 a, float4 b) {
-  const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-  return split_eight(x);
-}
 // Accumulator registers 8 s2 .. 8 s2 + 7 as a B operand.
 __device__ inline Pieces split_accumulator(const floatx16& acc, int s2) {
   float x[8];

@@ -2,7 +2,7 @@
 // gradients as the token-by-token kernels of gdn_backward.hip
 // (RecurrenceForward / RecurrenceBackward, src/llm/layers/
 // sequence_delta_net.cc:55-102 and :171-253), computed 64 tokens at a time on
-// the FP32 matrix cores, and with one saved state per chunk instead of one per
+// the matrix cores in FP32, and with one saved state per chunk instead of one per
 // token.
 //
 // For a chunk entered with state S (rows: key channels, columns: value
@@ -42,14 +42,12 @@
 // accumulator, whose lanes are columns and whose registers are four neighbouring rows,
 // is stored in that order as it is.
 //
-// Matrix products run on v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32, whose
-// rate bounds all of this (about 55 GFLOP at 2048 tokens of 48 heads, 360 us of the
-// card's FP32 matrix rate); the triangular factors are multiplied by halves.  At that
-// size the kernels of this file take 770 us, where one kernel a term of the
-// formulas above, with M and B, took 1766 us.
+// Matrix products of the parallel kernels run on v_mfma_f32_32x32x2_f32 and
+// v_mfma_f32_16x16x4_f32; the triangular factors are multiplied by halves.  Those of the
+// sequential kernels take three bf16 pieces of every factor (bf16_pieces.h).
 #include "gdn.h"
 
-#include "mfma_tile.h"
+#include "bf16_pieces.h"
 
 #include <type_traits>
 
@@ -146,22 +144,6 @@ __device__ inline floatx4 mma16(floatx4 acc, float4 a, floatx4 b) {
   return mma16(acc, a, make_float4(b[0], b[1], b[2], b[3]));
 }
 
-// One product of several tiles with the same left operand: their chains take turns.
-template <int TILES, class F>
-__device__ inline void mma16_tiles(floatx4 (&acc)[TILES], float4 a, F right) {
-  float4 b[TILES];
-#pragma unroll
-  for (int c = 0; c < TILES; ++c) b[c] = right(c);
-#pragma unroll
-  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[c].x, acc[c], 0, 0, 0);
-#pragma unroll
-  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[c].y, acc[c], 0, 0, 0);
-#pragma unroll
-  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[c].z, acc[c], 0, 0, 0);
-#pragma unroll
-  for (int c = 0; c < TILES; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[c].w, acc[c], 0, 0, 0);
-}
-
 __device__ inline float4 gather4(const float* p, int stride) {
   return make_float4(p[0], p[stride], p[2 * stride], p[3 * stride]);
 }
@@ -237,11 +219,12 @@ struct Memory {
     else
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rsrc, lane, uniform, 0);
   }
+  // The uniform part is added in either case: a store of four registers at a scalar offset
+  // still reads them when the next instruction may already write them (seen as a fourth
+  // element taken from a later value), and the compiler keeps the two apart only where
+  // the offset is no register.
   __device__ void put4(float4 v, unsigned lane, unsigned uniform) const {
-    if (TOKENS)
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint32x4, v), rsrc, lane + uniform, 0, 0);
-    else
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint32x4, v), rsrc, lane, uniform, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint32x4, v), rsrc, lane + uniform, 0, 0);
   }
 };
 using Record = Memory<false>;
@@ -315,7 +298,8 @@ chunk_prepare_kernel(ChunkedArgs a) {
     float g[kC], beta[kC], fk[kC];
   } sm;
   const ChunkView v(a, blockIdx.x, blockIdx.y);
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int h = lane / 32, n = lane % 32, quarter = lane / 16, n16 = lane % 16;
   float* gates = a.r.gates + v.rec * kGateRows * kC;
 
@@ -605,12 +589,40 @@ __device__ inline Slice slice_of_block(const ChunkedArgs& a) {
 }
 
 // The state of a slice lives in accumulators: tile t of wave w holds rows 32 w + 16 t ..
-// + 15 of sixteen columns.  The LDS copy [column][row] is what the other waves multiply
-// and where the rows of the saved state come from.
-__device__ inline void publish_state(const floatx4& first, const floatx4& second, float* rows) {
-  store4(rows, make_float4(first[0], first[1], first[2], first[3]));
-  store4(rows + 16, make_float4(second[0], second[1], second[2], second[3]));
+// + 15 of sixteen columns.  Its pieces (see bf16_pieces.h) go to LDS in operand order,
+// where the contraction index runs over both tiles: element e of quarter q of step s is row
+// 32 s + 16 (e / 4) + 4 q + e % 4, so that a wave's accumulators are step w as they are,
+// and of 64 tokens a wave's are half of step w / 2.  The left operands come from the
+// records as FP32, two pieces of four columns a lane and step, and are split between the
+// products of the step before.
+template <int STEPS>
+struct OperandLds {
+  uint4 part[STEPS][3][64];
+  __device__ void put(int step, int lane, const Pieces& p) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) part[step][i][lane] = __builtin_bit_cast(uint4, p.part[i]);
+  }
+  // four elements of a lane: the first or second half of a step's
+  __device__ void put_half(int step, int half, int lane, float4 v) {
+    uint32_t words[3][2];
+    split_pair(v.x, v.y, words[0][0], words[1][0], words[2][0]);
+    split_pair(v.z, v.w, words[0][1], words[1][1], words[2][1]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      reinterpret_cast<uint2*>(&part[step][i][lane])[half] = make_uint2(words[i][0], words[i][1]);
+  }
+  __device__ Pieces get(int step, int lane) const {
+    Pieces p;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) p.part[i] = as_bf16x8(part[step][i][lane]);
+    return p;
+  }
+};
+__device__ inline Pieces state_pieces(const floatx4& first, const floatx4& second) {
+  return split_eight(make_float4(first[0], first[1], first[2], first[3]),
+                     make_float4(second[0], second[1], second[2], second[3]));
 }
+__device__ inline float4 as_float4(const floatx4& v) { return make_float4(v[0], v[1], v[2], v[3]); }
 
 // The records of a head as the sequential kernels walk them: one descriptor for all
 // chunks, a lane offset that moves with the chunk and a uniform place in the record.
@@ -626,316 +638,385 @@ __device__ inline Record head_records(const ChunkedArgs& a, const float* records
 // that publishes it.  The fences keep that order.
 __device__ inline void keep_order() { __builtin_amdgcn_sched_barrier(0); }
 
-// S entering every chunk, Dl and O of every chunk.  Wave w computes rows 16 w .. 16 w +
-// 15 of Dl and O from the whole state and then its rows of the new state from all of
-// Dl: 112 matrix instructions a wave, chunk and tile, the 48 of O off the chain.
-// Operands are requested a chunk ahead.
+// The products of one left operand while the next one is made and its right sides are
+// read (step -1: they stay): a matrix instruction and a few vector instructions take turns.
+template <int TILES, int STEPS>
+__device__ inline void step(floatx4 (&acc)[TILES], Pieces& left, Pieces (&right)[TILES], float4 next_a, float4 next_b,
+                            const OperandLds<STEPS>* from, int next_step, int lane) {
+  keep_order();
+  Pieces read[TILES];
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) read[c] = next_step >= 0 ? from[c].get(next_step, lane) : right[c];
+  keep_order();
+  Splitter next(next_a, next_b);
+  constexpr int kLeft[6] = {2, 1, 1, 0, 0, 0}, kRight[6] = {0, 1, 0, 2, 1, 0};  // smallest products first
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) {
+      acc[c] = mfma16(left.part[kLeft[i]], right[c].part[kRight[i]], acc[c]);
+#pragma unroll
+      for (int s = 0; s < 2 / TILES; ++s)
+        if ((i * TILES + c) * (2 / TILES) + s < Splitter::kSteps) next((i * TILES + c) * (2 / TILES) + s, true);
+      keep_order();
+    }
+  }
+  left = next.pieces();
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) right[c] = read[c];
+}
+template <int TILES, int STEPS>
+__device__ inline void read_right(Pieces (&right)[TILES], const OperandLds<STEPS>* from, int step, int lane) {
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) right[c] = from[c].get(step, lane);
+}
+
+// Eight waves: the first four carry the chain, wave w rows 16 w .. + 15 of the 64-row
+// products and rows 32 w .. + 31 of the state; the others do what the chain does not wait
+// for, the same rows.  Two waves a SIMD cover each other's waits for LDS and barriers.
+// A chunk of two tiles is 2700 cycles of matrix instructions a SIMD, 5000 of vector
+// instructions and 120 KiB of operands a compute unit, which at the 20 bytes a clock that
+// one gets of a busy L2 are 6000: with 48 heads a chunk takes 9400.  Operands kept as
+// pieces (6 bytes an element instead of 4 bytes and the splitting) took 178 and 159 us
+// where these take 147 and 139, with the FP32 instruction 184 and 187 (2048 tokens, 48
+// heads).
+constexpr int kSequentialThreads = 512;
+
+// S entering every chunk, Dl and O of every chunk.  84 matrix instructions a row of waves,
+// chunk and tile, the 36 of O off the chain.  Operands are requested a chunk ahead.
 template <int TILES>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kSequentialThreads)
 chunk_states_forward_kernel(ChunkedArgs a) {
-  __shared__ __attribute__((aligned(16))) float state[TILES][kTile][kWidePad], delta[TILES][kTile][kSquarePad],
-      left_delta[TILES][kTile][kSquarePad];
+  __shared__ OperandLds<4> state[TILES];
+  __shared__ OperandLds<2> delta[TILES], left_delta[TILES];
   const Slice slice = slice_of_block<TILES>(a);
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int quarter = lane / 16, n = lane % 16;
+  const int lane = threadIdx.x % 64, quarter = lane / 16, n = lane % 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64 % 4);
+  const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x) < kSequentialThreads / 2;
   const int rows = 16 * wave + 4 * quarter;  // of the lane's part of Dl and O
-  float4 w[8], q[8], k[2][4], p[4], u[TILES], e_rows, l_rows;
-  float decay;
   const int head = slice.head, key_head = head / (a.vh / a.kh);
-  const Record w_memory = head_records(a, a.r.w_rows, head, kWide), q_memory = head_records(a, a.r.q_rows, key_head, kWide),
-               k_memory = head_records(a, a.r.k_columns, key_head, kWide),
-               p_memory = head_records(a, a.r.p_rows, head, kSquare), u_memory = head_records(a, a.r.u_columns, head, kWide),
-               dl_memory = head_records(a, a.r.dl_rows, head, kWide),
-               s0_memory = head_records(a, a.r.s0, head, kState),
-               gates = head_records(a, a.r.gates, head, kGateRows * kC);
+  const Record gates = head_records(a, a.r.gates, head, kGateRows * kC);
   // the lane's places in the records of the chunk whose operands are requested next
-  // four tokens of a column -> four columns of a token: the lane's place in rows(Dl)
+  // four rows of a column -> four columns of a row: the lane's place in rows(Dl), rows(S)
   const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;
-  const unsigned core_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
   unsigned wide_at = 16 * lane, square_at = 16 * lane, gates_at = 4 * rows;
-  const unsigned u_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
-  auto request_w = [&](int s) { w[s] = w_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
-  auto request_q = [&](int s) { q[s] = q_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
-  auto request_k = [&](int t, int s) { k[t][s] = k_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
-  auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
-  auto request_rest = [&]() {
-#pragma unroll
-    for (int c = 0; c < TILES; ++c) u[c] = u_memory.get4(wide_at, u_at + piece_at<kC>(c, 0));
-    e_rows = gates.get4(gates_at, 4 * kE * kC);
-    l_rows = gates.get4(gates_at, 4 * kL * kC);
-    decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
-  };
   const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
-  floatx4 acc[2][TILES];
+  Pieces left, right[TILES];  // the operands of the products that come next
+  if (chain) {
+    __builtin_amdgcn_s_setprio(2);
+    float4 w[8], k[2][4], u[TILES], l_rows;
+    float decay;
+    const Record w_memory = head_records(a, a.r.w_rows, head, kWide),
+                 k_memory = head_records(a, a.r.k_columns, key_head, kWide),
+                 u_memory = head_records(a, a.r.u_columns, head, kWide),
+                 dl_memory = head_records(a, a.r.dl_rows, head, kWide),
+                 s0_memory = head_records(a, a.r.s0, head, kState);
+    const unsigned u_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
+    auto request_w = [&](int s) { w[s] = w_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
+    auto request_k = [&](int t, int s) { k[t][s] = k_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+    auto request_rest = [&]() {
 #pragma unroll
-  for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
-  {
+      for (int c = 0; c < TILES; ++c) u[c] = u_memory.get4(wide_at, u_at + piece_at<kC>(c, 0));
+      l_rows = gates.get4(gates_at, 4 * kL * kC);
+      decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
+    };
+    floatx4 acc[2][TILES];
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
     // in the loop's order, so that the waits in it need not cover another one
 #pragma unroll
     for (int s = 0; s < 8; ++s) request_w(s), keep_order();
     request_rest();
     keep_order();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_q(s), keep_order();
+    for (int s = 0; s < 8; ++s) request_k(s / 2 % 2, s / 4 * 2 + s % 2), keep_order();
+    left = split_eight(w[0], w[1]);
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+      // past the end the last chunk's operands are requested again
+      const unsigned delta_now = wide_at + transposed_at, state_now = 16 * lane + transposed_at + chunk * (kState * 4);
+      const bool more = chunk + 1 < a.chunks;
+      wide_at += more ? kWide * 4 : 0, gates_at += more ? kGateRows * kC * 4 : 0;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_k(s % 2, s / 2), keep_order();
-#pragma unroll
-    for (int s = 0; s < 4; ++s) request_p(s), keep_order();
-  }
-  for (int chunk = 0; chunk < a.chunks; ++chunk) {
-    const Tokens core = ChunkView(a, chunk, head).heads(a.core);
-    // past the end the last chunk's operands are requested again
-    const unsigned delta_now = wide_at + transposed_at, state_now = 16 * lane + chunk * (kState * 4);
-    if (chunk + 1 < a.chunks)
-      wide_at += kWide * 4, square_at += kSquare * 4, gates_at += kGateRows * kC * 4;
-#pragma unroll
-    for (int c = 0; c < TILES; ++c) publish_state(acc[0][c], acc[1][c], &state[c][n][32 * wave + 4 * quarter]);
-    keep_order();
-    lds_barrier();
-    floatx4 part[2][TILES], out[TILES];
-    float4 b[TILES][8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int c = 0; c < TILES; ++c) b[c][s] = load4(&state[c][n][16 * s + 4 * quarter]);
-#pragma unroll
-    for (int c = 0; c < TILES; ++c) part[0][c] = part[1][c] = out[c] = none;
-    keep_order();  // all of them before the first is waited for
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      mma16_tiles<TILES>(part[s % 2], w[s], [&](int c) { return b[c][s]; });
+      for (int c = 0; c < TILES; ++c) state[c].put(wave, lane, state_pieces(acc[0][c], acc[1][c]));
       keep_order();
-      request_w(s);
+      lds_barrier();
+      floatx4 part[TILES];
+      read_right<TILES>(right, state, 0, lane);
+      request_w(0), request_w(1);  // split before the loop and at its end
       keep_order();
-    }
-    float4 dl[TILES];
-#pragma unroll
-    for (int c = 0; c < TILES; ++c) {
-      const floatx4 ws = part[0][c] + part[1][c];
-      dl[c] = make_float4(u[c].x - ws[0], u[c].y - ws[1], u[c].z - ws[2], u[c].w - ws[3]);
-      store4(&delta[c][n][rows], dl[c]);
-      store4(&left_delta[c][n][rows],
-             make_float4(dl[c].x * l_rows.x, dl[c].y * l_rows.y, dl[c].z * l_rows.z, dl[c].w * l_rows.w));
-      acc[0][c] *= decay;
-      acc[1][c] *= decay;
-    }
-    const float4 e_now = e_rows;
-    keep_order();
-    request_rest();
-#pragma unroll
-    for (int c = 0; c < TILES; ++c)
-      dl_memory.put4(quad_transpose(dl[c]), delta_now, piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
-    keep_order();
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      mma16_tiles<TILES>(out, q[s], [&](int c) { return b[c][s]; });
-      keep_order();
-      request_q(s);
-      if (s % 4 == 3) {
-        const int t = s / 4;  // rows(S): 16 rows a store, four columns a lane
-#pragma unroll
-        for (int c = 0; c < TILES; ++c)
-          s0_memory.put4(gather4(&state[c][4 * quarter][32 * wave + 16 * t + n], kWidePad), state_now,
-                      piece_at<kD>(2 * wave + t, (slice.col0 + kTile * c) / 4));
-      }
-      keep_order();
-    }
-    lds_barrier();
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
+      // rows(S): 16 rows a store, four columns a lane
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
-        b[c][s] = load4(&left_delta[c][n][16 * s + 4 * quarter]);
-        b[c][4 + s] = load4(&delta[c][n][16 * s + 4 * quarter]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          s0_memory.put4(quad_transpose(as_float4(acc[t][c])), state_now,
+                         piece_at<kD>(2 * wave + t, (slice.col0 + kTile * c) / 4));
+        part[c] = none;
       }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        step<TILES>(part, left, right, s < 3 ? w[2 * s + 2] : k[0][0], s < 3 ? w[2 * s + 3] : k[0][1], state,
+                    s < 3 ? s + 1 : -1, lane);
+        if (s < 3) request_w(2 * s + 2), request_w(2 * s + 3);
+      }
+      float4 dl[TILES];
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) {
+        dl[c] = make_float4(u[c].x - part[c][0], u[c].y - part[c][1], u[c].z - part[c][2], u[c].w - part[c][3]);
+        left_delta[c].put_half(wave / 2, wave % 2, lane,
+                               make_float4(dl[c].x * l_rows.x, dl[c].y * l_rows.y, dl[c].z * l_rows.z, dl[c].w * l_rows.w));
+        delta[c].put_half(wave / 2, wave % 2, lane, dl[c]);
+        acc[0][c] *= decay;
+        acc[1][c] *= decay;
+      }
+      keep_order();
+      lds_barrier();
+      read_right<TILES>(right, left_delta, 0, lane);
+      request_rest();
+      request_k(0, 0), request_k(0, 1);
+      keep_order();
+#pragma unroll
+      for (int c = 0; c < TILES; ++c)
+        dl_memory.put4(quad_transpose(dl[c]), delta_now, piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
+      // k[t][2 s], k[t][2 s + 1] in the order s, t
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = (i + 1) % 2, s = (i + 1) / 2;
+        step<TILES>(acc[i % 2], left, right, i < 3 ? k[t][2 * s] : w[0], i < 3 ? k[t][2 * s + 1] : w[1], left_delta,
+                    i == 1 ? 1 : -1, lane);
+        if (i < 3) request_k(t, 2 * s), request_k(t, 2 * s + 1);
+      }
+    }
+  } else {
+    float4 q[8], p[4], e_rows;
+    const Record q_memory = head_records(a, a.r.q_rows, key_head, kWide),
+                 p_memory = head_records(a, a.r.p_rows, head, kSquare);
+    const unsigned core_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
+    auto request_q = [&](int s) { q[s] = q_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
+    auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
+#pragma unroll
+    for (int s = 0; s < 8; ++s) request_q(s), keep_order();
+    e_rows = gates.get4(gates_at, 4 * kE * kC);
     keep_order();
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < 4; ++s) request_p(s), keep_order();
+    left = split_eight(q[0], q[1]);
+    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+      const Tokens core = ChunkView(a, chunk, head).heads(a.core);
+      const bool more = chunk + 1 < a.chunks;
+      wide_at += more ? kWide * 4 : 0, square_at += more ? kSquare * 4 : 0, gates_at += more ? kGateRows * kC * 4 : 0;
+      lds_barrier();
+      floatx4 out[TILES];
+      read_right<TILES>(right, state, 0, lane);
+      request_q(0), request_q(1);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        mma16_tiles<TILES>(acc[t], k[t][s], [&](int c) { return b[c][s]; });
-        keep_order();
-        request_k(t, s);
-        keep_order();
+      for (int c = 0; c < TILES; ++c) out[c] = none;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        step<TILES>(out, left, right, s < 3 ? q[2 * s + 2] : p[0], s < 3 ? q[2 * s + 3] : p[1], state,
+                    s < 3 ? s + 1 : -1, lane);
+        if (s < 3) request_q(2 * s + 2), request_q(2 * s + 3);
       }
-    }
 #pragma unroll
-    for (int c = 0; c < TILES; ++c)
-      out[c][0] *= e_now.x, out[c][1] *= e_now.y, out[c][2] *= e_now.z, out[c][3] *= e_now.w;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      mma16_tiles<TILES>(out, p[s], [&](int c) { return b[c][4 + s]; });
+      for (int c = 0; c < TILES; ++c)
+        out[c][0] *= e_rows.x, out[c][1] *= e_rows.y, out[c][2] *= e_rows.z, out[c][3] *= e_rows.w;
       keep_order();
-      request_p(s);
-      keep_order();
-    }
+      e_rows = gates.get4(gates_at, 4 * kE * kC);
+      request_p(0), request_p(1);
+      lds_barrier();
+      read_right<TILES>(right, delta, 0, lane);
+      step<TILES>(out, left, right, p[2], p[3], delta, 1, lane);
+      request_p(2), request_p(3);
+      step<TILES>(out, left, right, q[0], q[1], delta, -1, lane);
 #pragma unroll
-    for (int c = 0; c < TILES; ++c) {
-      // four tokens of a column -> four columns of a token
-      const float4 o =
-          quad_transpose(make_float4(round_if(out[c][0], a.round), round_if(out[c][1], a.round),
-                                     round_if(out[c][2], a.round), round_if(out[c][3], a.round)));
-      core.put4(o, core_at, 4 * kTile * c);
+      for (int c = 0; c < TILES; ++c) {
+        // four tokens of a column -> four columns of a token
+        const float4 o =
+            quad_transpose(make_float4(round_if(out[c][0], a.round), round_if(out[c][1], a.round),
+                                       round_if(out[c][2], a.round), round_if(out[c][3], a.round)));
+        core.put4(o, core_at, 4 * kTile * c);
+      }
     }
   }
 }
 
 // The gradient of the state leaving every chunk and dDl of every chunk, chunks in
-// reverse.  112 matrix instructions a wave, chunk and tile, those with dO off the chain
-// (Q^ dO fills the wait for the other waves' dDl).
+// reverse.  84 matrix instructions a row of waves, chunk and tile, the 36 with dO off the
+// chain: the other waves leave P^T dO and (diag(E) Q^)^T dO of the next chunk in LDS.
 template <int TILES>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kSequentialThreads)
 chunk_states_backward_kernel(ChunkedArgs a) {
-  __shared__ __attribute__((aligned(16))) float state[TILES][kTile][kWidePad], delta[TILES][kTile][kSquarePad],
-      grad[TILES][kTile][kSquarePad], query_grad[TILES][kTile][kSquarePad];
+  __shared__ OperandLds<4> state[TILES];
+  __shared__ OperandLds<2> delta[TILES], grad[TILES], query_grad[TILES];
+  // [P^T dO, two row tiles of Q^T dO]: a wave's accumulators
+  __shared__ floatx4 handed[2][3][TILES][4][64];
   const Slice slice = slice_of_block<TILES>(a);
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int quarter = lane / 16, n = lane % 16;
+  const int lane = threadIdx.x % 64, quarter = lane / 16, n = lane % 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64 % 4);
+  const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x) < kSequentialThreads / 2;
   const int rows = 16 * wave + 4 * quarter;
-  float4 k[8], p[4], q[2][4], w[2][4], out[TILES], k_scale, q_scale;
-  float decay;
   const int head = slice.head, key_head = head / (a.vh / a.kh);
-  const Record k_memory = head_records(a, a.r.k_rows, key_head, kWide),
-               p_memory = head_records(a, a.r.p_columns, head, kSquare),
-               q_memory = head_records(a, a.r.q_columns, key_head, kWide),
-               w_memory = head_records(a, a.r.w_columns, head, kWide),
-               ddl_memory = head_records(a, a.r.ddl_columns, head, kWide),
-               ddl_rows = head_records(a, a.r.ddl_rows, head, kWide), ds1_memory = head_records(a, a.r.ds1, head, kState),
-               gates = head_records(a, a.r.gates, head, kGateRows * kC);
+  const Record gates = head_records(a, a.r.gates, head, kGateRows * kC);
   const unsigned last = a.chunks - 1;
   unsigned wide_at = 16 * lane + last * (kWide * 4), square_at = 16 * lane + last * (kSquare * 4),
            gates_at = 4 * rows + last * (kGateRows * kC * 4);
-  const unsigned delta_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
-  const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;  // as above
-  const unsigned out_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
-  auto request_out = [&](int chunk) {
-    const Tokens d_out = ChunkView(a, max(chunk, 0), head).heads(a.dcore);
-#pragma unroll
-    for (int c = 0; c < TILES; ++c) out[c] = d_out.get4(out_at, 4 * kTile * c);
-    q_scale = gates.get4(gates_at, 4 * kE * kC);
-    k_scale = gates.get4(gates_at, 4 * kL * kC);
-    decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
-  };
-  auto request_k = [&](int s) { k[s] = k_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
-  auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
-  auto request_q = [&](int t, int s) { q[t][s] = q_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
-  auto request_w = [&](int t, int s) { w[t][s] = w_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
   const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
-  floatx4 acc[2][TILES];
+  Pieces left, right[TILES];  // the operands of the products that come next
+  if (chain) {
+    __builtin_amdgcn_s_setprio(2);
+    float4 k[8], w[2][4], k_scale;
+    float decay;
+    const Record k_memory = head_records(a, a.r.k_rows, key_head, kWide),
+                 w_memory = head_records(a, a.r.w_columns, head, kWide),
+                 ddl_memory = head_records(a, a.r.ddl_columns, head, kWide),
+                 ddl_rows = head_records(a, a.r.ddl_rows, head, kWide), ds1_memory = head_records(a, a.r.ds1, head, kState);
+    const unsigned delta_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
+    const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;  // as above
+    auto request_k = [&](int s) { k[s] = k_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
+    auto request_w = [&](int t, int s) { w[t][s] = w_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+    auto request_gates = [&]() {
+      k_scale = gates.get4(gates_at, 4 * kL * kC);
+      decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
+    };
+    floatx4 acc[2][TILES];
 #pragma unroll
-  for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
-  {
+    for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
     // in the loop's order, so that the waits in it need not cover another one
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      request_k(2 * s), keep_order();
-      request_k(2 * s + 1), keep_order();
-      request_p(s), keep_order();
+    for (int s = 0; s < 8; ++s) request_k(s), keep_order();
+    request_gates();
+    keep_order();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) request_w(s / 2 % 2, s / 4 * 2 + s % 2), keep_order();
+    left = split_eight(k[0], k[1]);
+    lds_barrier();  // the first chunk's dO is in LDS,
+    lds_barrier();  // and what the other waves hand over
+    for (int chunk = a.chunks - 1; chunk >= 0; --chunk) {
+      // before the first the first chunk's operands are requested again
+      const unsigned wide_now = wide_at, state_now = 16 * lane + transposed_at + chunk * (kState * 4);
+      const bool more = chunk > 0;
+      wide_at -= more ? kWide * 4 : 0, gates_at -= more ? kGateRows * kC * 4 : 0;
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) state[c].put(wave, lane, state_pieces(acc[0][c], acc[1][c]));
+      keep_order();
+      lds_barrier();
+      floatx4 part[TILES];
+      read_right<TILES>(right, state, 0, lane);
+      request_k(0), request_k(1);
+      keep_order();
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          ds1_memory.put4(quad_transpose(as_float4(acc[t][c])), state_now,
+                          piece_at<kD>(2 * wave + t, (slice.col0 + kTile * c) / 4));
+        part[c] = none;
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        step<TILES>(part, left, right, s < 3 ? k[2 * s + 2] : w[0][0], s < 3 ? k[2 * s + 3] : w[0][1], state,
+                    s < 3 ? s + 1 : -1, lane);
+        if (s < 3) request_k(2 * s + 2), request_k(2 * s + 3);
+      }
+      float4 dd[TILES];
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) {
+        const floatx4 from_out = handed[chunk % 2][0][c][wave][lane];
+        dd[c] = make_float4(from_out[0] + k_scale.x * part[c][0], from_out[1] + k_scale.y * part[c][1],
+                            from_out[2] + k_scale.z * part[c][2], from_out[3] + k_scale.w * part[c][3]);
+        delta[c].put_half(wave / 2, wave % 2, lane, scaled(dd[c], -1.0f));
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int c = 0; c < TILES; ++c) {
+          const floatx4 queries = handed[chunk % 2][1 + t][c][wave][lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[t][c][e] = fmaf(acc[t][c][e], decay, queries[e]);
+        }
+      keep_order();
+      lds_barrier();
+      read_right<TILES>(right, delta, 0, lane);
+      request_gates();
+      request_w(0, 0), request_w(0, 1);
+      keep_order();
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) {
+        ddl_memory.put4(dd[c], wide_now, delta_at + piece_at<kC>(c, 0));
+        ddl_rows.put4(quad_transpose(dd[c]), wide_now + transposed_at,
+                      piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
+      }
+      // w[t][2 s], w[t][2 s + 1] in the order s, t
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = (i + 1) % 2, s = (i + 1) / 2;
+        step<TILES>(acc[i % 2], left, right, i < 3 ? w[t][2 * s] : k[0], i < 3 ? w[t][2 * s + 1] : k[1], delta,
+                    i == 1 ? 1 : -1, lane);
+        if (i < 3) request_w(t, 2 * s), request_w(t, 2 * s + 1);
+      }
     }
+  } else {
+    float4 p[4], q[2][4], out[TILES], q_scale;
+    const Record p_memory = head_records(a, a.r.p_columns, head, kSquare),
+                 q_memory = head_records(a, a.r.q_columns, key_head, kWide);
+    const unsigned out_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
+    auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
+    auto request_q = [&](int t, int s) { q[t][s] = q_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+    auto request_out = [&](int chunk) {
+      const Tokens d_out = ChunkView(a, max(chunk, 0), head).heads(a.dcore);
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) out[c] = d_out.get4(out_at, 4 * kTile * c);
+      q_scale = gates.get4(gates_at, 4 * kE * kC);
+    };
     request_out(last);
     keep_order();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_q(s % 2, s / 2), keep_order();
+    for (int s = 0; s < 4; ++s) request_p(s), keep_order();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_w(s % 2, s / 2), keep_order();
-  }
-  for (int chunk = a.chunks - 1; chunk >= 0; --chunk) {
-    // before the first the first chunk's operands are requested again
-    const unsigned wide_now = wide_at, state_now = 16 * lane + chunk * (kState * 4);
-    if (chunk > 0) wide_at -= kWide * 4, square_at -= kSquare * 4, gates_at -= kGateRows * kC * 4;
+    for (int s = 0; s < 8; ++s) request_q(s / 2 % 2, s / 4 * 2 + s % 2), keep_order();
+    left = split_eight(p[0], p[1]);
+    // a chunk ahead of the chain: what is handed over lies in LDS before the chain's
+    // chunk begins
+    for (int chunk = a.chunks - 1; chunk >= -1; --chunk) {
+      const bool more = chunk > 0;
+      wide_at -= more ? kWide * 4 : 0, square_at -= more ? kSquare * 4 : 0, gates_at -= more ? kGateRows * kC * 4 : 0;
 #pragma unroll
-    for (int c = 0; c < TILES; ++c) {
-      publish_state(acc[0][c], acc[1][c], &state[c][n][32 * wave + 4 * quarter]);
-      const float4 o = quad_transpose(out[c]);  // four columns of a token -> four tokens of a column
-      store4(&grad[c][n][rows], o);
-      store4(&query_grad[c][n][rows],
-             make_float4(o.x * q_scale.x, o.y * q_scale.y, o.z * q_scale.z, o.w * q_scale.w));
-    }
-    const float4 scale = k_scale;
-    const float decay_now = decay;
-    keep_order();
-    lds_barrier();
-    floatx4 from_out[TILES], part[2][TILES];
-    float4 b[TILES][8], g[TILES][4];
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int c = 0; c < TILES; ++c) b[c][s] = load4(&state[c][n][16 * s + 4 * quarter]);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int c = 0; c < TILES; ++c) g[c][s] = load4(&grad[c][n][16 * s + 4 * quarter]);
-#pragma unroll
-    for (int c = 0; c < TILES; ++c) part[0][c] = part[1][c] = from_out[c] = none;
-    keep_order();
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        mma16_tiles<TILES>(part[half], k[2 * s + half], [&](int c) { return b[c][2 * s + half]; });
-        keep_order();
-        request_k(2 * s + half);
-        keep_order();
+      for (int c = 0; c < TILES; ++c) {
+        const float4 o = quad_transpose(out[c]);  // four columns of a token -> four tokens of a column
+        grad[c].put_half(wave / 2, wave % 2, lane, o);
+        query_grad[c].put_half(wave / 2, wave % 2, lane,
+                               make_float4(o.x * q_scale.x, o.y * q_scale.y, o.z * q_scale.z, o.w * q_scale.w));
       }
-      mma16_tiles<TILES>(from_out, p[s], [&](int c) { return g[c][s]; });
       keep_order();
-      request_p(s);
-      keep_order();
-    }
-    float4 dd[TILES];
+      lds_barrier();
+      if (chunk >= 0) {
+        floatx4 from_out[TILES], queries[2][TILES];
+        read_right<TILES>(right, grad, 0, lane);
+        request_out(chunk - 1);
+        request_p(0), request_p(1);
 #pragma unroll
-    for (int c = 0; c < TILES; ++c) {
-      const floatx4 ks = part[0][c] + part[1][c];
-      dd[c] = make_float4(from_out[c][0] + scale.x * ks[0], from_out[c][1] + scale.y * ks[1],
-                          from_out[c][2] + scale.z * ks[2], from_out[c][3] + scale.w * ks[3]);
-      store4(&delta[c][n][rows], scaled(dd[c], -1.0f));
-      acc[0][c] *= decay_now;
-      acc[1][c] *= decay_now;
-    }
+        for (int c = 0; c < TILES; ++c) from_out[c] = queries[0][c] = queries[1][c] = none;
+        step<TILES>(from_out, left, right, p[2], p[3], grad, 1, lane);
+        request_p(2), request_p(3);
+        step<TILES>(from_out, left, right, q[0][0], q[0][1], query_grad, 0, lane);
+        request_q(0, 0), request_q(0, 1);
+        // q[t][2 s], q[t][2 s + 1] in the order s, t
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int c = 0; c < TILES; ++c) g[c][s] = load4(&query_grad[c][n][16 * s + 4 * quarter]);
-    keep_order();
-    request_out(chunk - 1);
-#pragma unroll
-    for (int c = 0; c < TILES; ++c) {
-      ddl_memory.put4(dd[c], wide_now, delta_at + piece_at<kC>(c, 0));
-      ddl_rows.put4(quad_transpose(dd[c]), wide_now + transposed_at,
-                    piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
-    }
-    keep_order();
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        mma16_tiles<TILES>(acc[t], q[t][s], [&](int c) { return g[c][s]; });
-        keep_order();
-        request_q(t, s);
-        if (s % 2 == 1 && t == 1) {
-#pragma unroll
-          for (int c = 0; c < TILES; ++c)
-            ds1_memory.put4(gather4(&state[c][4 * quarter][32 * wave + 16 * (s / 2) + n], kWidePad), state_now,
-                         piece_at<kD>(2 * wave + s / 2, (slice.col0 + kTile * c) / 4));
+        for (int i = 0; i < 4; ++i) {
+          const int t = (i + 1) % 2, s = (i + 1) / 2;
+          step<TILES>(queries[i % 2], left, right, i < 3 ? q[t][2 * s] : p[0], i < 3 ? q[t][2 * s + 1] : p[1],
+                      query_grad, i == 1 ? 1 : -1, lane);
+          if (i < 3) request_q(t, 2 * s), request_q(t, 2 * s + 1);
         }
-        keep_order();
+#pragma unroll
+        for (int c = 0; c < TILES; ++c) {
+          handed[chunk & 1][0][c][wave][lane] = from_out[c];
+          handed[chunk & 1][1][c][wave][lane] = queries[0][c];
+          handed[chunk & 1][2][c][wave][lane] = queries[1][c];
+        }
       }
-    }
-    lds_barrier();
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int c = 0; c < TILES; ++c) g[c][s] = load4(&delta[c][n][16 * s + 4 * quarter]);
-    keep_order();
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        mma16_tiles<TILES>(acc[t], w[t][s], [&](int c) { return g[c][s]; });
-        keep_order();
-        request_w(t, s);
-        keep_order();
-      }
+      keep_order();
+      lds_barrier();
     }
   }
 }
@@ -1406,18 +1487,18 @@ int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBack
   const int status = launch_status();
   if (status != 0) return status;
   if (column_tiles(a.vh) == 2)
-    chunk_states_forward_kernel<2><<<a.vh * (kD / (2 * kTile)), 256, 0, stream>>>(a);
+    chunk_states_forward_kernel<2><<<a.vh * (kD / (2 * kTile)), kSequentialThreads, 0, stream>>>(a);
   else
-    chunk_states_forward_kernel<1><<<a.vh * (kD / kTile), 256, 0, stream>>>(a);
+    chunk_states_forward_kernel<1><<<a.vh * (kD / kTile), kSequentialThreads, 0, stream>>>(a);
   return launch_status();
 }
 
 int launch_gdn_backward_chunked_reverse(hipStream_t stream, const GdnChunkedBackward& c) {
   const ChunkedArgs a = make_args(c);
   if (column_tiles(a.vh) == 2)
-    chunk_states_backward_kernel<2><<<a.vh * (kD / (2 * kTile)), 256, 0, stream>>>(a);
+    chunk_states_backward_kernel<2><<<a.vh * (kD / (2 * kTile)), kSequentialThreads, 0, stream>>>(a);
   else
-    chunk_states_backward_kernel<1><<<a.vh * (kD / kTile), 256, 0, stream>>>(a);
+    chunk_states_backward_kernel<1><<<a.vh * (kD / kTile), kSequentialThreads, 0, stream>>>(a);
   const int status = launch_status();
   if (status != 0) return status;
   chunk_gradients_kernel<<<dim3(a.chunks, a.vh), 256, 0, stream>>>(a);

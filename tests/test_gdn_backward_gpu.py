@@ -172,6 +172,16 @@ def test_long_sequence_two_heads_matches_oracle(capi):
         assert_close(got[name], want[name], 2e-4, "%s %s" % (name, shape))
 
 
+@pytest.mark.parametrize("length,key_heads", [(1, 33), (64, 11), (65, 3), (130, 33)])
+def test_two_column_tiles_a_workgroup_match_the_oracle(capi, length, key_heads):
+    """More heads than the compute units take one column tile of each: 33 of them, no
+    multiple of the XCDs, for one chunk, a full one, one token more and three."""
+    shape = (length, key_heads, 33, 128, 128, 4)
+    got, want, _, _ = run(capi, shape, False, seed=length)
+    for name in want:
+        assert_close(got[name], want[name], 2e-4, "%s %s" % (name, shape))
+
+
 def test_benchmarked_shape_against_token_by_token_kernels(capi):
     """The shape bench.py times (T=2048, sixteen 128 x 128 heads, every parameter
     trains): the chunked kernels against the token-by-token kernels of the same
