@@ -33,6 +33,18 @@ struct SplitArgs {
   float* dv = nullptr;
 };
 
+// Rows of one head that a workgroup of 256 threads takes of the gates' backward, `d / 8` lanes
+// a row: 64 where that still makes several workgroups a compute unit, fewer for shorter
+// sequences, down to what the workgroup holds at once. 24 heads, 64 rows and so: 64 tokens
+// 8.1 and 4.1 us at width 128, 11.0 and 4.3 at 256; 300 tokens 9.0 and 5.5, 12.5 and 9.2;
+// 1024 tokens 11.0 and 9.0, 30 and 25; 3000 tokens 26.3 and 25.7, 69 and 67.
+inline int gate_group_rows(int length, int heads, int d) {
+  const int least = 2048 / d;
+  int rows = 64;
+  while (rows > least && 1LL * (length + rows - 1) / rows * heads < 2048) rows /= 2;
+  return rows;
+}
+
 bool split_attention_supported(int length, int heads, int head_dim);
 int launch_split_forward(hipStream_t stream, const SplitArgs& args);
 // dC = dy * Round(sigmoid(gate)) into args.d_core and args.deltas;

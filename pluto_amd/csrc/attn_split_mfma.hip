@@ -338,15 +338,15 @@ split_forward_kernel(SplitArgs a) {
     finish(std::integral_constant<int, kHalfBlocks>());
 }
 
-// 32 lanes a row, eight channels a lane; a workgroup walks 64 rows of one head.
+// 32 lanes a row, eight channels a lane; a workgroup walks `rows` rows of one head.
 // WIDE: the caller's tensors are 16-byte aligned.
 template <bool WIDE>
 __global__ void __launch_bounds__(256)
 split_gate_kernel(SplitArgs a, const uint16_t* __restrict__ qg, const float* __restrict__ dy,
-                  float* __restrict__ dqg) {
+                  float* __restrict__ dqg, int rows) {
   const int c = 8 * (threadIdx.x % 32), head = blockIdx.y;
-  for (int i = 0; i < 64; i += 8) {
-    const int row = blockIdx.x * 64 + i + threadIdx.x / 32;
+  for (int i = 0; i < rows; i += 8) {
+    const int row = blockIdx.x * rows + i + threadIdx.x / 32;
     if (row >= a.length) continue;  // a row's lanes leave together
     const long long unit = 1LL * row * a.heads + head;
     float gate[8], core[8], grad[8], d_gate[8];
@@ -686,13 +686,14 @@ int launch_split_forward(hipStream_t stream, const SplitArgs& a) {
 
 int launch_split_gate(hipStream_t stream, const SplitArgs& a, const void* qg, const float* dy,
                       float* dqg) {
-  const dim3 grid((a.length + 63) / 64, a.heads);
+  const int rows = gate_group_rows(a.length, a.heads, D);
+  const dim3 grid((a.length + rows - 1) / rows, a.heads);
   const auto* gates = static_cast<const uint16_t*>(qg);
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   if (aligned(qg) && aligned(dy) && aligned(dqg))
-    split_gate_kernel<true><<<grid, 256, 0, stream>>>(a, gates, dy, dqg);
+    split_gate_kernel<true><<<grid, 256, 0, stream>>>(a, gates, dy, dqg, rows);
   else
-    split_gate_kernel<false><<<grid, 256, 0, stream>>>(a, gates, dy, dqg);
+    split_gate_kernel<false><<<grid, 256, 0, stream>>>(a, gates, dy, dqg, rows);
   return launch_status();
 }
 

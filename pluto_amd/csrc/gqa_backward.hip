@@ -14,6 +14,7 @@
 //                                            with the per-kv-head sums and the first
 //                                            level of ReduceNormKernel (:230-239)
 //   norm_weight_kernel                       its second level, fixed order
+#include "attn_split_mfma.h"
 #include "gqa.h"
 #include "mfma_tile.h"
 
@@ -66,7 +67,7 @@ gate_backward_kernel(const uint16_t* qg, const float* core, const float* dy, lon
 // The same for the matrix-core kernels, which take dC as bf16 together with two
 // values of each row: -sum(dC * core) and the row's log2-sum-exp in the form
 // FlashBackwardArgs states.  Sixteen bytes of bf16 a lane, D / 8 lanes a row; a
-// workgroup walks 64 rows of one head, whose statistics are then contiguous.
+// workgroup walks `rows` rows of one head, whose statistics are then contiguous.
 // 350 MB in and out at T = 8192, 24 heads of 128; written as an FP32 dC that
 // the query-owned kernel read again in pieces of its own rows, the same work moved
 // 550 MB (83 us for this pass alone).  WIDE: every tensor is 16-byte aligned.
@@ -74,13 +75,13 @@ template <int D, bool WIDE>
 __global__ void __launch_bounds__(256)
 gate_rows_kernel(const uint16_t* __restrict__ qg, const uint16_t* __restrict__ core,
                  const float* __restrict__ dy, const float* __restrict__ maxima,
-                 const float* __restrict__ normalizers, int length, int heads, float scale2,
+                 const float* __restrict__ normalizers, int length, int rows, int heads, float scale2,
                  uint16_t* __restrict__ dc, float* __restrict__ dqg, float* __restrict__ deltas,
                  float* __restrict__ lse2) {
   constexpr int LANES = D / 8, ROWS = 256 / LANES;
   const int piece = threadIdx.x % LANES, head = blockIdx.y;
-  for (int i = 0; i < 64; i += ROWS) {
-    const int row = blockIdx.x * 64 + i + threadIdx.x / LANES;
+  for (int i = 0; i < rows; i += ROWS) {
+    const int row = blockIdx.x * rows + i + threadIdx.x / LANES;
     const bool exists = row < length;
     const long long unit = 1LL * min(row, length - 1) * heads + head;
     float grad[8], gates[8], values[8];
@@ -374,15 +375,16 @@ int launch_gate_backward(hipStream_t stream, const void* qg, const float* core, 
 int launch_gate_rows(hipStream_t stream, const void* qg, const void* core, const float* dy,
                      const float* maxima, const float* normalizers, int length, int qh, int d,
                      float scale2, uint16_t* dc, float* dqg, float* deltas, float* lse2) {
-  const dim3 grid((length + 63) / 64, qh);
+  const int rows = gate_group_rows(length, qh, d);
+  const dim3 grid((length + rows - 1) / rows, qh);
   const auto* gates = static_cast<const uint16_t*>(qg);
   const auto* values = static_cast<const uint16_t*>(core);
   bool wide = true;
   for (const void* p : {qg, core, static_cast<const void*>(dy), static_cast<const void*>(dqg)})
     wide = wide && (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
   auto launch = [&](auto kernel) {
-    kernel<<<grid, 256, 0, stream>>>(gates, values, dy, maxima, normalizers, length, qh, scale2, dc,
-                                     dqg, deltas, lse2);
+    kernel<<<grid, 256, 0, stream>>>(gates, values, dy, maxima, normalizers, length, rows, qh, scale2,
+                                     dc, dqg, deltas, lse2);
   };
   if (d == 64)
     launch(wide ? gate_rows_kernel<64, true> : gate_rows_kernel<64, false>);
