@@ -376,3 +376,26 @@ def test_tensors_off_sixteen_bytes(capi, T, qh, kh, d, rot, with_saved):
     for name, a, b in zip(names, want, once(1, 1, 1)):
         # a bf16 ulp (2^-8) in one element of a thousand: 2^-8 sqrt(1e-3) of the norm
         assert (a - b).norm() <= 2.0 ** -8 * 1e-3 ** 0.5 * a.norm(), name
+
+
+@pytest.mark.parametrize("T,d", [(1, 128), (9, 256), (1001, 256), (1100, 64), (2750, 128), (5501, 64)])
+def test_gate_gradients_of_every_row(capi, T, d):
+    """24 heads of lengths whose gate gradients go 8 to 64 rows a workgroup, the last one
+    not full.  The gradient is dy core s (1 - s) and the forward's output the product of
+    the rounded core and the rounded s, rounded: apart by two roundings to eight bits."""
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    normal = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    qh, kh = 24, 4
+    p = capi.attention_params(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=d // 4, capacity=T,
+                              round_to_bfloat16=True)
+    qg = normal(T, qh, 2, d).to(torch.bfloat16)
+    k, v = normal(T, kh, d).to(torch.bfloat16), normal(T, kh, d).to(torch.bfloat16)
+    qw, kw_, dy = 0.1 * normal(d), 0.1 * normal(d), normal(T, qh, d)
+    cache = capi.KvCache(T, kh, d)
+    saved = capi.gqa_prefill_saved(p, T, cache)
+    out = capi.gqa_prefill(p, qg, k, v, qw, kw_, cache, saved=saved)
+    dqg = capi.gqa_prefill_backward(p, qg, k, v, qw, kw_, dy, saved=saved)[0]
+    torch.cuda.synchronize()
+    want = dy.double() * out.double() * (1 - torch.sigmoid(qg[:, :, 1].double()))
+    error = (dqg[:, :, 1].double() - want).abs()
+    assert (error <= 2.0 ** -6.9 * want.abs() + 1e-6).all(), error.max().item()
