@@ -30,6 +30,8 @@
 // 8 x batch x heads way parallelism.
 #include "gdn.h"
 
+#include <type_traits>
+
 namespace pluto_hip {
 namespace {
 
@@ -77,6 +79,29 @@ __device__ inline void split_operand(const floatx4& first, const floatx4& second
   }
 }
 
+// Sum of the squares of eight bf16 numbers, and of sixteen neighbouring lanes' values.
+__device__ inline float squares(const uint4& v) {
+  const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+  float even = 0.0f, odd = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float low = __uint_as_float(words[i] << 16), high = __uint_as_float(words[i] & 0xffff0000u);
+    even += low * low;
+    odd += high * high;
+  }
+  return even + odd;
+}
+__device__ inline float row_sum(float v) {
+  auto step = [&](auto control) {
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(control)::value, 0xf, 0xf, true));
+  };
+  step(std::integral_constant<int, 0xB1>());   // quad_perm 1, 0, 3, 2
+  step(std::integral_constant<int, 0x4E>());   // quad_perm 2, 3, 0, 1
+  step(std::integral_constant<int, 0x141>());  // row_half_mirror
+  step(std::integral_constant<int, 0x140>());  // row_mirror
+  return v;
+}
+
 // 35 KiB, so that four workgroups share a compute unit's LDS (the kernel is a
 // chain of short, barrier-separated phases and lives on occupancy): once the
 // Gram matrices are done the rows of K make room for A, and A in turn for the
@@ -110,16 +135,34 @@ gdn_chunk_prepare(GdnArgs a) {
   const int valid = min(C, a.length - t0);
 
   // ---- stage K and Q rows (16-byte pieces), zero beyond the sequence --------
-  for (int piece = tid; piece < C * (DK / 8); piece += 256) {
-    const int row = piece / (DK / 8), c8 = piece % (DK / 8);
-    uint4 kb = make_uint4(0, 0, 0, 0), qb = kb;
-    if (row < valid) {
-      const long long token = static_cast<long long>(seq) * a.length + t0 + row;
-      kb = *reinterpret_cast<const uint4*>(a.k + token * a.k_token_stride + key_head * DK + 8 * c8);
-      qb = *reinterpret_cast<const uint4*>(a.q + token * a.q_token_stride + key_head * DK + 8 * c8);
+  // Sixteen lanes hold a row and add up its squares as it arrives (read back from LDS
+  // one channel at a time, four lanes a row: 83 us at 8191 tokens of 48 heads, 78 so).
+  {
+    constexpr int kLoads = C * (DK / 8) / 256;
+    const int c8 = tid % (DK / 8);
+    uint4 kb[kLoads], qb[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int row = i * (256 / (DK / 8)) + tid / (DK / 8);
+      kb[i] = qb[i] = make_uint4(0, 0, 0, 0);
+      if (row < valid) {
+        const long long token = static_cast<long long>(seq) * a.length + t0 + row;
+        kb[i] = *reinterpret_cast<const uint4*>(a.k + token * a.k_token_stride + key_head * DK + 8 * c8);
+        qb[i] = *reinterpret_cast<const uint4*>(a.q + token * a.q_token_stride + key_head * DK + 8 * c8);
+      }
     }
-    *reinterpret_cast<uint4*>(&sm.k[row][8 * c8]) = kb;
-    *reinterpret_cast<uint4*>(&sm.q[row][8 * c8]) = qb;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int row = i * (256 / (DK / 8)) + tid / (DK / 8);
+      *reinterpret_cast<uint4*>(&sm.k[row][8 * c8]) = kb[i];
+      *reinterpret_cast<uint4*>(&sm.q[row][8 * c8]) = qb[i];
+      const float kk = row_sum(squares(kb[i])), qq = row_sum(squares(qb[i]));
+      if (c8 == 0) {
+        // sequence_delta_net.cc:84-85: x * rsqrt(sum(x^2) + 1e-6)
+        sm.inv_k[row] = a.normalize_qk ? rsqrtf(kk + 1e-6f) : 1.0f;
+        sm.q_factor[row] = a.normalize_qk ? a.q_scale * rsqrtf(qq + 1e-6f) : a.q_scale;
+      }
+    }
   }
   if (wave == 0) {
     float g = 0.0f, b = 0.0f;
@@ -135,27 +178,6 @@ gdn_chunk_prepare(GdnArgs a) {
     }
     sm.cum[lane] = g;
     sm.beta[lane] = b;
-  }
-  __syncthreads();
-  {
-    // row norms: 4 threads per row, 32 channels each
-    const int row = tid / 4, part = tid % 4;
-    float kk = 0.0f, qq = 0.0f;
-    for (int c = 32 * part; c < 32 * part + 32; ++c) {
-      const float kv = bf16_bits_to_float(sm.k[row][c]);
-      const float qv = bf16_bits_to_float(sm.q[row][c]);
-      kk += kv * kv;
-      qq += qv * qv;
-    }
-    kk += __shfl_xor(kk, 1, 64);
-    kk += __shfl_xor(kk, 2, 64);
-    qq += __shfl_xor(qq, 1, 64);
-    qq += __shfl_xor(qq, 2, 64);
-    if (part == 0) {
-      // sequence_delta_net.cc:84-85: x * rsqrt(sum(x^2) + 1e-6)
-      sm.inv_k[row] = a.normalize_qk ? rsqrtf(kk + 1e-6f) : 1.0f;
-      sm.q_factor[row] = a.normalize_qk ? a.q_scale * rsqrtf(qq + 1e-6f) : a.q_scale;
-    }
   }
   __syncthreads();
 
@@ -186,12 +208,24 @@ gdn_chunk_prepare(GdnArgs a) {
       }
       const int col = 32 * tj + n;  // token j
       const float cum_j = sm.cum[col], inv_kj = sm.inv_k[col];
+      // four rows a register quad; values are chosen, not branched around: a branch with
+      // a read of LDS in it for each of 32 elements took 7400 of the kernel's 21000 cycles
+      // (78 us; 70 so)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int row = 32 * ti + 8 * (i / 4) + 4 * h + (i % 4);  // token i
-        const float decay = __expf(fminf(sm.cum[row] - cum_j, 0.0f));
-        if (col < row) av[i] = sm.beta[row] * decay * sm.inv_k[row] * inv_kj * gk[i];
-        if (col <= row) a2v[i] = decay * sm.q_factor[row] * inv_kj * gq[i];
+      for (int j = 0; j < 4; ++j) {
+        const int row0 = 32 * ti + 8 * j + 4 * h;  // token i
+        const floatx4 cum = *reinterpret_cast<const floatx4*>(&sm.cum[row0]),
+                      beta = *reinterpret_cast<const floatx4*>(&sm.beta[row0]),
+                      inv_k = *reinterpret_cast<const floatx4*>(&sm.inv_k[row0]),
+                      q_factor = *reinterpret_cast<const floatx4*>(&sm.q_factor[row0]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float decay = __expf(fminf(cum[e] - cum_j, 0.0f));
+          float k = beta[e] * decay * inv_k[e] * inv_kj * gk[4 * j + e], q = decay * q_factor[e] * inv_kj * gq[4 * j + e];
+          asm("" : "+v"(k), "+v"(q));
+          av[4 * j + e] = col < row0 + e ? k : 0.0f;
+          a2v[4 * j + e] = col <= row0 + e ? q : 0.0f;
+        }
       }
     }
     __syncthreads();  // nobody reads the rows of K and Q any more
