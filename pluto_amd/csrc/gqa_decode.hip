@@ -15,7 +15,11 @@
 //           workgroup that owns a sequence's last block also prepares the new
 //           K row and the V row, appends them to the cache and keeps a copy
 //           in LDS: it is the only one that needs them, and takes them from
-//           there.
+//           there.  A sequence alone is a chain of waits (777 rows at width
+//           256: 48000 cycles, of which this step took 11300 and the
+//           combination 13800): a wave's vectors are requested before any cache
+//           row and normalised side by side, and what the combination needs
+//           is requested together: 7000 and 10600 cycles, 20.4 -> 18.2 us.
 //   scores  S^T[token, head] = K[token, :] . q[head, :] with
 //           v_mfma_f32_16x16x32_bf16: the A operand (16 tokens x 32 channels) is
 //           loaded straight from global memory, 16 bytes per lane, the four
@@ -89,63 +93,90 @@ __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// One wave prepares one head vector (RMSNorm with (1 + w), split-half partial
-// RoPE, bf16 rounding points as in normalize_rotate) with a single round trip
-// to memory: every lane loads its D/64 channels and weights at once, the RoPE
-// partner comes from the LDS row the result is left in.  `row` receives the
-// bf16 bits; `cosine`/`sine` hold this lane's rounded table entries per slot.
+// A head vector on its way: the D / 64 elements of a lane as they lie in memory, and the
+// norm's weights.  Requested before anything else, looked at when the cache rows travel.
 template <int D>
-__device__ inline void prepare_head(const void* base, long long offset, int dtype,
-                                    const float* weight, int rotary_dim, float epsilon,
-                                    const float (&cosine)[D / 64], const float (&sine)[D / 64],
-                                    uint16_t* row) {
+struct HeadVector {
+  static constexpr int SLOTS = D / 64;
+  uint32_t bits[SLOTS];
+  float weight[SLOTS];
+  __device__ void request(const void* base, long long offset, int dtype, const float* weights) {
+    const int lane = threadIdx.x % 64;
+    if (dtype == PLUTO_HIP_BF16) {
+      const uint16_t* in = static_cast<const uint16_t*>(base) + offset;
+#pragma unroll
+      for (int i = 0; i < SLOTS; ++i) bits[i] = in[lane + 64 * i];
+    } else {
+      const uint32_t* in = static_cast<const uint32_t*>(base) + offset;
+#pragma unroll
+      for (int i = 0; i < SLOTS; ++i) bits[i] = in[lane + 64 * i];
+    }
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) weight[i] = weights[lane + 64 * i];
+  }
+};
+
+// One wave prepares VECTORS head vectors side by side (RMSNorm with (1 + w), split-half partial
+// RoPE, bf16 rounding points as in normalize_rotate); the RoPE partner comes from the LDS
+// row the result is left in.  `rows` receive the bf16 bits; `cosine`/`sine` hold this
+// lane's rounded table entries per slot.
+template <int D, int VECTORS>
+__device__ inline void prepare_heads(const HeadVector<D> (&input)[VECTORS], int dtype, int rotary_dim, float epsilon,
+                                     const float (&cosine)[D / 64], const float (&sine)[D / 64],
+                                     uint16_t* const (&rows)[VECTORS]) {
   constexpr int SLOTS = D / 64;
   const int lane = threadIdx.x % 64;
-  float x[SLOTS], w[SLOTS];
-  if (dtype == PLUTO_HIP_BF16) {
-    const uint16_t* in = static_cast<const uint16_t*>(base) + offset;
+  float x[VECTORS][SLOTS];
+  double square[VECTORS];
 #pragma unroll
-    for (int i = 0; i < SLOTS; ++i) x[i] = bf16_bits_to_float(in[lane + 64 * i]);
-  } else {
-    const float* in = static_cast<const float*>(base) + offset;
+  for (int v = 0; v < VECTORS; ++v) {
+    square[v] = 0.0;
 #pragma unroll
-    for (int i = 0; i < SLOTS; ++i) x[i] = in[lane + 64 * i];
+    for (int i = 0; i < SLOTS; ++i) {
+      x[v][i] = __uint_as_float(dtype == PLUTO_HIP_BF16 ? input[v].bits[i] << 16 : input[v].bits[i]);
+      square[v] += static_cast<double>(x[v][i] * x[v][i]);
+    }
   }
 #pragma unroll
-  for (int i = 0; i < SLOTS; ++i) w[i] = weight[lane + 64 * i];
-  double square = 0.0;
+  for (int offset = 32; offset > 0; offset >>= 1)
 #pragma unroll
-  for (int i = 0; i < SLOTS; ++i) square += static_cast<double>(x[i] * x[i]);
-  square = wave_sum_f64(square);
-  const double inverse = 1.0 / sqrt(square / D + static_cast<double>(epsilon));
-  float normal[SLOTS];
+    for (int v = 0; v < VECTORS; ++v) square[v] += __shfl_xor(square[v], offset, 64);
+  float normal[VECTORS][SLOTS];
 #pragma unroll
-  for (int i = 0; i < SLOTS; ++i) {
-    normal[i] = round_to_bf16(
-        static_cast<float>(x[i] * inverse * (1.0 + static_cast<double>(w[i]))));
-    row[lane + 64 * i] = static_cast<uint16_t>(__float_as_uint(normal[i]) >> 16);
+  for (int v = 0; v < VECTORS; ++v) {
+    const double inverse = 1.0 / sqrt(square[v] / D + static_cast<double>(epsilon));
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+      normal[v][i] = round_to_bf16(
+          static_cast<float>(x[v][i] * inverse * (1.0 + static_cast<double>(input[v].weight[i]))));
+      rows[v][lane + 64 * i] = static_cast<uint16_t>(__float_as_uint(normal[v][i]) >> 16);
+    }
   }
-  // the wave's normalised row is in LDS before partners are read from it
+  // the wave's normalised rows are in LDS before partners are read from them
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_wave_barrier();
   const int half = rotary_dim / 2;
-  float result[SLOTS];
+  float result[VECTORS][SLOTS];
 #pragma unroll
-  for (int i = 0; i < SLOTS; ++i) {
-    const int c = lane + 64 * i;
-    result[i] = normal[i];
-    if (c < rotary_dim) {
-      const float partner = bf16_bits_to_float(row[c < half ? c + half : c - half]);
-      const float a = round_to_bf16(normal[i] * cosine[i]);
-      const float b = round_to_bf16(partner * sine[i]);
-      result[i] = round_to_bf16(c < half ? a - b : a + b);
+  for (int v = 0; v < VECTORS; ++v)
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+      const int c = lane + 64 * i;
+      result[v][i] = normal[v][i];
+      if (c < rotary_dim) {
+        const float partner = bf16_bits_to_float(rows[v][c < half ? c + half : c - half]);
+        const float a = round_to_bf16(normal[v][i] * cosine[i]);
+        const float b = round_to_bf16(partner * sine[i]);
+        result[v][i] = round_to_bf16(c < half ? a - b : a + b);
+      }
     }
-  }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int i = 0; i < SLOTS; ++i)
-    row[lane + 64 * i] = static_cast<uint16_t>(__float_as_uint(result[i]) >> 16);
+  for (int v = 0; v < VECTORS; ++v)
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i)
+      rows[v][lane + 64 * i] = static_cast<uint16_t>(__float_as_uint(result[v][i]) >> 16);
 }
 
 // Compile-time loop: f(std::integral_constant<int, I>) for I = FIRST .. LAST-1.
@@ -315,7 +346,35 @@ __device__ inline void decode_block(const DecodeArgs& a, const BlockContext& ctx
   const int groups = per_wave / 16;  // 16-token groups of this wave (<= GROUPS)
   const int wave_t0 = t0 + wave * per_wave;
 
-  // ---- V stages: requested before anything else when the block size is only
+  // ---- the vectors to prepare, requested first: wave w has query heads w and 4 + w and, in
+  // the last block, wave 3 the new K row and wave 2 the new V row ------------
+  constexpr int VECTORS = GROUP > 4 || LAST ? 2 : 1;
+  const bool key_second = LAST && GROUP <= 7 && wave == 3;  // head 7 leaves wave 3 no room
+  HeadVector<D> inputs[VECTORS];
+  uint16_t* rows_out[VECTORS];
+  float new_value[D / 64];
+  bool has[VECTORS];
+  const long long new_in = (static_cast<long long>(seq) * kh + g) * D;
+  {
+    const long long first_head = static_cast<long long>(seq) * a.query_heads + g * GROUP;
+#pragma unroll
+    for (int v = 0; v < VECTORS; ++v) {
+      const int hh = wave + 4 * v;
+      const bool key = v == 1 && key_second;
+      has[v] = hh < GROUP || key;
+      rows_out[v] = key ? new_row[0] : q_lds[min(hh, GROUP - 1)];
+      if (key)
+        inputs[v].request(a.k, new_in, a.io_dtype, a.k_norm);
+      else if (has[v])
+        inputs[v].request(a.q_gate, (first_head + hh) * 2 * D, a.io_dtype, a.q_norm);
+    }
+    if (LAST && wave == 2) {
+#pragma unroll
+      for (int i = 0; i < D / 64; ++i) new_value[i] = load_element(a.v, new_in + lane + 64 * i, a.io_dtype);
+    }
+  }
+
+  // ---- V stages: requested before any other cache row when the block size is only
   // known at run time, between the last score steps otherwise ---------------
   unsigned char* stage_base = value_area + wave * kStages * kStageBytes;
   uint32_t fill_offset[FILLS];
@@ -383,28 +442,44 @@ __device__ inline void decode_block(const DecodeArgs& a, const BlockContext& ctx
       if (c < a.rotary_dim && (wave < GROUP || LAST)) {
         const double angle =
             static_cast<double>(position) * a.inverse_frequency[c < half ? c : c - half];
-        cosine[i] = round_to_bf16(static_cast<float>(cos(angle)));
-        sine[i] = round_to_bf16(static_cast<float>(sin(angle)));
+        double sine_of, cosine_of;
+        sincos(angle, &sine_of, &cosine_of);
+        cosine[i] = round_to_bf16(static_cast<float>(cosine_of));
+        sine[i] = round_to_bf16(static_cast<float>(sine_of));
       }
     }
-    for (int hh = wave; hh < GROUP; hh += 4)
-      prepare_head<D>(a.q_gate,
-                      (static_cast<long long>(seq) * a.query_heads + g * GROUP + hh) * 2 * D,
-                      a.io_dtype, a.q_norm, a.rotary_dim, a.epsilon, cosine, sine, q_lds[hh]);
+    if (VECTORS == 2 && has[VECTORS - 1]) {
+      if (has[0]) {
+        prepare_heads<D, VECTORS>(inputs, a.io_dtype, a.rotary_dim, a.epsilon, cosine, sine, rows_out);
+      } else {
+        const HeadVector<D> one[1] = {inputs[VECTORS - 1]};
+        uint16_t* const out[1] = {rows_out[VECTORS - 1]};
+        prepare_heads<D, 1>(one, a.io_dtype, a.rotary_dim, a.epsilon, cosine, sine, out);
+      }
+    } else if (has[0]) {
+      const HeadVector<D> one[1] = {inputs[0]};
+      uint16_t* const out[1] = {rows_out[0]};
+      prepare_heads<D, 1>(one, a.io_dtype, a.rotary_dim, a.epsilon, cosine, sine, out);
+    }
     if constexpr (LAST) {
       // cached_attention_ops.cc:64-77: the rotated key and the rounded value
       // become row `position` of the cache
-      const long long in = (static_cast<long long>(seq) * kh + g) * D;
       const long long at = static_cast<long long>(position) * a.token_stride;
       if (wave == 3) {
-        prepare_head<D>(a.k, in, a.io_dtype, a.k_norm, a.rotary_dim, a.epsilon, cosine, sine,
-                        new_row[0]);
+        if (!key_second) {
+          HeadVector<D> one[1];
+          one[0].request(a.k, new_in, a.io_dtype, a.k_norm);
+          uint16_t* const out[1] = {new_row[0]};
+          prepare_heads<D, 1>(one, a.io_dtype, a.rotary_dim, a.epsilon, cosine, sine, out);
+        }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_wave_barrier();
         for (int c = lane; c < D; c += 64) ctx.keys[at + c] = new_row[0][c];
       } else if (wave == 2) {
-        for (int c = lane; c < D; c += 64) {
-          const uint16_t bits = float_to_bf16_bits(load_element(a.v, in + c, a.io_dtype));
+#pragma unroll
+        for (int i = 0; i < D / 64; ++i) {
+          const int c = lane + 64 * i;
+          const uint16_t bits = float_to_bf16_bits(new_value[i]);
           new_row[1][c] = bits;
           ctx.values[at + c] = bits;
         }
@@ -686,8 +761,17 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
   const long long first_slot = (a.block_base + batch.block_start[b]) * kh + g;
   const long long slot_step = kh;  // consecutive blocks of one kv head
   float2 o[kPairs];
+  uint32_t logits[kPairs][2];  // as they lie in memory; for the end, requested now
 #pragma unroll
-  for (int u = 0; u < kPairs; ++u) o[u] = make_float2(0.0f, 0.0f);
+  for (int u = 0; u < kPairs; ++u) {
+    o[u] = make_float2(0.0f, 0.0f);
+    const int i = min(2 * (tid + u * kThreads), GROUP * D - 2);
+    const long long at = ((static_cast<long long>(seq) * a.query_heads + g * GROUP + i / D) * 2 + 1) * D + i % D;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      logits[u][e] = a.io_dtype == PLUTO_HIP_BF16 ? static_cast<const uint16_t*>(a.q_gate)[at + e]
+                                                  : static_cast<const uint32_t*>(a.q_gate)[at + e];
+  }
   if (tid < GROUP) {
     head_state[0 * GROUP + tid] = kMasked;  // running maximum
     head_state[1 * GROUP + tid] = 0.0f;     // running normalizer
@@ -708,10 +792,19 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
       }
     };
     request(0);
+    float maxima[(GROUP + 3) / 4], sums[(GROUP + 3) / 4];
+#pragma unroll
+    for (int v = 0; v < (GROUP + 3) / 4; ++v) {
+      const long long at = (first_slot + (j0 + min(ctx.lane, count - 1)) * slot_step) * GROUP +
+                           min(ctx.wave + 4 * v, GROUP - 1);
+      maxima[v] = load_shared(&a.part_m[at]), sums[v] = load_shared(&a.part_l[at]);
+    }
     __syncthreads();  // the chunk before has been added up, and the states written
-    for (int hh = ctx.wave; hh < GROUP; hh += 4) {
-      const long long at = (first_slot + (j0 + min(ctx.lane, count - 1)) * slot_step) * GROUP + hh;
-      const float block_max = load_shared(&a.part_m[at]), block_sum = load_shared(&a.part_l[at]);
+#pragma unroll
+    for (int v = 0; v < (GROUP + 3) / 4; ++v) {
+      const int hh = ctx.wave + 4 * v;
+      if (hh >= GROUP) continue;
+      const float block_max = maxima[v], block_sum = sums[v];
       const float old_max = head_state[0 * GROUP + hh], old_sum = head_state[1 * GROUP + hh];
       const float maximum = fmaxf(old_max, max_over_wave(block_max));
       const float weight =
@@ -760,7 +853,7 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
     const float core[2] = {o[u].x / head_state[1 * GROUP + hh], o[u].y / head_state[1 * GROUP + hh]};
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const float logit = load_element(a.q_gate, (at * 2 + 1) * D + c + e, a.io_dtype);
+      const float logit = __uint_as_float(a.io_dtype == PLUTO_HIP_BF16 ? logits[u][e] << 16 : logits[u][e]);
       const float sigmoid = gate_sigmoid(logit);
       store_element(a.out, at * D + c + e, a.io_dtype,
                     round_to_bf16(round_to_bf16(core[e]) * round_to_bf16(sigmoid)));
