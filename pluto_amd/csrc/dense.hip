@@ -128,9 +128,16 @@ __device__ inline void wait_loads() {
 // out[m, n] = bias[n] + sum_k left[m, k] right[n, k]; depth % 64 == 0.  A
 // workgroup of four waves, arranged 2 x 2, owns a 64 x (64 JN) tile and each wave
 // a 32 x (32 JN) part of it.  Two LDS stages of 64 contraction elements: one is
-// filled while the other is multiplied.
-template <bool HALF, int JN>
-__global__ void __launch_bounds__(kThreads)
+// filled while the other is multiplied.  GROUPS: as many such sets of four waves share the
+// tile, each with every GROUPS-th stage of the contraction, and add their sums through LDS
+// in order.  A step is a chain of waits of 0.5 us (memory, barrier, LDS; eight stages in
+// flight took 0.44), which several workgroups on a compute unit cover for each other;
+// where there are too few of them, the groups do: 256 rows, 768 -> 2304 and its input
+// gradient take 8.0 and 18.6 us with one group, 6.1 and 11.8 with four; 512 rows 9.4 and
+// 19.2, 9.3 (two groups: 288 workgroups) and 12.7; 2000 rows of 2304 -> 768 20.4 and 18.1
+// (two).
+template <bool HALF, int JN, int GROUPS>
+__global__ void __launch_bounds__(kThreads * GROUPS)
 product_rows_kernel(ProductArgs a) {
   constexpr int KS = kDepth / 16;  // matrix instructions along the contraction per stage
   constexpr int TM = 64, TN = 64 * JN;
@@ -138,8 +145,9 @@ product_rows_kernel(ProductArgs a) {
   constexpr int kStageBytes = kLeftBytes + kRightBytes;
   constexpr int LEFT_LOADS = TM * (kDepth / 8) / kThreads;
   constexpr int RIGHT_LOADS = TN * (kDepth / 8) / kThreads;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * GROUPS * kStageBytes];
+  const int tid = threadIdx.x % kThreads, wave = tid / 64, lane = tid % 64;
+  const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads);
   const int h = lane / 32, n = lane % 32;
   const int n_tiles = (a.n_rows + TN - 1) / TN;
   const int logical = xcd_logical_block();
@@ -166,26 +174,30 @@ product_rows_kernel(ProductArgs a) {
 #pragma unroll
   for (int jn = 0; jn < JN; ++jn) {
     const int column = n0 + wn + 32 * jn + n;
-    const float start = (a.bias && column < a.n_rows) ? a.bias[column] : 0.0f;
+    const float start = (group == 0 && a.bias && column < a.n_rows) ? a.bias[column] : 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[jn][i] = start;
   }
   const uint16_t* left = a.left + static_cast<long long>(m0) * a.depth;
   const uint16_t* right = a.right + static_cast<long long>(n0) * a.depth;
   const int steps = a.depth / kDepth;
-  auto fill_stage = [&](int step) {
-    unsigned char* stage = lds + (step % 2) * kStageBytes;
+  // turn t of group g is step t GROUPS + g
+  auto fill_stage = [&](int turn) {
+    const int step = turn * GROUPS + group;
+    if (step >= steps) return;
+    unsigned char* stage = lds + (2 * group + turn % 2) * kStageBytes;
     tile_fill<kDepth, LEFT_LOADS>(stage, wave, left + step * kDepth, a.depth, m0, a.m_rows,
                                   left_fill);
     tile_fill<kDepth, RIGHT_LOADS>(stage + kLeftBytes, wave, right + step * kDepth, a.depth, n0,
                                    a.n_rows, right_fill);
   };
   fill_stage(0);
-  for (int step = 0; step < steps; ++step) {
+  for (int turn = 0; turn * GROUPS < steps; ++turn) {
     wait_loads<0>();
     lds_barrier();
-    if (step + 1 < steps) fill_stage(step + 1);
-    const unsigned char* left_tile = lds + (step % 2) * kStageBytes;
+    fill_stage(turn + 1);
+    if (turn * GROUPS + group >= steps) break;  // the last turn
+    const unsigned char* left_tile = lds + (2 * group + turn % 2) * kStageBytes;
     const unsigned char* right_tile = left_tile + kLeftBytes;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -198,6 +210,23 @@ product_rows_kernel(ProductArgs a) {
       for (int jn = 0; jn < JN; ++jn) acc[jn] = mma<HALF>(l, r[jn], acc[jn]);
     }
   }
+  if constexpr (GROUPS > 1) {
+    // the groups' sums in order; group g finishes registers 16 / GROUPS g ..
+    static_assert(JN == 1 && GROUPS * kThreads * 16 * 4 <= sizeof(lds));
+    float (*sums)[16][kThreads] = reinterpret_cast<float (*)[16][kThreads]>(lds);
+    lds_barrier();  // every group is done with its stages
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sums[group][i][tid] = acc[0][i];
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (i / (16 / GROUPS) != group) continue;
+      float sum = sums[0][i][tid];
+#pragma unroll
+      for (int g = 1; g < GROUPS; ++g) sum += sums[g][i][tid];
+      acc[0][i] = sum;
+    }
+  }
   // 32 lanes store 32 consecutive columns of a row: 64 or 128 contiguous bytes
 #pragma unroll
   for (int jn = 0; jn < JN; ++jn) {
@@ -205,6 +234,7 @@ product_rows_kernel(ProductArgs a) {
     if (column >= a.n_rows) continue;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
+      if (GROUPS > 1 && i / (16 / GROUPS) != group) continue;
       const int row = m0 + wm + 8 * (i / 4) + 4 * h + i % 4;
       if (row >= a.m_rows) continue;
       const long long at = static_cast<long long>(row) * a.n_rows + column;
@@ -424,9 +454,13 @@ void launch_product_rows(hipStream_t s, const ProductArgs& p) {
     }
     product_rows_wide_kernel<HALF, 4, 3, true><<<blocks(kWideTile), 256, 0, s>>>(p);
   } else if (medium <= small) {
-    product_rows_kernel<HALF, 2><<<blocks(kMediumTile), kThreads, 0, s>>>(p);
+    product_rows_kernel<HALF, 2, 1><<<blocks(kMediumTile), kThreads, 0, s>>>(p);
+  } else if (blocks(kSmallTile) <= 256) {
+    product_rows_kernel<HALF, 1, 4><<<blocks(kSmallTile), 4 * kThreads, 0, s>>>(p);
+  } else if (blocks(kSmallTile) <= 512) {
+    product_rows_kernel<HALF, 1, 2><<<blocks(kSmallTile), 2 * kThreads, 0, s>>>(p);
   } else {
-    product_rows_kernel<HALF, 1><<<blocks(kSmallTile), kThreads, 0, s>>>(p);
+    product_rows_kernel<HALF, 1, 1><<<blocks(kSmallTile), kThreads, 0, s>>>(p);
   }
 }
 
@@ -717,10 +751,19 @@ column_partial_kernel(const float* in, int rows, int width, float* partial, uint
   const int r0 = part * kBiasRows, r1 = min(r0 + kBiasRows, rows);
   float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   if (width % 4 == 0 && c < width) {
-#pragma unroll 4
-    for (int r = r0 + lane; r < r1; r += 16) {
+    // all of a thread's rows are requested together (four at a time: 13.1 us at 256
+    // rows of 2304, 55 at 16384; 8.0 and 47 so)
+    float4 values[kBiasRows / 16];
+#pragma unroll
+    for (int i = 0; i < kBiasRows / 16; ++i)
+      values[i] = *reinterpret_cast<const float4*>(
+          in + static_cast<long long>(min(r0 + lane + 16 * i, r1 - 1)) * width + c);
+#pragma unroll
+    for (int i = 0; i < kBiasRows / 16; ++i) {
+      const int r = r0 + lane + 16 * i;
+      if (r >= r1) break;
       const long long at = static_cast<long long>(r) * width + c;
-      const float4 value = *reinterpret_cast<const float4*>(in + at);
+      const float4 value = values[i];
       sum[0] += value.x, sum[1] += value.y, sum[2] += value.z, sum[3] += value.w;
       if (copy) {
         ushort4 out;

@@ -187,3 +187,33 @@ def test_rejects_bad_arguments(capi):
     assert lib.pluto_hip_dense_forward(stream, capi.BF16, None, px, px, 8, 64, 64, px, px, size) != 0
     assert lib.pluto_hip_dense_backward(stream, capi.BF16, px, px, px, 8, 0, 64, px, px, px, px,
                                         size) != 0
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,n_in,n_out", [(1, 64, 64), (65, 128, 64), (63, 192, 128), (130, 256, 320), (257, 320, 576),
+                                             (2113, 192, 512), (1037, 512, 1088), (256, 1088, 64), (273, 64, 1088)])
+def test_groups_of_waves_that_split_the_contraction(capi, dtype, rows, n_in, n_out):
+    """Grids of up to 256 tiles and up to 512, contractions of one stage to seventeen: groups
+    with as many stages as the others, one fewer, and none.  The bias sums over a
+    partition's last rows.  Against float64 products of the rounded operands: FP32 sums of
+    at most 1088 terms, each within half a unit of its place (2^-24 a term, 2^-13 of the
+    magnitudes in all), results in bf16 within 2^-8 more."""
+    gen = torch.Generator(device="cuda").manual_seed(rows + n_in)
+    normal = lambda *shape: torch.randn(shape, generator=gen, device="cuda")
+    half = torch.bfloat16 if dtype == "bf16" else torch.float16
+    x = normal(rows, n_in).to(torch.bfloat16 if dtype == "bf16" else torch.float32)
+    w, b, dy = normal(n_in, n_out), normal(n_out), normal(rows, n_out)
+    y = capi.dense_forward(x, w, b)
+    dx, dw, db = capi.dense_backward(x, w, dy)
+    torch.cuda.synchronize()
+    xo, wo, go = (v.to(half).double() for v in (x, w, dy))
+    result = 2.0 ** -8 if dtype == "bf16" else 0.0
+    for name, got, left, right, start, extra in (("y", y, xo, wo, b.double(), result), ("dx", dx, go, wo.t(), 0.0, 0.0),
+                                                 ("dw", dw, xo.t(), go, 0.0, 0.0)):
+        want = left @ right + start
+        magnitude = left.abs() @ right.abs() + abs(start)
+        terms = max(left.shape[1], 1088)
+        bound = extra * want.abs() + terms * 2.0 ** -24 * magnitude
+        assert ((got.double() - want).abs() <= bound).all(), (name, (got.double() - want).abs().max().item())
+    total = dy.double().sum(0)
+    assert ((db.double() - total).abs() <= rows * 2.0 ** -24 * dy.double().abs().sum(0)).all()
