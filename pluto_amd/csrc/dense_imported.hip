@@ -887,7 +887,8 @@ __device__ inline void add_waves(float (&partial)[kTileWaves][ELEMENTS][64], con
 // 8 q .. + 7 of each block of weight row n16 and of tokens n16 (and 16 + n16): operands of
 // v_mfma_f32_16x16x32_bf16 as they lie in memory, four lanes a 64-byte piece of a row.
 // Bound by the addresses of those pieces, sixteen rows a load.  5120 -> 16480, 9, 16 and 32
-// tokens: 62.7, 75.1 and 98.3 us with one tile of 32 rows a workgroup, 36.7, 37.7 and 75.5
+// tokens (at any element: global memory takes wide accesses unaligned): 62.7, 75.1 and 98.3
+// us with one tile of 32 rows a workgroup, 36.7, 37.7 and 75.5
 // so (32 tokens take twice the registers, so that the rows travel in several passes).
 template <int BLOCKS, int TOKEN_PARTS, bool ONE_PASS>
 __global__ void __launch_bounds__(64 * kTileWaves)
@@ -1215,15 +1216,15 @@ void launch_few(hipStream_t s, const FewArgs& a) {
 // to eight tokens of rows that fit in LDS, and more.  Everything else, and up to eight
 // tokens of longer rows, is the vector path's; what up to eight tokens take does not
 // depend on their number, so that a token's results do not either.  Weights are read by
-// buffer loads, which take whole words; tokens in pieces of sixteen bytes, but for the
-// kernel that makes FP8 codes of more than eight, which takes elements.
+// buffer loads, which take whole words; up to eight tokens in pieces of sixteen bytes, more
+// at any element.
 bool matrix_cores(int storage, int matrices, const void* const* weights, const void* input, int tokens, int input_dim) {
   if (storage == PLUTO_HIP_MATRIX_F32 || input_dim % kGroup != 0) return false;
   auto aligned = [](const void* p, unsigned bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; };
   for (int i = 0; i < matrices; ++i)
     if (!aligned(weights[i], 4)) return false;
   if (tokens <= kFewTokens && input_dim > kFewColumns) return false;
-  return aligned(input, 16) || (tokens > kFewTokens && storage == PLUTO_HIP_MATRIX_FP8_E4M3);
+  return tokens > kFewTokens || aligned(input, 16);
 }
 
 template <int STORAGE, int TOKENS, bool PREPARE>
