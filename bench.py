@@ -225,8 +225,8 @@ def gqa_prefill_bwd(torch, capi):
     qw = torch.from_numpy(values(np, d, 0.2, 0.3)).cuda()
     kw = torch.from_numpy(values(np, d, 0.8, 0.4)).cuda()
 
-    # the forward pass of the training step leaves the attention output, the
-    # row statistics and the prepared heads for this call (outside the timed region)
+    # the forward pass of the training step leaves the attention output and the
+    # row statistics for this call (outside the timed region)
     cache = capi.KvCache(T, kh, d)
     saved = capi.gqa_prefill_saved(p, T, cache)
     capi.gqa_prefill(p, qg, k, v, qw, kw, cache, saved=saved)
@@ -240,7 +240,7 @@ def gqa_prefill_bwd(torch, capi):
                 peak=PEAK_BF16_TFLOPS,
                 config={"workload": "qwen_gqa_sequence_backward", "batch": 1, "seq_len": T,
                         "query_heads": qh, "kv_heads": kh, "head_dim": d,
-                        "counted": "5 attention GEMMs; attention output, row statistics and prepared heads saved "
+                        "counted": "5 attention GEMMs; attention output and row statistics saved "
                                    "by the forward call"},
                 cpu=None)
 

@@ -201,10 +201,13 @@ int pluto_hip_attention_params_validate(const pluto_hip_attention_params* p);
  *   lse  optional fp32 [length, qh]: max + log(normalizer) of each row
  *   saved  optional, pluto_hip_gqa_prefill_saved_bytes(...) bytes: what
  *        pluto_hip_gqa_prefill_backward would otherwise recompute (the
- *        attention output before the gate, the row statistics, the normalised
- *        and rotated heads; the counterpart of the state SequenceForward hands
- *        to SequenceBackward, qwen_attention.cc:445-447, without its quadratic
- *        tensors).  Only for start_position 0 and where that size is not 0:
+ *        attention output before the gate and the row statistics, at head_dim
+ *        256 also the normalised and rotated heads; the counterpart of the
+ *        state SequenceForward hands to SequenceBackward, qwen_attention.cc:
+ *        445-447, without its quadratic tensors).  About length * qh *
+ *        (2 * head_dim + 8) bytes at head_dim 64 and 128, and three times as
+ *        many and 4 * length * kh * head_dim at 256.
+ *        Only for start_position 0 and where that size is not 0:
  *        round_to_bfloat16, a BF16 cache and head_dim 64, 128 or 256;
  *        PLUTO_HIP_EUNSUPPORTED otherwise.  At head_dim 256 the output is then
  *        made from FP32 softmax weights, as the backward's factors are (without
@@ -237,9 +240,9 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p,
  * [qh, length, length] each) is kept between the passes.
  *   dy       fp32 [length, qh, d]     gradient of the layer output
  *   saved    optional: the block pluto_hip_gqa_prefill filled for the same
- *            inputs and parameters; the preparation and the attention forward
- *            are then not repeated (a quarter of the call at length 8192 of
- *            head_dim 128).  NULL recomputes.
+ *            inputs and parameters; the attention forward (at head_dim 256 the
+ *            preparation too) is then not repeated, a quarter of the call at
+ *            length 8192 of head_dim 128.  NULL recomputes.
  *   dqg      fp32 [length, qh, 2, d]  query gradients at [..,0,:], gate at [..,1,:]
  *   dk, dv   fp32 [length, kh, d]
  *   dq_norm, dk_norm  optional fp32 [d]: the norm weights' gradients are ADDED

@@ -196,15 +196,18 @@ long long decode_blocks_bound(const pluto_hip_attention_params* p, int batch, co
   return blocks;
 }
 
-// What the forward pass can leave for the backward pass, from the block's first multiple of
-// 256 bytes on: the attention output before the gate (bf16 at head width 64 and 128, FP32
-// at 256, [length, qh * d]) and the two row statistics (fp32 [qh, length] each), as the
-// matrix-core backward kernels read them, and what the preparation made: the normalised
-// and rotated heads (bf16) and the rotation's table.  The copies cost the forward 4 us at
-// 8192 rows of 24 + 4 heads of 128, making them again took the backward 42.
+// What the forward pass can leave for the backward pass: the attention output before the
+// gate (bf16 at head width 64 and 128, FP32 at 256, [length, qh * d]) and the two row
+// statistics (fp32 [qh, length] each), as the matrix-core backward kernels read them.  At
+// head width 256, where the backward's kernels take FP32 factors, also what the
+// preparation made: the normalised and rotated heads (bf16) and the rotation's table.  At
+// 64 and 128 they are made again: with them the block is 119 instead of 52 MB at 8192 rows
+// of 24 + 4 heads of 128, held for every layer between the passes, for 1.6 % of the
+// training step (1784 instead of 1812 us).
 struct SavedLayout {
   size_t core, maxima, normalizers, queries, keys, values, cosines, sines, total;
 };
+bool saved_heads(const pluto_hip_attention_params* p) { return p->head_dim == kSplitHeadDim; }
 SavedLayout saved_layout(const pluto_hip_attention_params* p, int length) {
   SavedLayout l{};
   const size_t T = static_cast<size_t>(length), d = p->head_dim;
@@ -218,16 +221,20 @@ SavedLayout saved_layout(const pluto_hip_attention_params* p, int length) {
   l.core = take(rows * d * (d == kSplitHeadDim ? 4 : 2));
   l.maxima = take(rows * 4);
   l.normalizers = take(rows * 4);
-  l.queries = take(rows * d * 2);
-  l.keys = take(kv_rows * d * 2);
-  l.values = take(kv_rows * d * 2);
-  l.cosines = take(T * (p->rotary_dim / 2) * 4);
-  l.sines = take(T * (p->rotary_dim / 2) * 4);
-  l.total = at + 256;
+  if (saved_heads(p)) {
+    l.queries = take(rows * d * 2);
+    l.keys = take(kv_rows * d * 2);
+    l.values = take(kv_rows * d * 2);
+    l.cosines = take(T * (p->rotary_dim / 2) * 4);
+    l.sines = take(T * (p->rotary_dim / 2) * 4);
+  }
+  l.total = at + (saved_heads(p) ? 256 : 0);
   return l;
 }
-char* saved_base(const void* saved) {
-  return reinterpret_cast<char*>(align_up(reinterpret_cast<size_t>(saved), 256));
+// The contents' address: the block itself, or with heads its first multiple of 256.
+char* saved_base(const pluto_hip_attention_params* p, const void* saved) {
+  const size_t address = reinterpret_cast<size_t>(saved);
+  return reinterpret_cast<char*>(saved_heads(p) ? align_up(address, 256) : address);
 }
 bool saved_supported(const pluto_hip_attention_params* p, int length, int cache_dtype) {
   return p->round_to_bfloat16 && cache_dtype == PLUTO_HIP_BF16 &&
@@ -307,8 +314,8 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   prep.epsilon = p->rms_norm_epsilon;
   prep.round = round;
   const SavedLayout sl = saved ? saved_layout(p, length) : SavedLayout{};
-  char* kept = saved ? saved_base(saved) : nullptr;
-  if (saved) {
+  char* kept = saved ? saved_base(p, saved) : nullptr;
+  if (saved && saved_heads(p)) {
     prep.q_copy = kept + sl.queries;
     prep.k_copy = kept + sl.keys;
     prep.v_copy = kept + sl.values;
@@ -321,7 +328,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
 
   const float scale = 1.0f / std::sqrt(static_cast<float>(d));
   const uint16_t* gate = static_cast<const uint16_t*>(qg) + d;
-  if (saved && d == kSplitHeadDim) {
+  if (saved && saved_heads(p)) {
     // The backward at this width starts from FP32 factors: the forward makes them, and its
     // output from them.  1024 rows of 24 / 4 heads: 44 us here, where the bf16 kernel took
     // 36 and the backward repeated the forward in another 42.
@@ -429,9 +436,9 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   const int E = qh * d;
   char *queries = scratch + l.queries, *keys = scratch + l.keys, *values = scratch + l.values;
 
-  // What the forward pass derived from the inputs -- normalised, rotated q and k
-  // (PrepareKernel, qwen_attention.cc:30-63), the attention core with its row statistics --
-  // is taken from the saved block or made again.
+  // What the forward pass derived from the inputs is taken from the saved block where that
+  // has it, or made again: the attention core with its row statistics, and the normalised,
+  // rotated q and k (PrepareKernel, qwen_attention.cc:30-63).
   void* core = scratch + l.core;
   float* maxima = reinterpret_cast<float*>(scratch + l.maxima);
   float* normalizers = reinterpret_cast<float*>(scratch + l.normalizers);
@@ -439,16 +446,19 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   const bool kept = saved && (l.flash || l.split);
   if (kept) {
     const SavedLayout sl = saved_layout(p, length);
-    char* base = saved_base(saved);
+    char* base = saved_base(p, saved);
     core = base + sl.core;
     maxima = reinterpret_cast<float*>(base + sl.maxima);
     normalizers = reinterpret_cast<float*>(base + sl.normalizers);
-    queries = base + sl.queries;
-    keys = base + sl.keys;
-    values = base + sl.values;
-    cosines = reinterpret_cast<float*>(base + sl.cosines);
-    sines = reinterpret_cast<float*>(base + sl.sines);
-  } else {
+    if (saved_heads(p)) {
+      queries = base + sl.queries;
+      keys = base + sl.keys;
+      values = base + sl.values;
+      cosines = reinterpret_cast<float*>(base + sl.cosines);
+      sines = reinterpret_cast<float*>(base + sl.sines);
+    }
+  }
+  if (!kept || !saved_heads(p)) {
     PrefillPrepareArgs prep;
     prep.qg = qg;
     prep.k = k;

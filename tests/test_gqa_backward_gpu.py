@@ -221,6 +221,41 @@ def test_benchmarked_shape_against_fp32_kernels(capi):
                                    "%s T%d vs fp32-arithmetic kernels" % (name, T), far=20.0)
 
 
+@pytest.mark.parametrize("T,qh,kh,d,rot", [(97, 4, 2, 64, 32), (130, 6, 2, 128, 32)])
+def test_saved_block_is_the_output_and_its_statistics(capi, T, qh, kh, d, rot):
+    """At head width 64 and 128 a block is held for every layer between the passes: the
+    attention output in bf16 and two floats a row and head, each rounded up to 256 bytes."""
+    import ctypes
+    p = capi.attention_params(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=rot, capacity=T,
+                              round_to_bfloat16=True)
+    size = capi.lib().pluto_hip_gqa_prefill_saved_bytes(ctypes.byref(p), T, capi.BF16)
+    assert T * qh * (2 * d + 8) <= size <= T * qh * (2 * d + 8) + 3 * 255
+
+
+@pytest.mark.parametrize("T,qh,kh,d,rot", [(97, 4, 2, 64, 32), (130, 6, 2, 128, 32)])
+def test_saved_block_can_be_moved(capi, T, qh, kh, d, rot):
+    """A block that is copied to an address with another remainder (kept on the host between
+    the passes, packed behind other tensors) is read as it was written."""
+    import ctypes
+    got, _, args, _ = run_case(capi, T, qh, kh, d, rot, True, seed=T + d)
+    p, qg, k, v, qw, kw_, dy = args
+    size = capi.lib().pluto_hip_gqa_prefill_saved_bytes(ctypes.byref(p), T, capi.BF16)
+    for filled_at, read_at in ((0, 16), (16, 0), (48, 208), (240, 128)):
+        space = torch.full((size + 512,), 0x7f, dtype=torch.uint8, device="cuda")
+        assert space.data_ptr() % 256 == 0
+        block = space[filled_at:filled_at + size]
+        capi.gqa_prefill(p, qg, k, v, qw, kw_, capi.KvCache(T, kh, d), saved=block)
+        kept = block.cpu()
+        space.fill_(0x7f)
+        block = space[read_at:read_at + size]
+        block.copy_(kept)
+        dq_norm, dk_norm = torch.zeros(d, device="cuda"), torch.zeros(d, device="cuda")
+        grads = capi.gqa_prefill_backward(p, qg, k, v, qw, kw_, dy, dq_norm=dq_norm, dk_norm=dk_norm, saved=block)
+        torch.cuda.synchronize()
+        for name, value in zip(("dqg", "dk", "dv", "dq_norm", "dk_norm"), grads + (dq_norm, dk_norm)):
+            assert np.array_equal(value.cpu().numpy(), got[name]), (name, filled_at, read_at)
+
+
 def test_saved_state_is_refused_where_none_is_kept(capi):
     T, qh, kh, d, rot = 16, 2, 1, 32, 8
     kw = dict(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=rot, capacity=T,
