@@ -13,14 +13,20 @@
 // attn_f32_mfma.hip: dq works on S^T (lane = query), dkv on S (lane = key), so the score
 // tile's accumulator is the B operand of the gradient product.
 //
-// 4 sequences x 12 heads x 256 x 64: dq 11.6, dkv 15.2 us (18.9 and 21.1 on the FP32
-// matrix instructions); 16 x 12 x 512 x 64 88 and 117.  Small calls are bound by the
+// Of a call, us, on the FP32 matrix instructions and now: 4 sequences x 12 heads x 256 x 64
+// 37.7, 25.0 (dq 11.6, dkv 15.2); 16 x 12 x 512 x 64 285, 194 (88, 117); 4 x 12 x 256 x 32
+// 21.9, 16.9; 8 x 12 x 512 x 32 74, 61; 4 x 6 x 256 x 128 53.4, 34.5; 8 x 6 x 512 x 128 191,
+// 146 (64, 86).  D = 128 leaves room for one workgroup a compute unit and takes 1.4 times
+// what D = 64 does for as much work; having the other arithmetic at hand (attn_f32_split.h)
+// costs it 2 %, its registers being all taken, the others nothing.  Small calls are bound by the
 // chain of a wave (its first tile's way from memory, the pieces, two products after each
 // other, the merge: 7 us with one tile), large ones by streaming every tile once for 32
 // rows.  Against 64-bit arithmetic the gradients are 2.4e-7 off for standard normal
 // inputs of 256 rows, 3.0e-7 with the FP32 matrix instructions.
 #include "attn_f32_split.h"
 #include "attn_generic.h"
+
+#include <type_traits>
 
 namespace pluto_hip {
 namespace {
@@ -126,10 +132,13 @@ __device__ __forceinline__ void f32_dq(const GenericBackwardArgs& a, const F32Un
   }
   sm.part_deltas[wave][lane] = part_delta;
   floatx16 acc[DB];
+  auto clear = [&]() {
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[db][i] = 0.0f;
+      for (int i = 0; i < 16; ++i) acc[db][i] = 0.0f;
+  };
+  clear();
   __syncthreads();
   float delta = 0.0f;
 #pragma unroll
@@ -137,34 +146,54 @@ __device__ __forceinline__ void f32_dq(const GenericBackwardArgs& a, const F32Un
   delta = half_swap_sum(delta);
   if (wave == 0 && h == 0 && query < T) a.deltas[stats + query] = delta;
 
-  for (int kt = wave; kt < key_tiles; kt += kWaves) {
-    const int k0 = kt * 32;
-    floatx16 s, dp;
+  auto walk = [&](auto pieces) {
+    constexpr bool PIECES = decltype(pieces)::value;
+    for (int kt = wave; kt < key_tiles; kt += kWaves) {
+      const int k0 = kt * 32;
+      floatx16 s, dp;
+      const float* k_tile = q_base + E + k0 * 3LL * E;
+      if constexpr (PIECES) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
-    Rows::keep(area, v_raw, lane);
-    request(v_raw, 2, kt + kWaves);
+        for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
+        Rows::keep(area, v_raw, lane);
+        request(v_raw, 2, kt + kWaves);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      dp = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(1), ks, lane), dp);
-    Rows::keep(area, k_raw, lane);  // in V's place
-    request(k_raw, 1, kt + kWaves);
+        for (int ks = 0; ks < KS; ++ks)
+          dp = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(1), ks, lane), dp);
+        Rows::keep(area, k_raw, lane);  // in V's place
+        request(k_raw, 1, kt + kWaves);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(0), ks, lane), s);
-    // register i = (key k0 + 8(i/4) + 4h + i%4, query n)
+        for (int ks = 0; ks < KS; ++ks)
+          s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(0), ks, lane), s);
+      } else {
+        dp = Rows::exact_rows(k_tile + E, 3LL * E, T - k0, a.d_out + (row0 + query_load) * E + unit.head * D, lane);
+        s = Rows::exact_rows(k_tile, 3LL * E, T - k0, q_base + query_load * 3LL * E, lane);
+      }
+      // register i = (key k0 + 8(i/4) + 4h + i%4, query n)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int key = k0 + 8 * (i / 4) + 4 * h + (i % 4);
-      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale, -maximum) * kLog2e) * inverse;
-      s[i] = key <= query_load ? p * (dp[i] - delta) * a.scale : 0.0f;
+      for (int i = 0; i < 16; ++i) {
+        const int key = k0 + 8 * (i / 4) + 4 * h + (i % 4);
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale, -maximum) * kLog2e) * inverse;
+        float ds = p * (dp[i] - delta) * a.scale;
+        asm("" : "+v"(ds));  // in every lane: no branch around it
+        s[i] = key <= query_load ? ds : 0.0f;
+      }
+      if constexpr (PIECES) {
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const Pieces ds = split_accumulator(s, s2);
+#pragma unroll
+          for (int db = 0; db < DB; ++db) acc[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), ds, acc[db]);
+        }
+      } else {
+        Rows::exact_transposed(acc, k_tile, 3LL * E, T - k0, s, lane);
+      }
     }
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const Pieces ds = split_accumulator(s, s2);
-#pragma unroll
-      for (int db = 0; db < DB; ++db) acc[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), ds, acc[db]);
-    }
+  };
+  walk(std::true_type());
+  if (__any(!all_finite(acc))) [[unlikely]] {
+    clear();
+    walk(std::false_type());
   }
   float4 own[4 * DB];
 #pragma unroll
@@ -228,66 +257,93 @@ __device__ __forceinline__ void f32_dkv(const GenericBackwardArgs& a, const F32U
     }
   }
   floatx16 dk[DB], dv[DB];
+  auto clear = [&]() {
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
+      for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.0f;
+  };
+  clear();
   __syncthreads();
-  for (int qt = k0 / 32 + wave; qt < query_tiles; qt += kWaves) {
-    const int q0 = qt * 32;
-    if (h == 0) {
-      const int row = min(q0 + n, T - 1);
-      const float normalizer = a.normalizers[stats + row];
-      row_stats[wave][0][n] = a.maxima[stats + row];
-      row_stats[wave][1][n] = 1.0f / (normalizer > 0.0f ? normalizer : 1.0f);
-      row_stats[wave][2][n] = OWN_DELTAS ? own_deltas[q0 + n] : a.deltas[stats + row];
-    }
-    floatx16 s, dp;
+  auto walk = [&](auto pieces) {
+    constexpr bool PIECES = decltype(pieces)::value;
+    for (int qt = k0 / 32 + wave; qt < query_tiles; qt += kWaves) {
+      const int q0 = qt * 32;
+      if (h == 0) {
+        const int row = min(q0 + n, T - 1);
+        const float normalizer = a.normalizers[stats + row];
+        row_stats[wave][0][n] = a.maxima[stats + row];
+        row_stats[wave][1][n] = 1.0f / (normalizer > 0.0f ? normalizer : 1.0f);
+        row_stats[wave][2][n] = OWN_DELTAS ? own_deltas[q0 + n] : a.deltas[stats + row];
+      }
+      floatx16 s, dp;
+      const float* q_tile = q_base + q0 * 3LL * E;
+      const float* g_tile = g_base + q0 * 1LL * E;
+      if constexpr (PIECES) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
-    // one area for Q, dO and Q again: two would leave room for one workgroup a compute unit
-    Rows::keep(area, q_raw, lane);
+        for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
+        // one area for Q, dO and Q again: two would leave room for one workgroup a compute unit
+        Rows::keep(area, q_raw, lane);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(0), ks, lane), s);
-    Rows::keep(area, g_raw, lane);
-    request_g(qt + kWaves);
+        for (int ks = 0; ks < KS; ++ks)
+          s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(0), ks, lane), s);
+        Rows::keep(area, g_raw, lane);
+        request_g(qt + kWaves);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      dp = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(1), ks, lane), dp);
-    // register i = (query q0 + 8(i/4) + 4h + i%4, key n)
+        for (int ks = 0; ks < KS; ++ks)
+          dp = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(sm.own(1), ks, lane), dp);
+      } else {
+        const float* own_key = q_base + E + key_load * 3LL * E;
+        s = Rows::exact_rows(q_tile, 3LL * E, T - q0, own_key, lane);
+        dp = Rows::exact_rows(g_tile, E, T - q0, own_key + E, lane);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // (the products spread over what follows: 24.7 -> 25.7 us above)
+      // register i = (query q0 + 8(i/4) + 4h + i%4, key n)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int at = 8 * j + 4 * h;
-      const float4 maximum = *reinterpret_cast<const float4*>(&row_stats[wave][0][at]);
-      const float4 inverse = *reinterpret_cast<const float4*>(&row_stats[wave][1][at]);
-      const float4 delta = *reinterpret_cast<const float4*>(&row_stats[wave][2][at]);
-      const float m[4] = {maximum.x, maximum.y, maximum.z, maximum.w};
-      const float r[4] = {inverse.x, inverse.y, inverse.z, inverse.w};
-      const float dl[4] = {delta.x, delta.y, delta.z, delta.w};
+      for (int j = 0; j < 4; ++j) {
+        const int at = 8 * j + 4 * h;
+        const float4 maximum = *reinterpret_cast<const float4*>(&row_stats[wave][0][at]);
+        const float4 inverse = *reinterpret_cast<const float4*>(&row_stats[wave][1][at]);
+        const float4 delta = *reinterpret_cast<const float4*>(&row_stats[wave][2][at]);
+        const float m[4] = {maximum.x, maximum.y, maximum.z, maximum.w};
+        const float r[4] = {inverse.x, inverse.y, inverse.z, inverse.w};
+        const float dl[4] = {delta.x, delta.y, delta.z, delta.w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 4 * j + e, query = q0 + at + e;
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale, -m[e]) * kLog2e) * r[e];
-        const bool visible = key <= query && query < T;
-        s[i] = visible ? p : 0.0f;
-        dp[i] = visible ? p * (dp[i] - dl[e]) * a.scale : 0.0f;
+        for (int e = 0; e < 4; ++e) {
+          const int i = 4 * j + e, query = q0 + at + e;
+          float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.scale, -m[e]) * kLog2e) * r[e];
+          float ds = p * (dp[i] - dl[e]) * a.scale;
+          asm("" : "+v"(p), "+v"(ds));  // in every lane: no branch around them
+          const bool visible = key <= query && query < T;
+          s[i] = visible ? p : 0.0f;
+          dp[i] = visible ? ds : 0.0f;
+        }
+      }
+      if constexpr (PIECES) {
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const Pieces p = split_accumulator(s, s2);
+#pragma unroll
+          for (int db = 0; db < DB; ++db) dv[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), p, dv[db]);
+        }
+        Rows::keep(area, q_raw, lane);
+        request_q(qt + kWaves);
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const Pieces ds = split_accumulator(dp, s2);
+#pragma unroll
+          for (int db = 0; db < DB; ++db) dk[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), ds, dk[db]);
+        }
+      } else {
+        Rows::exact_transposed(dv, g_tile, E, T - q0, s, lane);
+        Rows::exact_transposed(dk, q_tile, 3LL * E, T - q0, dp, lane);
       }
     }
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const Pieces p = split_accumulator(s, s2);
-#pragma unroll
-      for (int db = 0; db < DB; ++db) dv[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), p, dv[db]);
-    }
-    Rows::keep(area, q_raw, lane);
-    request_q(qt + kWaves);
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const Pieces ds = split_accumulator(dp, s2);
-#pragma unroll
-      for (int db = 0; db < DB; ++db) dk[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), ds, dk[db]);
-    }
+  };
+  walk(std::true_type());
+  if (__any(!all_finite(dk) || !all_finite(dv))) [[unlikely]] {
+    clear();
+    walk(std::false_type());
   }
   float4 own[8 * DB];
 #pragma unroll

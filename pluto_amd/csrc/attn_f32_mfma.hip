@@ -8,9 +8,11 @@
 // LDS in wave order.  A row block near the end of a sequence has many tiles and there
 // are few row blocks, so splitting the keys is what fills the machine; the row
 // blocks are handed out heaviest first, and a wave's next tiles travel while it
-// works on the ones it has.  4 sequences x 12 heads x 256 x 64 10.0 us (12.3 on the FP32
-// matrix instructions), 16 x 12 x 512 x 64 77; outputs 1.7e-7 off 64-bit arithmetic for
-// standard normal inputs, 2.2e-7 with those instructions.  As in
+// works on the ones it has.  Of a call, us, on the FP32 matrix instructions and now:
+// 4 sequences x 12 heads x 256 x 64 12.1, 10.0; 16 x 12 x 512 x 64 86, 71-75; 4 x 12 x 256 x
+// 32 8.3, 7.5; 8 x 12 x 512 x 32 25.6, 24.0; 4 x 6 x 256 x 128 17.5, 15.7; 8 x 6 x 512 x 128
+// 57.7, 52.8 (looking at the results costs 0.2 us of a small call).  Outputs 1.7e-7 off
+// 64-bit arithmetic for standard normal inputs, 2.2e-7 with those instructions.  As in
 // the bf16 kernels the products are transposed,
 // S^T = K Q^T and O^T = V^T P^T, so that a lane owns one query column: its row
 // maximum and sum are lane-local up to one exchange between the two lane
@@ -18,6 +20,8 @@
 // wave's area: with one each a compute unit would hold one workgroup.
 #include "attn_f32_split.h"
 #include "attn_generic.h"
+
+#include <type_traits>
 
 namespace pluto_hip {
 namespace {
@@ -67,56 +71,80 @@ f32_forward_kernel(GenericForwardArgs a) {
     Rows::keep_own(own, ks, lane, split_eight(row[0], row[1]));
   }
   floatx16 o[DB];
+  float running_max, running_sum;  // base-2 scaled scores
+  auto clear = [&]() {
 #pragma unroll
-  for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
-  float running_max = kMasked, running_sum = 0.0f;  // base-2 scaled scores
+      for (int i = 0; i < 16; ++i) o[db][i] = 0.0f;
+    running_max = kMasked;
+    running_sum = 0.0f;
+  };
+  clear();
   __syncthreads();
 
   const int last_key = min(a.start_position + query, a.kv_rows - 1);  // keys beyond it are masked
-  for (int kt = wave; kt < key_tiles; kt += kKeySplit) {
-    Rows::keep(area, k_raw, lane);
-    request(k_raw, k_base, a.k.row_stride, kt + kKeySplit);
-    floatx16 s;
+  auto walk = [&](auto pieces) {
+    constexpr bool PIECES = decltype(pieces)::value;
+    for (int kt = wave; kt < key_tiles; kt += kKeySplit) {
+      const int k0 = kt * 32;
+      floatx16 s;
+      if constexpr (PIECES) {
+        Rows::keep(area, k_raw, lane);
+        request(k_raw, k_base, a.k.row_stride, kt + kKeySplit);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(own, ks, lane), s);
-    Rows::keep(area, v_raw, lane);  // in K's place
-    request(v_raw, v_base, a.v.row_stride, kt + kKeySplit);
-    // register i = (key kt*32 + 8(i/4) + 4h + i%4, query n)
-    const int last = last_key - kt * 32 - 4 * h;
-    float tile_max = kMasked;
+        for (int ks = 0; ks < KS; ++ks)
+          s = mma_pieces(Rows::read_rows(area, ks, lane), Rows::read_own(own, ks, lane), s);
+        Rows::keep(area, v_raw, lane);  // in K's place
+        request(v_raw, v_base, a.v.row_stride, kt + kKeySplit);
+      } else {
+        s = Rows::exact_rows(k_base + k0 * a.k.row_stride, a.k.row_stride, a.kv_rows - k0,
+                             q_base + query_load * a.q.row_stride, lane);
+      }
+      // register i = (key k0 + 8(i/4) + 4h + i%4, query n)
+      const int last = last_key - k0 - 4 * h;
+      float tile_max = kMasked;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s[i] = 8 * (i / 4) + i % 4 <= last ? s[i] * scale2 : kMasked;
-      tile_max = fmaxf(tile_max, s[i]);
+      for (int i = 0; i < 16; ++i) {
+        s[i] = 8 * (i / 4) + i % 4 <= last ? s[i] * scale2 : kMasked;
+        tile_max = fmaxf(tile_max, s[i]);
+      }
+      tile_max = half_swap_max(tile_max);
+      const float new_max = fmaxf(running_max, tile_max);
+      const float correction = __builtin_amdgcn_exp2f(running_max - new_max);
+      running_max = new_max;
+      float tile_sum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float p = s[i] == kMasked ? 0.0f : __builtin_amdgcn_exp2f(s[i] - new_max);
+        s[i] = p;
+        tile_sum += p;
+      }
+      running_sum = running_sum * correction + half_swap_sum(tile_sum);
+      if (__any(correction != 1.0f)) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[db][i] *= correction;
+      }
+      if constexpr (PIECES) {
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          const Pieces p = split_accumulator(s, s2);
+#pragma unroll
+          for (int db = 0; db < DB; ++db) o[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), p, o[db]);
+        }
+      } else {
+        Rows::exact_transposed(o, v_base + k0 * a.v.row_stride, a.v.row_stride, a.kv_rows - k0, s, lane);
+      }
     }
-    tile_max = half_swap_max(tile_max);
-    const float new_max = fmaxf(running_max, tile_max);
-    const float correction = __builtin_amdgcn_exp2f(running_max - new_max);
-    running_max = new_max;
-    float tile_sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float p = s[i] == kMasked ? 0.0f : __builtin_amdgcn_exp2f(s[i] - new_max);
-      s[i] = p;
-      tile_sum += p;
-    }
-    running_sum = running_sum * correction + half_swap_sum(tile_sum);
-    if (__any(correction != 1.0f)) {
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[db][i] *= correction;
-    }
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const Pieces p = split_accumulator(s, s2);
-#pragma unroll
-      for (int db = 0; db < DB; ++db) o[db] = mma_pieces(Rows::read_transposed(area, db, s2, lane), p, o[db]);
-    }
+  };
+  walk(std::true_type());
+  if (__any(!all_finite(o) || running_sum != running_sum)) [[unlikely]] {
+    clear();
+    walk(std::false_type());
   }
   // ---- merge: every wave's result is relative to its own maximum; the waves take turns at
   // the groups of four channels

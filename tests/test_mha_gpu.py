@@ -156,6 +156,63 @@ def test_fp32_non_finite_rows_stay_in_their_tile(capi):
         assert not torch.isfinite(grads2[:41, 2, 5]).any()
 
 
+INF, NEAR_TOP = float("inf"), 3.4e38  # the latter rounds to an infinity in bf16
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B", [1, 40])  # both backward kernels in one launch, and in two
+@pytest.mark.parametrize("what", ["V inf", "V -inf", "V near top", "score -inf", "score near bottom",
+                                  "score overflows", "K inf", "dO inf", "dO near top"])
+def test_fp32_beyond_what_pieces_hold(capi, D, B, what):
+    """Infinities, and finite values whose nearest bf16 is one, give what FP32 arithmetic
+    gives, element for element the same numbers, infinities and NaNs as the any-shape
+    kernels.  Numbers: to FP32 rounding of sums that a row's largest element leads; where
+    queries of 1e25 multiply differences that are rounded to 2^-24 of their terms (some ten,
+    added up over 160 queries), also to 4e-6 of the channel's largest."""
+    T, H = 160, 2
+    E = H * D
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn((B * T, 3 * E), generator=gen, device="cuda")
+    d_out = torch.randn((B * T, E), generator=gen, device="cuda")
+    if what.startswith("V"):
+        x[70, 2 * E + 5] = {"V inf": INF, "V -inf": -INF, "V near top": NEAR_TOP}[what]
+    elif what.startswith("dO"):
+        d_out[70, 5] = INF if what == "dO inf" else NEAR_TOP
+    else:
+        x[:T, 5] = x[:T, 5].abs() + 0.1
+        if what == "score near bottom":
+            x[:T, 5] *= 1e-2
+        if what == "score overflows":
+            x[:T, 5] += 1.2345678e25
+        x[70, E + 5] = {"score -inf": -INF, "score near bottom": -NEAR_TOP, "score overflows": -1.2345678e25,
+                        "K inf": INF}[what]
+        if what == "score overflows":  # the other keys of that channel do not
+            x[:70, E + 5] = 0
+            x[71:T, E + 5] = 0
+
+    def once():
+        out, maxima, normalizers = capi.mha_forward(x, T, H)
+        path = capi.last_path()
+        grads = capi.mha_backward(x, out, d_out, maxima, normalizers, T, H)
+        torch.cuda.synchronize()
+        return path, (out, maxima, normalizers, grads)
+
+    path, got = once()
+    assert path == capi.PATH_MATRIX_F32
+    with capi.force_generic():
+        want = once()[1]
+    for name, a, b in zip(("out", "maxima", "normalizers", "gradients"), got, want):
+        a, b = a.double(), b.double()
+        assert torch.equal(a.isnan(), b.isnan()), name
+        assert torch.equal(torch.where(a.isinf(), a, 0), torch.where(b.isinf(), b, 0)), name
+        finite = b.isfinite()
+        a, b = torch.where(finite, a, 0), torch.where(finite, b, 0)
+        bound = FP32_REL * b.abs().amax(-1, keepdim=True)
+        if what == "score overflows":
+            bound = bound + 4e-6 * b.abs().amax(0, keepdim=True)
+        assert ((a - b).abs() <= bound).all(), name
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_peaked_scores(capi, oracle, bf16):
     check(capi, oracle, 65, 1, 64, 2, bf16, seed=5, qk_scale=20.0 if not bf16 else 4.0)
