@@ -206,7 +206,9 @@ int pluto_hip_attention_params_validate(const pluto_hip_attention_params* p);
  *        state SequenceForward hands to SequenceBackward, qwen_attention.cc:
  *        445-447, without its quadratic tensors).  About length * qh *
  *        (2 * head_dim + 8) bytes at head_dim 64 and 128, and three times as
- *        many and 4 * length * kh * head_dim at 256.
+ *        many and 4 * length * kh * head_dim at 256.  The contents begin where
+ *        the block does: it may be copied to another address between the
+ *        calls.  At head_dim 256 it starts at a multiple of 4 (PLUTO_HIP_EINVAL).
  *        Only for start_position 0 and where that size is not 0:
  *        round_to_bfloat16, a BF16 cache and head_dim 64, 128 or 256;
  *        PLUTO_HIP_EUNSUPPORTED otherwise.  At head_dim 256 the output is then

@@ -228,13 +228,13 @@ SavedLayout saved_layout(const pluto_hip_attention_params* p, int length) {
     l.cosines = take(T * (p->rotary_dim / 2) * 4);
     l.sines = take(T * (p->rotary_dim / 2) * 4);
   }
-  l.total = at + (saved_heads(p) ? 256 : 0);
+  l.total = at;
   return l;
 }
-// The contents' address: the block itself, or with heads its first multiple of 256.
-char* saved_base(const pluto_hip_attention_params* p, const void* saved) {
-  const size_t address = reinterpret_cast<size_t>(saved);
-  return reinterpret_cast<char*>(saved_heads(p) ? align_up(address, 256) : address);
+// Offsets count from where the block starts, so that it can be moved.  The kernels of head
+// width 256 bring its rows to LDS through buffer loads, which take whole words.
+bool saved_misplaced(const pluto_hip_attention_params* p, const void* saved) {
+  return saved_heads(p) && (reinterpret_cast<uintptr_t>(saved) & 3u) != 0;
 }
 bool saved_supported(const pluto_hip_attention_params* p, int length, int cache_dtype) {
   return p->round_to_bfloat16 && cache_dtype == PLUTO_HIP_BF16 &&
@@ -282,6 +282,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   // the saved state describes a whole sequence attended from position 0
   if (saved && (start_position != 0 || !saved_supported(p, length, cache->dtype)))
     return PLUTO_HIP_EUNSUPPORTED;
+  if (saved_misplaced(p, saved)) return PLUTO_HIP_EINVAL;
   const PrefillLayout layout = prefill_layout(p, length);
   if (!workspace || workspace_bytes < layout.partial) return PLUTO_HIP_EWORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -314,7 +315,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p, int
   prep.epsilon = p->rms_norm_epsilon;
   prep.round = round;
   const SavedLayout sl = saved ? saved_layout(p, length) : SavedLayout{};
-  char* kept = saved ? saved_base(p, saved) : nullptr;
+  char* kept = static_cast<char*>(saved);
   if (saved && saved_heads(p)) {
     prep.q_copy = kept + sl.queries;
     prep.k_copy = kept + sl.keys;
@@ -427,6 +428,7 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   if (l.attention_bytes == 0) return PLUTO_HIP_EINVAL;
   if (!workspace || workspace_bytes < l.total) return PLUTO_HIP_EWORKSPACE;
   if (saved && !saved_supported(p, length, PLUTO_HIP_BF16)) return PLUTO_HIP_EUNSUPPORTED;
+  if (saved_misplaced(p, saved)) return PLUTO_HIP_EINVAL;
   hipStream_t s = static_cast<hipStream_t>(stream);
   char* scratch = reinterpret_cast<char*>(align_up(reinterpret_cast<size_t>(workspace), 256));
   const float* cosines = reinterpret_cast<float*>(scratch + l.cosines);
@@ -446,7 +448,7 @@ int pluto_hip_gqa_prefill_backward(void* stream, const pluto_hip_attention_param
   const bool kept = saved && (l.flash || l.split);
   if (kept) {
     const SavedLayout sl = saved_layout(p, length);
-    char* base = saved_base(p, saved);
+    char* base = static_cast<char*>(const_cast<void*>(saved));
     core = base + sl.core;
     maxima = reinterpret_cast<float*>(base + sl.maxima);
     normalizers = reinterpret_cast<float*>(base + sl.normalizers);

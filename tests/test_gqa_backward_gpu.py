@@ -232,7 +232,7 @@ def test_saved_block_is_the_output_and_its_statistics(capi, T, qh, kh, d, rot):
     assert T * qh * (2 * d + 8) <= size <= T * qh * (2 * d + 8) + 3 * 255
 
 
-@pytest.mark.parametrize("T,qh,kh,d,rot", [(97, 4, 2, 64, 32), (130, 6, 2, 128, 32)])
+@pytest.mark.parametrize("T,qh,kh,d,rot", [(97, 4, 2, 64, 32), (130, 6, 2, 128, 32), (130, 6, 2, 256, 64)])
 def test_saved_block_can_be_moved(capi, T, qh, kh, d, rot):
     """A block that is copied to an address with another remainder (kept on the host between
     the passes, packed behind other tensors) is read as it was written."""
@@ -240,7 +240,7 @@ def test_saved_block_can_be_moved(capi, T, qh, kh, d, rot):
     got, _, args, _ = run_case(capi, T, qh, kh, d, rot, True, seed=T + d)
     p, qg, k, v, qw, kw_, dy = args
     size = capi.lib().pluto_hip_gqa_prefill_saved_bytes(ctypes.byref(p), T, capi.BF16)
-    for filled_at, read_at in ((0, 16), (16, 0), (48, 208), (240, 128)):
+    for filled_at, read_at in ((0, 16), (16, 0), (48, 208), (240, 4), (12, 128), (0, 100)):
         space = torch.full((size + 512,), 0x7f, dtype=torch.uint8, device="cuda")
         assert space.data_ptr() % 256 == 0
         block = space[filled_at:filled_at + size]
@@ -254,6 +254,23 @@ def test_saved_block_can_be_moved(capi, T, qh, kh, d, rot):
         torch.cuda.synchronize()
         for name, value in zip(("dqg", "dk", "dv", "dq_norm", "dk_norm"), grads + (dq_norm, dk_norm)):
             assert np.array_equal(value.cpu().numpy(), got[name]), (name, filled_at, read_at)
+
+
+def test_saved_block_off_a_word_is_refused_at_head_width_256(capi):
+    T, qh, kh, d = 33, 2, 1, 256
+    p = capi.attention_params(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=64, capacity=T,
+                              round_to_bfloat16=True)
+    cache = capi.KvCache(T, kh, d)
+    block = torch.zeros(capi.gqa_prefill_saved(p, T, cache).numel() + 2, dtype=torch.uint8, device="cuda")[2:]
+    qg = torch.zeros((T, qh, 2, d), dtype=torch.bfloat16, device="cuda")
+    k = torch.zeros((T, kh, d), dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(d, device="cuda")
+    with pytest.raises(capi.PlutoHipError) as info:
+        capi.gqa_prefill(p, qg, k, k, w, w, cache, saved=block)
+    assert info.value.code == capi.EINVAL
+    with pytest.raises(capi.PlutoHipError) as info:
+        capi.gqa_prefill_backward(p, qg, k, k, w, w, torch.zeros((T, qh, d), device="cuda"), saved=block)
+    assert info.value.code == capi.EINVAL
 
 
 def test_saved_state_is_refused_where_none_is_kept(capi):
