@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "dense.h"
+#include "imported_offsets.h"
 
 namespace pluto_hip {
 namespace {
@@ -680,13 +681,13 @@ imported_several_kernel(FewArgs m, int panels) {
   const uint32_t row_bytes = m.cols * (FP8 ? 1 : 2);
   const bool whole = steps * kStepColumns == m.cols;
   float* token_scales = reinterpret_cast<float*>(few_lds + QUADS * steps * kReads * 64);
-  const uint32_t lane_at = i4 * row_bytes + block * 16;
+  const uint32_t row_start = i4 * row_bytes;
   uint4 raw[STEPS];
   auto request = [&](const FewUnit& u, int panel, int step) {
     const uint32_t at = (panel * STEPS + step) * 256;
-    // what lies past the end of a row reads zero
-    const uint32_t mine = whole || at + block * 16 < row_bytes ? lane_at : 0x80000000u;
-    raw[step] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(u.weights, mine, at, 0));
+    const SeveralPlace place = several_place(row_bytes, row_start, at, block);
+    raw[step] = __builtin_bit_cast(
+        uint4, __builtin_amdgcn_raw_buffer_load_b128(u.weights, place.lane, place.step, 0));
   };
   // a panel's scales: lane l holds that of group l of it
   auto request_scales = [&](const FewUnit& u, int panel) {
