@@ -385,10 +385,10 @@ __global__ void __launch_bounds__(256) imported_matvec_ragged_kernel(MatVecArgs 
 // how many there are.  FP8: codes are exact in bf16, and the sixteen elements of a piece lie
 // in one block of scales, which multiply their sum (see below).
 // On the vector units every token is another FMA a weight and another read of its values.
-// Hot weights (in the memory-side cache), us for 1, 2, 4, 8 tokens, before and now:
-// 5120 -> 16480 in FP8 19.0, 34.1, 50.1, 84.2 and 17.5, 19.7, 20.8, 24.5; 6144 -> 5120
-// in FP8 8.5, 13.8, 20.9, 35.4 and 9.3, 11.8, 13.2, 18.4; 5120 -> 16480 in bf16 26.4,
-// 31.7, 47.3, 70.3 and 26.2, 26.6, 29.1, 30.0 (169 MB: 6.3 TB/s).
+// Hot weights (in the memory-side cache), us for 1, 2, 4, 8 tokens in a captured graph, on
+// the vector units and now: 5120 -> 16480 in FP8 19.2, 33.2, 50.3, 82.6 and 17.5, 20.1, 21.1,
+// 24.4; 6144 -> 5120 in FP8 8.8, 13.9, 21.4, 35.7 and 7.7, 12.2, 13.6, 18.7; 5120 -> 16480 in
+// bf16 26.9, 31.9, 47.9, 70.3 and 27.0, 27.5, 30.0, 30.9 (169 MB: 6.3 TB/s).
 typedef __attribute__((ext_vector_type(4))) short shortx4;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
@@ -1128,8 +1128,12 @@ void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t) {
   const unsigned grid = std::min(t.first_block[t.matrices], 256);
   int passes = 1;
   auto launch = [&](auto kernel) { kernel<<<grid, 64 * kTileWaves, 0, s>>>(t, passes); };
-  // as many blocks as a wave's registers hold
-  constexpr int kMost = PARTS * TOKEN_PARTS == 4 ? 5 : 6;
+  // As many blocks as a wave's registers hold for the next tile; where a workgroup has one
+  // tile of 32 rows and nothing to request ahead for, as few as its first request: the
+  // products begin when that has arrived.  6144 -> 5120, 9 and 32 tokens: 16.7 us in one
+  // pass of six blocks, 14.1 in two of three and 17.2; 5120 -> 5120 14.1 and 18.6 in one
+  // pass of five, 13.6 and 16.9.
+  constexpr int kMost = PARTS == 2 ? 4 : 6;
   if (owned > kMost) {
     passes = (owned + 3) / 4;
     return (owned + passes - 1) / passes == 3 ? launch(imported_tile_fp8_kernel<3, PARTS, TOKEN_PARTS, false>)
@@ -1140,9 +1144,8 @@ void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t) {
     case 2: return launch(imported_tile_fp8_kernel<2, PARTS, TOKEN_PARTS, true>);
     case 3: return launch(imported_tile_fp8_kernel<3, PARTS, TOKEN_PARTS, true>);
     case 4: return launch(imported_tile_fp8_kernel<4, PARTS, TOKEN_PARTS, true>);
-    case 5: return launch(imported_tile_fp8_kernel<5, PARTS, TOKEN_PARTS, true>);
-    default:
-      if constexpr (kMost == 6) launch(imported_tile_fp8_kernel<6, PARTS, TOKEN_PARTS, true>);
+    case 5: if constexpr (kMost == 6) return launch(imported_tile_fp8_kernel<5, PARTS, TOKEN_PARTS, true>);
+    default: if constexpr (kMost == 6) return launch(imported_tile_fp8_kernel<6, PARTS, TOKEN_PARTS, true>);
   }
 }
 

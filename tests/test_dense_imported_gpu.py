@@ -175,7 +175,8 @@ def test_matrix_core_batch_matches_the_oracle(capi, oracle):
 
 
 @pytest.mark.parametrize("cols,rows,tokens", [(128, 8200, 9), (5120, 8210, 32), (6144, 8192, 17), (7168, 8200, 32),
-                                              (4096, 100, 16), (6144, 33, 32), (9216, 130, 31)])
+                                              (4096, 100, 16), (6144, 33, 32), (9216, 130, 31), (5120, 130, 16),
+                                              (4608, 65, 32), (6144, 200, 9)])
 def test_fp8_tiles_match_float64_products(capi, cols, rows, tokens):
     """More than eight tokens of FP8 matrices: workgroups that walk over tiles of 16 rows
     (8192 rows and more) or of 32, with one pass over the columns or several, partial
