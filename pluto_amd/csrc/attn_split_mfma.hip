@@ -192,6 +192,32 @@ split_forward_kernel(SplitArgs a) {
 #pragma unroll
   for (int db = 0; db < DB; ++db) o[db] = zero16();
   float running_max = kMasked, running_sum = 0.0f;  // of the scaled scores
+  // scores to weights; register i = (key k0 + 8(i/4) + 4h + i%4, query n)
+  auto softmax = [&](floatx16& s, int k0) {
+    const int limit = query_load - k0 - 4 * h;
+    float tile_max = kMasked;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = 8 * (i / 4) + (i % 4) > limit ? kMasked : s[i] * a.scale;
+      tile_max = fmaxf(tile_max, s[i]);
+    }
+    const float new_max = fmaxf(running_max, half_swap_max(tile_max));
+    const float correction = __builtin_amdgcn_exp2f((running_max - new_max) * kLog2e);
+    running_max = new_max;
+    float tile_sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = s[i] == kMasked ? 0.0f : __builtin_amdgcn_exp2f((s[i] - new_max) * kLog2e);
+      tile_sum += s[i];
+    }
+    running_sum = running_sum * correction + half_swap_sum(tile_sum);
+    if (__any(correction != 1.0f)) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[db][i] *= correction;
+    }
+  };
   for (int step = 0; step < w.steps; ++step) {
     const int k0 = (2 * step + w.parity) * kRows;
     stage_ready();
@@ -221,30 +247,7 @@ split_forward_kernel(SplitArgs a) {
     vt[0] = at.transposed(v_tile, 0, 0);
     vt[1] = at.transposed(v_tile, 1, 0);
     fence_schedule();
-    // register i = (key k0 + 8(i/4) + 4h + i%4, query n)
-    const int limit = query_load - k0 - 4 * h;
-    float tile_max = kMasked;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s[i] = 8 * (i / 4) + (i % 4) > limit ? kMasked : s[i] * a.scale;
-      tile_max = fmaxf(tile_max, s[i]);
-    }
-    const float new_max = fmaxf(running_max, half_swap_max(tile_max));
-    const float correction = __builtin_amdgcn_exp2f((running_max - new_max) * kLog2e);
-    running_max = new_max;
-    float tile_sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s[i] = s[i] == kMasked ? 0.0f : __builtin_amdgcn_exp2f((s[i] - new_max) * kLog2e);
-      tile_sum += s[i];
-    }
-    running_sum = running_sum * correction + half_swap_sum(tile_sum);
-    if (__any(correction != 1.0f)) {
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[db][i] *= correction;
-    }
+    softmax(s, k0);
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
       const Pieces p = split_accumulator(s, s2);
@@ -260,6 +263,38 @@ split_forward_kernel(SplitArgs a) {
             vt[(at_step + 2) % 3] = at.transposed(v_tile, (at_step + 2) % DB, (at_step + 2) / DB);
           if (part == 1 && at_step < 2 * kLoads) fill.request(step + 1, 2 * kLoads + at_step);
         }
+      }
+    }
+  }
+  if (__any(!all_finite(o) || running_sum != running_sum)) [[unlikely]] {
+    // An infinity in V by a weight in pieces is NaN (a piece may be zero or negative), by the
+    // weight it is the infinity: the wave's tiles again, straight from memory, the weights
+    // as they are.  (The scores' factors are bf16: no pieces.)
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o[db] = zero16();
+    running_max = kMasked, running_sum = 0.0f;
+    const long long kv_row = 1LL * (a.heads / a.group) * D;
+    for (int k0 = w.parity * kRows; k0 <= w.first_query + 31 && k0 < T; k0 += 2 * kRows) {
+      const long long tile = k0 * kv_row + head / a.group * D;
+      const int rows = T - k0;  // those beyond count as zero
+      floatx16 s = zero16();
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const uint4 key = *reinterpret_cast<const uint4*>(a.k + tile + (n < rows ? n : 0) * kv_row + 16 * ks + 8 * h);
+        const uint4 q = *reinterpret_cast<const uint4*>(a.q + query_load * q_row + head * D + 16 * ks + 8 * h);
+        s = mfma32(as_bf16x8(n < rows ? key : make_uint4(0, 0, 0, 0)), as_bf16x8(q), s);
+      }
+      softmax(s, k0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = 8 * (i / 4) + 4 * h + i % 4;
+        const uint16_t* values = a.v + tile + (row < rows ? row : 0) * kv_row + n;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          const float value = bf16_bits_to_float(values[32 * db]);
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(row < rows ? value : 0.0f, s[i], o[db], 0, 0, 0);
+        }
+        fence_schedule();
       }
     }
   }

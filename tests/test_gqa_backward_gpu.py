@@ -256,6 +256,36 @@ def test_saved_block_can_be_moved(capi, T, qh, kh, d, rot):
             assert np.array_equal(value.cpu().numpy(), got[name]), (name, filled_at, read_at)
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("T", [33, 130])
+def test_saved_forward_with_non_finite_values(capi, T, bad):
+    """Head width 256: the forward that fills the block gives the numbers (to the 2^-9 of the
+    other's bf16 weights), infinities and NaNs that it gives without the block, and the
+    block's output before the gate the same."""
+    qh, kh, d = 4, 2, 256
+    p = capi.attention_params(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=64, capacity=T,
+                              round_to_bfloat16=True)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    qg = torch.randn((T, qh, 2, d), generator=gen, device="cuda").to(torch.bfloat16)
+    k, v = (torch.randn((T, kh, d), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    v[T // 2, 1, 5] = bad
+    w = torch.zeros(d, device="cuda")
+    cache = capi.KvCache(T, kh, d)
+    saved = capi.gqa_prefill_saved(p, T, cache)
+    got = capi.gqa_prefill(p, qg, k, v, w, w, cache, saved=saved)
+    assert capi.last_path() == capi.PATH_MATRIX_F32
+    want = capi.gqa_prefill(p, qg, k, v, w, w, cache)
+    torch.cuda.synchronize()
+    core = saved[:T * qh * d * 4].view(torch.float32).view(T, qh, d)
+    a, b = got.double(), want.double()
+    assert torch.equal(a.isnan(), b.isnan())
+    assert torch.equal(torch.where(a.isinf(), a, 0), torch.where(b.isinf(), b, 0))
+    assert torch.equal(core.isnan(), b.isnan()) and torch.equal(core.isinf(), b.isinf())
+    finite = b.isfinite()
+    a, b = torch.where(finite, a, 0), torch.where(finite, b, 0)
+    assert ((a - b).norm(dim=-1) <= 1e-2 * b.norm(dim=-1)).all()
+
+
 def test_saved_block_off_a_word_is_refused_at_head_width_256(capi):
     T, qh, kh, d = 33, 2, 1, 256
     p = capi.attention_params(query_heads=qh, key_value_heads=kh, head_dim=d, rotary_dim=64, capacity=T,
