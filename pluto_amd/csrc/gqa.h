@@ -28,7 +28,7 @@ struct PrefillPrepareArgs {
   void* q_out = nullptr;  // [T, qh, d], bf16 when rounding, else fp32
   int q_out_dtype = PLUTO_HIP_BF16;
   CacheView cache;
-  // optional second copies for the backward pass, 16-byte aligned: the prepared queries
+  // optional second copies for the backward pass, in one block with the table: the prepared queries
   // [T, qh, d] as q_out, keys and values [T, kh, d] in the cache's storage
   void* q_copy = nullptr;
   void* k_copy = nullptr;

@@ -202,8 +202,8 @@ long long decode_blocks_bound(const pluto_hip_attention_params* p, int batch, co
 // head width 256, where the backward's kernels take FP32 factors, also what the
 // preparation made: the normalised and rotated heads (bf16) and the rotation's table.  At
 // 64 and 128 they are made again: with them the block is 119 instead of 52 MB at 8192 rows
-// of 24 + 4 heads of 128, held for every layer between the passes, for 1.6 % of the
-// training step (1784 instead of 1812 us).
+// of 24 + 4 heads of 128, held for every layer between the passes, for 1.9 % of the
+// training step (1726 instead of 1759 us).
 struct SavedLayout {
   size_t core, maxima, normalizers, queries, keys, values, cosines, sines, total;
 };

@@ -306,3 +306,30 @@ def test_rejects_bad_arguments(capi):
     rc = lib.pluto_hip_gdn_layer_backward(capi.current_stream(), ctypes.byref(p), 1, 5, None,
                                           *ptrs[1:], None, None, None, None, capi.ptr(x), size)
     assert rc != 0  # null input
+
+
+def test_values_near_the_top_of_the_range_stay_finite(capi):
+    """A value between bf16's largest number and FP32's (2^128 - 2^120 to 2^128) rounds to an
+    infinity in bf16: the matrix cores' pieces of it must still add up to it."""
+    T, kh, vh = 200, 1, 2
+    c = make_case(T, kh, vh, 128, 128, 4, seed=3)
+    channel = 2 * kh * 128 + 5
+    c["conv"][channel] = [0, 0, 0, 1.003]
+    c["qkv"][0, :, channel] = 0
+    c["qkv"][0, 100, channel] = 2.0 ** 128 - 2.0 ** 120  # 3.4e38 after the convolution
+    c["b"][0, 100, 0] = 60  # and as the state's change
+    # decaying slowly the state keeps the outputs so large that their norm's inverse is zero
+    c["a_log"][:], c["dt_bias"][:] = 0, -3
+    p = capi.delta_params(key_heads=kh, value_heads=vh, key_head_dim=128, value_head_dim=128, conv_kernel_dim=4,
+                          round_to_bfloat16=False)
+    bf = torch.bfloat16
+    args = (p, dev(c["qkv"], bf), dev(c["z"], bf), dev(c["a"], bf), dev(c["b"], bf), dev(c["conv"]),
+            dev(c["a_log"]), dev(c["dt_bias"]), dev(c["norm"]), dev(c["dy"]))
+    got = capi.gdn_layer_backward(*args)
+    with capi.force_generic():
+        want = capi.gdn_layer_backward(*args)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dqkv", "dz", "da", "db"), got, want):
+        a, b = a.cpu().numpy(), b.cpu().numpy()
+        assert np.isfinite(b).all() and np.isfinite(a).all(), name
+        assert_close(a, b, 2e-4, name)  # the tolerance against the oracle
