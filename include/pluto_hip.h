@@ -243,7 +243,7 @@ int pluto_hip_gqa_prefill(void* stream, const pluto_hip_attention_params* p,
  *   dy       fp32 [length, qh, d]     gradient of the layer output
  *   saved    optional: the block pluto_hip_gqa_prefill filled for the same
  *            inputs and parameters; the attention forward (at head_dim 256 the
- *            preparation too) is then not repeated, a quarter of the call at
+ *            preparation too) is then not repeated, a fifth of the call at
  *            length 8192 of head_dim 128.  NULL recomputes.
  *   dqg      fp32 [length, qh, 2, d]  query gradients at [..,0,:], gate at [..,1,:]
  *   dk, dv   fp32 [length, kh, d]

@@ -6,6 +6,8 @@
 // take 192 cycles where the FP32 instruction needs 512 for the same depth, six
 // v_mfma_f32_16x16x32_bf16 96 where it needs 256; making the pieces costs 44 cycles of
 // vector instructions a pair of numbers.
+// An infinity has no such pieces, and a number from 2^128 - 2^119 on, which rounds to one, not
+// by rounding alone: what the kernels do about them stands beside them.
 #pragma once
 
 #include "mfma_tile.h"
