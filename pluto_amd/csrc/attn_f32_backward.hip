@@ -15,10 +15,10 @@
 //
 // Of a call, us, on the FP32 matrix instructions and now: 4 sequences x 12 heads x 256 x 64
 // 37.7, 25.0 (dq 11.6, dkv 15.2); 16 x 12 x 512 x 64 285, 194 (88, 117); 4 x 12 x 256 x 32
-// 21.9, 16.9; 8 x 12 x 512 x 32 74, 61; 4 x 6 x 256 x 128 53.4, 34.5; 8 x 6 x 512 x 128 191,
-// 146 (64, 86).  D = 128 leaves room for one workgroup a compute unit and takes 1.4 times
-// what D = 64 does for as much work; having the other arithmetic at hand (attn_f32_split.h)
-// costs it 2 %, its registers being all taken, the others nothing.  Small calls are bound by the
+// 21.9, 17.0; 8 x 12 x 512 x 32 74, 62; 4 x 6 x 256 x 128 53.4, 33.6; 8 x 6 x 512 x 128 191,
+// 143 (63, 83).  D = 128 leaves room for one workgroup a compute unit and takes 1.4 times
+// what D = 64 does for as much work.  Having the other arithmetic at hand (attn_f32_split.h)
+// costs 0.1 to 0.2 us of a small call.  Small calls are bound by the
 // chain of a wave (its first tile's way from memory, the pieces, two products after each
 // other, the merge: 7 us with one tile), large ones by streaming every tile once for 32
 // rows.  Against 64-bit arithmetic the gradients are 2.4e-7 off for standard normal
@@ -148,6 +148,7 @@ __device__ __forceinline__ void f32_dq(const GenericBackwardArgs& a, const F32Un
 
   auto walk = [&](auto pieces) {
     constexpr bool PIECES = decltype(pieces)::value;
+    const int lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;  // ranges the addresses need to share bases
     for (int kt = wave; kt < key_tiles; kt += kWaves) {
       const int k0 = kt * 32;
       floatx16 s, dp;
@@ -267,6 +268,7 @@ __device__ __forceinline__ void f32_dkv(const GenericBackwardArgs& a, const F32U
   __syncthreads();
   auto walk = [&](auto pieces) {
     constexpr bool PIECES = decltype(pieces)::value;
+    const int lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;  // ranges the addresses need to share bases
     for (int qt = k0 / 32 + wave; qt < query_tiles; qt += kWaves) {
       const int q0 = qt * 32;
       if (h == 0) {

@@ -11,7 +11,7 @@
 // works on the ones it has.  Of a call, us, on the FP32 matrix instructions and now:
 // 4 sequences x 12 heads x 256 x 64 12.1, 10.0; 16 x 12 x 512 x 64 86, 71-75; 4 x 12 x 256 x
 // 32 8.3, 7.5; 8 x 12 x 512 x 32 25.6, 24.0; 4 x 6 x 256 x 128 17.5, 15.7; 8 x 6 x 512 x 128
-// 57.7, 52.8 (looking at the results costs 0.2 us of a small call).  Outputs 1.7e-7 off
+// 57.7, 52.2 (looking at the results costs 0.2 us of a small call).  Outputs 1.7e-7 off
 // 64-bit arithmetic for standard normal inputs, 2.2e-7 with those instructions.  As in
 // the bf16 kernels the products are transposed,
 // S^T = K Q^T and O^T = V^T P^T, so that a lane owns one query column: its row
@@ -86,6 +86,7 @@ f32_forward_kernel(GenericForwardArgs a) {
   const int last_key = min(a.start_position + query, a.kv_rows - 1);  // keys beyond it are masked
   auto walk = [&](auto pieces) {
     constexpr bool PIECES = decltype(pieces)::value;
+    const int lane = threadIdx.x % 64, h = lane / 32;  // ranges the addresses need to share bases
     for (int kt = wave; kt < key_tiles; kt += kKeySplit) {
       const int k0 = kt * 32;
       floatx16 s;
