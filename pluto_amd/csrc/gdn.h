@@ -42,8 +42,22 @@ struct GdnArgs {
   float q_scale = 1.0f;
 };
 
+// The layer's inputs in front of the chunked scan: GdnArgs' q, k and v are then where the
+// preparation leaves the convolved rows (bf16, all of one stride), its gates are unused.
+struct GdnLayerInputs {
+  const uint16_t* qkv = nullptr;  // bf16 [batch, T, channels], the stride of q, k and v
+  const uint16_t* a = nullptr;    // bf16 [batch, T, vh]
+  const uint16_t* b = nullptr;
+  const float* conv_weight = nullptr;  // [channels, 4]
+  const float* a_log = nullptr;
+  const float* dt_bias = nullptr;
+};
+
 bool gdn_chunked_supported(const GdnArgs& args, int chunk);
-int launch_gdn_chunked(hipStream_t stream, const GdnArgs& args);
+// layer: null where q, k, v and the gates are there already
+int launch_gdn_chunked(hipStream_t stream, const GdnArgs& args, const GdnLayerInputs* layer = nullptr);
+// Whether the chunk preparation can take over the convolution and the gates.
+bool gdn_layer_rows_supported(const GdnLayerInputs& layer, int taps);
 int launch_gdn_recurrence(hipStream_t stream, const GdnArgs& args, int out_dtype);
 
 // Layer-level pieces around the scan (gdn_layer.hip).

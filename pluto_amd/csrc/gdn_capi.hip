@@ -152,12 +152,6 @@ int pluto_hip_gdn_layer_forward(void* stream, const pluto_hip_delta_params* p, i
   float* log_decay = reinterpret_cast<float*>(scratch + layout.log_decay);
   float* beta = reinterpret_cast<float*>(scratch + layout.beta);
   void* core = scratch + layout.core;
-  status = launch_gdn_conv_sequence(s, qkv, PLUTO_HIP_BF16, conv_weight, batch, length, channels,
-                                    p->conv_kernel_dim, round, post, mid_dtype);
-  if (status != 0) return status;
-  status = launch_gdn_gates(s, a, b, PLUTO_HIP_BF16, a_log, dt_bias, tokens, vh, round,
-                            log_decay, beta);
-  if (status != 0) return status;
   const size_t element = round ? 2 : 4;
   GdnArgs g;
   g.q = static_cast<const uint16_t*>(post);
@@ -182,10 +176,23 @@ int pluto_hip_gdn_layer_forward(void* stream, const pluto_hip_delta_params* p, i
   g.q_scale = 1.0f / std::sqrt(static_cast<float>(kd));
   const bool chunked = round && !force_generic() && gdn_chunked_supported(g, 64);
   note_path(chunked ? PLUTO_HIP_PATH_CHUNKED : PLUTO_HIP_PATH_RECURRENCE);
-  if (chunked)
-    status = launch_gdn_chunked(s, g);
-  else
-    status = launch_gdn_recurrence(s, g, mid_dtype);
+  GdnLayerInputs layer;
+  layer.qkv = static_cast<const uint16_t*>(qkv);
+  layer.a = static_cast<const uint16_t*>(a);
+  layer.b = static_cast<const uint16_t*>(b);
+  layer.conv_weight = conv_weight;
+  layer.a_log = a_log;
+  layer.dt_bias = dt_bias;
+  if (chunked && gdn_layer_rows_supported(layer, p->conv_kernel_dim)) {
+    status = launch_gdn_chunked(s, g, &layer);
+  } else {
+    status = launch_gdn_conv_sequence(s, qkv, PLUTO_HIP_BF16, conv_weight, batch, length, channels,
+                                      p->conv_kernel_dim, round, post, mid_dtype);
+    if (status != 0) return status;
+    status = launch_gdn_gates(s, a, b, PLUTO_HIP_BF16, a_log, dt_bias, tokens, vh, round, log_decay, beta);
+    if (status != 0) return status;
+    status = chunked ? launch_gdn_chunked(s, g) : launch_gdn_recurrence(s, g, mid_dtype);
+  }
   if (status != 0) return status;
   return launch_gdn_output(s, core, mid_dtype, z, PLUTO_HIP_BF16, norm, tokens * vh, vd,
                            p->rms_norm_epsilon, round, out, PLUTO_HIP_BF16);

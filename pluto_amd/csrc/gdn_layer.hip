@@ -4,6 +4,7 @@
 // the reference is kept (src/llm/layers/sequence_delta_net.cc:31-51,88-96,
 // 104-121 and src/llm/layers/util/cached_attention_ops.cc:180-203,253-272).
 #include "gdn.h"
+#include "gdn_activation.h"
 #include "mfma_tile.h"
 
 namespace pluto_hip {
@@ -31,18 +32,6 @@ conv_sequence_kernel(const void* input, int in_dtype, const float* __restrict__ 
   }
   sum = maybe_round(sum, round);
   store_element(post, i, post_dtype, maybe_round(sum / (1.0f + expf(-sum)), round));
-}
-
-// x / (1 + exp(-x)) from the hardware's exponential and reciprocal, with the correction
-// and the last instruction of a division, which restores what the others make of
-// infinities.  The uncorrected product rounds 5.9375, whose value lies next to a tie, to the
-// wrong bf16 (0.1 % of the activations where inputs have four times unit size: states 2 %
-// further from the specification); with it every bf16 argument above -87 rounds as with
-// expf and a division.
-__device__ inline float silu(float x) {
-  const float d = 1.0f + __builtin_amdgcn_exp2f(-x * kLog2e);
-  const float inverse = __builtin_amdgcn_rcpf(d), y = x * inverse;
-  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-y, d, x), inverse, y), d, x);
 }
 
 // Eight bf16 of a 16-byte piece as floats.
@@ -94,18 +83,12 @@ conv_rows_kernel(const uint16_t* __restrict__ input, const float* __restrict__ w
       uint32_t packed[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float value[2];
+        float taps[2][4];
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int e = 2 * i + k;
-          float sum = 0.0f;
+        for (int k = 0; k < 2; ++k)
 #pragma unroll
-          for (int tap = 0; tap < 4; ++tap) sum += x[tap][e] * w[e][tap];
-          value[k] = sum;
-        }
-        const uint32_t sums = pack_bf16(value[0], value[1]);
-        const float first = __uint_as_float(sums << 16), second = __uint_as_float(sums & 0xffff0000u);
-        packed[i] = pack_bf16(silu(first), silu(second));
+          for (int tap = 0; tap < 4; ++tap) taps[k][tap] = x[tap][2 * i + k];
+        packed[i] = convolved_pair(taps[0], w[2 * i], taps[1], w[2 * i + 1]);
       }
       if (base + j < rows)
         *reinterpret_cast<uint4*>(out + static_cast<long long>(base + j) * channels) =
@@ -152,11 +135,8 @@ gates_kernel(const void* a, const void* b, int in_dtype, const float* __restrict
   const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= rows * heads) return;
   const int head = static_cast<int>(i % heads);
-  const float alpha = load_element(a, i, in_dtype) + dt_bias[head];
-  // stable softplus: no overflow for strongly positive time steps
-  const float softplus = fmaxf(alpha, 0.0f) + log1pf(expf(-fabsf(alpha)));
-  log_decay[i] = -expf(a_log[head]) * softplus;
-  beta[i] = maybe_round(1.0f / (1.0f + expf(-load_element(b, i, in_dtype))), round);
+  log_decay[i] = log_decay_of(load_element(a, i, in_dtype) + dt_bias[head], a_log[head]);
+  beta[i] = maybe_round(beta_of(load_element(b, i, in_dtype)), round);
 }
 
 // One wave per (token, head) row of value_dim <= 256 channels.

@@ -21,7 +21,8 @@
 // Kernel 1 (gdn_chunk_prepare, one workgroup per chunk, fully parallel): the
 // two Gram matrices on the matrix cores from the raw bf16 inputs, T by a block
 // forward substitution on the matrix cores, and 14 KiB per chunk written out:
-// T and M o (Q K^T) as bf16 matrix-core operands, and the per-token factors.
+// T and M o (Q K^T) as bf16 matrix-core operands, and the per-token factors.  For the layer
+// it also makes the rows of K, Q and V from the layer's inputs.
 // Kernel 2 (gdn_chunk_scan, one workgroup per (sequence, head, 16 state
 // columns)): walks the chunks with v_mfma_f32_16x16x32_bf16, the state in FP32
 // accumulator registers of one wave, a second wave computing the outputs, two
@@ -29,6 +30,7 @@
 // State columns are independent, which is what gives the sequential part
 // 8 x batch x heads way parallelism.
 #include "gdn.h"
+#include "gdn_activation.h"
 
 #include <type_traits>
 
@@ -70,27 +72,50 @@ __device__ inline bf16x8 tiles_to_operand(const floatx4& lo, const floatx4& hi) 
 // bf16(v - hi).
 __device__ inline void split_operand(const floatx4& first, const floatx4& second, bf16x8& hi,
                                      bf16x8& lo) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float v = e < 4 ? first[e] : second[e - 4];
-    const __bf16 h = static_cast<__bf16>(v);
-    hi[e] = h;
-    lo[e] = static_cast<__bf16>(v - static_cast<float>(h));
-  }
-}
-
-// Sum of the squares of eight bf16 numbers, and of sixteen neighbouring lanes' values.
-__device__ inline float squares(const uint4& v) {
-  const uint32_t words[4] = {v.x, v.y, v.z, v.w};
-  float even = 0.0f, odd = 0.0f;
+  uint32_t high[4], low[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
+    const floatx4& from = i < 2 ? first : second;
+    const float v0 = from[2 * (i % 2)], v1 = from[2 * (i % 2) + 1];
+    high[i] = pack_bf16(v0, v1);
+    low[i] = pack_bf16(v0 - __uint_as_float(high[i] << 16), v1 - __uint_as_float(high[i] & 0xffff0000u));
+  }
+  hi = bits_to_bf16x8(make_uint4(high[0], high[1], high[2], high[3]));
+  lo = bits_to_bf16x8(make_uint4(low[0], low[1], low[2], low[3]));
+}
+
+// One tile so, and the product of two of sixteen contraction elements.
+struct SplitTile {
+  shortx4 hi, lo;
+};
+__device__ inline SplitTile split_operand(const floatx4& v) {
+  const uint32_t high[2] = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+  uint32_t low[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    low[i] = pack_bf16(v[2 * i] - __uint_as_float(high[i] << 16), v[2 * i + 1] - __uint_as_float(high[i] & 0xffff0000u));
+  return {__builtin_bit_cast(shortx4, make_uint2(high[0], high[1])), __builtin_bit_cast(shortx4, make_uint2(low[0], low[1]))};
+}
+__device__ inline floatx4 product16(const SplitTile& a, const SplitTile& b, floatx4 c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.hi, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.lo, b.hi, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.lo, c, 0, 0, 0);
+}
+
+// Sum of the squares of eight or four bf16 numbers, and of sixteen neighbouring lanes' values.
+template <int WORDS>
+__device__ inline float squares(const uint32_t (&words)[WORDS]) {
+  float even = 0.0f, odd = 0.0f;
+#pragma unroll
+  for (int i = 0; i < WORDS; ++i) {
     const float low = __uint_as_float(words[i] << 16), high = __uint_as_float(words[i] & 0xffff0000u);
     even += low * low;
     odd += high * high;
   }
   return even + odd;
 }
+__device__ inline float squares(const uint4& v) { return squares<4>({v.x, v.y, v.z, v.w}); }
+__device__ inline float squares(const uint2& v) { return squares<2>({v.x, v.y}); }
 __device__ inline float row_sum(float v) {
   auto step = [&](auto control) {
     v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(control)::value, 0xf, 0xf, true));
@@ -102,42 +127,133 @@ __device__ inline float row_sum(float v) {
   return v;
 }
 
-// 35 KiB, so that four workgroups share a compute unit's LDS (the kernel is a
-// chain of short, barrier-separated phases and lives on occupancy): once the
-// Gram matrices are done the rows of K make room for A, and A in turn for the
-// finished inverse; the rows of Q make room for the second bf16 result.
+// Once the Gram matrices are done the rows of K and Q make room for A, and A in turn for
+// the finished inverse.  The kernel is a chain of short, barrier-separated phases and lives on
+// occupancy: 35 KiB for one head, four workgroups of four waves a compute unit; 80 KiB for
+// three, two of twelve waves.
+template <int HEADS>
 struct ChunkSmem {
-  union {
-    uint16_t k[C][DK + 8];  // raw K rows (bf16)
-    float a[C][C + 4];      // then: strictly lower triangular A (FP32) and the blocks of its solve
-    uint16_t t[C][C + 8];   // last: (I + A)^-1, bf16
-  };
-  union {
-    uint16_t q[C][DK + 8];  // raw Q rows
-    uint16_t a2[C][C + 8];  // later: M o (Q K^T) with all factors, bf16
-  };
-  float cum[C];             // inclusive cumulative log decay
-  float beta[C];
+  using Rows = uint16_t[C][DK + 8];     // raw K or Q rows (bf16)
+  using Square = float[C][C + 4];       // strictly lower triangular A (FP32) and the blocks of its solve
+  using Operand = uint16_t[C][C + 8];   // (I + A)^-1; M o (Q K^T) with all factors: bf16
+  static_assert(sizeof(Rows) == sizeof(Square) && sizeof(Operand) <= sizeof(Rows));
+  unsigned char blocks[HEADS < 2 ? 2 : HEADS][sizeof(Rows)];
+  unsigned char products[HEADS < 2 ? 0 : HEADS][sizeof(Operand)];
+  float cum[HEADS][C];      // inclusive cumulative log decay
+  float beta[HEADS][C];
   float inv_k[C];           // 1/|k| (or 1)
   float q_factor[C];        // q_scale / |q| (or q_scale)
+  __device__ Rows& k() { return *reinterpret_cast<Rows*>(blocks[0]); }
+  __device__ Rows& q() { return *reinterpret_cast<Rows*>(blocks[1]); }
+  __device__ Square& a(int head) { return *reinterpret_cast<Square*>(blocks[head]); }
+  __device__ Operand& t(int head) { return *reinterpret_cast<Operand*>(blocks[head]); }
+  __device__ Operand& a2(int head) {
+    return *reinterpret_cast<Operand*>(HEADS < 2 ? blocks[1] : products[head]);
+  }
 };
 
-__global__ void __launch_bounds__(256)
-gdn_chunk_prepare(GdnArgs a) {
-  __shared__ __attribute__((aligned(16))) ChunkSmem sm;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+// One head's 128 channels of a chunk through the convolution and SiLU, four channels and
+// eight rows a thread of 256.  The rows go to memory, where the sequential kernel reads
+// them, and to LDS with zeros beyond the sequence, the sums of their squares to `use_square`.
+template <typename UseSquare>
+__device__ inline void convolve_head(const uint16_t* in, const float* weight, uint16_t* out, long long stride,
+                                     int t0, int valid, int tid, bool store, uint16_t (*rows)[DK + 8],
+                                     UseSquare&& use_square) {
+  constexpr int kRun = 8;
+  const int c0 = 4 * (tid % 32), first = tid / 32 * kRun;
+  uint2 raw[kRun + 3];
+#pragma unroll
+  for (int j = 0; j < kRun + 3; ++j) {
+    // rows behind the sequence are not used, those before it are zero
+    raw[j] = *reinterpret_cast<const uint2*>(in + min(max(first + j - 3, -t0), valid - 1) * stride + c0);
+    if (j < 3 && t0 + first + j < 3) raw[j] = make_uint2(0, 0);
+  }
+  float w[4][4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float4 v = *reinterpret_cast<const float4*>(weight + 4 * (c0 + e));
+    w[e][0] = v.x, w[e][1] = v.y, w[e][2] = v.z, w[e][3] = v.w;
+  }
+#pragma unroll
+  for (int j = 0; j < kRun; ++j) {
+    float x[4][4];  // channel, tap
+#pragma unroll
+    for (int tap = 0; tap < 4; ++tap) {
+      x[0][tap] = __uint_as_float(raw[j + tap].x << 16), x[1][tap] = __uint_as_float(raw[j + tap].x & 0xffff0000u);
+      x[2][tap] = __uint_as_float(raw[j + tap].y << 16), x[3][tap] = __uint_as_float(raw[j + tap].y & 0xffff0000u);
+    }
+    const int row = first + j;
+    const uint2 post = make_uint2(convolved_pair(x[0], w[0], x[1], w[1]), convolved_pair(x[2], w[2], x[3], w[3]));
+    if (store && row < valid) *reinterpret_cast<uint2*>(out + row * stride + c0) = post;
+    if (rows) {
+      *reinterpret_cast<uint2*>(&rows[row][c0]) = post;
+      float square = row_sum(squares(post));
+      square += __shfl_xor(square, 16, 64);
+      if (tid % 32 == 0) use_square(row, row < valid ? square : 0.0f);
+    }
+  }
+  if (rows && valid < C) {
+#pragma unroll
+    for (int j = 0; j < kRun; ++j)
+      if (first + j >= valid) *reinterpret_cast<uint2*>(&rows[first + j][c0]) = make_uint2(0, 0);
+  }
+}
+
+// A workgroup of 256 HEADS threads prepares a chunk for HEADS value heads of one key head.
+// LAYER: from the layer's inputs; the rows of K and Q are convolved once for the heads of a
+// workgroup, and every head's V on the way.  8191 tokens of 16/48 heads: 112 us for 427 MB;
+// as passes of their own the convolution took 67, the gates 5 and the preparation 63, of 16/16
+// heads 57 and 43 + 5 + 27.  Vector instructions are 60 % of it (42 million; 50 with an
+// activation that carries a division's correction, factors rounded one by one, zeros in the
+// operands of the solve and every wave substituting its own block).
+template <int HEADS, bool LAYER>
+__global__ void __launch_bounds__(256 * HEADS)
+__attribute__((amdgpu_waves_per_eu(HEADS == 3 ? 6 : 4)))
+gdn_chunk_prepare(GdnArgs a, GdnLayerInputs layer) {
+  __shared__ __attribute__((aligned(16))) ChunkSmem<HEADS> sm;
+  const int local = HEADS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / 256);  // of the workgroup's heads
+  const int tid = threadIdx.x % 256, wave = tid / 64, lane = tid % 64;
   const int chunks = (a.length + C - 1) / C;
-  const int chunk = blockIdx.x % chunks;
-  const int bh = blockIdx.x / chunks;            // sequence * value_heads + head
-  const int head = bh % a.value_heads, seq = bh / a.value_heads;
-  const int key_head = head / (a.value_heads / a.key_heads);
+  const int group = a.value_heads / a.key_heads, parts = group / HEADS;
+  // chunks of a head after each other; LAYER: heads of a chunk, neighbouring columns of its rows
+  const int unit = LAYER ? blockIdx.x % (a.key_heads * parts) : blockIdx.x / chunks % a.value_heads;
+  const int chunk = LAYER ? blockIdx.x / (a.key_heads * parts) % chunks : blockIdx.x % chunks;
+  const int seq = blockIdx.x / (a.key_heads * parts) / chunks;
+  const int head = HEADS * unit + local, key_head = unit / parts, part = unit % parts;
+  const int bh = seq * a.value_heads + head;
   const int t0 = chunk * C;
   const int valid = min(C, a.length - t0);
+  const long long token0 = static_cast<long long>(seq) * a.length + t0;
+  uint16_t(&sm_k)[C][DK + 8] = sm.k(), (&sm_q)[C][DK + 8] = sm.q();
+  float(&sm_a)[C][C + 4] = sm.a(local);
+  uint16_t(&sm_t)[C][C + 8] = sm.t(local), (&sm_a2)[C][C + 8] = sm.a2(local);
+  float(&sm_cum)[C] = sm.cum[local], (&sm_beta)[C] = sm.beta[local];
 
-  // ---- stage K and Q rows (16-byte pieces), zero beyond the sequence --------
-  // Sixteen lanes hold a row and add up its squares as it arrives (read back from LDS
-  // one channel at a time, four lanes a row: 83 us at 8191 tokens of 48 heads, 78 so).
-  {
+  // sequence_delta_net.cc:84-85: x * rsqrt(sum(x^2) + 1e-6)
+  auto use_k = [&](int row, float square) { sm.inv_k[row] = a.normalize_qk ? rsqrtf(square + 1e-6f) : 1.0f; };
+  auto use_q = [&](int row, float square) {
+    sm.q_factor[row] = a.normalize_qk ? a.q_scale * rsqrtf(square + 1e-6f) : a.q_scale;
+  };
+  // the convolution of a head's columns; `which` is the place of its rows in GdnArgs
+  auto convolve = [&](const uint16_t* which, int column, int thread, bool store, uint16_t (*rows)[DK + 8], auto&& use) {
+    const int at = static_cast<int>(which - a.q) + column;
+    convolve_head(layer.qkv + token0 * a.q_token_stride + at, layer.conv_weight + 4 * at,
+                  const_cast<uint16_t*>(a.q) + token0 * a.q_token_stride + at, a.q_token_stride, t0, valid, thread,
+                  store, rows, use);
+  };
+  // sixteen rows of a head's V
+  auto convolve_v = [&](int of, int quarter) {
+    convolve(a.v, (head - local + of) * DV, 64 * quarter + lane, true, nullptr, [](int, float) {});
+  };
+  if constexpr (LAYER) {
+    // the first head's waves have K, the second's Q, the third's its V
+    if (local == 0) convolve(a.k, key_head * DK, tid, part == 0, sm_k, use_k);
+    if (local == (HEADS == 1 ? 0 : 1)) convolve(a.q, key_head * DK, tid, part == 0, sm_q, use_q);
+    if (local == 2) convolve_v(2, wave);
+  } else {
+    // ---- stage K and Q rows (16-byte pieces), zero beyond the sequence --------
+    // Sixteen lanes hold a row and add up its squares as it arrives (read back from LDS
+    // one channel at a time, four lanes a row: 83 us at 8191 tokens of 48 heads, 78 so).
     constexpr int kLoads = C * (DK / 8) / 256;
     const int c8 = tid % (DK / 8);
     uint4 kb[kLoads], qb[kLoads];
@@ -146,38 +262,38 @@ gdn_chunk_prepare(GdnArgs a) {
       const int row = i * (256 / (DK / 8)) + tid / (DK / 8);
       kb[i] = qb[i] = make_uint4(0, 0, 0, 0);
       if (row < valid) {
-        const long long token = static_cast<long long>(seq) * a.length + t0 + row;
-        kb[i] = *reinterpret_cast<const uint4*>(a.k + token * a.k_token_stride + key_head * DK + 8 * c8);
-        qb[i] = *reinterpret_cast<const uint4*>(a.q + token * a.q_token_stride + key_head * DK + 8 * c8);
+        kb[i] = *reinterpret_cast<const uint4*>(a.k + (token0 + row) * a.k_token_stride + key_head * DK + 8 * c8);
+        qb[i] = *reinterpret_cast<const uint4*>(a.q + (token0 + row) * a.q_token_stride + key_head * DK + 8 * c8);
       }
     }
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int row = i * (256 / (DK / 8)) + tid / (DK / 8);
-      *reinterpret_cast<uint4*>(&sm.k[row][8 * c8]) = kb[i];
-      *reinterpret_cast<uint4*>(&sm.q[row][8 * c8]) = qb[i];
+      *reinterpret_cast<uint4*>(&sm_k[row][8 * c8]) = kb[i];
+      *reinterpret_cast<uint4*>(&sm_q[row][8 * c8]) = qb[i];
       const float kk = row_sum(squares(kb[i])), qq = row_sum(squares(qb[i]));
-      if (c8 == 0) {
-        // sequence_delta_net.cc:84-85: x * rsqrt(sum(x^2) + 1e-6)
-        sm.inv_k[row] = a.normalize_qk ? rsqrtf(kk + 1e-6f) : 1.0f;
-        sm.q_factor[row] = a.normalize_qk ? a.q_scale * rsqrtf(qq + 1e-6f) : a.q_scale;
-      }
+      if (c8 == 0) use_k(row, kk), use_q(row, qq);
     }
   }
-  if (wave == 0) {
+  if (wave == (local + 1) % 4) {
     float g = 0.0f, b = 0.0f;
     if (lane < valid) {
-      const long long at = (static_cast<long long>(seq) * a.length + t0 + lane) * a.value_heads + head;
-      g = a.log_decay[at];
-      b = a.beta[at];
+      const long long at = (token0 + lane) * a.value_heads + head;
+      if constexpr (LAYER) {
+        g = log_decay_of(bf16_bits_to_float(layer.a[at]) + layer.dt_bias[head], layer.a_log[head]);
+        b = round_to_bf16(beta_of(bf16_bits_to_float(layer.b[at])));
+      } else {
+        g = a.log_decay[at];
+        b = a.beta[at];
+      }
     }
     // inclusive prefix sum over the 64 lanes
     for (int offset = 1; offset < 64; offset <<= 1) {
       const float up = __shfl_up(g, offset, 64);
       if (lane >= offset) g += up;
     }
-    sm.cum[lane] = g;
-    sm.beta[lane] = b;
+    sm_cum[lane] = g;
+    sm_beta[lane] = b;
   }
   __syncthreads();
 
@@ -200,40 +316,44 @@ gdn_chunk_prepare(GdnArgs a) {
       }
 #pragma unroll
       for (int ks = 0; ks < DK / 16; ++ks) {
-        const bf16x8 kr = bits_to_bf16x8(*reinterpret_cast<const uint4*>(&sm.k[32 * ti + n][16 * ks + 8 * h]));
-        const bf16x8 qr = bits_to_bf16x8(*reinterpret_cast<const uint4*>(&sm.q[32 * ti + n][16 * ks + 8 * h]));
-        const bf16x8 kc = bits_to_bf16x8(*reinterpret_cast<const uint4*>(&sm.k[32 * tj + n][16 * ks + 8 * h]));
+        const bf16x8 kr = bits_to_bf16x8(*reinterpret_cast<const uint4*>(&sm_k[32 * ti + n][16 * ks + 8 * h]));
+        const bf16x8 qr = bits_to_bf16x8(*reinterpret_cast<const uint4*>(&sm_q[32 * ti + n][16 * ks + 8 * h]));
+        const bf16x8 kc = bits_to_bf16x8(*reinterpret_cast<const uint4*>(&sm_k[32 * tj + n][16 * ks + 8 * h]));
         gk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kr, kc, gk, 0, 0, 0);
         gq = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qr, kc, gq, 0, 0, 0);
       }
       const int col = 32 * tj + n;  // token j
-      const float cum_j = sm.cum[col], inv_kj = sm.inv_k[col];
+      const float cum_j = sm_cum[col], inv_kj = sm.inv_k[col];
       // four rows a register quad; values are chosen, not branched around: a branch with
       // a read of LDS in it for each of 32 elements took 7400 of the kernel's 21000 cycles
       // (78 us; 70 so)
+      const int above = col - 32 * ti - 4 * h;  // of the lane's first row
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int row0 = 32 * ti + 8 * j + 4 * h;  // token i
-        const floatx4 cum = *reinterpret_cast<const floatx4*>(&sm.cum[row0]),
-                      beta = *reinterpret_cast<const floatx4*>(&sm.beta[row0]),
+        const floatx4 cum = *reinterpret_cast<const floatx4*>(&sm_cum[row0]),
+                      beta = *reinterpret_cast<const floatx4*>(&sm_beta[row0]),
                       inv_k = *reinterpret_cast<const floatx4*>(&sm.inv_k[row0]),
                       q_factor = *reinterpret_cast<const floatx4*>(&sm.q_factor[row0]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float decay = __expf(fminf(cum[e] - cum_j, 0.0f));
-          float k = beta[e] * decay * inv_k[e] * inv_kj * gk[4 * j + e], q = decay * q_factor[e] * inv_kj * gq[4 * j + e];
+          const float decay = __expf(fminf(cum[e] - cum_j, 0.0f)) * inv_kj;
+          float k = beta[e] * inv_k[e] * decay * gk[4 * j + e], q = decay * q_factor[e] * gq[4 * j + e];
           asm("" : "+v"(k), "+v"(q));
-          av[4 * j + e] = col < row0 + e ? k : 0.0f;
-          a2v[4 * j + e] = col <= row0 + e ? q : 0.0f;
+          av[4 * j + e] = above < 8 * j + e ? k : 0.0f;
+          a2v[4 * j + e] = above <= 8 * j + e ? q : 0.0f;
         }
       }
     }
     __syncthreads();  // nobody reads the rows of K and Q any more
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < 16; i += 2) {
       const int row = 32 * ti + 8 * (i / 4) + 4 * h + (i % 4);
-      sm.a[row][32 * tj + n] = av[i];  // the tile above the diagonal is zero
-      sm.a2[row][32 * tj + n] = float_to_bf16_bits(a2v[i]);
+      sm_a[row][32 * tj + n] = av[i];  // the tile above the diagonal is zero
+      sm_a[row + 1][32 * tj + n] = av[i + 1];
+      const uint32_t pair = pack_bf16(a2v[i], a2v[i + 1]);
+      sm_a2[row][32 * tj + n] = static_cast<uint16_t>(pair);
+      sm_a2[row + 1][32 * tj + n] = static_cast<uint16_t>(pair >> 16);
     }
   }
   __syncthreads();
@@ -244,17 +364,20 @@ gdn_chunk_prepare(GdnArgs a) {
   // Every factor enters as a sum of two bf16 numbers (value = hi + lo, products
   // hi*hi + lo*hi + hi*lo), which keeps the result to about 2^-16 relative.
   //
-  // T_b by forward substitution on the identity: wave b, lane = column; the
-  // result replaces the diagonal block of A, which nothing else reads.
-  if (lane < 16) {
-    const int base = 16 * wave;
+  // T_b by forward substitution on the identity: sixteen lanes a block, lane = column, by
+  // one wave of a head's (of each head's another, which the hardware deals to another SIMD);
+  // the result replaces the diagonal block of A, which nothing else reads.  The other waves
+  // convolve the V that are left meanwhile (behind the kernel's end, all of them: 112 us at
+  // 8191 tokens of 16/48 heads).
+  if (wave == local) {
+    const int base = 16 * (lane / 16), column = lane % 16;
     float t[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      float acc = (i == lane) ? 1.0f : 0.0f;
+      float acc = (i == column) ? 1.0f : 0.0f;
 #pragma unroll
       for (int j4 = 0; j4 < (i + 3) / 4; ++j4) {
-        const float4 row = *reinterpret_cast<const float4*>(&sm.a[base + i][base + 4 * j4]);
+        const float4 row = *reinterpret_cast<const float4*>(&sm_a[base + i][base + 4 * j4]);
         acc -= row.x * t[4 * j4];
         if (4 * j4 + 1 < i) acc -= row.y * t[4 * j4 + 1];
         if (4 * j4 + 2 < i) acc -= row.z * t[4 * j4 + 2];
@@ -263,7 +386,11 @@ gdn_chunk_prepare(GdnArgs a) {
       t[i] = acc;
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sm.a[base + i][base + lane] = t[i];
+    for (int i = 0; i < 16; ++i) sm_a[base + i][base + column] = t[i];
+  }
+  if constexpr (LAYER) {
+    const int turn = wave == local ? 3 * HEADS + local : 3 * local + wave - (wave > local);
+    if (turn < 4 * min(HEADS, 2)) convolve_v(turn / 4, turn % 4);
   }
   __syncthreads();
 
@@ -279,43 +406,43 @@ gdn_chunk_prepare(GdnArgs a) {
     for (int b = 0; b < 4; ++b) {
       x[b] = zero;
       if (b < wave) continue;  // uniform over the wave
-      floatx4 r = zero;
       if (b == wave) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = (4 * hq + e == m) ? 1.0f : 0.0f;
+        for (int e = 0; e < 4; ++e) x[b][e] = sm_a[16 * b + 4 * hq + e][16 * b + m];
+        continue;
       }
-      // R_b -= [A_b,k0 | A_b,k1] [X_k0; X_k1]: contraction slot (hq, e) is row
+      // r = sum [A_b,k0 | A_b,k1] [X_k0; X_k1]: contraction slot (hq, e) is row
       // 4 hq + e % 4 of block k0 (e < 4) or k1
+      floatx4 r = zero;
 #pragma unroll
       for (int k0 = 0; k0 < b; k0 += 2) {
         if (k0 + 1 < wave) continue;  // both blocks of X are zero
-        const bool both = k0 + 1 < b;
-        const float4 first = *reinterpret_cast<const float4*>(&sm.a[16 * b + m][16 * k0 + 4 * hq]);
-        float4 second = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (both) second = *reinterpret_cast<const float4*>(&sm.a[16 * b + m][16 * k0 + 16 + 4 * hq]);
-        bf16x8 a_hi, a_lo, b_hi, b_lo;
-        split_operand(floatx4{-first.x, -first.y, -first.z, -first.w},
-                      floatx4{-second.x, -second.y, -second.z, -second.w}, a_hi, a_lo);
-        split_operand(x[k0], both ? x[k0 + 1] : zero, b_hi, b_lo);
-        r = mfma16(a_hi, b_hi, r);
-        r = mfma16(a_lo, b_hi, r);
-        r = mfma16(a_hi, b_lo, r);
+        const floatx4 first = *reinterpret_cast<const floatx4*>(&sm_a[16 * b + m][16 * k0 + 4 * hq]);
+        if (k0 + 1 == b) {
+          r = product16(split_operand(first), split_operand(x[k0]), r);
+        } else {
+          const floatx4 second = *reinterpret_cast<const floatx4*>(&sm_a[16 * b + m][16 * k0 + 16 + 4 * hq]);
+          bf16x8 a_hi, a_lo, b_hi, b_lo;
+          split_operand(first, second, a_hi, a_lo);
+          split_operand(x[k0], x[k0 + 1], b_hi, b_lo);
+          r = mfma16(a_hi, b_hi, r);
+          r = mfma16(a_lo, b_hi, r);
+          r = mfma16(a_hi, b_lo, r);
+        }
       }
-      // X_b = T_b R_b
-      const float4 t4 = *reinterpret_cast<const float4*>(&sm.a[16 * b + m][16 * b + 4 * hq]);
-      bf16x8 t_hi, t_lo, r_hi, r_lo;
-      split_operand(floatx4{t4.x, t4.y, t4.z, t4.w}, zero, t_hi, t_lo);
-      split_operand(r, zero, r_hi, r_lo);
-      floatx4 acc = mfma16(t_hi, r_hi, zero);
-      acc = mfma16(t_lo, r_hi, acc);
-      x[b] = mfma16(t_hi, r_lo, acc);
+      // X_b = -T_b r
+      const floatx4 t = *reinterpret_cast<const floatx4*>(&sm_a[16 * b + m][16 * b + 4 * hq]);
+      x[b] = -product16(split_operand(t), split_operand(r), zero);
     }
     __syncthreads();  // every wave has read what it needs of A: T takes its place
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        sm.t[16 * b + 4 * hq + e][16 * wave + m] = float_to_bf16_bits(x[b][e]);
+      for (int e = 0; e < 4; e += 2) {
+        const uint32_t pair = pack_bf16(x[b][e], x[b][e + 1]);
+        sm_t[16 * b + 4 * hq + e][16 * wave + m] = static_cast<uint16_t>(pair);
+        sm_t[16 * b + 4 * hq + e + 1][16 * wave + m] = static_cast<uint16_t>(pair >> 16);
+      }
   }
   __syncthreads();
 
@@ -332,22 +459,22 @@ gdn_chunk_prepare(GdnArgs a) {
     const int tile = f < 2 ? f : 2 + (f - 2) / 2, kb = f < 2 ? 0 : (f - 2) % 2;
     const int hq = l / 16, m = l % 16;
     const int row = 16 * tile + m, lo = 32 * kb + 4 * hq;
-    uint2 w0 = *reinterpret_cast<const uint2*>(&sm.t[row][lo]);
-    uint2 w1 = *reinterpret_cast<const uint2*>(&sm.t[row][lo + 16]);
+    uint2 w0 = *reinterpret_cast<const uint2*>(&sm_t[row][lo]);
+    uint2 w1 = *reinterpret_cast<const uint2*>(&sm_t[row][lo + 16]);
     t_out[piece] = make_uint4(w0.x, w0.y, w1.x, w1.y);
-    w0 = *reinterpret_cast<const uint2*>(&sm.a2[row][lo]);
-    w1 = *reinterpret_cast<const uint2*>(&sm.a2[row][lo + 16]);
+    w0 = *reinterpret_cast<const uint2*>(&sm_a2[row][lo]);
+    w1 = *reinterpret_cast<const uint2*>(&sm_a2[row][lo + 16]);
     a2_out[piece] = make_uint4(w0.x, w0.y, w1.x, w1.y);
   }
   // per-token factors, and the decay of the whole chunk
   float* factors = reinterpret_cast<float*>(out + kGdnOffsetFactors);
-  const float cum_last = sm.cum[C - 1];
+  const float cum_last = sm_cum[C - 1];
   if (tid < C) {
-    const float grown = __expf(sm.cum[tid]);
-    factors[tid] = sm.beta[tid];
-    factors[C + tid] = sm.beta[tid] * grown * sm.inv_k[tid];
+    const float grown = __expf(sm_cum[tid]);
+    factors[tid] = sm_beta[tid];
+    factors[C + tid] = sm_beta[tid] * grown * sm.inv_k[tid];
     factors[2 * C + tid] = sm.q_factor[tid] * grown;
-    factors[3 * C + tid] = __expf(cum_last - sm.cum[tid]) * sm.inv_k[tid];
+    factors[3 * C + tid] = __expf(cum_last - sm_cum[tid]) * sm.inv_k[tid];
   } else if (tid < 2 * C) {
     // the rest of the block is loaded with it: keep it defined
     factors[4 * C + tid - C] = tid == C ? __expf(cum_last) : 0.0f;
@@ -1003,12 +1130,27 @@ bool gdn_chunked_supported(const GdnArgs& a, int chunk) {
          aligned(a.q) && aligned(a.k) && aligned(a.v) && aligned(a.workspace);
 }
 
-int launch_gdn_chunked(hipStream_t stream, const GdnArgs& a) {
+bool gdn_layer_rows_supported(const GdnLayerInputs& layer, int taps) {
+  auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+  return taps == 4 && aligned(layer.qkv) && aligned(layer.conv_weight);
+}
+
+int launch_gdn_chunked(hipStream_t stream, const GdnArgs& a, const GdnLayerInputs* layer) {
   const long long chunks = (a.length + C - 1) / C;
   const long long heads = static_cast<long long>(a.batch) * a.value_heads;
   if (heads * chunks > 0x7fffffffLL) return PLUTO_HIP_EINVAL;
-  if (kernel_enabled(kAuxiliaryKernel))
-    gdn_chunk_prepare<<<static_cast<unsigned>(heads * chunks), 256, 0, stream>>>(a);
+  if (kernel_enabled(kAuxiliaryKernel)) {
+    const int group = a.value_heads / a.key_heads;
+    const unsigned blocks = static_cast<unsigned>(heads * chunks);
+    if (layer == nullptr)
+      gdn_chunk_prepare<1, false><<<blocks, 256, 0, stream>>>(a, {});
+    else if (group % 3 == 0)
+      gdn_chunk_prepare<3, true><<<blocks / 3, 768, 0, stream>>>(a, *layer);
+    else if (group % 2 == 0)
+      gdn_chunk_prepare<2, true><<<blocks / 2, 512, 0, stream>>>(a, *layer);
+    else
+      gdn_chunk_prepare<1, true><<<blocks, 256, 0, stream>>>(a, *layer);
+  }
   int status = launch_status();
   if (status != 0) return status;
   if (!kernel_enabled(kMainKernel)) return 0;

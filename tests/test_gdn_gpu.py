@@ -416,6 +416,35 @@ def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T):
         assert torch.equal(got[i], want[0]) and torch.equal(state[i], one[0]), i
 
 
+@pytest.mark.parametrize("kh,vh", [(2, 2), (2, 4), (2, 6), (1, 4), (2, 10), (1, 6)])
+@pytest.mark.parametrize("T", [1, 2, 63, 64, 66, 131])
+def test_preparation_that_convolves_on_the_way(capi, kh, vh, T):
+    """One, two or three value heads of a key head a workgroup, several workgroups of a key
+    head, chunks with one row and rows whose taps lie in the chunk before.  Against the
+    convolution as a pass of its own, which weights off a 16-byte boundary take: the rows
+    are the same, their norms and the solve are summed in another order, so that a value
+    may fall the other way of a bf16 rounding and move by 2^-8 of itself."""
+    B, d = 2, 128
+    channels = 2 * kh * d + vh * d
+    p = capi.delta_params(kh, vh, d, d)
+    gen = torch.Generator(device="cuda").manual_seed(100 * T + vh)
+
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    qkv, z, a, b = values(B, T, channels), values(B, T, vh * d), values(B, T, vh), values(B, T, vh)
+    conv, a_log, dt, norm = (dev(w) for w in layer_weights(kh, vh, d, d, 4))
+    space = torch.empty(conv.numel() + 4, device="cuda")
+    shifted = space[1:1 + conv.numel()].view(conv.shape)
+    shifted.copy_(conv)
+    results = []
+    for weight in (conv, shifted):
+        state = torch.zeros((B, vh, d, d), device="cuda")
+        results.append((capi.gdn_layer_forward(p, qkv, z, a, b, weight, a_log, dt, norm, state).double(), state.double()))
+    for got, want in zip(*results):
+        assert torch.isfinite(got).all()
+        assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+
+
 @pytest.mark.parametrize("T", [1, 64, 65, 200, 449])
 def test_scan_with_two_slices_a_workgroup(capi, T):
     """48 heads are more single slices than compute units, so a workgroup walks two of
