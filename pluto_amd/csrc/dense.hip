@@ -504,7 +504,11 @@ product_columns_kernel(GramArgs a) {
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
   const int n_tiles = (a.n_cols + kWidth - 1) / kWidth, m_tiles = (a.m_cols + kWidth - 1) / kWidth;
-  const int tile = blockIdx.x % (n_tiles * m_tiles), slice = blockIdx.x / (n_tiles * m_tiles);
+  // The tiles of a slice read the same rows: neighbours share an XCD's L2.  Dealt out to all
+  // of them, 16000 rows of 768 -> 768 took 39.8 us instead of 25.2; in wide tiles, 16384 rows
+  // of 768 -> 2304, 62.2 instead of 57.5 (353 MB from beyond the L2).
+  const int logical = xcd_contiguous_block();
+  const int tile = logical % (n_tiles * m_tiles), slice = logical / (n_tiles * m_tiles);
   const int m0 = (tile / n_tiles) * kWidth, n0 = (tile % n_tiles) * kWidth;
   const int wm = 64 * (wave / 2), wn = 64 * (wave % 2);
   const int per_slice = ((a.rows + a.slices - 1) / a.slices + kRows - 1) / kRows * kRows;
@@ -602,8 +606,9 @@ product_columns_wide_kernel(GramArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int h = lane / 32, n = lane % 32;
   const int n_tiles = (a.n_cols + TN - 1) / TN, m_tiles = (a.m_cols + TM - 1) / TM;
-  const int tile = blockIdx.x % (n_tiles * m_tiles);
-  const int slice = __builtin_amdgcn_readfirstlane(blockIdx.x / (n_tiles * m_tiles));
+  const int logical = xcd_contiguous_block();
+  const int tile = logical % (n_tiles * m_tiles);
+  const int slice = __builtin_amdgcn_readfirstlane(logical / (n_tiles * m_tiles));
   const int m0 = __builtin_amdgcn_readfirstlane(tile / n_tiles * TM);
   const int n0 = __builtin_amdgcn_readfirstlane(tile % n_tiles * TN);
   const int wm = 32 * JM * (wave / 2), wn = 32 * JN * (wave % 2);

@@ -273,4 +273,11 @@ __device__ inline int xcd_logical_block() {
   return (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
 }
 
+// The same for any grid: an XCD has one block more than the last ones where the number is no
+// multiple of 8.
+__device__ inline int xcd_contiguous_block() {
+  const int xcd = blockIdx.x % 8, each = gridDim.x / 8, more = gridDim.x % 8;
+  return xcd * each + min(xcd, more) + blockIdx.x / 8;
+}
+
 }  // namespace pluto_hip
