@@ -282,12 +282,13 @@ int pluto_hip_gdn_step_batch(void* stream, const pluto_hip_delta_params* p, int 
   float* beta = reinterpret_cast<float*>(scratch + offset);
   offset += align_up(n * vh * 4, 256);
   float* core = reinterpret_cast<float*>(scratch + offset);
+  if (!force_generic() && gdn_step_fused_supported(kd, vd))
+    return launch_gdn_step_fused(s, qkv, z, a, b, io_dtype, conv_weight, a_log, dt_bias, norm, batch, kh, vh, kd, vd,
+                                 p->conv_kernel_dim, p->rms_norm_epsilon, round, conv_states, recurrent_states,
+                                 output, convolved);
   status = launch_gdn_conv_step(s, qkv, io_dtype, conv_weight, batch, channels,
                                 p->conv_kernel_dim, round, conv_states, convolved);
   if (status != 0) return status;
-  if (!force_generic() && gdn_step_fused_supported(kd, vd))
-    return launch_gdn_step_fused(s, convolved, z, a, b, io_dtype, a_log, dt_bias, norm, batch, kh,
-                                 vh, kd, vd, p->rms_norm_epsilon, round, recurrent_states, output);
   status = launch_gdn_gates(s, a, b, io_dtype, a_log, dt_bias, batch, vh, round, log_decay, beta);
   if (status != 0) return status;
   GdnArgs g;

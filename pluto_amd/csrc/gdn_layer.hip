@@ -128,6 +128,28 @@ conv_step_kernel(const void* __restrict__ input, int in_dtype, const float* __re
   output[c] = maybe_round(sum / (1.0f + expf(-sum)), round);
 }
 
+// One channel of four taps, its registers in one access each way: the same arithmetic.
+__device__ inline float conv_step4(float4 taps, float4 w, float input, bool round, float* state) {
+  const float current = maybe_round(input, round);
+  *reinterpret_cast<float4*>(state) = make_float4(taps.y, taps.z, taps.w, current);
+  float sum = 0.0f;
+  sum += taps.y * w.x;
+  sum += taps.z * w.y;
+  sum += taps.w * w.z;
+  sum = maybe_round(sum + current * w.w, round);
+  return maybe_round(sum / (1.0f + expf(-sum)), round);
+}
+__global__ void __launch_bounds__(256)
+conv_step4_kernel(const void* input, int in_dtype, const float* weight, int channels, bool round, float* state,
+                  float* output) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= channels) return;
+  const size_t index = static_cast<size_t>(blockIdx.y) * channels + c;
+  output[index] = conv_step4(*reinterpret_cast<const float4*>(state + 4 * index),
+                             *reinterpret_cast<const float4*>(weight + 4 * static_cast<size_t>(c)),
+                             load_element(input, index, in_dtype), round, state + 4 * index);
+}
+
 __global__ void __launch_bounds__(256)
 gates_kernel(const void* a, const void* b, int in_dtype, const float* __restrict__ a_log,
              const float* __restrict__ dt_bias, long long rows, int heads, bool round,
@@ -232,6 +254,9 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // for.
 struct StepArgs {
   const float* convolved = nullptr;  // [batch, channels] q | k | v after conv + SiLU
+  const void* qkv = nullptr;         // [batch, channels] before it, of z's type, and its shift
+  float* conv_state = nullptr;       // registers [batch, channels, 4]: step128_kernel's CONV
+  const float* conv_weight = nullptr;
   const void* z = nullptr;           // [batch, vh * vd], fp32 or bf16 (template argument)
   const void* a = nullptr;           // [batch, vh]
   const void* b = nullptr;
@@ -240,7 +265,7 @@ struct StepArgs {
   const float* norm = nullptr;
   float* state = nullptr;            // [batch, vh, kd, vd]
   void* out = nullptr;               // [batch, vh * vd], same type as z
-  int kh = 0, vh = 0, kd = 0, vd = 0;
+  int batch = 0, kh = 0, vh = 0, kd = 0, vd = 0;
   float epsilon = 1e-6f;
   bool round = true;
 };
@@ -359,19 +384,212 @@ step_kernel(StepArgs a) {
                 IO == PLUTO_HIP_BF16 ? result : maybe_round(result, a.round));
 }
 
+// The same for heads of 128 x 128: four waves a head, wave w columns 32 w .. + 31, its lane (r,
+// c) = (lane / 8, lane % 8) rows r, r + 8, ... of columns 4 c .. + 3.  Sums over rows stay
+// within a wave; the workgroup meets for the rows of k and q and for the mean square only.
+// Workgroups are persistent, two a compute unit, and request a head's state before they work
+// on the one before it.  Sequences of 16/48 heads, with workgroups of 1024 threads a head and
+// eight barriers, whose vector instructions were 45 % of it, and so: 6 sequences 14.7 -> 10.7 us,
+// 21 33.1 -> 22.1, 40 (255 MB) 56.4 -> 41.5.
+// CONV: the shift registers too; a workgroup then walks all value heads of a key head, which
+// share the channels of q and k (what one of them shifts, another one must have read).  28
+// sequences, with the convolution's launch and without: 44.0 + 4.9 -> 30.6, 64 96.3 + 11.1 -> 73.8.
+constexpr int kStepSlots = 512;
+struct HeadLoads {
+  float4 state[16];
+  float4 v, z;
+  float a, b, a_log, dt_bias, row;  // row: of k (threads below 128) or q
+  float4 taps, taps_weight;         // CONV: of v (threads below 128)
+  float current;
+};
+struct Head {
+  int sequence, head;
+};
+
+__device__ inline float4 load_four(const void* base, size_t index, int dtype) {
+  if (dtype != PLUTO_HIP_BF16) return *reinterpret_cast<const float4*>(static_cast<const float*>(base) + index);
+  const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + index);
+  return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                     __uint_as_float(v.y & 0xffff0000u));
+}
+
+template <int IO, bool CONV>
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+step128_kernel(StepArgs a) {
+  __shared__ float rows[2][2][128];    // k and q, element r of row block i at 16 r + i
+  __shared__ __attribute__((aligned(16))) float values[2][128];  // CONV: v
+  __shared__ float parts[2][4];
+  const int tid = threadIdx.x, lane = tid % 64, r = lane / 8;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int column = 32 * wave + 4 * (lane % 8);
+  const int group = a.vh / a.kh, channels = (2 * a.kh + a.vh) * 128;
+  const int units = a.batch * (CONV ? a.kh : a.vh);
+  const float4 weight = *reinterpret_cast<const float4*>(a.norm + column);
+  // the heads of this workgroup in order
+  auto head_of = [&](int unit, int member) {
+    return CONV ? Head{unit / a.kh, unit % a.kh * group + member} : Head{unit / a.vh, unit % a.vh};
+  };
+  auto request = [&](HeadLoads& l, Head at) {
+    const size_t head = static_cast<size_t>(at.sequence) * a.vh + at.head;
+    const float* state = a.state + head * (128 * 128) + r * 128 + column;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) l.state[i] = *reinterpret_cast<const float4*>(state + 8 * 128 * i);
+    l.z = load_four(a.z, head * 128 + column, IO);
+    l.a = load_element(a.a, head, IO), l.b = load_element(a.b, head, IO);
+    l.a_log = a.a_log[at.head], l.dt_bias = a.dt_bias[at.head];
+    if constexpr (CONV) {
+      if (tid < 128) {
+        const int channel = (2 * a.kh + at.head) * 128 + tid;
+        const size_t index = static_cast<size_t>(at.sequence) * channels + channel;
+        l.taps = *reinterpret_cast<const float4*>(a.conv_state + 4 * index);
+        l.taps_weight = *reinterpret_cast<const float4*>(a.conv_weight + 4 * channel);
+        l.current = load_element(a.qkv, index, IO);
+      }
+    } else {
+      const float* token = a.convolved + static_cast<size_t>(at.sequence) * channels;
+      l.row = token[(tid < 128 ? a.kh + at.head / group : at.head / group) * 128 + tid % 128];
+      l.v = *reinterpret_cast<const float4*>(token + (2 * a.kh + at.head) * 128 + column);
+    }
+  };
+  const int row_place = tid % 8 * 16 + tid % 128 / 8;
+  float k_scale = 0.0f, q_scale = 0.0f, k[16], q[16];
+  int parity = 0;
+  // one head; `next` is requested before it is worked on
+  auto process = [&](HeadLoads& l, HeadLoads& following, Head at, bool first, bool more, Head next) {
+    if constexpr (CONV) {
+      if (first) {
+        const int channel = ((tid < 128 ? a.kh : 0) + at.head / group) * 128 + tid % 128;
+        const size_t index = static_cast<size_t>(at.sequence) * channels + channel;
+        rows[parity][tid / 128][row_place] =
+            conv_step4(*reinterpret_cast<const float4*>(a.conv_state + 4 * index),
+                       *reinterpret_cast<const float4*>(a.conv_weight + 4 * channel),
+                       load_element(a.qkv, index, IO), a.round, a.conv_state + 4 * index);
+      }
+      if (tid < 128) {
+        const size_t index = static_cast<size_t>(at.sequence) * channels + (2 * a.kh + at.head) * 128 + tid;
+        values[parity][tid] = conv_step4(l.taps, l.taps_weight, l.current, a.round, a.conv_state + 4 * index);
+      }
+    } else {
+      rows[parity][tid / 128][row_place] = l.row;
+    }
+    if (more) request(following, next);
+    // LDS alone: the requests stay in flight
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (!CONV || first) {
+      // 1e-6 inside the roots: cached_attention_ops.cc:224-228
+      const float k0 = rows[parity][0][lane], k1 = rows[parity][0][lane + 64];
+      const float q0 = rows[parity][1][lane], q1 = rows[parity][1][lane + 64];
+      k_scale = rsqrtf(wave_sum(k0 * k0 + k1 * k1) + 1e-6f);
+      q_scale = rsqrtf(wave_sum(q0 * q0 + q1 * q1) + 1e-6f) / sqrtf(128.0f);
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) {
+        const float4 k4 = *reinterpret_cast<const float4*>(&rows[parity][0][16 * r + i]);
+        const float4 q4 = *reinterpret_cast<const float4*>(&rows[parity][1][16 * r + i]);
+        k[i] = k4.x * k_scale, k[i + 1] = k4.y * k_scale, k[i + 2] = k4.z * k_scale, k[i + 3] = k4.w * k_scale;
+        q[i] = q4.x * q_scale, q[i + 1] = q4.y * q_scale, q[i + 2] = q4.z * q_scale, q[i + 3] = q4.w * q_scale;
+      }
+    }
+    const float decay = __expf(log_decay_of(l.a + l.dt_bias, l.a_log));
+    const float beta = maybe_round(beta_of(l.b), a.round);
+    const float4 v = CONV ? *reinterpret_cast<const float4*>(&values[parity][column]) : l.v;
+    // over the eight row lanes of a column
+    auto across_rows = [&](float4 x) {
+#pragma unroll
+      for (int offset = 8; offset < 64; offset *= 2) {
+        x.x += __shfl_xor(x.x, offset, 64), x.y += __shfl_xor(x.y, offset, 64);
+        x.z += __shfl_xor(x.z, offset, 64), x.w += __shfl_xor(x.w, offset, 64);
+      }
+      return x;
+    };
+    float4 predicted = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float4& s = l.state[i];
+      s.x *= decay, s.y *= decay, s.z *= decay, s.w *= decay;
+      predicted.x += s.x * k[i], predicted.y += s.y * k[i], predicted.z += s.z * k[i], predicted.w += s.w * k[i];
+    }
+    predicted = across_rows(predicted);
+    const float4 delta = make_float4((v.x - predicted.x) * beta, (v.y - predicted.y) * beta,
+                                     (v.z - predicted.z) * beta, (v.w - predicted.w) * beta);
+    float4 core = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const size_t head = static_cast<size_t>(at.sequence) * a.vh + at.head;
+    float* state = a.state + head * (128 * 128) + r * 128 + column;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float4& s = l.state[i];
+      s.x += k[i] * delta.x, s.y += k[i] * delta.y, s.z += k[i] * delta.z, s.w += k[i] * delta.w;
+      core.x += s.x * q[i], core.y += s.y * q[i], core.z += s.z * q[i], core.w += s.w * q[i];
+      *reinterpret_cast<float4*>(state + 8 * 128 * i) = s;
+    }
+    core = across_rows(core);
+    core = make_float4(maybe_round(core.x, a.round), maybe_round(core.y, a.round), maybe_round(core.z, a.round),
+                       maybe_round(core.w, a.round));
+    // RMSNorm over the head's columns, then the SiLU(z) gate
+    float square = (core.x * core.x + core.y * core.y) + (core.z * core.z + core.w * core.w);
+#pragma unroll
+    for (int offset = 1; offset < 8; offset *= 2) square += __shfl_xor(square, offset, 64);
+    if (lane == 0) parts[parity][wave] = square;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (r == 0) {
+      const float total = (parts[parity][0] + parts[parity][1]) + (parts[parity][2] + parts[parity][3]);
+      const float inverse = rsqrtf(total / 128.0f + a.epsilon);
+      auto finish = [&](float x, float w, float gate) {
+        const float affine = maybe_round(maybe_round(x * inverse, a.round) * w, a.round);
+        const float result = affine * (gate / (1.0f + expf(-gate)));
+        // a bf16 result is rounded once, by the store, as in step_kernel
+        return IO == PLUTO_HIP_BF16 ? result : maybe_round(result, a.round);
+      };
+      const float4 out = make_float4(finish(core.x, weight.x, l.z.x), finish(core.y, weight.y, l.z.y),
+                                     finish(core.z, weight.z, l.z.z), finish(core.w, weight.w, l.z.w));
+      if (IO == PLUTO_HIP_BF16)
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + head * 128 + column) =
+            make_uint2(pack_bf16(out.x, out.y), pack_bf16(out.z, out.w));
+      else
+        *reinterpret_cast<float4*>(static_cast<float*>(a.out) + head * 128 + column) = out;
+    }
+    parity ^= 1;
+  };
+  const int members = CONV ? group : 1;
+  int unit = blockIdx.x, member = 0;
+  HeadLoads loads[2];
+  request(loads[0], head_of(unit, 0));
+  while (true) {
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const Head at = head_of(unit, member);
+      const bool first = member == 0;
+      if (++member == members) member = 0, unit += gridDim.x;
+      const bool more = unit < units;
+      process(loads[side], loads[side ^ 1], at, first, more, more ? head_of(unit, member) : at);
+      if (!more) return;
+    }
+  }
+}
+
 }  // namespace
 
 bool gdn_step_fused_supported(int key_dim, int value_dim) {
   return key_dim <= 128 && value_dim <= 128;
 }
 
-int launch_gdn_step_fused(hipStream_t stream, const float* convolved, const void* z,
-                          const void* a, const void* b, int io_dtype, const float* a_log,
-                          const float* dt_bias, const float* norm, int batch, int key_heads,
-                          int value_heads, int key_dim, int value_dim, float epsilon, bool round,
-                          float* state, void* out) {
+// What step128_kernel reads and writes four at a time.
+static bool step128_supported(const StepArgs& s, int io_dtype) {
+  const uintptr_t io = io_dtype == PLUTO_HIP_BF16 ? 8 : 16;
+  return s.kd == 128 && s.vd == 128 && aligned16(s.state) && aligned16(s.norm) && aligned16(s.convolved) &&
+         reinterpret_cast<uintptr_t>(s.z) % io == 0 && reinterpret_cast<uintptr_t>(s.out) % io == 0;
+}
+
+int launch_gdn_step_fused(hipStream_t stream, const void* qkv, const void* z, const void* a, const void* b,
+                          int io_dtype, const float* conv_weight, const float* a_log, const float* dt_bias,
+                          const float* norm, int batch, int key_heads, int value_heads, int key_dim, int value_dim,
+                          int taps, float epsilon, bool round, float* conv_state, float* state, void* out,
+                          float* convolved) {
   StepArgs s;
   s.convolved = convolved;
+  s.qkv = qkv;
+  s.conv_state = conv_state;
+  s.conv_weight = conv_weight;
   s.z = z;
   s.a = a;
   s.b = b;
@@ -380,13 +598,37 @@ int launch_gdn_step_fused(hipStream_t stream, const float* convolved, const void
   s.norm = norm;
   s.state = state;
   s.out = out;
+  s.batch = batch;
   s.kh = key_heads;
   s.vh = value_heads;
   s.kd = key_dim;
   s.vd = value_dim;
   s.epsilon = epsilon;
   s.round = round;
-  if (io_dtype == PLUTO_HIP_BF16)
+  const bool wide = step128_supported(s, io_dtype), bf16 = io_dtype == PLUTO_HIP_BF16;
+  // The convolution's launch is saved where walking all heads of a key head makes no
+  // workgroup's list longer.
+  auto turns = [](long long units) { return (units + kStepSlots - 1) / kStepSlots; };
+  const long long heads = 1LL * batch * value_heads, key_units = 1LL * batch * key_heads;
+  if (wide && taps == 4 && aligned16(conv_state) && aligned16(conv_weight) &&
+      turns(key_units) * (value_heads / key_heads) <= turns(heads)) {
+    const unsigned blocks = static_cast<unsigned>(key_units < kStepSlots ? key_units : kStepSlots);
+    if (bf16)
+      step128_kernel<PLUTO_HIP_BF16, true><<<blocks, 256, 0, stream>>>(s);
+    else
+      step128_kernel<PLUTO_HIP_F32, true><<<blocks, 256, 0, stream>>>(s);
+    return launch_status();
+  }
+  const int channels = 2 * key_heads * key_dim + value_heads * value_dim;
+  const int status =
+      launch_gdn_conv_step(stream, qkv, io_dtype, conv_weight, batch, channels, taps, round, conv_state, convolved);
+  if (status != 0) return status;
+  const unsigned blocks = static_cast<unsigned>(heads < kStepSlots ? heads : kStepSlots);
+  if (wide && bf16)
+    step128_kernel<PLUTO_HIP_BF16, false><<<blocks, 256, 0, stream>>>(s);
+  else if (wide)
+    step128_kernel<PLUTO_HIP_F32, false><<<blocks, 256, 0, stream>>>(s);
+  else if (bf16)
     step_kernel<PLUTO_HIP_BF16><<<batch * value_heads, kStepThreads, 0, stream>>>(s);
   else
     step_kernel<PLUTO_HIP_F32><<<batch * value_heads, kStepThreads, 0, stream>>>(s);
@@ -422,8 +664,12 @@ int launch_gdn_conv_sequence(hipStream_t stream, const void* input, int in_dtype
 int launch_gdn_conv_step(hipStream_t stream, const void* input, int in_dtype, const float* weight,
                          int batch, int channels, int kernel, bool round, float* state,
                          float* output) {
-  conv_step_kernel<<<dim3((channels + 127) / 128, batch), 128, 0, stream>>>(
-      input, in_dtype, weight, channels, kernel, round, state, output);
+  if (kernel == 4 && aligned16(weight) && aligned16(state))
+    conv_step4_kernel<<<dim3((channels + 255) / 256, batch), 256, 0, stream>>>(input, in_dtype, weight, channels, round,
+                                                                               state, output);
+  else
+    conv_step_kernel<<<dim3((channels + 127) / 128, batch), 128, 0, stream>>>(
+        input, in_dtype, weight, channels, kernel, round, state, output);
   return launch_status();
 }
 

@@ -277,6 +277,40 @@ def test_batched_step_is_the_single_step_of_every_sequence(capi, oracle, dim, ro
         np.testing.assert_array_equal(together.conv[s].cpu().numpy(), alone[s].conv.cpu().numpy())
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("kh,vh,batch", [(16, 48, 22), (16, 48, 21), (16, 48, 54), (16, 16, 33), (8, 32, 33), (1, 3, 1)])
+def test_persistent_steps_are_the_single_step_of_every_sequence(capi, kh, vh, batch, dtype):
+    """Workgroups that walk one or several heads, with the convolution inside (a key head's
+    heads after each other) or in front, the last turn full or not: bit for bit the call
+    for one sequence, over two tokens."""
+    d = 128
+    kind = torch.bfloat16 if dtype == "bf16" else torch.float32
+    p = capi.delta_params(kh, vh, d, d)
+    channels = 2 * kh * d + vh * d
+    weights = [dev(w) for w in layer_weights(kh, vh, d, d, 4)]
+    gen = torch.Generator(device="cuda").manual_seed(batch)
+
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(kind)
+    together = capi.DeltaNetStep(p, batch=batch)
+    together.state.copy_(values(*together.state.shape))
+    together.conv.copy_(values(*together.conv.shape))
+    chosen = sorted({0, batch // 2, batch - 1})
+    alone = {s: capi.DeltaNetStep(p, batch=1) for s in chosen}
+    for s in chosen:
+        alone[s].state.copy_(together.state[s:s + 1])
+        alone[s].conv.copy_(together.conv[s:s + 1])
+    for _ in range(2):
+        qkv, z, a, b = values(batch, channels), values(batch, vh * d), values(batch, vh), values(batch, vh)
+        got = together.step(qkv, z, a, b, *weights)
+        assert torch.isfinite(got).all()
+        for s in chosen:
+            want = alone[s].step(qkv[s:s + 1], z[s:s + 1], a[s:s + 1], b[s:s + 1], *weights)
+            assert torch.equal(got[s], want[0]), s
+    for s in chosen:
+        assert torch.equal(together.state[s], alone[s].state[0]) and torch.equal(together.conv[s], alone[s].conv[0]), s
+
+
 def test_batched_step_rejects_bad_arguments(capi):
     import ctypes
     p = capi.delta_params(2, 4, 16, 16)
