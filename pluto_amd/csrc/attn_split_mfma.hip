@@ -10,12 +10,13 @@
 // are 2^-24 of the product, what one FP32 rounding costs.  Per 32 x 32 block of
 // scores in products of depth 256: S 1, P V 3 (forward); S 1, dP 3, dQ 3; and
 // S 1, dP 3, dK 3, dV 6.  At sixteen times the rate of the FP32 matrix
-// instruction that is a third of its time.  T = 1024, 24/4 heads: 0.043 (0.050
-// with the gated output), 0.065 and 0.108 ms for the three kernels, where the kernels that
-// multiply one element at a time took 3.9, 5.0 and 7.4 ms.  What bounds them: one wave a
-// SIMD in the longest workgroup's chain of tiles (16 steps of 112 matrix instructions for
-// dQ, half of whose time is softmax arithmetic, splits and waits beside an idle matrix
-// pipe), and 384 workgroups of lengths 1 to 16 on 256 compute units.
+// instruction that is a third of its time.  T = 1024, 24/4 heads: 0.043 (0.047
+// with the gated output) and 0.149 ms for the forward and the gradients, where the kernels that
+// multiply one element at a time took 3.9 and 12.4 ms.  What bounds them: one wave a SIMD in
+// a workgroup's chain of tiles (a step is 112 matrix instructions in the gradients, half of whose
+// time is softmax arithmetic, splits and waits beside an idle matrix pipe), about 8 us before
+// the first and after the last tile of each of 768 workgroups, and for the forward 384
+// workgroups of lengths 1 to 16 on 256 compute units.
 //
 // Shape of the kernels as in flash_bwd_mfma.hip: four waves of 32 queries (keys)
 // each, tiles of 32 rows of the other side through two LDS stages filled by
@@ -100,9 +101,7 @@ constexpr int kQueries = 64;
 constexpr int kQueryStageBytes = 4 * kTileBytes;  // K and V of two tiles
 struct QueryWave {
   int head, half, parity, steps, first_query, query, query_load;
-  __device__ QueryWave(const SplitArgs& a, int wave, int n) {
-    head = blockIdx.x % a.heads;
-    const int q0 = ((a.length + kQueries - 1) / kQueries - 1 - static_cast<int>(blockIdx.x) / a.heads) * kQueries;
+  __device__ QueryWave(const SplitArgs& a, int wave, int n, int head_, int q0) : head(head_) {
     half = wave % 2;
     parity = wave / 2;
     steps = ((min(q0 + kQueries, a.length) - 1) / kRows) / 2 + 1;  // two tiles each
@@ -180,7 +179,8 @@ split_forward_kernel(SplitArgs a) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQueryStageBytes];
   __shared__ float wave_stats[2][2][2][64];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
-  const QueryWave w(a, wave, n);
+  const QueryWave w(a, wave, n, blockIdx.x % a.heads,
+                    ((a.length + kQueries - 1) / kQueries - 1 - static_cast<int>(blockIdx.x) / a.heads) * kQueries);
   const int T = a.length, query = w.query, query_load = w.query_load, head = w.head;
   const long long q_row = 1LL * a.heads * D;
   const TileAccess at(wave, lane, 1LL * (a.heads / a.group) * D);
@@ -415,12 +415,11 @@ split_gate_kernel(SplitArgs a, const uint16_t* __restrict__ qg, const float* __r
   }
 }
 
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-split_dq_kernel(SplitArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQueryStageBytes];
+// dQ of 64 queries.
+__device__ __forceinline__ void split_query_owned(const SplitArgs& a, unsigned char* lds, int head, int q0) {
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, h = lane / 32, n = lane % 32;
-  const QueryWave w(a, wave, n);
-  const int T = a.length, query = w.query, query_load = w.query_load, head = w.head;
+  const QueryWave w(a, wave, n, head, q0);
+  const int T = a.length, query = w.query, query_load = w.query_load;
   const long long q_row = 1LL * a.heads * D;
   const TileAccess at(wave, lane, 1LL * (a.heads / a.group) * D);
   QueryFill fill(a, lds, wave, head, at);
@@ -686,14 +685,34 @@ __device__ __forceinline__ void split_key_owned(const SplitArgs& a, unsigned cha
                       acc[db][4 * j + 2] * factor, acc[db][4 * j + 3] * factor);
 }
 
+// All gradients in one launch, longest workgroups first: a compute unit holds one, and those
+// of the last queries' tiles and of the first keys' take many times what the others do, so
+// that dQ and dK/dV in launches of their own each end with most compute units idle.  24
+// heads, 59.3 + 98.4 us at 1024 tokens and 149 so, 900 52.8 + 87.7 and 127, 400 27.6 + 43.8 and
+// 46, 70 15.5 + 16.1 and 17.7.
+enum class Gradients { kQueries, kKeys, kBoth };  // which of them a launch makes
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-split_dkv_kernel(SplitArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kDkvStageBytes];
-  const int unit = blockIdx.x % (2 * a.heads), k0 = static_cast<int>(blockIdx.x) / (2 * a.heads) * kKeys;
-  if (unit < a.heads)
-    split_key_owned<true>(a, lds, unit, k0);
-  else
-    split_key_owned<false>(a, lds, unit - a.heads, k0);
+split_backward_kernel(SplitArgs a, Gradients which) {
+  constexpr int kLds = 2 * (kQueryStageBytes > kDkvStageBytes ? kQueryStageBytes : kDkvStageBytes);
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
+  const int query_tiles = which == Gradients::kKeys ? 0 : (a.length + kQueries - 1) / kQueries;
+  const int key_tiles = which == Gradients::kQueries ? 0 : (a.length + kKeys - 1) / kKeys;
+  const int rows = (a.length + kRows - 1) / kRows;
+  int query = query_tiles - 1, key = 0, block = blockIdx.x;
+  while (true) {
+    // The longest tile that is left: of keys, once for each gradient, or of queries.  A step of
+    // the one takes about as long as one of the other (2.4 us).
+    const int query_steps = query < 0 ? 0 : (min((query + 1) * kQueries, a.length) - 1) / kRows / 2 + 1;
+    const int key_steps = key >= key_tiles ? 0 : rows - key * (kKeys / kRows);
+    if (key_steps > query_steps) {
+      if (block < a.heads) return split_key_owned<true>(a, lds, block, key * kKeys);
+      if (block < 2 * a.heads) return split_key_owned<false>(a, lds, block - a.heads, key * kKeys);
+      block -= 2 * a.heads, ++key;
+    } else {
+      if (block < a.heads) return split_query_owned(a, lds, block, query * kQueries);
+      block -= a.heads, --query;
+    }
+  }
 }
 
 unsigned tile_grid(const SplitArgs& a, int owned) {
@@ -733,10 +752,11 @@ int launch_split_gate(hipStream_t stream, const SplitArgs& a, const void* qg, co
 }
 
 int launch_split_backward(hipStream_t stream, const SplitArgs& a) {
-  if (kernel_enabled(kQueryKernel)) split_dq_kernel<<<tile_grid(a, kQueries), kThreads, 0, stream>>>(a);
-  const int status = launch_status();
-  if (status != 0) return status;
-  if (kernel_enabled(kMainKernel)) split_dkv_kernel<<<2 * tile_grid(a, kKeys), kThreads, 0, stream>>>(a);
+  const bool queries = kernel_enabled(kQueryKernel), keys = kernel_enabled(kMainKernel);
+  const unsigned grid = (queries ? tile_grid(a, kQueries) : 0) + (keys ? 2 * tile_grid(a, kKeys) : 0);
+  if (grid == 0) return 0;
+  split_backward_kernel<<<grid, kThreads, 0, stream>>>(
+      a, queries && keys ? Gradients::kBoth : queries ? Gradients::kQueries : Gradients::kKeys);
   return launch_status();
 }
 

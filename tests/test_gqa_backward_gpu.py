@@ -160,6 +160,31 @@ def test_saved_block_holds_what_both_passes_need(capi, T, qh, kh, d, rot):
             assert np.array_equal(value.cpu().numpy(), got[name]), name
 
 
+@pytest.mark.parametrize("T,qh,kh", [(1, 2, 1), (32, 3, 1), (33, 6, 2), (64, 4, 2), (65, 6, 1), (129, 2, 2), (300, 5, 1),
+                                     (513, 3, 3)])
+def test_gradients_in_one_launch_are_those_of_two(capi, T, qh, kh):
+    """Head width 256: the workgroups of query and key tiles in one launch, longest first,
+    with tiles of either side that are ragged or the only one.  Bit for bit what launches of
+    their own make."""
+    d = 256
+    p = capi.attention_params(qh, kh, d, 64, capacity=T)
+    gen = torch.Generator(device="cuda").manual_seed(T)
+
+    def values(*shape, dtype=torch.bfloat16):
+        return torch.randn(shape, generator=gen, device="cuda").to(dtype)
+    args = (p, values(T, qh, 2, d), values(T, kh, d), values(T, kh, d), values(d, dtype=torch.float32),
+            values(d, dtype=torch.float32), values(T, qh, d, dtype=torch.float32))
+    together = capi.gqa_prefill_backward(*args)
+    with capi.only_kernels(capi.QUERY_KERNEL | capi.AUXILIARY_KERNELS):
+        queries = capi.gqa_prefill_backward(*args)
+    with capi.only_kernels(capi.MAIN_KERNEL | capi.AUXILIARY_KERNELS):
+        keys = capi.gqa_prefill_backward(*args)
+    torch.cuda.synchronize()
+    assert all(torch.isfinite(g).all() for g in together)
+    assert torch.equal(together[0], queries[0])
+    assert torch.equal(together[1], keys[1]) and torch.equal(together[2], keys[2])
+
+
 def test_long_sequence_with_saved_state_matches_oracle(capi):
     """T=1024, one kv group of six 128-wide heads (the grouping of the benchmarked
     shape): eight query tiles, so the unpaired heaviest-first grid, with the block
