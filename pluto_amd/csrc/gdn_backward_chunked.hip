@@ -68,9 +68,9 @@ struct Records {
   // of a key head                                                        [64][128]
   float *q_rows, *q_columns, *k_rows, *k_columns;
   float *w_rows, *w_columns;                          // W              [64][128]
-  float *u_columns, *dl_rows, *ddl_rows, *ddl_columns;  // U, Dl, dDl    [64][128]
+  float *u_columns, *dl_rows, *ddl_rows;              // U, Dl, dDl     [64][128]
   float *p_rows, *p_columns;                          // P               [64][64]
-  float *t_rows, *t_columns;                          // T               [64][64]
+  float *t_columns;                                   // T               [64][64]
   float *kkd;                 // columns(strict_lower((k^_i . k^_j) D_ij)) [64][64]
   float *gates;               // [6][64], see Gate
   float *s0, *ds1;            // rows(state entering the chunk), rows(gradient of the one leaving)
@@ -81,7 +81,7 @@ struct Records {
 enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kGateRows };
 
 constexpr size_t kKeyRecordFloats = 4 * static_cast<size_t>(kWide);
-constexpr size_t kRecordFloats = 6 * static_cast<size_t>(kWide) + 5 * kSquare + kGateRows * kC +
+constexpr size_t kRecordFloats = 5 * static_cast<size_t>(kWide) + 4 * kSquare + kGateRows * kC +
                                  2 * static_cast<size_t>(kState);
 
 struct ChunkedArgs {
@@ -530,10 +530,9 @@ chunk_prepare_kernel(ChunkedArgs a) {
   __builtin_amdgcn_sched_barrier(0);
   lds_barrier();
   {
-    const Record t_rows = v.square(a.r.t_rows), t_columns = v.square(a.r.t_columns);
+    const Record t_columns = v.square(a.r.t_columns);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      t_rows.put4(load4(&sm.t[16 * wave + n16][16 * s + 4 * quarter]), 16 * lane, piece_at<kC>(wave, 4 * s));
       t_columns.put4(gather4(&sm.t[16 * s + 4 * quarter][16 * wave + n16], kSquarePad), 16 * lane,
                      piece_at<kC>(wave, 4 * s));
     }
@@ -894,9 +893,7 @@ chunk_states_backward_kernel(ChunkedArgs a) {
     float decay;
     const Record k_memory = head_records(a, a.r.k_rows, key_head, kWide),
                  w_memory = head_records(a, a.r.w_columns, head, kWide),
-                 ddl_memory = head_records(a, a.r.ddl_columns, head, kWide),
                  ddl_rows = head_records(a, a.r.ddl_rows, head, kWide), ds1_memory = head_records(a, a.r.ds1, head, kState);
-    const unsigned delta_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
     const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;  // as above
     auto request_k = [&](int s) { k[s] = k_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
     auto request_w = [&](int t, int s) { w[t][s] = w_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
@@ -968,7 +965,6 @@ chunk_states_backward_kernel(ChunkedArgs a) {
       keep_order();
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
-        ddl_memory.put4(dd[c], wide_now, delta_at + piece_at<kC>(c, 0));
         ddl_rows.put4(quad_transpose(dd[c]), wide_now + transposed_at,
                       piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
       }
@@ -1060,7 +1056,12 @@ chunk_states_backward_kernel(ChunkedArgs a) {
 //      dv = diag(beta) T^T dDl;  dq and dk back through the normalisations
 //   4. d log-decay and d beta from row and column sums of the above, through the gates
 //      to da, db and the contribution to d A_log
-// 75 KiB of LDS and 256 registers: two workgroups a compute unit.
+// 75 KiB of LDS and 256 registers, none of them spilled: two workgroups a compute unit.  2048
+// tokens of 48 heads 267 -> 226 us when 45 registers no longer went to scratch (140 MB there
+// and back): the contributions of U before those of W, one product's accumulator at a time,
+// and a sum whose factors the compiler kept for its end.  dDl and T are read here in the one
+// order they are kept in and exchanged between lanes (230 us; the kernels that write them 137
+// -> 129 and 106 -> 103).
 constexpr int kSlab = 32;
 constexpr unsigned kSlabBytes = kC * kSlab * 4;
 struct GradientSmem {
@@ -1098,14 +1099,13 @@ chunk_gradients_kernel(ChunkedArgs a) {
   float dot = 0.0f;
   const int tile_col = 32 * tj_own + n;
   const unsigned square_at = lane_piece<kC>(h, n);
-  const Record p_memory = v.square(a.r.p_columns), kkd = v.square(a.r.kkd), t_rows = v.square(a.r.t_rows),
-               t_columns = v.square(a.r.t_columns), ddl = v.wide(a.r.ddl_columns), q_memory = v.key(a.r.q_columns),
-               k_memory = v.key(a.r.k_columns), k_rows = v.key(a.r.k_rows);
-  const Tokens v_memory = v.v(), dv = v.dv();
   // the lane's places in columns(M) of [64, 64] and [64, 128] matrices (four rows of one
   // column, as in an accumulator), and a token's in the activations
   const unsigned tile_at = square_at + piece_at<kC>(2 * tj_own, 8 * ti_own);
   const unsigned column_at = square_at + piece_at<kC>(2 * wave, 0);
+  // Rows of a matrix that is kept in columns, and the other way round: four columns of one of
+  // four rows a lane, exchanged between neighbouring lanes when they have arrived.
+  const unsigned quad_at = n / 4 * kPiece + (4 * h + n % 4) * 16;
   // rows of tokens are read and written four columns of one token a lane: token n % 4 of
   // the four of a register quad, columns 4 (n / 4) .. + 3 of the wave's
   const unsigned token_row = 4 * h + n % 4, token_column = 4 * (32 * wave + n / 4 * 4);
@@ -1167,6 +1167,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         dot += (s0[g].x * s1[g].x + s0[g].y * s1[g].y) + (s0[g].z * s1[g].z + s0[g].w * s1[g].w);
+        asm volatile("" : "+v"(dot));  // here, not where it is needed: its factors' registers are
 #pragma unroll
         for (int ti = 0; ti < 2; ++ti) {
           dw[ti] = mma(dw[ti], operand(0, ti, g), s0[g]);
@@ -1193,8 +1194,11 @@ chunk_gradients_kernel(ChunkedArgs a) {
     for (int i = 0; i < 16; ++i) sm.dw[32 * ti + tile_row(i, h)][col] = -dw[ti][i];
   keep_order();
   // Everything the [64, 64] part reads is requested a step before it is used.
+  // (Descriptors of what is read or written are made where that is: all at once they do not
+  // fit in the scalar registers and go to scratch.)
   float4 p_tile[4], k_own[kD / 8];
   if (lower) {
+    const Record p_memory = v.square(a.r.p_columns), k_rows = v.key(a.r.k_rows);
 #pragma unroll
     for (int j = 0; j < 4; ++j) p_tile[j] = p_memory.get4(tile_at, piece_at<kC>(0, 2 * j));
     keep_order();
@@ -1232,6 +1236,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
   float4 t_own[8];  // T^T for rows of the tile, then T for its columns
   keep_order();
   if (lower) {
+    const Record t_columns = v.square(a.r.t_columns);
 #pragma unroll
     for (int s = 0; s < 8; ++s)
       if (s >= 4 * ti_own) t_own[s] = t_columns.get4(square_at, piece_at<kC>(2 * ti_own, 2 * s));
@@ -1249,6 +1254,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
   keep_order();
   // columns of K^ and Q^, both as operands and in the accumulators' rows
   float4 kc[8], qc[8], kkd_tile[4];
+  const Record k_memory = v.key(a.r.k_columns);
 #pragma unroll
   for (int s = 0; s < 8; ++s) kc[s] = k_memory.get4(column_at, piece_at<kC>(0, 2 * s));
   keep_order();
@@ -1260,13 +1266,15 @@ chunk_gradients_kernel(ChunkedArgs a) {
     for (int s = 0; s < 8; ++s)
       if (s >= 4 * ti_own) z = mma(z, t_own[s], gather4(&sm.x[8 * s + 4 * h][tile_col], kSquarePad));
     keep_order();
+    const Record t_columns = v.square(a.r.t_columns), kkd = v.square(a.r.kkd);
 #pragma unroll
     for (int s = 0; s < 8; ++s)
-      if (s < 4 * (tj_own + 1)) t_own[s] = t_rows.get4(square_at, piece_at<kC>(2 * tj_own, 2 * s));
+      if (s < 4 * (tj_own + 1)) t_own[s] = t_columns.get4(quad_at, piece_at<kC>(s / 2, 8 * tj_own) + 128 * (s % 2));
 #pragma unroll
     for (int j = 0; j < 4; ++j) kkd_tile[j] = kkd.get4(tile_at, piece_at<kC>(0, 2 * j));
   }
   keep_order();
+  const Record q_memory = v.key(a.r.q_columns);
 #pragma unroll
   for (int s = 0; s < 8; ++s) qc[s] = q_memory.get4(column_at, piece_at<kC>(0, 2 * s));
   keep_order();
@@ -1280,7 +1288,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
   if (lower) {
 #pragma unroll
     for (int s = 0; s < 8; ++s)
-      if (s < 4 * (tj_own + 1)) da = mma(da, load4(&sm.x[32 * ti_own + n][8 * s + 4 * h]), t_own[s]);
+      if (s < 4 * (tj_own + 1)) da = mma(da, load4(&sm.x[32 * ti_own + n][8 * s + 4 * h]), quad_transpose(t_own[s]));
   }
   lds_barrier();
   if (lower) {
@@ -1299,10 +1307,12 @@ chunk_gradients_kernel(ChunkedArgs a) {
   keep_order();
   // T^T for both row tiles (the columns of T of the second start at row 32), dDl's columns
   float4 t_first[8], t_second[4], dd[8];
+  const Record t_columns = v.square(a.r.t_columns), ddl = v.wide(a.r.ddl_rows);
+  const Tokens v_memory = v.v(), dv = v.dv();
 #pragma unroll
   for (int s = 0; s < 8; ++s) t_first[s] = t_columns.get4(square_at, piece_at<kC>(0, 2 * s));
 #pragma unroll
-  for (int s = 0; s < 8; ++s) dd[s] = ddl.get4(column_at, piece_at<kC>(0, 2 * s));
+  for (int s = 0; s < 8; ++s) dd[s] = ddl.get4(quad_at, piece_at<kD>(s / 2, 8 * wave) + 128 * (s % 2));
   keep_order();
   auto row_sums = [&](RowSum which, int ti, const float (&values)[16]) {
     const float sum = half_sums(values);
@@ -1327,43 +1337,51 @@ chunk_gradients_kernel(ChunkedArgs a) {
   keep_order();
   lds_barrier();
 #pragma unroll
+  for (int s = 0; s < 8; ++s) dd[s] = quad_transpose(dd[s]);
+#pragma unroll
   for (int ti = 0; ti < 2; ++ti) {
     const int m = 32 * ti + n;
     auto t_col = [&](int s) { return ti == 0 ? t_first[s] : t_second[s - 4]; };
     float products[16];
-    floatx16 tu = zero_tile();
-#pragma unroll
-    for (int s = 4 * ti; s < 8; ++s) tu = mma(tu, t_col(s), dd[s]);
-    floatx16 tw = zero_tile();
-#pragma unroll
-    for (int s = 4 * ti; s < 8; ++s) tw = mma(tw, t_col(s), gather4(&sm.dw[8 * s + 4 * h][col], kWidePad));
-    keep_order();
     float4 values[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) values[j] = v_memory.get4(token_at, (32 * ti + 8 * j) * v.row_bytes);
-    if (ti == 0) {
+    keep_order();
+    {
+      floatx16 tu = zero_tile();
 #pragma unroll
-      for (int s = 4; s < 8; ++s) t_second[s - 4] = t_columns.get4(square_at, piece_at<kC>(2, 2 * s));
+      for (int s = 4 * ti; s < 8; ++s) tu = mma(tu, t_col(s), dd[s]);
+      keep_order();
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 value = quad_transpose(values[j]), beta = rows4(sm.gate[kBeta], ti, j);
+        products[4 * j] = tu[4 * j] * value.x, products[4 * j + 1] = tu[4 * j + 1] * value.y;
+        products[4 * j + 2] = tu[4 * j + 2] * value.z, products[4 * j + 3] = tu[4 * j + 3] * value.w;
+        dv.put4(quad_transpose(make_float4(beta.x * tu[4 * j], beta.y * tu[4 * j + 1], beta.z * tu[4 * j + 2],
+                                           beta.w * tu[4 * j + 3])),
+                token_at, (32 * ti + 8 * j) * v.row_bytes);
+      }
+      row_sums(kSumV, ti, products);
     }
     keep_order();
+    {
+      floatx16 tw = zero_tile();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float e = element(rows4(sm.gate[kE], ti, i / 4), i);
-      products[i] = tw[i] * element(kc[4 * ti + i / 4], i) * e;
-      dk[ti][i] += element(rows4(sm.gate[kBeta], ti, i / 4), i) * e * tw[i];
-    }
-    row_sums(kSumW, ti, products);
-    keep_order();
+      for (int s = 4 * ti; s < 8; ++s) tw = mma(tw, t_col(s), gather4(&sm.dw[8 * s + 4 * h][col], kWidePad));
+      keep_order();
+      if (ti == 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float4 value = quad_transpose(values[j]), beta = rows4(sm.gate[kBeta], ti, j);
-      products[4 * j] = tu[4 * j] * value.x, products[4 * j + 1] = tu[4 * j + 1] * value.y;
-      products[4 * j + 2] = tu[4 * j + 2] * value.z, products[4 * j + 3] = tu[4 * j + 3] * value.w;
-      dv.put4(quad_transpose(make_float4(beta.x * tu[4 * j], beta.y * tu[4 * j + 1], beta.z * tu[4 * j + 2],
-                                         beta.w * tu[4 * j + 3])),
-              token_at, (32 * ti + 8 * j) * v.row_bytes);
+        for (int s = 4; s < 8; ++s) t_second[s - 4] = t_columns.get4(square_at, piece_at<kC>(2, 2 * s));
+      }
+      keep_order();
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float e = element(rows4(sm.gate[kE], ti, i / 4), i);
+        products[i] = tw[i] * element(kc[4 * ti + i / 4], i) * e;
+        dk[ti][i] += element(rows4(sm.gate[kBeta], ti, i / 4), i) * e * tw[i];
+      }
+      row_sums(kSumW, ti, products);
     }
-    row_sums(kSumV, ti, products);
     keep_order();
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -1471,10 +1489,8 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
   a.r.u_columns = take(kWide);
   a.r.dl_rows = take(kWide);
   a.r.ddl_rows = take(kWide);
-  a.r.ddl_columns = take(kWide);
   a.r.p_rows = take(kSquare);
   a.r.p_columns = take(kSquare);
-  a.r.t_rows = take(kSquare);
   a.r.t_columns = take(kSquare);
   a.r.kkd = take(kSquare);
   a.r.gates = take(kGateRows * kC);
