@@ -93,9 +93,9 @@ int launch_gdn_output(hipStream_t stream, const void* core, int core_dtype, cons
 
 // Chunked form of the recurrence part of the backward for 128 x 128 heads
 // (gdn_backward_chunked.hip): `forward` leaves the outputs in `core`, `reverse`
-// (after `dcore` is known) leaves dv in `dpost` and the q/k and gate gradients
-// as one partial per (token, value head), in the layout the token-by-token
-// kernels use with a single column tile.
+// (after `dcore` is known) leaves dv in `dpost`, da and db, the q/k gradients as one
+// partial per (token, value head), in the layout the token-by-token kernels use with
+// a single column tile, and the parameters' of the gates as one per (chunk, value head).
 struct GdnChunkedBackward {
   const float* post = nullptr;   // [T, channels] convolved, activated q | k | v
   const uint16_t* a = nullptr;   // bf16 [T, vh]
@@ -106,7 +106,9 @@ struct GdnChunkedBackward {
   float* core = nullptr;         // [T, vh, 128]
   float* dpost = nullptr;
   float* qk_partials = nullptr;      // [T, vh, 2, 128]
-  float* scalar_partials = nullptr;  // [T, vh, 3]
+  float* da = nullptr;               // [T, vh]
+  float* db = nullptr;
+  float* scalar_partials = nullptr;  // [chunks, vh, 2]: parts of d A_log and d dt_bias
   float* records = nullptr;          // gdn_backward_chunked_bytes(...)
   int length = 0, key_heads = 0, value_heads = 0;
   bool round = true;

@@ -8,7 +8,8 @@
 //   output_backward_kernel       OutputBackward         (:125-155)
 //   recurrence_backward_kernel   RecurrenceBackward     (:171-253)
 //   gather_qk_kernel             GatherQkGradient       (:255-276)
-//   gather_scalar_kernel         GatherScalarGradient   (:278-305)
+//   gather_scalar_kernel         GatherScalarGradient   (:278-305); finish_parameters_kernel
+//                                with the chunked kernels
 //   conv_silu_backward_kernel    ConvSiluBackward       (:307-318)
 //   conv_input_backward_kernel   ConvInputBackward      (:320-336)
 //   conv_weight_*_kernel         ConvWeightBackward     (:338-355), two levels
@@ -849,6 +850,79 @@ conv_weight_final_kernel(const float* partial, long long elements, int slices, f
   dw[i] += sum;
 }
 
+// The ends of the chunked backward's parameter gradients in one launch: the first blocks add
+// up the norm's as sum_columns_kernel does, two columns each, the next the gates', 32 heads
+// each, and the rest the convolution's.  (Three launches of 4.9, 9.5 and 4.7 us at 2048 tokens
+// of 48 heads, most of it the arrival of code and arguments, now 5.6; da and db came the way of
+// the gates' parameters then.)
+struct FinishArgs {
+  const float* norm_parts = nullptr;    // [norm_rows, norm_width]
+  float* d_norm = nullptr;
+  int norm_rows = 0, norm_width = 0, norm_blocks = 0;
+  const float* scalar_parts = nullptr;  // [chunks, heads, 2]
+  float *d_a_log = nullptr, *d_dt_bias = nullptr;
+  int chunks = 0, heads = 0, head_blocks = 0;
+  const float* conv_parts = nullptr;    // [slices, weights]
+  float* d_conv = nullptr;
+  long long weights = 0;
+  int slices = 0;
+};
+__global__ void __launch_bounds__(256)
+finish_parameters_kernel(FinishArgs a) {
+  const int tid = threadIdx.x, block = blockIdx.x;
+  if (block < a.norm_blocks) {
+    __shared__ float sums[128][2], groups[16][2];
+    const int k = tid % 2, g = tid / 2, c = 2 * block + k;
+    float sum = 0.0f;
+#pragma unroll 8
+    for (int row = g; row < a.norm_rows; row += 128) sum += a.norm_parts[1LL * row * a.norm_width + c];
+    sums[g][k] = sum;
+    __syncthreads();
+    if (g < 16) {
+      float total = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) total += sums[8 * g + i][k];
+      groups[g][k] = total;
+    }
+    __syncthreads();
+    if (g != 0) return;
+    float total = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) total += groups[i][k];
+    a.d_norm[c] += total;
+    return;
+  }
+  if (block < a.norm_blocks + a.head_blocks) {
+    // a head's chunks in eight parts
+    __shared__ float parts[8][32][2];
+    const int head = 32 * (block - a.norm_blocks) + tid % 32, part = tid / 32;
+    float log_sum = 0.0f, bias_sum = 0.0f;
+    if (head < a.heads) {
+#pragma unroll 4
+      for (int chunk = part; chunk < a.chunks; chunk += 8) {
+        const float2 v = *reinterpret_cast<const float2*>(a.scalar_parts + 2 * (1LL * chunk * a.heads + head));
+        log_sum += v.x;
+        bias_sum += v.y;
+      }
+    }
+    parts[part][tid % 32][0] = log_sum;
+    parts[part][tid % 32][1] = bias_sum;
+    __syncthreads();
+    if (part != 0 || head >= a.heads) return;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) log_sum += parts[i][tid][0], bias_sum += parts[i][tid][1];
+    if (a.d_a_log) a.d_a_log[head] += log_sum;
+    if (a.d_dt_bias) a.d_dt_bias[head] += bias_sum;
+    return;
+  }
+  const long long i = (block - a.norm_blocks - a.head_blocks) * 256LL + tid;
+  if (i >= a.weights) return;
+  float sum = 0.0f;
+#pragma unroll 16
+  for (int slice = 0; slice < a.slices; ++slice) sum += a.conv_parts[slice * a.weights + i];
+  a.d_conv[i] += sum;
+}
+
 // gradient[c] += sum over rows of partials[row, c], two levels, fixed order.
 // Sum of rows first..last-1 of a [rows, width] matrix (width <= 256), per
 // column.  The 256 threads form up to 8 groups of `width`; group g takes rows
@@ -1007,6 +1081,8 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
   c.core = core;
   c.dpost = dpost;
   c.qk_partials = qk_partials;
+  c.da = da;
+  c.db = db;
   c.scalar_partials = scalar_partials;
   c.records = states;
   c.length = length;
@@ -1020,6 +1096,7 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     status = launch_status();
   }
   if (status != 0) return status;
+  int norm_rows = 0;  // of the partial sums for the norm's gradient
   if (vd == 128) {
     const long long rows = 1LL * length * vh, runs = (rows + 15) / 16;
     const int blocks = static_cast<int>(runs < kOutputBlocks ? runs : kOutputBlocks);
@@ -1030,7 +1107,8 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     else
       output_backward128_kernel<false><<<blocks, 256, 0, stream>>>(
           core, gates, norm, dy, rows, p->rms_norm_epsilon, round, dcore, dz, norm_partials);
-    if (d_norm) sum_columns_kernel<<<16, 1024, 0, stream>>>(norm_partials, blocks, vd, d_norm);
+    norm_rows = blocks;
+    if (d_norm && !chunked) sum_columns_kernel<<<16, 1024, 0, stream>>>(norm_partials, blocks, vd, d_norm);
   } else {
     output_backward_kernel<<<static_cast<unsigned>(length) * vh, 64, 0, stream>>>(
         core, static_cast<const uint16_t*>(z), norm, dy, vd, p->rms_norm_epsilon, round, dcore, dz,
@@ -1052,9 +1130,37 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
     status = launch_status();
   }
   if (status != 0) return status;
-  gather_scalar_kernel<<<vh, 256, 0, stream>>>(scalar_partials, length, vh, tiles, da, db, d_a_log,
-                                               d_dt_bias);
+  if (!chunked)
+    gather_scalar_kernel<<<vh, 256, 0, stream>>>(scalar_partials, length, vh, tiles, da, db, d_a_log,
+                                                 d_dt_bias);
   const long long weights = 1LL * channels * kernel;
+  auto finish_parameters = [&](int conv_slices) {
+    if (!chunked) {
+      if (d_conv_weight)
+        conv_weight_final_kernel<<<blocks_for(weights), 256, 0, stream>>>(conv_partials, weights, conv_slices,
+                                                                          d_conv_weight);
+      return launch_status();
+    }
+    FinishArgs f;
+    f.norm_parts = norm_partials;
+    f.d_norm = d_norm;
+    f.norm_rows = norm_rows;
+    f.norm_width = vd;
+    f.norm_blocks = d_norm ? vd / 2 : 0;
+    f.scalar_parts = scalar_partials;
+    f.d_a_log = d_a_log;
+    f.d_dt_bias = d_dt_bias;
+    f.chunks = (length + 63) / 64;
+    f.heads = vh;
+    f.head_blocks = d_a_log || d_dt_bias ? (vh + 31) / 32 : 0;
+    f.conv_parts = conv_partials;
+    f.d_conv = d_conv_weight;
+    f.weights = d_conv_weight ? weights : 0;
+    f.slices = conv_slices;
+    const unsigned blocks = f.norm_blocks + f.head_blocks + static_cast<unsigned>((f.weights + 255) / 256);
+    if (blocks > 0) finish_parameters_kernel<<<blocks, 256, 0, stream>>>(f);
+    return launch_status();
+  };
   if (taps4) {
     ConvBackwardArgs b;
     b.input = static_cast<const uint16_t*>(qkv);
@@ -1080,10 +1186,7 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
       conv_backward4_kernel<true><<<grid, 256, 0, stream>>>(b);
     else
       conv_backward4_kernel<false><<<grid, 256, 0, stream>>>(b);
-    if (d_conv_weight)
-      conv_weight_final_kernel<<<blocks_for(weights), 256, 0, stream>>>(conv_partials, weights, runs,
-                                                                        d_conv_weight);
-    return launch_status();
+    return finish_parameters(runs);
   }
   gather_qk_kernel<<<dim3(kh, length), 128, 0, stream>>>(qk_partials, kh, vh, kd, tiles, channels,
                                                          dpost);
@@ -1095,14 +1198,11 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
                                                                            dpre);
   conv_input_backward_kernel<1><<<blocks_for(elements), 256, 0, stream>>>(
       dpre, conv_weight, length, channels, kernel, dqkv);
-  if (d_conv_weight) {
+  if (d_conv_weight)
     conv_weight_partial_kernel<<<dim3((channels + 255) / 256, kernel, kConvSlices), 256, 0, stream>>>(
         static_cast<const uint16_t*>(qkv), dpre, length, channels, kernel, kConvSlices,
         conv_partials);
-    conv_weight_final_kernel<<<blocks_for(weights), 256, 0, stream>>>(conv_partials, weights,
-                                                                      kConvSlices, d_conv_weight);
-  }
-  return launch_status();
+  return finish_parameters(kConvSlices);
 }
 
 }  // namespace pluto_hip

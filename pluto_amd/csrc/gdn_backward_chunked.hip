@@ -94,7 +94,9 @@ struct ChunkedArgs {
   float* core = nullptr;           // [T, vh, 128]
   float* dpost = nullptr;          // [T, channels]: the value part is written
   float* qk_partials = nullptr;    // [T, vh, 2, 128]
-  float* scalar_partials = nullptr;  // [T, vh, 3]
+  float* da = nullptr;             // [T, vh]
+  float* db = nullptr;
+  float* scalar_partials = nullptr;  // [chunks, vh, 2]: a chunk's part of d A_log and d dt_bias
   Records r;
   int length = 0, chunks = 0, kh = 0, vh = 0;
   bool round = true;
@@ -1446,18 +1448,25 @@ chunk_gradients_kernel(ChunkedArgs a) {
     const float after = __shfl_down(dg, offset, 64);
     if (lane + offset < 64) dg += after;
   }
-  const int t = v.t0 + lane;
-  if (lane >= v.tokens) return;
+  const bool valid = lane < v.tokens;
+  const size_t at = static_cast<size_t>(v.t0 + min(lane, v.tokens - 1)) * a.vh + v.head;
   const float dbeta = row_n + r + across_waves(kSumV, lane);
-  const float alpha = bf16_bits_to_float(a.a[static_cast<size_t>(t) * a.vh + v.head]) + a.dt_bias[v.head];
+  const float alpha = bf16_bits_to_float(a.a[at]) + a.dt_bias[v.head];
   const float softplus = fmaxf(alpha, 0.0f) + logf(1.0f + expf(-fabsf(alpha)));
   const float rate = expf(a.a_log[v.head]);
-  const float bv = bf16_bits_to_float(a.b[static_cast<size_t>(t) * a.vh + v.head]);
+  const float bv = bf16_bits_to_float(a.b[at]);
   const float sigmoid = 1.0f / (1.0f + expf(-bv));
-  float* out = a.scalar_partials + (static_cast<size_t>(t) * a.vh + v.head) * 3;
-  out[0] = -dg * rate / (1.0f + expf(-alpha));
-  out[1] = dbeta * sigmoid * (1.0f - sigmoid);
-  out[2] = -dg * rate * softplus;
+  const float d_alpha = -dg * rate / (1.0f + expf(-alpha));
+  if (valid) {
+    a.da[at] = d_alpha;
+    a.db[at] = dbeta * sigmoid * (1.0f - sigmoid);
+  }
+  const float log_sum = wave_sum(valid ? -dg * rate * softplus : 0.0f), bias_sum = wave_sum(valid ? d_alpha : 0.0f);
+  if (lane == 0) {
+    float* out = a.scalar_partials + (static_cast<size_t>(blockIdx.x) * a.vh + v.head) * 2;
+    out[0] = log_sum;
+    out[1] = bias_sum;
+  }
 }
 
 ChunkedArgs make_args(const GdnChunkedBackward& c) {
@@ -1471,6 +1480,8 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
   a.core = c.core;
   a.dpost = c.dpost;
   a.qk_partials = c.qk_partials;
+  a.da = c.da;
+  a.db = c.db;
   a.scalar_partials = c.scalar_partials;
   a.length = c.length;
   a.chunks = (c.length + kC - 1) / kC;

@@ -333,3 +333,29 @@ def test_values_near_the_top_of_the_range_stay_finite(capi):
         a, b = a.cpu().numpy(), b.cpu().numpy()
         assert np.isfinite(b).all() and np.isfinite(a).all(), name
         assert_close(a, b, 2e-4, name)  # the tolerance against the oracle
+
+
+@pytest.mark.parametrize("T,kh,vh,taps", [(1, 1, 1, 4), (65, 3, 33, 4), (200, 2, 2, 3)])
+def test_each_parameter_gradient_alone(capi, T, kh, vh, taps):
+    """The chunked backward ends with one launch over whichever parameters have gradients:
+    any of them alone has the bits it has with the others, none is a valid call, and what
+    a head's time steps share, dt_bias, has the sum of their gradients (256 additions at
+    most, each within 2^-24 of the magnitudes so far)."""
+    c = make_case(T, kh, vh, 128, 128, taps, seed=T)
+    p = capi.delta_params(kh, vh, 128, 128, taps)
+    bf = torch.bfloat16
+    args = [dev(c["qkv"], bf), dev(c["z"], bf), dev(c["a"], bf), dev(c["b"], bf), dev(c["conv"]), dev(c["a_log"]),
+            dev(c["dt_bias"]), dev(c["norm"]), dev(c["dy"])]
+    shapes = dict(conv_weight=c["conv"].shape, a_log=(vh,), dt_bias=(vh,), norm=(128,))
+    zeros = lambda *names: {n: torch.zeros(shapes[n], device="cuda") for n in names}
+    every = zeros(*shapes)
+    activations = capi.gdn_layer_backward(p, *args, parameter_grads=every)
+    for name in list(shapes) + [None]:
+        one = zeros(*([name] if name else []))
+        again = capi.gdn_layer_backward(p, *args, parameter_grads=one)
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(activations, again)), name
+        if name:
+            assert torch.equal(one[name], every[name]), name
+    da = activations[2].double()
+    assert ((every["dt_bias"].double() - da.sum((0, 1))).abs() <= 256 * 2.0 ** -24 * da.abs().sum((0, 1)) + 1e-30).all()
