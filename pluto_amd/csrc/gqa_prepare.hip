@@ -96,33 +96,49 @@ prefill_prepare_kernel(PrefillPrepareArgs a) {
 
 // Vectorised form of the same preparation for bf16 inputs, a bf16 query buffer
 // and a bf16 cache with rounding on: a thread owns 8 consecutive channels (one
-// 16-byte load and store), the D/8 threads of a (row, head) are neighbouring
-// lanes.  Requires rotary_dim/2 to be a multiple of 8 so that a thread's RoPE
-// partners all sit in one other thread.  Arithmetic and rounding points are
-// those of normalize_rotate above.  ANGLES: the workgroup makes the cosines and sines of
-// its rows itself, while the rows travel, instead of reading the table.
-template <int D, bool ANGLES>
-__global__ void __launch_bounds__(256)
-prefill_prepare_bf16_kernel(PrefillPrepareArgs a, std::conditional_t<ANGLES, RopeFrequencies, int> frequencies) {
-  constexpr int LANES = D / 8, UNITS = 256 / LANES;
-  __shared__ __attribute__((aligned(16))) float angles[2][ANGLES ? UNITS * (D / 2) : 4];
-  const int heads = a.query_heads + a.key_value_heads;
-  const long long thread = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  const long long units = static_cast<long long>(a.length) * heads;
-  const long long unit = min(thread / LANES, units - 1);
-  const bool outside = thread / LANES >= units;  // whole groups
-  const int first_row = static_cast<int>(static_cast<long long>(blockIdx.x) * UNITS / heads);
-  const int chunk = static_cast<int>(thread % LANES);
-  const int row = static_cast<int>(unit / heads);
-  const int head = static_cast<int>(unit % heads);
+// 16-byte load and store), the D/8 threads of a head are neighbouring lanes, a workgroup
+// has `group` heads of one row (all that fit).  Requires rotary_dim/2 to be a multiple of 8
+// so that a thread's RoPE partners all sit in one other thread.  Arithmetic and rounding
+// points are those of normalize_rotate above.  The cosines and sines of the row are made
+// by a wave of their own while the others normalise; a caller that reads them later finds
+// them in the table.  24 + 4 heads, with a launch for the table in front and so: 1531 rows of
+// 256 channels 4.8 + 14.0 and 13.9 us, 8192 rows of 128 4.9 + 33.8 and 34.4, 300 rows of 256
+// (angles made by 2100 workgroups of 256 threads) 7.6 and 6.7.  Workgroups of 1024 threads hold
+// two a compute unit back at their barrier: 5000 rows of 256 channels 49 us, 42.5 in those of
+// 512.
+constexpr int kPrepareThreads = 512;
+template <int D>
+__global__ void __launch_bounds__(kPrepareThreads)
+prefill_prepare_bf16_kernel(PrefillPrepareArgs a, RopeFrequencies frequencies, int group) {
+  constexpr int LANES = D / 8;
+  __shared__ __attribute__((aligned(16))) float cosines[128], sines[128];
+  const int row = blockIdx.x, part = blockIdx.y;
   const int half = a.rotary_dim / 2;
+  if (threadIdx.x >= blockDim.x - 64) {
+    for (int f = threadIdx.x % 64; f < half; f += 64) {
+      float c, s;
+      rope_angle(a.start_position + row, frequencies.value[f], a.round, c, s);
+      cosines[f] = c;
+      sines[f] = s;
+      if (a.keep_table && part == 0) {
+        a.cosines[static_cast<long long>(row) * half + f] = c;
+        a.sines[static_cast<long long>(row) * half + f] = s;
+      }
+    }
+    __syncthreads();
+    return;
+  }
+  const int heads = a.query_heads + a.key_value_heads;
+  const int own_head = part * group + threadIdx.x / LANES, head = min(own_head, heads - 1);
+  const bool outside = own_head >= heads || static_cast<int>(threadIdx.x / LANES) >= group;  // whole groups
+  const int chunk = static_cast<int>(threadIdx.x % LANES);
   const bool is_query = head < a.query_heads;
   const int kv = head - a.query_heads;
   const uint16_t* in;
   uint16_t* out;
   uint16_t* copy;
   const float* weight;
-  // the unit's place among the heads of its side
+  // the head's place among the heads of its side
   const long long at = (is_query ? static_cast<long long>(row) * a.query_heads + head
                                  : static_cast<long long>(row) * a.key_value_heads + kv) * D;
   if (is_query) {
@@ -139,15 +155,6 @@ prefill_prepare_bf16_kernel(PrefillPrepareArgs a, std::conditional_t<ANGLES, Rop
     weight = a.k_norm;
   }
   const uint4 bits = *reinterpret_cast<const uint4*>(in + 8 * chunk);
-  if constexpr (ANGLES) {
-    const long long last_unit = min(static_cast<long long>(blockIdx.x + 1) * UNITS, units) - 1;
-    const int count = (static_cast<int>(last_unit / heads) - first_row + 1) * half;
-    for (int i = threadIdx.x; i < count; i += 256)
-      rope_angle(a.start_position + first_row + i / half, frequencies.value[i % half], a.round, angles[0][i],
-                 angles[1][i]);
-    __syncthreads();
-  }
-  if (outside) return;
   const uint32_t words[4] = {bits.x, bits.y, bits.z, bits.w};
   float x[8];
 #pragma unroll
@@ -183,12 +190,11 @@ prefill_prepare_bf16_kernel(PrefillPrepareArgs a, std::conditional_t<ANGLES, Rop
   uint32_t partner[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) partner[i] = __shfl(normalized[i], partner_lane, 64);
+  __syncthreads();
+  if (outside) return;
   uint32_t result[4] = {normalized[0], normalized[1], normalized[2], normalized[3]};
   if (rotated) {
-    const long long table =
-        static_cast<long long>(row - (ANGLES ? first_row : 0)) * half + (lower ? first : first - half);
-    const float* cosines = ANGLES ? angles[0] : a.cosines;
-    const float* sines = ANGLES ? angles[1] : a.sines;
+    const int table = lower ? first : first - half;
     const float4 c0 = *reinterpret_cast<const float4*>(cosines + table);
     const float4 c1 = *reinterpret_cast<const float4*>(cosines + table + 4);
     const float4 s0 = *reinterpret_cast<const float4*>(sines + table);
@@ -271,11 +277,6 @@ decode_prepare_kernel(DecodePrepareArgs a, DecodeBatch batch) {
 
 }  // namespace
 
-// Below, what is left of a table launch (5 us) is more than the angles cost when every
-// workgroup makes those of its rows: 19 rows of 24 + 4 heads of 256 channels took 20.0 us
-// in all with the table, 18.1 without.
-constexpr long long kOwnAnglesBlocks = 2048;
-
 int launch_prefill_prepare(hipStream_t stream, const PrefillPrepareArgs& a) {
   const long long units =
       static_cast<long long>(a.length) * (a.query_heads + a.key_value_heads);
@@ -289,33 +290,27 @@ int launch_prefill_prepare(hipStream_t stream, const PrefillPrepareArgs& a) {
       aligned(a.k) && aligned(a.v) && aligned(a.q_out) && aligned(a.cache.keys) &&
       aligned(a.cache.values) && aligned(a.q_norm) && aligned(a.k_norm) && aligned(a.cosines) &&
       aligned(a.sines);
-  const long long blocks = (units * (d / 8) + 255) / 256;
   const RopeFrequencies& frequencies = rope_frequencies(a.theta, a.rotary_dim);
-  const bool own_angles = vectorised && !a.keep_table && blocks <= kOwnAnglesBlocks;
-  if (!own_angles) {
-    const long long count = static_cast<long long>(a.length) * (a.rotary_dim / 2);
-    if (count > 0) {
-      rope_table_kernel<<<static_cast<unsigned>((count + 255) / 256), 256, 0, stream>>>(
-          a.start_position, a.length, a.rotary_dim, frequencies, a.round, a.cosines, a.sines);
-      const int status = launch_status();
-      if (status != 0) return status;
-    }
-  }
   if (vectorised) {
-    auto launch = [&](auto width) {
-      constexpr int D = decltype(width)::value;
-      if (own_angles)
-        prefill_prepare_bf16_kernel<D, true><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(a, frequencies);
-      else
-        prefill_prepare_bf16_kernel<D, false><<<static_cast<unsigned>(blocks), 256, 0, stream>>>(a, 0);
-    };
+    // as many heads as fit in a workgroup beside the wave for the angles, in equal parts
+    const int heads = a.query_heads + a.key_value_heads, lanes = d / 8, most = (kPrepareThreads - 64) / lanes;
+    const int parts = (heads + most - 1) / most, group = (heads + parts - 1) / parts;
+    const int threads = (group * lanes + 63) / 64 * 64 + 64;
+    const dim3 grid(a.length, parts);
     if (d == 64)
-      launch(std::integral_constant<int, 64>());
+      prefill_prepare_bf16_kernel<64><<<grid, threads, 0, stream>>>(a, frequencies, group);
     else if (d == 128)
-      launch(std::integral_constant<int, 128>());
+      prefill_prepare_bf16_kernel<128><<<grid, threads, 0, stream>>>(a, frequencies, group);
     else
-      launch(std::integral_constant<int, 256>());
+      prefill_prepare_bf16_kernel<256><<<grid, threads, 0, stream>>>(a, frequencies, group);
     return launch_status();
+  }
+  const long long count = static_cast<long long>(a.length) * (a.rotary_dim / 2);
+  if (count > 0) {
+    rope_table_kernel<<<static_cast<unsigned>((count + 255) / 256), 256, 0, stream>>>(
+        a.start_position, a.length, a.rotary_dim, frequencies, a.round, a.cosines, a.sines);
+    const int status = launch_status();
+    if (status != 0) return status;
   }
   prefill_prepare_kernel<<<static_cast<unsigned>((units + 3) / 4), 256, 0, stream>>>(a);
   return launch_status();

@@ -732,3 +732,33 @@ def test_prefill_probabilities_are_causal_rows_that_match_decode(capi, oracle, d
     np.testing.assert_allclose(tail.astype(np.float64).sum(-1), 1.0, atol=2e-6)
     for row in range(5):
         assert np.all(tail[:, row, T + row + 1:] == 0) and np.all(tail[:, row, :T + row + 1] > 0)
+
+
+@pytest.mark.parametrize("qh,kh,d,rot", [(2, 1, 64, 16), (5, 1, 64, 64), (56, 8, 64, 16), (24, 4, 128, 32), (27, 3, 128, 128),
+                                         (14, 1, 256, 64), (13, 1, 256, 64), (32, 8, 256, 256)])
+@pytest.mark.parametrize("T", [1, 67])
+def test_preparation_by_rows_is_that_by_heads(capi, qh, kh, d, rot, T):
+    """One workgroup a row and group of heads, with heads that fill its waves, end within one,
+    or make several groups, against one wave a head and a table of angles (norm weights off a
+    16-byte boundary): cached keys and values, and so the output, have the same bits."""
+    start = 5
+    p = capi.attention_params(qh, kh, d, rot, capacity=start + T)
+    gen = torch.Generator(device="cuda").manual_seed(T + qh)
+
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda")
+    qg, k, v = (values(T, *s, d).to(torch.bfloat16) for s in ((qh, 2), (kh,), (kh,)))
+    norms = [0.3 * values(d), 0.3 * values(d)]
+    cached = values(2, *capi.KvCache(start + T, kh, d).keys.shape).to(torch.bfloat16)
+    results = []
+    for shift in (0, 1):
+        space = [torch.empty(d + 4, device="cuda") for _ in norms]
+        weights = [s[shift:shift + d].copy_(n) for s, n in zip(space, norms)]
+        cache = capi.KvCache(start + T, kh, d)
+        cache.keys.copy_(cached[0])
+        cache.values.copy_(cached[1])
+        out = capi.gqa_prefill(p, qg, k, v, *weights, cache, start_position=start)
+        torch.cuda.synchronize()
+        results.append((cache.keys, cache.values, out))
+    for rows, heads in zip(*results):
+        assert torch.equal(rows, heads)
