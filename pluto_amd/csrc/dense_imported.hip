@@ -848,7 +848,7 @@ struct TileManyArgs {
   uint16_t* out[kManyMax];
   int rows[kManyMax];
   int first_block[kManyMax + 1];
-  int matrices = 0;
+  int matrices = 0, tile_rows = 16;
   const void* tokens = nullptr;         // bf16 [count, cols]; FP8: one pass in operand order
   const float* token_scales = nullptr;  // FP8 only: [count, cols / 128]
   int cols = 0, count = 0;              // count <= 32
@@ -858,11 +858,10 @@ struct TileManyArgs {
 struct TilePlace {
   int which, row;
 };
-template <int ROWS>
 __device__ inline TilePlace tile_place(const TileManyArgs& m, int tile) {
   int which = 0;
   while (which + 1 < m.matrices && tile >= m.first_block[which + 1]) ++which;
-  return {which, (tile - m.first_block[which]) * ROWS};
+  return {which, (tile - m.first_block[which]) * m.tile_rows};
 }
 
 // The partial tiles of the waves (`elements` of 64 lanes each) added in wave order; element
@@ -911,9 +910,9 @@ imported_tile_bf16_kernel(TileManyArgs m, int passes) {
   };
   // rows past the end read zeros
   auto rows_of = [&](int tile) {
-    const TilePlace place = tile_place<16>(m, tile);
+    const TilePlace place = tile_place(m, tile);
     const size_t first = static_cast<size_t>(place.row) * m.cols * 2;
-    const int rows = min(16, m.rows[place.which] - place.row);
+    const int rows = min(m.tile_rows, m.rows[place.which] - place.row);
     return __builtin_amdgcn_make_buffer_rsrc(
         const_cast<unsigned char*>(static_cast<const unsigned char*>(m.weights[place.which]) + first), 0,
         rows * m.cols * 2, 0x00020000);
@@ -945,7 +944,7 @@ imported_tile_bf16_kernel(TileManyArgs m, int passes) {
   __builtin_amdgcn_sched_barrier(0);
   int buffer = 0;
   for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, buffer ^= 1) {
-    const TilePlace place = tile_place<16>(m, tile);
+    const TilePlace place = tile_place(m, tile);
     const int rows = m.rows[place.which];
     floatx4 total[TOKEN_PARTS];
 #pragma unroll
@@ -974,7 +973,7 @@ imported_tile_bf16_kernel(TileManyArgs m, int passes) {
     // element e is row 4 q + e % 4, token 16 (e / 4) + n
     add_waves(partial[buffer], own, wave, lane, [&](int e, float sum) {
       const int row = place.row + 4 * q + e % 4, token = 16 * (e / 4) + n;
-      if (row < rows && token < m.count)
+      if (row < min(rows, place.row + m.tile_rows) && token < m.count)
         m.out[place.which][static_cast<size_t>(token) * rows + row] = float_to_bf16_bits(sum);
     });
   }
@@ -1013,9 +1012,9 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
             uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, lane_at + 16 * t * m.cols, at + 64 * half, 0));
   };
   auto rows_of = [&](int tile) {
-    const TilePlace place = tile_place<16 * PARTS>(m, tile);
+    const TilePlace place = tile_place(m, tile);
     const size_t first = static_cast<size_t>(place.row) * m.cols;
-    const int rows = min(16 * PARTS, m.rows[place.which] - place.row);
+    const int rows = min(m.tile_rows, m.rows[place.which] - place.row);
     return __builtin_amdgcn_make_buffer_rsrc(
         const_cast<unsigned char*>(static_cast<const unsigned char*>(m.weights[place.which]) + first), 0,
         rows * m.cols, 0x00020000);
@@ -1043,9 +1042,12 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
   __builtin_amdgcn_sched_barrier(0);
   int buffer = 0;
   for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, buffer ^= 1) {
-    const TilePlace place = tile_place<16 * PARTS>(m, tile);
+    const TilePlace place = tile_place(m, tile);
     const int rows = m.rows[place.which];
     const float* block_scale = m.weight_scales[place.which] + static_cast<size_t>(place.row / kGroup) * groups;
+    // a tile of other than 16 rows may reach into the next 128, which have scales of their own
+    const int own_rows = kGroup - place.row % kGroup;
+    const bool crosses = PARTS > 1 && own_rows < min(m.tile_rows, rows - place.row);
     floatx4 total[PARTS][TOKEN_PARTS];
 #pragma unroll
     for (int i = 0; i < PARTS; ++i)
@@ -1061,6 +1063,8 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
         // a block past the end contributes nothing (its scale is read in range)
         const int g = block_of(pass, b);
         const float weight_scale = g < groups ? block_scale[min(g, groups - 1)] : 0.0f;
+        const float next_scale =
+            PARTS > 1 && g < groups ? block_scale[min(g, groups - 1) + (crosses ? groups : 0)] : 0.0f;
         floatx4 acc[PARTS][TOKEN_PARTS];
 #pragma unroll
         for (int i = 0; i < PARTS; ++i)
@@ -1095,7 +1099,16 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
 #pragma unroll
         for (int i = 0; i < PARTS; ++i)
 #pragma unroll
-          for (int j = 0; j < TOKEN_PARTS; ++j) total[i][j] += acc[i][j] * (weight_scale * group_scale[b][j]);
+          for (int j = 0; j < TOKEN_PARTS; ++j) {
+            if (PARTS == 1 || !crosses) {
+              total[i][j] += acc[i][j] * (weight_scale * group_scale[b][j]);
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                total[i][j][e] +=
+                    acc[i][j][e] * ((16 * i + 4 * q + e < own_rows ? weight_scale : next_scale) * group_scale[b][j]);
+            }
+          }
       }
     }
     constexpr int kElements = 4 * TOKEN_PARTS * PARTS;
@@ -1106,21 +1119,36 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
     add_waves(partial[buffer], own, wave, lane, [&](int e, float sum) {
       const int row = place.row + 16 * (e / (4 * TOKEN_PARTS)) + 4 * q + e % 4;
       const int token = 16 * (e / 4 % TOKEN_PARTS) + n;
-      if (row < rows && token < m.count)
+      if (row < min(rows, place.row + m.tile_rows) && token < m.count)
         m.out[place.which][static_cast<size_t>(token) * rows + row] = float_to_bf16_bits(sum);
     });
   }
 }
 
-// Where every compute unit walks over several tiles they have 16 rows (shorter ends: 516 x
-// 32 rows of 5120 columns 27.4 us in tiles of 32 rows, 24.7 in tiles of 16).  Fewer have
-// 32, for the tokens, as many bytes as a tile's weights, are loaded for one tile only
-// (160 x 32 rows of 6144 columns: 14.3 us, 15.5 in tiles of 16).
-int fp8_tile_rows(int matrices, const int* rows) {
+// The rows of a tile: at most 16 PARTS, and as few as leave the longest list of a workgroup as
+// long as with that many, so that all lists have about as many bytes: 5120 -> 16480 is 1030 tiles
+// of 16 rows, five for six workgroups and four for the others, or 1269 of 13.  bf16, 14 tokens:
+// 5120 -> 16480 36.8 -> 32.2 us, 6144 -> 5120 (320 tiles, 512 so) 22.8 -> 17.7; 30 tokens 77.4 ->
+// 72.1, 37.2 -> 32.8.  FP8 6144 -> 5120 (160 tiles of 32 rows, 256 of 20), 11 tokens 11.9 -> 10.6
+// us, 32 13.6 -> 12.5.  FP8 tiles of 16 rows are bound by their conversions as much as by their
+// bytes (5120 -> 16480 in tiles of 13, 11 tokens 21.1 -> 20.7, 32 23.4 -> 24.4): they stay whole.
+long long tiles_of(int matrices, const int* rows, int tile_rows) {
   long long tiles = 0;
-  for (int i = 0; i < matrices; ++i) tiles += (rows[i] + 31) / 32;
-  return tiles >= 256 ? 16 : 32;
+  for (int i = 0; i < matrices; ++i) tiles += (rows[i] + tile_rows - 1) / tile_rows;
+  return tiles;
 }
+int balanced_rows(int matrices, const int* rows, int most) {
+  const long long turns = (tiles_of(matrices, rows, most) + 255) / 256;
+  int tile_rows = most;
+  while (tile_rows > 1 && tiles_of(matrices, rows, tile_rows - 1) <= 256 * turns) --tile_rows;
+  return tile_rows;
+}
+
+// Where every compute unit walks over several tiles they have up to 16 rows (shorter ends: 516 x
+// 32 rows of 5120 columns 27.4 us in tiles of 32 rows, 24.7 in tiles of 16).  Fewer have
+// up to 32, for the tokens, as many bytes as a tile's weights, are loaded for one tile only
+// (160 x 32 rows of 6144 columns: 14.3 us, 15.5 in tiles of 16).
+int fp8_parts(int matrices, const int* rows) { return tiles_of(matrices, rows, 32) >= 256 ? 1 : 2; }
 
 template <int PARTS, int TOKEN_PARTS>
 void launch_fp8_tiles(hipStream_t s, const TileManyArgs& t) {
@@ -1369,8 +1397,9 @@ int launch_dense_imported_forward(hipStream_t s, int storage, int matrices,
     return launch_status();
   }
   TileManyArgs t;
-  const int tile_rows = fp8 ? fp8_tile_rows(matrices, output_dims) : 16;
-  fill(t, t.weight_scales, tile_rows);
+  const int parts = fp8 ? fp8_parts(matrices, output_dims) : 1;
+  t.tile_rows = fp8 && parts == 1 ? 16 : balanced_rows(matrices, output_dims, 16 * parts);
+  fill(t, t.weight_scales, t.tile_rows);
   const unsigned char* token_bytes = static_cast<const unsigned char*>(input);
   if (fp8) {
     unsigned char* codes = static_cast<unsigned char*>(workspace);
@@ -1386,7 +1415,7 @@ int launch_dense_imported_forward(hipStream_t s, int storage, int matrices,
     t.tokens = token_bytes + static_cast<size_t>(done) * input_dim * (fp8 ? 1 : 2);
     if (!fp8)
       t.count <= 16 ? launch_bf16_tiles<1>(s, t) : launch_bf16_tiles<2>(s, t);
-    else if (tile_rows == 16)
+    else if (parts == 1)
       t.count <= 16 ? launch_fp8_tiles<1, 1>(s, t) : launch_fp8_tiles<1, 2>(s, t);
     else
       t.count <= 16 ? launch_fp8_tiles<2, 1>(s, t) : launch_fp8_tiles<2, 2>(s, t);

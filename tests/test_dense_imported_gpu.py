@@ -176,7 +176,9 @@ def test_matrix_core_batch_matches_the_oracle(capi, oracle):
 
 @pytest.mark.parametrize("cols,rows,tokens", [(128, 8200, 9), (5120, 8210, 32), (6144, 8192, 17), (7168, 8200, 32),
                                               (4096, 100, 16), (6144, 33, 32), (9216, 130, 31), (5120, 130, 16),
-                                              (4608, 65, 32), (6144, 200, 9)])
+                                              (4608, 65, 32), (6144, 200, 9),
+                                              # tiles of 17, 20 and 31 rows, across the scales' 128
+                                              (256, 4200, 9), (256, 5120, 32), (384, 7900, 17)])
 def test_fp8_tiles_match_float64_products(capi, cols, rows, tokens):
     """More than eight tokens of FP8 matrices: workgroups that walk over tiles of 16 rows
     (8192 rows and more) or of 32, with one pass over the columns or several, partial
@@ -341,7 +343,7 @@ def test_a_non_finite_token_gives_nan_and_touches_no_other(capi, oracle, tokens,
 
 @pytest.mark.parametrize("storage", ["bf16", "fp8"])
 @pytest.mark.parametrize("cols,heights", [(128, [1]), (256, [3, 4]), (384, [130]), (1152, [5, 1, 2050]),
-                                          (5120, [129, 7]), (8448, [6]), (9216, [9, 64]), (9344, [5])])
+                                          (5120, [129, 7]), (256, [3000, 2500]), (8448, [6]), (9216, [9, 64]), (9344, [5])])
 def test_few_and_many_tokens_of_whole_blocks(capi, storage, cols, heights):
     """The matrix-core kernels for one, several and more than eight tokens at the edges
     of their panels (and one width past them): row quadruples that end early, more than
