@@ -76,6 +76,39 @@ struct TileAccess {
   }
 };
 
+// A wave's own rows of a tensor as operands, sixteen bytes of one row a lane, cost the compute
+// unit's address path 64 cycles a load instruction: 7 of the 8.9 us before a query-owned
+// gradient workgroup's first tile at T = 1024.  Brought to LDS as tiles of 32 rows, 1 KiB a
+// request, they cost a quarter.  Rows beyond the sequence repeat the last one.
+__device__ inline void request_own_tile(const uint16_t* tensor, long long row_stride, int length, int row0,
+                                        unsigned char* tile, int wave, int lane) {
+  const int32x4 rsrc = make_rsrc(tensor, tile_bytes<D>(0, length, row_stride));
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int position = (wave * kLoads + i) * 64 + lane, row = position / KCH, slot = position % KCH;
+    const uint32_t at = static_cast<uint32_t>(min(row0 + row, length - 1) * row_stride * 2) + (slot ^ tile_swizzle(row)) * 16;
+    lds_fill<16>(rsrc, tile + (wave * kLoads + i) * 1024, at);
+  }
+}
+// The other way round: sixteen-byte pieces of 32 rows, a row a lane, through `area`, which no
+// other wave touches, to whole rows of CHUNKS pieces.  piece(c) is the lane's piece c of its
+// row n (c's parity is the lane's half); use(round, row, c, piece) has pieces of neighbouring
+// lanes next to each other.
+template <int CHUNKS, typename Piece, typename Use>
+__device__ inline void by_rows(unsigned char* area, int lane, Piece&& piece, Use&& use) {
+  const int h = lane / 32, n = lane % 32;
+  float4* pieces = reinterpret_cast<float4*>(area);
+#pragma unroll
+  for (int c = 0; c < CHUNKS; c += 2) pieces[n * CHUNKS + ((c + h) ^ (n & 15))] = piece(c);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  constexpr int kRowsAtOnce = 64 / CHUNKS;
+#pragma unroll
+  for (int r = 0; r < 32; r += kRowsAtOnce) {
+    const int row = r + lane / CHUNKS, c = lane % CHUNKS;
+    use(r / kRowsAtOnce, row, c, pieces[row * CHUNKS + (c ^ (row & 15))]);
+  }
+}
+
 // Nothing moves across.  Operands are requested two or three steps ahead of their use
 // and what a step requests stands between its matrix instructions: one wave a SIMD
 // issues in order, so whatever stands before them in a burst runs beside none.  (Left to
@@ -187,7 +220,17 @@ split_forward_kernel(SplitArgs a) {
   QueryFill fill(a, lds, wave, head, at);
   fill.request_all(0);
   bf16x8 qf[KS];
-  load_row_operand(a.q + query_load * q_row + head * D, h, qf);
+  {
+    // the queries in the stage that is filled second
+    unsigned char* own = lds + kQueryStageBytes;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+      request_own_tile(a.q + head * D, q_row, T, w.first_query + 32 * (half - w.half), own + half * kTileBytes, wave, lane);
+    stage_ready();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = at.row(own + w.half * kTileBytes, ks);
+    lds_barrier();
+  }
   floatx16 o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) o[db] = zero16();
@@ -305,21 +348,21 @@ split_forward_kernel(SplitArgs a) {
     hand_over<0>(lds, w.half, lane, o);
   wave_stats[w.half][w.parity][0][lane] = running_max;
   wave_stats[w.half][w.parity][1][lane] = running_sum;
-  const long long unit = 1LL * query_load * a.heads + head;
+  // 128 channels a wave leave as whole rows: lane l of round r has four channels of row 2 r +
+  // l / 32
   auto finish = [&](auto first) {
     constexpr int FIRST = decltype(first)::value;
-    const long long at_channel = 32 * FIRST + 4 * h;
+    auto place = [&](int row) {  // of a query's channels among all
+      return (1LL * min(w.first_query + row, T - 1) * a.heads + head) * D + 32 * FIRST + 4 * (lane % 32);
+    };
+    auto gate_place = [&](int row) { return 2 * place(row) + D - 32 * FIRST - 4 * (lane % 32); };
     // the gates travel while the waves meet
-    [[maybe_unused]] uint2 gates[kHalfBlocks][4];
-    [[maybe_unused]] const uint16_t* gate = a.qg + (2 * unit + 1) * D + at_channel;
+    [[maybe_unused]] uint2 gates[16];
     if constexpr (OUTPUT == Gated::kWide) {
 #pragma unroll
-      for (int i = 0; i < kHalfBlocks; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) gates[i][j] = *reinterpret_cast<const uint2*>(gate + 32 * i + 8 * j);
+      for (int r = 0; r < 16; ++r) gates[r] = *reinterpret_cast<const uint2*>(a.qg + gate_place(2 * r + h));
     }
     lds_barrier();
-    if (query >= T) return;
     // a wave without tiles has weight 2^(kMasked - maximum) = 0
     const float other_max = wave_stats[w.half][1 - w.parity][0][lane];
     const float maximum = fmaxf(running_max, other_max);
@@ -328,44 +371,47 @@ split_forward_kernel(SplitArgs a) {
     const float own_sum = running_sum * own, other_sum = wave_stats[w.half][1 - w.parity][1][lane] * other;
     const float sum = own_sum + other_sum;
     const float inverse = 1.0f / (sum > 0.0f ? sum : 1.0f);
-    float* out = a.core + unit * D + at_channel;
-#pragma unroll
-    for (int i = 0; i < kHalfBlocks; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float4 u = handed_over<FIRST>(lds, w.half, lane, i, j);
-        const floatx16& from = o[FIRST + i];
-        const float c[4] = {(from[4 * j] * own + u.x * other) * inverse, (from[4 * j + 1] * own + u.y * other) * inverse,
-                            (from[4 * j + 2] * own + u.z * other) * inverse,
-                            (from[4 * j + 3] * own + u.w * other) * inverse};
-        *reinterpret_cast<float4*>(out + 32 * i + 8 * j) = make_float4(c[0], c[1], c[2], c[3]);
-        if constexpr (OUTPUT != Gated::kNone) {
-          // qwen_attention.cc:103-108
-          uint16_t* gated = a.out + unit * D + at_channel + 32 * i + 8 * j;
-          float logits[4], g[4];
-          if constexpr (OUTPUT == Gated::kWide) {
-            const uint2 bits = gates[i][j];
-            logits[0] = __uint_as_float(bits.x << 16), logits[1] = __uint_as_float(bits.x & 0xffff0000u);
-            logits[2] = __uint_as_float(bits.y << 16), logits[3] = __uint_as_float(bits.y & 0xffff0000u);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) logits[e] = bf16_bits_to_float(gate[32 * i + 8 * j + e]);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) g[e] = round_to_bf16(c[e]) * round_to_bf16(gate_sigmoid(logits[e]));
-          if constexpr (OUTPUT == Gated::kWide) {
-            *reinterpret_cast<uint2*>(gated) = make_uint2(pack_bf16(g[0], g[1]), pack_bf16(g[2], g[3]));
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gated[e] = float_to_bf16_bits(g[e]);
-          }
-        }
-      }
-    if (FIRST == 0 && h == 0) {
+    if (FIRST == 0 && h == 0 && query < T) {
       a.maxima[1LL * head * T + query] = maximum;
       a.inverses[1LL * head * T + query] = inverse;
-      if (OUTPUT != Gated::kNone && a.lse) a.lse[unit] = maximum + logf(sum > 0.0f ? sum : 1.0f);
+      if (OUTPUT != Gated::kNone && a.lse) a.lse[1LL * query * a.heads + head] = maximum + logf(sum > 0.0f ? sum : 1.0f);
     }
+    by_rows<32>(lds + (4 + wave) * kTileBytes, lane,
+                [&](int c) {
+                  const int i = c / 8, j = c % 8 / 2;
+                  const float4 u = handed_over<FIRST>(lds, w.half, lane, i, j);
+                  const floatx16& from = o[FIRST + i];
+                  return make_float4((from[4 * j] * own + u.x * other) * inverse,
+                                     (from[4 * j + 1] * own + u.y * other) * inverse,
+                                     (from[4 * j + 2] * own + u.z * other) * inverse,
+                                     (from[4 * j + 3] * own + u.w * other) * inverse);
+                },
+                [&](int round, int row, int, float4 core) {
+                  if (w.first_query + row >= T) return;
+                  *reinterpret_cast<float4*>(a.core + place(row)) = core;
+                  if constexpr (OUTPUT != Gated::kNone) {
+                    // qwen_attention.cc:103-108
+                    const float c[4] = {core.x, core.y, core.z, core.w};
+                    uint16_t* gated = a.out + place(row);
+                    float logits[4], g[4];
+                    if constexpr (OUTPUT == Gated::kWide) {
+                      const uint2 bits = gates[round];
+                      logits[0] = __uint_as_float(bits.x << 16), logits[1] = __uint_as_float(bits.x & 0xffff0000u);
+                      logits[2] = __uint_as_float(bits.y << 16), logits[3] = __uint_as_float(bits.y & 0xffff0000u);
+                    } else {
+#pragma unroll
+                      for (int e = 0; e < 4; ++e) logits[e] = bf16_bits_to_float(a.qg[gate_place(row) + e]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) g[e] = round_to_bf16(c[e]) * round_to_bf16(gate_sigmoid(logits[e]));
+                    if constexpr (OUTPUT == Gated::kWide) {
+                      *reinterpret_cast<uint2*>(gated) = make_uint2(pack_bf16(g[0], g[1]), pack_bf16(g[2], g[3]));
+                    } else {
+#pragma unroll
+                      for (int e = 0; e < 4; ++e) gated[e] = float_to_bf16_bits(g[e]);
+                    }
+                  }
+                });
   };
   if (w.parity == 0)
     finish(std::integral_constant<int, 0>());
@@ -423,14 +469,25 @@ __device__ __forceinline__ void split_query_owned(const SplitArgs& a, unsigned c
   const long long q_row = 1LL * a.heads * D;
   const TileAccess at(wave, lane, 1LL * (a.heads / a.group) * D);
   QueryFill fill(a, lds, wave, head, at);
-  fill.request_all(0);
-  bf16x8 qf[KS], gf[3][KS];
-  load_row_operand(a.q + query_load * q_row + head * D, h, qf);
-#pragma unroll
-  for (int part = 0; part < 3; ++part)
-    load_row_operand(a.d_core + part * a.piece + query_load * q_row + head * D, h, gf[part]);
   const long long stat = 1LL * head * T + query_load;
   const float maximum = a.maxima[stat], inverse = a.inverses[stat], delta = a.deltas[stat];
+  bf16x8 qf[KS], gf[3][KS];
+  // Q and the three pieces of dC of both halves take both stages
+#pragma unroll
+  for (int tensor = 0; tensor < 4; ++tensor)
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+      request_own_tile((tensor == 0 ? a.q : a.d_core + (tensor - 1) * a.piece) + head * D, q_row, T, q0 + 32 * half,
+                       lds + (2 * tensor + half) * kTileBytes, wave, lane);
+  stage_ready();
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    qf[ks] = at.row(lds + w.half * kTileBytes, ks);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) gf[part][ks] = at.row(lds + (2 + 2 * part + w.half) * kTileBytes, ks);
+  }
+  lds_barrier();
+  fill.request_all(0);
   floatx16 dq[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) dq[db] = zero16();
@@ -502,20 +559,21 @@ __device__ __forceinline__ void split_query_owned(const SplitArgs& a, unsigned c
   else
     hand_over<0>(lds, w.half, lane, dq);
   __syncthreads();
-  if (query >= T) return;
+  // the sums of 128 channels a wave leave as whole rows
   auto finish = [&](auto first) {
     constexpr int FIRST = decltype(first)::value;
-    float* out = a.dq + query * q_row + head * D + 32 * FIRST + 4 * h;
-#pragma unroll
-    for (int i = 0; i < kHalfBlocks; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float4 u = handed_over<FIRST>(lds, w.half, lane, i, j);
-        const floatx16& from = dq[FIRST + i];
-        *reinterpret_cast<float4*>(out + 32 * i + 8 * j) =
-            make_float4((from[4 * j] + u.x) * a.scale, (from[4 * j + 1] + u.y) * a.scale,
-                        (from[4 * j + 2] + u.z) * a.scale, (from[4 * j + 3] + u.w) * a.scale);
-      }
+    float* out = a.dq + head * D + 32 * FIRST;
+    by_rows<32>(lds + (4 + wave) * kTileBytes, lane,
+                [&](int c) {
+                  const int i = c / 8, j = c % 8 / 2;
+                  const float4 u = handed_over<FIRST>(lds, w.half, lane, i, j);
+                  const floatx16& from = dq[FIRST + i];
+                  return make_float4((from[4 * j] + u.x) * a.scale, (from[4 * j + 1] + u.y) * a.scale,
+                                     (from[4 * j + 2] + u.z) * a.scale, (from[4 * j + 3] + u.w) * a.scale);
+                },
+                [&](int, int row, int c, float4 v) {
+                  if (w.first_query + row < T) *reinterpret_cast<float4*>(out + (w.first_query + row) * q_row + 4 * c) = v;
+                });
   };
   if (w.parity == 0)
     finish(std::integral_constant<int, 0>());
@@ -567,8 +625,18 @@ __device__ __forceinline__ void split_key_owned(const SplitArgs& a, unsigned cha
   };
   request_all(first_tile);
   bf16x8 kf[KS], vf[VALUES ? 1 : KS];
-  load_row_operand(a.k + key_load * kv_row + head / a.group * D, h, kf);
-  if constexpr (!VALUES) load_row_operand(a.v + key_load * kv_row + head / a.group * D, h, vf);
+  {
+    // the keys in the stage that is filled second (what V would save there it would wait)
+    unsigned char* own = lds + ((first_tile + 1) & 1) * kDkvStageBytes;
+#pragma unroll
+    for (int tile = 0; tile < 4; ++tile)
+      request_own_tile(a.k + head / a.group * D, kv_row, T, k0 + 32 * tile, own + tile * kTileBytes, wave, lane);
+    if constexpr (!VALUES) load_row_operand(a.v + key_load * kv_row + head / a.group * D, h, vf);
+    stage_ready();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kf[ks] = at.row(own + wave * kTileBytes, ks);
+    lds_barrier();
+  }
   floatx16 acc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) acc[db] = zero16();
@@ -672,17 +740,18 @@ __device__ __forceinline__ void split_key_owned(const SplitArgs& a, unsigned cha
       }
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the requests beyond the last tile
-  if (key >= T) return;
+  stage_ready();  // the requests beyond the last tile; nobody reads the stages any more
   const float factor = VALUES ? 1.0f : a.scale;
-  float* out = (VALUES ? a.dv : a.dk) + key * q_row + head * D + 4 * h;
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<float4*>(out + 32 * db + 8 * j) =
-          make_float4(acc[db][4 * j] * factor, acc[db][4 * j + 1] * factor,
-                      acc[db][4 * j + 2] * factor, acc[db][4 * j + 3] * factor);
+  float* out = (VALUES ? a.dv : a.dk) + head * D;
+  by_rows<64>(lds + wave * 2 * kTileBytes, lane,
+              [&](int c) {
+                const int db = c / 8, j = c % 8 / 2;
+                return make_float4(acc[db][4 * j] * factor, acc[db][4 * j + 1] * factor, acc[db][4 * j + 2] * factor,
+                                   acc[db][4 * j + 3] * factor);
+              },
+              [&](int, int row, int c, float4 v) {
+                if (first_key + row < T) *reinterpret_cast<float4*>(out + (first_key + row) * q_row + 4 * c) = v;
+              });
 }
 
 // All gradients in one launch, longest workgroups first: a compute unit holds one, and those
