@@ -26,6 +26,8 @@
 
 #include "mfma_tile.h"
 
+#include <type_traits>
+
 namespace pluto_hip {
 namespace {
 
@@ -137,43 +139,79 @@ flash_dq_kernel(FlashBackwardArgs a) {
       row_delta = -a.deltas[stats_base + q_load];
       row_lse2 = -a.lse2[stats_base + q_load] * scale2;
     } else {
-      const uint16_t* o_base = a.out + seq_row0 * E + head * D;
-      const float* g_base = a.d_out + seq_row0 * E + head * D;
-      float partial = 0.0f;
+      // Rows travel whole and become operands through the wave's own area: sixteen bytes of
+      // a row of its own a lane, which is what an operand is, cost the compute unit's address
+      // path 64 cycles a load, four times as much as whole rows, and the workgroups of a
+      // one-round grid all load at once.  The bf16 copy of dO leaves from the rows.
+      // 16 sequences of 1024, 12 heads: 68.8 -> 65.8 us; 4 of 256: 15.4 -> 14.2.
+      // Rows beyond the sequence read as zero and are not stored.
+      int own = lane;
+      asm volatile("" : "+v"(own));  // addresses of this part only: none is kept over the loop
+      const int quad = own % 16, chunk = own % 8, own_n = own % 32, own_h = own / 32;
+      const int own_row = __builtin_amdgcn_readfirstlane(wave_first_row);
+      const int first = min(own_row, T - 1), left = min(T - own_row, 32);
+      auto rows_of = [&](const void* base, long long stride, int row_bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<void*>(base), 0, left <= 0 ? 0 : static_cast<int>((left - 1) * stride + row_bytes), 0x00020000);
+      };
+      const auto g_rows = rows_of(a.d_out + (seq_row0 + first) * E + head * D, 4LL * E, 4 * D);
+      const auto o_rows = rows_of(a.out + (seq_row0 + first) * E + head * D, 2LL * E, 2 * D);
+      const auto q_rows = rows_of(q_base + first * q_stride, 2 * q_stride, 2 * D);
+      const auto gb_rows = rows_of(gb_base + static_cast<long long>(first) * E, 2LL * E, 2 * D);
+      const uint32_t at = own / 16 * (4u * E) + 16 * quad;
+      const uint32_t q_at = own / 8 * (2u * static_cast<uint32_t>(q_stride)) + 16 * chunk;
+      uint32x4 g[8], q[4];
+      uint32x2 o[8];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int c = 16 * ks + 8 * h;
-        qf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-            q_base + q_load * q_stride + c));
-        const float4 g0 = *reinterpret_cast<const float4*>(g_base + static_cast<long long>(q_load) * E + c);
-        const float4 g1 = *reinterpret_cast<const float4*>(g_base + static_cast<long long>(q_load) * E + c + 4);
-        const uint4 o = *reinterpret_cast<const uint4*>(o_base + static_cast<long long>(q_load) * E + c);
-        const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-        const uint32_t ow[4] = {o.x, o.y, o.z, o.w};
-        uint32_t packed[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          partial += g[2 * i] * __uint_as_float(ow[i] << 16);
-          partial += g[2 * i + 1] * __uint_as_float(ow[i] & 0xffff0000u);
-          packed[i] = pack_bf16(g[2 * i], g[2 * i + 1]);
-        }
-        const uint4 bits = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        gf[ks] = as_bf16x8(bits);
-        copy_area[n * KCH + ((2 * ks + h) ^ (n & 7))] = bits;
+      for (int i = 0; i < 8; ++i) {
+        g[i] = __builtin_amdgcn_raw_buffer_load_b128(g_rows, at, i * (16 * E), 0);
+        o[i] = __builtin_amdgcn_raw_buffer_load_b64(o_rows, at / 2, i * (8 * E), 0);
       }
-      // The bf16 copy of dO leaves through the wave's own area: a lane holds 16-byte pieces of its
-      // own row, and stored from there a store instruction touches 32 lines;
-      // from LDS it writes whole rows (25 MB in 17 us against 5 us).
 #pragma unroll
-      for (int i = 0; i < 32 * KCH / 64; ++i) {
-        const int at = i * 64 + lane, row = at / KCH, chunk = at % KCH;
-        const uint4 bits = copy_area[row * KCH + (chunk ^ (row & 7))];
-        if (wave_first_row + row < T)
-          *reinterpret_cast<uint4*>(gb_base + static_cast<long long>(wave_first_row + row) * E +
-                                    8 * chunk) = bits;
-      }
+      for (int i = 0; i < 4; ++i)
+        q[i] = __builtin_amdgcn_raw_buffer_load_b128(q_rows, q_at, i * (16 * static_cast<int>(q_stride)), 0);
       // delta of attention.cc:283-291 (uses the stored, rounded output)
-      row_delta = half_swap_sum(partial);
+      float delta[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int local = 4 * i + own / 16;
+        const float x = __uint_as_float(g[i][0]), y = __uint_as_float(g[i][1]);
+        const float z = __uint_as_float(g[i][2]), w = __uint_as_float(g[i][3]);
+        delta[i] = x * __uint_as_float(o[i][0] << 16) + y * __uint_as_float(o[i][0] & 0xffff0000u) +
+                   (z * __uint_as_float(o[i][1] << 16) + w * __uint_as_float(o[i][1] & 0xffff0000u));
+        const uint32x2 bits = {pack_bf16(x, y), pack_bf16(z, w)};
+        reinterpret_cast<uint32x2*>(copy_area)[(local * KCH + ((quad / 2) ^ (local & 7))) * 2 + quad % 2] = bits;
+        __builtin_amdgcn_raw_buffer_store_b64(bits, gb_rows, at / 2, i * (8 * E), 0);
+      }
+      // a wave's accesses to LDS are carried out in order: the compiler only has to keep it
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) gf[ks] = as_bf16x8(copy_area[own_n * KCH + ((2 * ks + own_h) ^ (own_n & 7))]);
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int local = 8 * i + own / 8;
+        reinterpret_cast<uint32x4*>(copy_area)[local * KCH + (chunk ^ (local & 7))] = q[i];
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) qf[ks] = as_bf16x8(copy_area[own_n * KCH + ((2 * ks + own_h) ^ (own_n & 7))]);
+      asm volatile("" ::: "memory");
+      // over a row's sixteen lanes, then from the row's to the query's
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        auto add = [&](auto control) {
+          delta[i] += __int_as_float(
+              __builtin_amdgcn_mov_dpp(__float_as_int(delta[i]), decltype(control)::value, 0xf, 0xf, true));
+        };
+        add(std::integral_constant<int, 0xB1>());   // quad_perm 1, 0, 3, 2
+        add(std::integral_constant<int, 0x4E>());   // quad_perm 2, 3, 0, 1
+        add(std::integral_constant<int, 0x141>());  // row_half_mirror
+        add(std::integral_constant<int, 0x140>());  // row_mirror
+        if (quad == 0) reinterpret_cast<float*>(copy_area)[4 * i + own / 16] = delta[i];
+      }
+      asm volatile("" ::: "memory");
+      row_delta = reinterpret_cast<const float*>(copy_area)[n];
       const float normalizer = a.normalizers[stats_base + q_load];
       row_lse2 = a.maxima[stats_base + q_load] * kLog2e +
                              __log2f(normalizer > 0.0f ? normalizer : 1.0f);
@@ -311,7 +349,9 @@ flash_dkv_kernel(FlashBackwardArgs a) {
   constexpr int kStatBytes = 256;  // 64 floats
   constexpr int kStageBytes = 2 * kTileBytes + 2 * kStatBytes;
   constexpr int kBlockBytes = 32 * D * 2;
+  constexpr int kOwnBytes = 32 * D * 2;  // the wave's rows of one tensor
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char own_rows[4 * 2 * kOwnBytes];
 
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int h = lane / 32, n = lane % 32;
@@ -350,15 +390,20 @@ flash_dkv_kernel(FlashBackwardArgs a) {
     dkv_fill_stage<D, BQ, LOADS>(lds + ((first_tile) & 1) * kStageBytes, wave, lane, q_base, g_base,
                                  lse2_base, delta_base, q_stride, E, (first_tile) * BQ, T, q_fill, g_fill);
   const int key_row = k0 + 32 * wave + n;
-  const int key_load = min(key_row, T - 1);
-  bf16x8 kf[KS], vf[KS];
+  // The wave's own keys and values arrive as whole rows and become operands after the first
+  // wait: sixteen bytes of a row of its own a lane, which is what an operand is, cost the
+  // address path 64 cycles a load where a fill of contiguous rows costs 16 (16 sequences of
+  // 1024, 12 heads: 75.5 -> 72.5 us).
+  unsigned char* own = own_rows + wave * 2 * kOwnBytes;
+  {
+    uint32_t own_fill[4];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    kf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-        k_base + key_load * kv_stride + 16 * ks + 8 * h));
-    vf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-        v_base + key_load * kv_stride + 16 * ks + 8 * h));
+    for (int i = 0; i < 4; ++i) own_fill[i] = tile_fill_offset<D>(i * 64 + lane, kv_stride);
+    const long long at = (k0 + 32 * wave) * kv_stride;
+    tile_fill<D, 4>(own, 0, k_base + at, kv_stride, k0 + 32 * wave, T, own_fill);
+    tile_fill<D, 4>(own + kOwnBytes, 0, v_base + at, kv_stride, k0 + 32 * wave, T, own_fill);
   }
+  bf16x8 kf[KS], vf[KS];
   floatx16 dk_acc[DB], dv_acc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -372,6 +417,13 @@ flash_dkv_kernel(FlashBackwardArgs a) {
   for (int tile = first_tile; tile < tiles; ++tile) {
     const int q0 = tile * BQ;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (tile == first_tile) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        kf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(own + row_read[ks]));
+        vf[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(own + kOwnBytes + row_read[ks]));
+      }
+    }
     __syncthreads();
     if (tile + 1 < tiles)
       dkv_fill_stage<D, BQ, LOADS>(lds + ((tile + 1) & 1) * kStageBytes, wave, lane, q_base, g_base,
