@@ -73,6 +73,8 @@ struct Config {
   static constexpr int kTileBytes = BN * D * 2;    // one K or V tile
   static constexpr int kStageBytes = 2 * kTileBytes;
   static constexpr int kLoads = BN * KCH / kThreads;  // 16-byte loads per lane per tensor
+  static constexpr int kOwnBytes = 32 * G * D * 2;    // a wave's rows of Q
+  static_assert(WAVES * kOwnBytes <= kStageBytes, "one stage holds the workgroup's rows");
   // waves per SIMD the register budget is sized for
   static constexpr int kOccupancy = (D == 64 && G == 1) ? 3 : (D == 256 ? 1 : 2);
 };
@@ -187,19 +189,34 @@ flash_forward_kernel(FlashForwardArgs a_in, int unit_count) {
     const int q0 = q_tile * BM;
     const int wave_q0 = q0 + 32 * G * wave;
 
-    // Q fragments (B operand of S^T): row, channels 16ks + 8h .. +7.
+    // Q fragments (B operand of S^T): row, channels 16ks + 8h .. +7.  The wave's rows arrive
+    // whole in the stage that the second tile will take, swizzled like K, and are read after
+    // the first wait: sixteen bytes of a row of its own a lane, which is what a fragment is,
+    // cost the address path 64 cycles a load, and all workgroups begin at once (8 sequences of
+    // 500, 4 heads of 128: 18.1 -> 16.9 us; 16 of 1024, 12 heads of 64: 45.6 -> 44.7).  The
+    // output stays as it is: through LDS it cost short sequences 0.4 us at heads of 64.
     bf16x8 qf[G][KS];
     int q_row[G], row_limit[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       q_row[g] = wave_q0 + 32 * g + n;
-      const int row = min(q_row[g], a.q_rows - 1);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        qf[g][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
-            q_base + static_cast<long long>(row) * a.q_row_stride + 16 * ks + 8 * h));
       // keys up to row_limit are visible to this lane's query
       row_limit[g] = min(a.start_position + q_row[g], a.kv_rows - 1);
+    }
+    unsigned char* own = lds + C::kStageBytes + wave * C::kOwnBytes;
+    {
+      const int own_row = __builtin_amdgcn_readfirstlane(min(wave_q0, a.q_rows - 1));
+      const int rows = min(a.q_rows - own_row, 32 * G);
+      const int32x4 rsrc = make_rsrc(q_base + own_row * a.q_row_stride,
+                                     static_cast<uint32_t>(((rows - 1) * a.q_row_stride + D) * 2));
+      int own_lane = lane;
+      asm volatile("" : "+v"(own_lane));  // offsets of this part only: none is kept over the loop
+#pragma unroll
+      for (int i = 0; i < C::kOwnBytes / 1024; ++i) {
+        const int p = i * 64 + own_lane, row = p / KCH;
+        lds_fill<16>(rsrc, own + i * 1024,
+                     static_cast<uint32_t>(row * a.q_row_stride * 2 + ((p % KCH) ^ (row & 7)) * 16));
+      }
     }
     floatx16 o_acc[G][DB];
     // Row sums come out of the matrix cores: an all-ones A operand makes every
@@ -236,6 +253,13 @@ flash_forward_kernel(FlashForwardArgs a_in, int unit_count) {
       const int k0 = tile * BN;
       // The tile's loads have landed; every wave is done with the other stage.
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (tile == 0) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks)
+            qf[g][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(own + g * 32 * KCH * 16 + k_read[ks]));
+      }
       __syncthreads();
       if (tile + 1 < tiles)
         fill_stage<D, C::kLoads>(lds + ((tile + 1) & 1) * C::kStageBytes, wave, k_base, v_base,
