@@ -44,7 +44,8 @@
 //
 // Matrix products of the parallel kernels run on v_mfma_f32_32x32x2_f32 and
 // v_mfma_f32_16x16x4_f32; the triangular factors are multiplied by halves.  Those of the
-// sequential kernels take three bf16 pieces of every factor (bf16_pieces.h).
+// sequential kernels take three bf16 pieces of a factor (bf16_pieces.h), of bf16 activations'
+// keys and queries one.
 #include "gdn.h"
 
 #include "bf16_pieces.h"
@@ -67,20 +68,22 @@ constexpr int kSquarePad = kC + 4;
 struct Records {
   // of a key head                                                        [64][128]
   float *q_rows, *q_columns, *k_rows, *k_columns;
+  uint16_t* keys;             // the four as bf16 operands, see KeyOperand
   float *w_rows, *w_columns;                          // W              [64][128]
   float *u_columns, *dl_rows, *ddl_rows;              // U, Dl, dDl     [64][128]
   float *p_rows, *p_columns;                          // P               [64][64]
   float *t_columns;                                   // T               [64][64]
   float *kkd;                 // columns(strict_lower((k^_i . k^_j) D_ij)) [64][64]
-  float *gates;               // [6][64], see Gate
+  float *gates;               // [8][64], see Gate
   float *s0, *ds1;            // rows(state entering the chunk), rows(gradient of the one leaving)
 };
 
 // Rows of a gates record; q^ and k^ are the convolved activations' rows times kQScale
 // and kKScale (zero beyond the sequence).
-enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kGateRows };
+// kEQ and kLK: kE and kL times the factors that the bf16 rows of Q and K lack.
+enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kEQ, kLK, kGateRows };
 
-constexpr size_t kKeyRecordFloats = 4 * static_cast<size_t>(kWide);
+constexpr size_t kKeyRecordFloats = 6 * static_cast<size_t>(kWide);
 constexpr size_t kRecordFloats = 5 * static_cast<size_t>(kWide) + 4 * kSquare + kGateRows * kC +
                                  2 * static_cast<size_t>(kState);
 
@@ -282,6 +285,34 @@ __device__ inline unsigned lane_piece(int h, int n) {
 }
 
 // ---------------------------------------------------------------------------
+// The rows of Q and K as operands of the sequential kernels where the activations are
+// bf16: a row times a power of two, which is what its scale is but for a fraction in [1, 2),
+// is bf16 as well and one piece instead of three, half the bytes and half the products; the
+// fractions go with the other factors of a token (kEQ, kLK).  A value times one row's scale
+// has lost nothing that bf16 holds: taken out of the scaled row again (q_whole, k_whole)
+// the fraction leaves the exact bf16 number.  Operand (row block, step) is 1 KiB: lane
+// (n, quarter) has elements 32 step + 16 (e / 4) + 4 quarter + e % 4 of row n of the block.
+struct KeyOperands {
+  static constexpr unsigned kRowsOfK = 0, kRowsOfQ = 2 * kWide, kColumnsOfK = 4 * kWide, kColumnsOfQ = 6 * kWide;
+  static constexpr unsigned kChunkBytes = 8 * kWide;
+  Record memory;
+  __device__ KeyOperands(const ChunkedArgs& a, int key_head)
+      : memory(reinterpret_cast<const float*>(a.r.keys) + static_cast<size_t>(key_head) * a.chunks * (kChunkBytes / 4),
+               static_cast<size_t>(a.chunks) * (kChunkBytes / 4)) {}
+  __device__ void put(float4 first, float4 second, unsigned lane, unsigned uniform) const {
+    const uint4 bits = make_uint4(pack_bf16(first.x, first.y), pack_bf16(first.z, first.w),
+                                  pack_bf16(second.x, second.y), pack_bf16(second.z, second.w));
+    memory.put4(__builtin_bit_cast(float4, bits), lane, uniform);
+  }
+  __device__ bf16x8 get(unsigned lane, unsigned uniform) const {
+    return __builtin_bit_cast(bf16x8, memory.get4(lane, uniform));
+  }
+};
+__device__ inline float fraction_of(float scale) {
+  return __uint_as_float((__float_as_uint(scale) & 0x007fffffu) | 0x3f800000u);
+}
+__device__ inline float4 product(float4 a, float4 b) { return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); }
+
 // T, W, U, P and the gates of one chunk.  68 KiB of LDS, two workgroups a compute
 // unit.  The inverse is made by blocks: the four 16 x 16 diagonal blocks by forward
 // substitution, one wave each, then -T22 A21 T11 twice on the matrix cores (a
@@ -298,6 +329,7 @@ chunk_prepare_kernel(ChunkedArgs a) {
       };
     };
     float g[kC], beta[kC], fk[kC];
+    float q_fraction[kC], k_fraction[kC], q_whole[kC], k_whole[kC];
   } sm;
   const ChunkView v(a, blockIdx.x, blockIdx.y);
   const int tid = threadIdx.x, lane = tid % 64;
@@ -367,13 +399,21 @@ chunk_prepare_kernel(ChunkedArgs a) {
         store4(&sm.k[i][4 * n16 + 64 * j], make_float4(kv[0] * ik, kv[1] * ik, kv[2] * ik, kv[3] * ik));
       }
       if (n16 == 0) {
-        gates[kQScale * kC + i] = iq / norm_scale;
+        const float q_scale = iq / norm_scale;
+        gates[kQScale * kC + i] = q_scale;
         gates[kKScale * kC + i] = ik;
+        // a scale's fraction in [1, 2) (a zero stays one), and what takes it out of a row again
+        const float q_fraction = q_scale == 0.0f ? 0.0f : fraction_of(q_scale);
+        const float k_fraction = ik == 0.0f ? 0.0f : fraction_of(ik);
+        sm.q_fraction[i] = q_fraction, sm.k_fraction[i] = k_fraction;
+        sm.q_whole[i] = q_fraction == 0.0f ? 0.0f : 1.0f / q_fraction;
+        sm.k_whole[i] = k_fraction == 0.0f ? 0.0f : 1.0f / k_fraction;
       }
     }
   }
   // gates (sequence_delta_net.cc:88-96); tokens beyond the sequence neither
   // decay nor write
+  float e = 0.0f, l = 0.0f;
   if (wave == 0) {
     const int t = v.t0 + lane;
     float g = 0.0f, beta = 0.0f;
@@ -393,7 +433,7 @@ chunk_prepare_kernel(ChunkedArgs a) {
       sum = lane >= i ? sum + next : sum;
     }
     g = sum;
-    const float e = expf(g), l = expf(__shfl(g, 63, 64) - g);
+    e = expf(g), l = expf(__shfl(g, 63, 64) - g);
     gates[kG * kC + lane] = g;
     gates[kBeta * kC + lane] = beta;
     gates[kE * kC + lane] = e;
@@ -403,13 +443,21 @@ chunk_prepare_kernel(ChunkedArgs a) {
     sm.fk[lane] = beta * e;
   }
   __syncthreads();
+  if (wave == 0) {
+    gates[kEQ * kC + lane] = e * sm.q_fraction[lane];
+    gates[kLK * kC + lane] = l * sm.k_fraction[lane];
+  }
   // k^ k^T and q^ k^T by 16 x 16 tiles on and below the diagonal: wave w takes row w of
   // the first and row 3 - w of the second, five tiles
   const bool first_of_group = v.head % (a.vh / a.kh) == 0;
-  const Record k_rows = v.key(a.r.k_rows), q_rows = v.key(a.r.q_rows);
   floatx4 kk[4], qk[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b) kk[b] = qk[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  const Record k_rows = v.key(a.r.k_rows), q_rows = v.key(a.r.q_rows);
+  const KeyOperands operands(a, v.key_head());
+  const unsigned operand_at = 16 * lane + blockIdx.x * KeyOperands::kChunkBytes;
+  float4 k_before, q_before;
+  const float k_whole = sm.k_whole[16 * wave + n16], q_whole = sm.q_whole[16 * (3 - wave) + n16];
 #pragma unroll
   for (int s = 0; s < kD / 16; ++s) {
     const float4 kr = load4(&sm.k[16 * wave + n16][16 * s + 4 * quarter]);
@@ -423,7 +471,15 @@ chunk_prepare_kernel(ChunkedArgs a) {
     }
     if (first_of_group) {
       k_rows.put4(kr, 16 * lane, piece_at<kD>(wave, 4 * s));
-      q_rows.put4(qr, 16 * lane, piece_at<kD>(3 - wave, 4 * s));
+      if (!a.round) {
+        q_rows.put4(qr, 16 * lane, piece_at<kD>(3 - wave, 4 * s));
+      } else if (s % 2 == 1) {
+        operands.put(scaled(k_before, k_whole), scaled(kr, k_whole), operand_at,
+                     KeyOperands::kRowsOfK + (4 * wave + s / 2) * 1024);
+        operands.put(scaled(q_before, q_whole), scaled(qr, q_whole), operand_at,
+                     KeyOperands::kRowsOfQ + (4 * (3 - wave) + s / 2) * 1024);
+      }
+      k_before = kr, q_before = qr;
     }
   }
   if (first_of_group) {
@@ -432,11 +488,17 @@ chunk_prepare_kernel(ChunkedArgs a) {
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const int b = 2 * wave + t;
-        k_columns.put4(gather4(&sm.k[16 * s + 4 * quarter][16 * b + n16], kWidePad), 16 * lane,
-                       piece_at<kC>(b, 4 * s));
-        q_columns.put4(gather4(&sm.q[16 * s + 4 * quarter][16 * b + n16], kWidePad), 16 * lane,
-                       piece_at<kC>(b, 4 * s));
+        const int b = 2 * wave + t, row = 16 * s + 4 * quarter;
+        float4 kc = gather4(&sm.k[row][16 * b + n16], kWidePad), qc = gather4(&sm.q[row][16 * b + n16], kWidePad);
+        k_columns.put4(kc, 16 * lane, piece_at<kC>(b, 4 * s));
+        q_columns.put4(qc, 16 * lane, piece_at<kC>(b, 4 * s));
+        if (!a.round) continue;
+        kc = product(kc, load4(&sm.k_whole[row])), qc = product(qc, load4(&sm.q_whole[row]));
+        if (s % 2 == 1) {
+          operands.put(k_before, kc, operand_at, KeyOperands::kColumnsOfK + (2 * b + s / 2) * 1024);
+          operands.put(q_before, qc, operand_at, KeyOperands::kColumnsOfQ + (2 * b + s / 2) * 1024);
+        }
+        k_before = kc, q_before = qc;
       }
   }
   lds_barrier();  // the rows of q^ make room for P, then A, and for T
@@ -665,30 +727,51 @@ __device__ inline Record head_records(const ChunkedArgs& a, const float* records
 // that publishes it.  The fences keep that order.
 __device__ inline void keep_order() { __builtin_amdgcn_sched_barrier(0); }
 
+// Eight elements of a left operand as they come from memory: FP32 numbers that become three
+// pieces, or bf16.
+struct Eight {
+  float4 first, second;
+};
+template <bool BF16>
+using KeyEight = std::conditional_t<BF16, bf16x8, Eight>;
+struct Nothing {};
+__device__ inline Pieces as_left(const Eight& e) { return split_eight(e.first, e.second); }
+
 // The products of one left operand while the next one is made and its right sides are
 // read (step -1: they stay): a matrix instruction and a few vector instructions take turns.
-template <int TILES, int STEPS>
-__device__ inline void step(floatx4 (&acc)[TILES], Pieces& left, Pieces (&right)[TILES], float4 next_a, float4 next_b,
-                            const OperandLds<STEPS>* from, int next_step, int lane) {
+template <int TILES, int STEPS, class Left, class Next>
+__device__ inline void step(floatx4 (&acc)[TILES], const Left& left, Pieces (&right)[TILES], const Next& next,
+                            Pieces& next_left, const OperandLds<STEPS>* from, int next_step, int lane) {
+  constexpr bool kThree = std::is_same_v<Left, Pieces>, kSplit = std::is_same_v<Next, Eight>;
   keep_order();
   Pieces read[TILES];
 #pragma unroll
   for (int c = 0; c < TILES; ++c) read[c] = next_step >= 0 ? from[c].get(next_step, lane) : right[c];
   keep_order();
-  Splitter next(next_a, next_b);
-  constexpr int kLeft[6] = {2, 1, 1, 0, 0, 0}, kRight[6] = {0, 1, 0, 2, 1, 0};  // smallest products first
+  Eight numbers{};
+  if constexpr (kSplit) numbers = next;
+  Splitter split(numbers.first, numbers.second);
+  // smallest products first
+  constexpr int kProducts = kThree ? 6 : 3, kSlots = kProducts * TILES;
+  constexpr int kLeft[6] = {2, 1, 1, 0, 0, 0}, kRight[6] = {0, 1, 0, 2, 1, 0};
 #pragma unroll
-  for (int i = 0; i < 6; ++i) {
+  for (int i = 0; i < kProducts; ++i) {
 #pragma unroll
     for (int c = 0; c < TILES; ++c) {
-      acc[c] = mfma16(left.part[kLeft[i]], right[c].part[kRight[i]], acc[c]);
+      if constexpr (kThree)
+        acc[c] = mfma16(left.part[kLeft[i]], right[c].part[kRight[i]], acc[c]);
+      else
+        acc[c] = mfma16(left, right[c].part[2 - i], acc[c]);
+      if constexpr (kSplit) {
+        constexpr int kEach = (Splitter::kSteps + kSlots - 1) / kSlots;
 #pragma unroll
-      for (int s = 0; s < 2 / TILES; ++s)
-        if ((i * TILES + c) * (2 / TILES) + s < Splitter::kSteps) next((i * TILES + c) * (2 / TILES) + s, true);
+        for (int s = 0; s < kEach; ++s)
+          if ((i * TILES + c) * kEach + s < Splitter::kSteps) split((i * TILES + c) * kEach + s, true);
+      }
       keep_order();
     }
   }
-  left = next.pieces();
+  if constexpr (kSplit) next_left = split.pieces();
 #pragma unroll
   for (int c = 0; c < TILES; ++c) right[c] = read[c];
 }
@@ -698,20 +781,64 @@ __device__ inline void read_right(Pieces (&right)[TILES], const OperandLds<STEPS
   for (int c = 0; c < TILES; ++c) right[c] = from[c].get(step, lane);
 }
 
+// The four steps of a product by keys or queries.  As bf16 they are multiplied from the
+// registers that they arrive in and requested again for the next chunk right after; a copy of
+// one that is still on its way would wait for it.  As FP32 each is split a step ahead.
+template <int TILES, bool BF16>
+struct KeySteps {
+  KeyEight<BF16> eight[4];
+  // the step before the first
+  template <int STEPS>
+  __device__ void enter(floatx4 (&acc)[TILES], Pieces& left, Pieces (&right)[TILES], const OperandLds<STEPS>* from,
+                        int next_step, int lane) {
+    if constexpr (BF16)
+      step<TILES>(acc, left, right, Nothing(), left, from, next_step, lane);
+    else
+      step<TILES>(acc, left, right, eight[0], left, from, next_step, lane);
+  }
+  template <class Request>
+  __device__ void entered(Request request) const {
+    if constexpr (!BF16) request(0);
+  }
+  // step i < 3
+  template <int STEPS, class Request>
+  __device__ void go(int i, floatx4 (&acc)[TILES], Pieces& left, Pieces (&right)[TILES], const OperandLds<STEPS>* from,
+                     int next_step, int lane, Request request) {
+    if constexpr (BF16) {
+      step<TILES>(acc, eight[i], right, Nothing(), left, from, next_step, lane);
+      request(i);
+    } else {
+      step<TILES>(acc, left, right, eight[i + 1], left, from, next_step, lane);
+      request(i + 1);
+    }
+  }
+  // the last one, next to the splitting of the next product's left operand
+  template <int STEPS, class Request>
+  __device__ void finish(floatx4 (&acc)[TILES], Pieces& left, Pieces (&right)[TILES], const Eight& next,
+                         const OperandLds<STEPS>* from, int next_step, int lane, Request request) {
+    if constexpr (BF16) {
+      step<TILES>(acc, eight[3], right, next, left, from, next_step, lane);
+      request(3);
+    } else {
+      step<TILES>(acc, left, right, next, left, from, next_step, lane);
+    }
+  }
+};
+
 // Eight waves: the first four carry the chain, wave w rows 16 w .. + 15 of the 64-row
 // products and rows 32 w .. + 31 of the state; the others do what the chain does not wait
 // for, the same rows.  Two waves a SIMD cover each other's waits for LDS and barriers.
-// A chunk of two tiles is 2700 cycles of matrix instructions a SIMD, 5000 of vector
-// instructions and 120 KiB of operands a compute unit, which at the 20 bytes a clock that
-// one gets of a busy L2 are 6000: with 48 heads a chunk takes 9400.  Operands kept as
-// pieces (6 bytes an element instead of 4 bytes and the splitting) took 178 and 159 us
-// where these take 147 and 139, with the FP32 instruction 184 and 187 (2048 tokens, 48
-// heads).
+// With bf16 activations a chunk of two tiles is 1900 cycles of matrix instructions a SIMD,
+// 3400 of vector instructions and 88 KiB of operands a compute unit, which at the 20 bytes a
+// clock that one gets of a busy L2 are 4400: with 48 heads a chunk takes 7900, 5700 of them
+// where few heads leave the memory idle.  2048 tokens of 48 heads: 127 and 104 us; with keys and
+// queries of three pieces 147 and 138, with all operands kept as pieces (6 bytes an element
+// instead of 4 and the splitting) 178 and 159, with the FP32 instruction 184 and 187.
 constexpr int kSequentialThreads = 512;
 
-// S entering every chunk, Dl and O of every chunk.  84 matrix instructions a row of waves,
-// chunk and tile, the 36 of O off the chain.  Operands are requested a chunk ahead.
-template <int TILES>
+// S entering every chunk, Dl and O of every chunk.  60 matrix instructions a row of waves,
+// chunk and tile, the 24 of O off the chain (84 and 36 with FP32 keys).  Operands are requested a chunk ahead.
+template <int TILES, bool BF16>
 __global__ void __launch_bounds__(kSequentialThreads)
 chunk_states_forward_kernel(ChunkedArgs a) {
   __shared__ OperandLds<4> state[TILES];
@@ -726,12 +853,16 @@ chunk_states_forward_kernel(ChunkedArgs a) {
   // the lane's places in the records of the chunk whose operands are requested next
   // four rows of a column -> four columns of a row: the lane's place in rows(Dl), rows(S)
   const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;
-  unsigned wide_at = 16 * lane, square_at = 16 * lane, gates_at = 4 * rows;
+  unsigned wide_at = 16 * lane, keys_at = 16 * lane, square_at = 16 * lane, gates_at = 4 * rows;
+  constexpr unsigned kKeysBytes = BF16 ? KeyOperands::kChunkBytes : kWide * 4;
+  const KeyOperands operands(a, key_head);
   const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
   Pieces left, right[TILES];  // the operands of the products that come next
   if (chain) {
     __builtin_amdgcn_s_setprio(2);
-    float4 w[8], k[2][4], u[TILES], l_rows;
+    Eight w[4];
+    KeySteps<TILES, BF16> k;  // step i: operand tile i % 2, tokens 32 (i / 2) ..
+    float4 u[TILES], l_rows;
     float decay;
     const Record w_memory = head_records(a, a.r.w_rows, head, kWide),
                  k_memory = head_records(a, a.r.k_columns, key_head, kWide),
@@ -739,12 +870,21 @@ chunk_states_forward_kernel(ChunkedArgs a) {
                  dl_memory = head_records(a, a.r.dl_rows, head, kWide),
                  s0_memory = head_records(a, a.r.s0, head, kState);
     const unsigned u_at = piece_at<kC>(slice.col0 / 16, 4 * wave);
-    auto request_w = [&](int s) { w[s] = w_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
-    auto request_k = [&](int t, int s) { k[t][s] = k_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+    auto request_w = [&](int s) {
+      w[s] = {w_memory.get4(wide_at, piece_at<kD>(wave, 8 * s)), w_memory.get4(wide_at, piece_at<kD>(wave, 8 * s + 4))};
+    };
+    auto request_k = [&](int i) {
+      const int block = 2 * wave + i % 2, s = i / 2;
+      if constexpr (BF16)
+        k.eight[i] = operands.get(keys_at, KeyOperands::kColumnsOfK + (2 * block + s) * 1024);
+      else
+        k.eight[i] = {k_memory.get4(keys_at, piece_at<kC>(block, 8 * s)),
+                      k_memory.get4(keys_at, piece_at<kC>(block, 8 * s + 4))};
+    };
     auto request_rest = [&]() {
 #pragma unroll
       for (int c = 0; c < TILES; ++c) u[c] = u_memory.get4(wide_at, u_at + piece_at<kC>(c, 0));
-      l_rows = gates.get4(gates_at, 4 * kL * kC);
+      l_rows = gates.get4(gates_at, 4 * (BF16 ? kLK : kL) * kC);
       decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
     };
     floatx4 acc[2][TILES];
@@ -752,24 +892,25 @@ chunk_states_forward_kernel(ChunkedArgs a) {
     for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
     // in the loop's order, so that the waits in it need not cover another one
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_w(s), keep_order();
+    for (int s = 0; s < 4; ++s) request_w(s), keep_order();
     request_rest();
     keep_order();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_k(s / 2 % 2, s / 4 * 2 + s % 2), keep_order();
-    left = split_eight(w[0], w[1]);
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+    for (int i = 0; i < 4; ++i) request_k(i), keep_order();
+    left = as_left(w[0]);
+    int chunk = 0;
+    do {
       // past the end the last chunk's operands are requested again
       const unsigned delta_now = wide_at + transposed_at, state_now = 16 * lane + transposed_at + chunk * (kState * 4);
       const bool more = chunk + 1 < a.chunks;
-      wide_at += more ? kWide * 4 : 0, gates_at += more ? kGateRows * kC * 4 : 0;
+      wide_at += more ? kWide * 4 : 0, keys_at += more ? kKeysBytes : 0, gates_at += more ? kGateRows * kC * 4 : 0;
 #pragma unroll
       for (int c = 0; c < TILES; ++c) state[c].put(wave, lane, state_pieces(acc[0][c], acc[1][c]));
       keep_order();
       lds_barrier();
       floatx4 part[TILES];
       read_right<TILES>(right, state, 0, lane);
-      request_w(0), request_w(1);  // split before the loop and at its end
+      request_w(0);  // split before the loop and at its end
       keep_order();
       // rows(S): 16 rows a store, four columns a lane
 #pragma unroll
@@ -781,11 +922,11 @@ chunk_states_forward_kernel(ChunkedArgs a) {
         part[c] = none;
       }
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        step<TILES>(part, left, right, s < 3 ? w[2 * s + 2] : k[0][0], s < 3 ? w[2 * s + 3] : k[0][1], state,
-                    s < 3 ? s + 1 : -1, lane);
-        if (s < 3) request_w(2 * s + 2), request_w(2 * s + 3);
+      for (int s = 0; s < 3; ++s) {
+        step<TILES>(part, left, right, w[s + 1], left, state, s + 1, lane);
+        request_w(s + 1);
       }
+      k.enter(part, left, right, state, -1, lane);
       float4 dl[TILES];
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
@@ -800,61 +941,65 @@ chunk_states_forward_kernel(ChunkedArgs a) {
       lds_barrier();
       read_right<TILES>(right, left_delta, 0, lane);
       request_rest();
-      request_k(0, 0), request_k(0, 1);
+      k.entered(request_k);
       keep_order();
 #pragma unroll
       for (int c = 0; c < TILES; ++c)
         dl_memory.put4(quad_transpose(dl[c]), delta_now, piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
-      // k[t][2 s], k[t][2 s + 1] in the order s, t
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = (i + 1) % 2, s = (i + 1) / 2;
-        step<TILES>(acc[i % 2], left, right, i < 3 ? k[t][2 * s] : w[0], i < 3 ? k[t][2 * s + 1] : w[1], left_delta,
-                    i == 1 ? 1 : -1, lane);
-        if (i < 3) request_k(t, 2 * s), request_k(t, 2 * s + 1);
-      }
-    }
+      for (int i = 0; i < 3; ++i) k.go(i, acc[i % 2], left, right, left_delta, i == 1 ? 1 : -1, lane, request_k);
+      k.finish(acc[1], left, right, w[0], left_delta, -1, lane, request_k);
+    } while (++chunk < a.chunks);
   } else {
-    float4 q[8], p[4], e_rows;
+    KeySteps<TILES, BF16> q;
+    Eight p[2];
+    float4 e_rows;
     const Record q_memory = head_records(a, a.r.q_rows, key_head, kWide),
                  p_memory = head_records(a, a.r.p_rows, head, kSquare);
     const unsigned core_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
-    auto request_q = [&](int s) { q[s] = q_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
-    auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
+    auto request_q = [&](int s) {
+      if constexpr (BF16)
+        q.eight[s] = operands.get(keys_at, KeyOperands::kRowsOfQ + (4 * wave + s) * 1024);
+      else
+        q.eight[s] = {q_memory.get4(keys_at, piece_at<kD>(wave, 8 * s)),
+                      q_memory.get4(keys_at, piece_at<kD>(wave, 8 * s + 4))};
+    };
+    auto request_p = [&](int s) {
+      p[s] = {p_memory.get4(square_at, piece_at<kC>(wave, 8 * s)), p_memory.get4(square_at, piece_at<kC>(wave, 8 * s + 4))};
+    };
+    auto request_e = [&]() { e_rows = gates.get4(gates_at, 4 * (BF16 ? kEQ : kE) * kC); };
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_q(s), keep_order();
-    e_rows = gates.get4(gates_at, 4 * kE * kC);
+    for (int s = 0; s < 4; ++s) request_q(s), keep_order();
+    request_e();
     keep_order();
 #pragma unroll
-    for (int s = 0; s < 4; ++s) request_p(s), keep_order();
-    left = split_eight(q[0], q[1]);
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+    for (int s = 0; s < 2; ++s) request_p(s), keep_order();
+    if constexpr (!BF16) left = as_left(q.eight[0]);
+    int chunk = 0;
+    do {
       const Tokens core = ChunkView(a, chunk, head).heads(a.core);
       const bool more = chunk + 1 < a.chunks;
-      wide_at += more ? kWide * 4 : 0, square_at += more ? kSquare * 4 : 0, gates_at += more ? kGateRows * kC * 4 : 0;
+      keys_at += more ? kKeysBytes : 0, square_at += more ? kSquare * 4 : 0, gates_at += more ? kGateRows * kC * 4 : 0;
       lds_barrier();
       floatx4 out[TILES];
       read_right<TILES>(right, state, 0, lane);
-      request_q(0), request_q(1);
+      q.entered(request_q);
 #pragma unroll
       for (int c = 0; c < TILES; ++c) out[c] = none;
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        step<TILES>(out, left, right, s < 3 ? q[2 * s + 2] : p[0], s < 3 ? q[2 * s + 3] : p[1], state,
-                    s < 3 ? s + 1 : -1, lane);
-        if (s < 3) request_q(2 * s + 2), request_q(2 * s + 3);
-      }
+      for (int s = 0; s < 3; ++s) q.go(s, out, left, right, state, s + 1, lane, request_q);
+      q.finish(out, left, right, p[0], state, -1, lane, request_q);
 #pragma unroll
       for (int c = 0; c < TILES; ++c)
         out[c][0] *= e_rows.x, out[c][1] *= e_rows.y, out[c][2] *= e_rows.z, out[c][3] *= e_rows.w;
       keep_order();
-      e_rows = gates.get4(gates_at, 4 * kE * kC);
-      request_p(0), request_p(1);
+      request_e();
+      request_p(0);
       lds_barrier();
       read_right<TILES>(right, delta, 0, lane);
-      step<TILES>(out, left, right, p[2], p[3], delta, 1, lane);
-      request_p(2), request_p(3);
-      step<TILES>(out, left, right, q[0], q[1], delta, -1, lane);
+      step<TILES>(out, left, right, p[1], left, delta, 1, lane);
+      request_p(1);
+      q.enter(out, left, right, delta, -1, lane);
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
         // four tokens of a column -> four columns of a token
@@ -863,14 +1008,14 @@ chunk_states_forward_kernel(ChunkedArgs a) {
                                        round_if(out[c][2], a.round), round_if(out[c][3], a.round)));
         core.put4(o, core_at, 4 * kTile * c);
       }
-    }
+    } while (++chunk < a.chunks);
   }
 }
 
 // The gradient of the state leaving every chunk and dDl of every chunk, chunks in
-// reverse.  84 matrix instructions a row of waves, chunk and tile, the 36 with dO off the
-// chain: the other waves leave P^T dO and (diag(E) Q^)^T dO of the next chunk in LDS.
-template <int TILES>
+// reverse.  60 matrix instructions a row of waves, chunk and tile, the 24 with dO off the
+// chain (84 and 36 with FP32 keys): the other waves leave P^T dO and (diag(E) Q^)^T dO of the next chunk in LDS.
+template <int TILES, bool BF16>
 __global__ void __launch_bounds__(kSequentialThreads)
 chunk_states_backward_kernel(ChunkedArgs a) {
   __shared__ OperandLds<4> state[TILES];
@@ -885,22 +1030,35 @@ chunk_states_backward_kernel(ChunkedArgs a) {
   const int head = slice.head, key_head = head / (a.vh / a.kh);
   const Record gates = head_records(a, a.r.gates, head, kGateRows * kC);
   const unsigned last = a.chunks - 1;
-  unsigned wide_at = 16 * lane + last * (kWide * 4), square_at = 16 * lane + last * (kSquare * 4),
-           gates_at = 4 * rows + last * (kGateRows * kC * 4);
+  constexpr unsigned kKeysBytes = BF16 ? KeyOperands::kChunkBytes : kWide * 4;
+  unsigned wide_at = 16 * lane + last * (kWide * 4), keys_at = 16 * lane + last * kKeysBytes,
+           square_at = 16 * lane + last * (kSquare * 4), gates_at = 4 * rows + last * (kGateRows * kC * 4);
+  const KeyOperands operands(a, key_head);
   const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
   Pieces left, right[TILES];  // the operands of the products that come next
   if (chain) {
     __builtin_amdgcn_s_setprio(2);
-    float4 k[8], w[2][4], k_scale;
+    KeySteps<TILES, BF16> k;
+    Eight w[2][2];
+    float4 k_scale;
     float decay;
     const Record k_memory = head_records(a, a.r.k_rows, key_head, kWide),
                  w_memory = head_records(a, a.r.w_columns, head, kWide),
                  ddl_rows = head_records(a, a.r.ddl_rows, head, kWide), ds1_memory = head_records(a, a.r.ds1, head, kState);
     const int transposed_at = n / 4 * kPiece + (4 * quarter + n % 4) * 16 - 16 * lane;  // as above
-    auto request_k = [&](int s) { k[s] = k_memory.get4(wide_at, piece_at<kD>(wave, 4 * s)); };
-    auto request_w = [&](int t, int s) { w[t][s] = w_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+    auto request_k = [&](int s) {
+      if constexpr (BF16)
+        k.eight[s] = operands.get(keys_at, KeyOperands::kRowsOfK + (4 * wave + s) * 1024);
+      else
+        k.eight[s] = {k_memory.get4(keys_at, piece_at<kD>(wave, 8 * s)),
+                      k_memory.get4(keys_at, piece_at<kD>(wave, 8 * s + 4))};
+    };
+    auto request_w = [&](int t, int s) {
+      w[t][s] = {w_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 8 * s)),
+                 w_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 8 * s + 4))};
+    };
     auto request_gates = [&]() {
-      k_scale = gates.get4(gates_at, 4 * kL * kC);
+      k_scale = gates.get4(gates_at, 4 * (BF16 ? kLK : kL) * kC);
       decay = gates.get(gates_at - 4 * rows, 4 * (kE * kC + kC - 1));
     };
     floatx4 acc[2][TILES];
@@ -908,26 +1066,27 @@ chunk_states_backward_kernel(ChunkedArgs a) {
     for (int c = 0; c < TILES; ++c) acc[0][c] = acc[1][c] = none;
     // in the loop's order, so that the waits in it need not cover another one
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_k(s), keep_order();
+    for (int s = 0; s < 4; ++s) request_k(s), keep_order();
     request_gates();
     keep_order();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_w(s / 2 % 2, s / 4 * 2 + s % 2), keep_order();
-    left = split_eight(k[0], k[1]);
+    for (int s = 0; s < 4; ++s) request_w(s % 2, s / 2), keep_order();
+    if constexpr (!BF16) left = as_left(k.eight[0]);
     lds_barrier();  // the first chunk's dO is in LDS,
     lds_barrier();  // and what the other waves hand over
-    for (int chunk = a.chunks - 1; chunk >= 0; --chunk) {
+    int chunk = a.chunks - 1;
+    do {
       // before the first the first chunk's operands are requested again
       const unsigned wide_now = wide_at, state_now = 16 * lane + transposed_at + chunk * (kState * 4);
       const bool more = chunk > 0;
-      wide_at -= more ? kWide * 4 : 0, gates_at -= more ? kGateRows * kC * 4 : 0;
+      wide_at -= more ? kWide * 4 : 0, keys_at -= more ? kKeysBytes : 0, gates_at -= more ? kGateRows * kC * 4 : 0;
 #pragma unroll
       for (int c = 0; c < TILES; ++c) state[c].put(wave, lane, state_pieces(acc[0][c], acc[1][c]));
       keep_order();
       lds_barrier();
       floatx4 part[TILES];
       read_right<TILES>(right, state, 0, lane);
-      request_k(0), request_k(1);
+      k.entered(request_k);
       keep_order();
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
@@ -938,11 +1097,8 @@ chunk_states_backward_kernel(ChunkedArgs a) {
         part[c] = none;
       }
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        step<TILES>(part, left, right, s < 3 ? k[2 * s + 2] : w[0][0], s < 3 ? k[2 * s + 3] : w[0][1], state,
-                    s < 3 ? s + 1 : -1, lane);
-        if (s < 3) request_k(2 * s + 2), request_k(2 * s + 3);
-      }
+      for (int s = 0; s < 3; ++s) k.go(s, part, left, right, state, s + 1, lane, request_k);
+      k.finish(part, left, right, w[0][0], state, -1, lane, request_k);
       float4 dd[TILES];
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
@@ -963,47 +1119,59 @@ chunk_states_backward_kernel(ChunkedArgs a) {
       lds_barrier();
       read_right<TILES>(right, delta, 0, lane);
       request_gates();
-      request_w(0, 0), request_w(0, 1);
+      request_w(0, 0);
       keep_order();
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
         ddl_rows.put4(quad_transpose(dd[c]), wide_now + transposed_at,
                       piece_at<kD>(wave, (slice.col0 + kTile * c) / 4));
       }
-      // w[t][2 s], w[t][2 s + 1] in the order s, t
+      // w[t][s] in the order s, t
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 3; ++i) {
         const int t = (i + 1) % 2, s = (i + 1) / 2;
-        step<TILES>(acc[i % 2], left, right, i < 3 ? w[t][2 * s] : k[0], i < 3 ? w[t][2 * s + 1] : k[1], delta,
-                    i == 1 ? 1 : -1, lane);
-        if (i < 3) request_w(t, 2 * s), request_w(t, 2 * s + 1);
+        step<TILES>(acc[i % 2], left, right, w[t][s], left, delta, i == 1 ? 1 : -1, lane);
+        request_w(t, s);
       }
-    }
+      k.enter(acc[1], left, right, delta, -1, lane);
+    } while (--chunk >= 0);
   } else {
-    float4 p[4], q[2][4], out[TILES], q_scale;
+    Eight p[2];
+    KeySteps<TILES, BF16> q;  // step i: operand tile i % 2, tokens 32 (i / 2) ..
+    float4 out[TILES], q_scale;
     const Record p_memory = head_records(a, a.r.p_columns, head, kSquare),
                  q_memory = head_records(a, a.r.q_columns, key_head, kWide);
     const unsigned out_at = (rows + n % 4) * (a.vh * kD * 4) + 4 * (slice.col0 + n / 4 * 4);
-    auto request_p = [&](int s) { p[s] = p_memory.get4(square_at, piece_at<kC>(wave, 4 * s)); };
-    auto request_q = [&](int t, int s) { q[t][s] = q_memory.get4(wide_at, piece_at<kC>(2 * wave + t, 4 * s)); };
+    auto request_p = [&](int s) {
+      p[s] = {p_memory.get4(square_at, piece_at<kC>(wave, 8 * s)), p_memory.get4(square_at, piece_at<kC>(wave, 8 * s + 4))};
+    };
+    auto request_q = [&](int i) {
+      const int block = 2 * wave + i % 2, s = i / 2;
+      if constexpr (BF16)
+        q.eight[i] = operands.get(keys_at, KeyOperands::kColumnsOfQ + (2 * block + s) * 1024);
+      else
+        q.eight[i] = {q_memory.get4(keys_at, piece_at<kC>(block, 8 * s)),
+                      q_memory.get4(keys_at, piece_at<kC>(block, 8 * s + 4))};
+    };
     auto request_out = [&](int chunk) {
       const Tokens d_out = ChunkView(a, max(chunk, 0), head).heads(a.dcore);
 #pragma unroll
       for (int c = 0; c < TILES; ++c) out[c] = d_out.get4(out_at, 4 * kTile * c);
-      q_scale = gates.get4(gates_at, 4 * kE * kC);
+      q_scale = gates.get4(gates_at, 4 * (BF16 ? kEQ : kE) * kC);
     };
     request_out(last);
     keep_order();
 #pragma unroll
-    for (int s = 0; s < 4; ++s) request_p(s), keep_order();
+    for (int s = 0; s < 2; ++s) request_p(s), keep_order();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) request_q(s / 2 % 2, s / 4 * 2 + s % 2), keep_order();
-    left = split_eight(p[0], p[1]);
+    for (int i = 0; i < 4; ++i) request_q(i), keep_order();
+    left = as_left(p[0]);
     // a chunk ahead of the chain: what is handed over lies in LDS before the chain's
     // chunk begins
-    for (int chunk = a.chunks - 1; chunk >= -1; --chunk) {
+    int chunk = a.chunks - 1;
+    do {
       const bool more = chunk > 0;
-      wide_at -= more ? kWide * 4 : 0, square_at -= more ? kSquare * 4 : 0, gates_at -= more ? kGateRows * kC * 4 : 0;
+      keys_at -= more ? kKeysBytes : 0, square_at -= more ? kSquare * 4 : 0, gates_at -= more ? kGateRows * kC * 4 : 0;
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
         const float4 o = quad_transpose(out[c]);  // four columns of a token -> four tokens of a column
@@ -1013,35 +1181,30 @@ chunk_states_backward_kernel(ChunkedArgs a) {
       }
       keep_order();
       lds_barrier();
-      if (chunk >= 0) {
-        floatx4 from_out[TILES], queries[2][TILES];
-        read_right<TILES>(right, grad, 0, lane);
-        request_out(chunk - 1);
-        request_p(0), request_p(1);
+      floatx4 from_out[TILES], queries[2][TILES];
+      read_right<TILES>(right, grad, 0, lane);
+      request_out(chunk - 1);
+      request_p(0);
 #pragma unroll
-        for (int c = 0; c < TILES; ++c) from_out[c] = queries[0][c] = queries[1][c] = none;
-        step<TILES>(from_out, left, right, p[2], p[3], grad, 1, lane);
-        request_p(2), request_p(3);
-        step<TILES>(from_out, left, right, q[0][0], q[0][1], query_grad, 0, lane);
-        request_q(0, 0), request_q(0, 1);
-        // q[t][2 s], q[t][2 s + 1] in the order s, t
+      for (int c = 0; c < TILES; ++c) from_out[c] = queries[0][c] = queries[1][c] = none;
+      step<TILES>(from_out, left, right, p[1], left, grad, 1, lane);
+      request_p(1);
+      q.enter(from_out, left, right, query_grad, 0, lane);
+      q.entered(request_q);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = (i + 1) % 2, s = (i + 1) / 2;
-          step<TILES>(queries[i % 2], left, right, i < 3 ? q[t][2 * s] : p[0], i < 3 ? q[t][2 * s + 1] : p[1],
-                      query_grad, i == 1 ? 1 : -1, lane);
-          if (i < 3) request_q(t, 2 * s), request_q(t, 2 * s + 1);
-        }
+      for (int i = 0; i < 3; ++i) q.go(i, queries[i % 2], left, right, query_grad, i == 1 ? 1 : -1, lane, request_q);
+      q.finish(queries[1], left, right, p[0], query_grad, -1, lane, request_q);
 #pragma unroll
-        for (int c = 0; c < TILES; ++c) {
-          handed[chunk & 1][0][c][wave][lane] = from_out[c];
-          handed[chunk & 1][1][c][wave][lane] = queries[0][c];
-          handed[chunk & 1][2][c][wave][lane] = queries[1][c];
-        }
+      for (int c = 0; c < TILES; ++c) {
+        handed[chunk & 1][0][c][wave][lane] = from_out[c];
+        handed[chunk & 1][1][c][wave][lane] = queries[0][c];
+        handed[chunk & 1][2][c][wave][lane] = queries[1][c];
       }
       keep_order();
       lds_barrier();
-    }
+    } while (--chunk >= 0);
+    lds_barrier();  // the chain's last chunk
+    lds_barrier();
   }
 }
 
@@ -1512,6 +1675,7 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
   a.r.q_columns = at + keys;
   a.r.k_rows = at + 2 * keys;
   a.r.k_columns = at + 3 * keys;
+  a.r.keys = reinterpret_cast<uint16_t*>(at + 4 * keys);
   return a;
 }
 
@@ -1519,6 +1683,11 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
 // tile gets a compute unit of its own one is faster; beyond that compute units hold
 // two tiles anyway, and one workgroup with both loads the operands once.
 int column_tiles(int value_heads) { return value_heads * (kD / kTile) > 256 ? 2 : 1; }
+template <class Launch>
+void by_tiles(const ChunkedArgs& a, Launch launch) {
+  auto with = [&](auto tiles) { a.round ? launch(tiles, std::true_type()) : launch(tiles, std::false_type()); };
+  column_tiles(a.vh) == 2 ? with(std::integral_constant<int, 2>()) : with(std::integral_constant<int, 1>());
+}
 
 }  // namespace
 
@@ -1539,19 +1708,17 @@ int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBack
   chunk_prepare_kernel<<<per_chunk, 256, 0, stream>>>(a);
   const int status = launch_status();
   if (status != 0) return status;
-  if (column_tiles(a.vh) == 2)
-    chunk_states_forward_kernel<2><<<a.vh * (kD / (2 * kTile)), kSequentialThreads, 0, stream>>>(a);
-  else
-    chunk_states_forward_kernel<1><<<a.vh * (kD / kTile), kSequentialThreads, 0, stream>>>(a);
+  by_tiles(a, [&](auto tiles, auto bf16) {
+    chunk_states_forward_kernel<tiles, bf16><<<a.vh * (kD / (tiles * kTile)), kSequentialThreads, 0, stream>>>(a);
+  });
   return launch_status();
 }
 
 int launch_gdn_backward_chunked_reverse(hipStream_t stream, const GdnChunkedBackward& c) {
   const ChunkedArgs a = make_args(c);
-  if (column_tiles(a.vh) == 2)
-    chunk_states_backward_kernel<2><<<a.vh * (kD / (2 * kTile)), kSequentialThreads, 0, stream>>>(a);
-  else
-    chunk_states_backward_kernel<1><<<a.vh * (kD / kTile), kSequentialThreads, 0, stream>>>(a);
+  by_tiles(a, [&](auto tiles, auto bf16) {
+    chunk_states_backward_kernel<tiles, bf16><<<a.vh * (kD / (tiles * kTile)), kSequentialThreads, 0, stream>>>(a);
+  });
   const int status = launch_status();
   if (status != 0) return status;
   chunk_gradients_kernel<<<dim3(a.chunks, a.vh), 256, 0, stream>>>(a);

@@ -359,3 +359,42 @@ def test_each_parameter_gradient_alone(capi, T, kh, vh, taps):
             assert torch.equal(one[name], every[name]), name
     da = activations[2].double()
     assert ((every["dt_bias"].double() - da.sum((0, 1))).abs() <= 256 * 2.0 ** -24 * da.abs().sum((0, 1)) + 1e-30).all()
+
+
+@pytest.mark.parametrize("T,kh,vh", [(1, 2, 2), (64, 3, 3), (129, 2, 32), (130, 11, 33), (200, 16, 48)])
+def test_rows_of_any_scale(capi, T, kh, vh):
+    """Where activations are bf16 the chunked kernels multiply by a row of Q or K times a power
+    of two and put the rest of its scale with the token's other factors: rows from 2^-100 to
+    2^58 (whose squares are 2^127 at most), rows whose squares leave the range (scale zero)
+    and rows of zeros, for one and two column tiles a workgroup, against the token-by-token
+    kernels.  Tolerances as against the oracle: FP32 accuracy for all but the values behind
+    a rounding that fell the other way, which are off by an operand's last bit."""
+    c = make_case(T, kh, vh, 128, 128, 4, seed=T + kh)
+    rng = np.random.default_rng(T)
+    keys = 2 * kh * 128
+    c["conv"][:keys] = [0, 0, 0, 1]
+    exponent = rng.choice([-100, -60, -13, -1, 0, 1, 12, 40, 58, 90], (1, T, 2 * kh, 1))
+    rows = c["qkv"][..., :keys].reshape(1, T, 2 * kh, 128)
+    rows *= np.exp2(exponent).astype(np.float32)
+    rows[rng.random((1, T, 2 * kh)) < 0.05] = 0
+    c["qkv"][..., :keys] = rows.reshape(1, T, keys)
+    p = capi.delta_params(kh, vh, 128, 128, 4)
+    bf = torch.bfloat16
+    args = (p, dev(c["qkv"], bf), dev(c["z"], bf), dev(c["a"], bf), dev(c["b"], bf), dev(c["conv"]),
+            dev(c["a_log"]), dev(c["dt_bias"]), dev(c["norm"]), dev(c["dy"]))
+    got = capi.gdn_layer_backward(*args)
+    assert capi.last_path() == capi.PATH_CHUNKED
+    with capi.force_generic():
+        want = capi.gdn_layer_backward(*args)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dqkv", "dz", "da", "db"), got, want):
+        a, b = a.double().cpu().numpy(), b.double().cpu().numpy()
+        assert np.isfinite(b).all() and np.isfinite(a).all(), name
+        if name == "dqkv":  # a row's gradient is as small as the row is large
+            a, b = (x.reshape(T, 2 * kh + vh, 128) for x in (a, b))
+            scale = np.abs(b).max(-1, keepdims=True) + 1e-30
+        else:
+            scale = np.abs(b) + np.sqrt(np.mean(b ** 2))
+        diff = np.abs(a - b)
+        assert np.all(diff <= 2e-2 * scale), name
+        assert np.mean(diff > 2e-4 * scale) <= 2e-2, name
