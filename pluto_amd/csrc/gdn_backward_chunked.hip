@@ -721,6 +721,62 @@ __device__ inline Record head_records(const ChunkedArgs& a, const float* records
   return Record(records + static_cast<size_t>(head) * a.chunks * elements, a.chunks * elements);
 }
 
+// A chunk's operands on their way into the XCD's L2 two chunks ahead of the products: a piece
+// of 8 KiB, 64 lines, is touched by one wave, and a head's workgroups share the pieces.  A
+// compute unit has few lines on their way at a time, and those from memory stay longest.
+// With two tiles a workgroup each wave off the chain touches one (2048 tokens, 48 heads,
+// both kernels: 232 -> 217 us).  With one tile a chunk is too short to wait for a touched line
+// before the operands behind it, as a wave's loads return in order, and a ninth wave does it
+// (8192 tokens, 16 heads: 605 -> 470 us; as with two tiles 567); with two tiles that wave took
+// registers that the others need (237).  Chunks of FP32 keys are long enough.
+template <int TILES, bool BF16>
+struct Ahead {
+  static constexpr bool kOwnWave = TILES == 1 && BF16;
+  static constexpr unsigned kBytes = 8192;
+  static constexpr int kChunks = 2;  // ahead
+  const void* base = nullptr;
+  unsigned at = 0, step = 0, bytes = 0;
+  float touched = 0.0f;
+  int index;  // of the pieces not yet given away
+  __device__ Ahead(const Slice& slice, int i) : index(slice.col0 / (kTile * TILES) * (2 * TILES) + i) {}
+  // a head's records of `per_chunk` bytes a chunk, of which `wanted` from `offset` on
+  __device__ void add(const void* records, size_t chunks, unsigned per_chunk, unsigned offset, unsigned wanted, int lane) {
+    const int pieces = wanted / kBytes;
+    if (index >= 0 && index < pieces) {
+      base = records, step = per_chunk, bytes = static_cast<unsigned>(chunks * per_chunk);
+      at = offset + index * kBytes + 128 * lane;
+    }
+    index -= pieces;
+  }
+  // a chunk's tokens of a head in [tokens, heads, 128]
+  __device__ void add_tokens(const float* head, int tokens, unsigned row_bytes, int lane) {
+    if (index >= 0 && index < 4) {
+      const size_t all = static_cast<size_t>(tokens - 1) * row_bytes + kD * 4;
+      base = head, step = kC * row_bytes, bytes = static_cast<unsigned>(all < 0xffffffffu ? all : 0xffffffffu);
+      at = (16 * index + lane / 4) * row_bytes + 128 * (lane % 4);
+    }
+    index -= 4;
+  }
+  // chunks that do not exist lie beyond the descriptor or are the first again
+  __device__ void touch(int chunk) {
+    asm volatile("" ::"v"(touched));
+    touched = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000),
+        at + max(chunk, 0) * step, 0, 0));
+  }
+};
+// The ninth wave: its pieces, chunk after chunk, and the barriers of the others.
+template <class Made>
+__device__ inline void touch_chunks(Made made, int first, int direction, int steps) {
+  auto one = made(0), two = made(1);
+  for (int i = 0; i < steps; ++i) {
+    one.touch(first + i * direction);
+    two.touch(first + i * direction);
+    lds_barrier();
+    lds_barrier();
+  }
+}
+
 // Both sequential kernels are chains of products with a barrier between them; requests
 // and stores stand between the multiplications, each request for a register right
 // after the multiplication that read it, and none between a product and the barrier
@@ -830,23 +886,25 @@ struct KeySteps {
 // for, the same rows.  Two waves a SIMD cover each other's waits for LDS and barriers.
 // With bf16 activations a chunk of two tiles is 1900 cycles of matrix instructions a SIMD,
 // 3400 of vector instructions and 88 KiB of operands a compute unit, which at the 20 bytes a
-// clock that one gets of a busy L2 are 4400: with 48 heads a chunk takes 7900, 5700 of them
-// where few heads leave the memory idle.  2048 tokens of 48 heads: 127 and 104 us; with keys and
+// clock that one gets of a busy L2 are 4400: with 48 heads a chunk takes 7300, 5700 of them
+// where few heads leave the memory idle.  2048 tokens of 48 heads: 117 and 101 us; with keys and
 // queries of three pieces 147 and 138, with all operands kept as pieces (6 bytes an element
-// instead of 4 and the splitting) 178 and 159, with the FP32 instruction 184 and 187.
-constexpr int kSequentialThreads = 512;
+// instead of 4 and the splitting) 178 and 159, with the FP32 instruction 184 and 187.  The
+// stores stay with the chain's waves: through LDS by the others they took 1 and 10 us more.
+template <int TILES, bool BF16>
+constexpr int kSequentialThreads = Ahead<TILES, BF16>::kOwnWave ? 576 : 512;
 
 // S entering every chunk, Dl and O of every chunk.  60 matrix instructions a row of waves,
 // chunk and tile, the 24 of O off the chain (84 and 36 with FP32 keys).  Operands are requested a chunk ahead.
 template <int TILES, bool BF16>
-__global__ void __launch_bounds__(kSequentialThreads)
+__global__ void __launch_bounds__((kSequentialThreads<TILES, BF16>))
 chunk_states_forward_kernel(ChunkedArgs a) {
   __shared__ OperandLds<4> state[TILES];
   __shared__ OperandLds<2> delta[TILES], left_delta[TILES];
   const Slice slice = slice_of_block<TILES>(a);
   const int lane = threadIdx.x % 64, quarter = lane / 16, n = lane % 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64 % 4);
-  const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x) < kSequentialThreads / 2;
+  const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x) < 256;
   const int rows = 16 * wave + 4 * quarter;  // of the lane's part of Dl and O
   const int head = slice.head, key_head = head / (a.vh / a.kh);
   const Record gates = head_records(a, a.r.gates, head, kGateRows * kC);
@@ -858,6 +916,23 @@ chunk_states_forward_kernel(ChunkedArgs a) {
   const KeyOperands operands(a, key_head);
   const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
   Pieces left, right[TILES];  // the operands of the products that come next
+  auto ahead_of = [&](int i) {
+    Ahead<TILES, BF16> ahead(slice, i);
+    const size_t of_head = static_cast<size_t>(head) * a.chunks;
+    ahead.add(a.r.w_rows + of_head * kWide, a.chunks, kWide * 4, 0, kWide * 4, lane);
+    ahead.add(a.r.u_columns + of_head * kWide, a.chunks, kWide * 4, 0, kWide * 4, lane);
+    ahead.add(a.r.p_rows + of_head * kSquare, a.chunks, kSquare * 4, 0, kSquare * 4, lane);
+    if constexpr (BF16) {
+      ahead.add(operands.memory.base, a.chunks, kKeysBytes, KeyOperands::kRowsOfQ, 2 * kWide, lane);
+      ahead.add(operands.memory.base, a.chunks, kKeysBytes, KeyOperands::kColumnsOfK, 2 * kWide, lane);
+    }
+    return ahead;
+  };
+  if constexpr (Ahead<TILES, BF16>::kOwnWave)
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 512) {
+      touch_chunks(ahead_of, Ahead<TILES, BF16>::kChunks, 1, a.chunks);
+      return;
+    }
   if (chain) {
     __builtin_amdgcn_s_setprio(2);
     Eight w[4];
@@ -974,6 +1049,7 @@ chunk_states_forward_kernel(ChunkedArgs a) {
     keep_order();
 #pragma unroll
     for (int s = 0; s < 2; ++s) request_p(s), keep_order();
+    Ahead<TILES, BF16> ahead = ahead_of(wave);
     if constexpr (!BF16) left = as_left(q.eight[0]);
     int chunk = 0;
     do {
@@ -989,6 +1065,7 @@ chunk_states_forward_kernel(ChunkedArgs a) {
 #pragma unroll
       for (int s = 0; s < 3; ++s) q.go(s, out, left, right, state, s + 1, lane, request_q);
       q.finish(out, left, right, p[0], state, -1, lane, request_q);
+      if constexpr (!ahead.kOwnWave) ahead.touch(chunk + ahead.kChunks);
 #pragma unroll
       for (int c = 0; c < TILES; ++c)
         out[c][0] *= e_rows.x, out[c][1] *= e_rows.y, out[c][2] *= e_rows.z, out[c][3] *= e_rows.w;
@@ -1016,7 +1093,7 @@ chunk_states_forward_kernel(ChunkedArgs a) {
 // reverse.  60 matrix instructions a row of waves, chunk and tile, the 24 with dO off the
 // chain (84 and 36 with FP32 keys): the other waves leave P^T dO and (diag(E) Q^)^T dO of the next chunk in LDS.
 template <int TILES, bool BF16>
-__global__ void __launch_bounds__(kSequentialThreads)
+__global__ void __launch_bounds__((kSequentialThreads<TILES, BF16>))
 chunk_states_backward_kernel(ChunkedArgs a) {
   __shared__ OperandLds<4> state[TILES];
   __shared__ OperandLds<2> delta[TILES], grad[TILES], query_grad[TILES];
@@ -1025,7 +1102,7 @@ chunk_states_backward_kernel(ChunkedArgs a) {
   const Slice slice = slice_of_block<TILES>(a);
   const int lane = threadIdx.x % 64, quarter = lane / 16, n = lane % 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64 % 4);
-  const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x) < kSequentialThreads / 2;
+  const bool chain = __builtin_amdgcn_readfirstlane(threadIdx.x) < 256;
   const int rows = 16 * wave + 4 * quarter;
   const int head = slice.head, key_head = head / (a.vh / a.kh);
   const Record gates = head_records(a, a.r.gates, head, kGateRows * kC);
@@ -1036,6 +1113,23 @@ chunk_states_backward_kernel(ChunkedArgs a) {
   const KeyOperands operands(a, key_head);
   const floatx4 none = {0.0f, 0.0f, 0.0f, 0.0f};
   Pieces left, right[TILES];  // the operands of the products that come next
+  auto ahead_of = [&](int i) {
+    Ahead<TILES, BF16> ahead(slice, i);
+    const size_t of_head = static_cast<size_t>(head) * a.chunks;
+    ahead.add(a.r.w_columns + of_head * kWide, a.chunks, kWide * 4, 0, kWide * 4, lane);
+    ahead.add_tokens(a.dcore + head * kD, a.length, a.vh * kD * 4, lane);
+    ahead.add(a.r.p_columns + of_head * kSquare, a.chunks, kSquare * 4, 0, kSquare * 4, lane);
+    if constexpr (BF16) {
+      ahead.add(operands.memory.base, a.chunks, kKeysBytes, KeyOperands::kRowsOfK, 2 * kWide, lane);
+      ahead.add(operands.memory.base, a.chunks, kKeysBytes, KeyOperands::kColumnsOfQ, 2 * kWide, lane);
+    }
+    return ahead;
+  };
+  if constexpr (Ahead<TILES, BF16>::kOwnWave)
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 512) {
+      touch_chunks(ahead_of, static_cast<int>(last) + 1 - Ahead<TILES, BF16>::kChunks, -1, a.chunks + 1);
+      return;
+    }
   if (chain) {
     __builtin_amdgcn_s_setprio(2);
     KeySteps<TILES, BF16> k;
@@ -1165,6 +1259,7 @@ chunk_states_backward_kernel(ChunkedArgs a) {
     for (int s = 0; s < 2; ++s) request_p(s), keep_order();
 #pragma unroll
     for (int i = 0; i < 4; ++i) request_q(i), keep_order();
+    Ahead<TILES, BF16> ahead = ahead_of(wave);
     left = as_left(p[0]);
     // a chunk ahead of the chain: what is handed over lies in LDS before the chain's
     // chunk begins
@@ -1194,6 +1289,7 @@ chunk_states_backward_kernel(ChunkedArgs a) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) q.go(i, queries[i % 2], left, right, query_grad, i == 1 ? 1 : -1, lane, request_q);
       q.finish(queries[1], left, right, p[0], query_grad, -1, lane, request_q);
+      if constexpr (!ahead.kOwnWave) ahead.touch(chunk - ahead.kChunks);
 #pragma unroll
       for (int c = 0; c < TILES; ++c) {
         handed[chunk & 1][0][c][wave][lane] = from_out[c];
@@ -1709,7 +1805,7 @@ int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBack
   const int status = launch_status();
   if (status != 0) return status;
   by_tiles(a, [&](auto tiles, auto bf16) {
-    chunk_states_forward_kernel<tiles, bf16><<<a.vh * (kD / (tiles * kTile)), kSequentialThreads, 0, stream>>>(a);
+    chunk_states_forward_kernel<tiles, bf16><<<a.vh * (kD / (tiles * kTile)), kSequentialThreads<tiles, bf16>, 0, stream>>>(a);
   });
   return launch_status();
 }
@@ -1717,7 +1813,7 @@ int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBack
 int launch_gdn_backward_chunked_reverse(hipStream_t stream, const GdnChunkedBackward& c) {
   const ChunkedArgs a = make_args(c);
   by_tiles(a, [&](auto tiles, auto bf16) {
-    chunk_states_backward_kernel<tiles, bf16><<<a.vh * (kD / (tiles * kTile)), kSequentialThreads, 0, stream>>>(a);
+    chunk_states_backward_kernel<tiles, bf16><<<a.vh * (kD / (tiles * kTile)), kSequentialThreads<tiles, bf16>, 0, stream>>>(a);
   });
   const int status = launch_status();
   if (status != 0) return status;
