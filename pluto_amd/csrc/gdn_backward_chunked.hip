@@ -153,6 +153,8 @@ __device__ inline float4 gather4(const float* p, int stride) {
   return make_float4(p[0], p[stride], p[2 * stride], p[3 * stride]);
 }
 
+__device__ inline void keep_order() { __builtin_amdgcn_sched_barrier(0); }
+
 // Barrier for data exchanged through LDS only: pending global loads and
 // stores stay in flight across it.
 __device__ inline void lds_barrier() {
@@ -288,9 +290,7 @@ __device__ inline unsigned lane_piece(int h, int n) {
 // The rows of Q and K as operands of the sequential kernels where the activations are
 // bf16: a row times a power of two, which is what its scale is but for a fraction in [1, 2),
 // is bf16 as well and one piece instead of three, half the bytes and half the products; the
-// fractions go with the other factors of a token (kEQ, kLK).  A value times one row's scale
-// has lost nothing that bf16 holds: taken out of the scaled row again (q_whole, k_whole)
-// the fraction leaves the exact bf16 number.  Operand (row block, step) is 1 KiB: lane
+// fractions go with the other factors of a token (kEQ, kLK).  Operand (row block, step) is 1 KiB: lane
 // (n, quarter) has elements 32 step + 16 (e / 4) + 4 quarter + e % 4 of row n of the block.
 struct KeyOperands {
   static constexpr unsigned kRowsOfK = 0, kRowsOfQ = 2 * kWide, kColumnsOfK = 4 * kWide, kColumnsOfQ = 6 * kWide;
@@ -299,10 +299,8 @@ struct KeyOperands {
   __device__ KeyOperands(const ChunkedArgs& a, int key_head)
       : memory(reinterpret_cast<const float*>(a.r.keys) + static_cast<size_t>(key_head) * a.chunks * (kChunkBytes / 4),
                static_cast<size_t>(a.chunks) * (kChunkBytes / 4)) {}
-  __device__ void put(float4 first, float4 second, unsigned lane, unsigned uniform) const {
-    const uint4 bits = make_uint4(pack_bf16(first.x, first.y), pack_bf16(first.z, first.w),
-                                  pack_bf16(second.x, second.y), pack_bf16(second.z, second.w));
-    memory.put4(__builtin_bit_cast(float4, bits), lane, uniform);
+  __device__ void put(const uint2 (&bits)[2], unsigned lane, unsigned uniform) const {
+    memory.put4(__builtin_bit_cast(float4, make_uint4(bits[0].x, bits[0].y, bits[1].x, bits[1].y)), lane, uniform);
   }
   __device__ bf16x8 get(unsigned lane, unsigned uniform) const {
     return __builtin_bit_cast(bf16x8, memory.get4(lane, uniform));
@@ -313,24 +311,56 @@ __device__ inline float fraction_of(float scale) {
 }
 __device__ inline float4 product(float4 a, float4 b) { return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); }
 
-// T, W, U, P and the gates of one chunk.  68 KiB of LDS, two workgroups a compute
-// unit.  The inverse is made by blocks: the four 16 x 16 diagonal blocks by forward
+// T, W, U, P and the gates of one chunk.  The inverse is made by blocks: the four 16 x 16 diagonal blocks by forward
 // substitution, one wave each, then -T22 A21 T11 twice on the matrix cores (a
 // substitution over all 64 rows by one wave held the other three up for a third of
 // the kernel).
-__global__ void __launch_bounds__(256)
-chunk_prepare_kernel(ChunkedArgs a) {
-  __shared__ __attribute__((aligned(16))) struct {
-    float k[kC][kWidePad];
-    union {
-      float q[kC][kWidePad];
-      struct {
-        float a[kC][kSquarePad], t[kC][kSquarePad];
-      };
+//
+// BF16: the activations are bf16, and the rows of K and Q are kept as such, each times the
+// power of two in its scale (KeyOperands), in row-major tiles of 16 KiB as in mfma_tile.h.  The
+// products of rows are then exact, those by T take three pieces of T and one of K or V, and
+// with 52 KiB of LDS and 168 registers three workgroups share a compute unit instead of two.
+// 2048 tokens of 48 heads 108.5 -> 80.6 us (350 MB, 67 us at the rate of a copy), one chunk 26 ->
+// 19: every product took the FP32 instruction, 34 us of it.
+template <bool BF16>
+struct PrepareSmem;
+template <>
+struct PrepareSmem<false> {
+  float k[kC][kWidePad];
+  union {
+    float q[kC][kWidePad];
+    struct {
+      float a[kC][kSquarePad], t[kC][kSquarePad];
     };
-    float g[kC], beta[kC], fk[kC];
-    float q_fraction[kC], k_fraction[kC], q_whole[kC], k_whole[kC];
-  } sm;
+  };
+  float g[kC], beta[kC], fk[kC];
+  __device__ float (&w())[kC][kWidePad] { return k; }
+};
+template <>
+struct PrepareSmem<true> {
+  unsigned char k_tile[kC * kD * 2];
+  union {
+    unsigned char q_tile[kC * kD * 2];
+    struct {
+      float a[kC][kSquarePad], t[kC][kSquarePad];
+    };
+    float w_rows[kC][kWidePad];
+  };
+  float g[kC], beta[kC], fk[kC], q_fraction[kC], k_fraction[kC];
+  __device__ float (&w())[kC][kWidePad] { return w_rows; }
+};
+// Place of a 16-byte piece of a row, of four rows of a column as a transpose read has them.
+__device__ inline int tile_piece(int row, int piece) { return (row * (kD / 8) + (piece ^ tile_swizzle(row))) * 16; }
+__device__ inline int tile_quad(int row, int column) { return tile_piece(row, column / 8) + column % 8 * 2; }
+__device__ inline float4 unpacked(uint2 bits) {
+  return make_float4(__uint_as_float(bits.x << 16), __uint_as_float(bits.x & 0xffff0000u),
+                     __uint_as_float(bits.y << 16), __uint_as_float(bits.y & 0xffff0000u));
+}
+
+template <bool BF16>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BF16 ? 3 : 2, BF16 ? 3 : 2)))
+chunk_prepare_kernel(ChunkedArgs a) {
+  __shared__ __attribute__((aligned(1024))) PrepareSmem<BF16> sm;
   const ChunkView v(a, blockIdx.x, blockIdx.y);
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -391,32 +421,40 @@ chunk_prepare_kernel(ChunkedArgs a) {
       const bool ok = i < v.tokens;
       const float iq = ok ? __shfl(inverse, 16 * quarter + 4 * g, 64) : 0.0f;
       const float ik = ok ? __shfl(inverse, 16 * quarter + 4 * g + 2, 64) : 0.0f;
+      const float q_scale = iq / norm_scale;
+      // a scale's power of two and its fraction in [1, 2); a zero has neither
+      const float q_fraction = q_scale == 0.0f ? 0.0f : fraction_of(q_scale);
+      const float k_fraction = ik == 0.0f ? 0.0f : fraction_of(ik);
+      const float q_power = __uint_as_float(__float_as_uint(q_scale) & 0x7f800000u);
+      const float k_power = __uint_as_float(__float_as_uint(ik) & 0x7f800000u);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const float(&qv)[4] = rows[2 * g][j], (&kv)[4] = rows[2 * g + 1][j];
-        store4(&sm.q[i][4 * n16 + 64 * j], make_float4(normed(qv[0] * iq), normed(qv[1] * iq), normed(qv[2] * iq),
-                                                       normed(qv[3] * iq)));
-        store4(&sm.k[i][4 * n16 + 64 * j], make_float4(kv[0] * ik, kv[1] * ik, kv[2] * ik, kv[3] * ik));
+        if constexpr (BF16) {
+          const int place = tile_quad(i, 4 * n16 + 64 * j);
+          *reinterpret_cast<uint2*>(sm.q_tile + place) = make_uint2(pack_bf16(qv[0] * q_power, qv[1] * q_power),
+                                                                    pack_bf16(qv[2] * q_power, qv[3] * q_power));
+          *reinterpret_cast<uint2*>(sm.k_tile + place) = make_uint2(pack_bf16(kv[0] * k_power, kv[1] * k_power),
+                                                                    pack_bf16(kv[2] * k_power, kv[3] * k_power));
+        } else {
+          store4(&sm.q[i][4 * n16 + 64 * j], make_float4(normed(qv[0] * iq), normed(qv[1] * iq), normed(qv[2] * iq),
+                                                         normed(qv[3] * iq)));
+          store4(&sm.k[i][4 * n16 + 64 * j], make_float4(kv[0] * ik, kv[1] * ik, kv[2] * ik, kv[3] * ik));
+        }
       }
       if (n16 == 0) {
-        const float q_scale = iq / norm_scale;
         gates[kQScale * kC + i] = q_scale;
         gates[kKScale * kC + i] = ik;
-        // a scale's fraction in [1, 2) (a zero stays one), and what takes it out of a row again
-        const float q_fraction = q_scale == 0.0f ? 0.0f : fraction_of(q_scale);
-        const float k_fraction = ik == 0.0f ? 0.0f : fraction_of(ik);
-        sm.q_fraction[i] = q_fraction, sm.k_fraction[i] = k_fraction;
-        sm.q_whole[i] = q_fraction == 0.0f ? 0.0f : 1.0f / q_fraction;
-        sm.k_whole[i] = k_fraction == 0.0f ? 0.0f : 1.0f / k_fraction;
+        if constexpr (BF16) sm.q_fraction[i] = q_fraction, sm.k_fraction[i] = k_fraction;
       }
     }
   }
   // gates (sequence_delta_net.cc:88-96); tokens beyond the sequence neither
   // decay nor write
-  float e = 0.0f, l = 0.0f;
+  float e = 0.0f, l = 0.0f, beta = 0.0f;
   if (wave == 0) {
     const int t = v.t0 + lane;
-    float g = 0.0f, beta = 0.0f;
+    float g = 0.0f;
     if (lane < v.tokens) {
       const float alpha =
           bf16_bits_to_float(a.a[static_cast<size_t>(t) * a.vh + v.head]) + a.dt_bias[v.head];
@@ -440,66 +478,117 @@ chunk_prepare_kernel(ChunkedArgs a) {
     gates[kL * kC + lane] = l;
     sm.g[lane] = g;
     sm.beta[lane] = beta;
-    sm.fk[lane] = beta * e;
+    if constexpr (!BF16) sm.fk[lane] = beta * e;
   }
   __syncthreads();
-  if (wave == 0) {
-    gates[kEQ * kC + lane] = e * sm.q_fraction[lane];
-    gates[kLK * kC + lane] = l * sm.k_fraction[lane];
-  }
+  if constexpr (BF16)
+    if (wave == 0) {
+      gates[kEQ * kC + lane] = e * sm.q_fraction[lane];
+      gates[kLK * kC + lane] = l * sm.k_fraction[lane];
+      sm.fk[lane] = beta * e * sm.k_fraction[lane];
+    }
   // k^ k^T and q^ k^T by 16 x 16 tiles on and below the diagonal: wave w takes row w of
   // the first and row 3 - w of the second, five tiles
   const bool first_of_group = v.head % (a.vh / a.kh) == 0;
+  const Record k_rows = v.key(a.r.k_rows);
   floatx4 kk[4], qk[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b) kk[b] = qk[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  const Record k_rows = v.key(a.r.k_rows), q_rows = v.key(a.r.q_rows);
-  const KeyOperands operands(a, v.key_head());
-  const unsigned operand_at = 16 * lane + blockIdx.x * KeyOperands::kChunkBytes;
-  float4 k_before, q_before;
-  const float k_whole = sm.k_whole[16 * wave + n16], q_whole = sm.q_whole[16 * (3 - wave) + n16];
+  if constexpr (BF16) {
+    auto row_operand = [&](const unsigned char* tile, int block, int s) {
+      return as_bf16x8(*reinterpret_cast<const uint4*>(tile + tile_piece(16 * block + n16, 4 * s + quarter)));
+    };
 #pragma unroll
-  for (int s = 0; s < kD / 16; ++s) {
-    const float4 kr = load4(&sm.k[16 * wave + n16][16 * s + 4 * quarter]);
-    const float4 qr = load4(&sm.q[16 * (3 - wave) + n16][16 * s + 4 * quarter]);
+    for (int s = 0; s < kD / 32; ++s) {
+      const bf16x8 kr = row_operand(sm.k_tile, wave, s), qr = row_operand(sm.q_tile, 3 - wave, s);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      if (b > wave && b > 3 - wave) continue;
-      const float4 kc = load4(&sm.k[16 * b + n16][16 * s + 4 * quarter]);
-      if (b <= wave) kk[b] = mma16(kk[b], kr, kc);
-      if (b <= 3 - wave) qk[b] = mma16(qk[b], qr, kc);
+      for (int b = 0; b < 4; ++b) {
+        if (b > wave && b > 3 - wave) continue;
+        const bf16x8 kc = row_operand(sm.k_tile, b, s);
+        if (b <= wave) kk[b] = mfma16(kr, kc, kk[b]);
+        if (b <= 3 - wave) qk[b] = mfma16(qr, kc, qk[b]);
+      }
     }
     if (first_of_group) {
-      k_rows.put4(kr, 16 * lane, piece_at<kD>(wave, 4 * s));
-      if (!a.round) {
-        q_rows.put4(qr, 16 * lane, piece_at<kD>(3 - wave, 4 * s));
-      } else if (s % 2 == 1) {
-        operands.put(scaled(k_before, k_whole), scaled(kr, k_whole), operand_at,
-                     KeyOperands::kRowsOfK + (4 * wave + s / 2) * 1024);
-        operands.put(scaled(q_before, q_whole), scaled(qr, q_whole), operand_at,
-                     KeyOperands::kRowsOfQ + (4 * (3 - wave) + s / 2) * 1024);
-      }
-      k_before = kr, q_before = qr;
-    }
-  }
-  if (first_of_group) {
-    const Record k_columns = v.key(a.r.k_columns), q_columns = v.key(a.r.q_columns);
+      const KeyOperands operands(a, v.key_head());
+      const unsigned operand_at = 16 * lane + blockIdx.x * KeyOperands::kChunkBytes;
+      const int row = 16 * wave + n16;
+      const float k_fraction = sm.k_fraction[row];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int s = 0; s < kD / 32; ++s) {
+        uint2 kr[2], qr[2];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int b = 2 * wave + t, row = 16 * s + 4 * quarter;
-        float4 kc = gather4(&sm.k[row][16 * b + n16], kWidePad), qc = gather4(&sm.q[row][16 * b + n16], kWidePad);
-        k_columns.put4(kc, 16 * lane, piece_at<kC>(b, 4 * s));
-        q_columns.put4(qc, 16 * lane, piece_at<kC>(b, 4 * s));
-        if (!a.round) continue;
-        kc = product(kc, load4(&sm.k_whole[row])), qc = product(qc, load4(&sm.q_whole[row]));
-        if (s % 2 == 1) {
-          operands.put(k_before, kc, operand_at, KeyOperands::kColumnsOfK + (2 * b + s / 2) * 1024);
-          operands.put(q_before, qc, operand_at, KeyOperands::kColumnsOfQ + (2 * b + s / 2) * 1024);
+        for (int half = 0; half < 2; ++half) {
+          const int place = tile_quad(row, 32 * s + 16 * half + 4 * quarter);
+          kr[half] = *reinterpret_cast<const uint2*>(sm.k_tile + place);
+          qr[half] = *reinterpret_cast<const uint2*>(sm.q_tile + place);
+          k_rows.put4(scaled(unpacked(kr[half]), k_fraction), 16 * lane, piece_at<kD>(wave, 8 * s + 4 * half));
         }
-        k_before = kc, q_before = qc;
+        operands.put(kr, operand_at, KeyOperands::kRowsOfK + (4 * wave + s) * 1024);
+        operands.put(qr, operand_at, KeyOperands::kRowsOfQ + (4 * wave + s) * 1024);
       }
+      const Record k_columns = v.key(a.r.k_columns), q_columns = v.key(a.r.q_columns);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int s = 0; s < kC / 32; ++s) {
+          const int b = 2 * wave + t;
+          uint2 kc[2], qc[2];
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            const int first = 32 * s + 16 * half + 4 * quarter;
+            const int place = tile_quad(first + n16 / 4, 16 * b + 4 * (n16 % 4));
+            kc[half] = lds_transpose_read(sm.k_tile, place);
+            qc[half] = lds_transpose_read(sm.q_tile, place);
+            k_columns.put4(product(unpacked(kc[half]), load4(&sm.k_fraction[first])), 16 * lane,
+                           piece_at<kC>(b, 8 * s + 4 * half));
+            q_columns.put4(product(unpacked(qc[half]), load4(&sm.q_fraction[first])), 16 * lane,
+                           piece_at<kC>(b, 8 * s + 4 * half));
+          }
+          operands.put(kc, operand_at, KeyOperands::kColumnsOfK + (2 * b + s) * 1024);
+          operands.put(qc, operand_at, KeyOperands::kColumnsOfQ + (2 * b + s) * 1024);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const float k_col = sm.k_fraction[16 * b + n16];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kk[b][e] *= sm.k_fraction[16 * wave + 4 * quarter + e] * k_col;
+        qk[b][e] *= sm.q_fraction[16 * (3 - wave) + 4 * quarter + e] * k_col;
+      }
+    }
+  } else {
+    const Record q_rows = v.key(a.r.q_rows);
+#pragma unroll
+    for (int s = 0; s < kD / 16; ++s) {
+      const float4 kr = load4(&sm.k[16 * wave + n16][16 * s + 4 * quarter]);
+      const float4 qr = load4(&sm.q[16 * (3 - wave) + n16][16 * s + 4 * quarter]);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        if (b > wave && b > 3 - wave) continue;
+        const float4 kc = load4(&sm.k[16 * b + n16][16 * s + 4 * quarter]);
+        if (b <= wave) kk[b] = mma16(kk[b], kr, kc);
+        if (b <= 3 - wave) qk[b] = mma16(qk[b], qr, kc);
+      }
+      if (first_of_group) {
+        k_rows.put4(kr, 16 * lane, piece_at<kD>(wave, 4 * s));
+        q_rows.put4(qr, 16 * lane, piece_at<kD>(3 - wave, 4 * s));
+      }
+    }
+    if (first_of_group) {
+      const Record k_columns = v.key(a.r.k_columns), q_columns = v.key(a.r.q_columns);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int b = 2 * wave + t;
+          k_columns.put4(gather4(&sm.k[16 * s + 4 * quarter][16 * b + n16], kWidePad), 16 * lane,
+                         piece_at<kC>(b, 4 * s));
+          q_columns.put4(gather4(&sm.q[16 * s + 4 * quarter][16 * b + n16], kWidePad), 16 * lane,
+                         piece_at<kC>(b, 4 * s));
+        }
+    }
   }
   lds_barrier();  // the rows of q^ make room for P, then A, and for T
   {
@@ -603,6 +692,14 @@ chunk_prepare_kernel(ChunkedArgs a) {
   }
   const Record w_columns = v.wide(a.r.w_columns), w_rows = v.wide(a.r.w_rows), u_columns = v.wide(a.r.u_columns);
   const unsigned column_at = piece_at<kC>(2 * wave, 0) + lane_piece<kC>(h, n);
+  bf16x8 value_rows[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const float4 first = values[2 * s], second = values[2 * s + 1];
+    value_rows[s] = as_bf16x8(make_uint4(pack_bf16(first.x, first.y), pack_bf16(first.z, first.w),
+                                         pack_bf16(second.x, second.y), pack_bf16(second.z, second.w)));
+  }
+  if constexpr (BF16) keep_order();
   floatx16 w[2];
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti) {
@@ -610,11 +707,27 @@ chunk_prepare_kernel(ChunkedArgs a) {
     w[ti] = zero_tile();
 #pragma unroll
     for (int s = 0; s < 4 * (ti + 1); ++s) {
+      if constexpr (BF16) {
+        if (s % 2 == 1) continue;
+        const int k = 8 * s + 4 * h;  // .. + 3 and eight further
+        const float4 t0 = load4(&sm.t[32 * ti + n][k]), t1 = load4(&sm.t[32 * ti + n][k + 8]);
+        const Pieces by_k = split_eight(product(t0, load4(&sm.fk[k])), product(t1, load4(&sm.fk[k + 8])));
+        const Pieces by_v = split_eight(product(t0, load4(&sm.beta[k])), product(t1, load4(&sm.beta[k + 8])));
+        const bf16x8 keys =
+            tile_transposed_operand<kD>(sm.k_tile + 8 * s * (kD * 2), tile_transpose_read<kD>(lane, wave), 0);
+#pragma unroll
+        for (int part = 2; part >= 0; --part) {
+          w[ti] = mfma32(by_k.part[part], keys, w[ti]);
+          u = mfma32(by_v.part[part], value_rows[s / 2], u);
+        }
+        continue;
+      }
       const int k = 8 * s + 4 * h;
-      const float4 t = load4(&sm.t[32 * ti + n][k]), f = load4(&sm.fk[k]), b = load4(&sm.beta[k]);
-      w[ti] = mma(w[ti], make_float4(t.x * f.x, t.y * f.y, t.z * f.z, t.w * f.w),
-                  gather4(&sm.k[k][col], kWidePad));
-      u = mma(u, make_float4(t.x * b.x, t.y * b.y, t.z * b.z, t.w * b.w), values[s]);
+      if constexpr (!BF16) {
+        const float4 t = load4(&sm.t[32 * ti + n][k]);
+        w[ti] = mma(w[ti], product(t, load4(&sm.fk[k])), gather4(&sm.k[k][col], kWidePad));
+        u = mma(u, product(t, load4(&sm.beta[k])), values[s]);
+      }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -623,15 +736,16 @@ chunk_prepare_kernel(ChunkedArgs a) {
       u_columns.put4(make_float4(u[4 * j], u[4 * j + 1], u[4 * j + 2], u[4 * j + 3]), column_at, at);
     }
   }
-  lds_barrier();  // the rows of k^ make room for W
+  lds_barrier();  // the rows of k^, or T, make room for W
+  auto& w_tile = sm.w();
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sm.k[32 * ti + tile_row(i, h)][col] = w[ti][i];
+    for (int i = 0; i < 16; ++i) w_tile[32 * ti + tile_row(i, h)][col] = w[ti][i];
   lds_barrier();
 #pragma unroll
   for (int s = 0; s < 8; ++s)
-    w_rows.put4(load4(&sm.k[16 * wave + n16][16 * s + 4 * quarter]), 16 * lane, piece_at<kD>(wave, 4 * s));
+    w_rows.put4(load4(&w_tile[16 * wave + n16][16 * s + 4 * quarter]), 16 * lane, piece_at<kD>(wave, 4 * s));
 }
 
 // ---------------------------------------------------------------------------
@@ -781,7 +895,6 @@ __device__ inline void touch_chunks(Made made, int first, int direction, int ste
 // and stores stand between the multiplications, each request for a register right
 // after the multiplication that read it, and none between a product and the barrier
 // that publishes it.  The fences keep that order.
-__device__ inline void keep_order() { __builtin_amdgcn_sched_barrier(0); }
 
 // Eight elements of a left operand as they come from memory: FP32 numbers that become three
 // pieces, or bf16.
@@ -1801,7 +1914,10 @@ size_t gdn_backward_chunked_bytes(const pluto_hip_delta_params* p, int length) {
 int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBackward& c) {
   const ChunkedArgs a = make_args(c);
   const dim3 per_chunk(a.chunks, a.vh);
-  chunk_prepare_kernel<<<per_chunk, 256, 0, stream>>>(a);
+  if (a.round)
+    chunk_prepare_kernel<true><<<per_chunk, 256, 0, stream>>>(a);
+  else
+    chunk_prepare_kernel<false><<<per_chunk, 256, 0, stream>>>(a);
   const int status = launch_status();
   if (status != 0) return status;
   by_tiles(a, [&](auto tiles, auto bf16) {
