@@ -97,7 +97,7 @@ int launch_gdn_output(hipStream_t stream, const void* core, int core_dtype, cons
 // partial per (token, value head), in the layout the token-by-token kernels use with
 // a single column tile, and the parameters' of the gates as one per (chunk, value head).
 struct GdnChunkedBackward {
-  const float* post = nullptr;   // [T, channels] convolved, activated q | k | v
+  const void* post = nullptr;      // [T, channels], bf16 with `round`, else FP32
   const uint16_t* a = nullptr;   // bf16 [T, vh]
   const uint16_t* b = nullptr;
   const float* a_log = nullptr;

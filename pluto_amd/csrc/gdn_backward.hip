@@ -23,6 +23,7 @@
 // row, added up by one thread per row).  What a token reads from global memory
 // is requested one token ahead.
 #include "gdn.h"
+#include "gdn_activation.h"
 #include "mfma_tile.h"
 
 namespace pluto_hip {
@@ -75,10 +76,11 @@ __device__ inline Pack<VEC> load_bf16s(const uint16_t* p) {
 }
 
 // One thread per VEC channels of a token (channels % VEC == 0).
-template <int VEC>
+// POST: float, or uint16_t for bf16 (then `round`).
+template <int VEC, class POST>
 __global__ void __launch_bounds__(256)
 conv_train_kernel(const uint16_t* input, const float* __restrict__ weight, int length,
-                  int channels, int kernel, bool round, float* pre, float* post) {
+                  int channels, int kernel, bool round, float* pre, POST* post) {
   const int groups = channels / VEC;
   const long long i = blockIdx.x * 256LL + threadIdx.x;
   if (i >= 1LL * length * groups) return;
@@ -100,7 +102,12 @@ conv_train_kernel(const uint16_t* input, const float* __restrict__ weight, int l
     activated.e[e] = round_if(sum.e[e] / (1.0f + expf(-sum.e[e])), round);
   }
   store_floats<VEC>(pre + 1LL * t * channels + c, sum);
-  store_floats<VEC>(post + 1LL * t * channels + c, activated);
+  if constexpr (sizeof(POST) == 4) {
+    store_floats<VEC>(post + 1LL * t * channels + c, activated);
+  } else {
+    static_assert(VEC == 1);
+    post[1LL * t * channels + c] = float_to_bf16_bits(activated.e[0]);
+  }
 }
 
 // ---- four taps ---------------------------------------------------------------
@@ -141,14 +148,14 @@ __device__ inline void read_taps(const float* weight, int c, float (&w)[VEC][4])
   }
 }
 
-// post = SiLU(conv(input)) as FP32, both rounded to bf16 on request.  (One channel
-// and one token a thread, four loads each, took 108 us at 2048 tokens of 10240
-// channels; in and out are 126 MB.)
+// post = SiLU(conv(input)) as FP32, both rounded to bf16 on request, or as bf16.  (One
+// channel and one token a thread, four loads each, took 108 us at 2048 tokens of 10240
+// channels.  Now 28.4 us as FP32, 126 MB in and out, 18.7 as bf16, 84 MB.)
 constexpr int kConvRun = 8;
-template <bool ALIGNED>
+template <bool ALIGNED, class POST>
 __global__ void __launch_bounds__(256)
 conv_train4_kernel(const uint16_t* __restrict__ input, const float* __restrict__ weight, int length,
-                   int channels, bool round, float* __restrict__ post) {
+                   int channels, bool round, POST* __restrict__ post) {
   constexpr int VEC = 4;
   const int c = (blockIdx.x * 256 + threadIdx.x) * VEC, t0 = blockIdx.y * kConvRun;
   if (c >= channels) return;
@@ -173,13 +180,20 @@ conv_train4_kernel(const uint16_t* __restrict__ input, const float* __restrict__
       float sum = 0.0f;
 #pragma unroll
       for (int tap = 0; tap < 4; ++tap) sum += x[tap][e] * w[e][tap];
-      sum = round_if(sum, round);
-      out[e] = round_if(sum / (1.0f + expf(-sum)), round);
+      if constexpr (sizeof(POST) == 4) {
+        sum = round_if(sum, round);
+        out[e] = round_if(sum / (1.0f + expf(-sum)), round);
+      } else {
+        out[e] = silu_of_bf16(round_to_bf16(sum));
+      }
       x[0][e] = x[1][e], x[1][e] = x[2][e], x[2][e] = x[3][e];
     }
-    if (t0 + r < length)
-      *reinterpret_cast<float4*>(post + 1LL * (t0 + r) * channels + c) =
-          make_float4(out[0], out[1], out[2], out[3]);
+    if (t0 + r >= length) continue;
+    POST* to = post + 1LL * (t0 + r) * channels + c;
+    if constexpr (sizeof(POST) == 4)
+      *reinterpret_cast<float4*>(to) = make_float4(out[0], out[1], out[2], out[3]);
+    else
+      *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16(out[0], out[1]), pack_bf16(out[2], out[3]));
   }
 }
 
@@ -1038,19 +1052,26 @@ int launch_gdn_backward(hipStream_t stream, const pluto_hip_delta_params* p, int
   const long long elements = 1LL * length * channels;
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   const bool rows_aligned = aligned(qkv) && aligned(conv_weight) && aligned(dqkv);
-  if (taps4) {
-    const dim3 grid((channels / 4 + 255) / 256, (length + kConvRun - 1) / kConvRun);
+  auto convolve = [&](auto* to) {
     const auto* input = static_cast<const uint16_t*>(qkv);
-    if (rows_aligned)
-      conv_train4_kernel<true><<<grid, 256, 0, stream>>>(input, conv_weight, length, channels, round, post);
-    else
-      conv_train4_kernel<false><<<grid, 256, 0, stream>>>(input, conv_weight, length, channels, round, post);
-  } else {
-    // one channel a thread: four (one wide access instead of four) were slower in the
-    // kernels for any number of taps that also read the weights
-    conv_train_kernel<1><<<blocks_for(elements), 256, 0, stream>>>(
-        static_cast<const uint16_t*>(qkv), conv_weight, length, channels, kernel, round, pre, post);
-  }
+    if (taps4) {
+      const dim3 grid((channels / 4 + 255) / 256, (length + kConvRun - 1) / kConvRun);
+      if (rows_aligned)
+        conv_train4_kernel<true><<<grid, 256, 0, stream>>>(input, conv_weight, length, channels, round, to);
+      else
+        conv_train4_kernel<false><<<grid, 256, 0, stream>>>(input, conv_weight, length, channels, round, to);
+    } else {
+      // one channel a thread: four (one wide access instead of four) were slower in the
+      // kernels for any number of taps that also read the weights
+      conv_train_kernel<1><<<blocks_for(elements), 256, 0, stream>>>(input, conv_weight, length, channels, kernel,
+                                                                     round, pre, to);
+    }
+  };
+  // the chunked kernels take what is rounded to bf16 as such
+  if (chunked && round)
+    convolve(reinterpret_cast<uint16_t*>(post));
+  else
+    convolve(post);
   int status = launch_status();
   if (status != 0) return status;
   RecurrenceArgs r;

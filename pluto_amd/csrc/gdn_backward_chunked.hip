@@ -88,7 +88,7 @@ constexpr size_t kRecordFloats = 5 * static_cast<size_t>(kWide) + 4 * kSquare + 
                                  2 * static_cast<size_t>(kState);
 
 struct ChunkedArgs {
-  const float* post = nullptr;     // [T, channels]
+  const void* post = nullptr;      // [T, channels], bf16 where they are rounded to it, else FP32
   const uint16_t* a = nullptr;     // bf16 [T, vh]
   const uint16_t* b = nullptr;
   const float* a_log = nullptr;
@@ -186,6 +186,11 @@ __device__ inline float half_sums(const float (&values)[16]) {
   return v[0] + __shfl_xor(v[0], 16, 64);
 }
 
+__device__ inline float4 unpacked(uint2 bits) {
+  return make_float4(__uint_as_float(bits.x << 16), __uint_as_float(bits.x & 0xffff0000u),
+                     __uint_as_float(bits.y << 16), __uint_as_float(bits.y & 0xffff0000u));
+}
+
 // Memory behind a buffer descriptor: a lane's byte offset, computed once, and a uniform
 // byte offset, so that a kernel keeps no addresses in vector registers.  Rows of
 // TOKENS may lie beyond the end: there the sum is the offset the descriptor checks,
@@ -215,6 +220,13 @@ struct Memory {
                              : __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane, uniform, 0);
     return __builtin_bit_cast(float4, bits);
   }
+  __device__ float4 get4_bf16(unsigned lane, unsigned uniform) const {
+    return unpacked(__builtin_bit_cast(uint2, get2(lane, uniform)));
+  }
+  __device__ uint32_t get_bf16(unsigned lane, unsigned uniform) const {
+    return static_cast<uint16_t>(TOKENS ? __builtin_amdgcn_raw_buffer_load_b16(rsrc, lane + uniform, 0, 0)
+                                        : __builtin_amdgcn_raw_buffer_load_b16(rsrc, lane, uniform, 0));
+  }
   // elements `stride` bytes apart
   __device__ float4 gather4(unsigned lane, unsigned uniform, unsigned stride) const {
     return make_float4(get(lane, uniform), get(lane, uniform + stride), get(lane, uniform + 2 * stride),
@@ -243,23 +255,28 @@ struct ChunkView {
   const ChunkedArgs& a;
   size_t rec;
   int t0, head, tokens, channels;
-  unsigned row_bytes, out_bytes;   // a token's row in the activations, in dO and O
+  unsigned post_bytes, row_bytes, out_bytes;  // a token's row in the activations, their gradients, and dO and O
   const float* gates;
   __device__ ChunkView(const ChunkedArgs& args, int chunk, int head_)
       : a(args), rec(static_cast<size_t>(head_) * args.chunks + chunk), t0(chunk * kC), head(head_),
         tokens(min(args.length - t0, kC)), channels(2 * args.kh * kD + args.vh * kD),
-        row_bytes(channels * 4), out_bytes(args.vh * kD * 4), gates(args.r.gates + rec * kGateRows * kC) {}
-  __device__ Tokens activations(const float* base, int column) const {
-    return Tokens(base + static_cast<size_t>(t0) * channels + column,
-                  static_cast<size_t>(tokens) * channels - column);
+        post_bytes(channels * (args.round ? 2 : 4)), row_bytes(channels * 4), out_bytes(args.vh * kD * 4), gates(args.r.gates + rec * kGateRows * kC) {}
+  __device__ Tokens activations(int column) const {
+    const int bytes = a.round ? 2 : 4;
+    return Tokens(reinterpret_cast<const float*>(static_cast<const char*>(a.post) +
+                                                 (static_cast<size_t>(t0) * channels + column) * bytes),
+                  (static_cast<size_t>(tokens) * channels - column) * bytes / 4);
   }
   __device__ int key_head() const { return head / (a.vh / a.kh); }
   __device__ int value_column() const { return (2 * a.kh + head) * kD; }
   __device__ Record key(const float* records) const {
     return Record(records + (static_cast<size_t>(key_head()) * a.chunks + t0 / kC) * kWide, kWide);
   }
-  __device__ Tokens v() const { return activations(a.post, value_column()); }
-  __device__ Tokens dv() const { return activations(a.dpost, value_column()); }
+  __device__ Tokens v() const { return activations(value_column()); }
+  __device__ Tokens dv() const {
+    return Tokens(a.dpost + static_cast<size_t>(t0) * channels + value_column(),
+                  static_cast<size_t>(tokens) * channels - value_column());
+  }
   __device__ Tokens heads(const float* base) const {  // O, dO
     return Tokens(base + (static_cast<size_t>(t0) * a.vh + head) * kD,
                   (static_cast<size_t>(tokens) * a.vh - head) * kD);
@@ -320,8 +337,9 @@ __device__ inline float4 product(float4 a, float4 b) { return make_float4(a.x * 
 // power of two in its scale (KeyOperands), in row-major tiles of 16 KiB as in mfma_tile.h.  The
 // products of rows are then exact, those by T take three pieces of T and one of K or V, and
 // with 52 KiB of LDS and 168 registers three workgroups share a compute unit instead of two.
-// 2048 tokens of 48 heads 108.5 -> 80.6 us (350 MB, 67 us at the rate of a copy), one chunk 26 ->
-// 19: every product took the FP32 instruction, 34 us of it.
+// 2048 tokens of 48 heads 108.5 -> 73 us (310 MB, 59 us at the rate of a copy; 80.6 while bf16
+// activations came as FP32), one chunk 26 -> 19: every product took the FP32 instruction, 34
+// us of it.
 template <bool BF16>
 struct PrepareSmem;
 template <>
@@ -352,10 +370,6 @@ struct PrepareSmem<true> {
 // Place of a 16-byte piece of a row, of four rows of a column as a transpose read has them.
 __device__ inline int tile_piece(int row, int piece) { return (row * (kD / 8) + (piece ^ tile_swizzle(row))) * 16; }
 __device__ inline int tile_quad(int row, int column) { return tile_piece(row, column / 8) + column % 8 * 2; }
-__device__ inline float4 unpacked(uint2 bits) {
-  return make_float4(__uint_as_float(bits.x << 16), __uint_as_float(bits.x & 0xffff0000u),
-                     __uint_as_float(bits.y << 16), __uint_as_float(bits.y & 0xffff0000u));
-}
 
 template <bool BF16>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BF16 ? 3 : 2, BF16 ? 3 : 2)))
@@ -375,15 +389,21 @@ chunk_prepare_kernel(ChunkedArgs a) {
   // eight rows share their steps.
   {
     const float norm_scale = sqrtf(static_cast<float>(kD)), inverse_norm_scale = 1.0f / norm_scale;
-    const Tokens q = v.activations(a.post, v.key_head() * kD),
-                 k = v.activations(a.post, (a.kh + v.key_head()) * kD);
-    const unsigned at = (16 * wave + quarter) * v.row_bytes + 16 * n16;
+    const Tokens q = v.activations(v.key_head() * kD), k = v.activations((a.kh + v.key_head()) * kD);
+    const unsigned at = (16 * wave + quarter) * v.post_bytes + (BF16 ? 8 : 16) * n16;
+    auto four = [&](const Tokens& from, unsigned uniform) {
+      if constexpr (BF16)
+        return from.get4_bf16(at, uniform);
+      else
+        return from.get4(at, uniform);
+    };
     float rows[8][2][4], squares[8][4];  // q^ and k^ of rows quarter, 4 + quarter, ...
 #pragma unroll
     for (int g = 0; g < 4; ++g)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const float4 qv = q.get4(at, 4 * g * v.row_bytes + 256 * j), kv = k.get4(at, 4 * g * v.row_bytes + 256 * j);
+        const unsigned uniform = 4 * g * v.post_bytes + (BF16 ? 128 : 256) * j;
+        const float4 qv = four(q, uniform), kv = four(k, uniform);
         rows[2 * g][j][0] = qv.x, rows[2 * g][j][1] = qv.y, rows[2 * g][j][2] = qv.z, rows[2 * g][j][3] = qv.w;
         rows[2 * g + 1][j][0] = kv.x, rows[2 * g + 1][j][1] = kv.y, rows[2 * g + 1][j][2] = kv.z,
         rows[2 * g + 1][j][3] = kv.w;
@@ -676,9 +696,17 @@ chunk_prepare_kernel(ChunkedArgs a) {
   const int col = 32 * wave + n;
   const auto value_memory = v.v();
   float4 values[8];
+  uint32_t value_bits[4][8];
+  if constexpr (BF16) {
+    const unsigned at = 4 * h * v.post_bytes + 2 * col;
 #pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    values[s] = value_memory.gather4(4 * h * v.row_bytes + 4 * col, 8 * s * v.row_bytes, v.row_bytes);
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) value_bits[s][e] = value_memory.get_bf16(at, (16 * s + 8 * (e / 4) + e % 4) * v.post_bytes);
+  } else {
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      values[s] = value_memory.gather4(4 * h * v.post_bytes + 4 * col, 8 * s * v.post_bytes, v.post_bytes);
   }
   __builtin_amdgcn_sched_barrier(0);
   lds_barrier();
@@ -693,13 +721,14 @@ chunk_prepare_kernel(ChunkedArgs a) {
   const Record w_columns = v.wide(a.r.w_columns), w_rows = v.wide(a.r.w_rows), u_columns = v.wide(a.r.u_columns);
   const unsigned column_at = piece_at<kC>(2 * wave, 0) + lane_piece<kC>(h, n);
   bf16x8 value_rows[4];
+  if constexpr (BF16) {
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const float4 first = values[2 * s], second = values[2 * s + 1];
-    value_rows[s] = as_bf16x8(make_uint4(pack_bf16(first.x, first.y), pack_bf16(first.z, first.w),
-                                         pack_bf16(second.x, second.y), pack_bf16(second.z, second.w)));
+    for (int s = 0; s < 4; ++s) {
+      auto pair = [&](int e) { return value_bits[s][e] | value_bits[s][e + 1] << 16; };
+      value_rows[s] = as_bf16x8(make_uint4(pair(0), pair(2), pair(4), pair(6)));
+    }
+    keep_order();
   }
-  if constexpr (BF16) keep_order();
   floatx16 w[2];
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti) {
@@ -1452,6 +1481,7 @@ struct GradientSmem {
 };
 enum RowSum { kSumQ, kSumK, kSumW, kSumV, kDotQ, kDotK };
 
+template <bool BF16>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 chunk_gradients_kernel(ChunkedArgs a) {
@@ -1498,10 +1528,13 @@ chunk_gradients_kernel(ChunkedArgs a) {
         make_rsrc(a.r.dl_rows + v.rec * kWide, kWide * 4), v.v().words()};
     const unsigned record_at = piece_at<kD>(wave, 0) + 16 * lane;
     const unsigned fill_at[4] = {record_at, (16 * wave + lane % 16) * v.out_bytes + lane / 16 * 16, record_at,
-                                 (16 * wave + lane % 16) * v.row_bytes + lane / 16 * 16};
+                                 (16 * wave + lane % 16) * v.post_bytes + lane / 16 * 16};
+    // (bf16 rows of V in one: eight columns a piece)
     auto fill = [&](int slab) {
+      if constexpr (BF16)
+        lds_fill<16>(sources[3], sm.slab[slab % 2][3] + 1024 * wave, fill_at[3] + slab * (kSlab * 2));
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
+      for (int m = 0; m < (BF16 ? 3 : 4); ++m)
 #pragma unroll
         for (int part = 0; part < 2; ++part) {
           const int quad = kSlab / 4 * slab + 4 * part;
@@ -1538,6 +1571,10 @@ chunk_gradients_kernel(ChunkedArgs a) {
       auto operand = [&](int m, int ti, int g) {
         return *reinterpret_cast<const float4*>(stage[m] + tile_row_at + piece_at<kSlab>(2 * ti, 2 * g));
       };
+      auto value_operand = [&](int ti, int g) {
+        if constexpr (!BF16) return operand(3, ti, g);
+        return unpacked(*reinterpret_cast<const uint2*>(stage[3] + 1024 * (2 * ti + n / 16) + 256 * g + n % 16 * 16 + 8 * h));
+      };
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         dot += (s0[g].x * s1[g].x + s0[g].y * s1[g].y) + (s0[g].z * s1[g].z + s0[g].w * s1[g].w);
@@ -1553,7 +1590,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
         keep_order();
         if (lower) {
           dp = mma(dp, operand(1, ti_own, g), operand(2, tj_own, g));
-          dt = mma(dt, operand(0, ti_own, g), scaled(operand(3, tj_own, g), fv));
+          dt = mma(dt, operand(0, ti_own, g), scaled(value_operand(tj_own, g), fv));
         }
         keep_order();
       }
@@ -1719,7 +1756,15 @@ chunk_gradients_kernel(ChunkedArgs a) {
     float products[16];
     float4 values[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) values[j] = v_memory.get4(token_at, (32 * ti + 8 * j) * v.row_bytes);
+    for (int j = 0; j < 4; ++j) {
+      const unsigned uniform = (32 * ti + 8 * j) * v.post_bytes;
+      if constexpr (BF16) {  // half of a row of gradients, unpacked where it is used
+        const float2 bits = v_memory.get2(token_at / 2, uniform);
+        values[j].x = bits.x, values[j].y = bits.y;
+      } else {
+        values[j] = v_memory.get4(token_at, uniform);
+      }
+    }
     keep_order();
     {
       floatx16 tu = zero_tile();
@@ -1728,6 +1773,7 @@ chunk_gradients_kernel(ChunkedArgs a) {
       keep_order();
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        if constexpr (BF16) values[j] = unpacked(make_uint2(__float_as_uint(values[j].x), __float_as_uint(values[j].y)));
         const float4 value = quad_transpose(values[j]), beta = rows4(sm.gate[kBeta], ti, j);
         products[4 * j] = tu[4 * j] * value.x, products[4 * j + 1] = tu[4 * j + 1] * value.y;
         products[4 * j + 2] = tu[4 * j + 2] * value.z, products[4 * j + 3] = tu[4 * j + 3] * value.w;
@@ -1933,7 +1979,10 @@ int launch_gdn_backward_chunked_reverse(hipStream_t stream, const GdnChunkedBack
   });
   const int status = launch_status();
   if (status != 0) return status;
-  chunk_gradients_kernel<<<dim3(a.chunks, a.vh), 256, 0, stream>>>(a);
+  if (a.round)
+    chunk_gradients_kernel<true><<<dim3(a.chunks, a.vh), 256, 0, stream>>>(a);
+  else
+    chunk_gradients_kernel<false><<<dim3(a.chunks, a.vh), 256, 0, stream>>>(a);
   return launch_status();
 }
 
