@@ -67,8 +67,8 @@ constexpr int kSquarePad = kC + 4;
 // Per (head, chunk) records in the workspace, in floats.
 struct Records {
   // of a key head                                                        [64][128]
-  float *q_rows, *q_columns, *k_rows, *k_columns;
-  uint16_t* keys;             // the four as bf16 operands, see KeyOperand
+  float *q_rows = nullptr, *q_columns = nullptr, *k_rows = nullptr, *k_columns = nullptr;
+  uint16_t* keys = nullptr;   // or, of bf16 activations, the four as KeyOperands has them
   float *w_rows, *w_columns;                          // W              [64][128]
   float *u_columns, *dl_rows, *ddl_rows;              // U, Dl, dDl     [64][128]
   float *p_rows, *p_columns;                          // P               [64][64]
@@ -83,7 +83,8 @@ struct Records {
 // kEQ and kLK: kE and kL times the factors that the bf16 rows of Q and K lack.
 enum Gate { kG, kBeta, kQScale, kKScale, kE, kL, kEQ, kLK, kGateRows };
 
-constexpr size_t kKeyRecordFloats = 6 * static_cast<size_t>(kWide);
+// FP32: q and k, rows and columns; bf16: KeyOperands.
+constexpr size_t key_record_floats(bool bf16) { return (bf16 ? 2 : 4) * static_cast<size_t>(kWide); }
 constexpr size_t kRecordFloats = 5 * static_cast<size_t>(kWide) + 4 * kSquare + kGateRows * kC +
                                  2 * static_cast<size_t>(kState);
 
@@ -260,7 +261,8 @@ struct ChunkView {
   __device__ ChunkView(const ChunkedArgs& args, int chunk, int head_)
       : a(args), rec(static_cast<size_t>(head_) * args.chunks + chunk), t0(chunk * kC), head(head_),
         tokens(min(args.length - t0, kC)), channels(2 * args.kh * kD + args.vh * kD),
-        post_bytes(channels * (args.round ? 2 : 4)), row_bytes(channels * 4), out_bytes(args.vh * kD * 4), gates(args.r.gates + rec * kGateRows * kC) {}
+        post_bytes(channels * (args.round ? 2 : 4)), row_bytes(channels * 4), out_bytes(args.vh * kD * 4),
+        gates(args.r.gates + rec * kGateRows * kC) {}
   __device__ Tokens activations(int column) const {
     const int bytes = a.round ? 2 : 4;
     return Tokens(reinterpret_cast<const float*>(static_cast<const char*>(a.post) +
@@ -337,9 +339,9 @@ __device__ inline float4 product(float4 a, float4 b) { return make_float4(a.x * 
 // power of two in its scale (KeyOperands), in row-major tiles of 16 KiB as in mfma_tile.h.  The
 // products of rows are then exact, those by T take three pieces of T and one of K or V, and
 // with 52 KiB of LDS and 168 registers three workgroups share a compute unit instead of two.
-// 2048 tokens of 48 heads 108.5 -> 73 us (310 MB, 59 us at the rate of a copy; 80.6 while bf16
-// activations came as FP32), one chunk 26 -> 19: every product took the FP32 instruction, 34
-// us of it.
+// 2048 tokens of 48 heads 108.5 -> 64 us (260 MB, 50 us at the rate of a copy; 80.6 while bf16
+// activations came as FP32 and these rows left as FP32 as well), one chunk 26 -> 18: every
+// product took the FP32 instruction, 34 us of it.
 template <bool BF16>
 struct PrepareSmem;
 template <>
@@ -510,7 +512,6 @@ chunk_prepare_kernel(ChunkedArgs a) {
   // k^ k^T and q^ k^T by 16 x 16 tiles on and below the diagonal: wave w takes row w of
   // the first and row 3 - w of the second, five tiles
   const bool first_of_group = v.head % (a.vh / a.kh) == 0;
-  const Record k_rows = v.key(a.r.k_rows);
   floatx4 kk[4], qk[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b) kk[b] = qk[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -533,7 +534,6 @@ chunk_prepare_kernel(ChunkedArgs a) {
       const KeyOperands operands(a, v.key_head());
       const unsigned operand_at = 16 * lane + blockIdx.x * KeyOperands::kChunkBytes;
       const int row = 16 * wave + n16;
-      const float k_fraction = sm.k_fraction[row];
 #pragma unroll
       for (int s = 0; s < kD / 32; ++s) {
         uint2 kr[2], qr[2];
@@ -542,12 +542,10 @@ chunk_prepare_kernel(ChunkedArgs a) {
           const int place = tile_quad(row, 32 * s + 16 * half + 4 * quarter);
           kr[half] = *reinterpret_cast<const uint2*>(sm.k_tile + place);
           qr[half] = *reinterpret_cast<const uint2*>(sm.q_tile + place);
-          k_rows.put4(scaled(unpacked(kr[half]), k_fraction), 16 * lane, piece_at<kD>(wave, 8 * s + 4 * half));
         }
         operands.put(kr, operand_at, KeyOperands::kRowsOfK + (4 * wave + s) * 1024);
         operands.put(qr, operand_at, KeyOperands::kRowsOfQ + (4 * wave + s) * 1024);
       }
-      const Record k_columns = v.key(a.r.k_columns), q_columns = v.key(a.r.q_columns);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -560,10 +558,6 @@ chunk_prepare_kernel(ChunkedArgs a) {
             const int place = tile_quad(first + n16 / 4, 16 * b + 4 * (n16 % 4));
             kc[half] = lds_transpose_read(sm.k_tile, place);
             qc[half] = lds_transpose_read(sm.q_tile, place);
-            k_columns.put4(product(unpacked(kc[half]), load4(&sm.k_fraction[first])), 16 * lane,
-                           piece_at<kC>(b, 8 * s + 4 * half));
-            q_columns.put4(product(unpacked(qc[half]), load4(&sm.q_fraction[first])), 16 * lane,
-                           piece_at<kC>(b, 8 * s + 4 * half));
           }
           operands.put(kc, operand_at, KeyOperands::kColumnsOfK + (2 * b + s) * 1024);
           operands.put(qc, operand_at, KeyOperands::kColumnsOfQ + (2 * b + s) * 1024);
@@ -579,7 +573,7 @@ chunk_prepare_kernel(ChunkedArgs a) {
       }
     }
   } else {
-    const Record q_rows = v.key(a.r.q_rows);
+    const Record k_rows = v.key(a.r.k_rows), q_rows = v.key(a.r.q_rows);
 #pragma unroll
     for (int s = 0; s < kD / 16; ++s) {
       const float4 kr = load4(&sm.k[16 * wave + n16][16 * s + 4 * quarter]);
@@ -702,7 +696,8 @@ chunk_prepare_kernel(ChunkedArgs a) {
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) value_bits[s][e] = value_memory.get_bf16(at, (16 * s + 8 * (e / 4) + e % 4) * v.post_bytes);
+      for (int e = 0; e < 8; ++e)
+        value_bits[s][e] = value_memory.get_bf16(at, (16 * s + 8 * (e / 4) + e % 4) * v.post_bytes);
   } else {
 #pragma unroll
     for (int s = 0; s < 8; ++s)
@@ -853,6 +848,11 @@ __device__ inline Pieces state_pieces(const floatx4& first, const floatx4& secon
 #pragma unroll
   for (int i = 0; i < 3; ++i) p.part[i] = as_bf16x8(make_uint4(words[i][0], words[i][1], words[i][2], words[i][3]));
   return p;
+}
+// Eight elements of any size.
+__device__ inline Pieces pieces_of_any(float4 a, float4 b) {
+  const floatx4 first = {a.x, a.y, a.z, a.w}, second = {b.x, b.y, b.z, b.w};
+  return state_pieces(first, second);
 }
 __device__ inline float4 as_float4(const floatx4& v) { return make_float4(v[0], v[1], v[2], v[3]); }
 
@@ -1459,12 +1459,18 @@ chunk_states_backward_kernel(ChunkedArgs a) {
 //      dv = diag(beta) T^T dDl;  dq and dk back through the normalisations
 //   4. d log-decay and d beta from row and column sums of the above, through the gates
 //      to da, db and the contribution to d A_log
-// 75 KiB of LDS and 256 registers, none of them spilled: two workgroups a compute unit.  2048
+// 78 KiB of LDS and 250 registers, none of them spilled: two workgroups a compute unit.  2048
 // tokens of 48 heads 267 -> 226 us when 45 registers no longer went to scratch (140 MB there
 // and back): the contributions of U before those of W, one product's accumulator at a time,
 // and a sum whose factors the compiler kept for its end.  dDl and T are read here in the one
 // order they are kept in and exchanged between lanes (230 us; the kernels that write them 137
 // -> 129 and 106 -> 103).
+// BF16: the products with rows of K and Q take three pieces and one (KeyOperands), their
+// fractions go with the other factor or, in sums over a row's channels, with the sum: 232 ->
+// 220 us, and the preparation, which no longer writes these rows as FP32, 73 -> 64.  What
+// multiplies them may be as large as FP32 holds (split_right; 3 us).  The other products stay
+// with the FP32 instruction: those with the states on pieces made by every wave took as long,
+// the vector instructions for them being as many as the matrix instructions saved.
 constexpr int kSlab = 32;
 constexpr unsigned kSlabBytes = kC * kSlab * 4;
 struct GradientSmem {
@@ -1492,7 +1498,15 @@ chunk_gradients_kernel(ChunkedArgs a) {
   const int h = lane / 32, n = lane % 32, col = 32 * wave + n;
   const int ti_own = wave / 2, tj_own = wave % 2;   // the [64, 64] tile
   const bool lower = ti_own >= tj_own;
-  for (int i = tid; i < kGateRows * kC; i += 256) sm.gate[i / kC][i % kC] = v.gates[i];
+  for (int i = tid; i < kGateRows * kC; i += 256) {
+    const int row = i / kC;
+    if (!BF16 || row < kEQ) {
+      sm.gate[row][i % kC] = v.gates[i];
+    } else {  // what the bf16 rows of Q and K lack
+      const float scale = v.gates[(row == kEQ ? kQScale : kKScale) * kC + i % kC];
+      sm.gate[row][i % kC] = scale == 0.0f ? 0.0f : fraction_of(scale);
+    }
+  }
   if (tid < kC) {
     sm.row_n[tid][0] = sm.row_n[tid][1] = sm.col_n[tid][0] = sm.col_n[tid][1] = 0.0f;
     sm.row_p[tid][0] = sm.row_p[tid][1] = sm.col_p[tid][0] = sm.col_p[tid][1] = 0.0f;
@@ -1514,6 +1528,29 @@ chunk_gradients_kernel(ChunkedArgs a) {
   // the four of a register quad, columns 4 (n / 4) .. + 3 of the wave's
   const unsigned token_row = 4 * h + n % 4, token_column = 4 * (32 * wave + n / 4 * 4);
   const unsigned token_at = token_row * v.row_bytes + token_column;
+  // Four tokens of a column or columns of a token of K or Q, as they are kept.  bf16: of
+  // quad s of a row of operand blocks, a lane's place and a uniform one.
+  using KeyQuad = std::conditional_t<BF16, uint2, float4>;
+  auto numbers = [](KeyQuad quad) {
+    if constexpr (BF16) {
+      asm volatile("" : "+v"(quad.x), "+v"(quad.y));  // unpacked at each use: the numbers take twice the registers
+      return unpacked(quad);
+    } else {
+      return quad;
+    }
+  };
+  const KeyOperands operands(a, v.key_head());
+  const unsigned key_lane = blockIdx.x * KeyOperands::kChunkBytes + (16 * h + n % 16) * 16;
+  auto key_quad = [&](unsigned lane_at, unsigned first, int quad) {
+    const unsigned place = first + quad / 4 * 1024 + quad % 2 * 512 + quad % 4 / 2 * 8;
+    return __builtin_bit_cast(uint2, operands.memory.get2(lane_at, place));
+  };
+  auto as_operand = [](uint2 first, uint2 second) { return as_bf16x8(make_uint4(first.x, first.y, second.x, second.y)); };
+  auto mma_exact = [](floatx16 acc, const Pieces& left, bf16x8 right) {
+#pragma unroll
+    for (int part = 2; part >= 0; --part) acc = mfma32(left.part[part], right, acc);
+    return acc;
+  };
   // row tile t of a per-row quantity in LDS, rows of register quad j
   auto rows4 = [&](const float* rows, int t, int j) { return load4(rows + 32 * t + 8 * j + 4 * h); };
   auto element = [](const float4& four, int i) {
@@ -1573,7 +1610,8 @@ chunk_gradients_kernel(ChunkedArgs a) {
       };
       auto value_operand = [&](int ti, int g) {
         if constexpr (!BF16) return operand(3, ti, g);
-        return unpacked(*reinterpret_cast<const uint2*>(stage[3] + 1024 * (2 * ti + n / 16) + 256 * g + n % 16 * 16 + 8 * h));
+        const int place = 1024 * (2 * ti + n / 16) + 256 * g + n % 16 * 16 + 8 * h;
+        return unpacked(*reinterpret_cast<const uint2*>(stage[3] + place));
       };
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
@@ -1607,15 +1645,23 @@ chunk_gradients_kernel(ChunkedArgs a) {
   // Everything the [64, 64] part reads is requested a step before it is used.
   // (Descriptors of what is read or written are made where that is: all at once they do not
   // fit in the scalar registers and go to scratch.)
-  float4 p_tile[4], k_own[kD / 8];
+  float4 p_tile[4];
+  KeyQuad k_own[kD / 8];
   if (lower) {
-    const Record p_memory = v.square(a.r.p_columns), k_rows = v.key(a.r.k_rows);
+    const Record p_memory = v.square(a.r.p_columns);
 #pragma unroll
     for (int j = 0; j < 4; ++j) p_tile[j] = p_memory.get4(tile_at, piece_at<kC>(0, 2 * j));
     keep_order();
-    const unsigned k_at = piece_at<kD>(2 * tj_own, 0) + lane_piece<kD>(h, n);
+    if constexpr (BF16) {
 #pragma unroll
-    for (int s = 0; s < kD / 8; ++s) k_own[s] = k_rows.get4(k_at, piece_at<kD>(0, 2 * s));
+      for (int s = 0; s < kD / 8; ++s)
+        k_own[s] = key_quad(key_lane + n / 16 * 4096, KeyOperands::kRowsOfK + 2 * tj_own * 4096, s);
+    } else {
+      const Record k_rows = v.key(a.r.k_rows);
+      const unsigned k_at = piece_at<kD>(2 * tj_own, 0) + lane_piece<kD>(h, n);
+#pragma unroll
+      for (int s = 0; s < kD / 8; ++s) k_own[s] = k_rows.get4(k_at, piece_at<kD>(0, 2 * s));
+    }
   }
   keep_order();
   // row and column sums of a tile held in an accumulator, for its rows and columns
@@ -1656,18 +1702,37 @@ chunk_gradients_kernel(ChunkedArgs a) {
   lds_barrier();
   if (lower) {
     const float fk = sm.gate[kBeta][tile_col] * sm.gate[kE][tile_col];
+    if constexpr (BF16) {
+      floatx16 by_k = zero_tile();
 #pragma unroll
-    for (int s = 0; s < kD / 8; ++s)
-      dt = mma(dt, load4(&sm.dw[32 * ti_own + n][8 * s + 4 * h]), scaled(k_own[s], fk));
+      for (int s = 0; s < kD / 8; s += 2) {
+        const float* row = &sm.dw[32 * ti_own + n][8 * s + 4 * h];
+        by_k = mma_exact(by_k, pieces_of_any(load4(row), load4(row + 8)), as_operand(k_own[s], k_own[s + 1]));
+      }
+      const float factor = fk * sm.gate[kLK][tile_col];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dt[i] = fmaf(factor, by_k[i], dt[i]);
+    } else {
+#pragma unroll
+      for (int s = 0; s < kD / 8; ++s)
+        dt = mma(dt, load4(&sm.dw[32 * ti_own + n][8 * s + 4 * h]), scaled(k_own[s], fk));
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) sm.x[32 * ti_own + tile_row(i, h)][tile_col] = dt[i];
   }
   keep_order();
   // columns of K^ and Q^, both as operands and in the accumulators' rows
-  float4 kc[8], qc[8], kkd_tile[4];
-  const Record k_memory = v.key(a.r.k_columns);
+  KeyQuad kc[8], qc[8];
+  float4 kkd_tile[4];
+  const unsigned key_columns = key_lane + n / 16 * 2048;
+  if constexpr (BF16) {
 #pragma unroll
-  for (int s = 0; s < 8; ++s) kc[s] = k_memory.get4(column_at, piece_at<kC>(0, 2 * s));
+    for (int s = 0; s < 8; ++s) kc[s] = key_quad(key_columns, KeyOperands::kColumnsOfK + 2 * wave * 2048, s);
+  } else {
+    const Record k_memory = v.key(a.r.k_columns);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) kc[s] = k_memory.get4(column_at, piece_at<kC>(0, 2 * s));
+  }
   keep_order();
   lds_barrier();
   floatx16 z = zero_tile();
@@ -1685,9 +1750,14 @@ chunk_gradients_kernel(ChunkedArgs a) {
     for (int j = 0; j < 4; ++j) kkd_tile[j] = kkd.get4(tile_at, piece_at<kC>(0, 2 * j));
   }
   keep_order();
-  const Record q_memory = v.key(a.r.q_columns);
+  if constexpr (BF16) {
 #pragma unroll
-  for (int s = 0; s < 8; ++s) qc[s] = q_memory.get4(column_at, piece_at<kC>(0, 2 * s));
+    for (int s = 0; s < 8; ++s) qc[s] = key_quad(key_columns, KeyOperands::kColumnsOfQ + 2 * wave * 2048, s);
+  } else {
+    const Record q_memory = v.key(a.r.q_columns);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) qc[s] = q_memory.get4(column_at, piece_at<kC>(0, 2 * s));
+  }
   keep_order();
   lds_barrier();
   if (lower) {
@@ -1725,9 +1795,13 @@ chunk_gradients_kernel(ChunkedArgs a) {
 #pragma unroll
   for (int s = 0; s < 8; ++s) dd[s] = ddl.get4(quad_at, piece_at<kD>(s / 2, 8 * wave) + 128 * (s % 2));
   keep_order();
+  // over the columns of products with rows of V, K or Q, which with bf16 lack their fraction
   auto row_sums = [&](RowSum which, int ti, const float (&values)[16]) {
     const float sum = half_sums(values);
-    if (n < 16) sm.parts[which][32 * ti + tile_row(n, h)][wave] = sum;
+    const int row = 32 * ti + tile_row(n % 16, h);
+    const bool query = which == kSumQ || which == kDotQ;
+    const float factor = !BF16 || which == kSumV ? 1.0f : sm.gate[query ? kEQ : kLK][row];
+    if (n < 16) sm.parts[which][row][wave] = sum * factor;
   };
 #pragma unroll
   for (int ti = 0; ti < 2; ++ti) {
@@ -1735,13 +1809,13 @@ chunk_gradients_kernel(ChunkedArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       dq[ti][i] *= element(rows4(sm.gate[kE], ti, i / 4), i);
-      products[i] = dq[ti][i] * element(qc[4 * ti + i / 4], i);
+      products[i] = dq[ti][i] * element(numbers(qc[4 * ti + i / 4]), i);
     }
     row_sums(kSumQ, ti, products);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       dk[ti][i] *= element(rows4(sm.gate[kL], ti, i / 4), i);
-      products[i] = dk[ti][i] * element(kc[4 * ti + i / 4], i);
+      products[i] = dk[ti][i] * element(numbers(kc[4 * ti + i / 4]), i);
     }
     row_sums(kSumK, ti, products);
   }
@@ -1797,25 +1871,44 @@ chunk_gradients_kernel(ChunkedArgs a) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float e = element(rows4(sm.gate[kE], ti, i / 4), i);
-        products[i] = tw[i] * element(kc[4 * ti + i / 4], i) * e;
+        products[i] = tw[i] * element(numbers(kc[4 * ti + i / 4]), i) * e;
         dk[ti][i] += element(rows4(sm.gate[kBeta], ti, i / 4), i) * e * tw[i];
       }
       row_sums(kSumW, ti, products);
     }
     keep_order();
+    if constexpr (BF16) {
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int k = 8 * s + 4 * h;
-      if (s < 4 * (ti + 1)) dq[ti] = mma(dq[ti], load4(&sm.pd[m][k]), kc[s]);
-      dk[ti] = mma(dk[ti], load4(&sm.x[m][k]), kc[s]);
-      if (s >= 4 * ti) dk[ti] = mma(dk[ti], gather4(&sm.pd[k][m], kSquarePad), qc[s]);
+      for (int s = 0; s < 8; s += 2) {
+        const int k = 8 * s + 4 * h;  // .. + 3 and eight further
+        const float4 k0 = load4(&sm.gate[kLK][k]), k1 = load4(&sm.gate[kLK][k + 8]);
+        const bf16x8 key = as_operand(kc[s], kc[s + 1]);
+        const float *pd = &sm.pd[m][k], *x = &sm.x[m][k];
+        if (s < 4 * (ti + 1))
+          dq[ti] = mma_exact(dq[ti], pieces_of_any(product(load4(pd), k0), product(load4(pd + 8), k1)), key);
+        dk[ti] = mma_exact(dk[ti], pieces_of_any(product(load4(x), k0), product(load4(x + 8), k1)), key);
+        if (s >= 4 * ti) {
+          const float4 q0 = load4(&sm.gate[kEQ][k]), q1 = load4(&sm.gate[kEQ][k + 8]);
+          const Pieces left = pieces_of_any(product(gather4(&sm.pd[k][m], kSquarePad), q0),
+                                            product(gather4(&sm.pd[k + 8][m], kSquarePad), q1));
+          dk[ti] = mma_exact(dk[ti], left, as_operand(qc[s], qc[s + 1]));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        const int k = 8 * s + 4 * h;
+        if (s < 4 * (ti + 1)) dq[ti] = mma(dq[ti], load4(&sm.pd[m][k]), kc[s]);
+        dk[ti] = mma(dk[ti], load4(&sm.x[m][k]), kc[s]);
+        if (s >= 4 * ti) dk[ti] = mma(dk[ti], gather4(&sm.pd[k][m], kSquarePad), qc[s]);
+      }
     }
     keep_order();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) products[i] = dq[ti][i] * element(qc[4 * ti + i / 4], i);
+    for (int i = 0; i < 16; ++i) products[i] = dq[ti][i] * element(numbers(qc[4 * ti + i / 4]), i);
     row_sums(kDotQ, ti, products);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) products[i] = dk[ti][i] * element(kc[4 * ti + i / 4], i);
+    for (int i = 0; i < 16; ++i) products[i] = dk[ti][i] * element(numbers(kc[4 * ti + i / 4]), i);
     row_sums(kDotK, ti, products);
     keep_order();
   }
@@ -1834,9 +1927,13 @@ chunk_gradients_kernel(ChunkedArgs a) {
   for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float4 q = qc[4 * ti + j], k = kc[4 * ti + j], q_dot = rows4(sm.dots[0], ti, j),
-                   k_dot = rows4(sm.dots[1], ti, j), q_scale = rows4(sm.gate[kQScale], ti, j),
+      const float4 q = numbers(qc[4 * ti + j]), k = numbers(kc[4 * ti + j]), q_scale = rows4(sm.gate[kQScale], ti, j),
                    k_scale = rows4(sm.gate[kKScale], ti, j);
+      float4 q_dot = rows4(sm.dots[0], ti, j), k_dot = rows4(sm.dots[1], ti, j);
+      if constexpr (BF16) {
+        q_dot = product(q_dot, rows4(sm.gate[kEQ], ti, j));
+        k_dot = product(k_dot, rows4(sm.gate[kLK], ti, j));
+      }
       float from_q[4], from_k[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -1926,11 +2023,14 @@ ChunkedArgs make_args(const GdnChunkedBackward& c) {
   a.r.s0 = take(kState);
   a.r.ds1 = take(kState);
   const size_t keys = static_cast<size_t>(a.chunks) * a.kh * kWide;
-  a.r.q_rows = at;
-  a.r.q_columns = at + keys;
-  a.r.k_rows = at + 2 * keys;
-  a.r.k_columns = at + 3 * keys;
-  a.r.keys = reinterpret_cast<uint16_t*>(at + 4 * keys);
+  if (a.round) {
+    a.r.keys = reinterpret_cast<uint16_t*>(at);
+  } else {
+    a.r.q_rows = at;
+    a.r.q_columns = at + keys;
+    a.r.k_rows = at + 2 * keys;
+    a.r.k_columns = at + 3 * keys;
+  }
   return a;
 }
 
@@ -1953,8 +2053,8 @@ bool gdn_backward_chunked_supported(const pluto_hip_delta_params* p) {
 
 size_t gdn_backward_chunked_bytes(const pluto_hip_delta_params* p, int length) {
   const size_t chunks = (static_cast<size_t>(length) + kC - 1) / kC;
-  return align_up(chunks * (p->value_heads * kRecordFloats + p->key_heads * kKeyRecordFloats) * sizeof(float),
-                  256);
+  const size_t keys = p->key_heads * key_record_floats(p->round_to_bfloat16 != 0);
+  return align_up(chunks * (p->value_heads * kRecordFloats + keys) * sizeof(float), 256);
 }
 
 int launch_gdn_backward_chunked_forward(hipStream_t stream, const GdnChunkedBackward& c) {

@@ -398,3 +398,33 @@ def test_rows_of_any_scale(capi, T, kh, vh):
         diff = np.abs(a - b)
         assert np.all(diff <= 2e-2 * scale), name
         assert np.mean(diff > 2e-4 * scale) <= 2e-2, name
+
+
+def test_largest_bf16_values_stay_finite(capi):
+    """The largest bf16 number among activations that are bf16, written to the state as it is:
+    the pieces of what it becomes (U, the states, their gradients' products with K and Q)
+    must not leave the range where the numbers do not.  Tolerances as for rows of any scale."""
+    T, kh, vh = 200, 1, 2
+    c = make_case(T, kh, vh, 128, 128, 4, seed=3)
+    channel = 2 * kh * 128 + 5
+    c["conv"][channel] = [0, 0, 0, 1]
+    c["qkv"][0, :, channel] = 0
+    c["qkv"][0, 100, channel] = 2.0 ** 128 - 2.0 ** 120
+    c["b"][0, 100, 0] = 60
+    c["a_log"][:], c["dt_bias"][:] = 0, -3
+    p = capi.delta_params(kh, vh, 128, 128, 4)
+    bf = torch.bfloat16
+    args = (p, dev(c["qkv"], bf), dev(c["z"], bf), dev(c["a"], bf), dev(c["b"], bf), dev(c["conv"]),
+            dev(c["a_log"]), dev(c["dt_bias"]), dev(c["norm"]), dev(c["dy"]))
+    got = capi.gdn_layer_backward(*args)
+    assert capi.last_path() == capi.PATH_CHUNKED
+    with capi.force_generic():
+        want = capi.gdn_layer_backward(*args)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dqkv", "dz", "da", "db"), got, want):
+        a, b = a.double().cpu().numpy(), b.double().cpu().numpy()
+        assert np.isfinite(b).all() and np.isfinite(a).all(), name
+        scale = np.abs(b) + np.sqrt(np.mean(b ** 2))
+        diff = np.abs(a - b)
+        assert np.all(diff <= 2e-2 * scale), name
+        assert np.mean(diff > 2e-4 * scale) <= 2e-2, name
