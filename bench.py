@@ -60,9 +60,9 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E (published)
 # kept as profiles/*_hbm_traffic.md.  None = not measured.
 MEASURED_TRAFFIC_BYTES = {
     # (workload, kernel group): (bytes read + written, commit the counters were read at)
-    ("mha_train_bf16", "flash_forward_kernel<64>"): (99.1e6 + 26.7e6, "4bff185"),
-    ("mha_train_bf16", "flash_dq_kernel"): (179.6e6 + 77.1e6, "4bff185"),
-    ("mha_train_bf16", "flash_dkv_kernel"): (154.5e6 + 100.7e6, "4bff185"),
+    ("mha_train_bf16", "flash_forward_kernel<64>"): (98.9e6 + 26.7e6, "2d9752b"),
+    ("mha_train_bf16", "flash_dq_kernel"): (179.5e6 + 77.1e6, "2d9752b"),
+    ("mha_train_bf16", "flash_dkv_kernel"): (155.2e6 + 100.7e6, "2d9752b"),
     ("gqa_prefill", "flash_forward_pipelined_kernel<128>"): (184.6e6 + 88.1e6, "4bff185"),
     ("gqa_prefill_d256", "flash_forward_pipelined_kernel<256>"): (444.9e6 + 100.9e6, "4bff185"),
     ("gqa_decode", "decode_fused_kernel<128,6>"): (1044.9e6 + 13.0e6, "4bff185"),
@@ -191,7 +191,7 @@ def gqa_prefill(torch, capi, d=128):
 
     work = 4.0 * qh * d * causal_pairs(T)
     return dict(step=step,
-                kernels=[("rope table + prepare", step, capi.AUXILIARY_KERNELS, None),
+                kernels=[("prepare", step, capi.AUXILIARY_KERNELS, None),
                          ("flash_forward_pipelined_kernel<%d>" % d, step,
                           capi.MAIN_KERNEL | capi.EIGHT_WAVE | capi.FROM_LENGTH, work)],
                 work=work,
