@@ -747,11 +747,15 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
   }
 
   // ---- combine: blocks in ascending order, kCombineChunk at a time --------
-  // A wave computes the weights of its heads with one block a lane; the partial
-  // outputs are requested kAhead blocks at a time, the first of them before the
-  // weights are known, two channels an access.  (With one channel an access, eight
-  // blocks at a time, and the weights summed by one thread a head, a block cost
-  // 0.36 us here: 11 us of a 36 us step at 32 blocks.)
+  // A wave computes weights with one block a lane.  Where the 128 channels that a
+  // wave adds up in one access are one head's (the wider heads), it computes that
+  // head's and reads a block's weight from its lane: no LDS, no barriers (before ->
+  // after, a step of one sequence of 3000 rows at 24/4 heads of 256: 50.4 -> 49.5 us,
+  // 777 rows 44.2 -> 43.9).  At 64 channels a wave spans two heads, so the weights go
+  // through the LDS.  The partial outputs are requested kAhead blocks at a time, the
+  // first of them before the weights are known, two channels an access.  (With one
+  // channel an access, eight blocks at a time, and the weights summed by one thread a
+  // head, a block cost 0.36 us here: 11 us of a 36 us step at 32 blocks.)
   float* chunk_w = shared_area;                            // [kCombineChunk][GROUP] weights
   float* head_state = shared_area + kCombineChunk * GROUP;  // [3][GROUP]: max, normalizer, rescale
   static_assert((kCombineChunk * GROUP + 3 * GROUP) * 4 <= value_area_bytes<D>());
@@ -772,7 +776,11 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
       logits[u][e] = a.io_dtype == PLUTO_HIP_BF16 ? static_cast<const uint16_t*>(a.q_gate)[at + e]
                                                   : static_cast<const uint32_t*>(a.q_gate)[at + e];
   }
-  if (tid < GROUP) {
+  constexpr bool kOwnHeads = D % 128 == 0;  // 128 channels of a wave are one head's
+  float own_max[kPairs], own_sum[kPairs];
+#pragma unroll
+  for (int u = 0; u < kPairs; ++u) own_max[u] = kMasked, own_sum[u] = 0.0f;
+  if (!kOwnHeads && tid < GROUP) {
     head_state[0 * GROUP + tid] = kMasked;  // running maximum
     head_state[1 * GROUP + tid] = 0.0f;     // running normalizer
   }
@@ -782,8 +790,8 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
     auto request = [&](int jj) {
 #pragma unroll
       for (int step = 0; step < kAhead; ++step) {
-        const int block_j = min(jj + step, count - 1);
-        const float* base = a.part_o + (first_slot + (j0 + block_j) * slot_step) * GROUP * D;
+        if (jj + step >= count) continue;
+        const float* base = a.part_o + (first_slot + (j0 + jj + step) * slot_step) * GROUP * D;
 #pragma unroll
         for (int u = 0; u < kPairs; ++u) {
           const int i = 2 * (tid + u * kThreads);
@@ -792,40 +800,62 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
       }
     };
     request(0);
-    float maxima[(GROUP + 3) / 4], sums[(GROUP + 3) / 4];
+    float weights[kPairs];
+    if constexpr (kOwnHeads) {
+      float maxima[kPairs], sums[kPairs];
 #pragma unroll
-    for (int v = 0; v < (GROUP + 3) / 4; ++v) {
-      const long long at = (first_slot + (j0 + min(ctx.lane, count - 1)) * slot_step) * GROUP +
-                           min(ctx.wave + 4 * v, GROUP - 1);
-      maxima[v] = load_shared(&a.part_m[at]), sums[v] = load_shared(&a.part_l[at]);
-    }
-    __syncthreads();  // the chunk before has been added up, and the states written
-#pragma unroll
-    for (int v = 0; v < (GROUP + 3) / 4; ++v) {
-      const int hh = ctx.wave + 4 * v;
-      if (hh >= GROUP) continue;
-      const float block_max = maxima[v], block_sum = sums[v];
-      const float old_max = head_state[0 * GROUP + hh], old_sum = head_state[1 * GROUP + hh];
-      const float maximum = fmaxf(old_max, max_over_wave(block_max));
-      const float weight =
-          ctx.lane < count ? __builtin_amdgcn_exp2f(block_max - maximum) : 0.0f;
-      const float sum = wave_sum(block_sum * weight);
-      const float rescale = __builtin_amdgcn_exp2f(old_max - maximum);
-      chunk_w[ctx.lane * GROUP + hh] = weight;
-      if (ctx.lane == 0) {
-        head_state[0 * GROUP + hh] = maximum;
-        head_state[1 * GROUP + hh] = old_sum * rescale + sum;
-        head_state[2 * GROUP + hh] = rescale;
+      for (int u = 0; u < kPairs; ++u) {
+        const int hh = min(2 * (64 * ctx.wave + u * kThreads) / D, GROUP - 1);
+        const long long at = (first_slot + (j0 + min(ctx.lane, count - 1)) * slot_step) * GROUP + hh;
+        maxima[u] = load_shared(&a.part_m[at]), sums[u] = load_shared(&a.part_l[at]);
       }
-    }
-    __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kPairs; ++u) {
-      const int i = 2 * (tid + u * kThreads);
-      if (i >= GROUP * D) continue;
-      const float rescale = head_state[2 * GROUP + i / D];
-      o[u].x *= rescale;
-      o[u].y *= rescale;
+      for (int u = 0; u < kPairs; ++u) {
+        const float maximum = fmaxf(own_max[u], max_over_wave(maxima[u]));
+        weights[u] = ctx.lane < count ? __builtin_amdgcn_exp2f(maxima[u] - maximum) : 0.0f;
+        const float sum = wave_sum(sums[u] * weights[u]);
+        const float rescale = __builtin_amdgcn_exp2f(own_max[u] - maximum);
+        own_max[u] = maximum;
+        own_sum[u] = own_sum[u] * rescale + sum;
+        o[u].x *= rescale;
+        o[u].y *= rescale;
+      }
+    } else {
+      float maxima[(GROUP + 3) / 4], sums[(GROUP + 3) / 4];
+#pragma unroll
+      for (int v = 0; v < (GROUP + 3) / 4; ++v) {
+        const long long at = (first_slot + (j0 + min(ctx.lane, count - 1)) * slot_step) * GROUP +
+                             min(ctx.wave + 4 * v, GROUP - 1);
+        maxima[v] = load_shared(&a.part_m[at]), sums[v] = load_shared(&a.part_l[at]);
+      }
+      __syncthreads();  // the chunk before has been added up, and the states written
+#pragma unroll
+      for (int v = 0; v < (GROUP + 3) / 4; ++v) {
+        const int hh = ctx.wave + 4 * v;
+        if (hh >= GROUP) continue;
+        const float block_max = maxima[v], block_sum = sums[v];
+        const float old_max = head_state[0 * GROUP + hh], old_sum = head_state[1 * GROUP + hh];
+        const float maximum = fmaxf(old_max, max_over_wave(block_max));
+        const float weight =
+            ctx.lane < count ? __builtin_amdgcn_exp2f(block_max - maximum) : 0.0f;
+        const float sum = wave_sum(block_sum * weight);
+        const float rescale = __builtin_amdgcn_exp2f(old_max - maximum);
+        chunk_w[ctx.lane * GROUP + hh] = weight;
+        if (ctx.lane == 0) {
+          head_state[0 * GROUP + hh] = maximum;
+          head_state[1 * GROUP + hh] = old_sum * rescale + sum;
+          head_state[2 * GROUP + hh] = rescale;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u) {
+        const int i = 2 * (tid + u * kThreads);
+        if (i >= GROUP * D) continue;
+        const float rescale = head_state[2 * GROUP + i / D];
+        o[u].x *= rescale;
+        o[u].y *= rescale;
+      }
     }
     for (int jj = 0; jj < count; jj += kAhead) {
       if (jj > 0) request(jj);
@@ -836,7 +866,9 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
         for (int u = 0; u < kPairs; ++u) {
           const int i = 2 * (tid + u * kThreads);
           if (i >= GROUP * D) continue;
-          const float weight = chunk_w[(jj + step) * GROUP + i / D];
+          const float weight =
+              kOwnHeads ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weights[u]), jj + step))
+                        : chunk_w[(jj + step) * GROUP + i / D];
           o[u].x += part[step][u].x * weight;
           o[u].y += part[step][u].y * weight;
         }
@@ -850,7 +882,8 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
     if (i >= GROUP * D) continue;
     const int hh = i / D, c = i % D;
     const long long at = static_cast<long long>(seq) * a.query_heads + g * GROUP + hh;
-    const float core[2] = {o[u].x / head_state[1 * GROUP + hh], o[u].y / head_state[1 * GROUP + hh]};
+    const float normalizer = kOwnHeads ? own_sum[u] : head_state[1 * GROUP + hh];
+    const float core[2] = {o[u].x / normalizer, o[u].y / normalizer};
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const float logit = __uint_as_float(a.io_dtype == PLUTO_HIP_BF16 ? logits[u][e] << 16 : logits[u][e]);

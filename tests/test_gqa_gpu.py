@@ -537,6 +537,35 @@ def test_decode_block_size_chosen_by_the_library(capi, d, batch):
         assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-4), length
 
 
+@pytest.mark.parametrize("d,qh,kh", [(256, 12, 2), (256, 1, 1), (128, 6, 2), (128, 16, 2), (64, 12, 2)])
+def test_decode_combine_of_few_and_many_blocks(capi, d, qh, kh):
+    """Blocks of 64 rows: 1, both sides of what is requested at once (8 and 16) and of
+    the 64 whose weights are computed together, and twice that; the largest score in the
+    first, in a middle and in the last block.  Within two bf16 ulps of the core of what
+    blocks of 512 rows give (the two add up in different orders)."""
+    rows = 129 * 64
+    p = capi.attention_params(qh, kh, d, 32, capacity=rows)
+    gen = torch.Generator(device="cuda").manual_seed(d + qh)
+    bf = torch.bfloat16
+    def values(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(bf)
+    q_gate, k, v = values(1, qh, 2, d), values(1, kh, d), values(1, kh, d)
+    w = torch.zeros(d, device="cuda")
+    cache = capi.KvCache(rows, kh, d)
+    keys = values(kh, rows, d)
+    cache.values.copy_(values(kh, rows, d))
+    for blocks in (1, 7, 8, 9, 15, 16, 17, 63, 64, 65, 128, 129):
+        for large in (0, blocks // 2, blocks - 1):
+            cache.keys.copy_(keys)
+            cache.keys[:, 64 * large:64 * large + 3] *= 4
+            length = 64 * blocks - 1
+            got = capi.gqa_decode(p, q_gate, k, v, w, w, [cache], positions=[length - 1], split_tokens=64,
+                                  advance=False).float()
+            want = capi.gqa_decode(p, q_gate, k, v, w, w, [cache], positions=[length - 1], split_tokens=512,
+                                   advance=False).float()
+            assert torch.all((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-4), (blocks, large)
+
+
 @pytest.mark.parametrize("d,rows,start", [(256, 34, 7336), (128, 61, 4000)])
 def test_prefill_without_room_for_parts(capi, d, rows, start):
     """A workspace that ends before the partial results is accepted: the call does not
