@@ -65,7 +65,7 @@ MEASURED_TRAFFIC_BYTES = {
     ("mha_train_bf16", "flash_dkv_kernel"): (155.2e6 + 100.7e6, "2d9752b"),
     ("gqa_prefill", "flash_forward_pipelined_kernel<128>"): (184.6e6 + 88.1e6, "4bff185"),
     ("gqa_prefill_d256", "flash_forward_pipelined_kernel<256>"): (444.9e6 + 100.9e6, "4bff185"),
-    ("gqa_decode", "decode_fused_kernel<128,6>"): (1044.9e6 + 13.0e6, "4bff185"),
+    ("gqa_decode", "decode_fused_kernel<128,6>"): (1044.9e6 + 13.0e6, "0b92232"),
     ("gdn_scan", "gdn_chunk_scan"): (528.7e6 + 145.1e6, "4bff185"),
 }
 
