@@ -144,7 +144,8 @@ flash_dq_kernel(FlashBackwardArgs a) {
       // path 64 cycles a load, four times as much as whole rows, and the workgroups of a
       // one-round grid all load at once.  The bf16 copy of dO leaves from the rows.
       // 16 sequences of 1024, 12 heads: 68.8 -> 65.8 us; 4 of 256: 15.4 -> 14.2.
-      // Rows beyond the sequence read as zero and are not stored.
+      // Rows beyond the sequence read as zero and are not stored: a row's whole offset is in
+      // the lane's, which is what the descriptor checks.
       int own = lane;
       asm volatile("" : "+v"(own));  // addresses of this part only: none is kept over the loop
       const int quad = own % 16, chunk = own % 8, own_n = own % 32, own_h = own / 32;
@@ -164,12 +165,12 @@ flash_dq_kernel(FlashBackwardArgs a) {
       uint32x2 o[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        g[i] = __builtin_amdgcn_raw_buffer_load_b128(g_rows, at, i * (16 * E), 0);
-        o[i] = __builtin_amdgcn_raw_buffer_load_b64(o_rows, at / 2, i * (8 * E), 0);
+        g[i] = __builtin_amdgcn_raw_buffer_load_b128(g_rows, at + i * (16 * E), 0, 0);
+        o[i] = __builtin_amdgcn_raw_buffer_load_b64(o_rows, at / 2 + i * (8 * E), 0, 0);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        q[i] = __builtin_amdgcn_raw_buffer_load_b128(q_rows, q_at, i * (16 * static_cast<int>(q_stride)), 0);
+        q[i] = __builtin_amdgcn_raw_buffer_load_b128(q_rows, q_at + i * (16 * static_cast<int>(q_stride)), 0, 0);
       // delta of attention.cc:283-291 (uses the stored, rounded output)
       float delta[8];
 #pragma unroll
@@ -181,7 +182,7 @@ flash_dq_kernel(FlashBackwardArgs a) {
                    (z * __uint_as_float(o[i][1] << 16) + w * __uint_as_float(o[i][1] & 0xffff0000u));
         const uint32x2 bits = {pack_bf16(x, y), pack_bf16(z, w)};
         reinterpret_cast<uint32x2*>(copy_area)[(local * KCH + ((quad / 2) ^ (local & 7))) * 2 + quad % 2] = bits;
-        __builtin_amdgcn_raw_buffer_store_b64(bits, gb_rows, at / 2, i * (8 * E), 0);
+        __builtin_amdgcn_raw_buffer_store_b64(bits, gb_rows, at / 2 + i * (8 * E), 0, 0);
       }
       // a wave's accesses to LDS are carried out in order: the compiler only has to keep it
       asm volatile("" ::: "memory");

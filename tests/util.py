@@ -101,3 +101,43 @@ def assert_close_bf16_gradient(actual, expected, what, outliers=2e-3, far=10.0):
     at 9.03 times the per-element bound (dK 4.4, dV 4.4; every call prints its
     own figure).  Max-norm and L2 bounds are the same 2e-2."""
     assert_close_bf16(actual, expected, what, outliers=outliers, far=far)
+
+
+class GuardedBuffers:
+    """Stands in for torch where `pluto_amd.capi` allocates, and places inputs: every buffer
+    lies between bytes that no call may write, behind inputs and in fresh buffers are bytes
+    that are no number in any of the types used (0xff), so that what is read there and counts
+    shows in the results."""
+    PAD = 1 << 20
+
+    def __init__(self, torch):
+        self.torch, self.buffers = torch, []
+
+    def __getattr__(self, name):
+        return getattr(self.torch, name)
+
+    def empty(self, *shape, dtype=None, device="cuda"):
+        shape = shape[0] if len(shape) == 1 and not isinstance(shape[0], int) else shape
+        dtype = dtype or self.torch.float32
+        size = int(np.prod(shape)) * dtype.itemsize
+        raw = self.torch.full((size + 2 * self.PAD,), 0xA5, dtype=self.torch.uint8, device=device)
+        self.buffers.append((raw, size, 0xA5))
+        raw[self.PAD:self.PAD + size] = 0xFF
+        return raw[self.PAD:self.PAD + size].view(dtype).reshape(shape)
+
+    def empty_like(self, tensor):
+        return self.empty(tuple(tensor.shape), dtype=tensor.dtype, device=tensor.device)
+
+    def place(self, tensor):
+        """A copy of an input."""
+        copy = self.empty_like(tensor)
+        raw, size, _ = self.buffers.pop()
+        raw.fill_(0xFF)
+        self.buffers.append((raw, size, 0xFF))
+        return copy.copy_(tensor)
+
+    def assert_intact(self, what):
+        for i, (raw, size, byte) in enumerate(self.buffers):
+            for side, part in (("before", raw[:self.PAD]), ("behind", raw[self.PAD + size:])):
+                touched = int((part != byte).sum())
+                assert touched == 0, "%s: %d bytes %s buffer %d of %d bytes written" % (what, touched, side, i, size)
