@@ -417,7 +417,7 @@ template <int IO, bool CONV>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 step128_kernel(StepArgs a) {
-  __shared__ float rows[2][2][128];    // k and q, element r of row block i at 16 r + i
+  __shared__ __attribute__((aligned(16))) float rows[2][2][128];  // k and q, element r of row block i at 16 r + i
   __shared__ __attribute__((aligned(16))) float values[2][128];  // CONV: v
   __shared__ float parts[2][4];
   const int tid = threadIdx.x, lane = tid % 64, r = lane / 8;
