@@ -428,12 +428,14 @@ def test_every_activation_rounds_as_the_scalar_kernel_rounds_it(capi):
     assert torch.equal(wide[0], narrow[0]) and torch.equal(wide[1], narrow[1])
 
 
+@pytest.mark.parametrize("kh,vh,d", [(8, 24, 64), (16, 48, 128)])
 @pytest.mark.parametrize("T", [1, 3, 4, 5, 15, 17, 70])
-def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T):
-    """The convolution walks sixteen rows a thread where there are enough of them and
-    four otherwise: the batch takes the one, its sequences alone the other.
-    Bit for bit the same, at row counts around either walk."""
-    kh, vh, kd, vd = 16, 48, 128, 128
+def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T, kh, vh, d):
+    """Bit for bit the same.  With heads of 64 the convolution is a pass of its own, which walks
+    sixteen rows a thread where there are enough of them and four otherwise: the batch takes
+    the one, its sequences alone the other, at row counts around either walk.  With heads
+    of 128 the preparation of the chunks convolves, in one way for any batch."""
+    kd = vd = d
     channels = 2 * kh * kd + vh * vd
     B = (1 << 23) // (T * channels) + 1
     p = capi.delta_params(kh, vh, kd, vd)
@@ -444,6 +446,7 @@ def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T):
     weights = tuple(dev(w) for w in layer_weights(kh, vh, kd, vd, 4))
     state = torch.zeros((B, vh, kd, vd), device="cuda")
     got = capi.gdn_layer_forward(p, qkv, z, a, b, *weights, state)
+    assert capi.last_path() == (capi.PATH_CHUNKED if d == 128 else capi.PATH_RECURRENCE)
     for i in sorted({0, 1, B - 1} & set(range(B))):
         one = torch.zeros((1, vh, kd, vd), device="cuda")
         want = capi.gdn_layer_forward(p, qkv[i:i + 1], z[i:i + 1], a[i:i + 1], b[i:i + 1], *weights, one)
