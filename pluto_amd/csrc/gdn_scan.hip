@@ -1130,6 +1130,15 @@ bool gdn_chunked_supported(const GdnArgs& a, int chunk) {
          aligned(a.q) && aligned(a.k) && aligned(a.v) && aligned(a.workspace);
 }
 
+// While every head of a chunk gets a compute unit of its own, three heads of one key head are
+// prepared faster by a workgroup each, though each convolves the rows of K and Q: the one
+// workgroup's 12 waves share a compute unit while others idle.  The whole forward of 16/48 heads,
+// three a workgroup and one: 17 tokens 29.2 and 25.6 us, 320 (240 heads of chunks) 39.7 and
+// 37.4, 400 (336) 45.2 and 44.4, 700 (528) 51.2 and 55.9, 8191 348 and 377; of 4/12 heads 1400
+// (264) 59.0 and 58.0, 2000 (384) 68.8 and 69.4.  (17 tokens took 27.0 with the convolution and
+// the gates as passes of their own.)
+constexpr unsigned kAlonePreparations = 256;
+
 bool gdn_layer_rows_supported(const GdnLayerInputs& layer, int taps) {
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
   return taps == 4 && aligned(layer.qkv) && aligned(layer.conv_weight);
@@ -1144,7 +1153,7 @@ int launch_gdn_chunked(hipStream_t stream, const GdnArgs& a, const GdnLayerInput
     const unsigned blocks = static_cast<unsigned>(heads * chunks);
     if (layer == nullptr)
       gdn_chunk_prepare<1, false><<<blocks, 256, 0, stream>>>(a, {});
-    else if (group % 3 == 0)
+    else if (group % 3 == 0 && blocks > kAlonePreparations)
       gdn_chunk_prepare<3, true><<<blocks / 3, 768, 0, stream>>>(a, *layer);
     else if (group % 2 == 0)
       gdn_chunk_prepare<2, true><<<blocks / 2, 512, 0, stream>>>(a, *layer);

@@ -434,7 +434,8 @@ def test_layer_forward_of_a_batch_is_the_forward_of_each_sequence(capi, T, kh, v
     """Bit for bit the same.  With heads of 64 the convolution is a pass of its own, which walks
     sixteen rows a thread where there are enough of them and four otherwise: the batch takes
     the one, its sequences alone the other, at row counts around either walk.  With heads
-    of 128 the preparation of the chunks convolves, in one way for any batch."""
+    of 128 the preparation of the chunks convolves, for three heads a workgroup in the
+    batch and for one a workgroup in its sequences alone."""
     kd = vd = d
     channels = 2 * kh * kd + vh * vd
     B = (1 << 23) // (T * channels) + 1
@@ -461,7 +462,8 @@ def test_preparation_that_convolves_on_the_way(capi, kh, vh, T):
     convolution as a pass of its own, which weights off a 16-byte boundary take: the rows
     are the same, their norms and the solve are summed in another order, so that a value
     may fall the other way of a bf16 rounding and move by 2^-8 of itself."""
-    B, d = 2, 128
+    # more than 256 heads of chunks where three can share a workgroup: fewer have one each
+    B, d = 48 if vh // kh % 3 == 0 else 2, 128
     channels = 2 * kh * d + vh * d
     p = capi.delta_params(kh, vh, d, d)
     gen = torch.Generator(device="cuda").manual_seed(100 * T + vh)
