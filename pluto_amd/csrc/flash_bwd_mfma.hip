@@ -161,6 +161,8 @@ flash_dq_kernel(FlashBackwardArgs a) {
       const auto gb_rows = rows_of(gb_base + static_cast<long long>(first) * E, 2LL * E, 2 * D);
       const uint32_t at = own / 16 * (4u * E) + 16 * quad;
       const uint32_t q_at = own / 8 * (2u * static_cast<uint32_t>(q_stride)) + 16 * chunk;
+      // requested with the rows: behind the orderings below they would be waited for by themselves
+      const float normalizer = a.normalizers[stats_base + q_load], maximum = a.maxima[stats_base + q_load];
       uint32x4 g[8], q[4];
       uint32x2 o[8];
 #pragma unroll
@@ -213,9 +215,7 @@ flash_dq_kernel(FlashBackwardArgs a) {
       }
       asm volatile("" ::: "memory");
       row_delta = reinterpret_cast<const float*>(copy_area)[n];
-      const float normalizer = a.normalizers[stats_base + q_load];
-      row_lse2 = a.maxima[stats_base + q_load] * kLog2e +
-                             __log2f(normalizer > 0.0f ? normalizer : 1.0f);
+      row_lse2 = maximum * kLog2e + __log2f(normalizer > 0.0f ? normalizer : 1.0f);
       if (h == 0 && q_row < T) {
         // the key-owned kernel starts its accumulators from these
         a.deltas[stats_base + q_row] = -row_delta;
