@@ -116,7 +116,7 @@ class GuardedBuffers:
     def __getattr__(self, name):
         return getattr(self.torch, name)
 
-    def empty(self, *shape, dtype=None, device="cuda"):
+    def empty(self, *shape, dtype=None, device=None):
         shape = shape[0] if len(shape) == 1 and not isinstance(shape[0], int) else shape
         dtype = dtype or self.torch.float32
         size = int(np.prod(shape)) * dtype.itemsize
