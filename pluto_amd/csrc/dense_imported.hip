@@ -1132,6 +1132,13 @@ imported_tile_fp8_kernel(TileManyArgs m, int passes) {
 // 72.1, 37.2 -> 32.8.  FP8 6144 -> 5120 (160 tiles of 32 rows, 256 of 20), 11 tokens 11.9 -> 10.6
 // us, 32 13.6 -> 12.5.  FP8 tiles of 16 rows are bound by their conversions as much as by their
 // bytes (5120 -> 16480 in tiles of 13, 11 tokens 21.1 -> 20.7, 32 23.4 -> 24.4): they stay whole.
+// Fewer than 256 whole tiles become tiles of few rows on all compute units.  The tokens, which
+// each loads then, come from the L2 and at the same time; whole and so, 9 / 16 / 32 tokens: bf16
+// 5120 -> 256 12.7 / 14.4 / 18.0 and 6.6 / 8.2 / 12.9 us (1 row), 768 13.0 / 14.7 / 18.5 and 8.0 /
+// 9.4 / 14.1 (3), 1024 13.1 / 14.8 / 18.6 and 8.5 / 10.1 / 14.6 (4), 768 -> 768 4.1 / 4.1 / 4.7 and
+// 3.1 / 3.2 / 3.9; FP8 5120 -> 1024 13.6 / 14.3 / 17.0 and 9.3 / 9.8 / 12.6 (4), 768 -> 768 6.3 / 6.4
+// / 6.7 and 5.2 / 5.3 / 5.8.  Fewer rows still make second tiles: 5120 -> 1024 bf16 in tiles of 2
+// 9.3 / 10.8 / 24.6.
 long long tiles_of(int matrices, const int* rows, int tile_rows) {
   long long tiles = 0;
   for (int i = 0; i < matrices; ++i) tiles += (rows[i] + tile_rows - 1) / tile_rows;

@@ -750,8 +750,9 @@ decode_fused_kernel(DecodeArgs a, DecodeBatch batch) {
   // A wave computes weights with one block a lane.  Where the 128 channels that a
   // wave adds up in one access are one head's (the wider heads), it computes that
   // head's and reads a block's weight from its lane: no LDS, no barriers (before ->
-  // after, a step of one sequence of 3000 rows at 24/4 heads of 256: 50.4 -> 49.5 us,
-  // 777 rows 44.2 -> 43.9).  At 64 channels a wave spans two heads, so the weights go
+  // after, a step of one sequence at 24/4 heads of 256 with its projections, replayed from a
+  // graph: 32000 rows 68.7 -> 66.8 us, 3000 50.8 -> 50.1, 777 44.8 -> 44.2; called one by one the
+  // last two do not show).  At 64 channels a wave spans two heads, so the weights go
   // through the LDS.  The partial outputs are requested kAhead blocks at a time, the
   // first of them before the weights are known, two channels an access.  (With one
   // channel an access, eight blocks at a time, and the weights summed by one thread a
