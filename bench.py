@@ -60,13 +60,13 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E (published)
 # kept as profiles/*_hbm_traffic.md.  None = not measured.
 MEASURED_TRAFFIC_BYTES = {
     # (workload, kernel group): (bytes read + written, commit the counters were read at)
-    ("mha_train_bf16", "flash_forward_kernel<64>"): (98.9e6 + 26.7e6, "2d9752b"),
-    ("mha_train_bf16", "flash_dq_kernel"): (179.5e6 + 77.1e6, "2d9752b"),
-    ("mha_train_bf16", "flash_dkv_kernel"): (155.2e6 + 100.7e6, "2d9752b"),
-    ("gqa_prefill", "flash_forward_pipelined_kernel<128>"): (184.6e6 + 88.1e6, "4bff185"),
-    ("gqa_prefill_d256", "flash_forward_pipelined_kernel<256>"): (444.9e6 + 100.9e6, "4bff185"),
-    ("gqa_decode", "decode_fused_kernel<128,6>"): (1044.9e6 + 13.0e6, "0b92232"),
-    ("gdn_scan", "gdn_chunk_scan"): (528.7e6 + 145.1e6, "4bff185"),
+    ("mha_train_bf16", "flash_forward_kernel<64>"): (99.0e6 + 26.7e6, "c19a8f3"),
+    ("mha_train_bf16", "flash_dq_kernel"): (179.7e6 + 77.1e6, "c19a8f3"),
+    ("mha_train_bf16", "flash_dkv_kernel"): (155.1e6 + 100.7e6, "c19a8f3"),
+    ("gqa_prefill", "flash_forward_pipelined_kernel<128>"): (184.7e6 + 88.1e6, "c19a8f3"),
+    ("gqa_prefill_d256", "flash_forward_pipelined_kernel<256>"): (444.9e6 + 100.9e6, "c19a8f3"),
+    ("gqa_decode", "decode_fused_kernel<128,6>"): (1045.2e6 + 13.0e6, "c19a8f3"),
+    ("gdn_scan", "gdn_chunk_scan"): (530.1e6 + 146.5e6, "c19a8f3"),
 }
 
 NAMES = ["mha_train_bf16", "mha_fwd_fp32", "gqa_prefill", "gqa_decode", "gdn_scan"]
