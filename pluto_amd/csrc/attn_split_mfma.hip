@@ -11,12 +11,13 @@
 // scores in products of depth 256: S 1, P V 3 (forward); S 1, dP 3, dQ 3; and
 // S 1, dP 3, dK 3, dV 6.  At sixteen times the rate of the FP32 matrix
 // instruction that is a third of its time.  T = 1024, 24/4 heads: 0.044 ms for the
-// forward with the gated output and 0.147 for the gradients (0.046 and 0.157 before the clock
-// has settled), where the kernels that multiply one element at a time took 3.9 and 12.4 ms.  What bounds them: one wave a SIMD in
-// a workgroup's chain of tiles (a step is 112 matrix instructions in the gradients, half of whose
-// time is softmax arithmetic, splits and waits beside an idle matrix pipe), about 8 us before
-// the first and after the last tile of each of 768 workgroups, and for the forward 384
-// workgroups of lengths 1 to 16 on 256 compute units.
+// forward with the gated output and 0.147 for the gradients (0.046 and 0.157 before the
+// clock has settled), where the kernels that multiply one element at a time took 3.9 and
+// 12.4 ms.  What bounds them: one wave a SIMD in a workgroup's chain of tiles (a step is 112
+// matrix instructions in the gradients, half of whose time is softmax arithmetic, splits and
+// waits beside an idle matrix pipe), about 8 us before the first and after the last tile of
+// each of 768 workgroups, and for the forward 384 workgroups of lengths 1 to 16 on 256 compute
+// units.
 //
 // Shape of the kernels as in flash_bwd_mfma.hip: four waves of 32 queries (keys)
 // each, tiles of 32 rows of the other side through two LDS stages filled by

@@ -1131,8 +1131,8 @@ bool gdn_chunked_supported(const GdnArgs& a, int chunk) {
 }
 
 // While every head of a chunk gets a compute unit of its own, three heads of one key head are
-// prepared faster by a workgroup each, though each convolves the rows of K and Q: the one
-// workgroup's 12 waves share a compute unit while others idle.  The whole forward of 16/48 heads,
+// prepared faster by a workgroup each (six by one for every two), though each convolves the
+// rows of K and Q: the one workgroup's 12 waves share a compute unit while others idle.  The whole forward of 16/48 heads,
 // three a workgroup and one: 17 tokens 29.2 and 25.6 us, 320 (240 heads of chunks) 39.7 and
 // 37.4, 400 (336) 45.2 and 44.4, 700 (528) 51.2 and 55.9, 8191 348 and 377; of 4/12 heads 1400
 // (264) 59.0 and 58.0, 2000 (384) 68.8 and 69.4.  (17 tokens took 27.0 with the convolution and
